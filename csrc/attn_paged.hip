@@ -258,7 +258,8 @@ __global__ __launch_bounds__(256) void paged_attn_v3_kernel(
     const int* __restrict__ block_tables, const int* __restrict__ ctx_lens,
     const int* __restrict__ row_seq, int max_blocks, int num_kv_heads,
     float scale, long q_stride, int h_total, int g_stride, int h_off,
-    float* __restrict__ partial) {
+    float* __restrict__ partial, const int* __restrict__ seq_start,
+    int max_portion) {
   constexpr int D = 128;
   const int row = blockIdx.x;
   const int kvh = blockIdx.y;
@@ -266,6 +267,8 @@ __global__ __launch_bounds__(256) void paged_attn_v3_kernel(
   const int H = h_total;
   const int ctx = ctx_lens[row];
   const int table = row_seq ? row_seq[row] : row;
+  if (seq_start && seq_start[table + 1] - seq_start[table] > max_portion)
+    return;
   const int* bt = block_tables + (long)table * max_blocks;
   const int nblocks = (ctx + ATTN_BS - 1) / ATTN_BS;
 
@@ -522,13 +525,16 @@ __global__ __launch_bounds__(256) void paged_attn_v3_merge_kernel(
   }
 }
 
+// With seq_start (and row_seq) only the rows of sequences that have at most
+// max_portion rows are computed.
 void launch_paged_attn(bf16* out, const bf16* q, const bf16* k_cache,
                        const bf16* v_cache, const int* block_tables,
                        const int* ctx_lens, const int* row_seq,
                        long num_rows, int num_kv_heads, int group, int D,
                        int max_blocks, int block_size, float scale,
                        long q_stride, float* split_ws, int split,
-                       bool kv_fp8, hipStream_t stream) {
+                       bool kv_fp8, const int* seq_start, int max_portion,
+                       hipStream_t stream) {
   if (block_size != ATTN_BS)
     throw std::runtime_error("paged_attn: block_size must be 16");
   // v3 (D=128): GROUP<=4 direct; GROUP=8 as two GROUP=4 half-calls over
@@ -550,12 +556,12 @@ void launch_paged_attn(bf16* out, const bf16* q, const bf16* k_cache,
             paged_attn_v3_kernel<G, true><<<grid, 256, 0, stream>>>(        \
                 out, q, k_cache, v_cache, block_tables, ctx_lens, row_seq,  \
                 max_blocks, num_kv_heads, scale, q_stride, h_total, group,  \
-                h_off, split_ws);                                           \
+                h_off, split_ws, seq_start, max_portion);                   \
           else                                                              \
             paged_attn_v3_kernel<G, false><<<grid, 256, 0, stream>>>(       \
                 out, q, k_cache, v_cache, block_tables, ctx_lens, row_seq,  \
                 max_blocks, num_kv_heads, scale, q_stride, h_total, group,  \
-                h_off, split_ws);                                           \
+                h_off, split_ws, seq_start, max_portion);                   \
           if (split > 1)                                                    \
             paged_attn_v3_merge_kernel<G><<<mgrid, 256, 0, stream>>>(       \
                 out, split_ws, split, h_total, group, h_off);               \
@@ -565,7 +571,7 @@ void launch_paged_attn(bf16* out, const bf16* q, const bf16* k_cache,
     }
     return;
   }
-  if (split != 1)
+  if (split != 1 || seq_start)
     throw std::runtime_error("paged_attn: split needs the v3 path");
   if (kv_fp8)
     throw std::runtime_error("paged_attn: fp8 KV needs head_dim 128");

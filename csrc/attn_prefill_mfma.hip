@@ -1,255 +1,388 @@
-// Flash-style varlen causal prefill attention on MFMA (gfx950), bf16,
-// head_dim 128.
+// Causal prompt attention on the matrix cores (gfx950), bf16, head_dim 128.
 //
-// Replaces the per-row prefill path (each query re-reading its context —
-// measured 1.34 ms/layer at 8k prefill tokens, profiles/r01): K/V stream
-// through LDS once per 256-row q tile and the matmuls run on the matrix
-// cores (v_mfma_f32_32x32x16_bf16).
+// Sequence s has the rows seq_start[s] .. seq_start[s + 1] of q; row i of it
+// sees the first before + i + 1 tokens.  Three places that keys and values
+// come from:
+//   ROWS    k and v beside q: whole prompts, before = 0
+//   PAGES   the bf16 pages: portions whose earlier tokens are cached,
+//           before = ctx_lens[first row] - 1
+//   PAGES8  the same with e4m3 pages
 //
-// Geometry (per /opt/skills/guides/cdna_hip_programming.md §B attention):
-//   workgroup = 8 waves (512 thr) = 256 q rows of ONE (seq, q-head);
-//   wave owns 32 rows; KV tiles of 64 tokens staged in LDS
-//   (K [64][128] row-major + XOR swizzle; V transposed to [128][64] at
-//   stage so the PV B-fragment reads rows).
-//   SWAPPED QK^T — mfma(A=K, B=Q) gives S^T with the q row in the lane
-//   column, so the online-softmax row reduction is one shfl_xor(32), not a
-//   cross-lane tree (guide T12 mechanism; P goes through a per-wave LDS
-//   tile instead of permlane packing — v1).
+// What bounds it: the matrix products, 4 * 128 operations a score, against
+// about as many cycles of vector work (exponential, maximum, sum,
+// conversion).  So: scores are formed transposed, S^T = K Q^T, with the K row
+// that feeds matrix row i permuted so that the scores a lane holds are 8
+// consecutive tokens of one query row, which is the operand P^T of
+// O^T = V^T P^T: weights never leave their registers, and the running maximum
+// and its rescaling are one value a lane.  The rescaling is left out while no
+// row's maximum grew by more than 2^GROW.  V^T is read with the transposing
+// LDS load.
+//
+// A workgroup is 4 waves of 32 rows: HG heads of one kv head share a tile of
+// 64 tokens, so that the causal edge of 4 heads costs 32 rows of work and not
+// 128.  Tiles are double-buffered and (bf16) go from memory to LDS directly,
+// 16 bytes a lane; 64 KB of LDS and 256 registers leave two workgroups a CU,
+// whose products and vector work overlap.  Heads vary fastest over the
+// workgroups: with 8 kv heads a die has one of them, and its keys and values
+// stay in the die's L2.  Later rows see more and start first.
+//
+// 32 heads, 8 kv heads: a prompt of 8192 tokens 661 us (832 TFLOP/s) where
+// weights that went through LDS and tiles of 256 rows of one head took 2628
+// (209); 8 prompts of 1000, 113 us; 7808 tokens after 8192 cached ones 2.22 ms
+// (696 TFLOP/s) where one workgroup a row took 37.6.
+//
+// Weights enter the matrix cores as one bf16 (ROWS), or as a high and a low
+// part (pages: about 16 bits, which the row-by-row kernel's float weights
+// need).
 #include <float.h>
 
 #include "common.h"
 
 namespace {
 
-typedef __attribute__((ext_vector_type(8))) short short8;
-typedef __attribute__((ext_vector_type(16))) float f32x16;
+constexpr int HD = 128;
+constexpr int KV = 64;            // tokens of a tile
+constexpr int WAVE_ROWS = 32;
+constexpr int PAGE = 16;
+constexpr float LOG2E = 1.4426950408889634f;
+constexpr float GROW = 8.f;
+enum Source { ROWS, PAGES, PAGES8 };
 
-#define QBLK 32       // q rows per wave
-#define NWAVE 8
-#define QTILE (QBLK * NWAVE)   // 256 q rows per workgroup
-#define KVBLK 64
-#define HD 128        // head_dim
+typedef __attribute__((ext_vector_type(4))) short short4_t;
+typedef __attribute__((ext_vector_type(2))) float float2_t;
 
-// XOR swizzle: spread a row-major [rows][128] bf16 tile's column slices
-// over LDS banks (guide G4: D=128 rows are a 16-way conflict unswizzled)
-DEV int swz(int row, int col_byte) { return col_byte ^ ((row & 7) << 4); }
+struct Prefill {
+  bf16* out;
+  const bf16* q;
+  const bf16* k;             // rows, or pages
+  const bf16* v;
+  const int* seq_start;
+  const int* ctx_lens;       // pages only
+  const int* block_tables;
+  int seqs, H, G, max_blocks, min_rows;
+  float scale;               // times log2(e), positive: its sign, or a scale
+  short q_and, q_xor;        // of zero, is applied to the bits of q
+  long sq, sk, sv;           // strides of a row
+};
 
-__global__ __launch_bounds__(512, 1) void attn_prefill_mfma_kernel(
-    bf16* __restrict__ out, const bf16* __restrict__ q,
-    const bf16* __restrict__ k, const bf16* __restrict__ v,
-    const int* __restrict__ seq_start, int num_heads, int num_kv_heads,
-    float scale, long sq, long sk, long sv) {
-  const int h = blockIdx.y;
-  const int kvh = h / (num_heads / num_kv_heads);
-  const int z = blockIdx.z;
-  const long t0 = seq_start[z];
-  const int n = seq_start[z + 1] - (int)t0;
-  const int q0 = blockIdx.x * QTILE;
-  if (q0 >= n) return;
+DEV float exp2_fast(float x) { return __builtin_amdgcn_exp2f(x); }
 
-  // LDS: K tile + V^T tile + per-wave P tiles + per-wave alpha/lsum
-  __shared__ __attribute__((aligned(16))) short k_lds[KVBLK * HD];
-  __shared__ __attribute__((aligned(16))) short vt_lds[HD * KVBLK];
-  __shared__ __attribute__((aligned(16))) short p_lds[NWAVE][QBLK * KVBLK];
-  __shared__ float alpha_lds[NWAVE][QBLK];
-  __shared__ float lsum_lds[NWAVE][QBLK];
+// 16 bytes a lane, to the wave's LDS address + lane * 16
+DEV void to_lds16(const void* g, void* l) {
+  __builtin_amdgcn_global_load_lds(
+      (const __attribute__((address_space(1))) unsigned*)g,
+      (__attribute__((address_space(3))) unsigned*)l, 16, 0, 0);
+}
 
-  const int tid = threadIdx.x;
-  const int wid = tid >> 6;
-  const int lane = tid & 63;
-  const int lcol = lane & 31;     // q column this lane owns in S^T
-  const int lhalf = lane >> 5;
+// four rows of one column: in every 16 lanes, lane i passes the address of
+// row i / 4, columns 4 (i % 4), and receives column i
+DEV short4_t lds_read_tr(const short* p) {
+  return __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+      (__attribute__((address_space(3))) short4_t*)p);
+}
 
-  // ---- load this wave's Q as 8 B-fragments (held for the whole loop) ----
-  // B[k=dim][j=q]: lane j = lcol, k = c*16 + lhalf*8 + e  (16B per chunk)
-  const int qrow = q0 + wid * QBLK + lcol;
-  short8 qfrag[8];
+// of the lanes i and i ^ 32
+DEV float max_halves(float x) {
+  const unsigned u = __float_as_uint(x);
+  const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
+// 16-byte unit c of row r of a tile in LDS (rows of 16 units): the reads of
+// 16 rows of one unit, and of 4 rows of 64 bytes each, spread over the banks
+DEV int k_unit(int r, int c) { return r * 16 + (c ^ (r & 15)); }
+DEV int v_unit(int r, int c) { return r * 16 + (c ^ (r & 3) << 2); }
+
+// 4 e4m3 bytes as bf16, exactly
+DEV uint2 widen(unsigned x) {
+  const float2_t a = __builtin_amdgcn_cvt_pk_f32_fp8(x, false);
+  const float2_t b = __builtin_amdgcn_cvt_pk_f32_fp8(x, true);
+  return uint2{cvt_pk_bf16(a.x, a.y), cvt_pk_bf16(b.x, b.y)};
+}
+
+template <int HG, int SRC>
+__global__ __launch_bounds__(256, 2) void attn_prefill_kernel(Prefill a) {
+  constexpr int RG = 4 / HG;                 // row groups of 32
+  constexpr int TILE_ROWS = RG * WAVE_ROWS;
+  constexpr bool SPLIT = SRC != ROWS;
+  __shared__ __attribute__((aligned(16))) short lds[2][2][KV * HD];
+
+  // Sequence s has the places seq_start[s] / TILE_ROWS + s and up, as many
+  // as its tiles or more; the last places come first.
+  const int w = gridDim.y - 1 - blockIdx.y;
+  int s = 0;
+  for (int hi = a.seqs; hi - s > 1;) {
+    const int mid = (s + hi) >> 1;
+    if (a.seq_start[mid] / TILE_ROWS + mid <= w) s = mid; else hi = mid;
+  }
+  const int t0 = a.seq_start[s], n = a.seq_start[s + 1] - t0;
+  const int r0 = (w - t0 / TILE_ROWS - s) * TILE_ROWS;   // first row in s
+  if (r0 >= n || n < a.min_rows) return;
+  const int before = SRC == ROWS ? 0 : a.ctx_lens[t0] - 1;
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int col = lane & 31, hf = lane >> 5;
+  const int h = blockIdx.x * HG + wid % HG;
+  const int g = blockIdx.x * HG / (a.H / a.G);   // one for HG heads
+  const int rw = r0 + wid / HG * WAVE_ROWS;      // the wave's first row
+  const int row = rw + col;
+  const int last = before + min(r0 + TILE_ROWS, n) - 1;  // last token seen
+  const int w_last = before + min(rw + WAVE_ROWS, n) - 1;
+
+  short8_t qf[8];
   {
-    const bf16* qp = q + (t0 + qrow) * sq + (long)h * HD;
+    const bf16* qp = a.q + (t0 + min(row, n - 1)) * a.sq + (long)h * HD;
     #pragma unroll
-    for (int c = 0; c < 8; ++c) {
-      if (qrow < n) {
-        qfrag[c] = *reinterpret_cast<const short8*>(
-            qp + c * 16 + lhalf * 8);
-      } else {
-        qfrag[c] = short8{0, 0, 0, 0, 0, 0, 0, 0};
+    for (int c = 0; c < 8; ++c)
+      qf[c] = (*reinterpret_cast<const short8_t*>(qp + c * 16 + hf * 8) &
+               a.q_and) ^ a.q_xor;
+  }
+  f32x16_t acc[4];
+  #pragma unroll
+  for (int e = 0; e < 4; ++e) acc[e] = f32x16_t(0.f);
+  float m = -FLT_MAX, l = 0.f;
+
+  // ---- tiles.  bf16: a wave brings 4 KB-units of K and of V, rows 16 j +
+  // 4 wid and the three after it; tokens past the last one read that again
+  // (their weight is zero).  A tile's pages are looked up one tile ahead.
+  const int* bt = SRC == ROWS ? nullptr
+                              : a.block_tables + (long)s * a.max_blocks;
+  const int last_page = last / PAGE;
+  int ids[4];
+  auto look_up = [&](int kv0) {
+    #pragma unroll
+    for (int j = 0; j < 4; ++j)
+      ids[j] = bt[min(kv0 / PAGE + j, last_page)];
+  };
+  const int lr = 4 * wid + (lane >> 4);          // row within 16
+  const int kc = ((lane & 15) ^ lr) * 8;         // its column of K, and of V
+  const int vc = ((lane & 15) ^ (lane >> 4) << 2) * 8;
+  const bf16* k0 = a.k + g * HD + kc;            // ROWS
+  const bf16* v0 = a.v + g * HD + vc;
+  uint4 raw[4];                                  // PAGES8: 32 bytes each
+  auto fetch = [&](int kv0, int buf) {
+    if constexpr (SRC == PAGES8) {
+      const int tok = tid >> 2;
+      const int id = ids[0] * (tok < 16) + ids[1] * (tok >> 4 == 1) +
+                     ids[2] * (tok >> 4 == 2) + ids[3] * (tok >> 4 == 3);
+      const long at = (((long)id * a.G + g) * PAGE + tok % PAGE) * HD +
+                      (tid & 3) * 32;
+      const char* kp = reinterpret_cast<const char*>(a.k) + at;
+      const char* vp = reinterpret_cast<const char*>(a.v) + at;
+      #pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        raw[i] = reinterpret_cast<const uint4*>(kp)[i];
+        raw[2 + i] = reinterpret_cast<const uint4*>(vp)[i];
+      }
+    } else {
+      #pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const bf16 *kp, *vp;
+        if constexpr (SRC == ROWS) {
+          const unsigned r = t0 + min(kv0 + 16 * j + lr, n - 1);
+          kp = k0 + (unsigned long)r * (unsigned)a.sk;
+          vp = v0 + (unsigned long)r * (unsigned)a.sv;
+        } else {
+          const long at = (((long)ids[j] * a.G + g) * PAGE + lr) * HD;
+          kp = a.k + at + kc;
+          vp = a.v + at + vc;
+        }
+        to_lds16(kp, &lds[buf][0][(16 * j + 4 * wid) * HD]);
+        to_lds16(vp, &lds[buf][1][(16 * j + 4 * wid) * HD]);
       }
     }
-  }
-
-  f32x16 acc[4];      // O[q][d] per 32-wide d tile
-  #pragma unroll
-  for (int dt = 0; dt < 4; ++dt) acc[dt] = f32x16(0.f);
-  float m_run = -FLT_MAX, l_run = 0.f;
-
-  const int q_hi = min(q0 + QTILE, n);         // exclusive
-  const int nkv_tiles = (q_hi + KVBLK - 1) / KVBLK;
-
-  for (int kt = 0; kt < nkv_tiles; ++kt) {
-    const int kv0 = kt * KVBLK;
-    const int kvn = min(KVBLK, n - kv0);
-    // ---- stage K [64][128] (swizzled) and V^T [128][64] ----
-    {
-      // K: 1024 16B units; unit u: row r = u/16, colb = (u%16)*16
-      for (int u = tid; u < KVBLK * 16; u += 512) {
-        const int r = u >> 4, cb = (u & 15) << 4;
-        uint4 val{0, 0, 0, 0};
-        if (r < kvn)
-          val = *reinterpret_cast<const uint4*>(
-              reinterpret_cast<const char*>(k + (t0 + kv0 + r) * sk +
-                                            (long)kvh * HD) + cb);
-        *reinterpret_cast<uint4*>(
-            reinterpret_cast<char*>(k_lds) + r * 256 + swz(r, cb)) = val;
+  };
+  auto store = [&](int buf) {                    // PAGES8
+    const int tok = tid >> 2;
+    #pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const unsigned* x = &raw[i].x;
+      uint4 u[2];
+      #pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const uint2 lo = widen(x[2 * j]), hi = widen(x[2 * j + 1]);
+        u[j] = uint4{lo.x, lo.y, hi.x, hi.y};
       }
-      // V^T: unit u handles kv rows (2p, 2p+1) x 8 dims: 32 pairs x 16
-      // dim-chunks = 512 units
-      for (int u = tid; u < 512; u += 512) {
-        const int p2 = u & 31, dc = u >> 5;          // pair, dim chunk
-        const int r0 = 2 * p2;
-        uint4 a{0, 0, 0, 0}, b{0, 0, 0, 0};
-        if (r0 < kvn)
-          a = *reinterpret_cast<const uint4*>(
-              v + (t0 + kv0 + r0) * sv + (long)kvh * HD + dc * 8);
-        if (r0 + 1 < kvn)
-          b = *reinterpret_cast<const uint4*>(
-              v + (t0 + kv0 + r0 + 1) * sv + (long)kvh * HD + dc * 8);
-        const unsigned* au = reinterpret_cast<const unsigned*>(&a);
-        const unsigned* bu = reinterpret_cast<const unsigned*>(&b);
+      #pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const int c = (tid & 3) * 4 + (i & 1) * 2 + j;
+        reinterpret_cast<uint4*>(lds[buf][i >> 1])
+            [i < 2 ? k_unit(tok, c) : v_unit(tok, c)] = u[j];
+      }
+    }
+  };
+
+  // matrix row i of a 32-token block takes this token's key, so that
+  // sc[b][r] is token 32 b + (r >> 3) * 16 + hf * 8 + (r & 7)
+  const int krow = (col & 16) + ((col >> 2) & 1) * 8 + ((col >> 3) & 1) * 4 +
+                   (col & 3);
+  const int k_at = k_unit(krow, hf) * 16;        // bytes; step c: ^ c << 5
+  // V^T: lane's part of a read of 4 tokens by 16 columns; block e: ^ e << 6
+  const int vr = hf * 8 + ((lane & 15) >> 2);
+  const int vcol = (lane >> 4 & 1) * 16 + (lane & 3) * 4;
+  const int v_at = v_unit(vr, vcol >> 3) * 16 + (vcol & 7) * 2;
+
+  auto compute = [&](int kv0, int buf) {
+    const char* kl = reinterpret_cast<const char*>(lds[buf][0]);
+    const char* vl = reinterpret_cast<const char*>(lds[buf][1]);
+    f32x16_t sc[2];
+    #pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      sc[b] = f32x16_t(0.f);
+      #pragma unroll
+      for (int c = 0; c < 8; ++c)
+        sc[b] = mfma32(*reinterpret_cast<const short8_t*>(
+                           kl + (k_at ^ c << 5) + b * 32 * HD * 2),
+                       qf[c], sc[b]);
+      // the operands of all parts are not to be in registers together
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (kv0 + KV - 1 > before + rw) {
+      #pragma unroll
+      for (int b = 0; b < 2; ++b)
+        #pragma unroll
+        for (int r = 0; r < 16; ++r)
+          if (kv0 + b * 32 + (r >> 3) * 16 + hf * 8 + (r & 7) > before + row)
+            sc[b][r] = -FLT_MAX;
+    }
+    float mx = -FLT_MAX;
+    #pragma unroll
+    for (int b = 0; b < 2; ++b)
+      #pragma unroll
+      for (int r = 0; r < 16; ++r) mx = fmaxf(mx, sc[b][r]);
+    mx = max_halves(mx) * a.scale;
+    if (__any(mx > m + GROW)) {
+      const float top = fmaxf(m, mx);
+      const float alpha = m == -FLT_MAX ? 0.f : exp2_fast(m - top);
+      #pragma unroll
+      for (int e = 0; e < 4; ++e)
+        #pragma unroll
+        for (int r = 0; r < 16; ++r) acc[e][r] *= alpha;
+      l *= alpha;
+      m = top;
+    }
+    const float base = m == -FLT_MAX ? 0.f : m;
+    __builtin_amdgcn_sched_barrier(0);
+    #pragma unroll
+    for (int b = 0; b < 2; ++b)
+      #pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        float p[8];
         #pragma unroll
         for (int j = 0; j < 8; ++j) {
-          const unsigned av = (au[j >> 1] >> ((j & 1) * 16)) & 0xffff;
-          const unsigned bv = (bu[j >> 1] >> ((j & 1) * 16)) & 0xffff;
-          const int d = dc * 8 + j;
-          *reinterpret_cast<unsigned*>(
-              reinterpret_cast<char*>(vt_lds) + d * (KVBLK * 2) +
-              swz(d, r0 * 2)) = av | (bv << 16);
+          p[j] = exp2_fast(fmaf(sc[b][c * 8 + j], a.scale, -base));
+          l += p[j];
         }
+        short8_t ph, pl;
+        if constexpr (SPLIT) {
+          split_bf16x8(p, &ph, &pl);
+        } else {
+          union { unsigned u[4]; short8_t v; } x;
+          #pragma unroll
+          for (int j = 0; j < 4; ++j)
+            x.u[j] = cvt_pk_bf16(p[2 * j], p[2 * j + 1]);
+          ph = x.v;
+        }
+        #pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          union { short4_t h[2]; short8_t v; } vf;
+          #pragma unroll
+          for (int i = 0; i < 2; ++i)
+            vf.h[i] = lds_read_tr(reinterpret_cast<const short*>(
+                vl + (v_at ^ e << 6) + (b * 32 + c * 16 + i * 4) * HD * 2));
+          acc[e] = mfma32(vf.v, ph, acc[e]);
+          if constexpr (SPLIT) acc[e] = mfma32(vf.v, pl, acc[e]);
+        }
+        if (c) __builtin_amdgcn_sched_barrier(0);
       }
-    }
-    __syncthreads();
+  };
 
-    // ---- QK^T (swapped): S^T[kv][q] in two 32-row tiles ----
-    f32x16 s[2];
-    #pragma unroll
-    for (int rt = 0; rt < 2; ++rt) {
-      s[rt] = f32x16(0.f);
-      const int arow = rt * 32 + lcol;         // K row this lane feeds
-      #pragma unroll
-      for (int c = 0; c < 8; ++c) {
-        short8 kf = *reinterpret_cast<const short8*>(
-            reinterpret_cast<char*>(k_lds) + arow * 256 +
-            swz(arow, c * 32 + lhalf * 16));
-        s[rt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qfrag[c],
-                                                        s[rt], 0, 0, 0);
-      }
-    }
-    // ---- online softmax on the lane's 32 scores (one q column) ----
-    const int qg = q0 + wid * QBLK + lcol;     // this lane's q row
-    float p[2][16];
-    float tile_max = -FLT_MAX;
-    #pragma unroll
-    for (int rt = 0; rt < 2; ++rt) {
-      #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int kvr = kv0 + rt * 32 + (r & 3) + 8 * (r >> 2) + 4 * lhalf;
-        float sv_ = s[rt][r] * scale;
-        if (kvr > qg || kvr >= n || qg >= n) sv_ = -FLT_MAX;
-        p[rt][r] = sv_;
-        tile_max = fmaxf(tile_max, sv_);
-      }
-    }
-    tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 32));
-    const float m_new = fmaxf(m_run, tile_max);
-    const float alpha = (m_run == -FLT_MAX || m_new == -FLT_MAX)
-        ? 0.f : __expf(m_run - m_new);
-    float lsum = 0.f;
-    #pragma unroll
-    for (int rt = 0; rt < 2; ++rt) {
-      #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const float e = (p[rt][r] == -FLT_MAX || m_new == -FLT_MAX)
-            ? 0.f : __expf(p[rt][r] - m_new);
-        p[rt][r] = e;
-        lsum += e;
-      }
-    }
-    lsum += __shfl_xor(lsum, 32);
-    l_run = l_run * alpha + lsum;
-    m_run = m_new;
-    if (lhalf == 0) alpha_lds[wid][lcol] = alpha;
-    // ---- P -> per-wave LDS [32 q][64 kv] bf16 (packed pair writes) ----
-    #pragma unroll
-    for (int rt = 0; rt < 2; ++rt) {
-      #pragma unroll
-      for (int r = 0; r < 16; r += 2) {
-        const int kvr = rt * 32 + (r & 3) + 8 * (r >> 2) + 4 * lhalf;
-        const unsigned lo = f2bf(p[rt][r]);
-        const unsigned hi = f2bf(p[rt][r + 1]);
-        *reinterpret_cast<unsigned*>(
-            reinterpret_cast<char*>(p_lds[wid]) + lcol * (KVBLK * 2) +
-            swz(lcol, kvr * 2)) = lo | (hi << 16);
-      }
-    }
-    // ---- rescale O by alpha of each C row (alphas via wave LDS) ----
-    #pragma unroll
-    for (int dt = 0; dt < 4; ++dt) {
-      #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int qrow_c = (r & 3) + 8 * (r >> 2) + 4 * lhalf;
-        acc[dt][r] *= alpha_lds[wid][qrow_c];
-      }
-    }
-    // ---- PV: O[q][d] += P[q][kv] * V[kv][d] ----
-    #pragma unroll
-    for (int dt = 0; dt < 4; ++dt) {
-      #pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        // A = P: i=q=lcol, k = c*16 + lhalf*8 (+e)
-        short8 pf = *reinterpret_cast<const short8*>(
-            reinterpret_cast<char*>(p_lds[wid]) + lcol * (KVBLK * 2) +
-            swz(lcol, c * 32 + lhalf * 16));
-        // B = V: j=d=dt*32+lcol, k = kv chunk -> V^T row j
-        const int vrow = dt * 32 + lcol;
-        short8 vf = *reinterpret_cast<const short8*>(
-            reinterpret_cast<char*>(vt_lds) + vrow * (KVBLK * 2) +
-            swz(vrow, c * 32 + lhalf * 16));
-        acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(pf, vf, acc[dt],
-                                                          0, 0, 0);
-      }
-    }
+  auto landed = [&](int buf) {
+    if constexpr (SRC == PAGES8) store(buf);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
+  };
+  if constexpr (SRC != ROWS) look_up(0);
+  fetch(0, 0);
+  if constexpr (SRC != ROWS) look_up(KV);
+  landed(0);
+  int buf = 0;
+  for (int kv0 = 0; kv0 <= last; kv0 += KV, buf ^= 1) {
+    const bool more = kv0 + KV <= last;
+    if (more) {
+      fetch(kv0 + KV, buf ^ 1);
+      if constexpr (SRC != ROWS) look_up(kv0 + 2 * KV);
+    }
+    if (rw < n && kv0 <= w_last) compute(kv0, buf);
+    if (more) landed(buf ^ 1);
   }
 
-  // ---- epilogue: O /= l, store masked rows ----
-  // (lsum_lds is wave-private; in-wave LDS ops are program-ordered)
-  if (lhalf == 0) lsum_lds[wid][lcol] = l_run;
+  l += __shfl_xor(l, 32);
+  if (row >= n) return;
+  // acc[e][r]: column e * 32 + (r >> 2) * 8 + hf * 4 + (r & 3)
+  const bool none = SRC == ROWS && !(l > 0.f);
+  const float inv = 1.f / l;
+  bf16* op = a.out + ((long)(t0 + row) * a.H + h) * HD + hf * 4;
   #pragma unroll
-  for (int dt = 0; dt < 4; ++dt) {
+  for (int e = 0; e < 4; ++e)
     #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int qrow_c = (r & 3) + 8 * (r >> 2) + 4 * lhalf;
-      const int qg = q0 + wid * QBLK + qrow_c;
-      if (qg >= n) continue;
-      const float l = lsum_lds[wid][qrow_c];
-      const float o = l > 0.f ? acc[dt][r] / l : 0.f;
-      *(unsigned short*)(out + ((t0 + qg) * (long)num_heads + h) * HD +
-                         dt * 32 + lcol) = f2bf(o);
+    for (int r = 0; r < 16; r += 4) {
+      float x[4];
+      #pragma unroll
+      for (int j = 0; j < 4; ++j) x[j] = none ? 0.f : acc[e][r + j] * inv;
+      *reinterpret_cast<uint2*>(op + e * 32 + r * 2) =
+          uint2{cvt_pk_bf16(x[0], x[1]), cvt_pk_bf16(x[2], x[3])};
     }
-  }
+}
+
+template <int SRC>
+void launch(const Prefill& p, long rows, hipStream_t stream) {
+  if (rows == 0 || p.seqs == 0) return;
+  Prefill a = p;
+  a.q_and = a.scale == 0.f ? 0 : -1;
+  a.q_xor = a.scale < 0.f ? (short)0x8000 : 0;
+  a.scale = a.scale == 0.f ? 1.f : fabsf(a.scale) * LOG2E;
+  const int group = a.H / a.G;
+  #define RUN(HG)                                                           \
+    attn_prefill_kernel<HG, SRC>                                            \
+        <<<dim3((unsigned)(a.H / HG),                                       \
+                (unsigned)(rows / (4 / HG * WAVE_ROWS) + a.seqs)),          \
+           256, 0, stream>>>(a)
+  if (group % 4 == 0) RUN(4);
+  else if (group % 2 == 0) RUN(2);
+  else RUN(1);
+  #undef RUN
 }
 
 }  // namespace
 
 void launch_attn_prefill_mfma(bf16* out, const bf16* q, const bf16* k,
                               const bf16* v, const int* seq_start,
-                              int num_seqs, int max_seqlen, int num_heads,
+                              int num_seqs, long rows, int num_heads,
                               int num_kv_heads, int head_dim, float scale,
                               long sq, long sk, long sv,
                               hipStream_t stream) {
   if (head_dim != HD)
     throw std::runtime_error("attn_prefill_mfma: head_dim must be 128");
-  dim3 grid((unsigned)((max_seqlen + QTILE - 1) / QTILE),
-            (unsigned)num_heads, (unsigned)num_seqs);
-  attn_prefill_mfma_kernel<<<grid, 512, 0, stream>>>(
-      out, q, k, v, seq_start, num_heads, num_kv_heads, scale, sq, sk, sv);
+  launch<ROWS>({out, q, k, v, seq_start, nullptr, nullptr, num_seqs,
+                num_heads, num_kv_heads, 0, 0, scale, 0, 0, sq, sk, sv},
+               rows, stream);
+}
+
+// portions of at least min_rows rows; the others' rows are left as they are
+void launch_attn_prefill_paged(bf16* out, const bf16* q, const bf16* k_cache,
+                               const bf16* v_cache, const int* block_tables,
+                               const int* ctx_lens, const int* seq_start,
+                               int num_seqs, long rows, int num_heads,
+                               int num_kv_heads, int max_blocks, int min_rows,
+                               float scale, long sq, bool kv_fp8,
+                               hipStream_t stream) {
+  const Prefill a{out, q, k_cache, v_cache, seq_start, ctx_lens, block_tables,
+                  num_seqs, num_heads, num_kv_heads, max_blocks, min_rows,
+                  scale, 0, 0, sq, 0, 0};
+  if (kv_fp8)
+    launch<PAGES8>(a, rows, stream);
+  else
+    launch<PAGES>(a, rows, stream);
 }

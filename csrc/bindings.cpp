@@ -19,10 +19,14 @@ void launch_rope_kv_append(bf16*, bf16*, const bf16*, const long*,
 void launch_paged_attn(bf16*, const bf16*, const bf16*, const bf16*,
                        const int*, const int*, const int*, long, int, int,
                        int, int, int, float, long, float*, int, bool,
-                       hipStream_t);
+                       const int*, int, hipStream_t);
 void launch_attn_prefill_mfma(bf16*, const bf16*, const bf16*,
-                              const bf16*, const int*, int, int, int, int,
+                              const bf16*, const int*, int, long, int, int,
                               int, float, long, long, long, hipStream_t);
+void launch_attn_prefill_paged(bf16*, const bf16*, const bf16*, const bf16*,
+                               const int*, const int*, const int*, int, long,
+                               int, int, int, int, float, long, bool,
+                               hipStream_t);
 template <typename T>
 void launch_gelu_mul(T*, const T*, long, int, hipStream_t);
 template <typename T>
@@ -203,7 +207,7 @@ void paged_attn(torch::Tensor out, torch::Tensor q, torch::Tensor k_cache,
                     block_tables.data_ptr<int>(), ctx_lens.data_ptr<int>(),
                     rs, R, KV, H / KV, D, (int)block_tables.size(1), BS,
                     (float)scale, q.stride(0), ws, (int)split, kv_fp8,
-                    stream());
+                    nullptr, 0, stream());
 }
 
 void attn_prefill_mfma(torch::Tensor out, torch::Tensor q, torch::Tensor k,
@@ -214,12 +218,60 @@ void attn_prefill_mfma(torch::Tensor out, torch::Tensor q, torch::Tensor k,
   check_qkv_view(k, "k");
   check_qkv_view(v, "v");
   check(seq_start, torch::kInt32, "seq_start");
+  TORCH_CHECK(seq_start.numel() >= 1, "seq_start");
   const int H = (int)q.size(1), D = (int)q.size(2);
   const int KV = (int)k.size(1);
+  TORCH_CHECK(KV > 0 && H % KV == 0, "GQA group");
+  // keys and values are read 16 bytes at a time straight into LDS
+  auto aligned = [](const torch::Tensor& t) {
+    return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0 &&
+                   t.stride(0) % 8 == 0
+               ? t : t.clone(at::MemoryFormat::Contiguous);
+  };
+  k = aligned(k);
+  v = aligned(v);
   launch_attn_prefill_mfma(
       bf(out), cbf(q), cbf(k), cbf(v), seq_start.data_ptr<int>(),
-      (int)seq_start.numel() - 1, (int)max_seqlen, H, KV, D, (float)scale,
+      (int)seq_start.numel() - 1, q.size(0), H, KV, D, (float)scale,
       q.stride(0), k.stride(0), v.stride(0), stream());
+}
+
+// Attention of portions over the pages, head_dim 128: on the matrix cores from
+// min_rows rows on; with `short_too` the rows of shorter ones one by one.
+void attn_portions(torch::Tensor out, torch::Tensor q, torch::Tensor k_cache,
+                   torch::Tensor v_cache, torch::Tensor block_tables,
+                   torch::Tensor ctx_lens, torch::Tensor row_seq,
+                   torch::Tensor seq_start, long min_rows, bool short_too,
+                   double scale) {
+  check(out, torch::kBFloat16, "out");
+  check_qkv_view(q, "q");
+  check(block_tables, torch::kInt32, "block_tables");
+  check(ctx_lens, torch::kInt32, "ctx_lens");
+  check(row_seq, torch::kInt32, "row_seq");
+  check(seq_start, torch::kInt32, "seq_start");
+  const long T = q.size(0), seqs = seq_start.numel() - 1;
+  const int H = (int)q.size(1), KV = (int)k_cache.size(1);
+  const int max_blocks = (int)block_tables.size(1);
+  TORCH_CHECK(KV > 0 && H % KV == 0, "GQA group");
+  TORCH_CHECK(q.size(2) == 128 && k_cache.size(3) == 128 &&
+                  k_cache.size(2) == 16, "attn_portions: shape");
+  TORCH_CHECK(v_cache.scalar_type() == k_cache.scalar_type() &&
+                  k_cache.is_contiguous() && v_cache.is_contiguous(),
+              "k/v cache");
+  TORCH_CHECK(ctx_lens.numel() == T && row_seq.numel() == T &&
+                  block_tables.size(0) >= seqs, "attn_portions: rows");
+  const bool fp8 = k_cache.scalar_type() == torch::kFloat8_e4m3fn;
+  if (short_too)
+    launch_paged_attn(bf(out), cbf(q), cbf(k_cache), cbf(v_cache),
+                      block_tables.data_ptr<int>(), ctx_lens.data_ptr<int>(),
+                      row_seq.data_ptr<int>(), T, KV, H / KV, 128, max_blocks,
+                      16, (float)scale, q.stride(0), nullptr, 1, fp8,
+                      seq_start.data_ptr<int>(), (int)min_rows - 1, stream());
+  launch_attn_prefill_paged(
+      bf(out), cbf(q), cbf(k_cache), cbf(v_cache),
+      block_tables.data_ptr<int>(), ctx_lens.data_ptr<int>(),
+      seq_start.data_ptr<int>(), (int)seqs, T, H, KV, max_blocks,
+      (int)min_rows, (float)scale, q.stride(0), fp8, stream());
 }
 
 void silu_mul(torch::Tensor out, torch::Tensor x) {
@@ -960,6 +1012,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("rope_kv_append", &rope_kv_append);
   m.def("paged_attn", &paged_attn);
   m.def("attn_prefill_mfma", &attn_prefill_mfma);
+  m.def("attn_portions", &attn_portions);
   m.def("silu_mul", &silu_mul);
   m.def("gelu_mul", &gelu_mul);
   m.def("embed_dyt", &embed_dyt);

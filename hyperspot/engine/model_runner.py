@@ -183,6 +183,8 @@ class ModelRunner:
             seq_start=torch.tensor(starts, dtype=torch.int32, device=d),
             max_seqlen=max((r.chunk_len or r.num_prompt_tokens)
                            for r in batch.requests),
+            min_seqlen=min((r.chunk_len or r.num_prompt_tokens)
+                           for r in batch.requests),
             fresh_prefill=fresh,
             row_seq=torch.tensor(row_seq, dtype=torch.int32, device=d),
             ctx_lens=(positions + 1).to(torch.int32),

@@ -53,6 +53,7 @@ class ForwardMeta:
     # prefill
     seq_start: Optional[torch.Tensor] = None   # [num_seqs+1] int32
     max_seqlen: int = 0
+    min_seqlen: int = 0            # 0: not known
     row_seq: Optional[torch.Tensor] = None     # [T] int32 row -> seq index
     ctx_lens: Optional[torch.Tensor] = None    # [T] int32 = position + 1
     # decode (block_tables also used by GPU prefill, indexed via row_seq)

@@ -1,0 +1,97 @@
+"""Prompt attention on the matrix cores: portions over the pages, and the
+edges of tiles, against the PyTorch reference in float64.
+
+Bounds: outputs are rounded to bf16 (2^-9 of the value) and are means of
+values of about one; weights enter as two bf16 parts over the pages (2^-16)
+and as one (2^-9) beside q."""
+
+import pytest
+import torch
+
+import hyperspot.engine  # noqa: F401  (before the models, which it imports)
+import hyperspot.ops as ops
+from hyperspot.models.llama import ForwardMeta
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+D = 128
+
+
+def _reference(q, k, v, before, scale):
+    """q [n, H, D] are the tokens after `before` of k, v [before + n, KV, D]."""
+    n, group = q.shape[0], q.shape[1] // k.shape[1]
+    k, v = (t.double().repeat_interleave(group, 1) for t in (k, v))
+    s = torch.einsum("qhd,khd->hqk", q.double().cpu(), k.cpu()) * scale
+    seen = torch.arange(k.shape[0])[None] <= before + torch.arange(n)[:, None]
+    s = s.masked_fill(~seen, float("-inf")).softmax(-1)
+    return torch.einsum("hqk,khd->qhd", s, v.cpu())
+
+
+def _check(out, ref, weight_step):
+    err = (out.double().cpu() - ref).abs()
+    bound = ref.abs() * 2.0 ** -8 + weight_step * 4
+    assert (err <= bound).all(), float((err - bound).max())
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("group,kv", [(4, 2), (8, 1), (2, 3), (1, 2)])
+@pytest.mark.parametrize("portions", [
+    [(0, 16), (16, 17), (47, 63), (64, 1)],     # (before, rows)
+    [(100, 130), (0, 64), (3, 15), (200, 32)],
+    [(1, 257)],
+])
+def test_portions_over_pages(portions, group, kv, fp8):
+    g = torch.Generator().manual_seed(3)
+    heads, lens = group * kv, [n for _, n in portions]
+    total = sum(lens)
+    q = torch.randn(total, heads, D, generator=g).bfloat16().to(DEV)
+    tables = [-(-(b + n) // 16) for b, n in portions]
+    pages = sum(tables) + 3
+    order = torch.randperm(pages, generator=g)
+    kind = torch.float8_e4m3fn if fp8 else torch.bfloat16
+    # what the last page holds after the last token is not a part of it
+    kc, vc = (torch.randn(pages, kv, 16, D, generator=g).to(kind).to(DEV)
+              for _ in range(2))
+    bt = torch.zeros(len(portions), max(tables) + 1, dtype=torch.int32)
+    at, starts, ctx, row_seq = 0, [0], [], []
+    for i, (b, n) in enumerate(portions):
+        bt[i, :tables[i]] = order[at:at + tables[i]]
+        at += tables[i]
+        starts.append(starts[-1] + n)
+        ctx += range(b + 1, b + n + 1)
+        row_seq += [i] * n
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    meta = ForwardMeta("prefill", None, None, seq_start=i32(starts),
+                       max_seqlen=max(lens), row_seq=i32(row_seq),
+                       ctx_lens=i32(ctx), block_tables=bt.to(DEV),
+                       fresh_prefill=False)
+    out = ops.attention(q, None, None, kc, vc, meta, D ** -0.5)
+    for i, (b, n) in enumerate(portions):
+        page = bt[i, :tables[i]].long().to(DEV)
+        k, v = (c[page].float().transpose(1, 2).reshape(-1, kv, D)[:b + n]
+                for c in (kc, vc))
+        rows = slice(starts[i], starts[i] + n)
+        _check(out[rows], _reference(q[rows], k, v, b, D ** -0.5), 2.0 ** -14)
+
+
+@pytest.mark.parametrize("scale", [D ** -0.5, -0.2, 0.0])
+@pytest.mark.parametrize("heads,kv", [(4, 1), (6, 2), (2, 1), (3, 3)])
+@pytest.mark.parametrize("lens", [[1, 31, 32, 33], [64, 129, 0, 2], [200]])
+def test_whole_prompts(lens, heads, kv, scale):
+    g = torch.Generator().manual_seed(4)
+    total = sum(lens)
+    # columns of one buffer, as the projection leaves them
+    qkv = torch.randn(total, (heads + 2 * kv) * D, generator=g) \
+        .bfloat16().to(DEV)
+    q, k, v = (t.view(total, -1, D) for t in
+               qkv.split([heads * D, kv * D, kv * D], -1))
+    starts = [sum(lens[:i]) for i in range(len(lens) + 1)]
+    meta = ForwardMeta("prefill", None, None, max_seqlen=max(lens),
+                       seq_start=torch.tensor(starts, dtype=torch.int32,
+                                              device=DEV))
+    out = ops.attention(q, k, v, k.new_empty(0, kv, 16, D), None, meta, scale)
+    for a, b in zip(starts, starts[1:]):
+        if a < b:
+            _check(out[a:b], _reference(q[a:b], k[a:b], v[a:b], 0, scale),
+                   2.0 ** -9)
