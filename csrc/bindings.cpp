@@ -109,6 +109,9 @@ void launch_moe_gemm_fp8(bf16*, float*, const unsigned char*, const float*,
                          const int*, int, int, int, int, int, hipStream_t);
 template <typename T>
 void launch_greedy_sample(long*, const T*, long, int, hipStream_t);
+template <typename T>
+void launch_sample(long*, const T*, const float*, const float*, const int*,
+                   const float*, long, int, hipStream_t);
 void launch_inv_cdf_sample(long*, const float*, const float*, long, int,
                            hipStream_t);
 
@@ -861,6 +864,29 @@ void greedy_sample(torch::Tensor out, torch::Tensor logits) {
                        (int)logits.size(1), stream());
 }
 
+void sample(torch::Tensor out, torch::Tensor logits,
+            torch::Tensor temperature, torch::Tensor top_p,
+            torch::Tensor top_k, torch::Tensor uniform) {
+  check(out, torch::kLong, "out");
+  check(logits, logits.scalar_type(), "logits");
+  TORCH_CHECK(logits.dim() == 2 && logits.size(1) > 0 &&
+                  logits.size(1) < (1l << 23), "logits");
+  const long rows = logits.size(0);
+  TORCH_CHECK(out.numel() == rows, "out");
+  check_param(temperature, rows, "temperature");
+  check_param(top_p, rows, "top_p");
+  check(top_k, torch::kInt32, "top_k");
+  TORCH_CHECK(top_k.numel() == rows, "top_k");
+  check_param(uniform, rows, "uniform");
+  by_dtype(logits, [&](auto tag) {
+    using T = ELEM(tag);
+    launch_sample<T>(out.data_ptr<long>(), ptr<T>(logits),
+                     ptr<float>(temperature), ptr<float>(top_p),
+                     top_k.data_ptr<int>(), ptr<float>(uniform), rows,
+                     (int)logits.size(1), stream());
+  });
+}
+
 void inv_cdf_sample(torch::Tensor out, torch::Tensor logits,
                     torch::Tensor uniform) {
   check(out, torch::kInt64, "out");
@@ -1038,5 +1064,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   register_latent(m);
   register_sublayer(m);
   m.def("greedy_sample", &greedy_sample);
+  m.def("sample", &sample);
   m.def("inv_cdf_sample", &inv_cdf_sample);
 }

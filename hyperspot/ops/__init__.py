@@ -328,34 +328,15 @@ def greedy_sample(logits: torch.Tensor) -> torch.Tensor:
 def sample(logits: torch.Tensor, temperature: torch.Tensor,
            top_p: torch.Tensor, top_k: torch.Tensor,
            uniform: torch.Tensor) -> torch.Tensor:
-    """Batch sampling. Greedy rows (temperature==0) take the argmax kernel;
-    stochastic rows go through filtering + an inverse-CDF draw."""
+    """Batch sampling: temperature (0: the largest logit), top-k, top-p and an
+    inverse-CDF draw over the tokens in order of their ids, in one kernel."""
     if not logits.is_cuda:
         return torch_ref.sample(logits, temperature, top_p, top_k, uniform)
-    if bool((temperature == 0).all()):
-        return greedy_sample(logits)
-    # Stochastic path: torch does the (sort-based) top-k/top-p filtering,
-    # the HIP kernel does temperature softmax + inverse-CDF in one pass.
-    lf = logits.float()
-    B, V = lf.shape
-    t = temperature.clamp_min(1e-6)[:, None]
-    row = lf / t
-    if bool((top_k > 0).any()):
-        k = top_k.clamp(0, V)
-        kth = torch.where(
-            k > 0,
-            row.topk(int(k.max().clamp(min=1)), dim=-1).values.gather(
-                1, (k.clamp(min=1) - 1)[:, None]).squeeze(1),
-            torch.full_like(row[:, 0], float("-inf")))
-        row = torch.where(row < kth[:, None], float("-inf"), row)
-    if bool((top_p < 1.0).any()):
-        sp, idx = row.softmax(-1).sort(descending=True)
-        cum = sp.cumsum(-1)
-        drop = (cum - sp) >= top_p[:, None]
-        row = row.masked_fill(drop.gather(1, idx.argsort(-1)), float("-inf"))
-    out = torch.empty(B, dtype=torch.long, device=logits.device)
-    _native().inv_cdf_sample(out, row, uniform)
-    greedy = temperature == 0
-    if bool(greedy.any()):
-        out = torch.where(greedy, greedy_sample(logits), out)
+    if logits.dtype not in (torch.bfloat16, torch.float32):
+        logits = logits.float()
+    out = torch.empty(logits.shape[0], dtype=torch.long, device=logits.device)
+    f32 = lambda t: t.to(logits.device, torch.float32).contiguous()
+    _native().sample(out, logits.contiguous(), f32(temperature), f32(top_p),
+                     top_k.to(logits.device, torch.int32).contiguous(),
+                     f32(uniform))
     return out

@@ -1,0 +1,96 @@
+"""The sampling kernel against temperature, top-k, top-p and draw in float64:
+descending order is by value, then by index.
+
+Bound: weights are 2^-40 fixed point of a float exponential (2^-22 of the
+weight), so that sums and boundaries lie within 1e-6 of the float64 ones."""
+
+import pytest
+import torch
+
+import hyperspot.ops as ops
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+EPS = 1e-6
+
+
+def _row(kind, v, g):
+    x = torch.randn(v, generator=g)
+    if kind == "peaked":
+        x[torch.randint(0, v, (9,), generator=g)] += 14
+    elif kind == "ties":
+        x = (x * 2).round()
+    elif kind == "masked":
+        x[torch.rand(v, generator=g) < 0.9] = float("-inf")
+    elif kind == "equal":
+        x.fill_(-3.0)
+    elif kind == "wide":
+        x = x * 1e4
+    elif kind == "huge":
+        x = torch.where(torch.rand(v, generator=g) < 0.5, -3e38, 3e38)
+    return x
+
+
+def _allowed(x, t, p, k, u):
+    """Whether a token may be drawn, by its place in the running sum."""
+    if t == 0:
+        return x == x.max(), None
+    y = (x.double() - x.max().double()) / max(t, 1e-6)
+    if 0 < k < len(y):
+        y = y.masked_fill(x < x.topk(k).values[-1], float("-inf"))
+    w = y.softmax(-1)
+    slack = EPS
+    if p < 1:
+        s, at = w.sort(descending=True, stable=True)
+        before = s.cumsum(-1) - s
+        w[at[before >= p]] = 0
+        near = (before - p).abs() < EPS
+        slack += float(s[near].sum())
+    c = w.cumsum(-1)
+    z = float(c[-1])
+    return (c + slack * 2 > u * z) & (c - w - slack * 2 <= u * z) \
+        & (w + slack > 0), w
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("vocab", [1, 7, 1000, 8193, 50257, 128256])
+def test_sample_against_float64(vocab, dtype):
+    g = torch.Generator().manual_seed(vocab)
+    kinds = ["normal", "peaked", "ties", "masked", "equal", "wide", "huge"]
+    options = [(1.0, 1.0, 0), (0.7, 0.9, 0), (1.3, 0.5, 40), (0.0, 1.0, 0),
+               (1.0, 1.0, 5), (0.8, 0.999, vocab), (2.0, 0.95, 600),
+               (1e-3, 0.9, 0), (0.9, 1e-7, 3)]
+    rows, want = [], []
+    for kind in kinds:
+        for t, p, k in options:
+            rows.append(_row(kind, vocab, g))
+            want.append((t, p, k))
+    x = torch.stack(rows).to(dtype)
+    t, p, k = (torch.tensor(c) for c in zip(*want))
+    u = torch.rand(len(rows), generator=g)
+    u[::7] = 0.0
+    u[3::7] = 1 - 2.0 ** -24
+    args = [a.to(DEV) for a in (x, t, p, k.int(), u)]
+    out = ops.sample(*args)
+    assert torch.equal(out, ops.sample(*args))        # no order in its sums
+    for b in range(len(rows)):
+        row = x[b].float().clamp(max=torch.finfo(torch.float32).max)
+        if not torch.isfinite(row).any():
+            continue
+        ok, _ = _allowed(row, float(t[b]), float(p[b]), int(k[b]),
+                         float(u[b]))
+        i = int(out[b])
+        assert ok[i], (kinds[b // len(options)], want[b], i, float(u[b]))
+        if t[b] == 0:
+            assert i == int(row.argmax())
+
+
+def test_rows_without_a_choice():
+    x = torch.full((3, 16), float("-inf"), device=DEV)
+    x[2] = torch.arange(16.0)
+    ones = torch.ones(3, device=DEV)
+    out = ops.sample(x, torch.tensor([0.0, 1.0, 1.0], device=DEV),
+                     torch.tensor([1.0, 1.0, 0.0], device=DEV),
+                     torch.zeros(3, dtype=torch.int32, device=DEV), ones / 2)
+    assert out.tolist() == [0, 15, 15]
