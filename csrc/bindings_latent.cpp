@@ -51,6 +51,8 @@ void launch_latent_attn_prefill(bf16*, const bf16*, const bf16*, const bf16*,
                                 long, hipStream_t);
 void launch_experts_route(float*, int*, const float*, int, int, int, bool,
                           bool, int, const float*, hipStream_t);
+void launch_experts_router(float*, int*, const void*, const float*,
+                           const bf16*, long, int, int, int, hipStream_t);
 void launch_experts_sort(int*, int*, int*, const int*, int, int, int, int,
                          hipStream_t);
 void launch_experts_route_sort(float*, int*, int*, int*, int*, const float*,
@@ -483,6 +485,26 @@ void experts_route(Tensor weight, Tensor ids, Tensor logits, long E, long top,
                        opt(correction), stream());
 }
 
+// choices and weights of the rows of x [T, W], bf16 or e4m3 with x_scale [T]
+void experts_router(Tensor weight, Tensor ids, Tensor x, Maybe x_scale,
+                    Tensor router, long top) {
+  check(x, x_scale.has_value() ? torch::kFloat8_e4m3fn : torch::kBFloat16,
+        "x");
+  check(router, torch::kBFloat16, "router");
+  TORCH_CHECK(x.dim() == 2 && router.dim() == 2 &&
+                  router.size(1) == x.size(1) && x.size(1) % 8 == 0,
+              "experts_router: shape");
+  const long T = x.size(0), E = router.size(0);
+  TORCH_CHECK(E >= 1 && E <= 64 && top >= 1 && top <= E && T < (1l << 31),
+              "experts_router: experts");
+  if (x_scale.has_value()) check_param(*x_scale, T, "x_scale");
+  check_param(weight, T * top, "weight");
+  check_ints(ids, T * top, "ids");
+  launch_experts_router(ptr<float>(weight), ids.data_ptr<int>(), x.data_ptr(),
+                        opt(x_scale), ptr<bf16>(router), T, (int)E, (int)top,
+                        (int)x.size(1), stream());
+}
+
 void check_sorted(const Tensor& order, const Tensor& expert,
                   const Tensor& place, long choices, long kinds, long bm) {
   const long tiles = expert.numel();
@@ -636,6 +658,7 @@ void register_latent(pybind11::module_& m) {
   m.def("experts_route", &experts_route, py::arg("weight"), py::arg("ids"),
         py::arg("logits"), py::arg("E"), py::arg("top"),
         py::arg("correction") = py::none(), py::arg("identity") = 0);
+  m.def("experts_router", &experts_router);
   m.def("experts_sort", &experts_sort);
   m.def("experts_route_sort", &experts_route_sort);
   m.def("experts_up", &experts_up);

@@ -130,6 +130,80 @@ __global__ __launch_bounds__(256) void route_kernel(Route r) {
   if (t < r.T) route_row<LE>(r, t);
 }
 
+// Router product and choice of one token a workgroup: logits x . router[e] in
+// float for N <= 64 outputs, then route_token.  x bf16, or e4m3 with a scale a
+// row, which count as their product rounded to bf16.  A token's E * W products
+// are too few for a tile of the matrix cores, and one launch replaces the
+// conversions, the product, the softmax, the selection and the division.
+template <bool FP8>
+__global__ __launch_bounds__(256) void router_kernel(
+    Route r, const void* __restrict__ x, const float* __restrict__ x_scale,
+    const bf16* __restrict__ router, int W) {
+  __shared__ float z[64];
+  const long t = blockIdx.x;
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  // columns (i * 64 + lane) * 8, up to COLS of them in registers at a time
+  constexpr int HELD = 8, COLS = HELD * 512;
+  float sum[16];                     // experts wid + 4 j
+  #pragma unroll
+  for (int j = 0; j < 16; ++j) sum[j] = 0.f;
+  for (int c0 = 0; c0 < W; c0 += COLS) {
+    float xv[HELD][8];
+    #pragma unroll
+    for (int i = 0; i < HELD; ++i) {
+      const int c = c0 + (i * 64 + lane) * 8;
+      #pragma unroll
+      for (int k = 0; k < 8; ++k) xv[i][k] = 0.f;
+      if (c >= W) continue;
+      if constexpr (FP8) {
+        const uint2 u = *reinterpret_cast<const uint2*>(
+            static_cast<const unsigned char*>(x) + t * W + c);
+        const float s = x_scale[t];
+        #pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const auto f = k & 1
+              ? __builtin_amdgcn_cvt_pk_f32_fp8(k < 2 ? u.x : u.y, true)
+              : __builtin_amdgcn_cvt_pk_f32_fp8(k < 2 ? u.x : u.y, false);
+          xv[i][2 * k] = bf2f(f2bf(f[0] * s));
+          xv[i][2 * k + 1] = bf2f(f2bf(f[1] * s));
+        }
+      } else {
+        load_vec<bf16, 8>(static_cast<const bf16*>(x) + t * W + c, xv[i]);
+      }
+    }
+    #pragma unroll
+    for (int j = 0; j < 16; ++j) {
+      const int e = wid + 4 * j;
+      if (e >= r.E) break;
+      #pragma unroll
+      for (int i = 0; i < HELD; ++i) {
+        const int c = c0 + (i * 64 + lane) * 8;
+        if (c >= W) continue;
+        const bf16x8 w = load_bf16x8(router + (long)e * W + c);
+        #pragma unroll
+        for (int k = 0; k < 8; ++k)
+          sum[j] = fmaf(xv[i][k], bf16x8_get(w, k), sum[j]);
+      }
+    }
+  }
+  #pragma unroll
+  for (int j = 0; j < 16; ++j) {
+    const int e = wid + 4 * j;
+    if (e >= r.E) break;
+    const float s = wave_reduce_sum(sum[j]);
+    if (lane == 0) z[e] = s;
+  }
+  __syncthreads();
+  if (wid) return;
+  int id;
+  float w;
+  route_token<1>(r, z, &id, &w);
+  if (lane < r.top) {
+    r.weight[t * r.top + lane] = w;
+    r.ids[t * r.top + lane] = id;
+  }
+}
+
 // One workgroup.  order[pos] = choice (-1: padding), expert[tile] (-1: none),
 // place[choice] = pos (-1: an identity expert).  ROUTE: the choices are made
 // here first.
@@ -446,6 +520,20 @@ void launch_experts_route(float* weight, int* ids, const float* logits, int T,
     route_kernel<LE><<<(unsigned)((T + 3) / 4), 256, 0, stream>>>(r)
   BY_EXPERTS(RUN);
   #undef RUN
+}
+
+// E <= 64, W a multiple of 8; x bf16, or e4m3 where x_scale is given
+void launch_experts_router(float* weight, int* ids, const void* x,
+                           const float* x_scale, const bf16* router, long T,
+                           int E, int top, int W, hipStream_t stream) {
+  if (T == 0) return;
+  const Route r{weight, ids, nullptr, (int)T, E, top, 0, 0, E, nullptr};
+  if (x_scale)
+    router_kernel<true><<<(unsigned)T, 256, 0, stream>>>(r, x, x_scale,
+                                                         router, W);
+  else
+    router_kernel<false><<<(unsigned)T, 256, 0, stream>>>(r, x, nullptr,
+                                                          router, W);
 }
 
 void launch_experts_sort(int* order, int* expert, int* place, const int* ids,

@@ -99,6 +99,10 @@ class MixtralMoE(nn.Module):
             # fp8 path: the fused norm producer already quantized x;
             # dequantize only the router's [T,E] logits input
             xq = x
+            if self._fused_router(xq.data) and get_ep_size() == 1:
+                weights, ids = ops.moe_router(xq, self.router, self.top_k)
+                return ops.moe_ffn_fp8(xq, self.w13, self.w13_scale, self.w2,
+                                       self.w2_scale, weights, ids)
             x = (xq.data.float() * xq.scale[:, None]).to(torch.bfloat16)
         T, H = x.shape
         weights, ids = ops.torch_ref.moe_route(x, self.router, self.top_k) \
@@ -108,20 +112,27 @@ class MixtralMoE(nn.Module):
                                    self.w2_scale, weights.float(),
                                    ids.to(torch.int32))
         if get_ep_size() == 1:
+            if x.is_cuda and ops.have_native():
+                # grouped MFMA kernels, capture-safe
+                return ops.moe_ffn(x, self.w13, self.w2, weights,
+                                   ids.to(torch.int32))
             return self._local_moe(x, weights.to(x.dtype), ids)
-        return self._ep_moe(x, weights.to(x.dtype), ids)
+        return self._ep_moe(x, weights.to(x.dtype), ids.long())
+
+    def _fused_router(self, x: torch.Tensor) -> bool:
+        return x.is_cuda and ops.have_native() and x.is_contiguous() \
+            and self.router.dtype == torch.bfloat16 \
+            and self.num_experts <= 64 and x.shape[1] % 8 == 0
 
     def _route_gpu(self, x: torch.Tensor):
+        if x.dtype == torch.bfloat16 and self._fused_router(x):
+            return ops.moe_router(x, self.router, self.top_k)
         logits = x.float() @ self.router.float().t()
         probs = logits.softmax(-1)
         w, ids = probs.topk(self.top_k, dim=-1)
         return w / w.sum(-1, keepdim=True), ids
 
     def _local_moe(self, x, weights, ids):
-        if x.is_cuda and ops.have_native():
-            # grouped MFMA kernels, capture-safe (csrc/moe.hip)
-            local = (ids - self.local_expert_start).to(torch.int32)
-            return ops.moe_ffn(x, self.w13, self.w2, weights, local)
         out = torch.zeros_like(x)
         flat_ids = ids.reshape(-1)
         flat_w = weights.reshape(-1)

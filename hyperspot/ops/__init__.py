@@ -242,6 +242,52 @@ def _moe_splitk(nblocks: int, nchunks: int, out_numel: int, dev):
     return s, torch.empty(s * out_numel, dtype=torch.float32, device=dev)
 
 
+def moe_router(x, router: torch.Tensor, top: int):
+    """(weights [T, top] float, expert ids [T, top] int32) of the rows of x, a
+    bf16 tensor or a QTensor: the softmax over the chosen.  GPU."""
+    data, scale = x if isinstance(x, QTensor) else (x, None)
+    T = data.shape[0]
+    weight = torch.empty(T, top, dtype=torch.float32, device=data.device)
+    ids = torch.empty(T, top, dtype=torch.int32, device=data.device)
+    _native().experts_router(weight, ids, data, scale, router, top)
+    return weight, ids
+
+
+# Rows per expert up to which tiles of 16 to 64 rows beside the streamed weights
+# are faster than the 256-row tiles, in us on an MI355X:
+#   experts of 14336 x 4096  1 row 274 : 463, 48 rows 788 : 831, 64 1049 : 846
+#   32 of 1024 x 2048        1 row  54 : 157, 64 rows 180 : 277, 128 269 : 305
+#   16 of 2048 x 4096        1 row 132 : 273, 64 rows 335 : 378,  96 397 : 391
+# The large tiles are late where they leave compute units without one.
+MOE_ROWS = 48
+MOE_ROWS_FEW = 95
+
+
+def _moe_rows(T: int, K: int, E: int, H: int, I: int) -> bool:
+    most = MOE_ROWS_FEW if E * (2 * I // 128) < 1024 else MOE_ROWS
+    return T * K <= most * E and H % 128 == 0 and I % 128 == 0 and E <= 64
+
+
+def _moe_ffn_rows(x, w13, w2, weights, ids):
+    n = _native()
+    (T, H), K, (E, _, I) = x.shape, ids.shape[1], w2.shape
+    pairs, mean = T * K, T * K / E
+    bm = 16 if mean <= 8 else 32 if mean <= 16 else 64
+    tiles = min(pairs, (pairs + E * (bm - 1)) // bm)
+    i32 = lambda m: torch.empty(m, dtype=torch.int32, device=x.device)
+    order, expert, place = i32(tiles * bm), i32(tiles), i32(pairs)
+    n.experts_sort(order, expert, place, ids.reshape(-1).to(torch.int32), E,
+                   bm)
+    h = torch.empty(tiles * bm, I, dtype=x.dtype, device=x.device)
+    y = torch.empty(tiles * bm, H, dtype=x.dtype, device=x.device)
+    n.experts_up(h, x, w13, None, order, expert, K, None, bm)
+    n.experts_down(y, h, w2, None, order, expert, bm)
+    out = torch.empty(T, H, dtype=x.dtype, device=x.device)
+    n.experts_sum(out, y, place.view(T, K), weights.float().contiguous(),
+                  None, None, None, None, 0.0)
+    return out
+
+
 def moe_ffn(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor,
             weights: torch.Tensor, ids: torch.Tensor) -> torch.Tensor:
     """Grouped expert SwiGLU FFN (GPU, hipGraph-capture-safe).
@@ -256,6 +302,8 @@ def moe_ffn(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor,
     K = ids.shape[1]
     E = w13.shape[0]
     TK = T * K
+    if x.is_contiguous() and _moe_rows(T, K, E, H, w2.shape[2]):
+        return _moe_ffn_rows(x, w13, w2, weights, ids)
     ntiles = (TK + E * (MOE_BM - 1) + MOE_BM - 1) // MOE_BM
     P = ntiles * MOE_BM
     dev = x.device

@@ -1,0 +1,64 @@
+"""Router kernel and grouped experts at both sides of the rule that chooses
+between row tiles and 256-row tiles, against float64.
+
+Bounds: the router's products are exact in float and summed in float (2^-22 of
+the sum of magnitudes); experts round their inner activation and their output
+to bf16 (2^-9 each)."""
+
+import pytest
+import torch
+
+import hyperspot.engine  # noqa: F401  (before the models, which it imports)
+import hyperspot.ops as ops
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("tokens,experts,top,width", [
+    (1, 8, 2, 4096), (3, 64, 6, 2048), (65, 5, 5, 264), (2, 1, 1, 8),
+    (7, 32, 4, 8200)])
+def test_router(tokens, experts, top, width, fp8):
+    g = torch.Generator().manual_seed(width)
+    x = torch.randn(tokens, width, generator=g).bfloat16().to(DEV)
+    router = torch.randn(experts, width, generator=g).bfloat16().to(DEV)
+    arg = x
+    if fp8:
+        arg = ops.quant_fp8(x)
+        x = (arg.data.float() * arg.scale[:, None]).bfloat16()
+    weight, ids = ops.moe_router(arg, router, top)
+    z = x.double() @ router.double().t()
+    slack = 2.0 ** -22 * (x.double().abs() @ router.double().abs().t()).max()
+    best = z.topk(top, -1)
+    got = z.gather(1, ids.long())
+    assert (got - best.values).abs().max() <= 2 * slack
+    assert all(len(set(r)) == top for r in ids.tolist())
+    ref = got.softmax(-1)
+    assert (weight.double() - ref).abs().max() <= 4 * slack + 1e-6
+
+
+@pytest.mark.parametrize("tokens", [1, 2, 33, 95, 96, 97, 191, 192, 193, 400])
+@pytest.mark.parametrize("experts,top,width,inner", [
+    (4, 2, 256, 128), (8, 1, 128, 384), (2, 2, 384, 32768)])
+def test_experts_around_the_rule(tokens, experts, top, width, inner):
+    g = torch.Generator().manual_seed(tokens)
+    rand = lambda *s: torch.randn(*s, generator=g)
+    x = rand(tokens, width).bfloat16().to(DEV)
+    w13 = (rand(experts, 2 * inner, width) * width ** -0.5).bfloat16().to(DEV)
+    w2 = (rand(experts, width, inner) * inner ** -0.5).bfloat16().to(DEV)
+    # one expert may have no row, another most of them
+    score = rand(tokens, experts)
+    score[:, 0] += 1
+    score[:, -1] -= 2
+    ids = score.topk(top, -1).indices.int().to(DEV)
+    weight = rand(tokens, top).abs().to(DEV)
+    out = ops.moe_ffn(x, w13, w2, weight, ids).double()
+    ref = torch.zeros_like(out)
+    for e in range(experts):
+        gate, up = (x.double() @ w13[e].double().t()).chunk(2, -1)
+        y = torch.nn.functional.silu(gate) * up @ w2[e].double().t()
+        ref += y * (weight * (ids == e)).sum(-1)[:, None].double()
+    assert (out - ref).norm() <= 2.0 ** -7 * ref.norm()
+    assert (out - ref).abs().max() <= 2.0 ** -5 * ref.abs().max()
