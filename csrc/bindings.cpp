@@ -90,6 +90,9 @@ void launch_recurrent_step(Kind, T*, float*, float*, float*, float*,
                            const float*, const long*, const int*, long, int,
                            int, int, int, long, float, float, float,
                            hipStream_t);
+bool gemm_rows_fits(long, long);
+void launch_gemm_rows(bf16*, const bf16*, const bf16*, int, int, int, long,
+                      long, long, hipStream_t);
 void launch_silu_mul(bf16*, const bf16*, long, int, hipStream_t);
 void launch_quant_fp8(unsigned char*, float*, const bf16*, long, int, long,
                       hipStream_t);
@@ -275,6 +278,26 @@ void attn_portions(torch::Tensor out, torch::Tensor q, torch::Tensor k_cache,
       block_tables.data_ptr<int>(), ctx_lens.data_ptr<int>(),
       seq_start.data_ptr<int>(), (int)seqs, T, H, KV, max_blocks,
       (int)min_rows, (float)scale, q.stride(0), fp8, stream());
+}
+
+// out = x w^T
+void gemm_rows(torch::Tensor out, torch::Tensor x, torch::Tensor w) {
+  for (const auto& t : {out, x, w})
+    TORCH_CHECK(t.is_cuda() && t.scalar_type() == torch::kBFloat16 &&
+                    t.dim() == 2 && t.stride(1) == 1, "gemm_rows: matrices");
+  const long M = x.size(0), K = x.size(1), N = w.size(0);
+  TORCH_CHECK(w.size(1) == K && out.size(0) == M && out.size(1) == N,
+              "gemm_rows: shape");
+  auto aligned = [](const torch::Tensor& t, long n) {
+    return reinterpret_cast<uintptr_t>(t.data_ptr()) % (2 * n) == 0 &&
+           t.stride(0) % n == 0;
+  };
+  TORCH_CHECK(gemm_rows_fits(M, K) && N % 4 == 0 && K % 8 == 0 &&
+                  N < (1l << 31) && aligned(x, 8) && aligned(w, 8) &&
+                  aligned(out, 4), "gemm_rows: sizes");
+  if (N == 0) return;
+  launch_gemm_rows(bf(out), cbf(x), cbf(w), (int)M, (int)N, (int)K,
+                   x.stride(0), w.stride(0), out.stride(0), stream());
 }
 
 void silu_mul(torch::Tensor out, torch::Tensor x) {
@@ -1039,6 +1062,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("paged_attn", &paged_attn);
   m.def("attn_prefill_mfma", &attn_prefill_mfma);
   m.def("attn_portions", &attn_portions);
+  m.def("gemm_rows", &gemm_rows);
+  m.def("gemm_rows_fits", &gemm_rows_fits);
   m.def("silu_mul", &silu_mul);
   m.def("gelu_mul", &gelu_mul);
   m.def("embed_dyt", &embed_dyt);

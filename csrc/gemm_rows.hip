@@ -1,0 +1,176 @@
+// out[M, N] = x[M, K] w[N, K]^T for few rows (gfx950), bf16 in and out, float
+// sums.
+//
+// What bounds it: reading w once.  So w is the A operand of 16x16x32 products
+// straight from memory.  The rows of x, which every tile of w needs whole, go
+// into LDS once a workgroup, and the workgroups stay: one or two a CU, each
+// with every gridDim-th tile of 16 rows of w.  (x from L2 beside every tile of
+// w costs as many load instructions as w itself for each 16 rows: 28672 x 4096
+// took 50 us for one row and 72 us for 16.)  The 8 waves divide K, so that
+// also a single tile has 8 KB of loads in flight a wave, and add up in LDS;
+// the next tile's loads are issued before that.
+//
+// us, library and here, weights from memory (which gives about 5 TB/s):
+//   28672 x 4096  1 row 60 46, 16 rows 61 48    4096 x 4096   1 16 10, 16 16 11
+//   32768 x 4096  1 row 64 52, 16 rows 63 55    2048 x 2048   1 11  5, 32 11  7
+//   32768 x 2048  1 row 35 29, 32 rows 36 34    3072 x 2048   1 11  6, 32 12  8
+#include "common.h"
+
+namespace {
+
+constexpr int WAVES = 8;
+constexpr int STEP = WAVES * 64;     // columns of a step of all waves
+constexpr int U = 4;                 // steps a batch
+
+struct Rows {
+  bf16* out;
+  const bf16* x;
+  const bf16* w;
+  int M, N, K;
+  long xs, ws, os;                   // row strides
+};
+
+// 16 bytes a lane, to the wave's LDS address + lane * 16
+DEV void to_lds16(const void* g, void* l) {
+  __builtin_amdgcn_global_load_lds(
+      (const __attribute__((address_space(1))) unsigned*)g,
+      (__attribute__((address_space(3))) unsigned*)l, 16, 0, 0);
+}
+
+// CT * 16 rows of x
+template <int CT>
+__global__ __launch_bounds__(WAVES * 64, 2)
+void gemm_rows_kernel(Rows a) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  float* red = reinterpret_cast<float*>(smem);
+  short* xl = reinterpret_cast<short*>(smem + WAVES * CT * 1024);
+  const int xp = a.K + 8;            // row of x in LDS: 16 rows, 16 banks
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  const int col = lane & 15, gr = lane >> 4;
+  const int tiles = (a.N + 15) / 16;
+  const int batches = (a.K + U * STEP - 1) / (U * STEP);
+
+  short8_t wf[U][2], wn[U][2];
+  auto fetch = [&](int tile, int batch) {
+    const int n = min(tile * 16 + col, a.N - 1);
+    const bf16* p = a.w + (long)n * a.ws + gr * 8;
+    const int k0 = batch * U * STEP + wid * 64;
+    #pragma unroll
+    for (int u = 0; u < U; ++u)
+      #pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        const int k = k0 + u * STEP + 32 * s;
+        wn[u][s] = k + gr * 8 < a.K
+            ? __builtin_nontemporal_load(
+                  reinterpret_cast<const short8_t*>(p + k))
+            : short8_t{};
+      }
+  };
+  int tile = blockIdx.x, batch = 0;
+  fetch(tile, 0);
+  if (a.K % 512 == 0) {              // a KB of a row a wave, straight to LDS
+    const int parts = a.K / 512, n = a.M * parts;
+    for (int i = __builtin_amdgcn_readfirstlane(wid); i < n; i += WAVES) {
+      const int m = i / parts, c = (i - m * parts) * 512;
+      to_lds16(a.x + m * a.xs + c + lane * 8, xl + m * xp + c);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  } else {
+    for (int m = 0; m < a.M; ++m)
+      for (int c = threadIdx.x * 8; c < a.K; c += WAVES * 64 * 8)
+        *reinterpret_cast<short8_t*>(xl + m * xp + c) =
+            *reinterpret_cast<const short8_t*>(a.x + m * a.xs + c);
+  }
+  const short* xr[CT];
+  #pragma unroll
+  for (int t = 0; t < CT; ++t)       // rows past the end: not stored
+    xr[t] = xl + min(t * 16 + col, a.M - 1) * xp + gr * 8;
+  f32x4_t acc[CT];
+  #pragma unroll
+  for (int t = 0; t < CT; ++t) acc[t] = f32x4_t(0.f);
+  __syncthreads();
+
+  while (tile < tiles) {
+    #pragma unroll
+    for (int u = 0; u < U; ++u)
+      #pragma unroll
+      for (int s = 0; s < 2; ++s) wf[u][s] = wn[u][s];
+    const int k0 = batch * U * STEP + wid * 64, now = tile;
+    if (++batch == batches) {
+      batch = 0;
+      tile += gridDim.x;
+    }
+    if (tile < tiles) fetch(tile, batch);
+    #pragma unroll
+    for (int u = 0; u < U; ++u)
+      #pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        // columns past the end: w is zero, and x is that of the last ones
+        const int k = min(k0 + u * STEP + 32 * s, a.K - 8 - gr * 8);
+        #pragma unroll
+        for (int t = 0; t < CT; ++t)
+          acc[t] = mfma16(wf[u][s], *reinterpret_cast<const short8_t*>(
+                                        xr[t] + k), acc[t]);
+      }
+    if (batch) continue;
+    #pragma unroll
+    for (int t = 0; t < CT; ++t) {
+      *reinterpret_cast<f32x4_t*>(red + ((wid * CT + t) * 64 + lane) * 4) =
+          acc[t];
+      acc[t] = f32x4_t(0.f);
+    }
+    __syncthreads();
+    if (wid < CT) {
+      f32x4_t y = f32x4_t(0.f);
+      #pragma unroll
+      for (int v = 0; v < WAVES; ++v)
+        y += *reinterpret_cast<const f32x4_t*>(
+            red + ((v * CT + wid) * 64 + lane) * 4);
+      const int n = now * 16 + gr * 4, m = wid * 16 + col;
+      if (m < a.M && n < a.N)          // N is a multiple of 4
+        *reinterpret_cast<uint2*>(a.out + m * a.os + n) =
+            uint2{cvt_pk_bf16(y[0], y[1]), cvt_pk_bf16(y[2], y[3])};
+    }
+    __syncthreads();
+  }
+}
+
+constexpr int LDS = 160 * 1024;
+
+// 16-row tiles of x a workgroup has
+int row_tiles(int M) { return M <= 16 ? 1 : M <= 32 ? 2 : 4; }
+
+int lds_bytes(int M, int K) {
+  return WAVES * row_tiles(M) * 1024 + M * (K + 8) * 2;
+}
+
+}  // namespace
+
+// whether M rows of K columns are taken
+bool gemm_rows_fits(long M, long K) {
+  return M >= 1 && M <= 64 && K >= 8 && K <= 65536 &&
+         lds_bytes((int)M, (int)K) <= LDS;
+}
+
+// N a multiple of 4, K of 8; rows of x and w 16-byte, of out 8-byte aligned
+void launch_gemm_rows(bf16* out, const bf16* x, const bf16* w, int M, int N,
+                      int K, long xs, long ws, long os, hipStream_t stream) {
+  const Rows a{out, x, w, M, N, K, xs, ws, os};
+  const int lds = lds_bytes(M, K), tiles = (N + 15) / 16;
+  const int most = lds * 2 <= LDS ? 512 : 256;     // that a CU holds at once
+  const unsigned grid = (unsigned)(tiles < most ? tiles : most);
+  #define RUN(CT)                                                           \
+    {                                                                       \
+      static const hipError_t set = hipFuncSetAttribute(                    \
+          reinterpret_cast<const void*>(&gemm_rows_kernel<CT>),             \
+          hipFuncAttributeMaxDynamicSharedMemorySize, LDS);                 \
+      HIP_CHECK(set);                                                       \
+      gemm_rows_kernel<CT><<<grid, WAVES * 64, lds, stream>>>(a);           \
+    }
+  switch (row_tiles(M)) {
+    case 1: RUN(1) break;
+    case 2: RUN(2) break;
+    default: RUN(4)
+  }
+  #undef RUN
+}

@@ -225,4 +225,4 @@ class LlamaForCausalLM(nn.Module):
             return x
         if meta.logits_indices is not None:
             x = x[meta.logits_indices]
-        return x @ self.lm_head.t()
+        return ops.linear(x, self.lm_head)

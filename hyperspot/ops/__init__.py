@@ -171,6 +171,34 @@ def silu_mul(gate_up: torch.Tensor) -> torch.Tensor:
     return torch_ref.silu_mul(gate_up)
 
 
+def _rows_gemm(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether csrc/gemm_rows.hip takes x w^T: few rows, and a weight whose
+    tiles of 16 rows divide evenly over the 256 compute units; the library is
+    as fast or faster elsewhere (us, library and kernel, one row: 6144 x 4096
+    14.4 14.8, 4096 x 14336 26.9 28.0, 2048 x 7168 13.2 13.2)."""
+    if not (x.is_cuda and x.dtype == w.dtype == torch.bfloat16
+            and x.dim() == 2 and w.dim() == 2 and 1 <= x.shape[0] <= 64):
+        return False
+    (M, K), N = x.shape, w.shape[0]
+    tiles = (N + 15) // 16
+    if K > 4096 or K % 8 or N % 4 or N * K < (1 << 20) \
+            or -(-tiles // 256) * 256 > 1.2 * tiles and tiles > 256:
+        return False
+    return _native().gemm_rows_fits(M, K) and all(
+        t.stride(1) == 1 and t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0
+        for t in (x, w))
+
+
+def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """x w^T for w [N, K]."""
+    if _rows_gemm(x, w):
+        out = torch.empty(x.shape[0], w.shape[0], dtype=x.dtype,
+                          device=x.device)
+        _native().gemm_rows(out, x, w)
+        return out
+    return x @ w.t()
+
+
 class QTensor(NamedTuple):
     """Per-token-scaled fp8 activation: data e4m3fn [T,K], scale fp32 [T].
 

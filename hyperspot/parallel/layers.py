@@ -114,7 +114,7 @@ class _LinearCompute(nn.Module):
             # CPU test path: identical numerics model, emulated in fp32
             wf = self.weight.float() * self.weight_scale[:, None]
             return ((xq.float() * xs[:, None]) @ wf.t()).to(x.dtype)
-        return x @ self.weight.t()
+        return _O.linear(x, self.weight)
 
 
 def _init_weight(out_f: int, in_f: int, dtype: torch.dtype, seed_tag: int):

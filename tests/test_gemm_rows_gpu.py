@@ -1,0 +1,51 @@
+"""Products of few rows against float64 at the edges of tiles, batches and
+what fits.
+
+Bound: products of bf16 are exact in float; a sum of K of them is off by at
+most K 2^-24 of the sum of magnitudes, and the result is rounded to bf16."""
+
+import pytest
+import torch
+
+import hyperspot.engine  # noqa: F401  (before the models, which it imports)
+import hyperspot.ops as ops
+from hyperspot import _C
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+
+
+@pytest.mark.parametrize("rows", [1, 3, 16, 17, 32, 33, 64])
+@pytest.mark.parametrize("n,k", [(16, 512), (20, 8), (260, 520), (4100, 1024),
+                                 (8212, 264), (48, 4104), (36, 14336)])
+def test_products_of_few_rows(rows, n, k):
+    if not _C.gemm_rows_fits(rows, k):
+        with pytest.raises(RuntimeError):
+            _C.gemm_rows(torch.empty(rows, n, device=DEV).bfloat16(),
+                         torch.empty(rows, k, device=DEV).bfloat16(),
+                         torch.empty(n, k, device=DEV).bfloat16())
+        return
+    g = torch.Generator().manual_seed(rows * n)
+    # rows of wider buffers
+    x = torch.randn(rows, k + 8, generator=g).bfloat16().to(DEV)[:, :k]
+    w = torch.randn(n, k + 16, generator=g).bfloat16() \
+        .to(DEV)[:, 8:k + 8]
+    out = torch.full((rows + 1, n + 4), 7.0, device=DEV).bfloat16()
+    _C.gemm_rows(out[:rows, :n], x, w)
+    assert (out[rows] == 7).all() and (out[:, n:] == 7).all()
+    ref = x.double() @ w.double().t()
+    slack = x.double().abs() @ w.double().abs().t() * k * 2.0 ** -24
+    err = (out[:rows, :n].double() - ref).abs()
+    assert (err <= slack + ref.abs() * 2.0 ** -8).all()
+
+
+@pytest.mark.parametrize("rows", [0, 1, 64, 65])
+def test_linear_takes_any_rows(rows):
+    g = torch.Generator().manual_seed(5)
+    x = torch.randn(rows, 1024, generator=g).bfloat16().to(DEV)
+    w = torch.randn(2048, 1024, generator=g).bfloat16().to(DEV)
+    ref = x.double() @ w.double().t()
+    out = ops.linear(x, w).double()
+    assert out.shape == ref.shape
+    assert rows == 0 or (out - ref).norm() <= 2.0 ** -8 * ref.norm()
