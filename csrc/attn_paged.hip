@@ -1,8 +1,8 @@
 // Unified paged attention for gfx950 — serves the decode step (one query
-// token per sequence) and short/odd-shape prefill fallback (the MFMA flash
-// kernel covers head_dim-128 prefill).
+// token per sequence), the rows of short portions, and prefill of other head
+// sizes than 128 (attn_prefill_mfma.hip has that).
 //
-// Geometry (memory-bound design, wave64-native):
+// Geometry of the general kernel (head_dim 64; wave64-native):
 //   grid = (num_query_rows, num_kv_heads); block = 256 threads = 4 waves.
 //   A workgroup owns one (row, kv_head): it processes the whole GQA group
 //   (GROUP query heads) so K/V stream from HBM exactly once per group.
@@ -218,312 +218,309 @@ __global__ __launch_bounds__(256) void paged_attn_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// v3 (D=128, GROUP<=4): latency-oriented redesign.  v2's q-in-register
-// layout (4 lanes/token, 32-elem q slice) cost 244 VGPRs -> occupancy 2
-// waves/SIMD, and its V read was 16x 4-byte loads/page; with two dependent
-// HBM round trips per page the kernel ran 5x off the KV-stream roofline
-// (334us/layer at bs=256 ctx=512, profiles/r01).  v3:
-//   - K phase: 8 lanes/token (16-elem slice) -> q_pk is GROUP*8 dwords
-//     (32 VGPRs at GROUP=4); dot via v_dot2_f32_bf16 (guide: packed bf16
-//     dot at f32 accumulate, 6x fewer VALU ops than scalar cvt+fma).
-//   - V phase: lane owns an 8-elem dim slice (lane&15) of 4 consecutive
-//     tokens (lane>>4) -> 4x dwordx4 loads/page; PV accumulates in f32
-//     FMAs, P stays f32 (no bf16 round).
-//   - All K+V loads for the page are issued together at the top of the
-//     loop so one HBM round trip covers both phases.
-//   - Softmax is shuffle-only (score all-reduce over slice lanes, max and
-//     denominator over token lanes); LDS is used once per page to move
-//     P from K-lane-layout to V-lane-layout (wave-private, DS ops of one
-//     wave are in program order).
+// head_dim 128: matrix cores (v_mfma_f32_16x16x32_bf16).
+//
+// What bounds it: reading the pages once, about 5 TB/s.  A dot product of four
+// heads with a token on the vector units takes longer than the token's 512
+// bytes; so up to 16 heads of a kv head are the columns of a product, however
+// few they are.  Scores are formed transposed, S^T = K Q^T, with the K row
+// that feeds matrix row i permuted so that the scores a lane holds are 8
+// consecutive tokens of one head, the operand P^T of O^T = V^T P^T; the
+// weights enter as a bf16 high and low part.  K goes from memory to its
+// operands; V is turned by an LDS tile of the wave's own and the transposing
+// LDS load, e4m3 pages are widened on the way.  A wave has 32 tokens at a time
+// and issues the next ones' loads as soon as these are in their operands; no
+// barrier until the waves' parts are added up.
+//
+// us against dot products on the vector units, ragged contexts around the
+// mean: 256 rows x 8 kv heads of 4, 1000 tokens 239 -> 208 (5.0 TB/s), with
+// e4m3 pages 214 -> 110; 64 rows 77 -> 59, e4m3 71 -> 32; 8 rows of 8000 in 4
+// parts 122 -> 61; 64 rows x 1 kv head of 8 in 4 parts 47 -> 16.
+//
+// SPLIT > 1 (flash-decode): gridDim.z workgroups share one (row, kvh), each
+// with every gridDim.z-th 4 blocks of 32 tokens; their (o, m, l) land in
+// `partial` [rows, kvh, split, group, D + 2] and a second kernel merges them.
 // ---------------------------------------------------------------------------
+namespace {
 
-DEV float dot2_bf16(unsigned a, unsigned b, float c) {
-  asm("v_dot2_f32_bf16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b));
-  return c;
+constexpr int HD = 128;
+constexpr int BLOCK = 32;            // tokens a wave has at a time
+constexpr float LOG2E = 1.4426950408889634f;
+constexpr float GROW = 8.f;          // rescale when a maximum grows by 2^GROW
+
+typedef __attribute__((ext_vector_type(4))) short short4_t;
+typedef __attribute__((ext_vector_type(4))) unsigned u32x4;
+typedef __attribute__((ext_vector_type(2))) float float2_t;
+
+DEV float exp2_fast(float x) { return __builtin_amdgcn_exp2f(x); }
+
+// four rows of one column: in every 16 lanes, lane i passes the address of
+// row i / 4, columns 4 (i % 4), and receives column i
+DEV short4_t lds_read_tr(const char* p) {
+  return __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+      (__attribute__((address_space(3))) short4_t*)p);
 }
 
-// fp8-KV support: unpack 4 e4m3fn bytes -> 2 packed-bf16 dwords (for the
-// dot2 K path) or 2 float2 (for the PV path).  gfx950-native converts.
-typedef __attribute__((ext_vector_type(2))) float float2v;
+// byte of 16-byte unit c of row r of a V tile: what 32 lanes read at a time,
+// 64 bytes of rows r .. r + 3 and r + 8 .. r + 11, has a bank each
+DEV int v_byte(int r, int c) {
+  return r * 256 + ((c ^ (r & 3) << 2 ^ (r >> 3 & 1) << 1) << 4);
+}
 
-// SPLIT > 1 (flash-decode): grid.z WGs share one (row, kvh), each owning
-// pages [4*z+wid :: 4*SPLIT]; per-WG partials (m, l, o) land in `partial`
-// [rows, kvh, SPLIT, GROUP, D+2] fp32 and a second kernel merges them.
-// Used when rows*kvh alone cannot fill the 256 CUs (small batch, or the
-// kvh=1 GQA shard of Llama-70B at TP=8).
-template <int GROUP, bool KV8>
-__global__ __launch_bounds__(256) void paged_attn_v3_kernel(
-    bf16* __restrict__ out, const bf16* __restrict__ q,
-    const bf16* __restrict__ k_cache, const bf16* __restrict__ v_cache,
-    const int* __restrict__ block_tables, const int* __restrict__ ctx_lens,
-    const int* __restrict__ row_seq, int max_blocks, int num_kv_heads,
-    float scale, long q_stride, int h_total, int g_stride, int h_off,
-    float* __restrict__ partial, const int* __restrict__ seq_start,
-    int max_portion) {
-  constexpr int D = 128;
-  const int row = blockIdx.x;
-  const int kvh = blockIdx.y;
-  const int split = gridDim.z;
-  const int H = h_total;
-  const int ctx = ctx_lens[row];
-  const int table = row_seq ? row_seq[row] : row;
-  if (seq_start && seq_start[table + 1] - seq_start[table] > max_portion)
+// 4 e4m3 bytes as bf16, exactly
+DEV uint2 widen(unsigned x) {
+  const float2_t a = __builtin_amdgcn_cvt_pk_f32_fp8(x, false);
+  const float2_t b = __builtin_amdgcn_cvt_pk_f32_fp8(x, true);
+  return uint2{cvt_pk_bf16(a.x, a.y), cvt_pk_bf16(b.x, b.y)};
+}
+DEV u32x4 widen(unsigned x, unsigned y) {
+  const uint2 a = widen(x), b = widen(y);
+  return u32x4{a.x, a.y, b.x, b.y};
+}
+
+struct Paged {
+  bf16* out;
+  const bf16* q;
+  const void* k_cache;
+  const void* v_cache;
+  const int* block_tables;
+  const int* ctx_lens;
+  const int* row_seq;
+  const int* seq_start;      // with row_seq: only sequences of at most
+  int max_portion;           // max_portion rows
+  int max_blocks, G, group;
+  float scale;               // times log2(e)
+  long qs;
+  float* partial;
+};
+
+template <bool KV8>
+__global__ __launch_bounds__(256, 3) void paged_attn_mfma_kernel(Paged a) {
+  __shared__ __attribute__((aligned(16))) char v_lds[4][BLOCK * HD * 2];
+  __shared__ float m_lds[4][16], l_lds[4][16];
+  const int row = blockIdx.x, g = blockIdx.y;
+  const int split = gridDim.z, z = blockIdx.z, group = a.group;
+  const int table = a.row_seq ? a.row_seq[row] : row;
+  if (a.seq_start &&
+      a.seq_start[table + 1] - a.seq_start[table] > a.max_portion)
     return;
-  const int* bt = block_tables + (long)table * max_blocks;
-  const int nblocks = (ctx + ATTN_BS - 1) / ATTN_BS;
-
-  __shared__ __attribute__((aligned(16))) float sc[4][GROUP][ATTN_BS];
-  __shared__ __attribute__((aligned(16))) float comb_o[4][GROUP][D];
-  __shared__ float comb_m[4][GROUP];
-  __shared__ float comb_l[4][GROUP];
-
-  const int wid = threadIdx.x >> 6;
+  const int ctx = a.ctx_lens[row];
+  const int* bt = a.block_tables + (long)table * a.max_blocks;
   const int lane = threadIdx.x & 63;
-  // K-phase role: token t_loc = lane>>3 (8 per pass, 2 passes/page),
-  // slice sl = lane&7 -> elems [sl*16, sl*16+16).
-  const int t_loc = lane >> 3;
-  const int sl = lane & 7;
-  // V-phase role: dim slice ds = lane&15 -> elems [ds*8, ds*8+8),
-  // token group g = lane>>4 -> tokens [4g, 4g+4).
-  const int ds = lane & 15;
-  const int g = lane >> 4;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int col = lane & 15, gr = lane >> 4;
 
-  // ---- query group: raw packed-bf16 slice, GROUP*8 dwords ----
-  unsigned q_pk[GROUP][8];
-  {
-    const bf16* qp = q + (long)row * q_stride
-                     + ((long)kvh * g_stride + h_off) * D + sl * 16;
-    #pragma unroll
-    for (int h = 0; h < GROUP; ++h) {
-      uint4 a = *reinterpret_cast<const uint4*>(qp + h * D);
-      uint4 b = *reinterpret_cast<const uint4*>(qp + h * D + 8);
-      q_pk[h][0] = a.x; q_pk[h][1] = a.y; q_pk[h][2] = a.z; q_pk[h][3] = a.w;
-      q_pk[h][4] = b.x; q_pk[h][5] = b.y; q_pk[h][6] = b.z; q_pk[h][7] = b.w;
-    }
-  }
-
-  float m[GROUP], l[GROUP];
-  float2 acc[GROUP][4];
+  // step c of the score product has columns 32 c + 8 gr; with e4m3, of which
+  // a lane reads 16 at a time, 64 (c / 2) + 16 gr + 8 (c % 2)
+  short8_t qf[4];
   #pragma unroll
-  for (int h = 0; h < GROUP; ++h) {
-    m[h] = -FLT_MAX; l[h] = 0.f;
-    #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[h][j] = make_float2(0.f, 0.f);
+  for (int c = 0; c < 4; ++c) {
+    const int d = KV8 ? (c >> 1) * 64 + gr * 16 + (c & 1) * 8
+                      : c * 32 + gr * 8;
+    qf[c] = col < group
+        ? *reinterpret_cast<const short8_t*>(
+              a.q + row * a.qs + (long)(g * group + col) * HD + d)
+        : short8_t{};
   }
+  f32x4_t acc[8];
+  #pragma unroll
+  for (int e = 0; e < 8; ++e) acc[e] = f32x4_t(0.f);
+  float m = -FLT_MAX, l = 0.f;
 
-  for (int b = 4 * blockIdx.z + wid; b < nblocks; b += 4 * split) {
-    const long blk = bt[b];
-    const int nb = min(ATTN_BS, ctx - b * ATTN_BS);
-    const long page_off = ((blk * num_kv_heads + kvh) * ATTN_BS) * D;
-    const bf16* pbase = k_cache + page_off;
-    const bf16* vbase = v_cache + page_off;
-    const unsigned char* pbase8 =
-        reinterpret_cast<const unsigned char*>(k_cache) + page_off;
-    const unsigned char* vbase8 =
-        reinterpret_cast<const unsigned char*>(v_cache) + page_off;
-    // ---- issue every load for this page up front (one round trip) ----
-    uint4 kr[2][KV8 ? 1 : 2];
-    uint4 vr4[KV8 ? 1 : 4];
-    uint2 vr2[KV8 ? 4 : 1];
+  // matrix row i of half t takes token 8 (i / 4) + 4 t + i % 4
+  const int tok0 = 8 * (col >> 2) + (col & 3);
+  const int blocks = (ctx + BLOCK - 1) / BLOCK;
+  const int last_page = (ctx - 1) / ATTN_BS;
+  const int step = 4 * split;
+  long b0 = 0, b1 = 0;               // page ids, read one block ahead
+  auto pages = [&](int i) {
+    b0 = bt[min(2 * i, last_page)];
+    b1 = bt[min(2 * i + 1, last_page)];
+  };
+  constexpr int ELEM = KV8 ? 1 : 2;
+  u32x4 kr[2][KV8 ? 2 : 4], vr[KV8 ? 4 : 8];
+  auto fetch = [&]() {
+    const long p0 = (b0 * a.G + g) * (ATTN_BS * HD * ELEM);
+    const long p1 = (b1 * a.G + g) * (ATTN_BS * HD * ELEM);
+    const char* kc = static_cast<const char*>(a.k_cache);
+    const char* vc = static_cast<const char*>(a.v_cache);
     #pragma unroll
-    for (int p = 0; p < 2; ++p) {
-      if constexpr (KV8) {
-        kr[p][0] = *reinterpret_cast<const uint4*>(
-            pbase8 + (p * 8 + t_loc) * D + sl * 16);
-      } else {
-        const bf16* kp = pbase + (p * 8 + t_loc) * D + sl * 16;
-        kr[p][0] = *reinterpret_cast<const uint4*>(kp);
-        kr[p][1] = *reinterpret_cast<const uint4*>(kp + 8);
-      }
-    }
-    #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      if constexpr (KV8)
-        vr2[i] = *reinterpret_cast<const uint2*>(vbase8 + (4 * g + i) * D
-                                                 + ds * 8);
-      else
-        vr4[i] = *reinterpret_cast<const uint4*>(vbase + (4 * g + i) * D
-                                                 + ds * 8);
-    }
-    // ---- scores: dot2 over the lane's 16-elem slice, then all-reduce
-    // over the 8 slice lanes (bits 0..2) ----
-    float s[GROUP][2];
-    #pragma unroll
-    for (int p = 0; p < 2; ++p) {
-      unsigned kw[8];
-      if constexpr (KV8) {
-        const unsigned* kq = reinterpret_cast<const unsigned*>(&kr[p][0]);
-        #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          float2v lo = __builtin_amdgcn_cvt_pk_f32_fp8(kq[i], false);
-          float2v hi = __builtin_amdgcn_cvt_pk_f32_fp8(kq[i], true);
-          kw[2 * i] = cvt_pk_bf16(lo.x, lo.y);
-          kw[2 * i + 1] = cvt_pk_bf16(hi.x, hi.y);
-        }
-      } else {
-        #pragma unroll
-        for (int j = 0; j < 8; ++j)
-          kw[j] = reinterpret_cast<const unsigned*>(&kr[p][0])[j];
-      }
+    for (int t = 0; t < 2; ++t) {
+      const int tok = tok0 + 4 * t;
+      const char* kp = kc + (tok < ATTN_BS ? p0 : p1) +
+                       (tok % ATTN_BS) * (HD * ELEM) + gr * 16;
       #pragma unroll
-      for (int h = 0; h < GROUP; ++h) {
-        float d = 0.f;
-        #pragma unroll
-        for (int j = 0; j < 8; ++j) d = dot2_bf16(q_pk[h][j], kw[j], d);
-        d += __shfl_xor(d, 1);
-        d += __shfl_xor(d, 2);
-        d += __shfl_xor(d, 4);
-        const int tok = p * 8 + t_loc;
-        s[h][p] = (tok < nb) ? d * scale : -FLT_MAX;
+      for (int c = 0; c < (KV8 ? 2 : 4); ++c)
+        kr[t][c] = *reinterpret_cast<const u32x4*>(kp + c * 64);
+    }
+    #pragma unroll
+    for (int i = 0; i < (KV8 ? 4 : 8); ++i)
+      vr[i] = *reinterpret_cast<const u32x4*>(
+          vc + (i < (KV8 ? 2 : 4) ? p0 : p1) +
+          (i % (KV8 ? 2 : 4)) * 1024 + lane * 16);
+  };
+  char* vl = v_lds[wid];
+  const int vr0 = gr * 8 + (col >> 2);
+  const int v_at = v_byte(vr0, (col & 3) >> 1) + (col & 1) * 8;
+
+  int i = z * 4 + wid;
+  if (i < blocks) {
+    pages(i);
+    fetch();
+    if (i + step < blocks) pages(i + step);
+  }
+  for (; i < blocks; i += step) {
+    f32x4_t sc[2];
+    #pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      sc[t] = f32x4_t(0.f);
+      #pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        union { u32x4 u; short8_t v; } k;
+        if constexpr (KV8) {
+          const u32x4 x = kr[t][c >> 1];
+          k.u = c & 1 ? widen(x.z, x.w) : widen(x.x, x.y);
+        } else {
+          k.u = kr[t][c];
+        }
+        sc[t] = mfma16(k.v, qf[c], sc[t]);
       }
     }
-    // ---- online softmax, shuffle-only (token index lives in bits 3..5) --
-    #pragma unroll
-    for (int h = 0; h < GROUP; ++h) {
-      float bm = fmaxf(s[h][0], s[h][1]);
-      bm = fmaxf(bm, __shfl_xor(bm, 8));
-      bm = fmaxf(bm, __shfl_xor(bm, 16));
-      bm = fmaxf(bm, __shfl_xor(bm, 32));
-      const float mn = fmaxf(m[h], bm);
-      const float alpha = (m[h] == -FLT_MAX) ? 0.f : __expf(m[h] - mn);
-      const float p0 = __expf(s[h][0] - mn);  // masked lanes underflow to 0
-      const float p1 = __expf(s[h][1] - mn);
-      float ps = p0 + p1;
-      ps += __shfl_xor(ps, 8);
-      ps += __shfl_xor(ps, 16);
-      ps += __shfl_xor(ps, 32);
-      l[h] = l[h] * alpha + ps;
-      m[h] = mn;
+    if constexpr (KV8) {             // rows 8 j + lane / 8
       #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        acc[h][j].x *= alpha;
-        acc[h][j].y *= alpha;
+        const int r = 8 * j + (lane >> 3), c = (lane & 7) * 2;
+        *reinterpret_cast<u32x4*>(vl + v_byte(r, c)) =
+            widen(vr[j].x, vr[j].y);
+        *reinterpret_cast<u32x4*>(vl + v_byte(r, c + 1)) =
+            widen(vr[j].z, vr[j].w);
       }
-      if (sl == 0) {
-        sc[wid][h][t_loc] = p0;
-        sc[wid][h][8 + t_loc] = p1;
-      }
-    }
-    // ---- PV: lane accumulates its dim slice over its 4 tokens ----
-    float4 p4[GROUP];
-    #pragma unroll
-    for (int h = 0; h < GROUP; ++h)
-      p4[h] = *reinterpret_cast<const float4*>(&sc[wid][h][4 * g]);
-    #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      float2 vf[4];
-      if constexpr (KV8) {
-        const unsigned* vw = reinterpret_cast<const unsigned*>(&vr2[i]);
-        #pragma unroll
-        for (int jj = 0; jj < 2; ++jj) {
-          float2v lo = __builtin_amdgcn_cvt_pk_f32_fp8(vw[jj], false);
-          float2v hi = __builtin_amdgcn_cvt_pk_f32_fp8(vw[jj], true);
-          vf[2 * jj].x = lo.x; vf[2 * jj].y = lo.y;
-          vf[2 * jj + 1].x = hi.x; vf[2 * jj + 1].y = hi.y;
-        }
-      } else {
-        const unsigned* vw = reinterpret_cast<const unsigned*>(&vr4[i]);
-        #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          vf[j].x = bf2f((unsigned short)(vw[j] & 0xffff));
-          vf[j].y = bf2f((unsigned short)(vw[j] >> 16));
-        }
-      }
+    } else {                         // rows 4 j + lane / 16
       #pragma unroll
-      for (int h = 0; h < GROUP; ++h) {
-        const float p = (&p4[h].x)[i];
-        #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          acc[h][j].x += p * vf[j].x;
-          acc[h][j].y += p * vf[j].y;
-        }
-      }
+      for (int j = 0; j < 8; ++j)
+        *reinterpret_cast<u32x4*>(vl + v_byte(4 * j + gr, col)) = vr[j];
     }
-  }
-
-  // ---- reduce the 4 token groups (bits 4..5); m,l are wave-uniform ----
-  #pragma unroll
-  for (int h = 0; h < GROUP; ++h) {
-    #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      acc[h][j].x += __shfl_xor(acc[h][j].x, 16);
-      acc[h][j].x += __shfl_xor(acc[h][j].x, 32);
-      acc[h][j].y += __shfl_xor(acc[h][j].y, 16);
-      acc[h][j].y += __shfl_xor(acc[h][j].y, 32);
+    if (i + step < blocks) {
+      fetch();
+      if (i + 2 * step < blocks) pages(i + 2 * step);
     }
-  }
-  // ---- combine the 4 waves via LDS ----
-  if (lane < 16) {
+    float p[8], mx = -FLT_MAX;
     #pragma unroll
-    for (int h = 0; h < GROUP; ++h)
+    for (int j = 0; j < 8; ++j) p[j] = sc[j >> 2][j & 3] * a.scale;
+    if ((i + 1) * BLOCK > ctx) {
       #pragma unroll
-      for (int j = 0; j < 4; ++j)
-        *reinterpret_cast<float2*>(&comb_o[wid][h][ds * 8 + j * 2]) =
-            acc[h][j];
-  }
-  if (lane == 0) {
-    #pragma unroll
-    for (int h = 0; h < GROUP; ++h) {
-      comb_m[wid][h] = m[h];
-      comb_l[wid][h] = l[h];
+      for (int j = 0; j < 8; ++j)
+        if (i * BLOCK + gr * 8 + j >= ctx) p[j] = -FLT_MAX;
     }
+    #pragma unroll
+    for (int j = 0; j < 8; ++j) mx = fmaxf(mx, p[j]);
+    mx = fmaxf(mx, __shfl_xor(mx, 16));
+    mx = fmaxf(mx, __shfl_xor(mx, 32));
+    if (__any(mx > m + GROW)) {
+      const float top = fmaxf(m, mx);
+      const float alpha = m == -FLT_MAX ? 0.f : exp2_fast(m - top);
+      #pragma unroll
+      for (int e = 0; e < 8; ++e)
+        #pragma unroll
+        for (int r = 0; r < 4; ++r) acc[e][r] *= alpha;
+      l *= alpha;
+      m = top;
+    }
+    const float base = m == -FLT_MAX ? 0.f : m;
+    #pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      p[j] = exp2_fast(p[j] - base);
+      l += p[j];
+    }
+    short8_t ph, pl;
+    split_bf16x8(p, &ph, &pl);
+    #pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      union { short4_t h[2]; short8_t v; } vf;
+      // row + 4: the same units; column block e: two units on
+      vf.h[0] = lds_read_tr(vl + (v_at ^ e << 5));
+      vf.h[1] = lds_read_tr(vl + (v_at ^ e << 5) + 4 * 256);
+      acc[e] = mfma16(vf.v, ph, acc[e]);
+      acc[e] = mfma16(vf.v, pl, acc[e]);
+    }
+  }
+  l += __shfl_xor(l, 16);
+  l += __shfl_xor(l, 32);
+  __syncthreads();
+  float* comb = reinterpret_cast<float*>(v_lds);     // [4][group][HD]
+  if (gr == 0) {
+    m_lds[wid][col] = m;
+    l_lds[wid][col] = l;
+  }
+  if (col < group) {
+    #pragma unroll
+    for (int e = 0; e < 8; ++e)
+      *reinterpret_cast<f32x4_t*>(
+          comb + (wid * group + col) * HD + e * 16 + gr * 4) = acc[e];
   }
   __syncthreads();
-  for (int i = threadIdx.x; i < GROUP * D; i += 256) {
-    const int h = i / D, d = i % D;
-    float M = fmaxf(fmaxf(comb_m[0][h], comb_m[1][h]),
-                    fmaxf(comb_m[2][h], comb_m[3][h]));
-    float o = 0.f, L = 0.f;
+  for (int u = threadIdx.x * 4; u < group * HD; u += 1024) {
+    const int h = u / HD, d = u % HD;
+    float top = -FLT_MAX, sum = 0.f;
+    #pragma unroll
+    for (int w = 0; w < 4; ++w) top = fmaxf(top, m_lds[w][h]);
+    f32x4_t o = f32x4_t(0.f);
     #pragma unroll
     for (int w = 0; w < 4; ++w) {
-      const float f = (comb_m[w][h] == -FLT_MAX) ? 0.f
-                                                 : __expf(comb_m[w][h] - M);
-      o += f * comb_o[w][h][d];
-      L += f * comb_l[w][h];
+      const float mw = m_lds[w][h];
+      const float f = mw == -FLT_MAX ? 0.f : exp2_fast(mw - top);
+      sum += f * l_lds[w][h];
+      o += *reinterpret_cast<const f32x4_t*>(comb + w * group * HD + u) * f;
     }
     if (split == 1) {
-      *(unsigned short*)(out +
-          ((long)row * H + kvh * g_stride + h + h_off) * D + d) =
-          f2bf(o / L);
+      const float inv = 1.f / sum;
+      *reinterpret_cast<uint2*>(
+          a.out + (((long)row * a.G + g) * group + h) * HD + d) =
+          uint2{cvt_pk_bf16(o[0] * inv, o[1] * inv),
+                cvt_pk_bf16(o[2] * inv, o[3] * inv)};
     } else {
-      // partial layout: [row][kvh][z][h][D+2] fp32 (o | m | l)
-      float* pr = partial +
-          ((((long)row * gridDim.y + kvh) * split + blockIdx.z) * GROUP + h)
-          * (D + 2);
-      pr[d] = o;
-      if (d == 0) { pr[D] = M; pr[D + 1] = L; }
+      float* pr = a.partial +
+          ((((long)row * a.G + g) * split + z) * group + h) * (HD + 2);
+      // rows of 130 floats: 8-byte aligned
+      *reinterpret_cast<float2*>(pr + d) = make_float2(o[0], o[1]);
+      *reinterpret_cast<float2*>(pr + d + 2) = make_float2(o[2], o[3]);
+      if (d == 0) *reinterpret_cast<float2*>(pr + HD) = make_float2(top, sum);
     }
   }
 }
 
-// merge the z-split partials: grid (rows, kvh); 256 threads cover GROUP*D
-template <int GROUP>
-__global__ __launch_bounds__(256) void paged_attn_v3_merge_kernel(
+// The parts of one (row, head) a wave, two columns a lane; lane z has part z's
+// maximum and sum, so that all loads are independent (one workgroup a (row,
+// kvh) that walked the parts took 17 us for one row, 16 parts).
+__global__ __launch_bounds__(256) void paged_attn_merge_kernel(
     bf16* __restrict__ out, const float* __restrict__ partial, int split,
-    int h_total, int g_stride, int h_off) {
-  constexpr int D = 128;
-  const int row = blockIdx.x;
-  const int kvh = blockIdx.y;
-  for (int i = threadIdx.x; i < GROUP * D; i += 256) {
-    const int h = i / D, d = i % D;
-    const float* base = partial +
-        (((long)row * gridDim.y + kvh) * split * GROUP + h) * (D + 2);
-    float M = -FLT_MAX;
-    for (int z = 0; z < split; ++z)
-      M = fmaxf(M, base[(long)z * GROUP * (D + 2) + D]);
-    float o = 0.f, L = 0.f;
-    for (int z = 0; z < split; ++z) {
-      const float* pz = base + (long)z * GROUP * (D + 2);
-      const float mz = pz[D];
-      const float f = (mz == -FLT_MAX) ? 0.f : __expf(mz - M);
-      o += f * pz[d];
-      L += f * pz[D + 1];
-    }
-    *(unsigned short*)(out +
-        ((long)row * h_total + kvh * g_stride + h + h_off) * D + d) =
-        f2bf(o / L);
+    int group, long heads) {
+  const long rh = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (rh >= heads) return;
+  const int lane = threadIdx.x & 63, h = (int)(rh % group);
+  const float* base = partial + (rh / group * split * group + h) * (HD + 2);
+  const long stride = (long)group * (HD + 2);
+  float2 ml = make_float2(-FLT_MAX, 0.f);
+  if (lane < split)
+    ml = *reinterpret_cast<const float2*>(base + lane * stride + HD);
+  const float top = wave_reduce_max(ml.x);
+  const float f = ml.x == -FLT_MAX ? 0.f : exp2_fast(ml.x - top);
+  const float sum = wave_reduce_sum(f * ml.y);
+  float x = 0.f, y = 0.f;
+  #pragma unroll 8
+  for (int z = 0; z < split; ++z) {
+    const float2 o =
+        *reinterpret_cast<const float2*>(base + z * stride + lane * 2);
+    const float fz = __shfl(f, z);
+    x += fz * o.x;
+    y += fz * o.y;
   }
+  const float inv = 1.f / sum;
+  *reinterpret_cast<unsigned*>(out + rh * HD + lane * 2) =
+      cvt_pk_bf16(x * inv, y * inv);
 }
+
+}  // namespace
 
 // With seq_start (and row_seq) only the rows of sequences that have at most
 // max_portion rows are computed.
@@ -537,42 +534,27 @@ void launch_paged_attn(bf16* out, const bf16* q, const bf16* k_cache,
                        hipStream_t stream) {
   if (block_size != ATTN_BS)
     throw std::runtime_error("paged_attn: block_size must be 16");
-  // v3 (D=128): GROUP<=4 direct; GROUP=8 as two GROUP=4 half-calls over
-  // the same KV stream (the kvh=1 70B-TP8 shard: 2x a small KV re-read
-  // buys the v3 structure + occupancy).  split>1 = flash-decode page
-  // split with an fp32 partial workspace + merge kernel.
-  if (D == 128 && (group <= 4 || group == 8)) {
-    const int calls = (group == 8) ? 2 : 1;
-    const int g = (group == 8) ? 4 : group;
-    const int h_total = num_kv_heads * group;
-    for (int c = 0; c < calls; ++c) {
-      const int h_off = c * 4;
-      dim3 grid((unsigned)num_rows, (unsigned)num_kv_heads,
-                (unsigned)split);
-      dim3 mgrid((unsigned)num_rows, (unsigned)num_kv_heads);
-      #define CASE3(G)                                                      \
-        if (g == G) {                                                       \
-          if (kv_fp8)                                                       \
-            paged_attn_v3_kernel<G, true><<<grid, 256, 0, stream>>>(        \
-                out, q, k_cache, v_cache, block_tables, ctx_lens, row_seq,  \
-                max_blocks, num_kv_heads, scale, q_stride, h_total, group,  \
-                h_off, split_ws, seq_start, max_portion);                   \
-          else                                                              \
-            paged_attn_v3_kernel<G, false><<<grid, 256, 0, stream>>>(       \
-                out, q, k_cache, v_cache, block_tables, ctx_lens, row_seq,  \
-                max_blocks, num_kv_heads, scale, q_stride, h_total, group,  \
-                h_off, split_ws, seq_start, max_portion);                   \
-          if (split > 1)                                                    \
-            paged_attn_v3_merge_kernel<G><<<mgrid, 256, 0, stream>>>(       \
-                out, split_ws, split, h_total, group, h_off);               \
-        }
-      CASE3(1) CASE3(2) CASE3(4)
-      #undef CASE3
+  if (D == HD && (group <= 4 || group == 8)) {
+    if (split > 64)
+      throw std::runtime_error("paged_attn: at most 64 parts");
+    const Paged a{out, q, k_cache, v_cache, block_tables, ctx_lens, row_seq,
+                  seq_start, max_portion, max_blocks, num_kv_heads, group,
+                  scale * LOG2E, q_stride, split_ws};
+    const dim3 grid((unsigned)num_rows, (unsigned)num_kv_heads,
+                    (unsigned)split);
+    if (kv_fp8)
+      paged_attn_mfma_kernel<true><<<grid, 256, 0, stream>>>(a);
+    else
+      paged_attn_mfma_kernel<false><<<grid, 256, 0, stream>>>(a);
+    if (split > 1) {
+      const long heads = num_rows * num_kv_heads * group;
+      paged_attn_merge_kernel<<<(unsigned)((heads + 3) / 4), 256, 0,
+                                stream>>>(out, split_ws, split, group, heads);
     }
     return;
   }
   if (split != 1 || seq_start)
-    throw std::runtime_error("paged_attn: split needs the v3 path");
+    throw std::runtime_error("paged_attn: split needs head_dim 128");
   if (kv_fp8)
     throw std::runtime_error("paged_attn: fp8 KV needs head_dim 128");
   dim3 grid((unsigned)num_rows, (unsigned)num_kv_heads);

@@ -95,3 +95,37 @@ def test_whole_prompts(lens, heads, kv, scale):
         if a < b:
             _check(out[a:b], _reference(q[a:b], k[a:b], v[a:b], 0, scale),
                    2.0 ** -9)
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("group,kv", [(1, 2), (2, 1), (3, 1), (4, 3), (8, 1)])
+@pytest.mark.parametrize("split", [1, 2, 5, 64])
+def test_decode_over_pages(split, group, kv, fp8):
+    from hyperspot import _C
+    g = torch.Generator().manual_seed(6)
+    ctx = [1, 15, 16, 17, 32, 33, 127, 128, 129, 700]
+    heads = group * kv
+    q = torch.randn(len(ctx), heads, D, generator=g).bfloat16().to(DEV)
+    tables = [-(-n // 16) for n in ctx]
+    pages = sum(tables) + 3
+    order = torch.randperm(pages, generator=g)
+    kind = torch.float8_e4m3fn if fp8 else torch.bfloat16
+    kc, vc = (torch.randn(pages, kv, 16, D, generator=g).to(kind).to(DEV)
+              for _ in range(2))
+    bt = torch.zeros(len(ctx), max(tables) + 1, dtype=torch.int32)
+    at = 0
+    for i, t in enumerate(tables):
+        bt[i, :t] = order[at:at + t]
+        at += t
+    lens = torch.tensor(ctx, dtype=torch.int32, device=DEV)
+    out = torch.empty_like(q)
+    ws = torch.empty(len(ctx) * heads * split * (D + 2), device=DEV) \
+        if split > 1 else None
+    _C.paged_attn(out, q, kc, vc, bt.to(DEV), lens, None, D ** -0.5, ws,
+                  split)
+    for i, n in enumerate(ctx):
+        page = bt[i, :tables[i]].long().to(DEV)
+        k, v = (c[page].float().transpose(1, 2).reshape(-1, kv, D)[:n]
+                for c in (kc, vc))
+        _check(out[i:i + 1], _reference(q[i:i + 1], k, v, n - 1, D ** -0.5),
+               2.0 ** -14)
