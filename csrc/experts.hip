@@ -135,26 +135,29 @@ __global__ __launch_bounds__(256) void route_kernel(Route r) {
 // row, which count as their product rounded to bf16.  A token's E * W products
 // are too few for a tile of the matrix cores, and one launch replaces the
 // conversions, the product, the softmax, the selection and the division.
-template <bool FP8>
-__global__ __launch_bounds__(256) void router_kernel(
+// What bounds it is the latency of one row of the router: 16 waves have JN
+// experts each, whose loads do not wait for each other.
+template <bool FP8, int JN>
+__global__ __launch_bounds__(1024) void router_kernel(
     Route r, const void* __restrict__ x, const float* __restrict__ x_scale,
     const bf16* __restrict__ router, int W) {
+  constexpr int HELD = 4, COLS = HELD * 512;   // columns at a time
   __shared__ float z[64];
   const long t = blockIdx.x;
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  // columns (i * 64 + lane) * 8, up to COLS of them in registers at a time
-  constexpr int HELD = 8, COLS = HELD * 512;
-  float sum[16];                     // experts wid + 4 j
+  float sum[JN];                     // experts wid + 16 j
   #pragma unroll
-  for (int j = 0; j < 16; ++j) sum[j] = 0.f;
+  for (int j = 0; j < JN; ++j) sum[j] = 0.f;
   for (int c0 = 0; c0 < W; c0 += COLS) {
+    bf16x8 w[JN][HELD];
     float xv[HELD][8];
     #pragma unroll
     for (int i = 0; i < HELD; ++i) {
-      const int c = c0 + (i * 64 + lane) * 8;
+      const int c = min(c0 + (i * 64 + lane) * 8, W - 8);
       #pragma unroll
-      for (int k = 0; k < 8; ++k) xv[i][k] = 0.f;
-      if (c >= W) continue;
+      for (int j = 0; j < JN; ++j)
+        w[j][i] = load_bf16x8(router + (long)min(wid + 16 * j, r.E - 1) * W +
+                              c);
       if constexpr (FP8) {
         const uint2 u = *reinterpret_cast<const uint2*>(
             static_cast<const unsigned char*>(x) + t * W + c);
@@ -172,26 +175,19 @@ __global__ __launch_bounds__(256) void router_kernel(
       }
     }
     #pragma unroll
-    for (int j = 0; j < 16; ++j) {
-      const int e = wid + 4 * j;
-      if (e >= r.E) break;
-      #pragma unroll
-      for (int i = 0; i < HELD; ++i) {
-        const int c = c0 + (i * 64 + lane) * 8;
-        if (c >= W) continue;
-        const bf16x8 w = load_bf16x8(router + (long)e * W + c);
+    for (int i = 0; i < HELD; ++i)
+      if (c0 + (i * 64 + lane) * 8 < W) {
         #pragma unroll
-        for (int k = 0; k < 8; ++k)
-          sum[j] = fmaf(xv[i][k], bf16x8_get(w, k), sum[j]);
+        for (int j = 0; j < JN; ++j)
+          #pragma unroll
+          for (int k = 0; k < 8; ++k)
+            sum[j] = fmaf(xv[i][k], bf16x8_get(w[j][i], k), sum[j]);
       }
-    }
   }
   #pragma unroll
-  for (int j = 0; j < 16; ++j) {
-    const int e = wid + 4 * j;
-    if (e >= r.E) break;
+  for (int j = 0; j < JN; ++j) {
     const float s = wave_reduce_sum(sum[j]);
-    if (lane == 0) z[e] = s;
+    if (lane == 0 && wid + 16 * j < r.E) z[wid + 16 * j] = s;
   }
   __syncthreads();
   if (wid) return;
@@ -528,12 +524,20 @@ void launch_experts_router(float* weight, int* ids, const void* x,
                            int E, int top, int W, hipStream_t stream) {
   if (T == 0) return;
   const Route r{weight, ids, nullptr, (int)T, E, top, 0, 0, E, nullptr};
-  if (x_scale)
-    router_kernel<true><<<(unsigned)T, 256, 0, stream>>>(r, x, x_scale,
-                                                         router, W);
-  else
-    router_kernel<false><<<(unsigned)T, 256, 0, stream>>>(r, x, nullptr,
-                                                          router, W);
+  #define RUN(FP8, JN)                                                      \
+    router_kernel<FP8, JN><<<(unsigned)T, 1024, 0, stream>>>(r, x, x_scale,  \
+                                                             router, W)
+  #define BY_EXPERTS16(FP8)                                                 \
+    if (E <= 16) RUN(FP8, 1);                                               \
+    else if (E <= 32) RUN(FP8, 2);                                          \
+    else RUN(FP8, 4)
+  if (x_scale) {
+    BY_EXPERTS16(true);
+  } else {
+    BY_EXPERTS16(false);
+  }
+  #undef BY_EXPERTS16
+  #undef RUN
 }
 
 void launch_experts_sort(int* order, int* expert, int* place, const int* ids,
