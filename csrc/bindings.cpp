@@ -90,6 +90,8 @@ void launch_recurrent_step(Kind, T*, float*, float*, float*, float*,
                            const float*, const long*, const int*, long, int,
                            int, int, int, long, float, float, float,
                            hipStream_t);
+void launch_decode_inputs(const long*, const int*, long*, long*, long*, int*,
+                          int*, int*, int, int, int, int, int, hipStream_t);
 bool gemm_rows_fits(long, long);
 void launch_gemm_rows(bf16*, const bf16*, const bf16*, int, int, int, long,
                       long, long, hipStream_t);
@@ -278,6 +280,35 @@ void attn_portions(torch::Tensor out, torch::Tensor q, torch::Tensor k_cache,
       block_tables.data_ptr<int>(), ctx_lens.data_ptr<int>(),
       seq_start.data_ptr<int>(), (int)seqs, T, H, KV, max_blocks,
       (int)min_rows, (float)scale, q.stride(0), fp8, stream());
+}
+
+// stage: long [5 * cap], then int [B, staged] page ids
+void decode_inputs(torch::Tensor stage, long B, long cap, long staged,
+                   torch::Tensor ids, torch::Tensor positions,
+                   torch::Tensor slots, torch::Tensor lens,
+                   c10::optional<torch::Tensor> state, torch::Tensor tables) {
+  check(stage, torch::kLong, "stage");
+  for (const auto& t : {ids, positions, slots}) check(t, torch::kLong, "ids");
+  check(lens, torch::kInt32, "lens");
+  check(tables, torch::kInt32, "tables");
+  if (state.has_value()) check(*state, torch::kInt32, "state");
+  const long bucket = ids.numel();
+  TORCH_CHECK(tables.dim() == 2 && tables.size(0) == bucket &&
+                  positions.numel() == bucket && slots.numel() == bucket &&
+                  lens.numel() == bucket &&
+                  (!state.has_value() || state->numel() == bucket),
+              "decode_inputs: rows");
+  TORCH_CHECK(B >= 0 && B <= bucket && B <= cap && staged >= 0 &&
+                  staged <= tables.size(1) &&
+                  stage.numel() * 8 >= cap * 40 + B * staged * 4,
+              "decode_inputs: sizes");
+  long* s = stage.data_ptr<long>();
+  launch_decode_inputs(s, reinterpret_cast<int*>(s + 5 * cap),
+                       ids.data_ptr<long>(), positions.data_ptr<long>(),
+                       slots.data_ptr<long>(), lens.data_ptr<int>(),
+                       state.has_value() ? state->data_ptr<int>() : nullptr,
+                       tables.data_ptr<int>(), (int)B, (int)bucket, (int)cap,
+                       (int)staged, (int)tables.size(1), stream());
 }
 
 // out = x w^T
@@ -1062,6 +1093,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("paged_attn", &paged_attn);
   m.def("attn_prefill_mfma", &attn_prefill_mfma);
   m.def("attn_portions", &attn_portions);
+  m.def("decode_inputs", &decode_inputs);
   m.def("gemm_rows", &gemm_rows);
   m.def("gemm_rows_fits", &gemm_rows_fits);
   m.def("silu_mul", &silu_mul);

@@ -125,13 +125,13 @@ class ModelRunner:
         # pinned staging for the decode hot path (vectorized input prep)
         pin = self.device.type == "cuda"
         cap = self.block_manager.capacity
-        self._st_ids = torch.empty(cap, dtype=torch.long, pin_memory=pin)
-        self._st_pos = torch.empty(cap, dtype=torch.long, pin_memory=pin)
-        self._st_slots = torch.empty(cap, dtype=torch.long, pin_memory=pin)
-        self._st_rows = torch.empty(cap, dtype=torch.int32, pin_memory=pin)
-        self._st_lens = torch.empty(cap, dtype=torch.int32, pin_memory=pin)
-        self._st_bt_flat = torch.empty(cap * self.max_blocks_per_seq,
-                                       dtype=torch.int32, pin_memory=pin)
+        # [id | position | slot | tokens | state row] of cap int64 each, then
+        # the page ids as int32
+        self._stage = torch.empty(
+            5 * cap + (cap * self.max_blocks_per_seq + 1) // 2,
+            dtype=torch.long, pin_memory=pin)
+        self._stage_dev = torch.empty_like(self._stage, device=self.device) \
+            if pin else self._stage
         self._st_event = torch.cuda.Event() if pin else None
         # guided-decoding logit-mask rows keyed by machine state
         self._guided_mask_cache: Dict[tuple, torch.Tensor] = {}
@@ -247,7 +247,8 @@ class ModelRunner:
 
     def _decode_inputs(self, batch: ScheduledBatch):
         """Vectorized decode-step prep: numpy state + pinned staging (the
-        per-sequence Python loop cost more than the GPU step at batch 256)."""
+        per-sequence Python loop cost more than the GPU step at batch 256),
+        one copy to the device.  (staged values, rows, page ids a row)"""
         import numpy as np
         bm = self.block_manager
         reqs = batch.requests
@@ -261,31 +262,34 @@ class ModelRunner:
         max_nt = int(bm.ntables_np[rows].max())
         bt = bm.tables_np[rows[:, None], np.arange(max_nt)[None, :]]
         if self._st_event is not None:
-            # the last step's copies may still be reading the staging
-            # buffers: a step need not end in a device synchronization
+            # the last step's copy may still be reading the staging buffer: a
+            # step need not end in a device synchronization
             self._st_event.synchronize()
-        self._st_ids.numpy()[:B] = ids
-        self._st_pos.numpy()[:B] = pos
-        self._st_slots.numpy()[:B] = slots
-        self._st_lens.numpy()[:B] = pos + 1
-        bt_stage = self._st_bt_flat[:B * max_nt].view(B, max_nt)
-        bt_stage.numpy()[:] = bt
-        d = self.device
-        nb = d.type == "cuda"
-        meta = ForwardMeta(
-            mode="decode",
-            positions=self._st_pos[:B].to(d, non_blocking=nb),
-            slot_mapping=self._st_slots[:B].to(d, non_blocking=nb),
-            block_tables=bt_stage.to(d, non_blocking=nb),
-            seq_lens=self._st_lens[:B].to(d, non_blocking=nb),
-        )
-        if self.spec.is_hybrid:
-            self._st_rows.numpy()[:B] = rows
-            meta.state_slots = self._st_rows[:B].to(d, non_blocking=nb)
-        input_ids = self._st_ids[:B].to(d, non_blocking=nb)
+        cap = bm.capacity
+        used = 5 * cap + (B * max_nt + 1) // 2
+        st = self._stage.numpy()
+        for i, x in enumerate((ids, pos, slots, pos + 1, rows)):
+            st[i * cap:i * cap + B] = x
+        st[5 * cap:].view(np.int32)[:B * max_nt] = bt.reshape(-1)
+        d = self._stage_dev
         if self._st_event is not None:
+            d[:used].copy_(self._stage[:used], non_blocking=True)
             self._st_event.record()
-        return input_ids, meta
+        return d, B, max_nt
+
+    def _decode_meta(self, staged):
+        """Tensors of an eager decode step from the staged values."""
+        d, B, max_nt = staged
+        cap = self.block_manager.capacity
+        part = lambda i: d[i * cap:i * cap + B].clone()
+        meta = ForwardMeta(
+            mode="decode", positions=part(1), slot_mapping=part(2),
+            block_tables=d[5 * cap:].view(torch.int32)[:B * max_nt]
+            .clone().view(B, max_nt),
+            seq_lens=part(3).to(torch.int32))
+        if self.spec.is_hybrid:
+            meta.state_slots = part(4).to(torch.int32)
+        return part(0), meta
 
     # ---------------- execution ----------------
 
@@ -302,8 +306,7 @@ class ModelRunner:
         within its portion) in that order.  `trail` collects the residual
         stream after every layer (prefill steps, eager)."""
         if batch.mode == "decode" and trail is None:
-            input_ids, meta = self._decode_inputs(batch)
-            logits = self._decode_forward(input_ids, meta)
+            logits = self._decode_forward(self._decode_inputs(batch))
             if want is not None:
                 logits = logits[[i for i, w in enumerate(want) for _ in w]]
             return logits
@@ -415,28 +418,17 @@ class ModelRunner:
         self._pgraphs[T] = g
         self._pgraph_io[T] = io
 
-    def _decode_forward(self, input_ids, meta):
-        B = input_ids.shape[0]
+    def _decode_forward(self, staged):
+        stage, B, max_nt = staged
         bucket = self._bucket_for(B)
         if bucket is None or self.device.type != "cuda" \
                 or self.config.enforce_eager:
+            input_ids, meta = self._decode_meta(staged)
             return self.model(input_ids, meta, self.kv_caches)
         if bucket not in self._graphs:
             self._capture(bucket)
         io = self._graph_io[bucket]
-        io["input_ids"][:B] = input_ids
-        io["input_ids"][B:] = 0
-        io["positions"][:B] = meta.positions
-        io["positions"][B:] = 0
-        io["slot_mapping"][:B] = meta.slot_mapping
-        io["slot_mapping"][B:] = -1          # padded rows write nothing
-        io["block_tables"].zero_()
-        io["block_tables"][:B, :meta.block_tables.shape[1]] = meta.block_tables
-        io["seq_lens"][:B] = meta.seq_lens
-        io["seq_lens"][B:] = 1
-        if self.spec.is_hybrid:
-            io["state_slots"][:B] = meta.state_slots
-            io["state_slots"][B:] = -1
+        ops.decode_inputs(stage, B, self.block_manager.capacity, max_nt, io)
         self._graphs[bucket].replay()
         return io["logits"][:B]
 

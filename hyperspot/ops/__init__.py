@@ -392,6 +392,16 @@ def moe_ffn_fp8(xq: "QTensor", w13q: torch.Tensor, w13s: torch.Tensor,
     return out
 
 
+def decode_inputs(stage: torch.Tensor, rows: int, cap: int, pages: int,
+                  io: dict) -> None:
+    """Put the staged values of `rows` rows (csrc/decode_inputs.hip) into the
+    input tensors of a captured decode step.  GPU."""
+    _native().decode_inputs(stage, rows, cap, pages, io["input_ids"],
+                            io["positions"], io["slot_mapping"],
+                            io["seq_lens"], io.get("state_slots"),
+                            io["block_tables"])
+
+
 def greedy_sample(logits: torch.Tensor) -> torch.Tensor:
     if logits.is_cuda:
         out = torch.empty(logits.shape[0], dtype=torch.long,
