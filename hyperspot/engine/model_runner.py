@@ -143,63 +143,63 @@ class ModelRunner:
 
     # ---------------- input preparation ----------------
 
-    def _prefill_inputs(self, batch: ScheduledBatch):
-        ids: List[int] = []
-        pos: List[int] = []
-        slots: List[int] = []
-        starts = [0]
-        logit_rows = []
+    def _to_device(self, *parts) -> List[torch.Tensor]:
+        """numpy arrays (int64 or int32) on the device, by one copy that the
+        host does not wait for."""
         import numpy as np
-        row_seq: List[int] = []
-        tables = []
+        size = [-(-p.nbytes // 8) for p in parts]
+        cuda = self.device.type == "cuda"
+        host = torch.empty(sum(size), dtype=torch.long, pin_memory=cuda)
+        at, flat = 0, host.numpy()
+        for p, n in zip(parts, size):
+            flat[at:at + n].view(p.dtype)[:p.size] = p.reshape(-1)
+            at += n
+        dev = host.to(self.device, non_blocking=cuda)
+        out, at = [], 0
+        for p, n in zip(parts, size):
+            t = dev[at:at + n]
+            if p.dtype == np.int32:
+                t = t.view(torch.int32)[:p.size]
+            out.append(t.view(p.shape))
+            at += n
+        return out
+
+    def _prefill_inputs(self, batch: ScheduledBatch):
+        import numpy as np
         bm = self.block_manager
         bs = bm.block_size
-        fresh = True
-        for si, req in enumerate(batch.requests):
-            cs = req.chunk_start
-            n = req.chunk_len or req.num_prompt_tokens
-            if cs > 0:
-                fresh = False      # continuation chunk attends over cache
-            ids.extend(req.tokens(cs, n))
-            pos.extend(range(cs, cs + n))
-            row = bm.row_of[req.request_id]
-            p = np.arange(cs, cs + n)
-            s = bm.tables_np[row, p // bs].astype(np.int64) * bs + p % bs
-            slots.extend(s.tolist())
-            starts.append(starts[-1] + n)
-            logit_rows.append(starts[-1] - 1)
-            row_seq.extend([si] * n)
-            tables.append(bm.table(req.request_id))
-        max_t = max(len(t) for t in tables)
-        bt = torch.zeros(len(tables), max_t, dtype=torch.int32)
-        for i, t in enumerate(tables):
-            bt[i, :len(t)] = torch.tensor(t, dtype=torch.int32)
-        d = self.device
-        positions = torch.tensor(pos, dtype=torch.long, device=d)
+        rows = [bm.row_of[r.request_id] for r in batch.requests]
+        begin = [r.chunk_start for r in batch.requests]
+        lens = [r.chunk_len or r.num_prompt_tokens for r in batch.requests]
+        starts = np.cumsum([0] + lens, dtype=np.int32)
+        ids = np.concatenate([np.asarray(r.tokens(b, n), dtype=np.int64)
+                              for r, b, n in zip(batch.requests, begin,
+                                                 lens)])
+        seq = np.repeat(np.arange(len(lens), dtype=np.int32), lens)
+        pos = np.arange(starts[-1], dtype=np.int64) \
+            + np.repeat(np.asarray(begin) - starts[:-1], lens)
+        slots = bm.tables_np[np.repeat(rows, lens), pos // bs] \
+            .astype(np.int64) * bs + pos % bs
+        nt = bm.ntables_np[rows]
+        table = bm.tables_np[rows, :int(nt.max())]
+        table = np.where(np.arange(table.shape[1]) < nt[:, None], table, 0) \
+            .astype(np.int32)
+        (input_ids, positions, slots, last, seq_start, seq, ctx,
+         table) = self._to_device(
+            ids, pos, slots, (starts[1:] - 1).astype(np.int64), starts, seq,
+            (pos + 1).astype(np.int32), table)
         meta = ForwardMeta(
-            mode="prefill",
-            positions=positions,
-            slot_mapping=torch.tensor(slots, dtype=torch.long, device=d),
-            seq_start=torch.tensor(starts, dtype=torch.int32, device=d),
-            max_seqlen=max((r.chunk_len or r.num_prompt_tokens)
-                           for r in batch.requests),
-            min_seqlen=min((r.chunk_len or r.num_prompt_tokens)
-                           for r in batch.requests),
-            fresh_prefill=fresh,
-            row_seq=torch.tensor(row_seq, dtype=torch.int32, device=d),
-            ctx_lens=(positions + 1).to(torch.int32),
-            block_tables=bt.to(d),
-            logits_indices=torch.tensor(logit_rows, dtype=torch.long, device=d),
-        )
+            mode="prefill", positions=positions, slot_mapping=slots,
+            seq_start=seq_start, max_seqlen=max(lens), min_seqlen=min(lens),
+            # a continuation chunk attends over the cache
+            fresh_prefill=not any(begin),
+            row_seq=seq, ctx_lens=ctx, block_tables=table,
+            logits_indices=last)
         if self.spec.is_hybrid:
-            rows = [bm.row_of[r.request_id] for r in batch.requests]
-            lens = [b - a for a, b in zip(starts, starts[1:])]
             self._add_hybrid_meta(meta, rows, lens)
-            if d.type == "cuda":
-                meta.latent = {w: self._latent_span(
-                    w, rows, [r.chunk_start for r in batch.requests], lens)
-                    for w in self.spec.latent_windows}
-        input_ids = torch.tensor(ids, dtype=torch.long, device=d)
+            if self.device.type == "cuda":
+                meta.latent = {w: self._latent_span(w, rows, begin, lens)
+                               for w in self.spec.latent_windows}
         return input_ids, meta
 
     def _add_hybrid_meta(self, meta: ForwardMeta, rows: List[int],
@@ -353,18 +353,20 @@ class ModelRunner:
         bm = self.block_manager
         row = bm.row_of[req.request_id]
         p = np.arange(n)
-        slots = bm.tables_np[row, p // bm.block_size].astype(np.int64)             * bm.block_size + p % bm.block_size
         io = self._pgraph_io[T]
-        d = self.device
-        io["input_ids"][:n] = torch.tensor(req.prompt_token_ids[:n],
-                                           dtype=torch.long, device=d)
-        io["input_ids"][n:] = 0
-        io["positions"][:n] = torch.arange(n, dtype=torch.long, device=d)
-        io["positions"][n:] = 0
-        io["slot_mapping"][:n] = torch.from_numpy(slots).to(d)
-        io["slot_mapping"][n:] = -1
-        io["lidx"][0] = n - 1
+        # one copy into the graph's inputs; pad tokens write no page
+        host = torch.zeros(io["inputs"].numel(), dtype=torch.long,
+                           pin_memory=True)
+        at = host.numpy()
+        at[:n] = req.prompt_token_ids[:n]
+        at[T:T + n] = p
+        at[2 * T:2 * T + n] = bm.tables_np[row, p // bm.block_size] \
+            .astype(np.int64) * bm.block_size + p % bm.block_size
+        at[2 * T + n:3 * T] = -1
+        at[3 * T] = n - 1
+        io["inputs"].copy_(host, non_blocking=True)
         if self.spec.is_hybrid:
+            d = self.device
             # the recurrence must stop at the last real token
             io["seq_start"][1] = n
             io["state_slots"][0] = row
@@ -376,12 +378,14 @@ class ModelRunner:
     def _capture_prefill(self, T: int) -> None:
         d = self.device
         log.info("capturing prefill hipGraph for tokens=%d", T)
+        inputs = torch.zeros(3 * T + 1, dtype=torch.long, device=d)
+        inputs[2 * T:3 * T] = -1
         io = {
-            "input_ids": torch.zeros(T, dtype=torch.long, device=d),
-            "positions": torch.zeros(T, dtype=torch.long, device=d),
-            "slot_mapping": torch.full((T,), -1, dtype=torch.long,
-                                       device=d),
-            "lidx": torch.zeros(1, dtype=torch.long, device=d),
+            "inputs": inputs,
+            "input_ids": inputs[:T],
+            "positions": inputs[T:2 * T],
+            "slot_mapping": inputs[2 * T:3 * T],
+            "lidx": inputs[3 * T:],
             "seq_start": torch.tensor([0, T], dtype=torch.int32, device=d),
         }
         meta = ForwardMeta(
