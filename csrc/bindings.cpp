@@ -103,15 +103,8 @@ void launch_fused_add_rmsnorm_fp8(unsigned char*, float*, const bf16*,
                                   hipStream_t);
 void launch_silu_mul_fp8(unsigned char*, float*, const bf16*, long, int,
                          hipStream_t);
-void launch_moe_align(int*, int*, int*, const int*, int, int, int,
-                      hipStream_t);
 void launch_moe_gemm(bf16*, float*, const bf16*, const bf16*, const int*,
                      const int*, int, int, int, int, int, hipStream_t);
-void launch_moe_combine(bf16*, const bf16*, const float*, const int*, long,
-                        int, int, hipStream_t);
-void launch_moe_gemm_fp8(bf16*, float*, const unsigned char*, const float*,
-                         const unsigned char*, const float*, const int*,
-                         const int*, int, int, int, int, int, hipStream_t);
 template <typename T>
 void launch_greedy_sample(long*, const T*, long, int, hipStream_t);
 template <typename T>
@@ -995,19 +988,6 @@ void silu_mul_fp8(torch::Tensor out, torch::Tensor scales, torch::Tensor x) {
 }
 
 
-void moe_align(torch::Tensor sorted_ids, torch::Tensor tile_expert,
-               torch::Tensor inv_pos, torch::Tensor flat_ids,
-               long num_experts) {
-  check(sorted_ids, torch::kInt, "sorted_ids");
-  check(tile_expert, torch::kInt, "tile_expert");
-  check(inv_pos, torch::kInt, "inv_pos");
-  check(flat_ids, torch::kInt, "flat_ids");
-  launch_moe_align(sorted_ids.data_ptr<int>(), tile_expert.data_ptr<int>(),
-                   inv_pos.data_ptr<int>(), flat_ids.data_ptr<int>(),
-                   (int)flat_ids.numel(), (int)num_experts,
-                   (int)tile_expert.numel(), stream());
-}
-
 void moe_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
               torch::Tensor sorted_ids, torch::Tensor tile_expert,
               long gather_div, long splitk,
@@ -1033,47 +1013,6 @@ void moe_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
                   (int)splitk, stream());
 }
 
-void moe_combine(torch::Tensor out, torch::Tensor y, torch::Tensor wts,
-                 torch::Tensor inv_pos, long topk) {
-  check(out, torch::kBFloat16, "out");
-  check(y, torch::kBFloat16, "y");
-  check(wts, torch::kFloat, "wts");
-  check(inv_pos, torch::kInt, "inv_pos");
-  launch_moe_combine(bf(out), cbf(y), wts.data_ptr<float>(),
-                     inv_pos.data_ptr<int>(), out.size(0), (int)topk,
-                     (int)out.size(-1), stream());
-}
-
-
-void moe_gemm_fp8(torch::Tensor out, torch::Tensor xq, torch::Tensor xs,
-                  torch::Tensor wq, torch::Tensor ws,
-                  torch::Tensor sorted_ids, torch::Tensor tile_expert,
-                  long gather_div, long splitk,
-                  c10::optional<torch::Tensor> skw) {
-  check(out, torch::kBFloat16, "out");
-  check(xq, torch::kFloat8_e4m3fn, "xq");
-  check(xs, torch::kFloat, "xs");
-  check(wq, torch::kFloat8_e4m3fn, "wq");
-  check(ws, torch::kFloat, "ws");
-  check(sorted_ids, torch::kInt, "sorted_ids");
-  check(tile_expert, torch::kInt, "tile_expert");
-  TORCH_CHECK(wq.dim() == 3, "wq must be [E, N, K]");
-  float* skp = nullptr;
-  if (splitk > 1) {
-    TORCH_CHECK(skw.has_value(),
-                "moe_gemm_fp8: splitk>1 needs a workspace");
-    check(*skw, torch::kFloat, "skw");
-    TORCH_CHECK(skw->numel() >= splitk * out.numel(),
-                "moe_gemm_fp8: workspace too small");
-    skp = skw->data_ptr<float>();
-  }
-  launch_moe_gemm_fp8(bf(out), skp, u8(xq), xs.data_ptr<float>(), u8(wq),
-                      ws.data_ptr<float>(), sorted_ids.data_ptr<int>(),
-                      tile_expert.data_ptr<int>(),
-                      (int)tile_expert.numel(), (int)wq.size(1),
-                      (int)wq.size(2), (int)gather_div, (int)splitk,
-                      stream());
-}
 
 void register_latent(pybind11::module_& m);    // bindings_latent.cpp
 void register_sublayer(pybind11::module_& m);  // bindings_sublayer.cpp
@@ -1084,10 +1023,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("quant_fp8", &quant_fp8);
   m.def("fused_add_rmsnorm_fp8", &fused_add_rmsnorm_fp8);
   m.def("silu_mul_fp8", &silu_mul_fp8);
-  m.def("moe_align", &moe_align);
   m.def("moe_gemm", &moe_gemm);
-  m.def("moe_combine", &moe_combine);
-  m.def("moe_gemm_fp8", &moe_gemm_fp8);
   m.def("fused_add_rmsnorm", &fused_add_rmsnorm);
   m.def("rope_kv_append", &rope_kv_append);
   m.def("paged_attn", &paged_attn);

@@ -53,6 +53,9 @@ void launch_experts_route(float*, int*, const float*, int, int, int, bool,
                           bool, int, const float*, hipStream_t);
 void launch_experts_router(float*, int*, const void*, const float*,
                            const bf16*, long, int, int, int, hipStream_t);
+void launch_experts_tiles(bool, bf16*, const void*, const void*, const float*,
+                          const float*, const int*, const int*, int, int, int,
+                          int, int, hipStream_t);
 void launch_experts_sort(int*, int*, int*, const int*, int, int, int, int,
                          hipStream_t);
 void launch_experts_route_sort(float*, int*, int*, int*, int*, const float*,
@@ -485,6 +488,41 @@ void experts_route(Tensor weight, Tensor ids, Tensor logits, long E, long top,
                        opt(correction), stream());
 }
 
+// out [tiles * bm, N] of sorted choices; div 0: x has a row for each of them,
+// otherwise choice c is of row c / div.  With scales x and w are e4m3.
+void experts_tiles(Tensor out, Tensor x, Tensor w, Maybe x_scale,
+                   Maybe w_scale, Tensor order, Tensor expert, bool gated,
+                   long div, long bm) {
+  const bool fp8 = x_scale.has_value();
+  const auto dt = fp8 ? torch::kFloat8_e4m3fn : torch::kBFloat16;
+  check(x, dt, "x");
+  check(w, dt, "w");
+  check(out, torch::kBFloat16, "out");
+  TORCH_CHECK(x.dim() == 2 && w.dim() == 3 && out.dim() == 2 && !(gated && fp8)
+                  && w_scale.has_value() == fp8, "experts_tiles: operands");
+  const long E = w.size(0), N = w.size(1) / (gated ? 2 : 1), K = w.size(2);
+  const long tiles = expert.numel(), chunk = fp8 ? 128 : 64;
+  TORCH_CHECK(bm == 64 || bm == 128 || bm == 256, "experts_tiles: bm");
+  TORCH_CHECK(K % chunk == 0 && K >= 2 * chunk &&
+                  w.size(1) % 128 == 0 && x.size(1) == K &&
+                  (div > 0 || x.size(0) == tiles * bm) &&
+                  out.size(0) == tiles * bm && out.size(1) == N,
+              "experts_tiles: shape");
+  for (const auto& t : {x, w, out})
+    TORCH_CHECK(reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0,
+                "experts_tiles: alignment");
+  check_ints(order, tiles * bm, "order");
+  check_ints(expert, tiles, "expert");
+  if (fp8) {
+    check_param(*x_scale, x.size(0), "x_scale");
+    check_param(*w_scale, E * N, "w_scale");
+  }
+  launch_experts_tiles(gated, ptr<bf16>(out), x.data_ptr(), w.data_ptr(),
+                       opt(x_scale), opt(w_scale), order.data_ptr<int>(),
+                       expert.data_ptr<int>(), (int)tiles, (int)N, (int)K,
+                       (int)div, (int)bm, stream());
+}
+
 // choices and weights of the rows of x [T, W], bf16 or e4m3 with x_scale [T]
 void experts_router(Tensor weight, Tensor ids, Tensor x, Maybe x_scale,
                     Tensor router, long top) {
@@ -659,6 +697,7 @@ void register_latent(pybind11::module_& m) {
         py::arg("logits"), py::arg("E"), py::arg("top"),
         py::arg("correction") = py::none(), py::arg("identity") = 0);
   m.def("experts_router", &experts_router);
+  m.def("experts_tiles", &experts_tiles);
   m.def("experts_sort", &experts_sort);
   m.def("experts_route_sort", &experts_route_sort);
   m.def("experts_up", &experts_up);

@@ -1,0 +1,263 @@
+// Grouped expert products in LDS tiles (gfx950), bf16 or e4m3 with scales.
+//
+//   out[p, n] = x[r] . w[e, n] of every choice, in the order of experts.hip's
+//   sort with bm rows a tile: r is p, or with div the token order[p] / div
+//   GATED: out[p, i] = silu(x[r] . w[e, i]) * (x[r] . w[e, N + i])
+//
+// A workgroup has bm choices of one expert and BN rows of its weights, K in
+// chunks of 128 bytes.  Both go from memory to LDS directly, 16 bytes a lane
+// and whole 128-byte lines, into a ring of chunks; weights are the A operand
+// of 32x32x16 products, so that a lane's results are 4 consecutive outputs of
+// one choice, and of every 16 rows of weights 8 are a gate's and 8 its up
+// row's: both of a pair are in one lane, and the activation needs no pass of
+// its own.
+//
+// What bounds it: the weights' bytes up to about 100 choices an expert, so bm
+// is what covers most counts (256 rows of x, mostly padding, beside 128 of
+// weights are two thirds of what is loaded), then the products.  Mixtral 8x7B
+// layer (8 experts, 14336 x 4096, 2.8 GB), us with 256-row tiles, row tiles
+// and here: 16 choices an expert 821 617 532, 48 831 792 543, 128 943 869 730,
+// 500 2355 2100 1740.  32 experts of 1024 x 2048, 64 choices 277 172 119.
+#include "common.h"
+
+namespace {
+
+typedef __attribute__((address_space(1))) const unsigned glob;
+typedef __attribute__((address_space(3))) unsigned shar;
+
+struct Tiles {
+  bf16* out;
+  const void* x;
+  const void* w;
+  const float* x_scale;        // FP8: of a row of x, and of a row of w
+  const float* w_scale;
+  const int* order;
+  const int* expert;
+  int N, K, div, nx;           // N outputs a choice, nx blocks of them
+};
+
+// 16-byte unit c of row r of a chunk in LDS: reads of 8 rows of one unit
+// spread over the banks
+DEV int unit(int r, int c) { return r * 128 + ((c ^ (r & 7)) << 4); }
+
+// BM choices, BN rows of weights; WM * WN waves have BM / WM by BN / WN
+template <int BM, int BN, int WM, int WN, int STAGES, bool GATED, bool FP8>
+__global__ __launch_bounds__(WM * WN * 64,
+                             WM * WN == 4 ? 2 : WM * WN / 4)
+void experts_tiles_kernel(Tiles a) {
+  constexpr int WAVES = WM * WN;
+  constexpr int NI = BN / WN / 32, MI = BM / WM / 32;
+  constexpr int LX = BM / 8 / WAVES, LW = BN / 8 / WAVES;  // loads a chunk
+  constexpr int STAGE = (BM + BN) * 128;
+  constexpr int OUT = GATED ? BN / 2 : BN;                 // outputs
+  constexpr int ELEM = FP8 ? 1 : 2;
+  static_assert(!(GATED && FP8), "the activation's scale needs whole rows");
+  static_assert(LX * WAVES * 8 == BM && LW * WAVES * 8 == BN, "loads");
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  const int tile = blockIdx.x / a.nx, e = a.expert[tile];
+  if (e < 0) return;
+  const int n0 = (blockIdx.x % a.nx) * OUT, p0 = tile * BM;
+  const int lane = threadIdx.x & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int col = lane & 31, hf = lane >> 5;
+  // a SIMD has waves of different choices: those without any do nothing
+  const int wm = wid / WN, wn = wid % WN;
+  const bool live = a.order[p0 + wm * (BM / WM)] >= 0;
+
+  // this lane's 16 bytes of row lane / 8 of each 1-KB load
+  const int lr = lane >> 3, lc = ((lane & 7) ^ lr) * 16;
+  const long row_bytes = (long)a.K * ELEM;
+  auto row_of = [&](int p) {
+    const int choice = a.order[p];
+    return a.div ? (choice >= 0 ? choice / a.div : 0) : p;
+  };
+  const char* xp[LX];
+  #pragma unroll
+  for (int j = 0; j < LX; ++j)
+    xp[j] = static_cast<const char*>(a.x) +
+            row_of(p0 + (wid * LX + j) * 8 + lr) * row_bytes + lc;
+  const char* wp[LW];
+  #pragma unroll
+  for (int j = 0; j < LW; ++j) {
+    int n = (wid * LW + j) * 8 + lr;
+    if constexpr (GATED)       // 8 gate rows, then their 8 up rows
+      n = n0 + (n >> 4) * 8 + (n & 7) + (n & 8 ? a.N : 0);
+    else
+      n += n0;
+    wp[j] = static_cast<const char*>(a.w) +
+            ((long)e * (GATED ? 2 * a.N : a.N) + n) * row_bytes + lc;
+  }
+  auto stage = [&](int slot, int chunk) {
+    char* base = lds + slot * STAGE;
+    #pragma unroll
+    for (int j = 0; j < LX; ++j)
+      __builtin_amdgcn_global_load_lds(
+          (glob*)(xp[j] + chunk * 128),
+          (shar*)(base + (wid * LX + j) * 1024), 16, 0, 0);
+    #pragma unroll
+    for (int j = 0; j < LW; ++j)
+      __builtin_amdgcn_global_load_lds(
+          (glob*)(wp[j] + chunk * 128),
+          (shar*)(base + BM * 128 + (wid * LW + j) * 1024), 16, 0, 0);
+  };
+
+  f32x16_t acc[NI][MI];
+  #pragma unroll
+  for (int n = 0; n < NI; ++n)
+    #pragma unroll
+    for (int m = 0; m < MI; ++m) acc[n][m] = f32x16_t(0.f);
+  const int x_at = unit(wm * MI * 32 + col, hf);
+  const int w_at = BM * 128 + unit(wn * NI * 32 + col, hf);
+  auto compute = [&](int slot) {
+    if (!live) return;
+    const char* base = lds + slot * STAGE;
+    #pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      short8_t xf[MI], wf[NI];
+      #pragma unroll
+      for (int m = 0; m < MI; ++m)
+        xf[m] = *reinterpret_cast<const short8_t*>(
+            base + (x_at ^ k << 5) + m * 32 * 128);
+      #pragma unroll
+      for (int n = 0; n < NI; ++n)
+        wf[n] = *reinterpret_cast<const short8_t*>(
+            base + (w_at ^ k << 5) + n * 32 * 128);
+      #pragma unroll
+      for (int n = 0; n < NI; ++n)
+        #pragma unroll
+        for (int m = 0; m < MI; ++m)
+          if constexpr (FP8) {     // 16 bytes a lane are two steps of 16
+            union { short8_t v; long l[2]; } u{wf[n]}, v{xf[m]};
+            acc[n][m] = __builtin_amdgcn_mfma_f32_32x32x16_fp8_fp8(
+                u.l[0], v.l[0], acc[n][m], 0, 0, 0);
+            acc[n][m] = __builtin_amdgcn_mfma_f32_32x32x16_fp8_fp8(
+                u.l[1], v.l[1], acc[n][m], 0, 0, 0);
+          } else {
+            acc[n][m] = mfma32(wf[n], xf[m], acc[n][m]);
+          }
+    }
+  };
+
+  const int chunks = (int)(row_bytes / 128);
+  if constexpr (STAGES == 2) {
+    // [chunk d landed | barrier | issue d + 1 | compute d]: the barrier also
+    // says that every wave is done with the slot that d + 1 takes
+    stage(0, 0);
+    for (int d = 0; d < chunks; ++d) {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      if (d + 1 < chunks) stage((d + 1) & 1, d + 1);
+      compute(d & 1);
+    }
+  } else {
+    // [compute d | issue d + 2 | d + 1 landed | barrier]: d + 2 takes the slot
+    // of d - 1, with which every wave was done before the last barrier
+    static_assert(STAGES == 3, "stages");
+    constexpr int LOADS = LX + LW;
+    stage(0, 0);
+    stage(1, 1);
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LOADS) : "memory");
+    __builtin_amdgcn_s_barrier();
+    int slot = 0, d = 0;
+    for (; d + 2 < chunks; ++d) {
+      compute(slot);
+      stage(slot == 0 ? 2 : slot - 1, d + 2);
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LOADS) : "memory");
+      __builtin_amdgcn_s_barrier();
+      slot = slot == 2 ? 0 : slot + 1;
+    }
+    compute(slot);                       // d == chunks - 2
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    compute(slot == 2 ? 0 : slot + 1);
+  }
+
+  // acc[n][m][r]: weight row (r >> 2) * 8 + hf * 4 + (r & 3) of block n,
+  // choice col of block m
+  #pragma unroll
+  for (int m = 0; m < MI; ++m) {
+    const int p = p0 + (wm * MI + m) * 32 + col;
+    if (a.order[p] < 0) continue;
+    bf16* op = a.out + (long)p * a.N + n0 + hf * 4;
+    const float xs = FP8 ? a.x_scale[row_of(p)] : 1.f;
+    #pragma unroll
+    for (int n = 0; n < NI; ++n) {
+      if constexpr (GATED) {
+        #pragma unroll
+        for (int r = 0; r < 16; r += 8) {
+          float y[4];
+          #pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const float g = acc[n][m][r + j], u = acc[n][m][r + 4 + j];
+            y[j] = g / (1.f + __expf(-g)) * u;
+          }
+          *reinterpret_cast<uint2*>(op + (wn * NI + n) * 16 + r) =
+              uint2{cvt_pk_bf16(y[0], y[1]), cvt_pk_bf16(y[2], y[3])};
+        }
+      } else {
+        const int c = (wn * NI + n) * 32;
+        #pragma unroll
+        for (int r = 0; r < 16; r += 4) {
+          float y[4];
+          #pragma unroll
+          for (int j = 0; j < 4; ++j) y[j] = acc[n][m][r + j];
+          if constexpr (FP8) {
+            const float4 ws = *reinterpret_cast<const float4*>(
+                a.w_scale + (long)e * a.N + n0 + c + r * 2 + hf * 4);
+            y[0] = y[0] * xs * ws.x;
+            y[1] = y[1] * xs * ws.y;
+            y[2] = y[2] * xs * ws.z;
+            y[3] = y[3] * xs * ws.w;
+          }
+          *reinterpret_cast<uint2*>(op + c + r * 2) =
+              uint2{cvt_pk_bf16(y[0], y[1]), cvt_pk_bf16(y[2], y[3])};
+        }
+      }
+    }
+  }
+}
+
+}  // namespace
+
+// bm 64, 128 or 256; rows of w of 128-byte chunks, at least two; outputs N a
+// multiple of 128 (gated: of 64).  x, w and out contiguous; with scales x and
+// w are e4m3.
+void launch_experts_tiles(bool gated, bf16* out, const void* x, const void* w,
+                          const float* x_scale, const float* w_scale,
+                          const int* order, const int* expert, int tiles,
+                          int N, int K, int div, int bm, hipStream_t stream) {
+  if (tiles == 0) return;
+  Tiles a{out, x, w, x_scale, w_scale, order, expert, N, K, div, 0};
+  #define RUN(BM, BN, WM, WN, STAGES, GATED, FP8)                           \
+    {                                                                       \
+      constexpr int BYTES = STAGES * (BM + BN) * 128;                       \
+      static const hipError_t set = hipFuncSetAttribute(                    \
+          reinterpret_cast<const void*>(                                    \
+              &experts_tiles_kernel<BM, BN, WM, WN, STAGES, GATED, FP8>),   \
+          hipFuncAttributeMaxDynamicSharedMemorySize, BYTES);               \
+      HIP_CHECK(set);                                                       \
+      a.nx = N / (GATED ? BN / 2 : BN);                                     \
+      experts_tiles_kernel<BM, BN, WM, WN, STAGES, GATED, FP8>              \
+          <<<(unsigned)(tiles * a.nx), WM * WN * 64, BYTES, stream>>>(a);   \
+    }
+  #define KINDS(BM, BN, WM, WN, STAGES)                                     \
+    if (x_scale) RUN(BM, BN, WM, WN, STAGES, false, true)                   \
+    else if (gated) RUN(BM, BN, WM, WN, STAGES, true, false)                \
+    else RUN(BM, BN, WM, WN, STAGES, false, false)
+  // 256 rows of weights need fewer loads of x and LDS reads, and leave units
+  // idle where they make few workgroups: Mixtral 8x7B, 500 choices an expert,
+  // up (2000 workgroups of 256) 1055 us against 1223, down (290) 753 against
+  // 682; 32 experts of 1024 x 2048, 250 choices, 120 108 and 79 67
+  const int wide = gated ? 128 : 256;
+  if (bm == 64) {
+    KINDS(64, 128, 2, 2, 3)
+  } else if (bm == 128) {
+    KINDS(128, 128, 2, 4, 3)
+  } else if (N % wide == 0 && (long)tiles * (N / wide) >= 1024) {
+    KINDS(256, 256, 4, 2, 2)
+  } else {
+    KINDS(256, 128, 4, 2, 3)
+  }
+  #undef KINDS
+  #undef RUN
+}

@@ -1,72 +1,15 @@
-// MoE kernels for gfx950: token alignment, grouped expert GEMM (MFMA),
-// weighted combine.  SURVEY.md §2.9 kernel obligations for Mixtral (EP).
+// Grouped expert GEMM in 256-row tiles for gfx950, for the large steps of the
+// designs whose experts have an activation or a shared expert of their own
+// (experts_tiles.hip has the gated experts, experts.hip the sort and the sum).
 //
-// Capture-safety is the design driver: decode steps replay as hipGraphs,
-// so every grid here is a function of (T, K, E) only — per-expert token
-// counts live in device memory and never reach the host.
+// Capture-safety is the design driver: decode steps replay as hipGraphs, so
+// every grid here is a function of (T, K, E) only.
 //
-//   moe_align:   top-k pair ids -> per-expert sorted order, padded to
-//                MOE_BM-row tiles; emits sorted_ids (pair idx | -1 pad),
-//                tile_expert (expert per 32-row tile | -1 unused) and
-//                inv_pos (pair -> sorted position) in ONE workgroup.
 //   moe_gemm:    out[p, n] = x[row(p)] @ W[expert(tile(p))]^T over the
-//                sorted space; 128x128 tile per workgroup (8 waves, each
-//                32x64 via 2x v_mfma_f32_32x32x16_bf16 per k-chunk), LDS
-//                XOR-swizzled A/B.  BM=128 is a WEIGHT-TRAFFIC choice:
-//                with 32-row tiles each expert's [N,K] matrix was
-//                re-streamed once per m-tile (~9x at batch 1024 -> the
-//                measured 139 ms Mixtral step); 128-row tiles cut the
-//                re-read to ceil(tokens_e/128) at the price of padding
-//                compute, and padding is cheap where HBM is the bound.
-//   moe_combine: out[t] = sum_k w[t,k] * y[inv_pos[t*K+k]]  (gather, no
-//                atomics).
+//                sorted space.
 #include "common.h"
 
 #define MOE_BM 256  // sorted rows per expert tile (the align granularity)
-
-// ---------------------------------------------------------------- align
-__global__ __launch_bounds__(256) void moe_align_kernel(
-    int* __restrict__ sorted_ids, int* __restrict__ tile_expert,
-    int* __restrict__ inv_pos, const int* __restrict__ flat_ids,
-    int num_pairs, int num_experts, int ntiles_max) {
-  extern __shared__ int lds[];   // [E] counts | [E+1] offsets | [E] cursor
-  int* cnt = lds;
-  int* off = lds + num_experts;
-  int* cur = lds + 2 * num_experts + 1;
-  for (int e = threadIdx.x; e < num_experts; e += 256) {
-    cnt[e] = 0;
-    cur[e] = 0;
-  }
-  __syncthreads();
-  for (int p = threadIdx.x; p < num_pairs; p += 256)
-    atomicAdd(&cnt[flat_ids[p]], 1);
-  __syncthreads();
-  if (threadIdx.x == 0) {        // serial prefix over E (E <= 64)
-    int acc = 0;
-    for (int e = 0; e < num_experts; ++e) {
-      off[e] = acc;
-      acc += (cnt[e] + MOE_BM - 1) / MOE_BM * MOE_BM;  // pad to tile
-    }
-    off[num_experts] = acc;
-  }
-  __syncthreads();
-  const int P = ntiles_max * MOE_BM;
-  for (int i = threadIdx.x; i < P; i += 256) sorted_ids[i] = -1;
-  for (int t = threadIdx.x; t < ntiles_max; t += 256) {
-    int e_of = -1;
-    const int r0 = t * MOE_BM;
-    for (int e = 0; e < num_experts; ++e)
-      if (r0 >= off[e] && r0 < off[e + 1]) { e_of = e; break; }
-    tile_expert[t] = e_of;
-  }
-  __syncthreads();
-  for (int p = threadIdx.x; p < num_pairs; p += 256) {
-    const int e = flat_ids[p];
-    const int pos = off[e] + atomicAdd(&cur[e], 1);
-    sorted_ids[pos] = p;
-    inv_pos[p] = pos;
-  }
-}
 
 // ------------------------------------------------------------- grouped GEMM
 typedef __attribute__((ext_vector_type(8))) short short8;
@@ -154,7 +97,7 @@ __global__ __launch_bounds__(512) void moe_gemm_v3_kernel(
   // dynamic LDS addressed by INTEGER offsets (pointer indirection decays
   // to generic AS => flat_load + vmcnt stalls in the MFMA stream)
   // ring layout: A0 A1 A2 | B0 B1 B2
-  extern __shared__ int lds[];     // shared decl w/ moe_align
+  extern __shared__ int lds[];
   unsigned char* dyn_lds = reinterpret_cast<unsigned char*>(lds);
 
   const int tid = threadIdx.x;
@@ -319,41 +262,6 @@ __global__ __launch_bounds__(256) void moe_sk_reduce_kernel(
       *reinterpret_cast<ushort4*>(o);
 }
 
-// ------------------------------------------------------------- combine
-__global__ __launch_bounds__(256) void moe_combine_kernel(
-    bf16* __restrict__ out, const bf16* __restrict__ y,
-    const float* __restrict__ wts, const int* __restrict__ inv_pos,
-    int topk, int hidden) {
-  const long t = blockIdx.x;
-  for (int j = threadIdx.x * 8; j < hidden; j += 256 * 8) {
-    float accv[8];
-    #pragma unroll
-    for (int i = 0; i < 8; ++i) accv[i] = 0.f;
-    for (int k = 0; k < topk; ++k) {
-      const float wk = wts[t * topk + k];
-      const long pos = inv_pos[t * topk + k];
-      bf16x8 v = load_bf16x8(y + pos * hidden + j);
-      #pragma unroll
-      for (int i = 0; i < 8; ++i) accv[i] += wk * bf16x8_get(v, i);
-    }
-    bf16x8 o;
-    #pragma unroll
-    for (int i = 0; i < 8; ++i) bf16x8_set(o, i, accv[i]);
-    store_bf16x8(out + t * hidden + j, o);
-  }
-}
-
-void launch_moe_align(int* sorted_ids, int* tile_expert, int* inv_pos,
-                      const int* flat_ids, int num_pairs, int num_experts,
-                      int ntiles_max, hipStream_t stream) {
-  if (num_experts > 64)
-    throw std::runtime_error("moe_align: num_experts > 64");
-  const int lds_bytes = (2 * num_experts + 1 + num_experts) * 4;
-  moe_align_kernel<<<1, 256, lds_bytes, stream>>>(
-      sorted_ids, tile_expert, inv_pos, flat_ids, num_pairs, num_experts,
-      ntiles_max);
-}
-
 // splitk segments (>1 needs ws = fp32 [splitk, ntiles*MOE_BM, N]);
 // nchunks must divide evenly — the python op picks splitk accordingly
 void launch_moe_gemm(bf16* out, float* ws, const bf16* x, const bf16* w,
@@ -390,218 +298,5 @@ void launch_moe_gemm(bf16* out, float* ws, const bf16* x, const bf16* w,
     const long PN = (long)ntiles_max * MOE_BM * N;
     moe_sk_reduce_kernel<<<dim3((unsigned)((PN / 4 + 255) / 256)), 256,
                            0, stream>>>(out, ws, PN, splitk);
-  }
-}
-
-void launch_moe_combine(bf16* out, const bf16* y, const float* wts,
-                        const int* inv_pos, long T, int topk, int hidden,
-                        hipStream_t stream) {
-  if (hidden % 8)
-    throw std::runtime_error("moe_combine: hidden % 8 != 0");
-  moe_combine_kernel<<<dim3((unsigned)T), 256, 0, stream>>>(
-      out, y, wts, inv_pos, topk, hidden);
-}
-
-// ----------------------------------------------------- fp8 grouped GEMM
-// Same 256x128 3-deep-ring structure as moe_gemm_v3_kernel, e4m3fn:
-// out[p,n] = (sum_k A8[p,k] * B8[e,n,k]) * a_scale[row(p)] * b_scale[e,n]
-// via v_mfma_f32_32x32x16_fp8_fp8.  128-B staged rows = BK 128 fp8
-// elements (byte-identical loader geometry; kk 0..7 per chunk).
-typedef long long i64;
-
-__global__ __launch_bounds__(512) void moe_gemm_fp8_v3_kernel(
-    bf16* __restrict__ out, float* __restrict__ skw,
-    const unsigned char* __restrict__ xq,
-    const float* __restrict__ xs, const unsigned char* __restrict__ wq,
-    const float* __restrict__ ws, const int* __restrict__ sorted_ids,
-    const int* __restrict__ tile_expert, int N, int K, int gather_div,
-    int ntiles, int use_xcd, int splitk) {
-  constexpr int BN = 128;
-  const int nb_base = (int)(gridDim.x / (unsigned)splitk);
-  const int seg = (int)blockIdx.x / nb_base;
-  const TileMap tm =
-      xcd_tile_map((int)blockIdx.x % nb_base, ntiles, N / BN, use_xcd);
-  if (tm.t < 0) return;
-  const int e = tile_expert[tm.t];
-  if (e < 0) return;
-  const int m0 = tm.t * MOE_BM;
-  const int n0 = tm.j * BN;
-
-  extern __shared__ int lds[];     // shared decl w/ moe_align
-  unsigned char* dyn_lds = reinterpret_cast<unsigned char*>(lds);
-
-  const int tid = threadIdx.x;
-  const int wid = tid >> 6;
-  const int lane = tid & 63;
-  const int lcol = lane & 31;
-  const int lhalf = lane >> 5;
-  const int wave_m = wid & 3;
-  const int wave_n = wid >> 2;
-
-  const int lrow = lane >> 3;
-  const int gbyte = ((lane & 7) * 16) ^ (lrow << 4);
-  const unsigned char* a_src[4];
-  #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int r = wid * 32 + j * 8 + lrow;
-    long row = 0;
-    if (gather_div > 0) {
-      const int pair = sorted_ids[m0 + r];
-      if (pair >= 0) row = pair / gather_div;
-    } else {
-      row = m0 + r;
-    }
-    a_src[j] = xq + row * (long)K + gbyte;
-  }
-  const unsigned char* b_src[2];
-  #pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int r = wid * 16 + j * 8 + lrow;
-    b_src[j] = wq + ((long)e * N + n0 + r) * (long)K + gbyte;
-  }
-
-  f32x16 acc[2][2];
-  #pragma unroll
-  for (int sm = 0; sm < 2; ++sm)
-    #pragma unroll
-    for (int nb = 0; nb < 2; ++nb)
-      #pragma unroll
-      for (int i = 0; i < 16; ++i) acc[sm][nb][i] = 0.f;
-
-  // padding skip: a wave whose 64 output rows are ALL padding keeps its
-  // acc at zero and skips fragment reads + MFMAs (it still issues its
-  // glds share and hits every barrier — the tile stage is cooperative).
-  // ~1/3 of tile rows are padding at bs1024 (256-row align granularity)
-  bool wave_live = true;
-  if (gather_div > 0) {
-    wave_live = false;
-    #pragma unroll
-    for (int r = 0; r < 64; r += 16)        // 4 probes/lane cover 64 rows
-      if (sorted_ids[m0 + wave_m * 64 + r + (lane & 15)] >= 0)
-        wave_live = true;
-    wave_live = __any(wave_live);
-  }
-
-  auto stage = [&](int slot, int k0) {
-    const long cb = (long)k0;          // 1 B per fp8 element
-    #pragma unroll
-    for (int j = 0; j < 4; ++j)
-      glds16(a_src[j] + cb,
-             &dyn_lds[slot * 32768 + wid * 4096 + j * 1024]);
-    #pragma unroll
-    for (int j = 0; j < 2; ++j)
-      glds16(b_src[j] + cb,
-             &dyn_lds[98304 + slot * 16384 + wid * 2048 + j * 1024]);
-  };
-
-  auto compute = [&](int slot) {
-    if (!wave_live) return;
-    const int a_base = slot * 32768;
-    const int b_base = 98304 + slot * 16384;
-    #pragma unroll
-    for (int kk = 0; kk < 8; ++kk) {
-      i64 af[2];
-      #pragma unroll
-      for (int sm = 0; sm < 2; ++sm)
-        af[sm] = *reinterpret_cast<const i64*>(
-            &dyn_lds[a_base + swz(wave_m * 64 + sm * 32 + lcol,
-                                  kk * 16 + lhalf * 8)]);
-      #pragma unroll
-      for (int nb = 0; nb < 2; ++nb) {
-        i64 bf = *reinterpret_cast<const i64*>(
-            &dyn_lds[b_base + swz(wave_n * 64 + nb * 32 + lcol,
-                                  kk * 16 + lhalf * 8)]);
-        #pragma unroll
-        for (int sm = 0; sm < 2; ++sm)
-          acc[sm][nb] = __builtin_amdgcn_mfma_f32_32x32x16_fp8_fp8(
-              af[sm], bf, acc[sm][nb], 0, 0, 0);
-      }
-    }
-  };
-
-  const int nchunks = (K >> 7) / splitk;
-  const int c0 = seg * nchunks;
-  // same race-free 3-slot pipeline as the bf16 kernel
-  stage(0, c0 << 7);
-  stage(1, (c0 + 1) << 7);
-  asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  int d = 0;
-  for (; d + 2 < nchunks; ++d) {
-    compute(d % 3);
-    stage((d + 2) % 3, (c0 + d + 2) << 7);
-    asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-  }
-  compute(d % 3);
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  ++d;
-  compute(d % 3);
-
-  // epilogue: scale by a_scale[row] * b_scale[e, col], store bf16
-  // (split-K partials are stored ALREADY scaled, so the reduce is a sum)
-  const long P = (long)ntiles * MOE_BM;
-  #pragma unroll
-  for (int sm = 0; sm < 2; ++sm)
-    #pragma unroll
-    for (int nb = 0; nb < 2; ++nb) {
-      const int col = n0 + wave_n * 64 + nb * 32 + lcol;
-      const float bs = ws[(long)e * N + col];
-      #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int m = (r & 3) + 8 * (r >> 2) + 4 * lhalf;
-        const int p = m0 + wave_m * 64 + sm * 32 + m;
-        float as = 1.f;
-        if (gather_div > 0) {
-          const int pair = sorted_ids[p];
-          as = pair >= 0 ? xs[pair / gather_div] : 0.f;
-        } else {
-          as = xs[p];
-        }
-        const float v = acc[sm][nb][r] * as * bs;
-        if (splitk == 1)
-          *(unsigned short*)(out + (long)p * N + col) = f2bf(v);
-        else
-          skw[((long)seg * P + p) * N + col] = v;
-      }
-    }
-}
-
-void launch_moe_gemm_fp8(bf16* out, float* skw, const unsigned char* xq,
-                         const float* xs, const unsigned char* wq,
-                         const float* ws, const int* sorted_ids,
-                         const int* tile_expert, int ntiles_max, int N,
-                         int K, int gather_div, int splitk,
-                         hipStream_t stream) {
-  if (K % 128 || K < 256 || N % 128)
-    throw std::runtime_error("moe_gemm_fp8: bad K/N alignment");
-  if (splitk < 1 || (K >> 7) % splitk || ((K >> 7) / splitk) < 2 ||
-      (splitk > 1 && !skw))
-    throw std::runtime_error("moe_gemm_fp8: bad splitk");
-  const int lds_bytes = 3 * (32 * 1024 + 16 * 1024);
-  static bool attr_set = false;
-  if (!attr_set) {
-    (void)hipFuncSetAttribute(
-        reinterpret_cast<const void*>(&moe_gemm_fp8_v3_kernel),
-        hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
-    attr_set = true;
-  }
-  static const int use_xcd = [] {
-    const char* v = getenv("HS_MOE_XCD");
-    return v ? atoi(v) : 0;
-  }();
-  const int nx = N / 128;
-  const long nblocks = use_xcd
-      ? 8L * 32 * ((ntiles_max + 7) / 8) * ((nx + 31) / 32)
-      : (long)nx * ntiles_max;
-  moe_gemm_fp8_v3_kernel<<<dim3((unsigned)(nblocks * splitk)), 512,
-                           lds_bytes, stream>>>(
-      out, skw, xq, xs, wq, ws, sorted_ids, tile_expert, N, K,
-      gather_div, ntiles_max, use_xcd, splitk);
-  if (splitk > 1) {
-    const long PN = (long)ntiles_max * MOE_BM * N;
-    moe_sk_reduce_kernel<<<dim3((unsigned)((PN / 4 + 255) / 256)), 256,
-                           0, stream>>>(out, skw, PN, splitk);
   }
 }

@@ -281,38 +281,44 @@ def moe_router(x, router: torch.Tensor, top: int):
     return weight, ids
 
 
-# Rows per expert up to which tiles of 16 to 64 rows beside the streamed weights
-# are faster than the 256-row tiles, in us on an MI355X:
-#   experts of 14336 x 4096  1 row 274 : 463, 48 rows 788 : 831, 64 1049 : 846
-#   32 of 1024 x 2048        1 row  54 : 157, 64 rows 180 : 277, 128 269 : 305
-#   16 of 2048 x 4096        1 row 132 : 273, 64 rows 335 : 378,  96 397 : 391
-# The large tiles are late where they leave compute units without one.
-MOE_ROWS = 48
-MOE_ROWS_FEW = 95
+# Mean rows per expert up to which tiles of 16, 64 and 128 rows are taken (and
+# 256 beyond).  64 and 128 leave room for the spread of the counts: a few rows
+# more and an expert's weights are read twice.  us on an MI355X for tiles of
+#   16 (rows), 64, 128, 256
+#   8 experts of 14336 x 4096   4 rows 544 536 565 710, 48 1723 543 589 732,
+#     64 - 665 594 728, 96 - 798 601 762, 150 - 1118 937 729
+#   16 of 2048 x 4096           4 rows 175 202 204 223, 16 254 202 207 230
+#   32 of 1024 x 2048           2 rows 93 92 102 116, 64 321 119 118 137
+MOE_ROWS, MOE_ROWS_64, MOE_ROWS_128 = 6, 52, 112
 
 
-def _moe_rows(T: int, K: int, E: int, H: int, I: int) -> bool:
-    most = MOE_ROWS_FEW if E * (2 * I // 128) < 1024 else MOE_ROWS
-    return T * K <= most * E and H % 128 == 0 and I % 128 == 0 and E <= 64
+def _moe_tile(T: int, K: int, E: int, least: int) -> int:
+    mean = T * K / E
+    if mean <= MOE_ROWS and least <= 16:
+        return 16
+    return 64 if mean <= MOE_ROWS_64 else 128 if mean <= MOE_ROWS_128 else 256
 
 
-def _moe_ffn_rows(x, w13, w2, weights, ids):
-    n = _native()
-    (T, H), K, (E, _, I) = x.shape, ids.shape[1], w2.shape
-    pairs, mean = T * K, T * K / E
-    bm = 16 if mean <= 8 else 32 if mean <= 16 else 64
+def _moe_sort(ids: torch.Tensor, E: int, H: int, I: int, bm: int):
+    """(order, expert, place) of the choices `ids` [T, K], sorted in tiles of
+    bm rows; refuses what the tiles cannot take."""
+    if E > 64 or H % 128 or I % 128:
+        raise RuntimeError(f"moe: {E} experts of {I} x {H}: at most 64, and "
+                           "sizes that are multiples of 128")
+    pairs = ids.numel()
     tiles = min(pairs, (pairs + E * (bm - 1)) // bm)
-    i32 = lambda m: torch.empty(m, dtype=torch.int32, device=x.device)
-    order, expert, place = i32(tiles * bm), i32(tiles), i32(pairs)
-    n.experts_sort(order, expert, place, ids.reshape(-1).to(torch.int32), E,
-                   bm)
-    h = torch.empty(tiles * bm, I, dtype=x.dtype, device=x.device)
-    y = torch.empty(tiles * bm, H, dtype=x.dtype, device=x.device)
-    n.experts_up(h, x, w13, None, order, expert, K, None, bm)
-    n.experts_down(y, h, w2, None, order, expert, bm)
-    out = torch.empty(T, H, dtype=x.dtype, device=x.device)
-    n.experts_sum(out, y, place.view(T, K), weights.float().contiguous(),
-                  None, None, None, None, 0.0)
+    i32 = lambda *s: torch.empty(*s, dtype=torch.int32, device=ids.device)
+    order, expert, place = i32(tiles * bm), i32(tiles), i32(*ids.shape)
+    _native().experts_sort(order, expert, place,
+                           ids.reshape(-1).to(torch.int32), E, bm)
+    return order, expert, place
+
+
+def _moe_sum(y, place, weights) -> torch.Tensor:
+    out = torch.empty(place.shape[0], y.shape[1], dtype=y.dtype,
+                      device=y.device)
+    _native().experts_sum(out, y, place, weights.float().contiguous(), None,
+                          None, None, None, 0.0)
     return out
 
 
@@ -324,35 +330,24 @@ def moe_ffn(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor,
     routing weights; ids [T,K] LOCAL expert indices.  Token->expert sorting,
     the two grouped MFMA GEMMs and the weighted combine all run on-device
     with grids that depend only on (T, K, E) — no host sync, no dynamic
-    shapes (SURVEY.md §2.9: MoE dispatch/combine + grouped GEMM).
+    shapes (MoE dispatch/combine + grouped GEMM).
     """
-    T, H = x.shape
-    K = ids.shape[1]
-    E = w13.shape[0]
-    TK = T * K
-    if x.is_contiguous() and _moe_rows(T, K, E, H, w2.shape[2]):
-        return _moe_ffn_rows(x, w13, w2, weights, ids)
-    ntiles = (TK + E * (MOE_BM - 1) + MOE_BM - 1) // MOE_BM
-    P = ntiles * MOE_BM
-    dev = x.device
-    flat = ids.reshape(-1).to(torch.int32)
-    sorted_ids = torch.empty(P, dtype=torch.int32, device=dev)
-    tile_expert = torch.empty(ntiles, dtype=torch.int32, device=dev)
-    inv_pos = torch.empty(TK, dtype=torch.int32, device=dev)
     n = _native()
-    n.moe_align(sorted_ids, tile_expert, inv_pos, flat, E)
-    I2 = w13.shape[1]
-    h1 = torch.empty(P, I2, dtype=torch.bfloat16, device=dev)
-    s1, ws1 = _moe_splitk(ntiles * (I2 // 128), H // 64, P * I2, dev)
-    n.moe_gemm(h1, x, w13, sorted_ids, tile_expert, K, s1, ws1)
-    a = silu_mul(h1)
-    y = torch.empty(P, H, dtype=torch.bfloat16, device=dev)
-    I = w2.shape[2]
-    s2, ws2 = _moe_splitk(ntiles * (H // 128), I // 64, P * H, dev)
-    n.moe_gemm(y, a, w2, sorted_ids, tile_expert, 0, s2, ws2)
-    out = torch.empty(T, H, dtype=torch.bfloat16, device=dev)
-    n.moe_combine(out, y, weights.float().contiguous(), inv_pos, K)
-    return out
+    (T, H), K, (E, _, I) = x.shape, ids.shape[1], w2.shape
+    if T == 0:
+        return torch.empty_like(x)
+    bm = _moe_tile(T, K, E, 16)
+    order, expert, place = _moe_sort(ids, E, H, I, bm)
+    P = order.shape[0]
+    h = torch.empty(P, I, dtype=torch.bfloat16, device=x.device)
+    y = torch.empty(P, H, dtype=torch.bfloat16, device=x.device)
+    if bm == 16:
+        n.experts_up(h, x, w13, None, order, expert, K, None, bm)
+        n.experts_down(y, h, w2, None, order, expert, bm)
+    else:
+        n.experts_tiles(h, x, w13, None, None, order, expert, True, K, bm)
+        n.experts_tiles(y, h, w2, None, None, order, expert, False, 0, bm)
+    return _moe_sum(y, place, weights)
 
 
 def moe_ffn_fp8(xq: "QTensor", w13q: torch.Tensor, w13s: torch.Tensor,
@@ -361,35 +356,22 @@ def moe_ffn_fp8(xq: "QTensor", w13q: torch.Tensor, w13s: torch.Tensor,
     """fp8 grouped expert FFN: e4m3fn activations (QTensor from the fused
     norm producer) x e4m3fn expert weights through
     v_mfma_f32_32x32x16_fp8_fp8; the silu stage re-quantizes via the fused
-    silu_mul_fp8 kernel so no extra passes appear.  ~2x the bf16 MoE
-    weight bandwidth (the binding constraint, profiles/r01)."""
-    T, H = xq.data.shape
-    K = ids.shape[1]
-    E = w13q.shape[0]
-    TK = T * K
-    ntiles = (TK + E * (MOE_BM - 1) + MOE_BM - 1) // MOE_BM
-    P = ntiles * MOE_BM
-    dev = xq.data.device
-    flat = ids.reshape(-1).to(torch.int32)
-    sorted_ids = torch.empty(P, dtype=torch.int32, device=dev)
-    tile_expert = torch.empty(ntiles, dtype=torch.int32, device=dev)
-    inv_pos = torch.empty(TK, dtype=torch.int32, device=dev)
+    silu_mul_fp8 kernel so no extra passes appear."""
     n = _native()
-    n.moe_align(sorted_ids, tile_expert, inv_pos, flat, E)
-    I2 = w13q.shape[1]
-    h1 = torch.empty(P, I2, dtype=torch.bfloat16, device=dev)
-    s1, ws1 = _moe_splitk(ntiles * (I2 // 128), H // 128, P * I2, dev)
-    n.moe_gemm_fp8(h1, xq.data, xq.scale, w13q, w13s, sorted_ids,
-                   tile_expert, K, s1, ws1)
-    a = silu_mul_q(h1)
-    y = torch.empty(P, H, dtype=torch.bfloat16, device=dev)
-    I = w2q.shape[2]
-    s2, ws2 = _moe_splitk(ntiles * (H // 128), I // 128, P * H, dev)
-    n.moe_gemm_fp8(y, a.data, a.scale, w2q, w2s, sorted_ids, tile_expert,
-                   0, s2, ws2)
-    out = torch.empty(T, H, dtype=torch.bfloat16, device=dev)
-    n.moe_combine(out, y, weights.float().contiguous(), inv_pos, K)
-    return out
+    (T, H), K, (E, _, I) = xq.data.shape, ids.shape[1], w2q.shape
+    if T == 0:
+        return torch.empty(0, H, dtype=torch.bfloat16, device=xq.data.device)
+    bm = _moe_tile(T, K, E, 64)
+    order, expert, place = _moe_sort(ids, E, H, I, bm)
+    P = order.shape[0]
+    new = lambda m: torch.empty(P, m, dtype=torch.bfloat16,
+                                device=xq.data.device)
+    h, y = new(2 * I), new(H)
+    n.experts_tiles(h, xq.data, w13q, xq.scale, w13s, order, expert, False, K,
+                    bm)
+    a = silu_mul_q(h)
+    n.experts_tiles(y, a.data, w2q, a.scale, w2s, order, expert, False, 0, bm)
+    return _moe_sum(y, place, weights)
 
 
 def decode_inputs(stage: torch.Tensor, rows: int, cap: int, pages: int,

@@ -1,5 +1,5 @@
-"""Router kernel and grouped experts at both sides of the rule that chooses
-between row tiles and 256-row tiles, against float64.
+"""Router kernel and grouped experts at both sides of the rules that choose
+tiles of 16, 64, 128 and 256 rows, against float64.
 
 Bounds: the router's products are exact in float and summed in float (2^-22 of
 the sum of magnitudes); experts round their inner activation and their output
@@ -39,7 +39,7 @@ def test_router(tokens, experts, top, width, fp8):
     assert (weight.double() - ref).abs().max() <= 4 * slack + 1e-6
 
 
-@pytest.mark.parametrize("tokens", [1, 2, 33, 95, 96, 97, 191, 192, 193, 400])
+@pytest.mark.parametrize("tokens", [1, 2, 12, 13, 64, 104, 105, 224, 225, 416, 600])
 @pytest.mark.parametrize("experts,top,width,inner", [
     (4, 2, 256, 128), (8, 1, 128, 384), (2, 2, 384, 32768)])
 def test_experts_around_the_rule(tokens, experts, top, width, inner):
@@ -62,3 +62,41 @@ def test_experts_around_the_rule(tokens, experts, top, width, inner):
         ref += y * (weight * (ids == e)).sum(-1)[:, None].double()
     assert (out - ref).norm() <= 2.0 ** -7 * ref.norm()
     assert (out - ref).abs().max() <= 2.0 ** -5 * ref.abs().max()
+
+
+@pytest.mark.parametrize("tokens", [1, 26, 27, 56, 57, 300])
+@pytest.mark.parametrize("experts,top,width,inner", [
+    (4, 2, 256, 384), (3, 1, 1024, 256)])
+def test_experts_with_8_bits(tokens, experts, top, width, inner):
+    """Against float64 on the quantized operands.  The inner activation is
+    rounded to e4m3: a step of at most 2^-3 of a value, 2^-4 / sqrt(3) of it on
+    average, and of the sum of such."""
+    from hyperspot.parallel.layers import quantize_weight_fp8
+    g = torch.Generator().manual_seed(tokens)
+    rand = lambda *s: torch.randn(*s, generator=g).to(DEV)
+    xq = ops.quant_fp8(rand(tokens, width).bfloat16())
+    w13, s13, w2, s2 = (torch.stack(t) for t in zip(*(
+        quantize_weight_fp8(rand(2 * inner, width) * width ** -0.5)
+        + quantize_weight_fp8(rand(width, inner) * inner ** -0.5)
+        for _ in range(experts))))
+    ids = rand(tokens, experts).topk(top, -1).indices.int()
+    weight = rand(tokens, top).abs()
+    out = ops.moe_ffn_fp8(xq, w13, s13, w2, s2, weight, ids).double()
+    x = xq.data.double() * xq.scale.double()[:, None]
+    ref = torch.zeros_like(out)
+    for e in range(experts):
+        gate, up = (x @ (w13[e].double() * s13[e].double()[:, None]).t()) \
+            .chunk(2, -1)
+        y = torch.nn.functional.silu(gate) * up \
+            @ (w2[e].double() * s2[e].double()[:, None]).t()
+        ref += y * (weight * (ids == e)).sum(-1)[:, None].double()
+    assert (out - ref).norm() <= 2.0 ** -4.5 * ref.norm()
+
+
+def test_refused_sizes():
+    x = torch.zeros(3, 192, device=DEV).bfloat16()
+    w13, w2 = (torch.zeros(2, *s, device=DEV).bfloat16()
+               for s in ((256, 192), (192, 128)))
+    ids = torch.zeros(3, 1, dtype=torch.int32, device=DEV)
+    with pytest.raises(RuntimeError):
+        ops.moe_ffn(x, w13, w2, torch.ones(3, 1, device=DEV), ids)
