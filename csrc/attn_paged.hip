@@ -226,7 +226,7 @@ __global__ __launch_bounds__(256) void paged_attn_kernel(
 // few they are.  Scores are formed transposed, S^T = K Q^T, with the K row
 // that feeds matrix row i permuted so that the scores a lane holds are 8
 // consecutive tokens of one head, the operand P^T of O^T = V^T P^T; the
-// weights enter as a bf16 high and low part.  K goes from memory to its
+// weights, floats, enter as three bf16 parts.  K goes from memory to its
 // operands; V is turned by an LDS tile of the wave's own and the transposing
 // LDS load, e4m3 pages are widened on the way.  A wave has 32 tokens at a time
 // and issues the next ones' loads as soon as these are in their operands; no
@@ -432,16 +432,16 @@ __global__ __launch_bounds__(256, 3) void paged_attn_mfma_kernel(Paged a) {
       p[j] = exp2_fast(p[j] - base);
       l += p[j];
     }
-    short8_t ph, pl;
-    split_bf16x8(p, &ph, &pl);
+    short8_t part[3];
+    split_bf16x8<3>(p, part);
     #pragma unroll
     for (int e = 0; e < 8; ++e) {
       union { short4_t h[2]; short8_t v; } vf;
       // row + 4: the same units; column block e: two units on
       vf.h[0] = lds_read_tr(vl + (v_at ^ e << 5));
       vf.h[1] = lds_read_tr(vl + (v_at ^ e << 5) + 4 * 256);
-      acc[e] = mfma16(vf.v, ph, acc[e]);
-      acc[e] = mfma16(vf.v, pl, acc[e]);
+      #pragma unroll
+      for (int n = 0; n < 3; ++n) acc[e] = mfma16(vf.v, part[n], acc[e]);
     }
   }
   l += __shfl_xor(l, 16);

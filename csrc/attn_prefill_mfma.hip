@@ -15,8 +15,8 @@
 // consecutive tokens of one query row, which is the operand P^T of
 // O^T = V^T P^T: weights never leave their registers, and the running maximum
 // and its rescaling are one value a lane.  The rescaling is left out while no
-// row's maximum grew by more than 2^GROW.  V^T is read with the transposing
-// LDS load.
+// row's maximum grew (pages: by more than 2^GROW).  V^T is read with the
+// transposing LDS load.
 //
 // A workgroup is 4 waves of 32 rows: HG heads of one kv head share a tile of
 // 64 tokens, so that the causal edge of 4 heads costs 32 rows of work and not
@@ -31,9 +31,11 @@
 // (209); 8 prompts of 1000, 113 us; 7808 tokens after 8192 cached ones 2.22 ms
 // (696 TFLOP/s) where one workgroup a row took 37.6.
 //
-// Weights enter the matrix cores as one bf16 (ROWS), or as a high and a low
-// part (pages: about 16 bits, which the row-by-row kernel's float weights
-// need).
+// ROWS: weights are rounded to bf16, relative to the maximum after each tile of
+// 64 tokens, and summed in a fixed order.  Both are a part of the result: a
+// model with 8-bit activations rounds it to few steps again, and a last bit
+// decides between two of them.  Pages: the weights are floats in the row-by-row kernel, so they enter
+// as a high and a low part (16 bits), with e4m3 pages as three (24 bits).
 #include <float.h>
 
 #include "common.h"
@@ -60,8 +62,8 @@ struct Prefill {
   const int* ctx_lens;       // pages only
   const int* block_tables;
   int seqs, H, G, max_blocks, min_rows;
-  float scale;               // times log2(e), positive: its sign, or a scale
-  short q_and, q_xor;        // of zero, is applied to the bits of q
+  float scale;               // positive: its sign, or a scale of zero, is
+  short q_and, q_xor;        // applied to the bits of q; pages: times log2(e)
   long sq, sk, sv;           // strides of a row
 };
 
@@ -79,6 +81,20 @@ DEV void to_lds16(const void* g, void* l) {
 DEV short4_t lds_read_tr(const short* p) {
   return __builtin_amdgcn_ds_read_tr16_b64_v4i16(
       (__attribute__((address_space(3))) short4_t*)p);
+}
+
+// not to become a part of a fused operation
+DEV float product(float x, float y) {
+  #pragma clang fp contract(off)
+  return x * y;
+}
+
+// x of the upper half of the lanes against y of the lower
+DEV void swap_halves(float& x, float& y) {
+  const auto r = __builtin_amdgcn_permlane32_swap(
+      __float_as_uint(x), __float_as_uint(y), false, false);
+  x = __uint_as_float(r[0]);
+  y = __uint_as_float(r[1]);
 }
 
 // of the lanes i and i ^ 32
@@ -104,7 +120,8 @@ template <int HG, int SRC>
 __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(Prefill a) {
   constexpr int RG = 4 / HG;                 // row groups of 32
   constexpr int TILE_ROWS = RG * WAVE_ROWS;
-  constexpr bool SPLIT = SRC != ROWS;
+  constexpr int PARTS = SRC == ROWS ? 1 : SRC == PAGES ? 2 : 3;
+  constexpr bool EACH = SRC == ROWS;         // rescale at each tile
   __shared__ __attribute__((aligned(16))) short lds[2][2][KV * HD];
 
   // Sequence s has the places seq_start[s] / TILE_ROWS + s and up, as many
@@ -252,17 +269,19 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(Prefill a) {
       #pragma unroll
       for (int r = 0; r < 16; ++r) mx = fmaxf(mx, sc[b][r]);
     mx = max_halves(mx) * a.scale;
-    if (__any(mx > m + GROW)) {
+    float alpha = 1.f;
+    if (__any(mx > (EACH ? m : m + GROW))) {
       const float top = fmaxf(m, mx);
-      const float alpha = m == -FLT_MAX ? 0.f : exp2_fast(m - top);
+      alpha = m == -FLT_MAX ? 0.f
+              : EACH ? __expf(m - top) : exp2_fast(m - top);
       #pragma unroll
       for (int e = 0; e < 4; ++e)
         #pragma unroll
         for (int r = 0; r < 16; ++r) acc[e][r] *= alpha;
-      l *= alpha;
       m = top;
     }
     const float base = m == -FLT_MAX ? 0.f : m;
+    float sum = 0.f;
     __builtin_amdgcn_sched_barrier(0);
     #pragma unroll
     for (int b = 0; b < 2; ++b)
@@ -271,18 +290,18 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(Prefill a) {
         float p[8];
         #pragma unroll
         for (int j = 0; j < 8; ++j) {
-          p[j] = exp2_fast(fmaf(sc[b][c * 8 + j], a.scale, -base));
-          l += p[j];
+          p[j] = EACH ? __expf(product(sc[b][c * 8 + j], a.scale) - base)
+                      : exp2_fast(fmaf(sc[b][c * 8 + j], a.scale, -base));
+          if constexpr (!EACH) sum += p[j];
         }
-        short8_t ph, pl;
-        if constexpr (SPLIT) {
-          split_bf16x8(p, &ph, &pl);
-        } else {
-          union { unsigned u[4]; short8_t v; } x;
+        short8_t part[PARTS];
+        split_bf16x8<PARTS>(p, part);
+        if constexpr (EACH) {
+          // a lane sums 4 of every 8 tokens: t .. t + 3, t + 8 .. t + 11
           #pragma unroll
-          for (int j = 0; j < 4; ++j)
-            x.u[j] = cvt_pk_bf16(p[2 * j], p[2 * j + 1]);
-          ph = x.v;
+          for (int j = 0; j < 4; ++j) swap_halves(p[j], p[4 + j]);
+          #pragma unroll
+          for (int j = 0; j < 8; ++j) sum += p[j];
         }
         #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -291,11 +310,18 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(Prefill a) {
           for (int i = 0; i < 2; ++i)
             vf.h[i] = lds_read_tr(reinterpret_cast<const short*>(
                 vl + (v_at ^ e << 6) + (b * 32 + c * 16 + i * 4) * HD * 2));
-          acc[e] = mfma32(vf.v, ph, acc[e]);
-          if constexpr (SPLIT) acc[e] = mfma32(vf.v, pl, acc[e]);
+          #pragma unroll
+          for (int n = 0; n < PARTS; ++n)
+            acc[e] = mfma32(vf.v, part[n], acc[e]);
         }
         if (c) __builtin_amdgcn_sched_barrier(0);
       }
+    if constexpr (EACH) {            // both halves, as the maximum
+      float other = sum;
+      swap_halves(sum, other);
+      sum += other;
+    }
+    l = fmaf(l, alpha, sum);
   };
 
   auto landed = [&](int buf) {
@@ -318,11 +344,10 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(Prefill a) {
     if (more) landed(buf ^ 1);
   }
 
-  l += __shfl_xor(l, 32);
+  if constexpr (!EACH) l += __shfl_xor(l, 32);
   if (row >= n) return;
   // acc[e][r]: column e * 32 + (r >> 2) * 8 + hf * 4 + (r & 3)
   const bool none = SRC == ROWS && !(l > 0.f);
-  const float inv = 1.f / l;
   bf16* op = a.out + ((long)(t0 + row) * a.H + h) * HD + hf * 4;
   #pragma unroll
   for (int e = 0; e < 4; ++e)
@@ -330,7 +355,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(Prefill a) {
     for (int r = 0; r < 16; r += 4) {
       float x[4];
       #pragma unroll
-      for (int j = 0; j < 4; ++j) x[j] = none ? 0.f : acc[e][r + j] * inv;
+      for (int j = 0; j < 4; ++j) x[j] = none ? 0.f : acc[e][r + j] / l;
       *reinterpret_cast<uint2*>(op + e * 32 + r * 2) =
           uint2{cvt_pk_bf16(x[0], x[1]), cvt_pk_bf16(x[2], x[3])};
     }
@@ -342,7 +367,8 @@ void launch(const Prefill& p, long rows, hipStream_t stream) {
   Prefill a = p;
   a.q_and = a.scale == 0.f ? 0 : -1;
   a.q_xor = a.scale < 0.f ? (short)0x8000 : 0;
-  a.scale = a.scale == 0.f ? 1.f : fabsf(a.scale) * LOG2E;
+  a.scale = a.scale == 0.f ? 1.f : fabsf(a.scale);
+  if (SRC != ROWS) a.scale *= LOG2E;
   const int group = a.H / a.G;
   #define RUN(HG)                                                           \
     attn_prefill_kernel<HG, SRC>                                            \

@@ -164,6 +164,25 @@ DEV void split_bf16x8(const float* f, short8_t* hi, short8_t* lo) {
   *lo = l.v;
 }
 
+// f = the sum of N bf16 operands: 8 bits of mantissa each, so that three hold
+// a float
+template <int N> DEV void split_bf16x8(const float* f, short8_t* part) {
+  float r[8];
+  #pragma unroll
+  for (int i = 0; i < 8; ++i) r[i] = f[i];
+  #pragma unroll
+  for (int n = 0; n < N; ++n) {
+    union { unsigned u[4]; short8_t v; } x;
+    #pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      x.u[i] = cvt_pk_bf16(r[2 * i], r[2 * i + 1]);
+      r[2 * i] -= bf2f((unsigned short)(x.u[i] & 0xffff));
+      r[2 * i + 1] -= bf2f((unsigned short)(x.u[i] >> 16));
+    }
+    part[n] = x.v;
+  }
+}
+
 DEV float bf16x8_at(const short8_t& v, int i) {
   return bf2f((unsigned short)v[i]);
 }

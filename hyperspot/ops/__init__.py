@@ -115,12 +115,12 @@ def paged_attn_decode(q: torch.Tensor, k_cache: torch.Tensor,
                                        seq_lens, scale)
 
 
-# Portions of at least this many rows attend on the matrix cores.  A tile of
-# 32 rows costs what it costs for one row, and has no other workgroups to share
-# its keys with; the row-by-row kernel reads the keys once per row, but spreads
-# them over more workgroups.  16 rows after 16000 tokens: 387 us against 473;
-# after 1000: 29 us against 35; 8 kv heads of 4 query heads.
-PORTION_ROWS = 16
+# Portions of at least this many rows attend on tiles of 32 rows, the others row
+# by row.  A tile takes a context's latency whatever it holds, a row its share
+# of the memory: one portion of 16, 64, 96 rows after 1000 tokens takes 31, 33,
+# 34 us in tiles and 15, 25, 35 by rows, after 16000 399, 402, 408 and 147,
+# 306, 447 (8 kv heads of 4).  Beside others tiles share the latency.
+PORTION_ROWS, PORTION_ROWS_ALONE = 16, 80
 
 
 def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
@@ -144,10 +144,12 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
                                         meta.max_seqlen, scale)
         elif q.shape[-1] == 128 and meta.seq_start is not None \
                 and q.shape[1] // k_cache.shape[1] in (1, 2, 4, 8):
+            least = PORTION_ROWS_ALONE if q.shape[0] < PORTION_ROWS_ALONE \
+                else PORTION_ROWS
             _native().attn_portions(
                 out, q, k_cache, v_cache, meta.block_tables, meta.ctx_lens,
-                meta.row_seq, meta.seq_start, PORTION_ROWS,
-                getattr(meta, "min_seqlen", 0) < PORTION_ROWS, scale)
+                meta.row_seq, meta.seq_start, least,
+                getattr(meta, "min_seqlen", 0) < least, scale)
         else:
             # row by row: odd head dims
             _native().paged_attn(out, q, k_cache, v_cache,

@@ -39,7 +39,7 @@ def _check(out, ref, weight_step):
 @pytest.mark.parametrize("portions", [
     [(0, 16), (16, 17), (47, 63), (64, 1)],     # (before, rows)
     [(100, 130), (0, 64), (3, 15), (200, 32)],
-    [(1, 257)],
+    [(1, 257)], [(40, 79)], [(40, 80)],
 ])
 def test_portions_over_pages(portions, group, kv, fp8):
     g = torch.Generator().manual_seed(3)
