@@ -237,6 +237,15 @@ __global__ __launch_bounds__(256) void paged_attn_kernel(
 // e4m3 pages 214 -> 110; 64 rows 77 -> 59, e4m3 71 -> 32; 8 rows of 8000 in 4
 // parts 122 -> 61; 64 rows x 1 kv head of 8 in 4 parts 47 -> 16.
 //
+// ROPE: q and k come as the projection left them.  A lane turns its part of q
+// in its registers; the wave that has the row's last token turns k and stores
+// it and v before it loads the last block.  A launch of its own for that is one
+// workgroup a token that goes to memory three times in a row, 5 us a layer;
+// here these loads pass beside the page ids and the first pages.  us of both
+// launches and of one: 1 row x 8 kv heads of 4, 1000 tokens 12.6 -> 10.1; 8 rows
+// of 8000 69 -> 63; 32 x 4 of 1000 27.7 -> 23.6; 256 x 8 of 1000 221 -> 206, of
+// 30 22.4 -> 21.9; e4m3 64 x 8 of 1000 38.5 -> 34.8.
+//
 // SPLIT > 1 (flash-decode): gridDim.z workgroups share one (row, kvh), each
 // with every gridDim.z-th 4 blocks of 32 tokens; their (o, m, l) land in
 // `partial` [rows, kvh, split, group, D + 2] and a second kernel merges them.
@@ -278,6 +287,11 @@ DEV u32x4 widen(unsigned x, unsigned y) {
   return u32x4{a.x, a.y, b.x, b.y};
 }
 
+// (x, y) by an angle, rounded as in rope_kv_append
+DEV float2 turn(float x, float y, float c, float s) {
+  return make_float2(fmaf(x, c, -(y * s)), fmaf(y, c, x * s));
+}
+
 struct Paged {
   bf16* out;
   const bf16* q;
@@ -292,9 +306,16 @@ struct Paged {
   float scale;               // times log2(e)
   long qs;
   float* partial;
+  // ROPE: rows are the last tokens of different sequences
+  const bf16* k;
+  const bf16* v;
+  const float* cos_sin;      // [positions, HD], cosines | sines
+  const long* positions;
+  const long* slots;         // -1: nothing is stored
+  long ks, vs;
 };
 
-template <bool KV8>
+template <bool KV8, bool ROPE>
 __global__ __launch_bounds__(256, 3) void paged_attn_mfma_kernel(Paged a) {
   __shared__ __attribute__((aligned(16))) char v_lds[4][BLOCK * HD * 2];
   __shared__ float m_lds[4][16], l_lds[4][16];
@@ -305,7 +326,9 @@ __global__ __launch_bounds__(256, 3) void paged_attn_mfma_kernel(Paged a) {
       a.seq_start[table + 1] - a.seq_start[table] > a.max_portion)
     return;
   const int ctx = a.ctx_lens[row];
-  const int* bt = a.block_tables + (long)table * a.max_blocks;
+  // scalar loads also after the stores to the pages
+  const auto bt = (const __attribute__((address_space(4))) int*)
+      (a.block_tables + (long)table * a.max_blocks);
   const int lane = threadIdx.x & 63;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 15, gr = lane >> 4;
@@ -322,6 +345,38 @@ __global__ __launch_bounds__(256, 3) void paged_attn_mfma_kernel(Paged a) {
               a.q + row * a.qs + (long)(g * group + col) * HD + d)
         : short8_t{};
   }
+  constexpr int ELEM = KV8 ? 1 : 2;
+  // to turn with, loaded before the first pages: of steps c and c + 2, columns
+  // d and d + 64; and by the wave that has the row's last token
+  f32x4_t co[2][2], si[2][2];
+  bool append = false;
+  float2 co_k, si_k;                 // lanes 0 to 31: columns j, j + 1 of k
+  unsigned lo = 0, hi = 0;           // and j + 64, j + 65; the others: 4 of v
+  long slot = -1;
+  const int j_new = lane % 32 * 2;
+  if constexpr (ROPE) {
+    const float* cs = a.cos_sin + a.positions[row] * HD;
+    slot = a.slots[row];
+    append = slot >= 0 &&
+             max(ctx - 1, 0) / BLOCK % (4 * split) == z * 4 + wid;
+    #pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      const int d = KV8 ? gr * 16 + c * 8 : c * 32 + gr * 8;
+      #pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        co[c][i] = *reinterpret_cast<const f32x4_t*>(cs + d + i * 4);
+        si[c][i] = *reinterpret_cast<const f32x4_t*>(cs + HD / 2 + d + i * 4);
+      }
+    }
+    if (append) {
+      co_k = *reinterpret_cast<const float2*>(cs + j_new);
+      si_k = *reinterpret_cast<const float2*>(cs + HD / 2 + j_new);
+      const bf16* p = lane < 32 ? a.k + row * a.ks + g * HD + j_new
+                                : a.v + row * a.vs + g * HD + j_new * 2;
+      lo = *reinterpret_cast<const unsigned*>(p);
+      hi = *reinterpret_cast<const unsigned*>(p + (lane < 32 ? HD / 2 : 2));
+    }
+  }
   f32x4_t acc[8];
   #pragma unroll
   for (int e = 0; e < 8; ++e) acc[e] = f32x4_t(0.f);
@@ -337,7 +392,6 @@ __global__ __launch_bounds__(256, 3) void paged_attn_mfma_kernel(Paged a) {
     b0 = bt[min(2 * i, last_page)];
     b1 = bt[min(2 * i + 1, last_page)];
   };
-  constexpr int ELEM = KV8 ? 1 : 2;
   u32x4 kr[2][KV8 ? 2 : 4], vr[KV8 ? 4 : 8];
   auto fetch = [&]() {
     const long p0 = (b0 * a.G + g) * (ATTN_BS * HD * ELEM);
@@ -364,10 +418,62 @@ __global__ __launch_bounds__(256, 3) void paged_attn_mfma_kernel(Paged a) {
   const int v_at = v_byte(vr0, (col & 3) >> 1) + (col & 1) * 8;
 
   int i = z * 4 + wid;
+  const bool at_once = !append || i + step < blocks;   // else stored first
   if (i < blocks) {
     pages(i);
-    fetch();
-    if (i + step < blocks) pages(i + step);
+    if (at_once) {
+      fetch();
+      if (i + step < blocks) pages(i + step);
+    }
+  }
+  if constexpr (ROPE) {
+    #pragma unroll
+    for (int c = 0; c < 2; ++c)
+      #pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const float x = bf2f((unsigned short)qf[c][i]);
+        const float y = bf2f((unsigned short)qf[c + 2][i]);
+        const float2 r = turn(x, y, co[c][i >> 2][i & 3],
+                              si[c][i >> 2][i & 3]);
+        qf[c][i] = (short)f2bf(r.x);
+        qf[c + 2][i] = (short)f2bf(r.y);
+      }
+    if (append) {
+      const long at =
+          ((slot / ATTN_BS * a.G + g) * ATTN_BS + slot % ATTN_BS) * HD * ELEM;
+      char* kp = static_cast<char*>(const_cast<void*>(a.k_cache)) + at;
+      char* vp = static_cast<char*>(const_cast<void*>(a.v_cache)) + at;
+      const int j = j_new;
+      const float x0 = __uint_as_float(lo << 16);
+      const float x1 = __uint_as_float(lo & 0xffff0000u);
+      const float y0 = __uint_as_float(hi << 16);
+      const float y1 = __uint_as_float(hi & 0xffff0000u);
+      if (lane < 32) {
+        const float2 t0 = turn(x0, y0, co_k.x, si_k.x);
+        const float2 t1 = turn(x1, y1, co_k.y, si_k.y);
+        if constexpr (KV8) {
+          *reinterpret_cast<unsigned short*>(kp + j) = (unsigned short)
+              __builtin_amdgcn_cvt_pk_fp8_f32(t0.x, t1.x, 0, false);
+          *reinterpret_cast<unsigned short*>(kp + HD / 2 + j) =
+              (unsigned short)__builtin_amdgcn_cvt_pk_fp8_f32(t0.y, t1.y, 0,
+                                                              false);
+        } else {
+          *reinterpret_cast<unsigned*>(kp + j * 2) = cvt_pk_bf16(t0.x, t1.x);
+          *reinterpret_cast<unsigned*>(kp + HD + j * 2) =
+              cvt_pk_bf16(t0.y, t1.y);
+        }
+      } else if constexpr (KV8) {
+        const int w = __builtin_amdgcn_cvt_pk_fp8_f32(x0, x1, 0, false);
+        *reinterpret_cast<int*>(vp + j * 2) =
+            __builtin_amdgcn_cvt_pk_fp8_f32(y0, y1, w, true);
+      } else {
+        *reinterpret_cast<uint2*>(vp + j * 4) = uint2{lo, hi};
+      }
+      if (!at_once && i < blocks) {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+        fetch();
+      }
+    }
   }
   for (; i < blocks; i += step) {
     f32x4_t sc[2];
@@ -401,6 +507,9 @@ __global__ __launch_bounds__(256, 3) void paged_attn_mfma_kernel(Paged a) {
         *reinterpret_cast<u32x4*>(vl + v_byte(4 * j + gr, col)) = vr[j];
     }
     if (i + step < blocks) {
+      // before the wave's last block: what it stored is in the page
+      if (ROPE && append && i + 2 * step >= blocks)
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
       fetch();
       if (i + 2 * step < blocks) pages(i + 2 * step);
     }
@@ -520,6 +629,21 @@ __global__ __launch_bounds__(256) void paged_attn_merge_kernel(
       cvt_pk_bf16(x * inv, y * inv);
 }
 
+template <bool ROPE>
+void launch_mfma(const Paged& a, long rows, int split, bool kv_fp8,
+                 hipStream_t stream) {
+  const dim3 grid((unsigned)rows, (unsigned)a.G, (unsigned)split);
+  if (kv_fp8)
+    paged_attn_mfma_kernel<true, ROPE><<<grid, 256, 0, stream>>>(a);
+  else
+    paged_attn_mfma_kernel<false, ROPE><<<grid, 256, 0, stream>>>(a);
+  if (split > 1) {
+    const long heads = rows * a.G * a.group;
+    paged_attn_merge_kernel<<<(unsigned)((heads + 3) / 4), 256, 0, stream>>>(
+        a.out, a.partial, split, a.group, heads);
+  }
+}
+
 }  // namespace
 
 // With seq_start (and row_seq) only the rows of sequences that have at most
@@ -537,20 +661,10 @@ void launch_paged_attn(bf16* out, const bf16* q, const bf16* k_cache,
   if (D == HD && (group <= 4 || group == 8)) {
     if (split > 64)
       throw std::runtime_error("paged_attn: at most 64 parts");
-    const Paged a{out, q, k_cache, v_cache, block_tables, ctx_lens, row_seq,
-                  seq_start, max_portion, max_blocks, num_kv_heads, group,
-                  scale * LOG2E, q_stride, split_ws};
-    const dim3 grid((unsigned)num_rows, (unsigned)num_kv_heads,
-                    (unsigned)split);
-    if (kv_fp8)
-      paged_attn_mfma_kernel<true><<<grid, 256, 0, stream>>>(a);
-    else
-      paged_attn_mfma_kernel<false><<<grid, 256, 0, stream>>>(a);
-    if (split > 1) {
-      const long heads = num_rows * num_kv_heads * group;
-      paged_attn_merge_kernel<<<(unsigned)((heads + 3) / 4), 256, 0,
-                                stream>>>(out, split_ws, split, group, heads);
-    }
+    launch_mfma<false>({out, q, k_cache, v_cache, block_tables, ctx_lens,
+                        row_seq, seq_start, max_portion, max_blocks,
+                        num_kv_heads, group, scale * LOG2E, q_stride,
+                        split_ws}, num_rows, split, kv_fp8, stream);
     return;
   }
   if (split != 1 || seq_start)
@@ -568,4 +682,22 @@ void launch_paged_attn(bf16* out, const bf16* q, const bf16* k_cache,
   CASE(1, 64) CASE(2, 64) CASE(4, 64) CASE(8, 64)
   #undef CASE
   throw std::runtime_error("paged_attn: unsupported (group, head_dim)");
+}
+
+// rope_kv_append and paged_attn of one token each of different sequences: q
+// [rows, kv heads * group, 128] as they come from the projection, rows 16-byte
+// aligned; q and k stay as they are.
+void launch_rope_paged_attn(bf16* out, const bf16* q, const bf16* k,
+                            const bf16* v, const long* positions,
+                            const float* cos_sin, const long* slots,
+                            bf16* k_cache, bf16* v_cache,
+                            const int* block_tables, const int* ctx_lens,
+                            long rows, int num_kv_heads, int group,
+                            int max_blocks, float scale, long qs, long ks,
+                            long vs, float* split_ws, int split, bool kv_fp8,
+                            hipStream_t stream) {
+  launch_mfma<true>({out, q, k_cache, v_cache, block_tables, ctx_lens, nullptr,
+                     nullptr, 0, max_blocks, num_kv_heads, group,
+                     scale * LOG2E, qs, split_ws, k, v, cos_sin, positions,
+                     slots, ks, vs}, rows, split, kv_fp8, stream);
 }

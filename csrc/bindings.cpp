@@ -20,6 +20,11 @@ void launch_paged_attn(bf16*, const bf16*, const bf16*, const bf16*,
                        const int*, const int*, const int*, long, int, int,
                        int, int, int, float, long, float*, int, bool,
                        const int*, int, hipStream_t);
+void launch_rope_paged_attn(bf16*, const bf16*, const bf16*, const bf16*,
+                            const long*, const float*, const long*, bf16*,
+                            bf16*, const int*, const int*, long, int, int,
+                            int, float, long, long, long, float*, int, bool,
+                            hipStream_t);
 void launch_attn_prefill_mfma(bf16*, const bf16*, const bf16*,
                               const bf16*, const int*, int, long, int, int,
                               int, float, long, long, long, hipStream_t);
@@ -209,6 +214,63 @@ void paged_attn(torch::Tensor out, torch::Tensor q, torch::Tensor k_cache,
                     rs, R, KV, H / KV, D, (int)block_tables.size(1), BS,
                     (float)scale, q.stride(0), ws, (int)split, kv_fp8,
                     nullptr, 0, stream());
+}
+
+// rope_kv_append and paged_attn in one launch; q and k stay as they are
+void rope_paged_attn(torch::Tensor out, torch::Tensor q, torch::Tensor k,
+                     torch::Tensor v, torch::Tensor positions,
+                     torch::Tensor cos_sin, torch::Tensor slot_mapping,
+                     torch::Tensor k_cache, torch::Tensor v_cache,
+                     torch::Tensor block_tables, torch::Tensor ctx_lens,
+                     double scale, c10::optional<torch::Tensor> split_ws,
+                     long split) {
+  check(out, torch::kBFloat16, "out");
+  for (const auto& t : {q, k, v}) {
+    check_qkv_view(t, "q, k, v");
+    TORCH_CHECK(t.stride(0) % 8 == 0 &&
+                    reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0,
+                "rope_paged_attn: rows of q, k, v must be 16-byte aligned");
+  }
+  check(cos_sin, torch::kFloat32, "cos_sin");
+  check(positions, torch::kInt64, "positions");
+  check(slot_mapping, torch::kInt64, "slot_mapping");
+  check(block_tables, torch::kInt32, "block_tables");
+  check(ctx_lens, torch::kInt32, "ctx_lens");
+  const long R = q.size(0);
+  const int H = (int)q.size(1), KV = (int)k.size(1);
+  TORCH_CHECK(KV > 0 && H % KV == 0, "GQA group");
+  const int group = H / KV;
+  TORCH_CHECK(group <= 4 || group == 8, "rope_paged_attn: group");
+  for (const auto& t : {k_cache, v_cache})
+    TORCH_CHECK(t.is_cuda() && t.is_contiguous() && t.dim() == 4 &&
+                    t.size(1) == KV && t.size(2) == 16 && t.size(3) == 128 &&
+                    t.scalar_type() == k_cache.scalar_type(),
+                "rope_paged_attn: k/v cache");
+  const bool kv_fp8 = k_cache.scalar_type() == torch::kFloat8_e4m3fn;
+  TORCH_CHECK(kv_fp8 || k_cache.scalar_type() == torch::kBFloat16,
+              "rope_paged_attn: k/v cache dtype");
+  TORCH_CHECK(q.size(2) == 128 && k.size(2) == 128 && v.size(2) == 128 &&
+                  k.size(0) == R && v.size(0) == R && v.size(1) == KV &&
+                  out.numel() == q.numel() && cos_sin.size(-1) == 128,
+              "rope_paged_attn: shape");
+  TORCH_CHECK(positions.numel() >= R && slot_mapping.numel() >= R &&
+                  ctx_lens.numel() >= R && block_tables.dim() == 2 &&
+                  block_tables.size(0) >= R, "rope_paged_attn: rows");
+  TORCH_CHECK(split >= 1 && split <= 64, "rope_paged_attn: 1 to 64 parts");
+  float* ws = nullptr;
+  if (split > 1) {
+    TORCH_CHECK(split_ws.has_value(), "split>1 needs a workspace");
+    check(*split_ws, torch::kFloat, "split_ws");
+    TORCH_CHECK(split_ws->numel() >= R * split * H * 130,
+                "split_ws too small");
+    ws = split_ws->data_ptr<float>();
+  }
+  launch_rope_paged_attn(
+      bf(out), cbf(q), cbf(k), cbf(v), positions.data_ptr<long>(),
+      cos_sin.data_ptr<float>(), slot_mapping.data_ptr<long>(), bf(k_cache),
+      bf(v_cache), block_tables.data_ptr<int>(), ctx_lens.data_ptr<int>(), R,
+      KV, group, (int)block_tables.size(1), (float)scale, q.stride(0),
+      k.stride(0), v.stride(0), ws, (int)split, kv_fp8, stream());
 }
 
 void attn_prefill_mfma(torch::Tensor out, torch::Tensor q, torch::Tensor k,
@@ -1027,6 +1089,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("fused_add_rmsnorm", &fused_add_rmsnorm);
   m.def("rope_kv_append", &rope_kv_append);
   m.def("paged_attn", &paged_attn);
+  m.def("rope_paged_attn", &rope_paged_attn);
   m.def("attn_prefill_mfma", &attn_prefill_mfma);
   m.def("attn_portions", &attn_portions);
   m.def("decode_inputs", &decode_inputs);

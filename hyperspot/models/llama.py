@@ -114,9 +114,9 @@ class Attention(nn.Module):
         q, k, v = self.qkv(x)
         T = q.shape[0]
         k_cache, v_cache = kv_cache[0], kv_cache[1]
-        ops.rope_kv_append(q, k, v, meta.positions, cos_sin,
-                           meta.slot_mapping, k_cache, v_cache)
-        o = ops.attention(q, k, v, k_cache, v_cache, meta, self.scale)
+        o = ops.rope_attention(q, k, v, meta.positions, cos_sin,
+                               meta.slot_mapping, k_cache, v_cache, meta,
+                               self.scale)
         o = o.view(T, -1)
         if self.o_proj.quant == "fp8" and o.is_cuda:
             o = ops.quant_fp8(o)   # fused amax+scale+pack (csrc/quant.hip)

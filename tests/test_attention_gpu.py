@@ -129,3 +129,50 @@ def test_decode_over_pages(split, group, kv, fp8):
                 for c in (kc, vc))
         _check(out[i:i + 1], _reference(q[i:i + 1], k, v, n - 1, D ** -0.5),
                2.0 ** -14)
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("group,kv", [(4, 2), (8, 1), (3, 2), (2, 3), (1, 4)])
+@pytest.mark.parametrize("lens", [
+    [1, 16, 17, 31, 32, 33], [127, 128, 129, 500, 2], [700],
+    list(range(1, 131)),                        # one part
+])
+def test_rope_in_decode_attention(lens, group, kv, fp8):
+    """Against the two launches: the same bytes in the pages; a row without a
+    slot leaves them and attends over what they hold.  A turned value may fall
+    on the other side of a rounding to bf16 (2^-8 of it, of outputs of about
+    one)."""
+    g = torch.Generator().manual_seed(5)
+    n, heads = len(lens), group * kv
+    kind = torch.float8_e4m3fn if fp8 else torch.bfloat16
+    tables = [-(-x // 16) for x in lens]
+    order = torch.randperm(sum(tables), generator=g).int()
+    caches = [torch.randn(sum(tables), kv, 16, D, generator=g).to(kind).to(DEV)
+              for _ in range(2)]
+    bt = torch.zeros(n, max(tables), dtype=torch.int32)
+    slots, at = [], 0
+    for i, (x, t) in enumerate(zip(lens, tables)):
+        bt[i, :t] = order[at:at + t]
+        at += t
+        slots.append(int(bt[i, t - 1]) * 16 + (x - 1) % 16 if i != 1 else -1)
+    ang = torch.rand(1000, D // 2, generator=g) * 6.3
+    cos_sin = torch.cat([ang.cos(), ang.sin()], -1).to(DEV)
+    lens, slots = torch.tensor(lens), torch.tensor(slots).to(DEV)
+    meta = ForwardMeta("decode", (lens - 1).to(DEV), slots,
+                       block_tables=bt.to(DEV), seq_lens=lens.int().to(DEV))
+    qkv = torch.randn(n, heads + 2 * kv, D, generator=g).bfloat16().to(DEV)
+    outs, pages = [], []
+    for fused in (True, False):
+        kc, vc = (c.clone() for c in caches)
+        q, k, v = qkv.clone().split([heads, kv, kv], 1)
+        assert ops._rope_in_attention(q, k, v, kc, meta)
+        if fused:
+            out = ops.rope_attention(q, k, v, meta.positions, cos_sin, slots,
+                                     kc, vc, meta, D ** -0.5)
+        else:
+            ops.rope_kv_append(q, k, v, meta.positions, cos_sin, slots, kc, vc)
+            out = ops.attention(q, k, v, kc, vc, meta, D ** -0.5)
+        outs.append(out.float())
+        pages.append([c.view(torch.uint8) for c in (kc, vc)])
+    assert all(torch.equal(a, b) for a, b in zip(*pages))
+    assert (outs[0] - outs[1]).abs().max() <= 2.0 ** -8 * outs[1].abs().max()
