@@ -98,6 +98,8 @@ void launch_recurrent_step(Kind, T*, float*, float*, float*, float*,
 void launch_decode_inputs(const long*, const int*, long*, long*, long*, int*,
                           int*, int*, int, int, int, int, int, hipStream_t);
 bool gemm_rows_fits(long, long);
+void launch_gemm_split(bf16*, float*, const bf16*, const bf16*, int, int, int,
+                       long, long, int, int, int, hipStream_t);
 void launch_gemm_rows(bf16*, const bf16*, const bf16*, int, int, int, long,
                       long, long, hipStream_t);
 void launch_silu_mul(bf16*, const bf16*, long, int, hipStream_t);
@@ -384,6 +386,41 @@ void gemm_rows(torch::Tensor out, torch::Tensor x, torch::Tensor w) {
   if (N == 0) return;
   launch_gemm_rows(bf(out), cbf(x), cbf(w), (int)M, (int)N, (int)K,
                    x.stride(0), w.stride(0), out.stride(0), stream());
+}
+
+// out = x w^T, K in `splits` parts that a second kernel adds up
+void gemm_split(torch::Tensor out, torch::Tensor x, torch::Tensor w,
+                c10::optional<torch::Tensor> part, long bm, long bn,
+                long splits) {
+  for (const auto& t : {out, x, w})
+    TORCH_CHECK(t.is_cuda() && t.scalar_type() == torch::kBFloat16 &&
+                    t.dim() == 2 && t.stride(1) == 1, "gemm_split: matrices");
+  const long M = x.size(0), K = x.size(1), N = w.size(0);
+  TORCH_CHECK(w.size(1) == K && out.size(0) == M && out.size(1) == N &&
+                  out.is_contiguous(), "gemm_split: shape");
+  auto aligned = [](const torch::Tensor& t) {
+    return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0 &&
+           t.stride(0) % 8 == 0;
+  };
+  TORCH_CHECK(N % 4 == 0 && K % 128 == 0 && M < (1l << 20) && K < (1l << 24) &&
+                  N < (1l << 24) && aligned(x) && aligned(w) &&
+                  reinterpret_cast<uintptr_t>(out.data_ptr()) % 8 == 0,
+              "gemm_split: sizes");
+  TORCH_CHECK((bm == 128 && (bn == 64 || bn == 128)) ||
+                  (bm == 256 && bn == 128), "gemm_split: tile");
+  TORCH_CHECK(splits >= 1 && splits <= 8 && splits <= K / 128,
+              "gemm_split: 1 to 8 parts");
+  float* ws = nullptr;
+  if (splits > 1) {
+    TORCH_CHECK(part.has_value(), "gemm_split: parts need a workspace");
+    check(*part, torch::kFloat, "part");
+    TORCH_CHECK(part->numel() >= splits * M * N, "gemm_split: workspace");
+    ws = part->data_ptr<float>();
+  }
+  if (M == 0 || N == 0) return;
+  launch_gemm_split(bf(out), ws, cbf(x), cbf(w), (int)M, (int)N, (int)K,
+                    x.stride(0), w.stride(0), (int)bm, (int)bn, (int)splits,
+                    stream());
 }
 
 void silu_mul(torch::Tensor out, torch::Tensor x) {
@@ -1095,6 +1132,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("decode_inputs", &decode_inputs);
   m.def("gemm_rows", &gemm_rows);
   m.def("gemm_rows_fits", &gemm_rows_fits);
+  m.def("gemm_split", &gemm_split);
   m.def("silu_mul", &silu_mul);
   m.def("gelu_mul", &gelu_mul);
   m.def("embed_dyt", &embed_dyt);

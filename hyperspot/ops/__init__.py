@@ -207,22 +207,53 @@ def silu_mul(gate_up: torch.Tensor) -> torch.Tensor:
     return torch_ref.silu_mul(gate_up)
 
 
+def _plain_bf16(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Matrices whose rows the kernels can load 16 bytes at a time."""
+    return x.is_cuda and x.dtype == w.dtype == torch.bfloat16 and all(
+        t.dim() == 2 and t.stride(1) == 1 and t.stride(0) % 8 == 0
+        and t.data_ptr() % 16 == 0 for t in (x, w))
+
+
 def _rows_gemm(x: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether csrc/gemm_rows.hip takes x w^T: few rows, and a weight whose
     tiles of 16 rows divide evenly over the 256 compute units; the library is
     as fast or faster elsewhere (us, library and kernel, one row: 6144 x 4096
     14.4 14.8, 4096 x 14336 26.9 28.0, 2048 x 7168 13.2 13.2)."""
-    if not (x.is_cuda and x.dtype == w.dtype == torch.bfloat16
-            and x.dim() == 2 and w.dim() == 2 and 1 <= x.shape[0] <= 64):
+    if not (_plain_bf16(x, w) and 1 <= x.shape[0] <= 64):
         return False
     (M, K), N = x.shape, w.shape[0]
     tiles = (N + 15) // 16
     if K > 4096 or K % 8 or N % 4 or N * K < (1 << 20) \
             or -(-tiles // 256) * 256 > 1.2 * tiles and tiles > 256:
         return False
-    return _native().gemm_rows_fits(M, K) and all(
-        t.stride(1) == 1 and t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0
-        for t in (x, w))
+    return _native().gemm_rows_fits(M, K)
+
+
+def _split_gemm(M: int, N: int, K: int):
+    """(rows, outputs of a tile, parts of K) where csrc/gemm_split.hip is
+    faster than the library, else None: products whose tiles, times the parts,
+    are one workgroup a compute unit or less.  More than a few parts pay for
+    their sums up to 128 rows and from 257 on (us, library and kernel: 8192 x
+    8192, 4 parts, 64 rows 33 43; 5120 x 8192, 3 parts, 320 rows 49 54), for
+    weights of 29 MB or more (2048 x 4096, 96 rows 10.6 12.5) and short rows not
+    at all (4096 x 2048, 256 rows 11 15); at 16 rows and fewer the library is
+    as fast.  Narrow tiles where K is short and they fill as many units."""
+    if not 16 < M <= 512 or K < 4096 or K % 128 or N % 4 \
+            or N * K < 14 << 20:
+        return None
+
+    def parts(bm, bn):
+        tiles = -(-M // bm) * -(-N // bn)
+        return min(8, 256 // tiles), tiles
+
+    wide, tiles = parts(128, 128)
+    if wide < (5 if M <= 128 else 2 if M <= 256 else 4):
+        tall, _ = parts(256, 128)
+        return (256, 128, tall) if M > 256 and tall >= 4 else None
+    narrow, more = parts(128, 64)
+    if M <= 256 and K < 8192 and more * narrow >= tiles * wide:
+        return 128, 64, narrow
+    return 128, 128, wide
 
 
 def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
@@ -232,6 +263,15 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
                           device=x.device)
         _native().gemm_rows(out, x, w)
         return out
+    if _plain_bf16(x, w):
+        M, N = x.shape[0], w.shape[0]
+        split = _split_gemm(M, N, x.shape[1])
+        if split is not None:
+            out = torch.empty(M, N, dtype=x.dtype, device=x.device)
+            part = torch.empty(split[2] * M * N, dtype=torch.float32,
+                               device=x.device) if split[2] > 1 else None
+            _native().gemm_split(out, x, w, part, *split)
+            return out
     return x @ w.t()
 
 
