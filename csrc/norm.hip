@@ -1,14 +1,17 @@
 // RMSNorm + fused residual-add RMSNorm, bf16, row-per-workgroup.
 //
-// Memory-bound (hidden <= 16k): one 256-thread workgroup per token row,
-// bf16x8 vector loads (scalar bf16 loads are ~2x slower on hipcc — guide
-// Common-mistake #2), fp32 accumulation, row held in registers between the
-// sumsq pass and the scale pass so each byte is read once.
+// What bounds it: many rows, memory (8192 rows of 4096 at 6.5 TB/s); few, the
+// trips to memory one after the other, so that all loads of a row, the weights
+// among them, are issued before anything waits (us for 1, 32, 256 rows of 4096
+// 2.7 3.0 3.4 when each waited for the one before, 2.4 2.5 3.1 so; of 8192 3.7
+// 4.0 5.0 and 3.2 3.4 4.6).  One 256-thread workgroup per token row, bf16x8
+// vector loads (scalar bf16 loads are ~2x slower), fp32 accumulation, row held
+// in registers between the sumsq pass and the scale pass so each byte is read
+// once.
 #include "common.h"
 
-// MAX_CHUNKS * 256 threads * 8 elems = 16384 max hidden size
-#define NORM_MAX_CHUNKS 8
-
+// CH * 256 threads * 8 elements hold a row
+template <int CH>
 __global__ __launch_bounds__(256) void rmsnorm_kernel(
     bf16* __restrict__ out, const bf16* __restrict__ x,
     const bf16* __restrict__ w, float eps, int hidden) {
@@ -17,37 +20,42 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(
   const bf16* xr = x + row * (long)hidden;
   bf16* orow = out + row * (long)hidden;
 
-  bf16x8 v[NORM_MAX_CHUNKS];
-  float ss = 0.f;
+  bf16x8 v[CH], wv[CH];
   #pragma unroll
-  for (int c = 0; c < NORM_MAX_CHUNKS; ++c) {
+  for (int c = 0; c < CH; ++c) {
     const int base = (c * 256 + threadIdx.x) * 8;
     if (base < hidden) {
       v[c] = load_bf16x8(xr + base);
+      wv[c] = load_bf16x8(w + base);
+    }
+  }
+  float ss = 0.f;
+  #pragma unroll
+  for (int c = 0; c < CH; ++c)
+    if ((c * 256 + threadIdx.x) * 8 < hidden) {
       #pragma unroll
       for (int i = 0; i < 8; ++i) {
         float f = bf16x8_get(v[c], i);
         ss += f * f;
       }
     }
-  }
   const float total = block_reduce_sum_256(ss, scratch);
   const float rs = rsqrtf(total / hidden + eps);
   #pragma unroll
-  for (int c = 0; c < NORM_MAX_CHUNKS; ++c) {
+  for (int c = 0; c < CH; ++c) {
     const int base = (c * 256 + threadIdx.x) * 8;
     if (base < hidden) {
-      bf16x8 wv = load_bf16x8(w + base);
       bf16x8 o;
       #pragma unroll
       for (int i = 0; i < 8; ++i)
-        bf16x8_set(o, i, bf16x8_get(v[c], i) * rs * bf16x8_get(wv, i));
+        bf16x8_set(o, i, bf16x8_get(v[c], i) * rs * bf16x8_get(wv[c], i));
       store_bf16x8(orow + base, o);
     }
   }
 }
 
 // x <- rmsnorm(residual + x) * w ; residual <- residual + x   (both in place)
+template <int CH>
 __global__ __launch_bounds__(256) void fused_add_rmsnorm_kernel(
     bf16* __restrict__ x, bf16* __restrict__ residual,
     const bf16* __restrict__ w, float eps, int hidden) {
@@ -56,18 +64,26 @@ __global__ __launch_bounds__(256) void fused_add_rmsnorm_kernel(
   bf16* xr = x + row * (long)hidden;
   bf16* rr = residual + row * (long)hidden;
 
-  float r[NORM_MAX_CHUNKS][8];
-  float ss = 0.f;
+  bf16x8 xv[CH], rv[CH], wv[CH];
   #pragma unroll
-  for (int c = 0; c < NORM_MAX_CHUNKS; ++c) {
+  for (int c = 0; c < CH; ++c) {
     const int base = (c * 256 + threadIdx.x) * 8;
     if (base < hidden) {
-      bf16x8 xv = load_bf16x8(xr + base);
-      bf16x8 rv = load_bf16x8(rr + base);
+      xv[c] = load_bf16x8(xr + base);
+      rv[c] = load_bf16x8(rr + base);
+      wv[c] = load_bf16x8(w + base);
+    }
+  }
+  float r[CH][8];
+  float ss = 0.f;
+  #pragma unroll
+  for (int c = 0; c < CH; ++c) {
+    const int base = (c * 256 + threadIdx.x) * 8;
+    if (base < hidden) {
       bf16x8 o;
       #pragma unroll
       for (int i = 0; i < 8; ++i) {
-        float f = bf16x8_get(xv, i) + bf16x8_get(rv, i);
+        float f = bf16x8_get(xv[c], i) + bf16x8_get(rv[c], i);
         r[c][i] = f;
         ss += f * f;
         bf16x8_set(o, i, f);
@@ -78,28 +94,38 @@ __global__ __launch_bounds__(256) void fused_add_rmsnorm_kernel(
   const float total = block_reduce_sum_256(ss, scratch);
   const float rs = rsqrtf(total / hidden + eps);
   #pragma unroll
-  for (int c = 0; c < NORM_MAX_CHUNKS; ++c) {
+  for (int c = 0; c < CH; ++c) {
     const int base = (c * 256 + threadIdx.x) * 8;
     if (base < hidden) {
-      bf16x8 wv = load_bf16x8(w + base);
       bf16x8 o;
       #pragma unroll
       for (int i = 0; i < 8; ++i)
-        bf16x8_set(o, i, r[c][i] * rs * bf16x8_get(wv, i));
+        bf16x8_set(o, i, r[c][i] * rs * bf16x8_get(wv[c], i));
       store_bf16x8(xr + base, o);
     }
   }
 }
 
+// chunks that hold a row of up to 4096, 8192 or 16384 elements
+static int chunks(int hidden) {
+  return hidden <= 4096 ? 2 : hidden <= 8192 ? 4 : 8;
+}
+
 void launch_rmsnorm(bf16* out, const bf16* x, const bf16* w, float eps,
                     long rows, int hidden, hipStream_t stream) {
-  rmsnorm_kernel<<<dim3((unsigned)rows), dim3(256), 0, stream>>>(
-      out, x, w, eps, hidden);
+  const auto kernel = chunks(hidden) == 2   ? rmsnorm_kernel<2>
+                      : chunks(hidden) == 4 ? rmsnorm_kernel<4>
+                                            : rmsnorm_kernel<8>;
+  kernel<<<dim3((unsigned)rows), dim3(256), 0, stream>>>(out, x, w, eps,
+                                                         hidden);
 }
 
 void launch_fused_add_rmsnorm(bf16* x, bf16* residual, const bf16* w,
                               float eps, long rows, int hidden,
                               hipStream_t stream) {
-  fused_add_rmsnorm_kernel<<<dim3((unsigned)rows), dim3(256), 0, stream>>>(
-      x, residual, w, eps, hidden);
+  const auto kernel = chunks(hidden) == 2   ? fused_add_rmsnorm_kernel<2>
+                      : chunks(hidden) == 4 ? fused_add_rmsnorm_kernel<4>
+                                            : fused_add_rmsnorm_kernel<8>;
+  kernel<<<dim3((unsigned)rows), dim3(256), 0, stream>>>(x, residual, w, eps,
+                                                         hidden);
 }

@@ -176,3 +176,30 @@ def test_rope_in_decode_attention(lens, group, kv, fp8):
         pages.append([c.view(torch.uint8) for c in (kc, vc)])
     assert all(torch.equal(a, b) for a, b in zip(*pages))
     assert (outs[0] - outs[1]).abs().max() <= 2.0 ** -8 * outs[1].abs().max()
+
+
+@pytest.mark.parametrize("parts", [2, 15, 16, 17, 33, 64])
+def test_parts_of_decode_attention(parts):
+    """More parts than one has 32 tokens for, and than are loaded at a time."""
+    g = torch.Generator().manual_seed(parts)
+    lens, kv, group = [1, 700, 4001], 2, 4
+    tables = [-(-x // 16) for x in lens]
+    caches = [torch.randn(sum(tables), kv, 16, D, generator=g).bfloat16()
+              for _ in range(2)]
+    order = torch.randperm(sum(tables), generator=g).int().split(tables)
+    bt = torch.zeros(3, max(tables), dtype=torch.int32)
+    for row, pages in zip(bt, order):
+        row[:len(pages)] = pages
+    q = torch.randn(3, kv * group, D, generator=g).bfloat16().to(DEV)
+    out = torch.empty_like(q)
+    ws = torch.full((3 * kv * group * parts * (D + 2),), float("nan"),
+                    device=DEV)
+    ops._native().paged_attn(
+        out, q, *(c.to(DEV) for c in caches), bt.to(DEV),
+        torch.tensor(lens, dtype=torch.int32, device=DEV), None, D ** -0.5,
+        ws, parts)
+    for i, n in enumerate(lens):
+        k, v = (c[order[i].long()].float().transpose(1, 2).reshape(-1, kv, D)
+                [:n] for c in caches)
+        _check(out[i:i + 1], _reference(q[i:i + 1], k, v, n - 1, D ** -0.5),
+               2.0 ** -14)

@@ -1,0 +1,63 @@
+"""Row kernels at the widths where the number of chunks that a thread holds
+changes, against float64.
+
+Bounds: bf16 results are rounded (2^-9 of them; the sum of squares of at most
+16384 floats and the reciprocal root add less than 2^-12); e4m3 results are the
+scale times a value rounded to 3 bits of mantissa (2^-4 of it, and half of the
+smallest step, 2^-10 of the scale)."""
+
+import pytest
+import torch
+
+import hyperspot.engine  # noqa: F401  (before the models, which it imports)
+import hyperspot.ops as ops
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+
+
+def _rows(rows, width, seed):
+    g = torch.Generator().manual_seed(seed)
+    return torch.randn(rows, width, generator=g).bfloat16()
+
+
+def _close(out, ref, quantised=False):
+    if quantised:
+        scale = out.scale.double().cpu()[:, None]
+        out, bound = out.data.double().cpu() * scale, \
+            ref.abs() * 2.0 ** -4 + scale * 2.0 ** -10
+        assert torch.allclose(scale[:, 0], ref.abs().amax(-1) / 448,
+                              rtol=2.0 ** -10)
+    else:
+        out, bound = out.double().cpu(), ref.abs() * 2.0 ** -8
+    assert ((out - ref).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("hidden", [8, 4096, 4104, 8192, 8200, 16384])
+def test_norms(hidden):
+    x, r, w = (_rows(n, hidden, n) for n in (3, 3, 1))
+    w = w[0]
+
+    def ref(y):
+        y = y.double()
+        return y / (y.square().mean(-1, keepdim=True) + 1e-5).sqrt() \
+            * w.double()
+
+    gx, gr, gw = x.to(DEV), r.to(DEV), w.to(DEV)
+    _close(ops.rmsnorm(gx, gw, 1e-5), ref(x))
+    _close(ops.quant_fp8(gx), x.double(), True)
+    both = x.double() + r.double()
+    q, res = ops.fused_add_rmsnorm_q(gx, gr.clone(), gw, 1e-5)
+    _close(q, ref(both), True)
+    _close(res, both)
+    y, res = ops.fused_add_rmsnorm(gx.clone(), gr.clone(), gw, 1e-5)
+    _close(y, ref(both))
+    _close(res, both)
+
+
+@pytest.mark.parametrize("inter", [8, 8192, 8200, 16384, 16392, 32768])
+def test_activation_in_e4m3(inter):
+    x = _rows(3, 2 * inter, 7)
+    g, u = x.double().split(inter, -1)
+    _close(ops.silu_mul_q(x.to(DEV)), g * g.sigmoid() * u, True)
