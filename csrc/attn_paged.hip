@@ -242,9 +242,9 @@ __global__ __launch_bounds__(256) void paged_attn_kernel(
 // it and v before it loads the last block.  A launch of its own for that is one
 // workgroup a token that goes to memory three times in a row, 5 us a layer;
 // here these loads pass beside the page ids and the first pages.  us of both
-// launches and of one: 1 row x 8 kv heads of 4, 1000 tokens 12.6 -> 10.1; 8 rows
-// of 8000 69 -> 63; 32 x 4 of 1000 27.7 -> 23.6; 256 x 8 of 1000 221 -> 206, of
-// 30 22.4 -> 21.9; e4m3 64 x 8 of 1000 38.5 -> 34.8.
+// launches and of one: 1 row x 8 kv heads of 4, 1000 tokens 12.6 -> 10.1; 8
+// rows of 8000 69 -> 63; 32 x 4 of 1000 27.7 -> 23.6; 256 x 8 of 1000 221 ->
+// 206, of 30 22.4 -> 21.9; e4m3 64 x 8 of 1000 38.5 -> 34.8.
 //
 // SPLIT > 1 (flash-decode): gridDim.z workgroups share one (row, kvh), each
 // with every gridDim.z-th 4 blocks of 32 tokens; their (o, m, l) land in

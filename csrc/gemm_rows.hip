@@ -4,16 +4,23 @@
 // What bounds it: reading w once.  So w is the A operand of 16x16x32 products
 // straight from memory.  The rows of x, which every tile of w needs whole, go
 // into LDS once a workgroup, and the workgroups stay: one or two a CU, each
-// with every gridDim-th tile of 16 rows of w.  (x from L2 beside every tile of
+// with every gridDim-th tile of up to 16 rows of w: of 12 or 8 where that
+// spreads them better, whose loads the other lanes sit out.  (x from L2 beside every tile of
 // w costs as many load instructions as w itself for each 16 rows: 28672 x 4096
 // took 50 us for one row and 72 us for 16.)  The 8 waves divide K, so that
 // also a single tile has 8 KB of loads in flight a wave, and add up in LDS;
 // the next tile's loads are issued before that.
 //
-// us, library and here, weights from memory (which gives about 5 TB/s):
-//   28672 x 4096  1 row 60 46, 16 rows 61 48    4096 x 4096   1 16 10, 16 16 11
-//   32768 x 4096  1 row 64 52, 16 rows 63 55    2048 x 2048   1 11  5, 32 11  7
-//   32768 x 2048  1 row 35 29, 32 rows 36 34    3072 x 2048   1 11  6, 32 12  8
+// us, library and here, weights from memory (which gives about 5 TB/s); and of
+// tiles of 16 rows where others are taken:
+//   28672 x 4096  1 row 64 46, 16 rows 66 48    4096 x 4096   1 15 10, 16 15 11
+//   32768 x 4096  1 row 64 52, 16 rows 63 55    32768 x 2048  1 35 28, 32 37 34
+//   12: 6144 x 4096  1 row 14.4 12.0 (14.5), 8 rows 14.4 13.5 (15.8)
+//       3072 x 2048  1 row 11.2  5.5  (6.0), 32 rows 11.7 7.8 (8.2)
+//       5120 x 4096  1 row 14.0 11.4 (13.7)
+//   8: 2048 x 2048   1 row  8.7  4.7  (5.3), 32 rows 8.6 7.1 (7.5)
+//      1536 x 4096   1 row 14.6  6.3  (7.9)
+//      10240 x 4096  1 row 27.1 19.4 (21.0); 14336 x 2048 16.3 13.3 (14.8)
 #include "common.h"
 
 namespace {
@@ -27,6 +34,7 @@ struct Rows {
   const bf16* x;
   const bf16* w;
   int M, N, K;
+  int rows;                          // of w a tile, at most 16
   long xs, ws, os;                   // row strides
 };
 
@@ -47,12 +55,12 @@ void gemm_rows_kernel(Rows a) {
   const int xp = a.K + 8;            // row of x in LDS: 16 rows, 16 banks
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   const int col = lane & 15, gr = lane >> 4;
-  const int tiles = (a.N + 15) / 16;
+  const int tiles = (a.N + a.rows - 1) / a.rows;
   const int batches = (a.K + U * STEP - 1) / (U * STEP);
 
   short8_t wf[U][2], wn[U][2];
   auto fetch = [&](int tile, int batch) {
-    const int n = min(tile * 16 + col, a.N - 1);
+    const int n = min(tile * a.rows + col, a.N - 1);
     const bf16* p = a.w + (long)n * a.ws + gr * 8;
     const int k0 = batch * U * STEP + wid * 64;
     #pragma unroll
@@ -60,7 +68,7 @@ void gemm_rows_kernel(Rows a) {
       #pragma unroll
       for (int s = 0; s < 2; ++s) {
         const int k = k0 + u * STEP + 32 * s;
-        wn[u][s] = k + gr * 8 < a.K
+        wn[u][s] = k + gr * 8 < a.K && col < a.rows
             ? __builtin_nontemporal_load(
                   reinterpret_cast<const short8_t*>(p + k))
             : short8_t{};
@@ -126,8 +134,8 @@ void gemm_rows_kernel(Rows a) {
       for (int v = 0; v < WAVES; ++v)
         y += *reinterpret_cast<const f32x4_t*>(
             red + ((v * CT + wid) * 64 + lane) * 4);
-      const int n = now * 16 + gr * 4, m = wid * 16 + col;
-      if (m < a.M && n < a.N)          // N is a multiple of 4
+      const int n = now * a.rows + gr * 4, m = wid * 16 + col;
+      if (m < a.M && n < a.N && gr * 4 < a.rows)     // multiples of 4
         *reinterpret_cast<uint2*>(a.out + m * a.os + n) =
             uint2{cvt_pk_bf16(y[0], y[1]), cvt_pk_bf16(y[2], y[3])};
     }
@@ -144,6 +152,20 @@ int lds_bytes(int M, int K) {
   return WAVES * row_tiles(M) * 1024 + M * (K + 8) * 2;
 }
 
+// rows of w a tile: those that the busiest CU has are fewest
+int tile_rows(int N) {
+  int best = 16, least = 0;
+  for (int rows = 16; rows >= 8; rows -= 4) {
+    const int tiles = (N + rows - 1) / rows;
+    const int most = (tiles + 255) / 256 * rows;
+    if (least == 0 || most < least) {
+      best = rows;
+      least = most;
+    }
+  }
+  return best;
+}
+
 }  // namespace
 
 // whether M rows of K columns are taken
@@ -155,8 +177,9 @@ bool gemm_rows_fits(long M, long K) {
 // N a multiple of 4, K of 8; rows of x and w 16-byte, of out 8-byte aligned
 void launch_gemm_rows(bf16* out, const bf16* x, const bf16* w, int M, int N,
                       int K, long xs, long ws, long os, hipStream_t stream) {
-  const Rows a{out, x, w, M, N, K, xs, ws, os};
-  const int lds = lds_bytes(M, K), tiles = (N + 15) / 16;
+  const int rows = tile_rows(N);
+  const Rows a{out, x, w, M, N, K, rows, xs, ws, os};
+  const int lds = lds_bytes(M, K), tiles = (N + rows - 1) / rows;
   const int most = lds * 2 <= LDS ? 512 : 256;     // that a CU holds at once
   const unsigned grid = (unsigned)(tiles < most ? tiles : most);
   #define RUN(CT)                                                           \

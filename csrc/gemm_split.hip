@@ -199,12 +199,12 @@ void launch_gemm_split(bf16* out, float* part, const bf16* x, const bf16* w,
                        int M, int N, int K, long xs, long ws, int bm,
                        int bn, int splits, hipStream_t stream) {
   Split a{out, part, x, w, M, N, K, xs, ws, 0, 0, splits};
-  #define RUN(BM, BN, WM, WN, STAGES, KC)                                       \
+  #define RUN(BM, BN, WM, WN, STAGES, KC)                                   \
     {                                                                       \
       constexpr int BYTES = STAGES * KC * (BM + BN) * 128;                  \
       static const hipError_t set = hipFuncSetAttribute(                    \
           reinterpret_cast<const void*>(                                    \
-              &gemm_split_kernel<BM, BN, WM, WN, STAGES, KC>),                  \
+              &gemm_split_kernel<BM, BN, WM, WN, STAGES, KC>),              \
           hipFuncAttributeMaxDynamicSharedMemorySize, BYTES);               \
       HIP_CHECK(set);                                                       \
       a.mt = (M + BM - 1) / BM;                                             \

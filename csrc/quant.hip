@@ -12,7 +12,8 @@
 // the store pass; fp8 packing via v_cvt_pk_fp8_f32 (native on gfx950).  Few
 // rows wait for memory, so all of a row's loads are issued first: 32 rows of
 // 4096 2.6 -> 2.3 us, with the norm 3.5 -> 2.9; the activation, by 512 threads
-// where it has more than 8192 outputs, of 14336 5.2 -> 4.4, of 28672 8.2 -> 6.7.
+// where it has more than 8192 outputs, of 14336 5.2 -> 4.4, of 28672 8.2 ->
+// 6.7.
 #include "common.h"
 
 #define QCHUNKS 8  // * 256 threads * 8 = 16384 max row width

@@ -216,16 +216,20 @@ def _plain_bf16(x: torch.Tensor, w: torch.Tensor) -> bool:
 
 def _rows_gemm(x: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether csrc/gemm_rows.hip takes x w^T: few rows, and a weight whose
-    tiles of 16 rows divide evenly over the 256 compute units; the library is
-    as fast or faster elsewhere (us, library and kernel, one row: 6144 x 4096
-    14.4 14.8, 4096 x 14336 26.9 28.0, 2048 x 7168 13.2 13.2)."""
+    tiles of 16, 12 or 8 rows divide evenly enough over the 256 compute units;
+    the library is as fast or faster elsewhere (us, library and kernel: 1 row
+    of 4096 x 14336 26.9 28.0; 32 rows of 14336 x 2048, in tiles of 12, 15.9
+    17.4)."""
     if not (_plain_bf16(x, w) and 1 <= x.shape[0] <= 64):
         return False
     (M, K), N = x.shape, w.shape[0]
-    tiles = (N + 15) // 16
-    if K > 4096 or K % 8 or N % 4 or N * K < (1 << 20) \
-            or -(-tiles // 256) * 256 > 1.2 * tiles and tiles > 256:
+    if K > 4096 or K % 8 or N % 4 or N * K < (1 << 20):
         return False
+    if N > 4096:
+        most = min(-(-N // (256 * r)) * r
+                   for r in ((16, 12, 8) if M <= 16 else (16,)))
+        if most * 256 > N * (1.34 if M <= 16 else 1.05):
+            return False
     return _native().gemm_rows_fits(M, K)
 
 

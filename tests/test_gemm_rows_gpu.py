@@ -49,3 +49,10 @@ def test_linear_takes_any_rows(rows):
     out = ops.linear(x, w).double()
     assert out.shape == ref.shape
     assert rows == 0 or (out - ref).norm() <= 2.0 ** -8 * ref.norm()
+
+
+@pytest.mark.parametrize("rows", [1, 16, 20])
+@pytest.mark.parametrize("n", [2044, 2052, 3068, 4096, 6144, 6148, 10244])
+def test_heights_of_tiles(rows, n):
+    """Tiles of 8, 12 and 16 rows of w, the last one whole or not."""
+    test_products_of_few_rows(rows, n, 528)
