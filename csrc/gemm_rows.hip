@@ -5,11 +5,11 @@
 // straight from memory.  The rows of x, which every tile of w needs whole, go
 // into LDS once a workgroup, and the workgroups stay: one or two a CU, each
 // with every gridDim-th tile of up to 16 rows of w: of 12 or 8 where that
-// spreads them better, whose loads the other lanes sit out.  (x from L2 beside every tile of
-// w costs as many load instructions as w itself for each 16 rows: 28672 x 4096
-// took 50 us for one row and 72 us for 16.)  The 8 waves divide K, so that
-// also a single tile has 8 KB of loads in flight a wave, and add up in LDS;
-// the next tile's loads are issued before that.
+// spreads them better, whose loads the other lanes sit out.  (x from L2 beside
+// every tile of w costs as many load instructions as w itself for each 16 rows:
+// 28672 x 4096 took 50 us for one row and 72 us for 16.)  The 8 waves divide K,
+// so that also a single tile has 8 KB of loads in flight a wave, and add up in
+// LDS; the next tile's loads are issued before that.
 //
 // us, library and here, weights from memory (which gives about 5 TB/s); and of
 // tiles of 16 rows where others are taken:

@@ -236,14 +236,15 @@ def _rows_gemm(x: torch.Tensor, w: torch.Tensor) -> bool:
 def _split_gemm(M: int, N: int, K: int):
     """(rows, outputs of a tile, parts of K) where csrc/gemm_split.hip is
     faster than the library, else None: products whose tiles, times the parts,
-    are one workgroup a compute unit or less.  More than a few parts pay for
-    their sums up to 128 rows and from 257 on (us, library and kernel: 8192 x
-    8192, 4 parts, 64 rows 33 43; 5120 x 8192, 3 parts, 320 rows 49 54), for
-    weights of 29 MB or more (2048 x 4096, 96 rows 10.6 12.5) and short rows not
-    at all (4096 x 2048, 256 rows 11 15); at 16 rows and fewer the library is
+    are one workgroup a compute unit or less.  Few parts gain less than the
+    library's tiles up to 128 rows and from 257 on (us, library and kernel:
+    8192 x 8192, 4 parts, 64 rows 33 43; 5120 x 8192, 3 parts, 320 rows 49 54),
+    and from there so do short rows (4096 x 4096, 4 parts, 512 rows 29 36);
+    below 29 MB of weights the sums take what is won (2048 x 4096, 96 rows 10.6
+    12.5; 4096 x 2048, 256 rows 11 15), and at 16 rows and fewer the library is
     as fast.  Narrow tiles where K is short and they fill as many units."""
-    if not 16 < M <= 512 or K < 4096 or K % 128 or N % 4 \
-            or N * K < 14 << 20:
+    if not 16 < M <= 512 or K < (4096 if M <= 256 else 7168) or K % 128 \
+            or N % 4 or N * K < 14 << 20:
         return None
 
     def parts(bm, bn):
