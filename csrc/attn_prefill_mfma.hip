@@ -26,16 +26,17 @@
 // workgroups: with 8 kv heads a die has one of them, and its keys and values
 // stay in the die's L2.  Later rows see more and start first.
 //
-// 32 heads, 8 kv heads: a prompt of 8192 tokens 661 us (832 TFLOP/s) where
+// 32 heads, 8 kv heads: a prompt of 8192 tokens 732 us (751 TFLOP/s) where
 // weights that went through LDS and tiles of 256 rows of one head took 2628
-// (209); 8 prompts of 1000, 113 us; 7808 tokens after 8192 cached ones 2.22 ms
-// (696 TFLOP/s) where one workgroup a row took 37.6.
+// (209); 8 prompts of 1000, 130 us; 7808 tokens after 8192 cached ones 2.17 ms
+// (712 TFLOP/s; e4m3 pages 2.64) where one workgroup a row took 37.6.
 //
 // ROWS: weights are rounded to bf16, relative to the maximum after each tile of
 // 64 tokens, and summed in a fixed order.  Both are a part of the result: a
 // model with 8-bit activations rounds it to few steps again, and a last bit
-// decides between two of them.  Pages: the weights are floats in the row-by-row kernel, so they enter
-// as a high and a low part (16 bits), with e4m3 pages as three (24 bits).
+// decides between two of them.  Pages: the weights are floats in the
+// row-by-row kernel, so they enter as a high and a low part (16 bits), with
+// e4m3 pages as three (24 bits).
 #include <float.h>
 
 #include "common.h"
