@@ -5,6 +5,8 @@
 // Vectorized bf16/f32 reads; fp32 math, sums of weights in 64-bit integers.
 #include <float.h>
 
+#include <type_traits>
+
 #include "common.h"
 
 // ---- greedy argmax (bf16 or float logits) ------------------------------
@@ -134,16 +136,20 @@ __global__ __launch_bounds__(256) void inv_cdf_sample_kernel(
 // at which the running sum of the others exceeds uniform * sum is drawn.
 // temperature 0: the largest logit, the first among equals.
 //
-// What bounds it: passes over the row, which stays in L2.  No sort: one
-// histogram of counts and weights over 2048 equal steps between the largest
-// and the smallest logit finds the step where the wanted count or share is
-// reached, and ranks the few values in it exactly (or divides that step
-// again).  Equal steps of the logit, and not digits of its bit pattern,
+// What bounds it: passes over the row, which stays in L2, about 12 us each for
+// 128256 values and more with their weights.  Where few values stay, and next-
+// token logits have a few dozen that matter, they are listed in the second pass
+// and the rest is done on the list.  Otherwise no sort either: one histogram of
+// counts and weights over 2048 equal steps between the largest and the smallest
+// logit finds the step where the wanted count or share is reached, and ranks
+// the few values in it exactly (or divides that step again).  Equal steps of the logit, and not digits of its bit pattern,
 // because next-token logits fill few exponents: 64 lanes that add to the
 // same few counters in LDS would go one by one.
 //
-// 64 rows of 128256, a mix of options: 139 us, where the library's sorts,
-// scans and selections took 2625.
+// 64 rows of 128256, 48 values far above the others, us with the histogram
+// alone and now: top_p 0.9 115 59, top_k 50 85 38, top_k 40 and top_p 141 38,
+// none 57 45; a mix 136 63, where the library's sorts, scans and selections
+// took 2625.  Normal logits, whose share is thousands of values, 155 146.
 //
 // Weights are 2^-40 fixed point relative to the largest, so every sum is
 // exact, does not depend on its order, and the same inputs give the same
@@ -154,12 +160,14 @@ typedef unsigned long long u64;
 constexpr int NT = 1024;          // threads
 constexpr int STEPS = 2048;       // of the histogram
 constexpr int LIST = 512;         // values ranked one by one
+constexpr int AHEAD = 2;          // loads of a thread on their way
+constexpr int FEW = 128;          // values that a share is looked for in
 
 struct Weight {
   float mx, hi, lo;               // hi + lo = log2(e) / temperature
   DEV u64 operator()(float x) const {
     const float d = x - mx, t = d * hi;
-    if (!(t > -60.f)) return 0;   // below half of 2^-40
+    if (!(t > -42.f)) return 0;   // below half of 2^-40
     const float r = fmaf(d, hi, -t) + d * lo;
     float e = __builtin_amdgcn_exp2f(t);
     e = fmaf(e * r, 0.69314718f, e) * 1099511627776.f + 0.5f;
@@ -192,6 +200,7 @@ struct Scratch {
   unsigned count[STEPS];
   float list[LIST];
   u64 list_mass[LIST];
+  int list_at[LIST];
   u64 wave_mass[16];
   unsigned wave_count[16];
   u64 before_mass, kept_mass;
@@ -204,81 +213,112 @@ struct Scratch {
 template <typename T, bool VEC> struct Row {
   const T* p;
   int vocab;
-  // the elements [at, at + 8), -inf past the end; not above FLT_MAX
-  DEV void load(int at, float* x) const {
-    if constexpr (VEC) {
-      if (at < vocab) {
-        load_vec<T, 8>(p + at, x);
-        #pragma unroll
-        for (int i = 0; i < 8; ++i) x[i] = fminf(x[i], FLT_MAX);
-        return;
-      }
-    }
-    #pragma unroll
-    for (int i = 0; i < 8; ++i)
-      x[i] = at + i < vocab ? fminf(Elem<T>::ld(p + at + i), FLT_MAX)
-                            : -INFINITY;
+  typedef __attribute__((ext_vector_type(8))) float f32x8;
+  struct Raw {                    // as loaded: nothing waits for it yet
+    typename std::conditional<sizeof(T) == 2, uint4, f32x8>::type v;
+  };
+  // the elements [at, at + 8), -inf from `end` on; not above FLT_MAX
+  DEV void fetch(int at, int end, Raw& r) const {
+    if constexpr (VEC)
+      if (at < end) r.v = *reinterpret_cast<const decltype(r.v)*>(p + at);
   }
-  template <typename F> DEV void each(F f) const {
-    #pragma unroll 2
-    for (int at = threadIdx.x * 8; at < vocab; at += NT * 8) {
-      float x[8];
-      load(at, x);
+  DEV void unpack(const Raw& r, int at, int end, float* x) const {
+    if constexpr (VEC) {
+      if constexpr (sizeof(T) == 2) {
+        const unsigned u[4] = {r.v.x, r.v.y, r.v.z, r.v.w};
+        #pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          x[2 * i] = __uint_as_float(u[i] << 16);
+          x[2 * i + 1] = __uint_as_float(u[i] & 0xffff0000u);
+        }
+      } else {
+        #pragma unroll
+        for (int i = 0; i < 8; ++i) x[i] = r.v[i];
+      }
       #pragma unroll
-      for (int i = 0; i < 8; ++i) f(x[i], at + i);
+      for (int i = 0; i < 8; ++i)
+        x[i] = at < end ? fminf(x[i], FLT_MAX) : -INFINITY;
+    } else {
+      #pragma unroll
+      for (int i = 0; i < 8; ++i)
+        x[i] = at + i < end ? fminf(Elem<T>::ld(p + at + i), FLT_MAX)
+                            : -INFINITY;
+    }
+  }
+  // f(x, index) of all values and of some -inf past the end
+  template <typename F> DEV void each(F f) const {
+    for (int at = threadIdx.x * 8; at < vocab; at += AHEAD * NT * 8) {
+      Raw r[AHEAD];
+      #pragma unroll
+      for (int q = 0; q < AHEAD; ++q) fetch(at + q * NT * 8, vocab, r[q]);
+      #pragma unroll
+      for (int q = 0; q < AHEAD; ++q) {
+        float x[8];
+        unpack(r[q], at + q * NT * 8, vocab, x);
+        #pragma unroll
+        for (int i = 0; i < 8; ++i) f(x[i], at + q * NT * 8 + i);
+      }
     }
   }
 
   // First index at which the running sum of w(x, index) exceeds the target
-  // that `of` makes of the whole sum; vocab - 1 if there is none.
+  // that `of` makes of the whole sum; vocab - 1 if there is none.  A wave has a
+  // sixteenth; the one where the target lies is divided again.
   template <typename W, typename F>
   DEV int walk(Scratch& s, W w, F of) const {
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    const int span = (vocab + 16 * 512 - 1) / (16 * 512) * 512;  // of a wave
-    const int first = wid * span, end = min(first + span, vocab);
-    u64 sum = 0;
-    #pragma unroll 2
-    for (int at = first + lane * 8; at < end; at += 512) {
-      float x[8];
-      load(at, x);
-      #pragma unroll
-      for (int i = 0; i < 8; ++i) sum += w(x[i], at + i);
-    }
-    sum = wave_scan(sum);
-    if (lane == 63) s.wave_mass[wid] = sum;
-    if (threadIdx.x == 0) s.found = vocab - 1;
-    __syncthreads();
-    u64 total = 0, before = 0;
-    for (int v = 0; v < 16; ++v) total += s.wave_mass[v];
-    const u64 target = of(total);
-    for (int v = 0; v < wid; ++v) before += s.wave_mass[v];
-    if (before <= target && before + s.wave_mass[wid] > target) {
-      for (int a0 = first; a0 < end; a0 += 512) {
-        float x[8];
-        u64 own[8], part = 0;
-        const int at = a0 + lane * 8;
-        load(at, x);
+    int first = 0, end = vocab;
+    u64 before = 0, target = 0;
+    for (bool whole = true;; whole = false) {
+      const int span = (end - first + 16 * 512 - 1) / (16 * 512) * 512;
+      const int mine = first + wid * span, stop = min(mine + span, end);
+      float x[8];                 // the first ones
+      u64 sum = 0;
+      for (int at = mine + lane * 8; at < stop; at += AHEAD * 512) {
+        Raw r[AHEAD];
         #pragma unroll
-        for (int i = 0; i < 8; ++i) part += own[i] = w(x[i], at + i);
-        const u64 upto = before + wave_scan(part);
-        if (const u64 over = __ballot(upto > target)) {
-          if (lane == __ffsll(over) - 1) {
-            u64 c = upto - part;
-            for (int i = 0; i < 8; ++i)
-              if ((c += own[i]) > target) {
-                s.found = at + i;
-                break;
-              }
-          }
-          break;
+        for (int q = 0; q < AHEAD; ++q) fetch(at + q * 512, stop, r[q]);
+        #pragma unroll
+        for (int q = AHEAD - 1; q >= 0; --q) {
+          unpack(r[q], at + q * 512, stop, x);
+          #pragma unroll
+          for (int i = 0; i < 8; ++i) sum += w(x[i], at + q * 512 + i);
         }
-        before = __shfl(upto, 63);
       }
+      const u64 upto = wave_scan(sum);
+      if (lane == 63) s.wave_mass[wid] = upto;
+      __syncthreads();
+      if (whole) {
+        u64 total = 0;
+        for (int v = 0; v < 16; ++v) total += s.wave_mass[v];
+        target = of(total);
+      }
+      int owner = 0;
+      while (owner < 16 && before + s.wave_mass[owner] <= target)
+        before += s.wave_mass[owner++];
+      if (owner == 16) {
+        __syncthreads();
+        return vocab - 1;
+      }
+      if (span == 512) {          // x has all of this wave's
+        const u64 over = __ballot(before + upto > target);
+        if (wid == owner && lane == __ffsll(over) - 1) {
+          u64 c = before + upto - sum;
+          for (int i = 0; i < 8; ++i)
+            if ((c += w(x[i], mine + lane * 8 + i)) > target) {
+              s.found = mine + lane * 8 + i;
+              break;
+            }
+        }
+        __syncthreads();
+        const int found = s.found;
+        __syncthreads();
+        return found;
+      }
+      __syncthreads();
+      first += owner * span;
+      end = min(first + span, end);
     }
-    __syncthreads();
-    const int found = s.found;
-    __syncthreads();
-    return found;
   }
 };
 
@@ -419,6 +459,117 @@ DEV void reach(Scratch& s, const R& row, const Weight& w, float lo, float hi,
   }
 }
 
+// The draw where all that stays is among few values: the want-th largest of the
+// threads' own largest values has at least that many values at or above it, and
+// hardly more.  Those are listed in one pass, ranked, and the token is drawn
+// from the list.  k 0: no top_k, and `all` is the weight of all values.  False
+// if the list is too short for the share or too long.
+template <typename R>
+DEV bool draw_from_few(Scratch& s, const R& row, const Weight& w, float own,
+                       int k, float p, float u, u64* all, int* drawn) {
+  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+  const int want_n = k > 0 ? k : FEW;
+  const unsigned key = ordered(own);
+  unsigned prefix = 0;            // 16 bits are close enough
+  for (int bit = 31; bit >= 16; --bit) {
+    const unsigned next = prefix | 1u << bit;
+    if (__syncthreads_count(key >= next) >= want_n) prefix = next;
+  }
+  const float least =
+      prefix > ordered(-FLT_MAX) ? from_ordered(prefix) : -FLT_MAX;
+  if (tid == 0) {
+    s.n = 0;
+    s.value = -INFINITY;
+  }
+  __syncthreads();
+  u64 z = 0;                      // the share is one of this
+  row.each([&](float x, int i) {
+    if (k == 0) z += w(x);
+    if (x >= least) {
+      const unsigned at = atomicAdd(&s.n, 1u);
+      if (at < LIST) {
+        s.list[at] = x;
+        s.list_at[at] = i;
+      }
+    }
+  });
+  z = wave_scan(z);
+  if (lane == 63) s.wave_mass[wid] = z;
+  __syncthreads();
+  const int n = (int)s.n;
+  z = 0;
+  for (int v = 0; v < 16; ++v) z += s.wave_mass[v];
+  *all = z;
+  float x = -INFINITY;
+  int index = 0;
+  u64 one = 0;
+  if (tid < n && n <= LIST) {
+    x = s.list[tid];
+    index = s.list_at[tid];
+    s.list_mass[tid] = one = w(x);
+  }
+  __syncthreads();
+  if (n > LIST) return false;
+  u64 above = 0;
+  int before = 0, equal = 0, earlier = 0;
+  if (tid < n)
+    #pragma unroll 4
+    for (int j = 0; j < n; ++j) {
+      const float y = s.list[j];
+      above += y > x ? s.list_mass[j] : 0;
+      before += y > x;
+      equal += y == x;
+      earlier += y == x && s.list_at[j] < index;
+    }
+  float low = -INFINITY;
+  if (k > 0) {
+    if (tid < n && before < k && before + equal >= k) {
+      s.value = x;                // every member of the group writes the same
+      s.kept_mass = above + one * equal;
+    }
+    __syncthreads();
+    low = s.value;
+    if (low > -INFINITY)
+      z = s.kept_mass;
+    else                          // fewer than k values: all are in the list
+      for (int j = 0; j < n; ++j) z += s.list_mass[j];
+  }
+  int last = row.vocab;
+  if (p < 1.f) {
+    const u64 want = (u64)ceil((double)p * (double)z);
+    if (tid == 0) s.found = -1;
+    __syncthreads();
+    if (tid < n && x >= low && above < want && above + one * equal >= want &&
+        (u64)earlier + 1 == (want - above + one - 1) / one) {
+      s.value = x;
+      s.found = index;
+    }
+    __syncthreads();
+    low = s.value;
+    last = s.found;
+    __syncthreads();
+    if (last < 0) return false;
+  }
+  const bool stays = tid < n && (x > low || (x == low && index <= last));
+  if (tid < n && !stays) s.list_mass[tid] = 0;
+  if (tid == 0) s.found = row.vocab - 1;
+  __syncthreads();
+  if (stays) {
+    u64 sum = 0, upto = 0;
+    #pragma unroll 4
+    for (int j = 0; j < n; ++j) {
+      const u64 m = s.list_mass[j];
+      sum += m;
+      upto += s.list_at[j] < index ? m : 0;
+    }
+    const u64 target = (u64)((double)u * (double)sum);
+    if (upto <= target && upto + one > target) s.found = index;
+  }
+  __syncthreads();
+  *drawn = s.found;
+  return true;
+}
+
 template <typename T, bool VEC>
 __global__ __launch_bounds__(NT) void sample_kernel(
     long* __restrict__ out, const T* __restrict__ logits,
@@ -440,6 +591,7 @@ __global__ __launch_bounds__(NT) void sample_kernel(
     }
     if (x >= -FLT_MAX) mn = fminf(mn, x);
   });
+  const float own = mx;
   #pragma unroll
   for (int o = 32; o > 0; o >>= 1) {
     const float x = __shfl_xor(mx, o);
@@ -480,19 +632,33 @@ __global__ __launch_bounds__(NT) void sample_kernel(
   int last = -1;                  // and its equals up to this index
   u64 kept = 0;                   // their weight, 0: not known
   const int k = top_k[b];
-  if (k > 0 && k < vocab) {
+  const float p = top_p[b];
+  if (p < 1.f && !(p > 0.f)) {    // nothing stays
+    if (tid == 0) out[b] = vocab - 1;
+    return;
+  }
+  const bool cut = k > 0 && k < vocab;
+  // a share is not looked for where many threads' largest values weigh more
+  // than 2^-7 of the largest: the list would be too short
+  if (cut ? k <= LIST / 2
+          : p < 1.f && __syncthreads_count((own - mx) * w.hi > -7.f) <=
+                           2 * FEW) {
+    int drawn;
+    if (draw_from_few(s, row, w, own, cut ? k : 0, p, uniform[b], &kept,
+                      &drawn)) {
+      if (tid == 0) out[b] = drawn;
+      return;
+    }
+    __syncthreads();
+  }
+  if (cut) {
     reach<true>(s, row, w, lo, mx, k);
     low = s.value;
     kept = s.keep == ~0u ? 0 : s.kept_mass;
     last = vocab;
     __syncthreads();
   }
-  const float p = top_p[b];
   if (p < 1.f) {
-    if (!(p > 0.f)) {             // nothing stays
-      if (tid == 0) out[b] = vocab - 1;
-      return;
-    }
     if (!kept)
       row.walk(s, [&](float x, int) { return w(x); }, [&](u64 z) {
         kept = z;

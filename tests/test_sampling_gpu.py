@@ -94,3 +94,21 @@ def test_rows_without_a_choice():
                      torch.tensor([1.0, 1.0, 0.0], device=DEV),
                      torch.zeros(3, dtype=torch.int32, device=DEV), ones / 2)
     assert out.tolist() == [0, 15, 15]
+
+
+@pytest.mark.parametrize("vocab", [130, 1025, 8192, 50257])
+def test_what_stays_is_few_or_not(vocab):
+    """Around the most that are listed, and shares that fill the list or not."""
+    g = torch.Generator().manual_seed(vocab)
+    options = [(t, p, k) for t in (0.3, 1.0, 3.0) for p in (1.0, 0.97, 0.3)
+               for k in (0, 1, 127, 128, 129, 256, 257, 513)]
+    x = torch.stack([_row(kind, vocab, g) * 3 for kind in
+                     ("normal", "peaked", "ties", "masked")
+                     for _ in options]).bfloat16()
+    t, p, k = (torch.tensor(c).repeat(4) for c in zip(*options))
+    u = torch.rand(len(x), generator=g)
+    out = ops.sample(*(a.to(DEV) for a in (x, t, p, k.int(), u)))
+    for b, row in enumerate(x.float()):
+        ok, _ = _allowed(row, float(t[b]), float(p[b]), int(k[b]),
+                         float(u[b]))
+        assert ok[int(out[b])], (b // len(options), options[b % len(options)])
