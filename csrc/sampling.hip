@@ -136,20 +136,23 @@ __global__ __launch_bounds__(256) void inv_cdf_sample_kernel(
 // at which the running sum of the others exceeds uniform * sum is drawn.
 // temperature 0: the largest logit, the first among equals.
 //
-// What bounds it: passes over the row, which stays in L2, about 12 us each for
-// 128256 values and more with their weights.  Where few values stay, and next-
-// token logits have a few dozen that matter, they are listed in the second pass
-// and the rest is done on the list.  Otherwise no sort either: one histogram of
-// counts and weights over 2048 equal steps between the largest and the smallest
-// logit finds the step where the wanted count or share is reached, and ranks
-// the few values in it exactly (or divides that step again).  Equal steps of the logit, and not digits of its bit pattern,
-// because next-token logits fill few exponents: 64 lanes that add to the
-// same few counters in LDS would go one by one.
+// What bounds it: vector instructions on every value, in passes over the row,
+// which stays in L2: 8 us for the largest, 20 for the weights of 128256.  So 8
+// values are looked at together where that decides about all of them.  Where
+// few values stay, and next-token logits have a few dozen that matter, they are
+// listed in the second pass and the rest is done on the list, up to 8 threads a
+// value.  Otherwise no sort either: one histogram of counts and weights over
+// 2048 equal steps between the largest and the smallest logit finds the step
+// where the wanted count or share is reached, and ranks the few values in it
+// exactly (or divides that step again).  Equal steps of the logit, and not
+// digits of its bit pattern, because next-token logits fill few exponents: 64
+// lanes that add to the same few counters in LDS would go one by one.
 //
 // 64 rows of 128256, 48 values far above the others, us with the histogram
-// alone and now: top_p 0.9 115 59, top_k 50 85 38, top_k 40 and top_p 141 38,
-// none 57 45; a mix 136 63, where the library's sorts, scans and selections
-// took 2625.  Normal logits, whose share is thousands of values, 155 146.
+// alone and now: greedy 15 11, temperature 57 38, top_p 0.9 115 39, top_k 50
+// 85 27, top_k 40 and top_p 141 28; a mix 138 45, where the library's sorts,
+// scans and selections took 2625.  Normal logits, whose share is thousands of
+// values, 155 132.
 //
 // Weights are 2^-40 fixed point relative to the largest, so every sum is
 // exact, does not depend on its order, and the same inputs give the same
@@ -165,9 +168,11 @@ constexpr int FEW = 128;          // values that a share is looked for in
 
 struct Weight {
   float mx, hi, lo;               // hi + lo = log2(e) / temperature
+  // false: weights of x and less are below half of 2^-40
+  DEV bool any(float x) const { return (x - mx) * hi > -42.f; }
   DEV u64 operator()(float x) const {
+    if (!any(x)) return 0;
     const float d = x - mx, t = d * hi;
-    if (!(t > -42.f)) return 0;   // below half of 2^-40
     const float r = fmaf(d, hi, -t) + d * lo;
     float e = __builtin_amdgcn_exp2f(t);
     e = fmaf(e * r, 0.69314718f, e) * 1099511627776.f + 0.5f;
@@ -183,6 +188,15 @@ DEV unsigned ordered(float x) {
 }
 DEV float from_ordered(unsigned u) {
   return __uint_as_float(u & 0x80000000u ? u & 0x7fffffffu : ~u);
+}
+
+DEV float largest(const float* x) {
+  return fmaxf(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])),
+               fmaxf(fmaxf(x[4], x[5]), fmaxf(x[6], x[7])));
+}
+DEV float smallest(const float* x) {
+  return fminf(fminf(fminf(x[0], x[1]), fminf(x[2], x[3])),
+               fminf(fminf(x[4], x[5]), fminf(x[6], x[7])));
 }
 
 template <typename I> DEV I wave_scan(I x) {      // inclusive
@@ -213,40 +227,44 @@ struct Scratch {
 template <typename T, bool VEC> struct Row {
   const T* p;
   int vocab;
+  bool finite;                    // known: no value is above FLT_MAX or NaN
   typedef __attribute__((ext_vector_type(8))) float f32x8;
   struct Raw {                    // as loaded: nothing waits for it yet
     typename std::conditional<sizeof(T) == 2, uint4, f32x8>::type v;
   };
   // the elements [at, at + 8), -inf from `end` on; not above FLT_MAX
   DEV void fetch(int at, int end, Raw& r) const {
-    if constexpr (VEC)
-      if (at < end) r.v = *reinterpret_cast<const decltype(r.v)*>(p + at);
-  }
-  DEV void unpack(const Raw& r, int at, int end, float* x) const {
     if constexpr (VEC) {
-      if constexpr (sizeof(T) == 2) {
-        const unsigned u[4] = {r.v.x, r.v.y, r.v.z, r.v.w};
-        #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          x[2 * i] = __uint_as_float(u[i] << 16);
-          x[2 * i + 1] = __uint_as_float(u[i] & 0xffff0000u);
-        }
-      } else {
-        #pragma unroll
-        for (int i = 0; i < 8; ++i) x[i] = r.v[i];
-      }
-      #pragma unroll
-      for (int i = 0; i < 8; ++i)
-        x[i] = at < end ? fminf(x[i], FLT_MAX) : -INFINITY;
-    } else {
-      #pragma unroll
-      for (int i = 0; i < 8; ++i)
-        x[i] = at + i < end ? fminf(Elem<T>::ld(p + at + i), FLT_MAX)
-                            : -INFINITY;
+      if (at < end)
+        r.v = *reinterpret_cast<const decltype(r.v)*>(p + at);
+      else if constexpr (sizeof(T) == 2)
+        r.v = uint4{0xff80ff80u, 0xff80ff80u, 0xff80ff80u, 0xff80ff80u};
+      else
+        r.v = f32x8(-INFINITY);
     }
   }
-  // f(x, index) of all values and of some -inf past the end
-  template <typename F> DEV void each(F f) const {
+  DEV void unpack(const Raw& r, int at, int end, float* x) const {
+    if constexpr (!VEC) {
+      #pragma unroll
+      for (int i = 0; i < 8; ++i)
+        x[i] = at + i < end ? Elem<T>::ld(p + at + i) : -INFINITY;
+    } else if constexpr (sizeof(T) == 2) {
+      const unsigned u[4] = {r.v.x, r.v.y, r.v.z, r.v.w};
+      #pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        x[2 * i] = __uint_as_float(u[i] << 16);
+        x[2 * i + 1] = __uint_as_float(u[i] & 0xffff0000u);
+      }
+    } else {
+      #pragma unroll
+      for (int i = 0; i < 8; ++i) x[i] = r.v[i];
+    }
+    if (!finite)
+      #pragma unroll
+      for (int i = 0; i < 8; ++i) x[i] = fminf(x[i], FLT_MAX);
+  }
+  // f(8 values, index of the first) of all values and of some -inf past the end
+  template <typename F> DEV void each8(F f) const {
     for (int at = threadIdx.x * 8; at < vocab; at += AHEAD * NT * 8) {
       Raw r[AHEAD];
       #pragma unroll
@@ -255,10 +273,15 @@ template <typename T, bool VEC> struct Row {
       for (int q = 0; q < AHEAD; ++q) {
         float x[8];
         unpack(r[q], at + q * NT * 8, vocab, x);
-        #pragma unroll
-        for (int i = 0; i < 8; ++i) f(x[i], at + q * NT * 8 + i);
+        f(x, at + q * NT * 8);
       }
     }
+  }
+  template <typename F> DEV void each(F f) const {
+    each8([&](const float* x, int at) {
+      #pragma unroll
+      for (int i = 0; i < 8; ++i) f(x[i], at + i);
+    });
   }
 
   // First index at which the running sum of w(x, index) exceeds the target
@@ -483,15 +506,21 @@ DEV bool draw_from_few(Scratch& s, const R& row, const Weight& w, float own,
   }
   __syncthreads();
   u64 z = 0;                      // the share is one of this
-  row.each([&](float x, int i) {
-    if (k == 0) z += w(x);
-    if (x >= least) {
-      const unsigned at = atomicAdd(&s.n, 1u);
-      if (at < LIST) {
-        s.list[at] = x;
-        s.list_at[at] = i;
-      }
-    }
+  row.each8([&](const float* x, int at) {
+    const float m = largest(x);
+    if (k == 0 && w.any(m))
+      #pragma unroll
+      for (int i = 0; i < 8; ++i) z += w(x[i]);
+    if (m >= least)
+      #pragma unroll
+      for (int i = 0; i < 8; ++i)
+        if (x[i] >= least) {
+          const unsigned n = atomicAdd(&s.n, 1u);
+          if (n < LIST) {
+            s.list[n] = x[i];
+            s.list_at[n] = at + i;
+          }
+        }
   });
   z = wave_scan(z);
   if (lane == 63) s.wave_mass[wid] = z;
@@ -500,30 +529,41 @@ DEV bool draw_from_few(Scratch& s, const R& row, const Weight& w, float own,
   z = 0;
   for (int v = 0; v < 16; ++v) z += s.wave_mass[v];
   *all = z;
-  float x = -INFINITY;
-  int index = 0;
-  u64 one = 0;
-  if (tid < n && n <= LIST) {
-    x = s.list[tid];
-    index = s.list_at[tid];
-    s.list_mass[tid] = one = w(x);
-  }
+  if (tid < n && n <= LIST) s.list_mass[tid] = w(s.list[tid]);
   __syncthreads();
   if (n > LIST) return false;
-  u64 above = 0;
+  // `share` neighbouring threads a value, each with a part of the others
+  const int share = n <= NT / 8 ? 8 : n <= NT / 4 ? 4 : 2;
+  const int mine = tid / share, part = tid % share;
+  const bool one_of = mine < n;
+  auto sum = [&](auto v) {
+    for (int o = 1; o < share; o <<= 1) v += __shfl_xor(v, o);
+    return v;
+  };
+  float x = -INFINITY;
+  int index = 0;
+  u64 one = 0, above = 0;
   int before = 0, equal = 0, earlier = 0;
-  if (tid < n)
-    #pragma unroll 4
-    for (int j = 0; j < n; ++j) {
+  if (one_of) {
+    x = s.list[mine];
+    index = s.list_at[mine];
+    one = s.list_mass[mine];
+    #pragma unroll 2
+    for (int j = part; j < n; j += share) {
       const float y = s.list[j];
       above += y > x ? s.list_mass[j] : 0;
       before += y > x;
       equal += y == x;
       earlier += y == x && s.list_at[j] < index;
     }
+  }
+  above = sum(above);
+  before = sum(before);
+  equal = sum(equal);
+  earlier = sum(earlier);
   float low = -INFINITY;
   if (k > 0) {
-    if (tid < n && before < k && before + equal >= k) {
+    if (one_of && before < k && before + equal >= k) {
       s.value = x;                // every member of the group writes the same
       s.kept_mass = above + one * equal;
     }
@@ -539,7 +579,7 @@ DEV bool draw_from_few(Scratch& s, const R& row, const Weight& w, float own,
     const u64 want = (u64)ceil((double)p * (double)z);
     if (tid == 0) s.found = -1;
     __syncthreads();
-    if (tid < n && x >= low && above < want && above + one * equal >= want &&
+    if (one_of && x >= low && above < want && above + one * equal >= want &&
         (u64)earlier + 1 == (want - above + one - 1) / one) {
       s.value = x;
       s.found = index;
@@ -550,21 +590,22 @@ DEV bool draw_from_few(Scratch& s, const R& row, const Weight& w, float own,
     __syncthreads();
     if (last < 0) return false;
   }
-  const bool stays = tid < n && (x > low || (x == low && index <= last));
-  if (tid < n && !stays) s.list_mass[tid] = 0;
+  const bool stays = one_of && (x > low || (x == low && index <= last));
+  if (one_of && !stays) s.list_mass[mine] = 0;
   if (tid == 0) s.found = row.vocab - 1;
   __syncthreads();
-  if (stays) {
-    u64 sum = 0, upto = 0;
-    #pragma unroll 4
-    for (int j = 0; j < n; ++j) {
+  u64 all_kept = 0, upto = 0;
+  if (stays)
+    #pragma unroll 2
+    for (int j = part; j < n; j += share) {
       const u64 m = s.list_mass[j];
-      sum += m;
+      all_kept += m;
       upto += s.list_at[j] < index ? m : 0;
     }
-    const u64 target = (u64)((double)u * (double)sum);
-    if (upto <= target && upto + one > target) s.found = index;
-  }
+  all_kept = sum(all_kept);
+  upto = sum(upto);
+  const u64 target = (u64)((double)u * (double)all_kept);
+  if (stays && upto <= target && upto + one > target) s.found = index;
   __syncthreads();
   *drawn = s.found;
   return true;
@@ -579,17 +620,25 @@ __global__ __launch_bounds__(NT) void sample_kernel(
   __shared__ Scratch s;
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
   const long b = blockIdx.x;
-  const Row<T, VEC> row{logits + b * vocab, vocab};
+  Row<T, VEC> row{logits + b * vocab, vocab, false};
 
-  // the largest value, its first index, and the smallest
+  // the largest value, where its first 8 values are, and the smallest
   float mx = -INFINITY, mn = INFINITY;
-  int at = vocab - 1;
-  row.each([&](float x, int i) {
-    if (x > mx) {
-      mx = x;
+  int at = vocab;
+  row.each8([&](const float* x, int i) {
+    const float m = largest(x);
+    if (m > mx) {
+      mx = m;
       at = i;
     }
-    if (x >= -FLT_MAX) mn = fminf(mn, x);
+    if constexpr (VEC) {
+      const float n = smallest(x);
+      if (i < vocab) mn = fminf(mn, n);
+    } else {
+      #pragma unroll
+      for (int j = 0; j < 8; ++j)
+        if (x[j] >= -FLT_MAX) mn = fminf(mn, x[j]);
+    }
   });
   const float own = mx;
   #pragma unroll
@@ -620,14 +669,23 @@ __global__ __launch_bounds__(NT) void sample_kernel(
   __syncthreads();
   const float t = temperature[b];
   if (t == 0.f || !(mx >= -FLT_MAX)) {          // or there is no value
-    if (tid == 0) out[b] = mx >= -FLT_MAX ? at : t == 0.f ? 0 : vocab - 1;
+    if (tid == 0) {
+      int first = t == 0.f ? 0 : vocab - 1;
+      if (mx >= -FLT_MAX) {
+        for (first = at; fminf(Elem<T>::ld(row.p + first), FLT_MAX) != mx;)
+          ++first;
+      }
+      out[b] = first;
+    }
     return;
   }
+  row.finite = mx < FLT_MAX;
 
   const double c = 1.4426950408889634 / (double)fmaxf(t, 1e-6f);
   const Weight w{mx, (float)c, (float)(c - (double)(float)c)};
   // below this weights are zero
-  const float lo = fmaxf(mn, mx - 64.f / (float)c);
+  const float floor = mx - 64.f / (float)c;
+  const float lo = mn >= -FLT_MAX ? fmaxf(mn, floor) : floor;
   float low = -INFINITY;          // values above it stay
   int last = -1;                  // and its equals up to this index
   u64 kept = 0;                   // their weight, 0: not known
