@@ -10,6 +10,8 @@
 
 void launch_rmsnorm(bf16*, const bf16*, const bf16*, float, long, int,
                     hipStream_t);
+void launch_parts_add_rmsnorm(bf16*, const float*, int, bf16*, const bf16*,
+                              float, long, int, hipStream_t);
 void launch_fused_add_rmsnorm(bf16*, bf16*, const bf16*, float, long, int,
                               hipStream_t);
 void launch_rope_kv_append(bf16*, bf16*, const bf16*, const long*,
@@ -136,6 +138,27 @@ void rmsnorm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
   TORCH_CHECK(hidden % 8 == 0 && hidden <= 16384, "hidden size");
   launch_rmsnorm(bf(out), cbf(x), cbf(w), (float)eps, x.numel() / hidden,
                  hidden, stream());
+}
+
+// x <- rmsnorm(residual + the sum of parts [splits, rows, hidden]) * w, and
+// residual that sum, the parts' rounded first
+void parts_add_rmsnorm(torch::Tensor x, torch::Tensor parts,
+                       torch::Tensor residual, torch::Tensor w, double eps) {
+  check(x, torch::kBFloat16, "x");
+  check(parts, torch::kFloat, "parts");
+  check(residual, torch::kBFloat16, "residual");
+  check(w, torch::kBFloat16, "w");
+  TORCH_CHECK(parts.dim() == 3 && parts.size(0) >= 2 && parts.size(0) <= 8,
+              "parts_add_rmsnorm: 2 to 8 parts");
+  const long rows = parts.size(1);
+  const int hidden = (int)parts.size(2);
+  TORCH_CHECK(hidden % 8 == 0 && hidden <= 8192 && w.numel() == hidden &&
+                  x.numel() == rows * hidden && residual.numel() == x.numel(),
+              "parts_add_rmsnorm: shape");
+  if (rows == 0) return;
+  launch_parts_add_rmsnorm(bf(x), parts.data_ptr<float>(), (int)parts.size(0),
+                           bf(residual), cbf(w), (float)eps, rows, hidden,
+                           stream());
 }
 
 void fused_add_rmsnorm(torch::Tensor x, torch::Tensor residual,
@@ -388,23 +411,28 @@ void gemm_rows(torch::Tensor out, torch::Tensor x, torch::Tensor w) {
                    x.stride(0), w.stride(0), out.stride(0), stream());
 }
 
-// out = x w^T, K in `splits` parts that a second kernel adds up
-void gemm_split(torch::Tensor out, torch::Tensor x, torch::Tensor w,
-                c10::optional<torch::Tensor> part, long bm, long bn,
-                long splits) {
-  for (const auto& t : {out, x, w})
+// out = x w^T, K in `splits` parts that a second kernel adds up; without out
+// the parts, [splits, M, N] floats, are the result
+void gemm_split(c10::optional<torch::Tensor> out, torch::Tensor x,
+                torch::Tensor w, c10::optional<torch::Tensor> part, long bm,
+                long bn, long splits) {
+  for (const auto& t : {out.value_or(x), x, w})
     TORCH_CHECK(t.is_cuda() && t.scalar_type() == torch::kBFloat16 &&
                     t.dim() == 2 && t.stride(1) == 1, "gemm_split: matrices");
   const long M = x.size(0), K = x.size(1), N = w.size(0);
-  TORCH_CHECK(w.size(1) == K && out.size(0) == M && out.size(1) == N &&
-                  out.is_contiguous(), "gemm_split: shape");
+  TORCH_CHECK(w.size(1) == K && (out.has_value() || splits > 1),
+              "gemm_split: shape");
+  if (out.has_value())
+    TORCH_CHECK(out->size(0) == M && out->size(1) == N &&
+                    out->is_contiguous() &&
+                    reinterpret_cast<uintptr_t>(out->data_ptr()) % 8 == 0,
+                "gemm_split: out");
   auto aligned = [](const torch::Tensor& t) {
     return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0 &&
            t.stride(0) % 8 == 0;
   };
   TORCH_CHECK(N % 4 == 0 && K % 128 == 0 && M < (1l << 20) && K < (1l << 24) &&
-                  N < (1l << 24) && aligned(x) && aligned(w) &&
-                  reinterpret_cast<uintptr_t>(out.data_ptr()) % 8 == 0,
+                  N < (1l << 24) && aligned(x) && aligned(w),
               "gemm_split: sizes");
   TORCH_CHECK((bm == 128 && (bn == 64 || bn == 128)) ||
                   (bm == 256 && bn == 128), "gemm_split: tile");
@@ -418,7 +446,7 @@ void gemm_split(torch::Tensor out, torch::Tensor x, torch::Tensor w,
     ws = part->data_ptr<float>();
   }
   if (M == 0 || N == 0) return;
-  launch_gemm_split(bf(out), ws, cbf(x), cbf(w), (int)M, (int)N, (int)K,
+  launch_gemm_split(out.has_value() ? bf(*out) : nullptr, ws, cbf(x), cbf(w), (int)M, (int)N, (int)K,
                     x.stride(0), w.stride(0), (int)bm, (int)bn, (int)splits,
                     stream());
 }
@@ -1133,6 +1161,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gemm_rows", &gemm_rows);
   m.def("gemm_rows_fits", &gemm_rows_fits);
   m.def("gemm_split", &gemm_split);
+  m.def("parts_add_rmsnorm", &parts_add_rmsnorm);
   m.def("silu_mul", &silu_mul);
   m.def("gelu_mul", &gelu_mul);
   m.def("embed_dyt", &embed_dyt);

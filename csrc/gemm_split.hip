@@ -194,7 +194,8 @@ __global__ __launch_bounds__(256) void gemm_sum_kernel(
 
 // Tiles of bm rows by bn outputs: 128 x 64, 128 x 128, 256 x 128.  out
 // contiguous; K a multiple of 128, N of 4; rows of x and w 16-byte aligned;
-// splits 1 to 8, at most K / 128, part with more than one.
+// splits 1 to 8, at most K / 128, part with more than one.  Without out the
+// parts are left for the norm that adds them up.
 void launch_gemm_split(bf16* out, float* part, const bf16* x, const bf16* w,
                        int M, int N, int K, long xs, long ws, int bm,
                        int bn, int splits, hipStream_t stream) {
@@ -220,7 +221,7 @@ void launch_gemm_split(bf16* out, float* part, const bf16* x, const bf16* w,
   else
     RUN(128, 64, 4, 2, 3, 2)
   #undef RUN
-  if (splits == 1) return;
+  if (splits == 1 || !out) return;
   const long quads = (long)M * N / 4;
   #define SUM(S)                                                            \
     case S:                                                                 \

@@ -106,6 +106,72 @@ __global__ __launch_bounds__(256) void fused_add_rmsnorm_kernel(
   }
 }
 
+// x <- rmsnorm(residual + y) * w ; residual <- residual + y, where y is the sum
+// of `parts` float products [parts, rows, hidden], rounded as a product is.
+// Adding them up here saves a launch and a trip to memory: us of product and
+// norm, 32 rows of 2048 x 7168 in 8 parts 14.2 -> 13.3, 256 of 4096 x 4096 in 2
+// 27.1 -> 24.3, 256 of 4096 x 14336 in 4 55 -> 51.5 (32 rows in 8, 29.6 29.8).
+template <int CH>
+__global__ __launch_bounds__(256) void parts_add_rmsnorm_kernel(
+    bf16* __restrict__ x, const float* __restrict__ part, int parts,
+    bf16* __restrict__ residual, const bf16* __restrict__ w, float eps,
+    int hidden) {
+  __shared__ float scratch[4];
+  const long row = blockIdx.x;
+  const long stride = (long)gridDim.x * hidden;     // of a part
+  bf16* xr = x + row * (long)hidden;
+  bf16* rr = residual + row * (long)hidden;
+
+  bf16x8 rv[CH], wv[CH];
+  f32x4_t y[CH][2];
+  #pragma unroll
+  for (int c = 0; c < CH; ++c) {
+    const int base = (c * 256 + threadIdx.x) * 8;
+    if (base < hidden) {
+      rv[c] = load_bf16x8(rr + base);
+      wv[c] = load_bf16x8(w + base);
+      const float* p = part + row * hidden + base;
+      y[c][0] = *reinterpret_cast<const f32x4_t*>(p);
+      y[c][1] = *reinterpret_cast<const f32x4_t*>(p + 4);
+      #pragma unroll 4
+      for (int z = 1; z < parts; ++z) {
+        y[c][0] += *reinterpret_cast<const f32x4_t*>(p + z * stride);
+        y[c][1] += *reinterpret_cast<const f32x4_t*>(p + z * stride + 4);
+      }
+    }
+  }
+  float r[CH][8];
+  float ss = 0.f;
+  #pragma unroll
+  for (int c = 0; c < CH; ++c) {
+    const int base = (c * 256 + threadIdx.x) * 8;
+    if (base < hidden) {
+      bf16x8 o;
+      #pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        float f = bf2f(f2bf(y[c][i >> 2][i & 3])) + bf16x8_get(rv[c], i);
+        r[c][i] = f;
+        ss += f * f;
+        bf16x8_set(o, i, f);
+      }
+      store_bf16x8(rr + base, o);   // new residual
+    }
+  }
+  const float total = block_reduce_sum_256(ss, scratch);
+  const float rs = rsqrtf(total / hidden + eps);
+  #pragma unroll
+  for (int c = 0; c < CH; ++c) {
+    const int base = (c * 256 + threadIdx.x) * 8;
+    if (base < hidden) {
+      bf16x8 o;
+      #pragma unroll
+      for (int i = 0; i < 8; ++i)
+        bf16x8_set(o, i, r[c][i] * rs * bf16x8_get(wv[c], i));
+      store_bf16x8(xr + base, o);
+    }
+  }
+}
+
 // chunks that hold a row of up to 4096, 8192 or 16384 elements
 static int chunks(int hidden) {
   return hidden <= 4096 ? 2 : hidden <= 8192 ? 4 : 8;
@@ -128,4 +194,15 @@ void launch_fused_add_rmsnorm(bf16* x, bf16* residual, const bf16* w,
                                             : fused_add_rmsnorm_kernel<8>;
   kernel<<<dim3((unsigned)rows), dim3(256), 0, stream>>>(x, residual, w, eps,
                                                          hidden);
+}
+
+// 2 to 8 parts, hidden at most 8192
+void launch_parts_add_rmsnorm(bf16* x, const float* part, int parts,
+                              bf16* residual, const bf16* w, float eps,
+                              long rows, int hidden, hipStream_t stream) {
+  const auto kernel = hidden <= 2048   ? parts_add_rmsnorm_kernel<1>
+                      : hidden <= 4096 ? parts_add_rmsnorm_kernel<2>
+                                       : parts_add_rmsnorm_kernel<4>;
+  kernel<<<dim3((unsigned)rows), dim3(256), 0, stream>>>(
+      x, part, parts, residual, w, eps, hidden);
 }

@@ -120,7 +120,7 @@ class Attention(nn.Module):
         o = o.view(T, -1)
         if self.o_proj.quant == "fp8" and o.is_cuda:
             o = ops.quant_fp8(o)   # fused amax+scale+pack (csrc/quant.hip)
-        return self.o_proj(o)
+        return self.o_proj.summands(o)
 
 
 class LlamaMLP(nn.Module):
@@ -139,7 +139,7 @@ class LlamaMLP(nn.Module):
         gu = self.gate_up(x)
         if self.down.quant == "fp8" and gu.is_cuda:
             return self.down(ops.silu_mul_q(gu))
-        return self.down(ops.silu_mul(gu))
+        return self.down.summands(ops.silu_mul(gu))
 
 
 class DecoderLayer(nn.Module):

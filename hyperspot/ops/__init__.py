@@ -37,6 +37,13 @@ def _native():
     return _C
 
 
+class Parts(NamedTuple):
+    """A product whose sum over parts of K is still to be formed: data
+    [parts, rows, outputs] float."""
+
+    data: torch.Tensor
+
+
 def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
     if x.is_cuda:
         out = torch.empty_like(x)
@@ -47,7 +54,13 @@ def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
 
 def fused_add_rmsnorm(x: torch.Tensor, residual: torch.Tensor,
                       weight: torch.Tensor, eps: float):
-    """residual += x (in place); x_out = rmsnorm(residual) (in place on x)."""
+    """residual += x (in place); x_out = rmsnorm(residual) (in place on x).
+
+    x may be the Parts of a product, which are added up on the way."""
+    if isinstance(x, Parts):
+        out = torch.empty_like(residual)
+        _native().parts_add_rmsnorm(out, x.data, residual, weight, eps)
+        return out, residual
     if x.is_cuda:
         _native().fused_add_rmsnorm(x, residual, weight, eps)
         return x, residual
@@ -259,6 +272,19 @@ def _split_gemm(M: int, N: int, K: int):
     if M <= 256 and K < 8192 and more * narrow >= tiles * wide:
         return 128, 64, narrow
     return 128, 128, wide
+
+
+def linear_parts(x: torch.Tensor, w: torch.Tensor):
+    """x w^T for w [N, K], as Parts where it is formed in parts of K."""
+    if not _rows_gemm(x, w) and _plain_bf16(x, w):
+        M, N = x.shape[0], w.shape[0]
+        split = _split_gemm(M, N, x.shape[1])
+        if split is not None and split[2] > 1 and N % 8 == 0 and N <= 8192:
+            part = torch.empty(split[2], M, N, dtype=torch.float32,
+                               device=x.device)
+            _native().gemm_split(None, x, w, part, *split)
+            return Parts(part)
+    return linear(x, w)
 
 
 def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:

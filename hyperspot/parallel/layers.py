@@ -258,6 +258,15 @@ class RowParallelLinear(_LinearCompute):
         out = self._mm(x)
         return tensor_model_parallel_all_reduce(out)
 
+    def summands(self, x):
+        """forward() for a residual add and norm, which also take a product
+        that is still in parts (ops.Parts)."""
+        from hyperspot import ops as _O
+        if self.quant is None and get_tp_size() == 1 \
+                and isinstance(x, torch.Tensor):
+            return _O.linear_parts(x, self.weight)
+        return self(x)
+
 
 class MergedRowParallelLinear(_LinearCompute):
     """The sum of several row-parallel projections as one GEMM over their

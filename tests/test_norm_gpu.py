@@ -61,3 +61,31 @@ def test_activation_in_e4m3(inter):
     x = _rows(3, 2 * inter, 7)
     g, u = x.double().split(inter, -1)
     _close(ops.silu_mul_q(x.to(DEV)), g * g.sigmoid() * u, True)
+
+
+@pytest.mark.parametrize("parts", [2, 3, 5, 8])
+@pytest.mark.parametrize("hidden", [8, 2048, 2056, 4096, 4104, 8192])
+def test_norm_of_parts(hidden, parts):
+    """The same bits as the sum, in order, and then the norm."""
+    g = torch.Generator().manual_seed(hidden)
+    part = torch.randn(parts, 5, hidden, generator=g).to(DEV)
+    r, w = _rows(5, hidden, 1).to(DEV), _rows(1, hidden, 2)[0].to(DEV)
+    total = part[0].clone()
+    for z in range(1, parts):
+        total += part[z]
+    y, res = ops.fused_add_rmsnorm(total.bfloat16(), r.clone(), w, 1e-5)
+    out = ops.fused_add_rmsnorm(ops.Parts(part), r, w, 1e-5)
+    assert torch.equal(out[0], y) and torch.equal(out[1], res)
+
+
+@pytest.mark.parametrize("rows", [16, 32, 200])
+def test_parts_of_a_product(rows):
+    x, w = _rows(rows, 4096, 3).to(DEV), _rows(4096, 4096, 4).to(DEV)
+    out = ops.linear_parts(x, w)
+    assert isinstance(out, ops.Parts) == (rows > 16)
+    if rows > 16:
+        out = out.data
+        for z in range(1, len(out)):
+            out[0] += out[z]
+        out = out[0].bfloat16()
+    assert torch.equal(out, ops.linear(x, w))
