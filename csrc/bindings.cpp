@@ -446,9 +446,9 @@ void gemm_split(c10::optional<torch::Tensor> out, torch::Tensor x,
     ws = part->data_ptr<float>();
   }
   if (M == 0 || N == 0) return;
-  launch_gemm_split(out.has_value() ? bf(*out) : nullptr, ws, cbf(x), cbf(w), (int)M, (int)N, (int)K,
-                    x.stride(0), w.stride(0), (int)bm, (int)bn, (int)splits,
-                    stream());
+  launch_gemm_split(out.has_value() ? bf(*out) : nullptr, ws, cbf(x), cbf(w),
+                    (int)M, (int)N, (int)K, x.stride(0), w.stride(0), (int)bm,
+                    (int)bn, (int)splits, stream());
 }
 
 void silu_mul(torch::Tensor out, torch::Tensor x) {
