@@ -28,15 +28,15 @@
 //
 // 32 heads, 8 kv heads: a prompt of 8192 tokens 732 us (751 TFLOP/s) where
 // weights that went through LDS and tiles of 256 rows of one head took 2628
-// (209); 8 prompts of 1000, 130 us; 7808 tokens after 8192 cached ones 2.17 ms
-// (712 TFLOP/s; e4m3 pages 2.64) where one workgroup a row took 37.6.
+// (209); 8 prompts of 1000, 130 us; 7808 tokens after 8192 cached ones 2.58 ms
+// (600 TFLOP/s; e4m3 pages 2.62) where one workgroup a row took 37.6.
 //
 // ROWS: weights are rounded to bf16, relative to the maximum after each tile of
 // 64 tokens, and summed in a fixed order.  Both are a part of the result: a
 // model with 8-bit activations rounds it to few steps again, and a last bit
 // decides between two of them.  Pages: the weights are floats in the
-// row-by-row kernel, so they enter as a high and a low part (16 bits), with
-// e4m3 pages as three (24 bits).
+// row-by-row kernel, so they enter as three parts, which hold the 24 bits of a
+// float; two were off by up to 2^-20 of what they weigh (and took 2.07 ms).
 #include <float.h>
 
 #include "common.h"
@@ -121,7 +121,7 @@ template <int HG, int SRC>
 __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(Prefill a) {
   constexpr int RG = 4 / HG;                 // row groups of 32
   constexpr int TILE_ROWS = RG * WAVE_ROWS;
-  constexpr int PARTS = SRC == ROWS ? 1 : SRC == PAGES ? 2 : 3;
+  constexpr int PARTS = SRC == ROWS ? 1 : 3;
   constexpr bool EACH = SRC == ROWS;         // rescale at each tile
   __shared__ __attribute__((aligned(16))) short lds[2][2][KV * HD];
 

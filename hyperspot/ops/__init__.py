@@ -133,10 +133,12 @@ def paged_attn_decode(q: torch.Tensor, k_cache: torch.Tensor,
 
 # Portions of at least this many rows attend on tiles of 32 rows, the others row
 # by row.  A tile takes a context's latency whatever it holds, a row its share
-# of the memory: one portion of 16, 64, 96 rows after 1000 tokens takes 31, 33,
-# 34 us in tiles and 15, 25, 35 by rows, after 16000 399, 402, 408 and 147,
-# 306, 447 (8 kv heads of 4).  Beside others tiles share the latency.
-PORTION_ROWS, PORTION_ROWS_ALONE = 16, 80
+# of the memory: one portion of 16, 64, 96, 112 rows after 1000 tokens takes 36,
+# 39, 41, 41 us in tiles and 16, 28, 38, 47 by rows, after 16000 491, 494, 495,
+# 494 and 144, 284, 418, 555 (8 kv heads of 4; with e4m3 pages 112 and 192 rows
+# after 1000 44, 46 and 34, 49).  Beside others tiles share the latency: 8
+# portions of 4, 8, 16 rows 41, 37, 37 us and 25, 44, 48.
+PORTION_ROWS, PORTION_ROWS_ALONE = 16, 104
 
 
 def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,

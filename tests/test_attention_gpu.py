@@ -2,8 +2,8 @@
 edges of tiles, against the PyTorch reference in float64.
 
 Bounds: outputs are rounded to bf16 (2^-9 of the value) and are means of
-values of about one; weights enter as two bf16 parts over the pages (2^-16)
-and as one (2^-9) beside q."""
+values of about one; weights enter as three bf16 parts over the pages (the
+bound is that of two, 2^-16) and as one (2^-9) beside q."""
 
 import pytest
 import torch
@@ -203,3 +203,38 @@ def test_parts_of_decode_attention(parts):
                 [:n] for c in caches)
         _check(out[i:i + 1], _reference(q[i:i + 1], k, v, n - 1, D ** -0.5),
                2.0 ** -14)
+
+
+@pytest.mark.parametrize("rows", [8, 103, 104])    # by rows, and in tiles
+def test_weights_over_bf16_pages_are_floats(rows):
+    """Values that cancel: what is left is the error of the weights.
+
+    Scores of at most one are off by a few 2^-24 and their exponentials by
+    about 2^-23; three bf16 parts hold a weight to 2^-25 and two to 2^-18."""
+    g = torch.Generator().manual_seed(8)
+    before, total = 64, 64 + rows
+    q = (torch.randn(D, generator=g) * 0.3).bfloat16()
+    k = (torch.randn(total, D, generator=g) * 0.3).bfloat16()
+    scale = D ** -0.5
+    w = (k[:before].double() @ q.double() * scale).exp()
+    v = torch.randn(before, D, generator=g).bfloat16()
+    for t in range(before - 4, before):         # each takes 2^-9 of the rest
+        v[t:] = 0
+        v[t] = (-(w @ v.double()) / w[t]).bfloat16()
+    # the portion's own tokens add nothing
+    v = torch.cat([v, torch.zeros(rows, D).bfloat16()])
+    pages = total // 16 + (total % 16 > 0)
+    kc, vc = (torch.zeros(pages * 16, 1, D).bfloat16() for _ in range(2))
+    kc[:total, 0], vc[:total, 0] = k, v
+    kc, vc = (c.view(pages, 16, 1, D).transpose(1, 2).contiguous().to(DEV)
+              for c in (kc, vc))
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    meta = ForwardMeta("prefill", None, None, seq_start=i32([0, rows]),
+                       row_seq=i32([0] * rows),
+                       ctx_lens=i32(list(range(before + 1, total + 1))),
+                       block_tables=i32([list(range(pages))]),
+                       fresh_prefill=False)
+    out = ops.attention(q.expand(rows, 1, D).contiguous().to(DEV), None, None,
+                        kc, vc, meta, scale)
+    size = (w[:, None] * v[:before].double().abs()).sum(0) / w.sum()
+    assert (out[:, 0].double().cpu().abs() <= 2.0 ** -21 * size).all()
