@@ -492,6 +492,14 @@ __global__ __launch_bounds__(256, 3) void paged_attn_mfma_kernel(Paged a) {
         sc[t] = mfma16(k.v, qf[c], sc[t]);
       }
     }
+    // what the page holds after the last token: a weight of zero does not hide
+    // a NaN
+    if ((i + 1) * BLOCK > ctx) {
+      #pragma unroll
+      for (int j = 0; j < (KV8 ? 4 : 8); ++j)
+        if (i * BLOCK + (KV8 ? 8 * j + (lane >> 3) : 4 * j + gr) >= ctx)
+          vr[j] = u32x4(0);
+    }
     if constexpr (KV8) {             // rows 8 j + lane / 8
       #pragma unroll
       for (int j = 0; j < 4; ++j) {

@@ -162,8 +162,10 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(Prefill a) {
   float m = -FLT_MAX, l = 0.f;
 
   // ---- tiles.  bf16: a wave brings 4 KB-units of K and of V, rows 16 j +
-  // 4 wid and the three after it; tokens past the last one read that again
-  // (their weight is zero).  A tile's pages are looked up one tile ahead.
+  // 4 wid and the three after it.  Tokens past the last one have a weight of
+  // zero, which does not hide a NaN: beside q the last one is read again, in
+  // the pages their values are cleared.  A tile's pages are looked up one tile
+  // ahead.
   const int* bt = SRC == ROWS ? nullptr
                               : a.block_tables + (long)s * a.max_blocks;
   const int last_page = last / PAGE;
@@ -211,8 +213,9 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(Prefill a) {
       }
     }
   };
-  auto store = [&](int buf) {                    // PAGES8
+  auto store = [&](int kv0, int buf) {           // PAGES8
     const int tok = tid >> 2;
+    if (kv0 + tok > last) raw[2] = raw[3] = uint4{0, 0, 0, 0};
     #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const unsigned* x = &raw[i].x;
@@ -325,15 +328,23 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(Prefill a) {
     l = fmaf(l, alpha, sum);
   };
 
-  auto landed = [&](int buf) {
-    if constexpr (SRC == PAGES8) store(buf);
+  auto landed = [&](int kv0, int buf) {
+    if constexpr (SRC == PAGES8) store(kv0, buf);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (SRC == PAGES && kv0 + KV - 1 > last) {   // what this lane brought
+      #pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (kv0 + 16 * j + lr > last)
+          *reinterpret_cast<uint4*>(
+              &lds[buf][1][(16 * j + 4 * wid) * HD + lane * 8]) =
+              uint4{0, 0, 0, 0};
+    }
     __syncthreads();
   };
   if constexpr (SRC != ROWS) look_up(0);
   fetch(0, 0);
   if constexpr (SRC != ROWS) look_up(KV);
-  landed(0);
+  landed(0, 0);
   int buf = 0;
   for (int kv0 = 0; kv0 <= last; kv0 += KV, buf ^= 1) {
     const bool more = kv0 + KV <= last;
@@ -342,7 +353,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(Prefill a) {
       if constexpr (SRC != ROWS) look_up(kv0 + 2 * KV);
     }
     if (rw < n && kv0 <= w_last) compute(kv0, buf);
-    if (more) landed(buf ^ 1);
+    if (more) landed(kv0 + KV, buf ^ 1);
   }
 
   if constexpr (!EACH) l += __shfl_xor(l, 32);

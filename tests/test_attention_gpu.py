@@ -238,3 +238,69 @@ def test_weights_over_bf16_pages_are_floats(rows):
                         kc, vc, meta, scale)
     size = (w[:, None] * v[:before].double().abs()).sum(0) / w.sum()
     assert (out[:, 0].double().cpu().abs() <= 2.0 ** -21 * size).all()
+
+
+def _pages_of(lens, kv, fp8, g):
+    """(k, v of every sequence in order, the pages with NaN after each one's
+    last token, block tables)"""
+    kind = torch.float8_e4m3fn if fp8 else torch.bfloat16
+    tables = [-(-n // 16) for n in lens]
+    order = torch.randperm(sum(tables), generator=g).split(tables)
+    bt = torch.zeros(len(lens), max(tables) + 1, dtype=torch.int32)
+    both = [[torch.randn(n, kv, D, generator=g).to(kind).float() for n in lens]
+            for _ in range(2)]
+    caches = []
+    for rows in both:
+        cache = torch.full((sum(tables), kv, 16, D), float("nan"))
+        for i, pages in enumerate(order):
+            bt[i, :tables[i]] = pages
+            whole = torch.full((tables[i] * 16, kv, D), float("nan"))
+            whole[:lens[i]] = rows[i]
+            cache[pages] = whole.view(-1, 16, kv, D).transpose(1, 2)
+        caches.append(cache.to(kind).to(DEV))
+    return both, caches, bt
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("split", [1, 3])
+def test_nan_after_the_last_token_in_decode(split, fp8):
+    from hyperspot import _C
+    g = torch.Generator().manual_seed(9)
+    lens, kv, heads = [1, 15, 17, 31, 33, 50, 64, 130, 400], 2, 8
+    (k, v), (kc, vc), bt = _pages_of(lens, kv, fp8, g)
+    q = torch.randn(len(lens), heads, D, generator=g).bfloat16().to(DEV)
+    out = torch.empty_like(q)
+    ws = torch.empty(len(lens) * heads * split * (D + 2), device=DEV) \
+        if split > 1 else None
+    _C.paged_attn(out, q, kc, vc, bt.to(DEV),
+                  torch.tensor(lens, dtype=torch.int32, device=DEV), None,
+                  D ** -0.5, ws, split)
+    for i, n in enumerate(lens):
+        _check(out[i:i + 1], _reference(q[i:i + 1], k[i], v[i], n - 1,
+                                        D ** -0.5), 2.0 ** -14)
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("portions", [
+    [(5, 90), (40, 17), (64, 3), (30, 33)], [(100, 130)], [(1, 103)],
+    [(1, 104)],
+])
+def test_nan_after_the_last_token_of_portions(portions, fp8):
+    g = torch.Generator().manual_seed(10)
+    kv, heads = 2, 8
+    lens, rows = [b + n for b, n in portions], [n for _, n in portions]
+    (k, v), (kc, vc), bt = _pages_of(lens, kv, fp8, g)
+    q = torch.randn(sum(rows), heads, D, generator=g).bfloat16().to(DEV)
+    starts = [sum(rows[:i]) for i in range(len(rows) + 1)]
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    meta = ForwardMeta("prefill", None, None, seq_start=i32(starts),
+                       row_seq=i32([i for i, n in enumerate(rows)
+                                    for _ in range(n)]),
+                       ctx_lens=i32([c + 1 for b, n in portions
+                                     for c in range(b, b + n)]),
+                       block_tables=bt.to(DEV), fresh_prefill=False)
+    out = ops.attention(q, None, None, kc, vc, meta, D ** -0.5)
+    for i, (b, n) in enumerate(portions):
+        at = slice(starts[i], starts[i + 1])
+        _check(out[at], _reference(q[at], k[i], v[i], b, D ** -0.5),
+               2.0 ** -14)
