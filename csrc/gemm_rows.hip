@@ -21,6 +21,8 @@
 //   8: 2048 x 2048   1 row  8.7  4.7  (5.3), 32 rows 8.6 7.1 (7.5)
 //      1536 x 4096   1 row 14.6  6.3  (7.9)
 //      10240 x 4096  1 row 27.1 19.4 (21.0); 14336 x 2048 16.3 13.3 (14.8)
+#include <type_traits>
+
 #include "common.h"
 
 namespace {
@@ -53,7 +55,8 @@ void gemm_rows_kernel(Rows a) {
   float* red = reinterpret_cast<float*>(smem);
   short* xl = reinterpret_cast<short*>(smem + WAVES * CT * 1024);
   const int xp = a.K + 8;            // row of x in LDS: 16 rows, 16 banks
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 15, gr = lane >> 4;
   const int tiles = (a.N + a.rows - 1) / a.rows;
   const int batches = (a.K + U * STEP - 1) / (U * STEP);
@@ -78,7 +81,7 @@ void gemm_rows_kernel(Rows a) {
   fetch(tile, 0);
   if (a.K % 512 == 0) {              // a KB of a row a wave, straight to LDS
     const int parts = a.K / 512, n = a.M * parts;
-    for (int i = __builtin_amdgcn_readfirstlane(wid); i < n; i += WAVES) {
+    for (int i = wid; i < n; i += WAVES) {
       const int m = i / parts, c = (i - m * parts) * 512;
       to_lds16(a.x + m * a.xs + c + lane * 8, xl + m * xp + c);
     }
@@ -109,17 +112,28 @@ void gemm_rows_kernel(Rows a) {
       tile += gridDim.x;
     }
     if (tile < tiles) fetch(tile, batch);
-    #pragma unroll
-    for (int u = 0; u < U; ++u)
+    auto products = [&](auto whole) {
       #pragma unroll
-      for (int s = 0; s < 2; ++s) {
-        // columns past the end: w is zero, and x is that of the last ones
-        const int k = min(k0 + u * STEP + 32 * s, a.K - 8 - gr * 8);
+      for (int u = 0; u < U; ++u)
         #pragma unroll
-        for (int t = 0; t < CT; ++t)
-          acc[t] = mfma16(wf[u][s], *reinterpret_cast<const short8_t*>(
-                                        xr[t] + k), acc[t]);
-      }
+        for (int s = 0; s < 2; ++s) {
+          // columns past the end: x is zero as w is, for the last ones may
+          // hold an infinity
+          const int k = k0 + u * STEP + 32 * s;
+          if (!whole && k >= a.K) continue;
+          const bool in = whole || k + gr * 8 < a.K;
+          #pragma unroll
+          for (int t = 0; t < CT; ++t) {
+            const short8_t v = *reinterpret_cast<const short8_t*>(
+                xr[t] + (in ? k : 0));
+            acc[t] = mfma16(wf[u][s], in ? v : short8_t{}, acc[t]);
+          }
+        }
+    };
+    if (k0 + (U - 1) * STEP + 64 <= a.K)
+      products(std::true_type{});
+    else
+      products(std::false_type{});
     if (batch) continue;
     #pragma unroll
     for (int t = 0; t < CT; ++t) {

@@ -56,3 +56,24 @@ def test_linear_takes_any_rows(rows):
 def test_heights_of_tiles(rows, n):
     """Tiles of 8, 12 and 16 rows of w, the last one whole or not."""
     test_products_of_few_rows(rows, n, 528)
+
+
+@pytest.mark.parametrize("rows,k", [
+    (1, 8), (1, 264), (1, 512), (1, 2056), (1, 4104), (16, 4104), (20, 8),
+    (20, 264), (20, 1536), (20, 2056), (64, 1000)])
+def test_infinities_in_the_last_columns(rows, k):
+    """K is not a multiple of what a batch of loads covers."""
+    g = torch.Generator().manual_seed(k)
+    x = torch.randn(rows, k, generator=g).bfloat16()
+    x[0, -1], x[-1, max(k - 9, 0)] = float("inf"), float("-inf")
+    w = torch.randn(36, k, generator=g).bfloat16()
+    w[w == 0] = 1
+    ref = x.double() @ w.double().t()
+    out = torch.empty(rows, 36, dtype=torch.bfloat16, device=DEV)
+    _C.gemm_rows(out, x.to(DEV), w.to(DEV))
+    out = out.double().cpu()
+    odd = ~ref.isfinite()                      # NaN where both signs meet
+    assert odd[0].all()
+    assert torch.equal(out[odd].nan_to_num(0.0, 1.0, -1.0),
+                       ref[odd].nan_to_num(0.0, 1.0, -1.0))
+    assert out[~odd].isfinite().all()
