@@ -134,7 +134,8 @@ __global__ __launch_bounds__(256) void inv_cdf_sample_kernel(
 // with top_p < 1 a token goes if the ones before it, in descending order and
 // by index among equals, have at least top_p of the weight; the first token
 // at which the running sum of the others exceeds uniform * sum is drawn.
-// temperature 0: the largest logit, the first among equals.
+// temperature 0: the largest logit, the first among equals.  A logit that is
+// NaN is not drawn.
 //
 // What bounds it: vector instructions on every value, in passes over the row,
 // which stays in L2: 8 us for the largest, 20 for the weights of 128256.  So 8
@@ -190,6 +191,9 @@ DEV float from_ordered(unsigned u) {
   return __uint_as_float(u & 0x80000000u ? u & 0x7fffffffu : ~u);
 }
 
+// an infinity as the largest finite value; NaN, which is never drawn, as -inf
+DEV float in_range(float x) { return fminf(fmaxf(x, -INFINITY), FLT_MAX); }
+
 DEV float largest(const float* x) {
   return fmaxf(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])),
                fmaxf(fmaxf(x[4], x[5]), fmaxf(x[6], x[7])));
@@ -227,12 +231,13 @@ struct Scratch {
 template <typename T, bool VEC> struct Row {
   const T* p;
   int vocab;
-  bool finite;                    // known: no value is above FLT_MAX or NaN
+  bool finite;                    // no value is above FLT_MAX, or it may be
   typedef __attribute__((ext_vector_type(8))) float f32x8;
   struct Raw {                    // as loaded: nothing waits for it yet
     typename std::conditional<sizeof(T) == 2, uint4, f32x8>::type v;
   };
-  // the elements [at, at + 8), -inf from `end` on; not above FLT_MAX
+  // the elements [at, at + 8), -inf from `end` on; not above FLT_MAX unless
+  // `finite` says so
   DEV void fetch(int at, int end, Raw& r) const {
     if constexpr (VEC) {
       if (at < end)
@@ -261,7 +266,7 @@ template <typename T, bool VEC> struct Row {
     }
     if (!finite)
       #pragma unroll
-      for (int i = 0; i < 8; ++i) x[i] = fminf(x[i], FLT_MAX);
+      for (int i = 0; i < 8; ++i) x[i] = in_range(x[i]);
   }
   // f(8 values, index of the first) of all values and of some -inf past the end
   template <typename F> DEV void each8(F f) const {
@@ -620,15 +625,16 @@ __global__ __launch_bounds__(NT) void sample_kernel(
   __shared__ Scratch s;
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
   const long b = blockIdx.x;
-  Row<T, VEC> row{logits + b * vocab, vocab, false};
+  Row<T, VEC> row{logits + b * vocab, vocab, true};
 
-  // the largest value, where its first 8 values are, and the smallest
+  // the largest value, where its first 8 values are, and the smallest; neither
+  // is that of a NaN
   float mx = -INFINITY, mn = INFINITY;
   int at = vocab;
   row.each8([&](const float* x, int i) {
     const float m = largest(x);
-    if (m > mx) {
-      mx = m;
+    if (m > mx && mx < FLT_MAX) {
+      mx = fminf(m, FLT_MAX);
       at = i;
     }
     if constexpr (VEC) {
@@ -666,13 +672,14 @@ __global__ __launch_bounds__(NT) void sample_kernel(
     }
     mn = fminf(mn, s.list[16 + v]);
   }
+  mn = fminf(mn, mx);
   __syncthreads();
   const float t = temperature[b];
   if (t == 0.f || !(mx >= -FLT_MAX)) {          // or there is no value
     if (tid == 0) {
       int first = t == 0.f ? 0 : vocab - 1;
       if (mx >= -FLT_MAX) {
-        for (first = at; fminf(Elem<T>::ld(row.p + first), FLT_MAX) != mx;)
+        for (first = at; in_range(Elem<T>::ld(row.p + first)) != mx;)
           ++first;
       }
       out[b] = first;

@@ -112,3 +112,25 @@ def test_what_stays_is_few_or_not(vocab):
         ok, _ = _allowed(row, float(t[b]), float(p[b]), int(k[b]),
                          float(u[b]))
         assert ok[int(out[b])], (b // len(options), options[b % len(options)])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("vocab", [1001, 8192])
+def test_nan_is_not_drawn(vocab, dtype):
+    """As if it were -inf, beside infinities too."""
+    g = torch.Generator().manual_seed(vocab)
+    options = [(0.0, 1.0, 0), (1.0, 1.0, 0), (0.7, 0.9, 0), (1.0, 1.0, 5),
+               (3.0, 0.8, 300)]
+    x = torch.stack([_row(kind, vocab, g) for kind in
+                     ("normal", "peaked", "ties", "wide") for _ in options])
+    x[::3, 77] = float("inf")
+    gone = torch.rand(x.shape, generator=g) < 0.3
+    gone[:, :16] = True                        # a thread's whole load
+    gone[-1] = True
+    t, p, k = (torch.tensor(c).repeat(4) for c in zip(*options))
+    u = torch.rand(len(x), generator=g)
+    nan, low = (ops.sample(*(a.to(DEV) for a in (
+        x.masked_fill(gone, fill).to(dtype), t, p, k.int(), u)))
+        for fill in (float("nan"), float("-inf")))
+    assert torch.equal(nan, low)
+    assert not gone[:-1].gather(1, nan[:-1, None].cpu()).any()
