@@ -509,11 +509,20 @@ def sample(logits: torch.Tensor, temperature: torch.Tensor,
     inverse-CDF draw over the tokens in order of their ids, in one kernel."""
     if not logits.is_cuda:
         return torch_ref.sample(logits, temperature, top_p, top_k, uniform)
+    rows, vocab = logits.shape
+    if top_k.dtype != torch.int32:
+        top_k = top_k.clamp(0, vocab)
+    # an option of one element is that of every row
+    option = lambda t, kind: t.to(logits.device, kind).expand(rows) \
+        .contiguous()
+    temperature, top_p = (option(t, torch.float32)
+                          for t in (temperature, top_p))
+    top_k = option(top_k, torch.int32)
+    if vocab >= 1 << 23:        # weights of up to 2^40 add up to 63 bits
+        return torch_ref.sample(logits, temperature, top_p, top_k, uniform)
     if logits.dtype not in (torch.bfloat16, torch.float32):
         logits = logits.float()
-    out = torch.empty(logits.shape[0], dtype=torch.long, device=logits.device)
-    f32 = lambda t: t.to(logits.device, torch.float32).contiguous()
-    _native().sample(out, logits.contiguous(), f32(temperature), f32(top_p),
-                     top_k.to(logits.device, torch.int32).contiguous(),
-                     f32(uniform))
+    out = torch.empty(rows, dtype=torch.long, device=logits.device)
+    _native().sample(out, logits.contiguous(), temperature, top_p, top_k,
+                     uniform.to(logits.device, torch.float32).contiguous())
     return out

@@ -134,3 +134,25 @@ def test_nan_is_not_drawn(vocab, dtype):
         for fill in (float("nan"), float("-inf")))
     assert torch.equal(nan, low)
     assert not gone[:-1].gather(1, nan[:-1, None].cpu()).any()
+
+
+def test_one_option_for_all_rows():
+    """Options of one element count for every row; top_k of 64 bits."""
+    g = torch.Generator().manual_seed(1)
+    x = torch.randn(9, 500, generator=g).to(DEV)
+    u = torch.rand(9, generator=g).to(DEV)
+    one = [torch.tensor([c], device=DEV) for c in (0.7, 0.9)]
+    k = torch.tensor([1 << 40], device=DEV)
+    ref = ops.sample(x, *(t.expand(9).contiguous() for t in one),
+                     torch.zeros(9, dtype=torch.int32, device=DEV), u)
+    assert torch.equal(ops.sample(x, *one, k, u), ref)
+
+
+def test_a_vocabulary_beyond_the_kernel():
+    v = (1 << 23) + 8
+    x = torch.zeros(2, v, device=DEV, dtype=torch.bfloat16)
+    x[:, v - 3] = 40
+    f = lambda *c: torch.tensor(c, device=DEV)
+    for t, p, k in ((0.0, 1.0, 0), (1.0, 1.0, 0), (1.0, 0.9, 50)):
+        out = ops.sample(x, f(t, 0.0), f(p, p), f(k, k).int(), f(0.3, 0.6))
+        assert out.tolist() == [v - 3] * 2
