@@ -121,8 +121,10 @@ class MixtralMoE(nn.Module):
 
     def _fused_router(self, x: torch.Tensor) -> bool:
         return x.is_cuda and ops.have_native() and x.is_contiguous() \
+            and ops.unrecorded(x, self.router) \
             and self.router.dtype == torch.bfloat16 \
-            and self.num_experts <= 64 and x.shape[1] % 8 == 0
+            and self.num_experts <= 64 \
+            and x.shape[1] % 8 == 0
 
     def _route_gpu(self, x: torch.Tensor):
         if x.dtype == torch.bfloat16 and self._fused_router(x):

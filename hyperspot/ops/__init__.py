@@ -222,11 +222,28 @@ def silu_mul(gate_up: torch.Tensor) -> torch.Tensor:
     return torch_ref.silu_mul(gate_up)
 
 
+def unrecorded(*tensors: torch.Tensor) -> bool:
+    """Whether a kernel may take the place of torch's operation on these: no
+    gradient or tangent is formed, and no subclass, transform, trace or mode
+    has to see the operation."""
+    return not torch.compiler.is_compiling() \
+        and all(type(t) in (torch.Tensor, torch.nn.Parameter)
+                for t in tensors) \
+        and not (torch.is_grad_enabled()
+                 and any(t.requires_grad for t in tensors)) \
+        and torch.autograd.forward_ad._current_level < 0 \
+        and torch._C._functorch.peek_interpreter_stack() is None \
+        and torch._C._len_torch_dispatch_stack() == 0 \
+        and torch._C._get_tracing_state() is None \
+        and not torch.is_autocast_enabled("cuda")
+
+
 def _plain_bf16(x: torch.Tensor, w: torch.Tensor) -> bool:
     """Matrices whose rows the kernels can load 16 bytes at a time."""
-    return x.is_cuda and x.dtype == w.dtype == torch.bfloat16 and all(
-        t.dim() == 2 and t.stride(1) == 1 and t.stride(0) % 8 == 0
-        and t.data_ptr() % 16 == 0 for t in (x, w))
+    return x.is_cuda and x.dtype == w.dtype == torch.bfloat16 \
+        and unrecorded(x, w) and all(
+            t.dim() == 2 and t.stride(1) == 1 and t.stride(0) % 8 == 0
+            and t.data_ptr() % 16 == 0 for t in (x, w))
 
 
 def _rows_gemm(x: torch.Tensor, w: torch.Tensor) -> bool:
