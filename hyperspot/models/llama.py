@@ -24,7 +24,7 @@ from hyperspot import ops
 from hyperspot.engine.config import ModelSpec
 from hyperspot.ops.torch_ref import rope_cos_sin
 from hyperspot.parallel import (QKVParallelLinear, RowParallelLinear,
-                                MergedColumnParallelLinear)
+                                MergedColumnParallelLinear, summands)
 from hyperspot.parallel.state import get_tp_size
 
 
@@ -111,6 +111,13 @@ class Attention(nn.Module):
 
     def forward(self, x, meta: ForwardMeta,
                 kv_cache: torch.Tensor, cos_sin: torch.Tensor) -> torch.Tensor:
+        return self.o_proj(self._heads(x, meta, kv_cache, cos_sin))
+
+    def _summands(self, *args):
+        return summands(self.o_proj, self._heads(*args))
+
+    def _heads(self, x, meta: ForwardMeta, kv_cache: torch.Tensor,
+               cos_sin: torch.Tensor):
         q, k, v = self.qkv(x)
         T = q.shape[0]
         k_cache, v_cache = kv_cache[0], kv_cache[1]
@@ -120,7 +127,7 @@ class Attention(nn.Module):
         o = o.view(T, -1)
         if self.o_proj.quant == "fp8" and o.is_cuda:
             o = ops.quant_fp8(o)   # fused amax+scale+pack (csrc/quant.hip)
-        return self.o_proj.summands(o)
+        return o
 
 
 class LlamaMLP(nn.Module):
@@ -136,10 +143,16 @@ class LlamaMLP(nn.Module):
         self.inter_shard = spec.intermediate_size // self.tp
 
     def forward(self, x) -> torch.Tensor:
+        return self.down(self._inner(x))
+
+    def _summands(self, x):
+        return summands(self.down, self._inner(x))
+
+    def _inner(self, x):
         gu = self.gate_up(x)
         if self.down.quant == "fp8" and gu.is_cuda:
-            return self.down(ops.silu_mul_q(gu))
-        return self.down.summands(ops.silu_mul(gu))
+            return ops.silu_mul_q(gu)
+        return ops.silu_mul(gu)
 
 
 class DecoderLayer(nn.Module):
@@ -157,9 +170,20 @@ class DecoderLayer(nn.Module):
     def forward(self, x: torch.Tensor, residual: Optional[torch.Tensor],
                 meta: ForwardMeta, kv_cache: torch.Tensor,
                 cos_sin: torch.Tensor):
+        h, residual = self._hidden(x, residual, meta, kv_cache, cos_sin)
+        return self.mlp(h), residual
+
+    def _summands(self, *args):
+        h, residual = self._hidden(*args)
+        return summands(self.mlp, h), residual
+
+    def _hidden(self, x, residual: Optional[torch.Tensor], meta: ForwardMeta,
+                kv_cache: torch.Tensor, cos_sin: torch.Tensor):
+        """The input of the feed-forward block, and the residual stream."""
         # fp8 GPU path: the norm kernels emit per-token-scaled fp8 directly
         # (csrc/quant.hip), so GEMM inputs never take an extra quant pass.
-        fp8 = self.attn.qkv.quant == "fp8" and x.is_cuda
+        fp8 = self.attn.qkv.quant == "fp8" \
+            and (x if residual is None else residual).is_cuda
         if residual is None:
             # x is the fresh embedding-gather output: safe to alias as the
             # residual (fused_add_rmsnorm mutates it in place from layer 1 on)
@@ -173,14 +197,13 @@ class DecoderLayer(nn.Module):
         else:
             h, residual = ops.fused_add_rmsnorm(x, residual,
                                                 self.input_norm_w, self.eps)
-        h = self.attn(h, meta, kv_cache, cos_sin)
+        h = summands(self.attn, h, meta, kv_cache, cos_sin)
         if fp8:
             h, residual = ops.fused_add_rmsnorm_q(h, residual,
                                                   self.post_norm_w, self.eps)
         else:
             h, residual = ops.fused_add_rmsnorm(h, residual, self.post_norm_w,
                                                 self.eps)
-        h = self.mlp(h)
         return h, residual
 
 
@@ -218,7 +241,8 @@ class LlamaForCausalLM(nn.Module):
         x = self.embed[input_ids]
         residual = None
         for i, layer in enumerate(self.layers):
-            x, residual = layer(x, residual, meta, kv_caches[i], self.cos_sin)
+            x, residual = summands(layer, x, residual, meta, kv_caches[i],
+                                   self.cos_sin)
         x, _ = ops.fused_add_rmsnorm(x, residual, self.final_norm_w,
                                      self.spec.rms_eps)
         if meta.return_hidden:

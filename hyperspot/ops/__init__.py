@@ -350,6 +350,8 @@ def fused_add_rmsnorm_q(x: torch.Tensor, residual: torch.Tensor,
                         weight: torch.Tensor, eps: float):
     """residual += x (in place); returns (QTensor of rmsnorm(residual)*w,
     residual).  GPU-only fused producer for the fp8 GEMM path."""
+    if isinstance(x, Parts):      # of a layer with 16-bit weights before it
+        x = x.data.sum(0).to(residual.dtype)
     assert x.is_cuda
     T, K = x.shape
     out = torch.empty(T, K, dtype=torch.float8_e4m3fn, device=x.device)

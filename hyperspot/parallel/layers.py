@@ -12,6 +12,7 @@ from __future__ import annotations
 
 import torch
 from torch import nn
+from torch.nn.modules.module import _has_any_global_hook
 
 from .state import (get_tp_rank, get_tp_size,
                     tensor_model_parallel_all_reduce)
@@ -57,6 +58,20 @@ def quant_fp8_rowwise(x: torch.Tensor):
     s = (xf.abs().amax(dim=-1) / FP8_MAX).clamp_min(1e-8)
     q = (xf / s[:, None]).clamp(-FP8_MAX, FP8_MAX).to(torch.float8_e4m3fn)
     return q, s
+
+
+def summands(module: nn.Module, *args):
+    """module(*args) for a residual add and norm, which also take a product
+    that is still in parts (ops.Parts), where the module's own class says how
+    (`_summands`) and nothing else sees or replaces the call."""
+    own = vars(type(module)).get("_summands")
+    if own is None or "forward" in vars(module) \
+            or module._compiled_call_impl is not None \
+            or module._forward_hooks or module._forward_pre_hooks \
+            or module._backward_hooks or module._backward_pre_hooks \
+            or _has_any_global_hook():
+        return module(*args)
+    return own(module, *args)
 
 
 class _LinearCompute(nn.Module):
@@ -258,14 +273,12 @@ class RowParallelLinear(_LinearCompute):
         out = self._mm(x)
         return tensor_model_parallel_all_reduce(out)
 
-    def summands(self, x):
-        """forward() for a residual add and norm, which also take a product
-        that is still in parts (ops.Parts)."""
+    def _summands(self, x):
         from hyperspot import ops as _O
         if self.quant is None and get_tp_size() == 1 \
                 and isinstance(x, torch.Tensor):
             return _O.linear_parts(x, self.weight)
-        return self(x)
+        return self.forward(x)
 
 
 class MergedRowParallelLinear(_LinearCompute):
