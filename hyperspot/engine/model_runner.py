@@ -262,8 +262,9 @@ class ModelRunner:
         max_nt = int(bm.ntables_np[rows].max())
         bt = bm.tables_np[rows[:, None], np.arange(max_nt)[None, :]]
         if self._st_event is not None:
-            # the last step's copy may still be reading the staging buffer: a
-            # step need not end in a device synchronization
+            # the last step may still be copying from the staging buffer, or
+            # reading its copy: a step need not end in a device
+            # synchronization, nor run on this one's stream
             self._st_event.synchronize()
         cap = bm.capacity
         used = 5 * cap + (B * max_nt + 1) // 2
@@ -276,6 +277,11 @@ class ModelRunner:
             d[:used].copy_(self._stage[:used], non_blocking=True)
             self._st_event.record()
         return d, B, max_nt
+
+    def _staged_read(self) -> None:
+        """The staged values are where the step reads them."""
+        if self._st_event is not None:
+            self._st_event.record()
 
     def _decode_meta(self, staged):
         """Tensors of an eager decode step from the staged values."""
@@ -428,11 +434,13 @@ class ModelRunner:
         if bucket is None or self.device.type != "cuda" \
                 or self.config.enforce_eager:
             input_ids, meta = self._decode_meta(staged)
+            self._staged_read()
             return self.model(input_ids, meta, self.kv_caches)
         if bucket not in self._graphs:
             self._capture(bucket)
         io = self._graph_io[bucket]
         ops.decode_inputs(stage, B, self.block_manager.capacity, max_nt, io)
+        self._staged_read()
         self._graphs[bucket].replay()
         return io["logits"][:B]
 

@@ -50,6 +50,29 @@ def test_incremental_decode_matches_full_recompute():
     assert out == ref
 
 
+def test_staging_is_free_when_the_step_has_read_it():
+    """The next step waits until this one's copy on the device is read too."""
+    eng, log = _engine(), []
+    runner = eng.runner
+
+    class Event:
+        def record(self):
+            log.append("record")
+
+        def synchronize(self):
+            log.append("wait")
+
+    runner._st_event = Event()
+    meta = runner._decode_meta
+    runner._decode_meta = lambda staged: (log.append("read"), meta(staged))[1]
+    model = runner.model
+    runner.model = lambda *a: (log.append("model"), model(*a))[1]
+    eng.generate([[3, 4, 5]], SamplingParams(temperature=0.0, max_tokens=4))
+    steps = " ".join(log).split("wait")[1:]
+    assert len(steps) == 3
+    assert all(s.split()[-3:] == ["read", "record", "model"] for s in steps)
+
+
 def test_batched_greedy_equals_single():
     eng = _engine()
     p1, p2 = [1, 2, 3, 4], [10, 20, 30, 40, 50, 60]
