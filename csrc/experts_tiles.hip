@@ -140,18 +140,19 @@ void experts_tiles_kernel(Tiles a) {
 
   const int chunks = (int)(row_bytes / 128);
   if constexpr (STAGES == 2) {
-    // [chunk d landed | barrier | issue d + 1 | compute d]: the barrier also
-    // says that every wave is done with the slot that d + 1 takes
+    // [chunk d landed, own reads of d - 1 done | barrier | issue d + 1 into the
+    // slot of d - 1 | compute d]
     stage(0, 0);
     for (int d = 0; d < chunks; ++d) {
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
       __builtin_amdgcn_s_barrier();
       if (d + 1 < chunks) stage((d + 1) & 1, d + 1);
       compute(d & 1);
     }
   } else {
-    // [compute d | issue d + 2 | d + 1 landed | barrier]: d + 2 takes the slot
-    // of d - 1, with which every wave was done before the last barrier
+    // [compute d | issue d + 2 | d + 1 landed, own reads of d done | barrier]:
+    // d + 2 takes the slot of d - 1, with which every wave was done before the
+    // last barrier
     static_assert(STAGES == 3, "stages");
     constexpr int LOADS = LX + LW;
     stage(0, 0);
@@ -162,7 +163,7 @@ void experts_tiles_kernel(Tiles a) {
     for (; d + 2 < chunks; ++d) {
       compute(slot);
       stage(slot == 0 ? 2 : slot - 1, d + 2);
-      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LOADS) : "memory");
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(LOADS) : "memory");
       __builtin_amdgcn_s_barrier();
       slot = slot == 2 ? 0 : slot + 1;
     }
