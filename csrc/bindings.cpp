@@ -346,7 +346,7 @@ void attn_portions(torch::Tensor out, torch::Tensor q, torch::Tensor k_cache,
   TORCH_CHECK(v_cache.scalar_type() == k_cache.scalar_type() &&
                   k_cache.is_contiguous() && v_cache.is_contiguous(),
               "k/v cache");
-  TORCH_CHECK(ctx_lens.numel() == T && row_seq.numel() == T &&
+  TORCH_CHECK(ctx_lens.numel() >= T && row_seq.numel() >= T &&
                   block_tables.size(0) >= seqs, "attn_portions: rows");
   const bool fp8 = k_cache.scalar_type() == torch::kFloat8_e4m3fn;
   if (short_too)

@@ -161,7 +161,8 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
             _native().attn_prefill_mfma(out, q, k, v, meta.seq_start,
                                         meta.max_seqlen, scale)
         elif q.shape[-1] == 128 and meta.seq_start is not None \
-                and q.shape[1] // k_cache.shape[1] in (1, 2, 4, 8):
+                and q.shape[1] // k_cache.shape[1] in (1, 2, 4, 8) \
+                and k_cache.data_ptr() % 16 == v_cache.data_ptr() % 16 == 0:
             least = PORTION_ROWS_ALONE if q.shape[0] < PORTION_ROWS_ALONE \
                 else PORTION_ROWS
             _native().attn_portions(
@@ -169,7 +170,7 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
                 meta.row_seq, meta.seq_start, least,
                 getattr(meta, "min_seqlen", 0) < least, scale)
         else:
-            # row by row: odd head dims
+            # row by row: odd head dims, pages that begin off 16 bytes
             _native().paged_attn(out, q, k_cache, v_cache,
                                  meta.block_tables, meta.ctx_lens,
                                  meta.row_seq, scale, None, 1)
