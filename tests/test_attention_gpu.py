@@ -304,3 +304,21 @@ def test_nan_after_the_last_token_of_portions(portions, fp8):
         at = slice(starts[i], starts[i + 1])
         _check(out[at], _reference(q[at], k[i], v[i], b, D ** -0.5),
                2.0 ** -14)
+
+
+@pytest.mark.parametrize("shift", [0, 4])      # elements: pages off 16 bytes
+def test_portions_with_longer_tables(shift):
+    """What the row-by-row kernel takes."""
+    g = torch.Generator().manual_seed(11)
+    kv, heads, before, n = 2, 8, 40, 120
+    (k, v), caches, bt = _pages_of([before + n], kv, False, g)
+    kc, vc = (torch.cat([c.new_zeros(shift), c.view(-1)])[shift:].view_as(c)
+              for c in caches)
+    q = torch.randn(n, heads, D, generator=g).bfloat16().to(DEV)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    meta = ForwardMeta("prefill", None, None, seq_start=i32([0, n]),
+                       row_seq=i32([0] * (n + 7)),
+                       ctx_lens=i32(list(range(before + 1, before + n + 8))),
+                       block_tables=bt.to(DEV), fresh_prefill=False)
+    out = ops.attention(q, None, None, kc, vc, meta, D ** -0.5)
+    _check(out, _reference(q, k[0], v[0], before, D ** -0.5), 2.0 ** -14)
