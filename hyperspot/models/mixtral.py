@@ -123,7 +123,7 @@ class MixtralMoE(nn.Module):
         return x.is_cuda and ops.have_native() and x.is_contiguous() \
             and ops.unrecorded(x, self.router) \
             and self.router.dtype == torch.bfloat16 \
-            and self.num_experts <= 64 \
+            and ops.moe_router_takes(x.shape[0], self.num_experts) \
             and x.shape[1] % 8 == 0
 
     def _route_gpu(self, x: torch.Tensor):

@@ -399,6 +399,17 @@ def _moe_splitk(nblocks: int, nchunks: int, out_numel: int, dev):
     return s, torch.empty(s * out_numel, dtype=torch.float32, device=dev)
 
 
+def moe_router_takes(tokens: int, experts: int) -> bool:
+    """Whether the router kernel, which reads the router's rows for every
+    token, is faster than torch's product, softmax and selection (us, torch
+    and kernel: 16 x 4096, 2048 tokens 70 25, 8192 111 86, 16384 182 186; 32 x
+    2048, 4096 tokens 72 52, 6144 78 74, 8192 86 98; 64 x 4096, 192 tokens 51
+    14, 1024 67 54, 1280 77 67, 2048 83 106, 8192 138 401; 64 x 2048, 1280 63
+    52, 2048 69 80)."""
+    return experts <= 64 and tokens <= (
+        16384 if experts <= 16 else 6144 if experts <= 32 else 1280)
+
+
 def moe_router(x, router: torch.Tensor, top: int):
     """(weights [T, top] float, expert ids [T, top] int32) of the rows of x, a
     bf16 tensor or a QTensor: the softmax over the chosen.  GPU."""

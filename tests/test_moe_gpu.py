@@ -100,3 +100,35 @@ def test_refused_sizes():
     ids = torch.zeros(3, 1, dtype=torch.int32, device=DEV)
     with pytest.raises(RuntimeError):
         ops.moe_ffn(x, w13, w2, torch.ones(3, 1, device=DEV), ids)
+
+
+@pytest.mark.parametrize("tokens", [1280, 1281])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_many_tokens_over_many_experts(tokens, fp8, monkeypatch):
+    """The kernel up to the rule's bound and torch's operations beyond it make
+    the same choices, but for logits that are as close as float sums are."""
+    from hyperspot.engine import ModelSpec
+    from hyperspot.models.mixtral import MixtralMoE
+    from hyperspot.parallel import layers
+    monkeypatch.setattr(layers, "_QUANT_MODE", "fp8" if fp8 else None)
+    monkeypatch.setattr(layers, "_INIT_DEVICE", DEV)
+    spec = ModelSpec("m", 256, 1, 2, 1, 128, 128 if not fp8 else 256, 64,
+                     num_experts=64, num_experts_per_tok=4)
+    moe = MixtralMoE(spec, 0, torch.bfloat16).to(DEV)
+    g = torch.Generator().manual_seed(tokens)
+    x = torch.randn(tokens, 256, generator=g).bfloat16().to(DEV)
+    moe.router.data.copy_(torch.randn(64, 256, generator=g))
+    seen = []
+    kernel = ops._native().experts_router
+    monkeypatch.setattr(ops._native(), "experts_router", lambda *a: (
+        seen.append(1), kernel(*a))[1])
+    xq = ops.quant_fp8(x) if fp8 else x
+    out = moe(xq)
+    assert len(seen) == (tokens == 1280)
+    weight, ids = ops.moe_router(xq, moe.router, 4)
+    ref = ops.moe_ffn_fp8(xq, moe.w13, moe.w13_scale, moe.w2, moe.w2_scale,
+                          weight, ids) if fp8 \
+        else ops.moe_ffn(x, moe.w13, moe.w2, weight, ids)
+    same = (out.float() - ref.float()).abs() <= 2.0 ** -7 * ref.float().abs() \
+        .max()
+    assert same.all(-1).float().mean() >= 0.99
