@@ -9,7 +9,10 @@
 // every tile of w costs as many load instructions as w itself for each 16 rows:
 // 28672 x 4096 took 50 us for one row and 72 us for 16.)  The 8 waves divide K,
 // so that also a single tile has 8 KB of loads in flight a wave, and add up in
-// LDS; the next tile's loads are issued before that.
+// LDS; the next tile's loads are issued before that.  x comes straight to LDS
+// where K is a multiple of 512, otherwise 4 units of 16 bytes a thread at once
+// (64 rows of 3904 x 384 12.4 -> 5.2 us, of 1760 x 768 12.8 -> 6.2, where each
+// waited for the one before).
 //
 // us, library and here, weights from memory (which gives about 5 TB/s); and of
 // tiles of 16 rows where others are taken:
@@ -86,11 +89,23 @@ void gemm_rows_kernel(Rows a) {
       to_lds16(a.x + m * a.xs + c + lane * 8, xl + m * xp + c);
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  } else {
-    for (int m = 0; m < a.M; ++m)
-      for (int c = threadIdx.x * 8; c < a.K; c += WAVES * 64 * 8)
-        *reinterpret_cast<short8_t*>(xl + m * xp + c) =
-            *reinterpret_cast<const short8_t*>(a.x + m * a.xs + c);
+  } else {                           // 4 units of 16 bytes a thread at once
+    constexpr int T = WAVES * 64;
+    const int units = a.K / 8, n = a.M * units;
+    for (int i = threadIdx.x; i < n; i += 4 * T) {
+      short8_t v[4];
+      int at[4];
+      #pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int u = min(i + j * T, n - 1);   // the last one again
+        const int m = u / units, c = (u - m * units) * 8;
+        v[j] = *reinterpret_cast<const short8_t*>(a.x + m * a.xs + c);
+        at[j] = m * xp + c;
+      }
+      #pragma unroll
+      for (int j = 0; j < 4; ++j)
+        *reinterpret_cast<short8_t*>(xl + at[j]) = v[j];
+    }
   }
   const short* xr[CT];
   #pragma unroll
