@@ -248,22 +248,49 @@ def _plain_bf16(x: torch.Tensor, w: torch.Tensor) -> bool:
 
 
 def _rows_gemm(x: torch.Tensor, w: torch.Tensor) -> bool:
-    """Whether csrc/gemm_rows.hip takes x w^T: few rows, and a weight whose
-    tiles of 16, 12 or 8 rows divide evenly enough over the 256 compute units;
-    the library is as fast or faster elsewhere (us, library and kernel: 1 row
-    of 4096 x 14336 26.9 28.0; 32 rows of 14336 x 2048, in tiles of 12, 15.9
-    17.4)."""
-    if not (_plain_bf16(x, w) and 1 <= x.shape[0] <= 64):
+    """Whether csrc/gemm_rows.hip takes x w^T: few rows, and sizes at which it
+    is faster than the library on average of some hundred random ones."""
+    return _plain_bf16(x, w) and _rows_gemm_sizes(x.shape[0], *w.shape) \
+        and _native().gemm_rows_fits(*x.shape)
+
+
+def _rows_gemm_sizes(M: int, N: int, K: int) -> bool:
+    """Measured at 1 to 64 rows, K of 256 to 4096 and N of 256 to 160000, 40000
+    random sizes (time of the kernel over the library's, means of a class).  Up
+    to 4096 outputs 0.53 to 0.84, but for more than 32 rows with K of 1280
+    (1.0).  Beyond, the tiles of 16, 12 or 8 rows of w have to divide evenly
+    over the 256 compute units (4608 x 2048, where the busiest has 1.33 times
+    its share, is at 0.57 for one row and 0.71 for 16).  The loads of a step
+    cover 2048 columns: K of 2048 is at 0.5 to 1.0 for all N, K of 4096 at 0.7 to 0.9 but
+    for 6657 to 8192 outputs (1.05) and a head of 128256 with 16 rows (1.1).
+    For other K the library is faster at 40961 to 65536 outputs (1.06 to 1.3);
+    beyond, for up to 16 rows with K up to 1024 (0.94 to 1.26) and more with
+    K up to 512 or beyond 3072 (1.0 to 1.3); below, for 17 to 32 rows with K
+    beyond 1024 (0.93 to 1.16), for 33 to 64 with more than 12288 outputs (0.96
+    to 1.6), for 32769 outputs and more with K up to 512 (1.0 to 1.8), and for
+    6145 to 8191 outputs with K beyond 2048 (0.9 to 1.0 for one row, 0.98 to
+    1.13 for 8 and 16).  2 to 6 of 100 sizes that are taken are more than 3 %
+    slower than the library, where it has a tile that fits them."""
+    if not 1 <= M <= 64 or K > 4096 or K % 8 or N % 4 or N * K < 1 << 20:
         return False
-    (M, K), N = x.shape, w.shape[0]
-    if K > 4096 or K % 8 or N % 4 or N * K < (1 << 20):
+    if N <= 4096:
+        return M <= 32 or not 1024 < K <= 1280
+    most = min(-(-N // (256 * r)) * r
+               for r in ((16, 12, 8) if M <= 16 else (16,)))
+    if most * 256 > N * (1.34 if M <= 16 else 1.05):
         return False
-    if N > 4096:
-        most = min(-(-N // (256 * r)) * r
-                   for r in ((16, 12, 8) if M <= 16 else (16,)))
-        if most * 256 > N * (1.34 if M <= 16 else 1.05):
-            return False
-    return _native().gemm_rows_fits(M, K)
+    if K % 2048 == 0:
+        return K == 2048 or not (6144 < N <= 8192 and M > 4
+                                 or N > 65536 and M > 8)
+    if M > 32:
+        return K <= 1024 and N <= 12288
+    if N > 65536:
+        return 1024 < K if M <= 16 else K <= 3072 and (K > 512 or M <= 24)
+    if N > (32768 if K <= 512 else 40960):
+        return False
+    if M > 16:
+        return K <= 1024 or K < 2048 and N <= 20480
+    return K < 2048 or M <= 4 or not 6144 < N < 8192
 
 
 def _split_gemm(M: int, N: int, K: int):

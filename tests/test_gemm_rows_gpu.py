@@ -77,3 +77,16 @@ def test_infinities_in_the_last_columns(rows, k):
     assert torch.equal(out[odd].nan_to_num(0.0, 1.0, -1.0),
                        ref[odd].nan_to_num(0.0, 1.0, -1.0))
     assert out[~odd].isfinite().all()
+
+
+def test_sizes_where_the_library_is_faster():
+    """Rows of K that fill the loads in part, and outputs of a head or of a
+    width that suits the library."""
+    for m, n, k in ((16, 50304, 1024), (1, 50304, 512), (17, 6144, 2560),
+                    (8, 7168, 3584), (16, 128256, 4096), (48, 16384, 512),
+                    (8, 65536, 2304), (48, 4096, 1280), (4, 128256, 768)):
+        assert not ops._rows_gemm_sizes(m, n, k)
+    for m, n, k in ((16, 4096, 1024), (64, 4096, 768), (1, 4608, 2304),
+                    (8, 32768, 4096), (32, 32768, 2048), (4, 7168, 4096),
+                    (16, 28672, 3584), (48, 12288, 512), (16, 40960, 1536)):
+        assert ops._rows_gemm_sizes(m, n, k)
