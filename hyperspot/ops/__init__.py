@@ -296,25 +296,39 @@ def _rows_gemm_sizes(M: int, N: int, K: int) -> bool:
 def _split_gemm(M: int, N: int, K: int):
     """(rows, outputs of a tile, parts of K) where csrc/gemm_split.hip is
     faster than the library, else None: products whose tiles, times the parts,
-    are one workgroup a compute unit or less.  Few parts gain less than the
-    library's tiles up to 128 rows and from 257 on (us, library and kernel:
-    8192 x 8192, 4 parts, 64 rows 33 43; 5120 x 8192, 3 parts, 320 rows 49 54),
-    and from there so do short rows (4096 x 4096, 4 parts, 512 rows 29 36);
-    below 29 MB of weights the sums take what is won (2048 x 4096, 96 rows 10.6
-    12.5; 4096 x 2048, 256 rows 11 15), and at 16 rows and fewer the library is
-    as fast.  Narrow tiles where K is short and they fill as many units."""
+    are one workgroup a compute unit or less on each of the 8 dies (3 tiles of
+    rows, 21 of outputs and 4 parts are 252, but 33 on some dies: 384 rows of
+    2688 x 7552 took 47 us, the library 37).  Measured at 17 to 512 rows, N of
+    512 to 9000 and K of 4096 to 20000: 0.67 of the library's time on average,
+    and more than 3 % slower at 1 of 100 sizes.  Few parts gain less than the library's tiles up to 128 rows and from 257 on
+    (us, library and kernel: 8192 x 8192, 4 parts, 64 rows 33 43; 5120 x 8192,
+    3 parts, 320 rows 49 54).  From 257 rows on short rows gain little or
+    nothing (3072 x 6144, 320 rows 28 30; 4096 x 6144 37 36, 512 rows 44 42).
+    Below 14M weights it is the faster one from K of 5120 on (2048 x 6144, 64
+    rows 19.5 12.3, 256 23 20) and about even with K of 4096 (2048 x 4096, 96
+    rows 12.7 12.6, 128 12.7 14.9); all these are left to the library.  So are
+    257 to 320 rows of up to 3264 outputs in tall tiles, K up to 12288 (3072
+    x 8192, 288 rows 34 38; 3136 x 7680, 257 rows 32 37), 129 to 144 rows of
+    more than 6528 outputs (7168 x 7168 42 45; 6400 x 6400 at 0.68), and up to
+    32 rows where those of w lie a multiple of 32 KB apart (4096 x 16384 31
+    42).  Narrow tiles where K is short and they fill as many units."""
     if not 16 < M <= 512 or K < (4096 if M <= 256 else 7168) or K % 128 \
             or N % 4 or N * K < 14 << 20:
         return None
+    if M <= 32 and K % 16384 == 0 and N >= 3072 \
+            or 128 < M <= 144 and N > 6528 and K <= 16384:
+        return None
 
     def parts(bm, bn):
-        tiles = -(-M // bm) * -(-N // bn)
-        return min(8, 256 // tiles), tiles
+        mt, nt = -(-M // bm), -(-N // bn)
+        die = 32 // mt * 8          # tiles of outputs and parts on all dies
+        return min(8, die // nt), mt * nt
 
     wide, tiles = parts(128, 128)
     if wide < (5 if M <= 128 else 2 if M <= 256 else 4):
         tall, _ = parts(256, 128)
-        return (256, 128, tall) if M > 256 and tall >= 4 else None
+        return (256, 128, tall) if M > 256 and tall >= 4 \
+            and (M > 320 or N > 3264 or K > 12288) else None
     narrow, more = parts(128, 64)
     if M <= 256 and K < 8192 and more * narrow >= tiles * wide:
         return 128, 64, narrow

@@ -45,7 +45,22 @@ def test_linear_takes_it(M, N, K):
     g = torch.Generator().manual_seed(M)
     x = torch.randn(M, K, generator=g).bfloat16().to(DEV)
     w = torch.randn(N, K, generator=g).bfloat16().to(DEV)
-    _check(ops.linear(x, w), x, w)
+    out = ops.linear(x, w)
+    _check(out, x, w)
+    route = "rows" if M == 17 and K == 4096 \
+        else "library" if M > 256 and (N, K) != (2048, 7168) else "split"
+    rule = None if ops._rows_gemm(x, w) else ops._split_gemm(M, N, K)
+    assert ops._rows_gemm(x, w) == (route == "rows")
+    assert (rule is None) == (route != "split")
+    again = torch.empty_like(out)
+    if route == "rows":
+        ops._native().gemm_rows(again, x, w)
+    elif route == "library":
+        again = x @ w.t()
+    else:
+        part = torch.empty(rule[2] * M * N, device=DEV)
+        ops._native().gemm_split(again, x, w, part, *rule)
+    assert torch.equal(out, again)
 
 
 def test_rule_stays_in_what_the_kernel_takes():
@@ -62,3 +77,26 @@ def test_rule_stays_in_what_the_kernel_takes():
                 assert 1 <= parts <= min(8, K // 128) and K % 128 == 0
                 assert -(-M // bm) * -(-N // bn) * parts <= 256
     assert taken
+
+
+def test_rule_leaves_no_workgroup_for_a_second_wave():
+    """Workgroups go to 8 dies of 32 units in turn, those of one tile of w to
+    the same."""
+    for M in range(17, 513, 5):
+        for N in range(512, 9000, 132):
+            for K in (4096, 7168, 8192, 13824):
+                rule = ops._split_gemm(M, N, K)
+                if rule is None:
+                    continue
+                bm, bn, parts = rule
+                assert -(-(-(-N // bn) * parts) // 8) * -(-M // bm) <= 32
+    assert ops._split_gemm(384, 2688, 7552) == (256, 128, 6)
+
+
+def test_sizes_where_the_library_is_faster():
+    for m, n, k in ((257, 3072, 8192), (17, 4096, 16384), (17, 1024, 8192),
+                    (144, 7168, 7168)):
+        assert ops._split_gemm(m, n, k) is None
+    for m, n, k in ((321, 3072, 8192), (257, 3584, 8192), (64, 4096, 16384),
+                    (144, 6144, 7168), (145, 7168, 7168)):
+        assert ops._split_gemm(m, n, k) is not None
