@@ -418,13 +418,14 @@ MOE_BM = 256  # sorted-pair tile granularity of the MoE kernels (csrc/moe.hip)
 
 
 def _moe_splitk(nblocks: int, nchunks: int, out_numel: int, dev):
-    """Split-K degree + fp32 workspace for a grouped GEMM launch.
+    """Split-K degree + fp32 workspace for a launch of csrc/moe.hip, the
+    grouped GEMM of large steps of the designs in ops/experts.py.
 
-    The w2 GEMM at Mixtral decode shapes has ~288 blocks for 256 CUs —
-    its ragged second wave idles most of the chip; splitting K into up
-    to 8 segments (each must keep >= 3 k-chunks for the LDS ring and
-    divide the chunk count) multiplies the block count back above ~4
-    per CU.  Shapes-only decision: hipGraph-capture-safe.
+    A launch of a few more blocks than the 256 CUs have idles most of the
+    chip in its second wave; splitting K into up to 8 segments (each must
+    keep >= 3 k-chunks for the LDS ring and divide the chunk count)
+    multiplies the block count back above ~4 per CU.  Shapes-only decision:
+    hipGraph-capture-safe.
     HS_MOE_SPLITK forces a degree (0 = auto)."""
     forced = int(os.environ.get("HS_MOE_SPLITK", "0"))
     s = 1

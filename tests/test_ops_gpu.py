@@ -258,67 +258,40 @@ def test_moe_grouped_ffn_matches_ref():
 
 
 @pytest.mark.gpu
-def test_moe_splitk_matches_single_segment():
-    """Split-K grouped GEMM (fp32 partials + reduce) == single-segment
-    kernel.  I=768 gives 12 k-chunks -> auto degree 4 at these tiny
-    block counts; HS_MOE_SPLITK pins each side."""
-    import os
+@pytest.mark.parametrize("segments", [1, 2, 4])
+def test_moe_splitk_matches_single_segment(segments):
+    """The grouped GEMM whose K may be split (fp32 partials + reduce), with
+    every degree that 12 k-chunks allow, against float64 on the same sorted
+    choices.  Bound: the result is rounded to bf16 (2^-9 of it), and sums of K
+    products are off by K 2^-24 of the sum of their sizes."""
     import hyperspot.ops as ops
+    from hyperspot import _C
     torch.manual_seed(1)
     dev = "cuda:0"
-    T, H, I, E, K = 160, 768, 768, 4, 2
-    x = (torch.randn(T, H, device=dev) * 0.3).to(torch.bfloat16)
-    w13 = (torch.randn(E, 2 * I, H, device=dev) * 0.04).to(torch.bfloat16)
-    w2 = (torch.randn(E, H, I, device=dev) * 0.04).to(torch.bfloat16)
-    logits = torch.randn(T, E, device=dev)
-    w, ids = logits.softmax(-1).topk(K, dim=-1)
-    w = (w / w.sum(-1, keepdim=True)).float()
-    ids = ids.to(torch.int32)
-    try:
-        os.environ["HS_MOE_SPLITK"] = "1"
-        base = ops.moe_ffn(x, w13, w2, w, ids)
-        os.environ["HS_MOE_SPLITK"] = "4"
-        sk = ops.moe_ffn(x, w13, w2, w, ids)
-    finally:
-        del os.environ["HS_MOE_SPLITK"]
-    # identical data path except fp32-partial accumulation order
-    err = (sk.float() - base.float()).abs().max().item()
-    assert err < 0.02 * base.float().abs().max().item() + 0.02, err
-    auto = ops.moe_ffn(x, w13, w2, w, ids)   # auto picks 4 here
-    err2 = (auto.float() - sk.float()).abs().max().item()
-    assert err2 == 0.0, err2
+    T, N, K, E, top = 160, 256, 768, 4, 2
+    x = (torch.randn(T, K, device=dev) * 0.3).to(torch.bfloat16)
+    w = (torch.randn(E, N, K, device=dev) * 0.04).to(torch.bfloat16)
+    ids = torch.randn(T, E, device=dev).topk(top, dim=-1).indices.int()
+    order, expert, place = ops._moe_sort(ids, E, N, K, ops.MOE_BM)
+    out = torch.full((order.numel(), N), float("nan"), dtype=torch.bfloat16,
+                     device=dev)
+    ws = torch.full((segments * out.numel(),), float("nan"), device=dev) \
+        if segments > 1 else None
+    _C.moe_gemm(out, x, w, order, expert, top, segments, ws)
+    xd, wd = x.double().cpu(), w.double().cpu()
+    got = out[place.long().view(-1)].double().cpu()
+    for c, e in enumerate(ids.view(-1).tolist()):
+        ref, size = wd[e] @ xd[c // top], wd[e].abs() @ xd[c // top].abs()
+        assert ((got[c] - ref).abs()
+                <= ref.abs() * 2.0 ** -8 + size * K * 2.0 ** -24).all()
 
 
 @pytest.mark.gpu
-def test_moe_splitk_fp8_matches_single_segment():
-    import os
+def test_moe_splitk_degree(monkeypatch):
+    """The degree that is chosen, and HS_MOE_SPLITK, which forces it."""
     import hyperspot.ops as ops
-    from hyperspot.parallel.layers import quantize_weight_fp8, \
-        quant_fp8_rowwise
-    torch.manual_seed(2)
-    dev = "cuda:0"
-    T, H, I, E, K = 128, 768, 768, 4, 2
-    x = (torch.randn(T, H, device=dev) * 0.3).to(torch.bfloat16)
-    w13 = [torch.randn(2 * I, H, device=dev) * 0.04 for _ in range(E)]
-    w2 = [torch.randn(H, I, device=dev) * 0.04 for _ in range(E)]
-    q13 = [quantize_weight_fp8(m) for m in w13]
-    q2 = [quantize_weight_fp8(m) for m in w2]
-    w13q = torch.stack([q for q, _ in q13])
-    w13s = torch.stack([s for _, s in q13])
-    w2q = torch.stack([q for q, _ in q2])
-    w2s = torch.stack([s for _, s in q2])
-    logits = torch.randn(T, E, device=dev)
-    w, ids = logits.softmax(-1).topk(K, dim=-1)
-    w = (w / w.sum(-1, keepdim=True)).float()
-    ids = ids.to(torch.int32)
-    xq_d, xq_s = quant_fp8_rowwise(x)
-    xq = ops.QTensor(xq_d, xq_s)
-    try:
-        os.environ["HS_MOE_SPLITK"] = "1"
-        base = ops.moe_ffn_fp8(xq, w13q, w13s, w2q, w2s, w, ids)
-        os.environ["HS_MOE_SPLITK"] = "4"
-        sk = ops.moe_ffn_fp8(xq, w13q, w13s, w2q, w2s, w, ids)
-    finally:
-        del os.environ["HS_MOE_SPLITK"]
-    err = (sk.float() - base.float()).abs().max().item()
-    assert err < 0.02 * base.float().abs().max().item() + 0.02, err
+    degree = lambda *a: ops._moe_splitk(*a, 64, "cuda:0")[0]
+    assert [degree(n, 12) for n in (12, 600, 1024)] == [4, 2, 1]
+    for forced in (1, 2, 4):
+        monkeypatch.setenv("HS_MOE_SPLITK", str(forced))
+        assert degree(12, 12) == forced and degree(1024, 12) == 1
