@@ -119,8 +119,6 @@ void launch_greedy_sample(long*, const T*, long, int, hipStream_t);
 template <typename T>
 void launch_sample(long*, const T*, const float*, const float*, const int*,
                    const float*, long, int, hipStream_t);
-void launch_inv_cdf_sample(long*, const float*, const float*, long, int,
-                           hipStream_t);
 
 namespace {
 
@@ -1061,16 +1059,6 @@ void sample(torch::Tensor out, torch::Tensor logits,
   });
 }
 
-void inv_cdf_sample(torch::Tensor out, torch::Tensor logits,
-                    torch::Tensor uniform) {
-  check(out, torch::kInt64, "out");
-  check(logits, torch::kFloat32, "logits");
-  check(uniform, torch::kFloat32, "uniform");
-  launch_inv_cdf_sample(out.data_ptr<long>(), logits.data_ptr<float>(),
-                        uniform.data_ptr<float>(), logits.size(0),
-                        (int)logits.size(1), stream());
-}
-
 }  // namespace
 
 
@@ -1188,5 +1176,4 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   register_sublayer(m);
   m.def("greedy_sample", &greedy_sample);
   m.def("sample", &sample);
-  m.def("inv_cdf_sample", &inv_cdf_sample);
 }

@@ -1,5 +1,5 @@
-// Sampling kernels: greedy argmax, inverse-CDF categorical draw, and the whole
-// of temperature, top-k, top-p and draw.
+// Sampling kernels: greedy argmax, and the whole of temperature, top-k, top-p
+// and draw.
 //
 // One workgroup per batch row over vocab-size logits (128256 for Llama-3).
 // Vectorized bf16/f32 reads; fp32 math, sums of weights in 64-bit integers.
@@ -55,77 +55,6 @@ __global__ __launch_bounds__(256) void greedy_sample_kernel(
       }
     out[blockIdx.x] = besti;
   }
-}
-
-// ---- inverse-CDF categorical draw (fp32 filtered logits) ----------------
-// logits already divided by temperature and masked (-inf) by top-k/top-p.
-// Exact semantics of the torch reference: j = first index with
-// cumsum(softmax(row)) > u (searchsorted right=False on the running CDF).
-__global__ __launch_bounds__(256) void inv_cdf_sample_kernel(
-    long* __restrict__ out, const float* __restrict__ logits,
-    const float* __restrict__ uniform, int vocab) {
-  __shared__ float scratch[4];
-  __shared__ float chunk_scan[256];
-  __shared__ int found;
-  const float* row = logits + (long)blockIdx.x * vocab;
-
-  // pass 1: max & normalizer
-  float mx = -FLT_MAX;
-  for (int t = threadIdx.x; t < vocab; t += 256)
-    mx = fmaxf(mx, row[t]);
-  mx = block_reduce_max_256(mx, scratch);
-  float z = 0.f;
-  for (int t = threadIdx.x; t < vocab; t += 256)
-    z += __expf(row[t] - mx);
-  z = block_reduce_sum_256(z, scratch);
-  const float target = uniform[blockIdx.x] * z;
-
-  // pass 2: walk 2048-element chunks; exclusive block scan over the 256
-  // per-thread partials finds the crossing chunk, then the owning thread
-  // walks its 8 elements.
-  if (threadIdx.x == 0) found = -1;
-  __syncthreads();
-  float running = 0.f;
-  for (int base = 0; base < vocab; base += 2048) {
-    float part = 0.f;
-    float e[8];
-    #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int t = base + threadIdx.x * 8 + i;
-      e[i] = (t < vocab) ? __expf(row[t] - mx) : 0.f;
-      part += e[i];
-    }
-    // inclusive scan over 256 thread partials (Hillis-Steele in LDS)
-    chunk_scan[threadIdx.x] = part;
-    __syncthreads();
-    for (int off = 1; off < 256; off <<= 1) {
-      const float prev = (threadIdx.x >= off)
-          ? chunk_scan[threadIdx.x - off] : 0.f;
-      __syncthreads();
-      chunk_scan[threadIdx.x] += prev;
-      __syncthreads();
-    }
-    const float total = chunk_scan[255];
-    if (found < 0 && running + total > target) {
-      const float before = running +
-          (threadIdx.x ? chunk_scan[threadIdx.x - 1] : 0.f);
-      if (before <= target && before + part > target) {
-        // this thread's 8-run contains the crossing
-        float c = before;
-        #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          c += e[i];
-          if (c > target) { found = base + threadIdx.x * 8 + i; break; }
-        }
-      }
-    }
-    __syncthreads();
-    if (found >= 0) break;
-    running += total;
-    __syncthreads();
-  }
-  if (threadIdx.x == 0)
-    out[blockIdx.x] = (found >= 0) ? min(found, vocab - 1) : vocab - 1;
 }
 
 // ---- temperature, top-k, top-p and draw ---------------------------------
@@ -782,10 +711,3 @@ template void launch_greedy_sample<bf16>(long*, const bf16*, long, int,
                                          hipStream_t);
 template void launch_greedy_sample<float>(long*, const float*, long, int,
                                           hipStream_t);
-
-void launch_inv_cdf_sample(long* out, const float* logits,
-                           const float* uniform, long rows, int vocab,
-                           hipStream_t stream) {
-  inv_cdf_sample_kernel<<<dim3((unsigned)rows), 256, 0, stream>>>(
-      out, logits, uniform, vocab);
-}
