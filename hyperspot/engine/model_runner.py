@@ -133,6 +133,7 @@ class ModelRunner:
         self._stage_dev = torch.empty_like(self._stage, device=self.device) \
             if pin else self._stage
         self._st_event = torch.cuda.Event() if pin else None
+        self._st_stream = None          # of the last decode step
         # guided-decoding logit-mask rows keyed by machine state
         self._guided_mask_cache: Dict[tuple, torch.Tensor] = {}
         self._graphs: Dict[int, torch.cuda.CUDAGraph] = {}
@@ -262,10 +263,14 @@ class ModelRunner:
         max_nt = int(bm.ntables_np[rows].max())
         bt = bm.tables_np[rows[:, None], np.arange(max_nt)[None, :]]
         if self._st_event is not None:
-            # the last step may still be copying from the staging buffer, or
-            # reading its copy: a step need not end in a device
-            # synchronization, nor run on this one's stream
+            # the last step's copy may still be reading the staging buffer: a
+            # step need not end in a device synchronization
             self._st_event.synchronize()
+            # nor run on this one's stream, which writes where it reads
+            stream = torch.cuda.current_stream(self.device)
+            if self._st_stream not in (None, stream):
+                stream.wait_stream(self._st_stream)
+            self._st_stream = stream
         cap = bm.capacity
         used = 5 * cap + (B * max_nt + 1) // 2
         st = self._stage.numpy()
@@ -277,11 +282,6 @@ class ModelRunner:
             d[:used].copy_(self._stage[:used], non_blocking=True)
             self._st_event.record()
         return d, B, max_nt
-
-    def _staged_read(self) -> None:
-        """The staged values are where the step reads them."""
-        if self._st_event is not None:
-            self._st_event.record()
 
     def _decode_meta(self, staged):
         """Tensors of an eager decode step from the staged values."""
@@ -434,13 +434,11 @@ class ModelRunner:
         if bucket is None or self.device.type != "cuda" \
                 or self.config.enforce_eager:
             input_ids, meta = self._decode_meta(staged)
-            self._staged_read()
             return self.model(input_ids, meta, self.kv_caches)
         if bucket not in self._graphs:
             self._capture(bucket)
         io = self._graph_io[bucket]
         ops.decode_inputs(stage, B, self.block_manager.capacity, max_nt, io)
-        self._staged_read()
         self._graphs[bucket].replay()
         return io["logits"][:B]
 

@@ -50,8 +50,8 @@ def test_incremental_decode_matches_full_recompute():
     assert out == ref
 
 
-def test_staging_is_free_when_the_step_has_read_it():
-    """The next step waits until this one's copy on the device is read too."""
+def test_a_step_on_another_stream_waits_for_the_last_one(monkeypatch):
+    """Its staged values go where the last step reads its own."""
     eng, log = _engine(), []
     runner = eng.runner
 
@@ -60,17 +60,21 @@ def test_staging_is_free_when_the_step_has_read_it():
             log.append("record")
 
         def synchronize(self):
-            log.append("wait")
+            log.append("host waits")
+
+    class Stream:
+        def wait_stream(self, other):
+            log.append((self, other))
 
     runner._st_event = Event()
-    meta = runner._decode_meta
-    runner._decode_meta = lambda staged: (log.append("read"), meta(staged))[1]
-    model = runner.model
-    runner.model = lambda *a: (log.append("model"), model(*a))[1]
-    eng.generate([[3, 4, 5]], SamplingParams(temperature=0.0, max_tokens=4))
-    steps = " ".join(log).split("wait")[1:]
-    assert len(steps) == 3
-    assert all(s.split()[-3:] == ["read", "record", "model"] for s in steps)
+    a, b = Stream(), Stream()
+    streams = iter([a, a, b, b, a])
+    monkeypatch.setattr(torch.cuda, "current_stream",
+                        lambda device=None: next(streams))
+    eng.generate([[3, 4, 5]], SamplingParams(temperature=0.0, max_tokens=6))
+    step = ["host waits", "record"]
+    assert log == [*step, *step, "host waits", (b, a), "record", *step,
+                   "host waits", (a, b), "record"]
 
 
 def test_batched_greedy_equals_single():
