@@ -298,7 +298,7 @@ void rope_paged_attn(torch::Tensor out, torch::Tensor q, torch::Tensor k,
 
 void attn_prefill_mfma(torch::Tensor out, torch::Tensor q, torch::Tensor k,
                        torch::Tensor v, torch::Tensor seq_start,
-                       long max_seqlen, double scale) {
+                       long /*max_seqlen*/, double scale) {
   check(out, torch::kBFloat16, "out");
   check_qkv_view(q, "q");
   check_qkv_view(k, "k");

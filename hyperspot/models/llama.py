@@ -52,7 +52,7 @@ class ForwardMeta:
     slot_mapping: torch.Tensor     # [T] int64 into the paged cache
     # prefill
     seq_start: Optional[torch.Tensor] = None   # [num_seqs+1] int32
-    max_seqlen: int = 0
+    max_seqlen: int = 0            # of the portions; no kernel needs it
     min_seqlen: int = 0            # 0: not known
     row_seq: Optional[torch.Tensor] = None     # [T] int32 row -> seq index
     ctx_lens: Optional[torch.Tensor] = None    # [T] int32 = position + 1
