@@ -36,9 +36,12 @@ struct Tiles {
   int N, K, div, nx;           // N outputs a choice, nx blocks of them
 };
 
-// 16-byte unit c of row r of a chunk in LDS: reads of 8 rows of one unit
-// spread over the banks
-DEV int unit(int r, int c) { return r * 128 + ((c ^ (r & 7)) << 4); }
+// 16-byte unit c of row r of a chunk in LDS.  16 lanes read at a time, 16 rows
+// of one unit, and two rows fill the 64 banks: so the unit turns with every
+// second row (with every row rows r and r + 8 met in a bank, and such reads ran
+// at 303 GB/s a compute unit, not 577; four prompts of 500 tokens through 4
+// layers of 8 experts of 14336 x 4096 5836 -> 5665 us).
+DEV int unit(int r, int c) { return r * 128 + ((c ^ (r >> 1 & 7)) << 4); }
 
 // BM choices, BN rows of weights; WM * WN waves have BM / WM by BN / WN
 template <int BM, int BN, int WM, int WN, int STAGES, bool GATED, bool FP8>
@@ -65,7 +68,8 @@ void experts_tiles_kernel(Tiles a) {
   const bool live = a.order[p0 + wm * (BM / WM)] >= 0;
 
   // this lane's 16 bytes of row lane / 8 of each 1-KB load
-  const int lr = lane >> 3, lc = ((lane & 7) ^ lr) * 16;
+  const int lr = lane >> 3;
+  auto column = [&](int r) { return ((lane & 7) ^ (r >> 1 & 7)) * 16; };
   const long row_bytes = (long)a.K * ELEM;
   auto row_of = [&](int p) {
     const int choice = a.order[p];
@@ -73,19 +77,22 @@ void experts_tiles_kernel(Tiles a) {
   };
   const char* xp[LX];
   #pragma unroll
-  for (int j = 0; j < LX; ++j)
-    xp[j] = static_cast<const char*>(a.x) +
-            row_of(p0 + (wid * LX + j) * 8 + lr) * row_bytes + lc;
+  for (int j = 0; j < LX; ++j) {
+    const int r = (wid * LX + j) * 8 + lr;
+    xp[j] = static_cast<const char*>(a.x) + row_of(p0 + r) * row_bytes +
+            column(r);
+  }
   const char* wp[LW];
   #pragma unroll
   for (int j = 0; j < LW; ++j) {
-    int n = (wid * LW + j) * 8 + lr;
+    const int r = (wid * LW + j) * 8 + lr;
+    int n = r;
     if constexpr (GATED)       // 8 gate rows, then their 8 up rows
       n = n0 + (n >> 4) * 8 + (n & 7) + (n & 8 ? a.N : 0);
     else
       n += n0;
     wp[j] = static_cast<const char*>(a.w) +
-            ((long)e * (GATED ? 2 * a.N : a.N) + n) * row_bytes + lc;
+            ((long)e * (GATED ? 2 * a.N : a.N) + n) * row_bytes + column(r);
   }
   auto stage = [&](int slot, int chunk) {
     char* base = lds + slot * STAGE;
