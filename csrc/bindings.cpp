@@ -118,7 +118,8 @@ template <typename T>
 void launch_greedy_sample(long*, const T*, long, int, hipStream_t);
 template <typename T>
 void launch_sample(long*, const T*, const float*, const float*, const int*,
-                   const float*, long, int, hipStream_t);
+                   const float*, void*, long, int, hipStream_t);
+long sample_workspace(long rows, int vocab);
 
 namespace {
 
@@ -1050,11 +1051,15 @@ void sample(torch::Tensor out, torch::Tensor logits,
   check(top_k, torch::kInt32, "top_k");
   TORCH_CHECK(top_k.numel() == rows, "top_k");
   check_param(uniform, rows, "uniform");
+  const long bytes = sample_workspace(rows, (int)logits.size(1));
+  torch::Tensor ws;
+  if (bytes) ws = torch::empty({bytes}, out.options().dtype(torch::kUInt8));
   by_dtype(logits, [&](auto tag) {
     using T = ELEM(tag);
     launch_sample<T>(out.data_ptr<long>(), ptr<T>(logits),
                      ptr<float>(temperature), ptr<float>(top_p),
-                     top_k.data_ptr<int>(), ptr<float>(uniform), rows,
+                     top_k.data_ptr<int>(), ptr<float>(uniform),
+                     bytes ? ws.data_ptr() : nullptr, rows,
                      (int)logits.size(1), stream());
   });
 }

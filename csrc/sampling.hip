@@ -66,27 +66,28 @@ __global__ __launch_bounds__(256) void greedy_sample_kernel(
 // temperature 0: the largest logit, the first among equals.  A logit that is
 // NaN is not drawn.
 //
-// What bounds it: vector instructions on every value, in passes over the row,
-// which stays in L2: 8 us for the largest, 20 for the weights of 128256.  So 8
-// values are looked at together where that decides about all of them.  Where
-// few values stay, and next-token logits have a few dozen that matter, they are
-// listed in the second pass and the rest is done on the list, up to 8 threads a
-// value.  Otherwise no sort either: one histogram of counts and weights over
-// 2048 equal steps between the largest and the smallest logit finds the step
-// where the wanted count or share is reached, and ranks the few values in it
-// exactly (or divides that step again).  Equal steps of the logit, and not
+// What bounds it: vector instructions on every value, about 20 for a weight, and
+// the chains of steps that a row's workgroup takes one after the other.  So a row
+// is divided into slices where there are few rows (below): 64 rows of 128256 are
+// 256 workgroups, 7 us for the largest values, 12 with the weights, and a second
+// kernel of 3 (greedy) to 13 us (a share).  8 values are looked at together where
+// that decides about all of them.  Where few values stay, and next-token logits
+// have a few dozen that matter, they are listed and the rest is done on the list,
+// up to 8 threads a value.  Otherwise no sort either: one histogram of counts and
+// weights over 2048 equal steps between the largest and the smallest logit finds
+// the step where the wanted count or share is reached, and ranks the few values
+// in it exactly (or divides that step again).  Equal steps of the logit, and not
 // digits of its bit pattern, because next-token logits fill few exponents: 64
 // lanes that add to the same few counters in LDS would go one by one.
 //
-// 64 rows of 128256, 48 values far above the others, us with the histogram
-// alone and now: greedy 15 11, temperature 57 38, top_p 0.9 115 39, top_k 50
-// 85 27, top_k 40 and top_p 141 28; a mix 138 45, where the library's sorts,
-// scans and selections took 2625.  Normal logits, whose share is thousands of
-// values, 155 132.
+// 64 rows of 128256, 48 values far above the others, us with a workgroup a row
+// and now: temperature 41 17, top_p 0.9 42 24, top_k 50 30 17, greedy 14 10; a
+// mix 43 24.5, where the library's sorts, scans and selections took 2625.
+// Normal logits, whose share is thousands of values, 132 124.
 //
-// Weights are 2^-40 fixed point relative to the largest, so every sum is
-// exact, does not depend on its order, and the same inputs give the same
-// token.
+// Weights are 2^-40 fixed point relative to the largest (of the row or of the
+// slice), so every sum is exact, does not depend on its order, and the same
+// inputs give the same token.
 namespace {
 
 typedef unsigned long long u64;
@@ -100,8 +101,10 @@ struct Weight {
   float mx, hi, lo;               // hi + lo = log2(e) / temperature
   // false: weights of x and less are below half of 2^-40
   DEV bool any(float x) const { return (x - mx) * hi > -42.f; }
-  DEV u64 operator()(float x) const {
-    if (!any(x)) return 0;
+  DEV u64 operator()(float x) const { return any(x) ? always(x) : 0; }
+  // the same without a branch: the weights that `any` rules out, an infinity's
+  // and a NaN's among them, come out as zero
+  DEV u64 always(float x) const {
     const float d = x - mx, t = d * hi;
     const float r = fmaf(d, hi, -t) + d * lo;
     float e = __builtin_amdgcn_exp2f(t);
@@ -142,12 +145,16 @@ template <typename I> DEV I wave_scan(I x) {      // inclusive
   return x;
 }
 
+struct alignas(16) Entry {        // one LDS load
+  u64 key, mass;
+};
+
 struct Scratch {
   u64 mass[STEPS];
   unsigned count[STEPS];
   float list[LIST];
-  u64 list_mass[LIST];
   int list_at[LIST];
+  Entry entry[LIST];
   u64 wave_mass[16];
   unsigned wave_count[16];
   u64 before_mass, kept_mass;
@@ -197,6 +204,32 @@ template <typename T, bool VEC> struct Row {
       #pragma unroll
       for (int i = 0; i < 8; ++i) x[i] = in_range(x[i]);
   }
+  // the same from anywhere: elements one by one where they are not aligned
+  DEV void hold(int at, int end, Raw& r) const {
+    if constexpr (VEC) {
+      fetch(at, end, r);
+    } else if constexpr (sizeof(T) == 2) {
+      unsigned u[4];
+      #pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        unsigned h[2];
+        #pragma unroll
+        for (int j = 0; j < 2; ++j)
+          h[j] = at + 2 * i + j < end
+              ? reinterpret_cast<const unsigned short*>(p)[at + 2 * i + j]
+              : 0xff80u;
+        u[i] = h[0] | h[1] << 16;
+      }
+      r.v = uint4{u[0], u[1], u[2], u[3]};
+    } else {
+      #pragma unroll
+      for (int i = 0; i < 8; ++i)
+        r.v[i] = at + i < end ? Elem<T>::ld(p + at + i) : -INFINITY;
+    }
+  }
+  DEV void spread(const Raw& r, float* x) const {
+    Row<T, true>{p, vocab, finite}.unpack({r.v}, 0, 0, x);
+  }
   // f(8 values, index of the first) of all values and of some -inf past the end
   template <typename F> DEV void each8(F f) const {
     for (int at = threadIdx.x * 8; at < vocab; at += AHEAD * NT * 8) {
@@ -218,13 +251,12 @@ template <typename T, bool VEC> struct Row {
     });
   }
 
-  // First index at which the running sum of w(x, index) exceeds the target
-  // that `of` makes of the whole sum; vocab - 1 if there is none.  A wave has a
-  // sixteenth; the one where the target lies is divided again.
+  // First index in [first, end) at which the running sum of w(x, index) exceeds
+  // the target that `of` makes of the whole sum; vocab - 1 if there is none.  A
+  // wave has a sixteenth; the one where the target lies is divided again.
   template <typename W, typename F>
-  DEV int walk(Scratch& s, W w, F of) const {
+  DEV int walk(Scratch& s, W w, F of, int first, int end) const {
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    int first = 0, end = vocab;
     u64 before = 0, target = 0;
     for (bool whole = true;; whole = false) {
       const int span = (end - first + 16 * 512 - 1) / (16 * 512) * 512;
@@ -276,6 +308,10 @@ template <typename T, bool VEC> struct Row {
       first += owner * span;
       end = min(first + span, end);
     }
+  }
+  template <typename W, typename F>
+  DEV int walk(Scratch& s, W w, F of) const {
+    return walk(s, w, of, 0, vocab);
   }
 };
 
@@ -365,7 +401,7 @@ DEV void reach(Scratch& s, const R& row, const Weight& w, float lo, float hi,
         const unsigned at = atomicAdd(&s.n, 1u);
         if (at < LIST) {
           s.list[at] = x;
-          s.list_mass[at] = w(x);
+          s.entry[at].mass = w(x);
         }
         const unsigned key = ordered(x);
         if (key < s.key_min) atomicMin(&s.key_min, key);
@@ -390,14 +426,14 @@ DEV void reach(Scratch& s, const R& row, const Weight& w, float lo, float hi,
     if (members <= LIST) {
       if (tid < members) {
         const float x = s.list[tid];
-        const u64 one = s.list_mass[tid];
+        const u64 one = s.entry[tid].mass;
         u64 mb = mass0;
         unsigned cb = count0, equal = 0;
         for (unsigned j = 0; j < members; ++j) {
           const float y = s.list[j];
           equal += y == x;
           if (y > x) {
-            mb += s.list_mass[j];
+            mb += s.entry[j].mass;
             ++cb;
           }
         }
@@ -414,6 +450,91 @@ DEV void reach(Scratch& s, const R& row, const Weight& w, float lo, float hi,
     }
     __syncthreads();
   }
+}
+
+DEV u64 sum_of_all(Scratch& s, u64 x) {
+  #pragma unroll
+  for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o);
+  if ((threadIdx.x & 63) == 0) s.wave_mass[threadIdx.x >> 6] = x;
+  __syncthreads();
+  x = 0;
+  #pragma unroll
+  for (int v = 0; v < 16; ++v) x += s.wave_mass[v];
+  return x;
+}
+
+// The draw from the s.n values that are listed, if all that stays is among
+// them.  k 0: no top_k, and z is the weight of all values, of which top_p is a
+// share.  False if the list is too short for the share or too long.
+DEV bool draw_from_list(Scratch& s, const Weight& w, int vocab, int k, float p,
+                        float u, u64 z, int* drawn) {
+  const int tid = threadIdx.x;
+  const int n = (int)s.n;
+  if (n > LIST) {
+    __syncthreads();
+    return false;
+  }
+  // in descending order, and by index among equals, larger keys are earlier;
+  // the zeros are equal
+  if (tid < n)
+    s.entry[tid] = {(u64)ordered(s.list[tid] + 0.f) << 32 |
+                        (unsigned)~s.list_at[tid],
+                    w(s.list[tid])};
+  if (tid == 0) s.found = vocab - 1;
+  __syncthreads();
+  // `share` neighbouring threads a value, each with a part of the others
+  const int share = n <= NT / 8 ? 8 : n <= NT / 4 ? 4 : 2;
+  const int mine = tid / share, part = tid % share;
+  const bool one_of = mine < n;
+  auto sum = [&](auto v) {
+    for (int o = 1; o < share; o <<= 1) v += __shfl_xor(v, o);
+    return v;
+  };
+  Entry own{0, 0};
+  u64 above = 0;
+  int greater = 0;
+  if (one_of) {
+    own = s.entry[mine];
+    #pragma unroll 4
+    for (int j = part; j < n; j += share) {
+      const Entry e = s.entry[j];
+      above += e.key > own.key ? e.mass : 0;
+      greater += (unsigned)(e.key >> 32) > (unsigned)(own.key >> 32);
+    }
+  }
+  above = sum(above);
+  greater = sum(greater);
+  bool stays = one_of && (k == 0 || greater < k);
+  const u64 listed = sum_of_all(s, stays && part == 0 ? own.mass : 0);
+  if (p < 1.f) {
+    const u64 want = (u64)ceil((double)p * (double)(k ? listed : z));
+    if (listed < want) {
+      __syncthreads();
+      return false;
+    }
+    stays = stays && above < want;
+  }
+  // every thread has read the entries: now by index, what does not stay as 0
+  const int index = (int)~(unsigned)own.key;
+  if (one_of && part == 0)
+    s.entry[mine] = {(u64)(unsigned)index, stays ? own.mass : 0};
+  __syncthreads();
+  u64 all = 0, upto = 0;
+  if (stays) {
+    #pragma unroll 4
+    for (int j = part; j < n; j += share) {
+      const Entry e = s.entry[j];
+      all += e.mass;
+      upto += (int)e.key < index ? e.mass : 0;
+    }
+  }
+  all = sum(all);
+  upto = sum(upto);
+  const u64 target = (u64)((double)u * (double)all);
+  if (stays && upto <= target && upto + own.mass > target) s.found = index;
+  __syncthreads();
+  *drawn = s.found;
+  return true;
 }
 
 // The draw where all that stays is among few values: the want-th largest of the
@@ -434,10 +555,7 @@ DEV bool draw_from_few(Scratch& s, const R& row, const Weight& w, float own,
   }
   const float least =
       prefix > ordered(-FLT_MAX) ? from_ordered(prefix) : -FLT_MAX;
-  if (tid == 0) {
-    s.n = 0;
-    s.value = -INFINITY;
-  }
+  if (tid == 0) s.n = 0;
   __syncthreads();
   u64 z = 0;                      // the share is one of this
   row.each8([&](const float* x, int at) {
@@ -459,123 +577,16 @@ DEV bool draw_from_few(Scratch& s, const R& row, const Weight& w, float own,
   z = wave_scan(z);
   if (lane == 63) s.wave_mass[wid] = z;
   __syncthreads();
-  const int n = (int)s.n;
   z = 0;
   for (int v = 0; v < 16; ++v) z += s.wave_mass[v];
   *all = z;
-  if (tid < n && n <= LIST) s.list_mass[tid] = w(s.list[tid]);
-  __syncthreads();
-  if (n > LIST) return false;
-  // `share` neighbouring threads a value, each with a part of the others
-  const int share = n <= NT / 8 ? 8 : n <= NT / 4 ? 4 : 2;
-  const int mine = tid / share, part = tid % share;
-  const bool one_of = mine < n;
-  auto sum = [&](auto v) {
-    for (int o = 1; o < share; o <<= 1) v += __shfl_xor(v, o);
-    return v;
-  };
-  float x = -INFINITY;
-  int index = 0;
-  u64 one = 0, above = 0;
-  int before = 0, equal = 0, earlier = 0;
-  if (one_of) {
-    x = s.list[mine];
-    index = s.list_at[mine];
-    one = s.list_mass[mine];
-    #pragma unroll 2
-    for (int j = part; j < n; j += share) {
-      const float y = s.list[j];
-      above += y > x ? s.list_mass[j] : 0;
-      before += y > x;
-      equal += y == x;
-      earlier += y == x && s.list_at[j] < index;
-    }
-  }
-  above = sum(above);
-  before = sum(before);
-  equal = sum(equal);
-  earlier = sum(earlier);
-  float low = -INFINITY;
-  if (k > 0) {
-    if (one_of && before < k && before + equal >= k) {
-      s.value = x;                // every member of the group writes the same
-      s.kept_mass = above + one * equal;
-    }
-    __syncthreads();
-    low = s.value;
-    if (low > -INFINITY)
-      z = s.kept_mass;
-    else                          // fewer than k values: all are in the list
-      for (int j = 0; j < n; ++j) z += s.list_mass[j];
-  }
-  int last = row.vocab;
-  if (p < 1.f) {
-    const u64 want = (u64)ceil((double)p * (double)z);
-    if (tid == 0) s.found = -1;
-    __syncthreads();
-    if (one_of && x >= low && above < want && above + one * equal >= want &&
-        (u64)earlier + 1 == (want - above + one - 1) / one) {
-      s.value = x;
-      s.found = index;
-    }
-    __syncthreads();
-    low = s.value;
-    last = s.found;
-    __syncthreads();
-    if (last < 0) return false;
-  }
-  const bool stays = one_of && (x > low || (x == low && index <= last));
-  if (one_of && !stays) s.list_mass[mine] = 0;
-  if (tid == 0) s.found = row.vocab - 1;
-  __syncthreads();
-  u64 all_kept = 0, upto = 0;
-  if (stays)
-    #pragma unroll 2
-    for (int j = part; j < n; j += share) {
-      const u64 m = s.list_mass[j];
-      all_kept += m;
-      upto += s.list_at[j] < index ? m : 0;
-    }
-  all_kept = sum(all_kept);
-  upto = sum(upto);
-  const u64 target = (u64)((double)u * (double)all_kept);
-  if (stays && upto <= target && upto + one > target) s.found = index;
-  __syncthreads();
-  *drawn = s.found;
-  return true;
+  return draw_from_list(s, w, row.vocab, k, p, u, z, drawn);
 }
 
-template <typename T, bool VEC>
-__global__ __launch_bounds__(NT) void sample_kernel(
-    long* __restrict__ out, const T* __restrict__ logits,
-    const float* __restrict__ temperature, const float* __restrict__ top_p,
-    const int* __restrict__ top_k, const float* __restrict__ uniform,
-    int vocab) {
-  __shared__ Scratch s;
-  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-  const long b = blockIdx.x;
-  Row<T, VEC> row{logits + b * vocab, vocab, true};
-
-  // the largest value, where its first 8 values are, and the smallest; neither
-  // is that of a NaN
-  float mx = -INFINITY, mn = INFINITY;
-  int at = vocab;
-  row.each8([&](const float* x, int i) {
-    const float m = largest(x);
-    if (m > mx && mx < FLT_MAX) {
-      mx = fminf(m, FLT_MAX);
-      at = i;
-    }
-    if constexpr (VEC) {
-      const float n = smallest(x);
-      if (i < vocab) mn = fminf(mn, n);
-    } else {
-      #pragma unroll
-      for (int j = 0; j < 8; ++j)
-        if (x[j] >= -FLT_MAX) mn = fminf(mn, x[j]);
-    }
-  });
-  const float own = mx;
+// Best of all threads: the largest value mx, the lowest index `at` of the 8
+// that hold it first, and the smallest value mn.
+DEV void best_of_all(Scratch& s, float& mx, int& at, float& mn) {
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   #pragma unroll
   for (int o = 32; o > 0; o >>= 1) {
     const float x = __shfl_xor(mx, o);
@@ -601,55 +612,41 @@ __global__ __launch_bounds__(NT) void sample_kernel(
     }
     mn = fminf(mn, s.list[16 + v]);
   }
-  mn = fminf(mn, mx);
   __syncthreads();
-  const float t = temperature[b];
-  if (t == 0.f || !(mx >= -FLT_MAX)) {          // or there is no value
-    if (tid == 0) {
-      int first = t == 0.f ? 0 : vocab - 1;
-      if (mx >= -FLT_MAX) {
-        for (first = at; in_range(Elem<T>::ld(row.p + first)) != mx;)
-          ++first;
-      }
-      out[b] = first;
-    }
-    return;
-  }
-  row.finite = mx < FLT_MAX;
+}
 
-  const double c = 1.4426950408889634 / (double)fmaxf(t, 1e-6f);
-  const Weight w{mx, (float)c, (float)(c - (double)(float)c)};
+// The index of the largest value mx, which is among the 8 from `at` on, the
+// first among equals; that of a row without a value
+template <typename T>
+DEV int greedy_index(const T* p, float mx, int at, int vocab, int none) {
+  if (!(mx >= -FLT_MAX)) return none;
+  float x[8];
+  #pragma unroll
+  for (int i = 0; i < 8; ++i)
+    x[i] = in_range(Elem<T>::ld(p + min(at + i, vocab - 1)));
+  int first = 7;
+  #pragma unroll
+  for (int i = 6; i >= 0; --i)
+    if (x[i] == mx) first = i;
+  return at + first;
+}
+
+// The draw by passes over the row.  kept: the weight of all values, or 0 where
+// it is not known.
+template <typename R>
+DEV int draw_from_row(Scratch& s, const R& row, const Weight& w, float mn,
+                      float c, int k, float p, float uniform, u64 kept) {
+  const float mx = w.mx;
   // below this weights are zero
-  const float floor = mx - 64.f / (float)c;
+  const float floor = mx - 64.f / c;
   const float lo = mn >= -FLT_MAX ? fmaxf(mn, floor) : floor;
   float low = -INFINITY;          // values above it stay
   int last = -1;                  // and its equals up to this index
-  u64 kept = 0;                   // their weight, 0: not known
-  const int k = top_k[b];
-  const float p = top_p[b];
-  if (p < 1.f && !(p > 0.f)) {    // nothing stays
-    if (tid == 0) out[b] = vocab - 1;
-    return;
-  }
-  const bool cut = k > 0 && k < vocab;
-  // a share is not looked for where many threads' largest values weigh more
-  // than 2^-7 of the largest: the list would be too short
-  if (cut ? k <= LIST / 2
-          : p < 1.f && __syncthreads_count((own - mx) * w.hi > -7.f) <=
-                           2 * FEW) {
-    int drawn;
-    if (draw_from_few(s, row, w, own, cut ? k : 0, p, uniform[b], &kept,
-                      &drawn)) {
-      if (tid == 0) out[b] = drawn;
-      return;
-    }
-    __syncthreads();
-  }
-  if (cut) {
+  if (k > 0) {
     reach<true>(s, row, w, lo, mx, k);
     low = s.value;
     kept = s.keep == ~0u ? 0 : s.kept_mass;
-    last = vocab;
+    last = row.vocab;
     __syncthreads();
   }
   if (p < 1.f) {
@@ -669,37 +666,423 @@ __global__ __launch_bounds__(NT) void sample_kernel(
                       [&](u64 z) { return min((u64)keep, z) - 1; });
     }
   }
-  const int drawn = row.walk(
+  return row.walk(
       s,
       [&](float x, int i) {
         return x > low || (x == low && i <= last) ? w(x) : 0;
       },
-      [&](u64 z) { return (u64)((double)uniform[b] * (double)z); });
+      [&](u64 z) { return (u64)((double)uniform * (double)z); });
+}
+
+struct Options {
+  float t, p, uniform, hi, lo;    // hi + lo = log2(e) / temperature
+  int k;                          // 0: no cut
+  DEV Weight weight(float mx) const { return {mx, hi, lo}; }
+};
+
+DEV Options options_of(long b, const float* temperature, const float* top_p,
+                       const int* top_k, const float* uniform, int vocab) {
+  Options o;
+  o.t = temperature[b];
+  o.p = top_p[b];
+  o.uniform = uniform[b];
+  const int k = top_k[b];
+  o.k = k > 0 && k < vocab ? k : 0;
+  const double c = 1.4426950408889634 / (double)fmaxf(o.t, 1e-6f);
+  o.hi = (float)c;
+  o.lo = (float)(c - (double)o.hi);
+  return o;
+}
+
+template <typename T, bool VEC>
+__global__ __launch_bounds__(NT) void sample_kernel(
+    long* __restrict__ out, const T* __restrict__ logits,
+    const float* __restrict__ temperature, const float* __restrict__ top_p,
+    const int* __restrict__ top_k, const float* __restrict__ uniform,
+    int vocab) {
+  __shared__ Scratch s;
+  const int tid = threadIdx.x;
+  const long b = blockIdx.x;
+  Row<T, VEC> row{logits + b * vocab, vocab, true};
+
+  // the largest value, where its first 8 values are, and the smallest; neither
+  // is that of a NaN
+  float mx = -INFINITY, mn = INFINITY;
+  int at = vocab;
+  row.each8([&](const float* x, int i) {
+    const float m = largest(x);
+    if (m > mx && mx < FLT_MAX) {
+      mx = fminf(m, FLT_MAX);
+      at = i;
+    }
+    if constexpr (VEC) {
+      const float n = smallest(x);
+      if (i < vocab) mn = fminf(mn, n);
+    } else {
+      #pragma unroll
+      for (int j = 0; j < 8; ++j)
+        if (x[j] >= -FLT_MAX) mn = fminf(mn, x[j]);
+    }
+  });
+  const float own = mx;
+  best_of_all(s, mx, at, mn);
+  mn = fminf(mn, mx);
+  const Options o = options_of(b, temperature, top_p, top_k, uniform, vocab);
+  if (o.t == 0.f || !(mx >= -FLT_MAX)) {        // or there is no value
+    if (tid == 0)
+      out[b] = greedy_index(row.p, mx, at, vocab,
+                            o.t == 0.f ? 0 : vocab - 1);
+    return;
+  }
+  row.finite = mx < FLT_MAX;
+  const Weight w = o.weight(mx);
+  if (o.p < 1.f && !(o.p > 0.f)) {              // nothing stays
+    if (tid == 0) out[b] = vocab - 1;
+    return;
+  }
+  u64 kept = 0;
+  int drawn;
+  // a share is not looked for where many threads' largest values weigh more
+  // than 2^-7 of the largest: the list would be too short
+  bool done = o.k ? o.k <= LIST / 2
+                  : o.p < 1.f && __syncthreads_count((own - mx) * w.hi > -7.f)
+                                     <= 2 * FEW;
+  if (done) {
+    done = draw_from_few(s, row, w, own, o.k, o.p, o.uniform, &kept, &drawn);
+    __syncthreads();
+  }
+  if (!done)
+    drawn = draw_from_row(s, row, w, mn, o.hi, o.k, o.p, o.uniform, kept);
   if (tid == 0) out[b] = drawn;
+}
+
+// ---- rows in slices -------------------------------------------------------
+// A row a workgroup leaves most of the chip idle.  Here a row is divided into
+// slices of a workgroup each, which read their values once; what they find out
+// meets in a second kernel, a workgroup a row.  Weights are relative to the
+// slice's own largest value, so that no slice waits for another one; the sums of
+// 512 values are exact, and are brought to the row's largest value by one factor
+// a slice.
+constexpr int HELD = 4;           // 8 values each, that a thread has
+constexpr int SLICES = 16;        // of a row at most
+constexpr int UNITS = 4;          // a thread of the second kernel has at most
+constexpr int CHUNKS = HELD * 16; // 512 values of a wave each
+
+struct Slice {
+  u64 mass[CHUNKS];               // weights of the chunks, where asked for
+  float mx, mn;                   // largest (-inf: no value), smallest
+  int at;                         // first of the 8 with the first largest
+  int pad;
+  float own[NT];                  // largest values of the threads, or of 2 or 4
+};
+
+// threads of a slice whose values are looked at together
+DEV int together(int slices) { return slices <= 4 ? 1 : slices <= 8 ? 2 : 4; }
+
+template <typename T, bool VEC>
+__global__ __launch_bounds__(NT) void sample_slice_kernel(
+    Slice* __restrict__ slice, const T* __restrict__ logits,
+    const float* __restrict__ temperature, const float* __restrict__ top_p,
+    const int* __restrict__ top_k, int vocab, int slices, int span) {
+  __shared__ Scratch s;
+  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+  const long b = blockIdx.x / slices;
+  const int first = (int)(blockIdx.x % slices) * span;
+  const int end = min(first + span, vocab);
+  Slice& mine = slice[blockIdx.x];
+  Row<T, VEC> row{logits + b * vocab, vocab, true};
+  typename Row<T, VEC>::Raw raw[HELD];
+  #pragma unroll
+  for (int q = 0; q < HELD; ++q)
+    row.hold(first + (q * NT + tid) * 8, end, raw[q]);
+  const Options o = options_of(b, temperature, top_p, top_k, temperature,
+                               vocab);
+  float mx = -INFINITY, mn = INFINITY;
+  int at = vocab;
+  #pragma unroll
+  for (int q = 0; q < HELD; ++q) {
+    const int i = first + (q * NT + tid) * 8;
+    float x[8];
+    row.spread(raw[q], x);
+    const float m = largest(x), n = smallest(x);
+    if (m > mx && mx < FLT_MAX) {
+      mx = fminf(m, FLT_MAX);
+      at = i;
+    }
+    if (i + 8 <= end) mn = fminf(mn, n);
+  }
+  float own = mx;
+  const int group = together(slices);
+  for (int i = 1; i < group; i <<= 1) own = fmaxf(own, __shfl_xor(own, i));
+  if (tid % group == 0) mine.own[tid / group] = own;
+  best_of_all(s, mx, at, mn);
+  if (tid == 0) {
+    mine.mx = mx;
+    mine.mn = mn;
+    mine.at = at;
+  }
+  if (o.t == 0.f || o.k || !(mx >= -FLT_MAX)) {
+    if (tid < CHUNKS) mine.mass[tid] = 0;
+    return;
+  }
+  const Weight w = o.weight(mx);
+  row.finite = mx < FLT_MAX;
+  #pragma unroll
+  for (int q = 0; q < HELD; ++q) {
+    float x[8];
+    row.spread(raw[q], x);
+    u64 z = 0;
+    if (w.any(largest(x)))
+      #pragma unroll
+      for (int i = 0; i < 8; ++i) z += w.always(x[i]);
+    #pragma unroll
+    for (int i = 32; i > 0; i >>= 1) z += __shfl_xor(z, i);
+    if (lane == 0) mine.mass[q * 16 + wid] = z;
+  }
+}
+
+template <typename T, bool VEC>
+__global__ __launch_bounds__(NT) void sample_slices_kernel(
+    long* __restrict__ out, const Slice* __restrict__ slice,
+    const T* __restrict__ logits, const float* __restrict__ temperature,
+    const float* __restrict__ top_p, const int* __restrict__ top_k,
+    const float* __restrict__ uniform, int vocab, int slices, int span) {
+  __shared__ Scratch s;
+  __shared__ int unit[LIST];
+  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+  const long b = blockIdx.x;
+  slice += b * slices;
+  Row<T, VEC> row{logits + b * vocab, vocab, true};
+  // All loads are issued before anything waits: chunk `tid` of the row, the
+  // largest values of UNITS units, and by lane i of 16 what slice i says.
+  const u64 chunk = slice[min(tid / CHUNKS, slices - 1)].mass[tid % CHUNKS];
+  const int group = together(slices), each = NT / group;   // units a slice
+  float own[UNITS];
+  #pragma unroll
+  for (int q = 0; q < UNITS; ++q) {
+    const int i = q * NT + tid;
+    own[q] = i < slices * each ? slice[i / each].own[i % each] : -INFINITY;
+  }
+  const Slice& head = slice[min(lane & 15, slices - 1)];
+  const float slice_mx = head.mx;
+  float mx = slice_mx, mn = head.mn;
+  int at = head.at;
+  const Options o = options_of(b, temperature, top_p, top_k, uniform, vocab);
+  if (tid == 0) s.n = 0;
+  s.count[tid] = 0;
+  #pragma unroll
+  for (int x = 1; x < 16; x <<= 1) {
+    const float m = __shfl_xor(mx, x);
+    const int i = __shfl_xor(at, x);
+    if (m > mx || (m == mx && i < at)) {
+      mx = m;
+      at = i;
+    }
+    mn = fminf(mn, __shfl_xor(mn, x));
+  }
+  mn = fminf(mn, mx);
+  if (o.t == 0.f || !(mx >= -FLT_MAX)) {
+    if (tid == 0)
+      out[b] = greedy_index(row.p, mx, at, vocab, o.t == 0.f ? 0 : vocab - 1);
+    return;
+  }
+  if (o.p < 1.f && !(o.p > 0.f)) {              // nothing stays
+    if (tid == 0) out[b] = vocab - 1;
+    return;
+  }
+  const Weight w = o.weight(mx);
+  u64 z = 0;                      // weight of all
+  if (!o.k) {
+    const double factor = exp2(((double)slice_mx - (double)mx) *
+                               ((double)o.hi + (double)o.lo));
+    const double share = __shfl(factor, tid / CHUNKS & 15);
+    const u64 mass = tid < slices * CHUNKS && chunk
+        ? (u64)rint((double)chunk * share) : 0;
+    const u64 upto = wave_scan(mass);
+    if (lane == 63) s.wave_mass[wid] = upto;
+    __syncthreads();
+    u64 before = 0;
+    for (int v = 0; v < 16; ++v) {
+      if (v == wid) before = z;
+      z += s.wave_mass[v];
+    }
+    if (!(o.p < 1.f)) {
+      // the token is in the chunk where the running sum passes the target;
+      // there sums are those of the slice's own weights again
+      const u64 target = (u64)((double)o.uniform * (double)z);
+      if (target >= z) {
+        if (tid == 0) out[b] = vocab - 1;
+        return;
+      }
+      // a wave has the chunks of one slice, in the order of its values
+      const u64 over = __ballot(before + upto > target);
+      if (before > target || !over) return;
+      const int i = __ffsll(over) - 1, of = wid;
+      const u64 all = __shfl(chunk, i);
+      const double part = (double)(target - before - __shfl(upto - mass, i)) /
+                          (double)__shfl(mass, i);
+      const u64 goal = min((u64)(part * (double)all), all - 1);
+      const Weight wi = o.weight(__shfl(slice_mx, of));
+      row.finite = wi.mx < FLT_MAX;
+      const int stop = min((of + 1) * span, vocab);
+      const int from = of * span + i * 512 + lane * 8;
+      typename Row<T, VEC>::Raw raw;
+      row.hold(from, stop, raw);
+      float x[8];
+      row.spread(raw, x);
+      u64 sum = 0;
+      #pragma unroll
+      for (int j = 0; j < 8; ++j) sum += wi.always(x[j]);
+      const u64 mine = wave_scan(sum);
+      const u64 here = __ballot(mine > goal);
+      if (lane == __ffsll(here) - 1) {
+        u64 c = mine - sum;
+        int found = 0;
+        #pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          c += wi.always(x[j]);
+          found += c <= goal;
+        }
+        out[b] = from + found;
+      }
+      return;
+    }
+  }
+  row.finite = mx < FLT_MAX;
+  // The draw where all that stays is among few values: the want-th largest of
+  // the units' largest values has at least that many values at or above it, and
+  // hardly more.  A share is not looked for where many units' largest values
+  // weigh more than 2^-7 of the largest: the list would be too short.
+  int near = 0;
+  #pragma unroll
+  for (int q = 0; q < UNITS; ++q)
+    near += __popcll(__ballot((own[q] - mx) * w.hi > -7.f));
+  // steps below the largest value, down to where weights are zero
+  const float zero = 43.f / w.hi;
+  const float scale = NT / fmaxf(mn >= -FLT_MAX ? fminf(mx - mn, zero) : zero,
+                                 1e-30f);
+  __syncthreads();
+  if (lane == 0) atomicAdd(&s.n, (unsigned)near);
+  #pragma unroll
+  for (int q = 0; q < UNITS; ++q) {
+    const float step = (mx - own[q]) * scale;
+    if (step < (float)NT) atomicAdd(&s.count[(int)step], 1u);
+  }
+  __syncthreads();
+  int drawn;
+  bool done = o.k ? o.k <= LIST / 2 : s.n <= 2 * FEW;
+  if (done) {
+    const unsigned upto = wave_scan(s.count[tid]);
+    if (lane == 63) s.wave_count[wid] = upto;
+    if (tid == 0) {
+      s.n = 0;
+      s.step = NT;
+    }
+    __syncthreads();
+    unsigned before = 0;
+    for (int v = 0; v < wid; ++v) before += s.wave_count[v];
+    const unsigned want = o.k ? o.k : FEW;
+    if (before + upto >= want && before + upto - s.count[tid] < want)
+      s.step = tid + 1;
+    __syncthreads();
+    const float end = (float)s.step;
+    #pragma unroll
+    for (int q = 0; q < UNITS; ++q)
+      if ((mx - own[q]) * scale < end) {
+        const unsigned n = atomicAdd(&s.n, 1u);
+        if (n < LIST) unit[n] = q * NT + tid;
+      }
+    __syncthreads();
+    const int units = (int)s.n;
+    __syncthreads();
+    if (tid == 0) s.n = 0;
+    __syncthreads();
+    done = units <= LIST;
+    if (done) {
+      // loads of 8 values: of `group` threads, as often as those loaded
+      const int loads = group * ((span + NT * 8 - 1) / (NT * 8));
+      for (int i = tid; i < units * loads; i += NT) {
+        const int u = unit[i / loads], j = i % loads, of = u / each;
+        const int from = of * span +
+            (j / group * NT + u % each * group + j % group) * 8;
+        typename Row<T, VEC>::Raw raw;
+        row.hold(from, min((of + 1) * span, vocab), raw);
+        float x[8];
+        row.spread(raw, x);
+        #pragma unroll
+        for (int v = 0; v < 8; ++v)
+          if ((mx - x[v]) * scale < end) {
+            const unsigned n = atomicAdd(&s.n, 1u);
+            if (n < LIST) {
+              s.list[n] = x[v];
+              s.list_at[n] = from + v;
+            }
+          }
+      }
+      __syncthreads();
+      done = draw_from_list(s, w, vocab, o.k, o.p, o.uniform, z, &drawn);
+    }
+    __syncthreads();
+  }
+  if (!done)
+    drawn = draw_from_row(s, row, w, mn, o.hi, o.k, o.p, o.uniform, z);
+  if (tid == 0) out[b] = drawn;
+}
+
+// Slices of a row, 0: none.  As many as give every compute unit a workgroup, if
+// each has a load for every thread.  Beyond two workgroups a unit the chip is
+// full of whole rows (256 rows of 128256 52 us, in 4 slices 57; of 50257 50 and
+// in 2 slices 50; of 32000 31 and in one 28).
+int sample_slices(long rows, int vocab) {
+  const int least = (vocab + HELD * NT * 8 - 1) / (HELD * NT * 8);
+  const int most = min(SLICES, max(1, vocab / (NT * 8)));
+  if (least > SLICES || rows * least > 512) return 0;
+  return max(least, min(most, (int)(256 / rows)));
 }
 
 }  // namespace
 
+// bytes of the workspace, 0: none is needed
+long sample_workspace(long rows, int vocab) {
+  return rows * sample_slices(rows, vocab) * (long)sizeof(Slice);
+}
+
+// ws null: a workgroup a row
 template <typename T>
 void launch_sample(long* out, const T* logits, const float* temperature,
                    const float* top_p, const int* top_k, const float* uniform,
-                   long rows, int vocab, hipStream_t stream) {
+                   void* ws, long rows, int vocab, hipStream_t stream) {
   if (rows == 0) return;
+  const bool vec = vocab % 8 == 0 && reinterpret_cast<size_t>(logits) % 16 == 0;
+  const int slices = ws ? sample_slices(rows, vocab) : 0;
+  const int span = slices ? ((vocab + slices - 1) / slices + 7) / 8 * 8 : 0;
+  Slice* slice = static_cast<Slice*>(ws);
   #define RUN(VEC)                                                          \
-    sample_kernel<T, VEC><<<dim3((unsigned)rows), NT, 0, stream>>>(         \
-        out, logits, temperature, top_p, top_k, uniform, vocab)
-  if (vocab % 8 == 0 && reinterpret_cast<size_t>(logits) % 16 == 0)
-    RUN(true);
-  else
-    RUN(false);
+    if (slices) {                                                           \
+      sample_slice_kernel<T, VEC>                                           \
+          <<<(unsigned)(rows * slices), NT, 0, stream>>>(                   \
+              slice, logits, temperature, top_p, top_k, vocab, slices,      \
+              span);                                                        \
+      sample_slices_kernel<T, VEC><<<(unsigned)rows, NT, 0, stream>>>(      \
+          out, slice, logits, temperature, top_p, top_k, uniform, vocab,    \
+          slices, span);                                                    \
+    } else {                                                                \
+      sample_kernel<T, VEC><<<(unsigned)rows, NT, 0, stream>>>(             \
+          out, logits, temperature, top_p, top_k, uniform, vocab);          \
+    }
+  if (vec) {
+    RUN(true)
+  } else {
+    RUN(false)
+  }
   #undef RUN
 }
 template void launch_sample<bf16>(long*, const bf16*, const float*,
                                   const float*, const int*, const float*,
-                                  long, int, hipStream_t);
+                                  void*, long, int, hipStream_t);
 template void launch_sample<float>(long*, const float*, const float*,
                                    const float*, const int*, const float*,
-                                   long, int, hipStream_t);
+                                   void*, long, int, hipStream_t);
 
 template <typename T>
 void launch_greedy_sample(long* out, const T* logits, long rows, int vocab,

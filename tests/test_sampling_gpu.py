@@ -136,6 +136,44 @@ def test_nan_is_not_drawn(vocab, dtype):
     assert not gone[:-1].gather(1, nan[:-1, None].cpu()).any()
 
 
+@pytest.mark.parametrize("vocab,rows", [
+    (16384, 1), (32768, 100), (32776, 100), (65537, 40), (128256, 1),
+    (128256, 30), (128256, 60), (128256, 129), (524288, 1), (524296, 1)])
+def test_rows_in_slices(vocab, rows):
+    """1 to 16 slices a row, one value more than a slice takes, and rows that
+    are not divided; what is likely lies in one slice, at its end or anywhere."""
+    g = torch.Generator().manual_seed(vocab + rows)
+    options = [(0.0, 1.0, 0), (1.0, 1.0, 0), (0.7, 0.9, 0), (0.9, 1.0, 50),
+               (0.8, 0.95, 40), (1.0, 0.5, 250), (1.0, 1.0, 300),
+               (3.0, 0.9, 0)]
+    x = torch.randn(8, vocab, generator=g)
+    x[0, -3:] += 9
+    x[1, :40] += 14
+    x[2, torch.randint(0, vocab, (60,), generator=g)] += 18
+    x[3] = (x[3] * 2).round()
+    x[4, : vocab // 2] = float("-inf")
+    x[5, 100:] = float("-inf")
+    x[6] = 1.0
+    x[7, vocab // 3] = float("inf")
+    x = x.bfloat16()
+    pick = [(i, o) for i in range(8) for o in range(8)]
+    pick = (pick * (rows // 64 + 1))[:max(rows, 64) // rows * rows]
+    u = torch.rand(len(pick), generator=g)
+    t, p, k = (torch.tensor(c)
+               for c in zip(*(options[o] for _, o in pick)))
+    which = torch.tensor([i for i, _ in pick])
+    out = torch.cat([
+        ops.sample(*(c.to(DEV) for c in (x[which[a]], t[a], p[a], k[a].int(),
+                                         u[a])))
+        for a in torch.arange(len(pick)).split(rows)]).tolist()
+    for b, (i, o) in enumerate(pick[:64]):
+        row = x[i].float().clamp(max=torch.finfo(torch.float32).max)
+        ok, _ = _allowed(row, *options[o], float(u[b]))
+        assert ok[out[b]], (i, options[o], out[b], float(u[b]))
+        if o == 0:
+            assert out[b] == int(row.argmax())
+
+
 def test_one_option_for_all_rows():
     """Options of one element count for every row; top_k of 64 bits."""
     g = torch.Generator().manual_seed(1)
