@@ -12,6 +12,9 @@ void launch_rmsnorm(bf16*, const bf16*, const bf16*, float, long, int,
                     hipStream_t);
 void launch_parts_add_rmsnorm(bf16*, const float*, int, bf16*, const bf16*,
                               float, long, int, hipStream_t);
+void launch_choices_add_rmsnorm(bf16*, const bf16*, const int*, const float*,
+                                int, bool, bf16*, const bf16*, float, long, int,
+                                hipStream_t);
 void launch_fused_add_rmsnorm(bf16*, bf16*, const bf16*, float, long, int,
                               hipStream_t);
 void launch_rope_kv_append(bf16*, bf16*, const bf16*, const long*,
@@ -158,6 +161,35 @@ void parts_add_rmsnorm(torch::Tensor x, torch::Tensor parts,
   launch_parts_add_rmsnorm(bf(x), parts.data_ptr<float>(), (int)parts.size(0),
                            bf(residual), cbf(w), (float)eps, rows, hidden,
                            stream());
+}
+
+// x <- rmsnorm(residual + y) * w and residual that sum, y the weighted sum of a
+// row's choices, rows of `data`: place [rows, n], weight [rows, n]
+void choices_add_rmsnorm(torch::Tensor x, torch::Tensor data,
+                         torch::Tensor place, torch::Tensor weight,
+                         bool direct, torch::Tensor residual, torch::Tensor w,
+                         double eps) {
+  check(x, torch::kBFloat16, "x");
+  check(data, torch::kBFloat16, "data");
+  check(place, torch::kInt32, "place");
+  check(weight, torch::kFloat, "weight");
+  check(residual, torch::kBFloat16, "residual");
+  check(w, torch::kBFloat16, "w");
+  TORCH_CHECK(data.dim() == 2 && place.dim() == 2 && place.size(1) >= 1 &&
+                  weight.sizes() == place.sizes(),
+              "choices_add_rmsnorm: shape");
+  const long rows = place.size(0);
+  const int hidden = (int)data.size(1);
+  TORCH_CHECK(hidden % 8 == 0 && hidden <= 8192 && w.numel() == hidden &&
+                  x.numel() == rows * hidden &&
+                  residual.numel() == x.numel() &&
+                  (!direct || data.size(0) >= place.numel()),
+              "choices_add_rmsnorm: shape");
+  if (rows == 0) return;
+  launch_choices_add_rmsnorm(bf(x), cbf(data), place.data_ptr<int>(),
+                             weight.data_ptr<float>(), (int)place.size(1),
+                             direct, bf(residual), cbf(w), (float)eps, rows,
+                             hidden, stream());
 }
 
 void fused_add_rmsnorm(torch::Tensor x, torch::Tensor residual,
@@ -1155,6 +1187,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gemm_rows_fits", &gemm_rows_fits);
   m.def("gemm_split", &gemm_split);
   m.def("parts_add_rmsnorm", &parts_add_rmsnorm);
+  m.def("choices_add_rmsnorm", &choices_add_rmsnorm);
   m.def("silu_mul", &silu_mul);
   m.def("gelu_mul", &gelu_mul);
   m.def("embed_dyt", &embed_dyt);

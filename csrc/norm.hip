@@ -172,6 +172,98 @@ __global__ __launch_bounds__(256) void parts_add_rmsnorm_kernel(
   }
 }
 
+// x <- rmsnorm(residual + y) * w ; residual <- residual + y, where y is the
+// weighted sum of a row's n choices, rounded as it would be on its own: weight
+// [row, k] * data[place[row, k]] (place -1: nothing; `direct`: data[row * n + k]
+// where place is not negative).  A launch and a trip to memory less than the sum
+// and the norm; the choices' rows are loaded 4 at a time beside the rest.
+// us of both and of one: 4 rows of 2048, 4 choices 5.9 -> 3.1; 192 of 4096, 2
+// choices 7.4 -> 3.7; 2000 of them 22 -> 13; 8000 75 -> 48.
+template <int CH>
+__global__ __launch_bounds__(256) void choices_add_rmsnorm_kernel(
+    bf16* __restrict__ x, const bf16* __restrict__ data,
+    const int* __restrict__ place, const float* __restrict__ weight, int n,
+    bool direct, bf16* __restrict__ residual, const bf16* __restrict__ w,
+    float eps, int hidden) {
+  __shared__ float scratch[4];
+  const long row = blockIdx.x;
+  bf16* xr = x + row * (long)hidden;
+  bf16* rr = residual + row * (long)hidden;
+
+  bf16x8 rv[CH], wv[CH];
+  #pragma unroll
+  for (int c = 0; c < CH; ++c) {
+    const int base = (c * 256 + threadIdx.x) * 8;
+    if (base < hidden) {
+      rv[c] = load_bf16x8(rr + base);
+      wv[c] = load_bf16x8(w + base);
+    }
+  }
+  float r[CH][8];
+  #pragma unroll
+  for (int c = 0; c < CH; ++c)
+    #pragma unroll
+    for (int i = 0; i < 8; ++i) r[c][i] = 0.f;
+  for (int k0 = 0; k0 < n; k0 += 4) {
+    long from[4];
+    float share[4];
+    #pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const long i = row * n + min(k0 + k, n - 1);
+      from[k] = k0 + k < n ? place[i] : -1;
+      share[k] = weight[i];
+      if (direct && from[k] >= 0) from[k] = i;
+    }
+    bf16x8 yv[4][CH];
+    #pragma unroll
+    for (int k = 0; k < 4; ++k)
+      #pragma unroll
+      for (int c = 0; c < CH; ++c) {
+        const int base = (c * 256 + threadIdx.x) * 8;
+        if (from[k] >= 0 && base < hidden)
+          yv[k][c] = load_bf16x8(data + from[k] * hidden + base);
+      }
+    #pragma unroll
+    for (int k = 0; k < 4; ++k)
+      if (from[k] >= 0) {
+        #pragma unroll
+        for (int c = 0; c < CH; ++c)
+          #pragma unroll
+          for (int i = 0; i < 8; ++i)
+            r[c][i] += share[k] * bf16x8_get(yv[k][c], i);
+      }
+  }
+  float ss = 0.f;
+  #pragma unroll
+  for (int c = 0; c < CH; ++c) {
+    const int base = (c * 256 + threadIdx.x) * 8;
+    if (base < hidden) {
+      bf16x8 o;
+      #pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const float f = bf2f(f2bf(r[c][i])) + bf16x8_get(rv[c], i);
+        r[c][i] = f;
+        ss += f * f;
+        bf16x8_set(o, i, f);
+      }
+      store_bf16x8(rr + base, o);   // new residual
+    }
+  }
+  const float total = block_reduce_sum_256(ss, scratch);
+  const float rs = rsqrtf(total / hidden + eps);
+  #pragma unroll
+  for (int c = 0; c < CH; ++c) {
+    const int base = (c * 256 + threadIdx.x) * 8;
+    if (base < hidden) {
+      bf16x8 o;
+      #pragma unroll
+      for (int i = 0; i < 8; ++i)
+        bf16x8_set(o, i, r[c][i] * rs * bf16x8_get(wv[c], i));
+      store_bf16x8(xr + base, o);
+    }
+  }
+}
+
 // chunks that hold a row of up to 4096, 8192 or 16384 elements
 static int chunks(int hidden) {
   return hidden <= 4096 ? 2 : hidden <= 8192 ? 4 : 8;
@@ -205,4 +297,16 @@ void launch_parts_add_rmsnorm(bf16* x, const float* part, int parts,
                                        : parts_add_rmsnorm_kernel<4>;
   kernel<<<dim3((unsigned)rows), dim3(256), 0, stream>>>(
       x, part, parts, residual, w, eps, hidden);
+}
+
+// hidden at most 8192
+void launch_choices_add_rmsnorm(bf16* x, const bf16* data, const int* place,
+                                const float* weight, int n, bool direct,
+                                bf16* residual, const bf16* w, float eps,
+                                long rows, int hidden, hipStream_t stream) {
+  const auto kernel = hidden <= 2048   ? choices_add_rmsnorm_kernel<1>
+                      : hidden <= 4096 ? choices_add_rmsnorm_kernel<2>
+                                       : choices_add_rmsnorm_kernel<4>;
+  kernel<<<dim3((unsigned)rows), dim3(256), 0, stream>>>(
+      x, data, place, weight, n, direct, residual, w, eps, hidden);
 }

@@ -21,7 +21,7 @@ from hyperspot import ops
 from hyperspot.engine.config import ModelSpec
 from hyperspot.models.llama import DecoderLayer, LlamaForCausalLM
 from hyperspot.parallel.layers import (_init_weight, _QUANT_MODE,
-                                       quantize_weight_fp8)
+                                       quantize_weight_fp8, summands)
 from hyperspot.parallel.state import get_ep_group, get_ep_rank, get_ep_size
 
 
@@ -118,6 +118,18 @@ class MixtralMoE(nn.Module):
                                    ids.to(torch.int32))
             return self._local_moe(x, weights.to(x.dtype), ids)
         return self._ep_moe(x, weights.to(x.dtype), ids.long())
+
+    def _summands(self, x):
+        """The experts' outputs before their sum, where all of them are here in
+        16 bits and the norm takes their width."""
+        if not isinstance(x, torch.Tensor) or not x.is_cuda \
+                or x.dtype != torch.bfloat16 or x.shape[0] == 0 \
+                or not 0 < x.shape[1] <= 8192 or self.quant is not None \
+                or get_ep_size() > 1 or not ops.have_native():
+            return self.forward(x)
+        weights, ids = self._route_gpu(x)
+        return ops.moe_choices(x, self.w13, self.w2, weights,
+                               ids.to(torch.int32))
 
     def _fused_router(self, x: torch.Tensor) -> bool:
         return x.is_cuda and ops.have_native() and x.is_contiguous() \
@@ -332,6 +344,9 @@ class _MoEAdapter(nn.Module):
 
     def forward(self, x):
         return self.moe(x)
+
+    def _summands(self, x):
+        return summands(self.moe, x)
 
 
 class MixtralForCausalLM(LlamaForCausalLM):

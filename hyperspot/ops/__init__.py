@@ -44,6 +44,17 @@ class Parts(NamedTuple):
     data: torch.Tensor
 
 
+class Choices(NamedTuple):
+    """Outputs of experts whose weighted sum is still to be formed: row t is the
+    sum over k of weights[t, k] * data[place[t, k]], without those of place -1.
+    direct: choice k of row t is data[t * K + k]."""
+
+    data: torch.Tensor
+    place: torch.Tensor          # [T, K] int32
+    weights: torch.Tensor        # [T, K] float
+    direct: bool
+
+
 def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
     if x.is_cuda:
         out = torch.empty_like(x)
@@ -56,7 +67,13 @@ def fused_add_rmsnorm(x: torch.Tensor, residual: torch.Tensor,
                       weight: torch.Tensor, eps: float):
     """residual += x (in place); x_out = rmsnorm(residual) (in place on x).
 
-    x may be the Parts of a product, which are added up on the way."""
+    x may be the Parts of a product or the Choices of experts, which are added
+    up on the way."""
+    if isinstance(x, Choices):
+        out = torch.empty_like(residual)
+        _native().choices_add_rmsnorm(out, x.data, x.place, x.weights,
+                                      x.direct, residual, weight, eps)
+        return out, residual
     if isinstance(x, Parts):
         out = torch.empty_like(residual)
         _native().parts_add_rmsnorm(out, x.data, residual, weight, eps)
@@ -394,6 +411,8 @@ def fused_add_rmsnorm_q(x: torch.Tensor, residual: torch.Tensor,
     residual).  GPU-only fused producer for the fp8 GEMM path."""
     if isinstance(x, Parts):      # of a layer with 16-bit weights before it
         x = x.data.sum(0).to(residual.dtype)
+    elif isinstance(x, Choices):
+        x = _moe_sum(x)
     assert x.is_cuda
     T, K = x.shape
     out = torch.empty(T, K, dtype=torch.float8_e4m3fn, device=x.device)
@@ -496,11 +515,12 @@ def _moe_sort(ids: torch.Tensor, E: int, H: int, I: int, bm: int):
     return order, expert, place
 
 
-def _moe_sum(y, place, weights) -> torch.Tensor:
+def _moe_sum(c: Choices) -> torch.Tensor:
+    y, place = c.data, c.place
     out = torch.empty(place.shape[0], y.shape[1], dtype=y.dtype,
                       device=y.device)
-    _native().experts_sum(out, y, place, weights.float().contiguous(), None,
-                          None, None, None, 0.0)
+    _native().experts_sum(out, y, place, c.weights, None, None, None, None,
+                          0.0)
     return out
 
 
@@ -514,10 +534,16 @@ def moe_ffn(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor,
     with grids that depend only on (T, K, E) — no host sync, no dynamic
     shapes (MoE dispatch/combine + grouped GEMM).
     """
+    if x.shape[0] == 0:
+        return torch.empty_like(x)
+    return _moe_sum(moe_choices(x, w13, w2, weights, ids))
+
+
+def moe_choices(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor,
+                weights: torch.Tensor, ids: torch.Tensor) -> Choices:
+    """moe_ffn of at least one token without its closing sum."""
     n = _native()
     (T, H), K, (E, _, I) = x.shape, ids.shape[1], w2.shape
-    if T == 0:
-        return torch.empty_like(x)
     bm = _moe_tile(T, K, E, 16)
     order, expert, place = _moe_sort(ids, E, H, I, bm)
     P = order.shape[0]
@@ -529,7 +555,7 @@ def moe_ffn(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor,
     else:
         n.experts_tiles(h, x, w13, None, None, order, expert, True, K, bm)
         n.experts_tiles(y, h, w2, None, None, order, expert, False, 0, bm)
-    return _moe_sum(y, place, weights)
+    return Choices(y, place, weights.float().contiguous(), False)
 
 
 def moe_ffn_fp8(xq: "QTensor", w13q: torch.Tensor, w13s: torch.Tensor,
@@ -553,7 +579,7 @@ def moe_ffn_fp8(xq: "QTensor", w13q: torch.Tensor, w13s: torch.Tensor,
                     bm)
     a = silu_mul_q(h)
     n.experts_tiles(y, a.data, w2q, a.scale, w2s, order, expert, False, 0, bm)
-    return _moe_sum(y, place, weights)
+    return _moe_sum(Choices(y, place, weights.float().contiguous(), False))
 
 
 def decode_inputs(stage: torch.Tensor, rows: int, cap: int, pages: int,
