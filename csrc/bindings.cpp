@@ -13,7 +13,7 @@ void launch_rmsnorm(bf16*, const bf16*, const bf16*, float, long, int,
 void launch_parts_add_rmsnorm(bf16*, const float*, int, bf16*, const bf16*,
                               float, long, int, hipStream_t);
 void launch_choices_add_rmsnorm(bf16*, const bf16*, const int*, const float*,
-                                int, bool, bf16*, const bf16*, float, long, int,
+                                int, bf16*, const bf16*, float, long, int,
                                 hipStream_t);
 void launch_fused_add_rmsnorm(bf16*, bf16*, const bf16*, float, long, int,
                               hipStream_t);
@@ -37,6 +37,8 @@ void launch_attn_prefill_paged(bf16*, const bf16*, const bf16*, const bf16*,
                                const int*, const int*, const int*, int, long,
                                int, int, int, int, float, long, bool,
                                hipStream_t);
+void launch_experts_few(bool, bf16*, int*, const bf16*, const bf16*, const int*,
+                        int, int, int, int, int, hipStream_t);
 template <typename T>
 void launch_gelu_mul(T*, const T*, long, int, hipStream_t);
 template <typename T>
@@ -167,8 +169,7 @@ void parts_add_rmsnorm(torch::Tensor x, torch::Tensor parts,
 // row's choices, rows of `data`: place [rows, n], weight [rows, n]
 void choices_add_rmsnorm(torch::Tensor x, torch::Tensor data,
                          torch::Tensor place, torch::Tensor weight,
-                         bool direct, torch::Tensor residual, torch::Tensor w,
-                         double eps) {
+                         torch::Tensor residual, torch::Tensor w, double eps) {
   check(x, torch::kBFloat16, "x");
   check(data, torch::kBFloat16, "data");
   check(place, torch::kInt32, "place");
@@ -182,14 +183,13 @@ void choices_add_rmsnorm(torch::Tensor x, torch::Tensor data,
   const int hidden = (int)data.size(1);
   TORCH_CHECK(hidden % 8 == 0 && hidden <= 8192 && w.numel() == hidden &&
                   x.numel() == rows * hidden &&
-                  residual.numel() == x.numel() &&
-                  (!direct || data.size(0) >= place.numel()),
+                  residual.numel() == x.numel(),
               "choices_add_rmsnorm: shape");
   if (rows == 0) return;
   launch_choices_add_rmsnorm(bf(x), cbf(data), place.data_ptr<int>(),
                              weight.data_ptr<float>(), (int)place.size(1),
-                             direct, bf(residual), cbf(w), (float)eps, rows,
-                             hidden, stream());
+                             bf(residual), cbf(w), (float)eps, rows, hidden,
+                             stream());
 }
 
 void fused_add_rmsnorm(torch::Tensor x, torch::Tensor residual,
@@ -200,6 +200,34 @@ void fused_add_rmsnorm(torch::Tensor x, torch::Tensor residual,
   TORCH_CHECK(hidden % 8 == 0 && hidden <= 16384, "hidden size");
   launch_fused_add_rmsnorm(bf(x), bf(residual), cbf(w), (float)eps,
                            x.numel() / hidden, hidden, stream());
+}
+
+// Products of P choices with their experts' weights w [E, 2N (up) or N, K]:
+// out [P, N], x [P / div, K] (up) or [P, K], ids [P] int32 from -1 (none); place
+// [P] int32 becomes p, or -1 where there is none
+void experts_few(bool up, torch::Tensor out,
+                 c10::optional<torch::Tensor> place, torch::Tensor x,
+                 torch::Tensor w, torch::Tensor ids, long div) {
+  check(out, torch::kBFloat16, "out");
+  check(x, torch::kBFloat16, "x");
+  check(w, torch::kBFloat16, "w");
+  check(ids, torch::kInt32, "ids");
+  TORCH_CHECK(out.dim() == 2 && x.dim() == 2 && w.dim() == 3 && div >= 1,
+              "experts_few: shape");
+  const long P = ids.numel(), N = out.size(1), K = x.size(1);
+  TORCH_CHECK(P >= 1 && P <= 384 && out.size(0) == P &&
+                  x.size(0) * (up ? div : 1) == P && w.size(2) == K &&
+                  w.size(1) == (up ? 2 * N : N) && w.size(0) >= 1 &&
+                  N % 128 == 0 && K % 128 == 0,
+              "experts_few: shape");
+  if (place.has_value()) {
+    check(*place, torch::kInt32, "place");
+    TORCH_CHECK(place->numel() == P, "experts_few: place");
+  }
+  launch_experts_few(up, bf(out),
+                     place.has_value() ? place->data_ptr<int>() : nullptr,
+                     cbf(x), cbf(w), ids.data_ptr<int>(), (int)P,
+                     (int)w.size(0), (int)N, (int)K, (int)div, stream());
 }
 
 // q/k/v may be strided views into one fused qkv buffer: require only the
@@ -1187,6 +1215,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gemm_rows_fits", &gemm_rows_fits);
   m.def("gemm_split", &gemm_split);
   m.def("parts_add_rmsnorm", &parts_add_rmsnorm);
+  m.def("experts_few", &experts_few);
   m.def("choices_add_rmsnorm", &choices_add_rmsnorm);
   m.def("silu_mul", &silu_mul);
   m.def("gelu_mul", &gelu_mul);

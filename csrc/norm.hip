@@ -174,17 +174,17 @@ __global__ __launch_bounds__(256) void parts_add_rmsnorm_kernel(
 
 // x <- rmsnorm(residual + y) * w ; residual <- residual + y, where y is the
 // weighted sum of a row's n choices, rounded as it would be on its own: weight
-// [row, k] * data[place[row, k]] (place -1: nothing; `direct`: data[row * n + k]
-// where place is not negative).  A launch and a trip to memory less than the sum
-// and the norm; the choices' rows are loaded 4 at a time beside the rest.
+// [row, k] * data[place[row, k]] (place -1: nothing).  A launch and a trip to
+// memory less than the sum and the norm; the choices' rows are loaded 4 at a time
+// beside the rest.
 // us of both and of one: 4 rows of 2048, 4 choices 5.9 -> 3.1; 192 of 4096, 2
 // choices 7.4 -> 3.7; 2000 of them 22 -> 13; 8000 75 -> 48.
 template <int CH>
 __global__ __launch_bounds__(256) void choices_add_rmsnorm_kernel(
     bf16* __restrict__ x, const bf16* __restrict__ data,
     const int* __restrict__ place, const float* __restrict__ weight, int n,
-    bool direct, bf16* __restrict__ residual, const bf16* __restrict__ w,
-    float eps, int hidden) {
+    bf16* __restrict__ residual, const bf16* __restrict__ w, float eps,
+    int hidden) {
   __shared__ float scratch[4];
   const long row = blockIdx.x;
   bf16* xr = x + row * (long)hidden;
@@ -212,7 +212,6 @@ __global__ __launch_bounds__(256) void choices_add_rmsnorm_kernel(
       const long i = row * n + min(k0 + k, n - 1);
       from[k] = k0 + k < n ? place[i] : -1;
       share[k] = weight[i];
-      if (direct && from[k] >= 0) from[k] = i;
     }
     bf16x8 yv[4][CH];
     #pragma unroll
@@ -301,12 +300,12 @@ void launch_parts_add_rmsnorm(bf16* x, const float* part, int parts,
 
 // hidden at most 8192
 void launch_choices_add_rmsnorm(bf16* x, const bf16* data, const int* place,
-                                const float* weight, int n, bool direct,
-                                bf16* residual, const bf16* w, float eps,
-                                long rows, int hidden, hipStream_t stream) {
+                                const float* weight, int n, bf16* residual,
+                                const bf16* w, float eps, long rows,
+                                int hidden, hipStream_t stream) {
   const auto kernel = hidden <= 2048   ? choices_add_rmsnorm_kernel<1>
                       : hidden <= 4096 ? choices_add_rmsnorm_kernel<2>
                                        : choices_add_rmsnorm_kernel<4>;
   kernel<<<dim3((unsigned)rows), dim3(256), 0, stream>>>(
-      x, data, place, weight, n, direct, residual, w, eps, hidden);
+      x, data, place, weight, n, residual, w, eps, hidden);
 }

@@ -46,13 +46,12 @@ class Parts(NamedTuple):
 
 class Choices(NamedTuple):
     """Outputs of experts whose weighted sum is still to be formed: row t is the
-    sum over k of weights[t, k] * data[place[t, k]], without those of place -1.
-    direct: choice k of row t is data[t * K + k]."""
+    sum over k of weights[t, k] * data[place[t, k]], without those of place
+    -1."""
 
     data: torch.Tensor
     place: torch.Tensor          # [T, K] int32
     weights: torch.Tensor        # [T, K] float
-    direct: bool
 
 
 def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
@@ -72,7 +71,7 @@ def fused_add_rmsnorm(x: torch.Tensor, residual: torch.Tensor,
     if isinstance(x, Choices):
         out = torch.empty_like(residual)
         _native().choices_add_rmsnorm(out, x.data, x.place, x.weights,
-                                      x.direct, residual, weight, eps)
+                                      residual, weight, eps)
         return out, residual
     if isinstance(x, Parts):
         out = torch.empty_like(residual)
@@ -482,15 +481,17 @@ def moe_router(x, router: torch.Tensor, top: int):
     return weight, ids
 
 
-# Mean rows per expert up to which tiles of 16, 64 and 128 rows are taken (and
-# 256 beyond).  64 and 128 leave room for the spread of the counts: a few rows
-# more and an expert's weights are read twice.  us on an MI355X for tiles of
-#   16 (rows), 64, 128, 256
-#   8 experts of 14336 x 4096   4 rows 544 536 565 710, 48 1723 543 589 732,
-#     64 - 665 594 728, 96 - 798 601 762, 150 - 1118 937 729
-#   16 of 2048 x 4096           4 rows 175 202 204 223, 16 254 202 207 230
-#   32 of 1024 x 2048           2 rows 93 92 102 116, 64 321 119 118 137
-MOE_ROWS, MOE_ROWS_64, MOE_ROWS_128 = 6, 52, 112
+# Mean rows per expert up to which the kernels without a sort, and tiles of 64
+# and 128 rows are taken (and 256 beyond).  64 and 128 leave room for the spread
+# of the counts: a few rows more and an expert's weights are read twice.  us on
+# an MI355X without a sort, and in tiles of 64, 128, 256
+#   8 experts of 14336 x 4096   1 row 336 398, 4 rows 481 492, 5 531 508, 48 -
+#     543 589 732, 64 - 665 594 728, 96 - 798 601 762, 150 - 1118 937 729
+#   16 of 2048 x 4096           1 row 107 132, 4 rows 151 173, 6 162 174, 16 -
+#     202 207 230
+#   32 of 1024 x 2048           2 rows 68 81, 5 84 90, 8 97 92, 64 - 119 118 137
+#   64 of 1024 x 2048           3 rows 141 166, 4.5 159 169, 6 174 171
+MOE_ROWS, MOE_ROWS_64, MOE_ROWS_128 = 5, 52, 112
 
 
 def _moe_tile(T: int, K: int, E: int, least: int) -> int:
@@ -500,12 +501,17 @@ def _moe_tile(T: int, K: int, E: int, least: int) -> int:
     return 64 if mean <= MOE_ROWS_64 else 128 if mean <= MOE_ROWS_128 else 256
 
 
-def _moe_sort(ids: torch.Tensor, E: int, H: int, I: int, bm: int):
-    """(order, expert, place) of the choices `ids` [T, K], sorted in tiles of
-    bm rows; refuses what the tiles cannot take."""
+def _moe_sizes(E: int, H: int, I: int) -> None:
+    """Refuses what the experts' kernels cannot take."""
     if E > 64 or H % 128 or I % 128:
         raise RuntimeError(f"moe: {E} experts of {I} x {H}: at most 64, and "
                            "sizes that are multiples of 128")
+
+
+def _moe_sort(ids: torch.Tensor, E: int, H: int, I: int, bm: int):
+    """(order, expert, place) of the choices `ids` [T, K], sorted in tiles of
+    bm rows."""
+    _moe_sizes(E, H, I)
     pairs = ids.numel()
     tiles = min(pairs, (pairs + E * (bm - 1)) // bm)
     i32 = lambda *s: torch.empty(*s, dtype=torch.int32, device=ids.device)
@@ -545,17 +551,22 @@ def moe_choices(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor,
     n = _native()
     (T, H), K, (E, _, I) = x.shape, ids.shape[1], w2.shape
     bm = _moe_tile(T, K, E, 16)
+    if bm == 16:
+        _moe_sizes(E, H, I)
+        ids = ids.to(torch.int32).contiguous()
+        place = torch.empty_like(ids)
+        h = torch.empty(T * K, I, dtype=torch.bfloat16, device=x.device)
+        y = torch.empty(T * K, H, dtype=torch.bfloat16, device=x.device)
+        n.experts_few(True, h, place, x, w13, ids, K)
+        n.experts_few(False, y, None, h, w2, ids, 1)
+        return Choices(y, place, weights.float().contiguous())
     order, expert, place = _moe_sort(ids, E, H, I, bm)
     P = order.shape[0]
     h = torch.empty(P, I, dtype=torch.bfloat16, device=x.device)
     y = torch.empty(P, H, dtype=torch.bfloat16, device=x.device)
-    if bm == 16:
-        n.experts_up(h, x, w13, None, order, expert, K, None, bm)
-        n.experts_down(y, h, w2, None, order, expert, bm)
-    else:
-        n.experts_tiles(h, x, w13, None, None, order, expert, True, K, bm)
-        n.experts_tiles(y, h, w2, None, None, order, expert, False, 0, bm)
-    return Choices(y, place, weights.float().contiguous(), False)
+    n.experts_tiles(h, x, w13, None, None, order, expert, True, K, bm)
+    n.experts_tiles(y, h, w2, None, None, order, expert, False, 0, bm)
+    return Choices(y, place, weights.float().contiguous())
 
 
 def moe_ffn_fp8(xq: "QTensor", w13q: torch.Tensor, w13s: torch.Tensor,
@@ -579,7 +590,7 @@ def moe_ffn_fp8(xq: "QTensor", w13q: torch.Tensor, w13s: torch.Tensor,
                     bm)
     a = silu_mul_q(h)
     n.experts_tiles(y, a.data, w2q, a.scale, w2s, order, expert, False, 0, bm)
-    return _moe_sum(Choices(y, place, weights.float().contiguous(), False))
+    return _moe_sum(Choices(y, place, weights.float().contiguous()))
 
 
 def decode_inputs(stage: torch.Tensor, rows: int, cap: int, pages: int,

@@ -64,6 +64,36 @@ def test_experts_around_the_rule(tokens, experts, top, width, inner):
     assert (out - ref).abs().max() <= 2.0 ** -5 * ref.abs().max()
 
 
+@pytest.mark.parametrize("tokens,experts,top,width,inner", [
+    (1, 4, 2, 128, 128), (5, 1, 1, 128, 256), (17, 4, 1, 256, 128),
+    (33, 7, 1, 384, 640), (64, 64, 5, 128, 128), (65, 13, 1, 128, 384)])
+@pytest.mark.parametrize("kind", ["spread", "one", "gaps"])
+def test_few_choices(tokens, experts, top, width, inner, kind):
+    """Choices that are named where they are, more than 16 or 64 of one expert,
+    and places without a choice."""
+    assert ops._moe_tile(tokens, top, experts, 16) == 16
+    g = torch.Generator().manual_seed(tokens)
+    rand = lambda *s: torch.randn(*s, generator=g)
+    x = rand(tokens, width).bfloat16().to(DEV)
+    w13 = (rand(experts, 2 * inner, width) * width ** -0.5).bfloat16().to(DEV)
+    w2 = (rand(experts, width, inner) * inner ** -0.5).bfloat16().to(DEV)
+    ids = rand(tokens, experts).topk(top, -1).indices.int()
+    if kind == "one":
+        ids[:, 0] = experts - 1
+    elif kind == "gaps":
+        ids[::3] = -1
+    ids = ids.to(DEV)
+    weight = rand(tokens, top).abs().to(DEV)
+    out = ops.moe_ffn(x, w13, w2, weight, ids).double()
+    ref = torch.zeros_like(out)
+    for e in range(experts):
+        gate, up = (x.double() @ w13[e].double().t()).chunk(2, -1)
+        y = torch.nn.functional.silu(gate) * up @ w2[e].double().t()
+        ref += y * (weight * (ids == e)).sum(-1)[:, None].double()
+    assert (out - ref).norm() <= 2.0 ** -7 * ref.norm()
+    assert (out - ref).abs().max() <= 2.0 ** -5 * ref.abs().max()
+
+
 @pytest.mark.parametrize("tokens", [1, 26, 27, 56, 57, 300])
 @pytest.mark.parametrize("experts,top,width,inner", [
     (4, 2, 256, 384), (3, 1, 1024, 256)])
