@@ -26,10 +26,17 @@
 // workgroups: with 8 kv heads a die has one of them, and its keys and values
 // stay in the die's L2.  Later rows see more and start first.
 //
-// 32 heads, 8 kv heads: a prompt of 8192 tokens 732 us (751 TFLOP/s) where
+// Within a tile the operands of 8 products are loaded ahead of them, and the next
+// 16 tokens' weights are formed between the products of the last 16, not before
+// them.  Long prompts are bound by power: with zeros as data 8192 cached tokens
+// and 7808 rows take 1.94 ms, with normal values 2.57.
+//
+// 32 heads, 8 kv heads: a prompt of 8192 tokens 734 us (749 TFLOP/s) where
 // weights that went through LDS and tiles of 256 rows of one head took 2628
-// (209); 8 prompts of 1000, 130 us; 7808 tokens after 8192 cached ones 2.58 ms
-// (600 TFLOP/s; e4m3 pages 2.62) where one workgroup a row took 37.6.
+// (209); of 512 17.9, and 18.9 with weights and products in turn; 8 prompts of
+// 1000, 133 us; 7808 tokens after 8192 cached ones 2.60 ms (2.65 in turn; e4m3
+// pages 2.69, 2.72), 500 after 500 36 us (41), where one workgroup a row took
+// 37.6 ms.
 //
 // ROWS: weights are rounded to bf16, relative to the maximum after each tile of
 // 64 tokens, and summed in a fixed order.  Both are a part of the result: a
@@ -50,6 +57,7 @@ constexpr int PAGE = 16;
 constexpr float LOG2E = 1.4426950408889634f;
 constexpr float GROW = 8.f;
 enum Source { ROWS, PAGES, PAGES8 };
+enum { VALU = 0x002, PRODUCT = 0x008, DS_READ = 0x100 };  // for the scheduler
 
 typedef __attribute__((ext_vector_type(4))) short short4_t;
 typedef __attribute__((ext_vector_type(2))) float float2_t;
@@ -248,17 +256,29 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(Prefill a) {
     const char* kl = reinterpret_cast<const char*>(lds[buf][0]);
     const char* vl = reinterpret_cast<const char*>(lds[buf][1]);
     f32x16_t sc[2];
+    short8_t kf[8];
+    auto key = [&](int b, int c) {
+      return *reinterpret_cast<const short8_t*>(kl + (k_at ^ c << 5) +
+                                                b * 32 * HD * 2);
+    };
     #pragma unroll
-    for (int b = 0; b < 2; ++b) {
-      sc[b] = f32x16_t(0.f);
-      #pragma unroll
-      for (int c = 0; c < 8; ++c)
-        sc[b] = mfma32(*reinterpret_cast<const short8_t*>(
-                           kl + (k_at ^ c << 5) + b * 32 * HD * 2),
-                       qf[c], sc[b]);
-      // the operands of all parts are not to be in registers together
-      __builtin_amdgcn_sched_barrier(0);
+    for (int c = 0; c < 8; ++c) kf[c] = key(0, c);
+    sc[0] = sc[1] = f32x16_t(0.f);
+    #pragma unroll
+    for (int c = 0; c < 8; ++c) {
+      sc[0] = mfma32(kf[c], qf[c], sc[0]);
+      kf[c] = key(1, c);
     }
+    #pragma unroll
+    for (int c = 0; c < 8; ++c) sc[1] = mfma32(kf[c], qf[c], sc[1]);
+    __builtin_amdgcn_sched_group_barrier(DS_READ, 8, 0);
+    #pragma unroll
+    for (int c = 0; c < 8; ++c) {
+      __builtin_amdgcn_sched_group_barrier(PRODUCT, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(DS_READ, 1, 0);
+    }
+    __builtin_amdgcn_sched_group_barrier(PRODUCT, 8, 0);
+    __builtin_amdgcn_sched_barrier(0);
     if (kv0 + KV - 1 > before + rw) {
       #pragma unroll
       for (int b = 0; b < 2; ++b)
@@ -286,40 +306,62 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(Prefill a) {
     }
     const float base = m == -FLT_MAX ? 0.f : m;
     float sum = 0.f;
+    union Values { short4_t h[2]; short8_t v; };
+    Values vf[2][4];
+    auto value = [&](int i, int e) {             // of tokens 16 i ..
+      Values r;
+      #pragma unroll
+      for (int h = 0; h < 2; ++h)
+        r.h[h] = lds_read_tr(reinterpret_cast<const short*>(
+            vl + (v_at ^ e << 6) + (i * 16 + h * 4) * HD * 2));
+      return r;
+    };
     __builtin_amdgcn_sched_barrier(0);
     #pragma unroll
-    for (int b = 0; b < 2; ++b)
+    for (int e = 0; e < 4; ++e) vf[0][e] = value(0, e);
+    short8_t part[2][PARTS];
+    auto weigh = [&](int i, short8_t* to) {
+      const int b = i >> 1, c = i & 1;
+      float p[8];
       #pragma unroll
-      for (int c = 0; c < 2; ++c) {
-        float p[8];
-        #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          p[j] = EACH ? __expf(product(sc[b][c * 8 + j], a.scale) - base)
-                      : exp2_fast(fmaf(sc[b][c * 8 + j], a.scale, -base));
-          if constexpr (!EACH) sum += p[j];
-        }
-        short8_t part[PARTS];
-        split_bf16x8<PARTS>(p, part);
-        if constexpr (EACH) {
-          // a lane sums 4 of every 8 tokens: t .. t + 3, t + 8 .. t + 11
-          #pragma unroll
-          for (int j = 0; j < 4; ++j) swap_halves(p[j], p[4 + j]);
-          #pragma unroll
-          for (int j = 0; j < 8; ++j) sum += p[j];
-        }
-        #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          union { short4_t h[2]; short8_t v; } vf;
-          #pragma unroll
-          for (int i = 0; i < 2; ++i)
-            vf.h[i] = lds_read_tr(reinterpret_cast<const short*>(
-                vl + (v_at ^ e << 6) + (b * 32 + c * 16 + i * 4) * HD * 2));
-          #pragma unroll
-          for (int n = 0; n < PARTS; ++n)
-            acc[e] = mfma32(vf.v, part[n], acc[e]);
-        }
-        if (c) __builtin_amdgcn_sched_barrier(0);
+      for (int j = 0; j < 8; ++j) {
+        p[j] = EACH ? __expf(product(sc[b][c * 8 + j], a.scale) - base)
+                    : exp2_fast(fmaf(sc[b][c * 8 + j], a.scale, -base));
+        if constexpr (!EACH) sum += p[j];
       }
+      split_bf16x8<PARTS>(p, to);
+      if constexpr (EACH) {
+        // a lane sums 4 of every 8 tokens: t .. t + 3, t + 8 .. t + 11
+        #pragma unroll
+        for (int j = 0; j < 4; ++j) swap_halves(p[j], p[4 + j]);
+        #pragma unroll
+        for (int j = 0; j < 8; ++j) sum += p[j];
+      }
+    };
+    weigh(0, part[0]);
+    #pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      __builtin_amdgcn_sched_barrier(0);
+      if (i < 3) {
+        #pragma unroll
+        for (int e = 0; e < 4; ++e) vf[(i + 1) & 1][e] = value(i + 1, e);
+        weigh(i + 1, part[(i + 1) & 1]);
+      }
+      #pragma unroll
+      for (int e = 0; e < 4; ++e)
+        #pragma unroll
+        for (int n = 0; n < PARTS; ++n)
+          acc[e] = mfma32(vf[i & 1][e].v, part[i & 1][n], acc[e]);
+      // between the products the next values' loads and the next weights
+      if (i < 3) {
+        #pragma unroll
+        for (int n = 0; n < 4 * PARTS; ++n) {
+          __builtin_amdgcn_sched_group_barrier(PRODUCT, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(DS_READ, PARTS == 1 ? 2 : 1, 0);
+          __builtin_amdgcn_sched_group_barrier(VALU, PARTS == 1 ? 12 : 6, 0);
+        }
+      }
+    }
     if constexpr (EACH) {            // both halves, as the maximum
       float other = sum;
       swap_halves(sum, other);
