@@ -491,7 +491,8 @@ void gemm_split(c10::optional<torch::Tensor> out, torch::Tensor x,
            t.stride(0) % 8 == 0;
   };
   TORCH_CHECK(N % 4 == 0 && K % 128 == 0 && M < (1l << 20) && K < (1l << 24) &&
-                  N < (1l << 24) && aligned(x) && aligned(w),
+                  N < (1l << 24) && aligned(x) && aligned(w) &&
+                  x.stride(0) < (1l << 22) && w.stride(0) < (1l << 22),
               "gemm_split: sizes");
   TORCH_CHECK((bm == 128 && (bn == 64 || bn == 128)) ||
                   (bm == 256 && bn == 128), "gemm_split: tile");

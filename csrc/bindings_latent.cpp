@@ -54,8 +54,8 @@ void launch_experts_route(float*, int*, const float*, int, int, int, bool,
 void launch_experts_router(float*, int*, const void*, const float*,
                            const bf16*, long, int, int, int, hipStream_t);
 void launch_experts_tiles(bool, bf16*, const void*, const void*, const float*,
-                          const float*, const int*, const int*, int, int, int,
-                          int, int, hipStream_t);
+                          const float*, const int*, const int*, long, int, int,
+                          int, int, int, hipStream_t);
 void launch_experts_sort(int*, int*, int*, const int*, int, int, int, int,
                          hipStream_t);
 void launch_experts_route_sort(float*, int*, int*, int*, int*, const float*,
@@ -519,8 +519,8 @@ void experts_tiles(Tensor out, Tensor x, Tensor w, Maybe x_scale,
   }
   launch_experts_tiles(gated, ptr<bf16>(out), x.data_ptr(), w.data_ptr(),
                        opt(x_scale), opt(w_scale), order.data_ptr<int>(),
-                       expert.data_ptr<int>(), (int)tiles, (int)N, (int)K,
-                       (int)div, (int)bm, stream());
+                       expert.data_ptr<int>(), x.size(0), (int)tiles, (int)N,
+                       (int)K, (int)div, (int)bm, stream());
 }
 
 // choices and weights of the rows of x [T, W], bf16 or e4m3 with x_scale [T]

@@ -18,12 +18,9 @@
 // layer (8 experts, 14336 x 4096, 2.8 GB), us with 256-row tiles, row tiles
 // and here: 16 choices an expert 821 617 532, 48 831 792 543, 128 943 869 730,
 // 500 2355 2100 1740.  32 experts of 1024 x 2048, 64 choices 277 172 119.
-#include "common.h"
+#include "tile_loop.h"
 
 namespace {
-
-typedef __attribute__((address_space(1))) const unsigned glob;
-typedef __attribute__((address_space(3))) unsigned shar;
 
 struct Tiles {
   bf16* out;
@@ -36,26 +33,17 @@ struct Tiles {
   int N, K, div, nx;           // N outputs a choice, nx blocks of them
 };
 
-// 16-byte unit c of row r of a chunk in LDS.  16 lanes read at a time, 16 rows
-// of one unit, and two rows fill the 64 banks: so the unit turns with every
-// second row (with every row rows r and r + 8 met in a bank, and such reads ran
-// at 303 GB/s a compute unit, not 577; four prompts of 500 tokens through 4
-// layers of 8 experts of 14336 x 4096 5836 -> 5665 us).
-DEV int unit(int r, int c) { return r * 128 + ((c ^ (r >> 1 & 7)) << 4); }
-
 // BM choices, BN rows of weights; WM * WN waves have BM / WM by BN / WN
-template <int BM, int BN, int WM, int WN, int STAGES, bool GATED, bool FP8>
+template <int BM, int BN, int WM, int WN, int STAGES, bool GATED, bool FP8,
+          bool FAR>
 __global__ __launch_bounds__(WM * WN * 64,
                              WM * WN == 4 ? 2 : WM * WN / 4)
 void experts_tiles_kernel(Tiles a) {
-  constexpr int WAVES = WM * WN;
-  constexpr int NI = BN / WN / 32, MI = BM / WM / 32;
-  constexpr int LX = BM / 8 / WAVES, LW = BN / 8 / WAVES;  // loads a chunk
-  constexpr int STAGE = (BM + BN) * 128;
+  using Loop = TileLoop<BM, BN, WM, WN, STAGES, 1, FP8>;
+  constexpr int LX = Loop::LX, LW = Loop::LW, NI = Loop::NI, MI = Loop::MI;
   constexpr int OUT = GATED ? BN / 2 : BN;                 // outputs
   constexpr int ELEM = FP8 ? 1 : 2;
   static_assert(!(GATED && FP8), "the activation's scale needs whole rows");
-  static_assert(LX * WAVES * 8 == BM && LW * WAVES * 8 == BN, "loads");
   extern __shared__ __attribute__((aligned(16))) char lds[];
   const int tile = blockIdx.x / a.nx, e = a.expert[tile];
   if (e < 0) return;
@@ -75,110 +63,46 @@ void experts_tiles_kernel(Tiles a) {
     const int choice = a.order[p];
     return a.div ? (choice >= 0 ? choice / a.div : 0) : p;
   };
-  const char* xp[LX];
+  auto w_row = [&](int r) {    // gated: 8 gate rows, then their 8 up rows
+    return GATED ? (r >> 4) * 8 + (r & 7) + (r & 8 ? a.N : 0) : r;
+  };
+  const char* w0 = static_cast<const char*>(a.w) +
+                   ((long)e * (GATED ? 2 * a.N : a.N) + n0) * row_bytes;
+  const char* x0 = static_cast<const char*>(a.x) + (a.div ? 0 : p0 * row_bytes);
+  const RowLoads x_rows(x0), w_rows(w0);
+  long x_off[LX], w_off[LW];   // below 4 GB but for FAR
   #pragma unroll
   for (int j = 0; j < LX; ++j) {
     const int r = (wid * LX + j) * 8 + lr;
-    xp[j] = static_cast<const char*>(a.x) + row_of(p0 + r) * row_bytes +
-            column(r);
+    x_off[j] = (row_of(p0 + r) - (a.div ? 0 : p0)) * row_bytes + column(r);
   }
-  const char* wp[LW];
   #pragma unroll
   for (int j = 0; j < LW; ++j) {
     const int r = (wid * LW + j) * 8 + lr;
-    int n = r;
-    if constexpr (GATED)       // 8 gate rows, then their 8 up rows
-      n = n0 + (n >> 4) * 8 + (n & 7) + (n & 8 ? a.N : 0);
-    else
-      n += n0;
-    wp[j] = static_cast<const char*>(a.w) +
-            ((long)e * (GATED ? 2 * a.N : a.N) + n) * row_bytes + column(r);
+    w_off[j] = w_row(r) * row_bytes + column(r);
   }
-  auto stage = [&](int slot, int chunk) {
-    char* base = lds + slot * STAGE;
+  auto load = [&](char* l, const RowLoads& rows, const char* base, long off,
+                  int d) {
+    if constexpr (FAR)
+      __builtin_amdgcn_global_load_lds(
+          (__attribute__((address_space(1))) const unsigned*)(base + off +
+                                                              d * 128),
+          (__attribute__((address_space(3))) unsigned*)l, 16, 0, 0);
+    else
+      rows.to_lds(l, (unsigned)off, d * 128);
+  };
+  auto stage = [&](int slot, int d) {
+    char* l = lds + slot * Loop::STAGE;
     #pragma unroll
     for (int j = 0; j < LX; ++j)
-      __builtin_amdgcn_global_load_lds(
-          (glob*)(xp[j] + chunk * 128),
-          (shar*)(base + (wid * LX + j) * 1024), 16, 0, 0);
+      load(l + (wid * LX + j) * 1024, x_rows, x0, x_off[j], d);
     #pragma unroll
     for (int j = 0; j < LW; ++j)
-      __builtin_amdgcn_global_load_lds(
-          (glob*)(wp[j] + chunk * 128),
-          (shar*)(base + BM * 128 + (wid * LW + j) * 1024), 16, 0, 0);
+      load(l + BM * 128 + (wid * LW + j) * 1024, w_rows, w0, w_off[j], d);
   };
-
-  f32x16_t acc[NI][MI];
-  #pragma unroll
-  for (int n = 0; n < NI; ++n)
-    #pragma unroll
-    for (int m = 0; m < MI; ++m) acc[n][m] = f32x16_t(0.f);
-  const int x_at = unit(wm * MI * 32 + col, hf);
-  const int w_at = BM * 128 + unit(wn * NI * 32 + col, hf);
-  auto compute = [&](int slot) {
-    if (!live) return;
-    const char* base = lds + slot * STAGE;
-    #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      short8_t xf[MI], wf[NI];
-      #pragma unroll
-      for (int m = 0; m < MI; ++m)
-        xf[m] = *reinterpret_cast<const short8_t*>(
-            base + (x_at ^ k << 5) + m * 32 * 128);
-      #pragma unroll
-      for (int n = 0; n < NI; ++n)
-        wf[n] = *reinterpret_cast<const short8_t*>(
-            base + (w_at ^ k << 5) + n * 32 * 128);
-      #pragma unroll
-      for (int n = 0; n < NI; ++n)
-        #pragma unroll
-        for (int m = 0; m < MI; ++m)
-          if constexpr (FP8) {     // 16 bytes a lane are two steps of 16
-            union { short8_t v; long l[2]; } u{wf[n]}, v{xf[m]};
-            acc[n][m] = __builtin_amdgcn_mfma_f32_32x32x16_fp8_fp8(
-                u.l[0], v.l[0], acc[n][m], 0, 0, 0);
-            acc[n][m] = __builtin_amdgcn_mfma_f32_32x32x16_fp8_fp8(
-                u.l[1], v.l[1], acc[n][m], 0, 0, 0);
-          } else {
-            acc[n][m] = mfma32(wf[n], xf[m], acc[n][m]);
-          }
-    }
-  };
-
-  const int chunks = (int)(row_bytes / 128);
-  if constexpr (STAGES == 2) {
-    // [chunk d landed, own reads of d - 1 done | barrier | issue d + 1 into the
-    // slot of d - 1 | compute d]
-    stage(0, 0);
-    for (int d = 0; d < chunks; ++d) {
-      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-      __builtin_amdgcn_s_barrier();
-      if (d + 1 < chunks) stage((d + 1) & 1, d + 1);
-      compute(d & 1);
-    }
-  } else {
-    // [compute d | issue d + 2 | d + 1 landed, own reads of d done | barrier]:
-    // d + 2 takes the slot of d - 1, with which every wave was done before the
-    // last barrier
-    static_assert(STAGES == 3, "stages");
-    constexpr int LOADS = LX + LW;
-    stage(0, 0);
-    stage(1, 1);
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LOADS) : "memory");
-    __builtin_amdgcn_s_barrier();
-    int slot = 0, d = 0;
-    for (; d + 2 < chunks; ++d) {
-      compute(slot);
-      stage(slot == 0 ? 2 : slot - 1, d + 2);
-      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(LOADS) : "memory");
-      __builtin_amdgcn_s_barrier();
-      slot = slot == 2 ? 0 : slot + 1;
-    }
-    compute(slot);                       // d == chunks - 2
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    compute(slot == 2 ? 0 : slot + 1);
-  }
+  Loop loop;
+  loop.run(lds, wm, wn, (int)(row_bytes / 128), live, stage);
+  auto& acc = loop.acc;
 
   // acc[n][m][r]: weight row (r >> 2) * 8 + hf * 4 + (r & 3) of block n,
   // choice col of block m
@@ -232,39 +156,51 @@ void experts_tiles_kernel(Tiles a) {
 // w are e4m3.
 void launch_experts_tiles(bool gated, bf16* out, const void* x, const void* w,
                           const float* x_scale, const float* w_scale,
-                          const int* order, const int* expert, int tiles,
-                          int N, int K, int div, int bm, hipStream_t stream) {
+                          const int* order, const int* expert, long x_rows,
+                          int tiles, int N, int K, int div, int bm,
+                          hipStream_t stream) {
   if (tiles == 0) return;
   Tiles a{out, x, w, x_scale, w_scale, order, expert, N, K, div, 0};
-  #define RUN(BM, BN, WM, WN, STAGES, GATED, FP8)                           \
+  #define RUN(BM, BN, WM, WN, STAGES, GATED, FP8, FAR)                      \
     {                                                                       \
       constexpr int BYTES = STAGES * (BM + BN) * 128;                       \
       static const hipError_t set = hipFuncSetAttribute(                    \
           reinterpret_cast<const void*>(                                    \
-              &experts_tiles_kernel<BM, BN, WM, WN, STAGES, GATED, FP8>),   \
+              &experts_tiles_kernel<BM, BN, WM, WN, STAGES, GATED, FP8,     \
+                                  FAR>),                                   \
           hipFuncAttributeMaxDynamicSharedMemorySize, BYTES);               \
       HIP_CHECK(set);                                                       \
       a.nx = N / (GATED ? BN / 2 : BN);                                     \
-      experts_tiles_kernel<BM, BN, WM, WN, STAGES, GATED, FP8>              \
+      experts_tiles_kernel<BM, BN, WM, WN, STAGES, GATED, FP8, FAR>         \
           <<<(unsigned)(tiles * a.nx), WM * WN * 64, BYTES, stream>>>(a);   \
     }
-  #define KINDS(BM, BN, WM, WN, STAGES)                                     \
-    if (x_scale) RUN(BM, BN, WM, WN, STAGES, false, true)                   \
-    else if (gated) RUN(BM, BN, WM, WN, STAGES, true, false)                \
-    else RUN(BM, BN, WM, WN, STAGES, false, false)
+  #define KINDS(BM, BN, WM, WN, STAGES, FAR)                                \
+    {                                                                       \
+      if (x_scale) RUN(BM, BN, WM, WN, STAGES, false, true, FAR)            \
+      else if (gated) RUN(BM, BN, WM, WN, STAGES, true, false, FAR)         \
+      else RUN(BM, BN, WM, WN, STAGES, false, false, FAR)                   \
+    }
   // 256 rows of weights need fewer loads of x and LDS reads, and leave units
   // idle where they make few workgroups: Mixtral 8x7B, 500 choices an expert,
   // up (2000 workgroups of 256) 1055 us against 1223, down (290) 753 against
   // 682; 32 experts of 1024 x 2048, 250 choices, 120 108 and 79 67
   const int wide = gated ? 128 : 256;
+  // what 32 bits of offset do not reach
+  const long row_bytes = (long)K * (x_scale ? 1 : 2);
+  const bool far = (div ? x_rows : bm) * row_bytes >= 1l << 32 ||
+                   (gated ? N + 256l : 256l) * row_bytes >= 1l << 32;
   if (bm == 64) {
-    KINDS(64, 128, 2, 2, 3)
+    if (far) KINDS(64, 128, 2, 2, 3, true)
+    else KINDS(64, 128, 2, 2, 3, false)
   } else if (bm == 128) {
-    KINDS(128, 128, 2, 4, 3)
+    if (far) KINDS(128, 128, 2, 4, 3, true)
+    else KINDS(128, 128, 2, 4, 3, false)
+  } else if (far) {
+    KINDS(256, 128, 4, 2, 3, true)
   } else if (N % wide == 0 && (long)tiles * (N / wide) >= 1024) {
-    KINDS(256, 256, 4, 2, 2)
+    KINDS(256, 256, 4, 2, 2, false)
   } else {
-    KINDS(256, 128, 4, 2, 3)
+    KINDS(256, 128, 4, 2, 3, false)
   }
   #undef KINDS
   #undef RUN

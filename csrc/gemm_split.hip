@@ -18,12 +18,9 @@
 //   4096 x 4096   32 rows 13 12, 96 22 14, 192 33 22, 256 23 23
 //   2048 x 7168   32 rows 19 11, 96 19 14, 192 25 19, 256 25 20, 512 32 29
 //   5120 x 8192   32 rows 25 23, 96 37 26, 192 61 36, 256 72 39
-#include "common.h"
+#include "tile_loop.h"
 
 namespace {
-
-typedef __attribute__((address_space(1))) const unsigned glob;
-typedef __attribute__((address_space(3))) unsigned shar;
 
 struct Split {
   bf16* out;
@@ -35,20 +32,13 @@ struct Split {
   int mt, nt, splits;          // tiles of rows, of outputs, parts of K
 };
 
-// 16-byte unit c of row r of a chunk in LDS: reads of 8 rows of one unit
-// spread over the banks
-DEV int unit(int r, int c) { return r * 128 + ((c ^ (r & 7)) << 4); }
-
 // BM rows of x, BN of w; WM * WN waves have BM / WM by BN / WN.  A stage has
 // KC chunks of 64 columns.
 template <int BM, int BN, int WM, int WN, int STAGES, int KC>
 __global__ __launch_bounds__(WM * WN * 64, WM * WN / 4)
 void gemm_split_kernel(Split a) {
-  constexpr int WAVES = WM * WN;
-  constexpr int NI = BN / WN / 32, MI = BM / WM / 32;
-  constexpr int LX = BM / 8 / WAVES, LW = BN / 8 / WAVES;  // loads a chunk
-  constexpr int SUB = (BM + BN) * 128, STAGE = SUB * KC;
-  static_assert(LX * WAVES * 8 == BM && LW * WAVES * 8 == BN, "loads");
+  using Loop = TileLoop<BM, BN, WM, WN, STAGES, KC, false>;
+  constexpr int LX = Loop::LX, LW = Loop::LW, NI = Loop::NI, MI = Loop::MI;
   extern __shared__ __attribute__((aligned(16))) char lds[];
   // workgroups go to the 8 XCDs in turn: those of one tile of w, which differ
   // in the rows of x, to the same, whose L2 then has it
@@ -67,86 +57,39 @@ void gemm_split_kernel(Split a) {
 
   // this lane's 16 bytes of row lane / 8 of each 1-KB load; rows past the end
   // are the last one
-  const int lr = lane >> 3, lc = ((lane & 7) ^ lr) * 8;
-  const bf16* xp[LX];
+  const RowLoads x_rows(a.x + m0 * a.xs + first * (64 * KC));
+  const RowLoads w_rows(a.w + n0 * a.ws + first * (64 * KC));
+  unsigned x_off[LX], w_off[LW];
   #pragma unroll
-  for (int j = 0; j < LX; ++j)
-    xp[j] = a.x + min(m0 + (wid * LX + j) * 8 + lr, a.M - 1) * a.xs + lc +
-            first * (64 * KC);
-  const bf16* wp[LW];
+  for (int j = 0; j < LX; ++j) {
+    const int r = (wid * LX + j) * 8 + (lane >> 3);
+    x_off[j] = (unsigned)(min(r, a.M - 1 - m0) * a.xs * 2) +
+               ((lane & 7) ^ (r >> 1 & 7)) * 16;
+  }
   #pragma unroll
-  for (int j = 0; j < LW; ++j)
-    wp[j] = a.w + min(n0 + (wid * LW + j) * 8 + lr, a.N - 1) * a.ws + lc +
-            first * (64 * KC);
-  auto stage = [&](int slot, int chunk) {
-    char* base = lds + slot * STAGE;
+  for (int j = 0; j < LW; ++j) {
+    const int r = (wid * LW + j) * 8 + (lane >> 3);
+    w_off[j] = (unsigned)(min(r, a.N - 1 - n0) * a.ws * 2) +
+               ((lane & 7) ^ (r >> 1 & 7)) * 16;
+  }
+  auto stage = [&](int slot, int d) {
+    char* base = lds + slot * Loop::STAGE;
     #pragma unroll
     for (int j = 0; j < LX; ++j)
       #pragma unroll
       for (int s = 0; s < KC; ++s)
-        __builtin_amdgcn_global_load_lds(
-            (glob*)(xp[j] + (chunk * KC + s) * 64),
-            (shar*)(base + s * SUB + (wid * LX + j) * 1024), 16, 0, 0);
+        x_rows.to_lds(base + s * Loop::SUB + (wid * LX + j) * 1024, x_off[j],
+                      (d * KC + s) * 128);
     #pragma unroll
     for (int j = 0; j < LW; ++j)
       #pragma unroll
       for (int s = 0; s < KC; ++s)
-        __builtin_amdgcn_global_load_lds(
-            (glob*)(wp[j] + (chunk * KC + s) * 64),
-            (shar*)(base + s * SUB + BM * 128 + (wid * LW + j) * 1024), 16, 0,
-            0);
+        w_rows.to_lds(base + s * Loop::SUB + BM * 128 + (wid * LW + j) * 1024,
+                      w_off[j], (d * KC + s) * 128);
   };
-
-  f32x16_t acc[NI][MI];
-  #pragma unroll
-  for (int n = 0; n < NI; ++n)
-    #pragma unroll
-    for (int m = 0; m < MI; ++m) acc[n][m] = f32x16_t(0.f);
-  const int x_at = unit(wm * MI * 32 + col, hf);
-  const int w_at = BM * 128 + unit(wn * NI * 32 + col, hf);
-  auto compute = [&](int slot) {
-    if (!live) return;
-    #pragma unroll
-    for (int k4 = 0; k4 < 4 * KC; ++k4) {
-      const int k = k4 & 3;
-      const char* base = lds + slot * STAGE + (k4 >> 2) * SUB;
-      short8_t xf[MI], wf[NI];
-      #pragma unroll
-      for (int m = 0; m < MI; ++m)
-        xf[m] = *reinterpret_cast<const short8_t*>(
-            base + (x_at ^ k << 5) + m * 32 * 128);
-      #pragma unroll
-      for (int n = 0; n < NI; ++n)
-        wf[n] = *reinterpret_cast<const short8_t*>(
-            base + (w_at ^ k << 5) + n * 32 * 128);
-      #pragma unroll
-      for (int n = 0; n < NI; ++n)
-        #pragma unroll
-        for (int m = 0; m < MI; ++m)
-          acc[n][m] = mfma32(wf[n], xf[m], acc[n][m]);
-    }
-  };
-
-  // [chunk d landed, own reads of d - 1 done | barrier | issue d + STAGES - 1
-  // into the slot of d - 1 | compute d]
-  constexpr int LOADS = (LX + LW) * KC, AHEAD = STAGES - 1;
-  static_assert((AHEAD - 1) * LOADS < 64, "the counter of loads");
-  #pragma unroll
-  for (int d = 0; d < AHEAD; ++d)
-    if (d < chunks) stage(d, d);
-  int slot = 0;
-  for (int d = 0; d < chunks; ++d) {
-    if (d + AHEAD <= chunks)
-      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((AHEAD - 1) * LOADS)
-                   : "memory");
-    else
-      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    if (d + AHEAD < chunks)
-      stage(slot == 0 ? STAGES - 1 : slot - 1, d + AHEAD);
-    compute(slot);
-    slot = slot == STAGES - 1 ? 0 : slot + 1;
-  }
+  Loop loop;
+  loop.run(lds, wm, wn, chunks, live, stage);
+  auto& acc = loop.acc;
 
   // acc[n][m][r]: row (r >> 2) * 8 + hf * 4 + (r & 3) of w of block n, row col
   // of x of block m

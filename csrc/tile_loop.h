@@ -1,0 +1,139 @@
+// The inner loop of products in LDS tiles (gfx950), bf16 or e4m3: x and w come
+// in chunks of 128 bytes of a row, from memory to LDS directly, into a ring.
+//
+// The operands of a step are read from LDS before the products of the step
+// before, and the first ones of a stage before the last products of the stage
+// before it, so that no product waits for a read.  What bounds it then: 256 x
+// 256 tiles the power that products may take (a product of 8192 x 28672 x 4096
+// without its loads 1325 us with random numbers, 1060 with zeros), smaller ones
+// the bytes in flight.  Four prompts of 500 tokens through 4 layers of 8 experts
+// of 14336 x 4096 5645 -> 5435 us, a prompt of 512 through 8 dense layers 2265 ->
+// 2240, where every step waited for its own reads.
+#pragma once
+
+#include "common.h"
+
+// Rows in memory from `base` on: 16 bytes a lane, of byte offset `at` (below
+// 4 GB) + `from`, which is uniform, to LDS address l + lane * 16.  Loads by a
+// buffer's address, for the compiler takes those by a global one for flat ones,
+// and then waits for all LDS reads where it needs the oldest.
+struct RowLoads {
+  __amdgpu_buffer_rsrc_t rows;
+  DEV explicit RowLoads(const void* base)
+      : rows(__builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0,
+                                               0xffffffff, 0x00020000)) {}
+  DEV void to_lds(char* l, unsigned at, unsigned from) const {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(
+        rows, (__attribute__((address_space(3))) unsigned*)l, 16, at, from, 0,
+        0);
+  }
+};
+
+// 16-byte unit c of row r of a chunk in LDS.  16 lanes read at a time, 16 rows
+// of one unit, and two rows fill the 64 banks: so the unit turns with every
+// second row.
+DEV int chunk_unit(int r, int c) { return r * 128 + ((c ^ (r >> 1 & 7)) << 4); }
+
+// BM rows of x, BN of w; WM * WN waves have BM / WM by BN / WN.  A stage has KC
+// chunks: BM rows of x, then BN of w, of each.
+template <int BM, int BN, int WM, int WN, int STAGES, int KC, bool FP8>
+struct TileLoop {
+  static constexpr int WAVES = WM * WN;
+  static constexpr int NI = BN / WN / 32, MI = BM / WM / 32;
+  static constexpr int LX = BM / 8 / WAVES, LW = BN / 8 / WAVES;  // a chunk
+  static constexpr int SUB = (BM + BN) * 128, STAGE = SUB * KC;
+  static constexpr int BYTES = STAGES * STAGE;
+  static constexpr int LOADS = (LX + LW) * KC, STEPS = 4 * KC;
+  static_assert(LX * WAVES * 8 == BM && LW * WAVES * 8 == BN, "loads");
+  static_assert((STAGES - 1) * LOADS < 64, "the counter of loads");
+
+  struct Frag {
+    short8_t x[MI], w[NI];
+  };
+  f32x16_t acc[NI][MI];
+
+  DEV void read(Frag& f, const char* base, int x_at, int w_at, int step) {
+    const char* p = base + (step >> 2) * SUB;
+    const int k = step & 3;
+    #pragma unroll
+    for (int n = 0; n < NI; ++n)
+      f.w[n] = *reinterpret_cast<const short8_t*>(
+          p + (w_at ^ k << 5) + n * 32 * 128);
+    #pragma unroll
+    for (int m = 0; m < MI; ++m)
+      f.x[m] = *reinterpret_cast<const short8_t*>(
+          p + (x_at ^ k << 5) + m * 32 * 128);
+  }
+  DEV void products(const Frag& f) {
+    #pragma unroll
+    for (int n = 0; n < NI; ++n)
+      #pragma unroll
+      for (int m = 0; m < MI; ++m)
+        if constexpr (FP8) {       // 16 bytes a lane are two steps of 16
+          union { short8_t v; long l[2]; } u{f.w[n]}, v{f.x[m]};
+          acc[n][m] = __builtin_amdgcn_mfma_f32_32x32x16_fp8_fp8(
+              u.l[0], v.l[0], acc[n][m], 0, 0, 0);
+          acc[n][m] = __builtin_amdgcn_mfma_f32_32x32x16_fp8_fp8(
+              u.l[1], v.l[1], acc[n][m], 0, 0, 0);
+        } else {
+          acc[n][m] = mfma32(f.w[n], f.x[m], acc[n][m]);
+        }
+  }
+
+  // stage(slot, d) issues this wave's LOADS loads of stage d of the ring.
+  // Every wave has to call this; those that are not live only load.
+  template <class Stage>
+  DEV void run(char* lds, int wm, int wn, int stages, bool live,
+               Stage stage) {
+    const int lane = threadIdx.x & 63, col = lane & 31, hf = lane >> 5;
+    const int x_at = chunk_unit(wm * MI * 32 + col, hf);
+    const int w_at = BM * 128 + chunk_unit(wn * NI * 32 + col, hf);
+    #pragma unroll
+    for (int n = 0; n < NI; ++n)
+      #pragma unroll
+      for (int m = 0; m < MI; ++m) acc[n][m] = f32x16_t(0.f);
+    #pragma unroll
+    for (int d = 0; d < STAGES; ++d)
+      if (d < stages) stage(d, d);
+    if (stages >= STAGES)
+      asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier"
+                   ::"n"((STAGES - 1) * LOADS) : "memory");
+    else
+      asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+    Frag f[2];
+    if (live) read(f[0], lds, x_at, w_at, 0);
+    int slot = 0;
+    for (int d = 0; d < stages; ++d) {
+      const char* base = lds + slot * STAGE;
+      if (live) {
+        #pragma unroll
+        for (int k = 0; k < STEPS - 1; ++k) {
+          read(f[(k + 1) & 1], base, x_at, w_at, k + 1);
+          __builtin_amdgcn_sched_barrier(0);
+          products(f[k & 1]);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+      const int next = slot == STAGES - 1 ? 0 : slot + 1;
+      if (d + 1 < stages) {
+        // stage d + 1 has landed and all of d has been read, by every wave:
+        // its slot is free
+        if (d + STAGES <= stages)
+          asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier"
+                       ::"n"((STAGES - 2) * LOADS) : "memory");
+        else
+          asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier"
+                       ::: "memory");
+        if (live) read(f[0], lds + next * STAGE, x_at, w_at, 0);
+        if (d + STAGES < stages) stage(slot, d + STAGES);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if (live) products(f[1]);
+      slot = next;
+      // The last sums are there before they are read.  The compiler's own wait
+      // was found missing on the way out of this loop, where it copies them
+      // from accumulation registers, so this one is inside.
+      if (d + 1 == stages) asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+    }
+  }
+};

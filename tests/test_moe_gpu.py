@@ -162,3 +162,25 @@ def test_many_tokens_over_many_experts(tokens, fp8, monkeypatch):
     same = (out.float() - ref.float()).abs() <= 2.0 ** -7 * ref.float().abs() \
         .max()
     assert same.all(-1).float().mean() >= 0.99
+
+
+@pytest.mark.gpu
+def test_rows_beyond_32_bits():
+    """Tokens whose rows do not lie within 4 GB of the first one."""
+    tokens, width, inner = (1 << 19) + 300, 4096, 128
+    g = torch.Generator(device=DEV).manual_seed(3)
+    x = torch.empty(tokens, width, dtype=torch.bfloat16, device=DEV)
+    x.normal_(generator=g)
+    new = lambda *s: torch.randn(*s, generator=g, device=DEV).bfloat16() * 0.02
+    w13, w2 = new(2, 2 * inner, width), new(2, width, inner)
+    ids = torch.randint(0, 2, (tokens, 1), generator=g, device=DEV,
+                        dtype=torch.int32)
+    ones = torch.ones(tokens, 1, device=DEV)
+    out = ops.moe_choices(x, w13, w2, ones, ids)
+    rows = torch.tensor([0, 1, 255, 1 << 18, (1 << 19) - 1, 1 << 19,
+                         tokens - 1], device=DEV)
+    got = out.data[out.place[rows, 0].long()]
+    few = ops.moe_choices(x[rows], w13, w2, ones[rows], ids[rows])
+    want = few.data[few.place[:, 0].long()].float()
+    # both round the inner values and the results to bf16
+    assert (got.float() - want).norm() <= 2.0 ** -7 * want.norm()
