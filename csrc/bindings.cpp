@@ -105,14 +105,18 @@ void launch_recurrent_step(Kind, T*, float*, float*, float*, float*,
 void launch_decode_inputs(const long*, const int*, long*, long*, long*, int*,
                           int*, int*, int, int, int, int, int, hipStream_t);
 bool gemm_rows_fits(long, long);
-void launch_gemm_split(bf16*, float*, const bf16*, const bf16*, int, int, int,
-                       long, long, int, int, int, hipStream_t);
+void launch_gemm_split(bf16*, float*, const void*, const void*, const float*,
+                       const float*, int, int, int, long, long, int, int, int,
+                       bool, hipStream_t);
 void launch_gemm_rows(bf16*, const bf16*, const bf16*, int, int, int, long,
                       long, long, hipStream_t);
 void launch_silu_mul(bf16*, const bf16*, long, int, hipStream_t);
 void launch_quant_fp8(unsigned char*, float*, const bf16*, long, int, long,
                       hipStream_t);
 void launch_fused_add_rmsnorm_fp8(unsigned char*, float*, const bf16*,
+                                  bf16*, const bf16*, float, long, int,
+                                  hipStream_t);
+void launch_parts_add_rmsnorm_fp8(unsigned char*, float*, const float*, int,
                                   bf16*, const bf16*, float, long, int,
                                   hipStream_t);
 void launch_silu_mul_fp8(unsigned char*, float*, const bf16*, long, int,
@@ -471,32 +475,50 @@ void gemm_rows(torch::Tensor out, torch::Tensor x, torch::Tensor w) {
 }
 
 // out = x w^T, K in `splits` parts that a second kernel adds up; without out
-// the parts, [splits, M, N] floats, are the result
+// the parts, [splits, M, N] floats, are the result.  With scales of the rows x
+// and w are e4m3.  gated: out = silu(gate) * up of the halves of w.
 void gemm_split(c10::optional<torch::Tensor> out, torch::Tensor x,
                 torch::Tensor w, c10::optional<torch::Tensor> part, long bm,
-                long bn, long splits) {
-  for (const auto& t : {out.value_or(x), x, w})
-    TORCH_CHECK(t.is_cuda() && t.scalar_type() == torch::kBFloat16 &&
-                    t.dim() == 2 && t.stride(1) == 1, "gemm_split: matrices");
+                long bn, long splits, c10::optional<torch::Tensor> x_scale,
+                c10::optional<torch::Tensor> w_scale, bool gated) {
+  const bool fp8 = x_scale.has_value();
+  const auto kind = fp8 ? torch::kFloat8_e4m3fn : torch::kBFloat16;
+  for (const auto& t : {x, w})
+    TORCH_CHECK(t.is_cuda() && t.scalar_type() == kind && t.dim() == 2 &&
+                    t.stride(1) == 1, "gemm_split: matrices");
   const long M = x.size(0), K = x.size(1), N = w.size(0);
-  TORCH_CHECK(w.size(1) == K && (out.has_value() || splits > 1),
-              "gemm_split: shape");
+  TORCH_CHECK(w.size(1) == K && (out.has_value() || splits > 1) &&
+                  w_scale.has_value() == fp8, "gemm_split: shape");
+  if (fp8) {
+    check(*x_scale, torch::kFloat, "x_scale");
+    check(*w_scale, torch::kFloat, "w_scale");
+    TORCH_CHECK(x_scale->numel() == M && w_scale->numel() == N &&
+                    reinterpret_cast<uintptr_t>(w_scale->data_ptr()) % 16 == 0,
+                "gemm_split: scales");
+  }
   if (out.has_value())
-    TORCH_CHECK(out->size(0) == M && out->size(1) == N &&
+    TORCH_CHECK(out->is_cuda() && out->scalar_type() == torch::kBFloat16 &&
+                    out->dim() == 2 && out->size(0) == M &&
+                    out->size(1) == (gated ? N / 2 : N) &&
                     out->is_contiguous() &&
                     reinterpret_cast<uintptr_t>(out->data_ptr()) % 8 == 0,
                 "gemm_split: out");
-  auto aligned = [](const torch::Tensor& t) {
+  const long unit = fp8 ? 16 : 8, chunk = fp8 ? 256 : 128;
+  auto aligned = [&](const torch::Tensor& t) {
     return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0 &&
-           t.stride(0) % 8 == 0;
+           t.stride(0) % unit == 0 && t.stride(0) < (1l << 22);
   };
-  TORCH_CHECK(N % 4 == 0 && K % 128 == 0 && M < (1l << 20) && K < (1l << 24) &&
-                  N < (1l << 24) && aligned(x) && aligned(w) &&
-                  x.stride(0) < (1l << 22) && w.stride(0) < (1l << 22),
+  TORCH_CHECK(N % 4 == 0 && K % chunk == 0 && K >= chunk && M < (1l << 20) &&
+                  K < (1l << 24) && N < (1l << 24) && aligned(x) && aligned(w),
               "gemm_split: sizes");
-  TORCH_CHECK((bm == 128 && (bn == 64 || bn == 128)) ||
-                  (bm == 256 && bn == 128), "gemm_split: tile");
-  TORCH_CHECK(splits >= 1 && splits <= 8 && splits <= K / 128,
+  TORCH_CHECK(fp8 ? bm == 64 && (bn == 32 || bn == 64)
+                  : ((bm == 64 || bm == 128) && (bn == 64 || bn == 128)) ||
+                        (bm == 256 && bn == 128), "gemm_split: tile");
+  if (gated)      // 32 bits of offset reach the up rows
+    TORCH_CHECK(!fp8 && splits == 1 && bm <= 128 && N % 8 == 0 &&
+                    (N / 2 + 128) * w.stride(0) < (1l << 31),
+                "gemm_split: gated");
+  TORCH_CHECK(splits >= 1 && splits <= 8 && splits <= K / chunk,
               "gemm_split: 1 to 8 parts");
   float* ws = nullptr;
   if (splits > 1) {
@@ -506,9 +528,11 @@ void gemm_split(c10::optional<torch::Tensor> out, torch::Tensor x,
     ws = part->data_ptr<float>();
   }
   if (M == 0 || N == 0) return;
-  launch_gemm_split(out.has_value() ? bf(*out) : nullptr, ws, cbf(x), cbf(w),
-                    (int)M, (int)N, (int)K, x.stride(0), w.stride(0), (int)bm,
-                    (int)bn, (int)splits, stream());
+  launch_gemm_split(out.has_value() ? bf(*out) : nullptr, ws, x.data_ptr(),
+                    w.data_ptr(), fp8 ? x_scale->data_ptr<float>() : nullptr,
+                    fp8 ? w_scale->data_ptr<float>() : nullptr, (int)M, (int)N,
+                    (int)K, x.stride(0), w.stride(0), (int)bm, (int)bn,
+                    (int)splits, gated, stream());
 }
 
 void silu_mul(torch::Tensor out, torch::Tensor x) {
@@ -1158,6 +1182,30 @@ void fused_add_rmsnorm_fp8(torch::Tensor out, torch::Tensor scales,
                                x.numel() / hidden, hidden, stream());
 }
 
+// the same, x the sum of float parts [parts, rows, hidden]
+void parts_add_rmsnorm_fp8(torch::Tensor out, torch::Tensor scales,
+                           torch::Tensor parts, torch::Tensor residual,
+                           torch::Tensor w, double eps) {
+  check(out, torch::kFloat8_e4m3fn, "out");
+  check(scales, torch::kFloat, "scales");
+  check(parts, torch::kFloat, "parts");
+  check(residual, torch::kBFloat16, "residual");
+  check(w, torch::kBFloat16, "w");
+  TORCH_CHECK(parts.dim() == 3 && parts.size(0) >= 2 && parts.size(0) <= 8,
+              "parts_add_rmsnorm_fp8: 2 to 8 parts");
+  const long rows = parts.size(1);
+  const int hidden = (int)parts.size(2);
+  TORCH_CHECK(hidden % 8 == 0 && hidden <= 8192 && w.numel() == hidden &&
+                  out.numel() == rows * hidden && scales.numel() == rows &&
+                  residual.numel() == out.numel(),
+              "parts_add_rmsnorm_fp8: shape");
+  if (rows == 0) return;
+  launch_parts_add_rmsnorm_fp8(
+      u8(out), scales.data_ptr<float>(), parts.data_ptr<float>(),
+      (int)parts.size(0), bf(residual), cbf(w), (float)eps, rows, hidden,
+      stream());
+}
+
 void silu_mul_fp8(torch::Tensor out, torch::Tensor scales, torch::Tensor x) {
   check(out, torch::kFloat8_e4m3fn, "out");
   check(scales, torch::kFloat, "scales");
@@ -1203,6 +1251,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("rmsnorm", &rmsnorm);
   m.def("quant_fp8", &quant_fp8);
   m.def("fused_add_rmsnorm_fp8", &fused_add_rmsnorm_fp8);
+  m.def("parts_add_rmsnorm_fp8", &parts_add_rmsnorm_fp8);
   m.def("silu_mul_fp8", &silu_mul_fp8);
   m.def("moe_gemm", &moe_gemm);
   m.def("fused_add_rmsnorm", &fused_add_rmsnorm);
@@ -1214,7 +1263,12 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("decode_inputs", &decode_inputs);
   m.def("gemm_rows", &gemm_rows);
   m.def("gemm_rows_fits", &gemm_rows_fits);
-  m.def("gemm_split", &gemm_split);
+  m.def("gemm_split", &gemm_split, pybind11::arg("out"), pybind11::arg("x"),
+        pybind11::arg("w"), pybind11::arg("part"), pybind11::arg("bm"),
+        pybind11::arg("bn"), pybind11::arg("splits"),
+        pybind11::arg("x_scale") = pybind11::none(),
+        pybind11::arg("w_scale") = pybind11::none(),
+        pybind11::arg("gated") = false);
   m.def("parts_add_rmsnorm", &parts_add_rmsnorm);
   m.def("experts_few", &experts_few);
   m.def("choices_add_rmsnorm", &choices_add_rmsnorm);

@@ -1,5 +1,5 @@
 // out[M, N] = x[M, K] w[N, K]^T for tens to hundreds of rows (gfx950), bf16 in
-// and out, float sums.
+// and out, float sums; or e4m3 in, with scales of the rows, for up to 128 rows.
 //
 // A product of 256 rows with 4096 outputs is 64 tiles of 128 x 128, a quarter
 // of the compute units; so K is divided too, until there is about one workgroup
@@ -18,6 +18,12 @@
 //   4096 x 4096   32 rows 13 12, 96 22 14, 192 33 22, 256 23 23
 //   2048 x 7168   32 rows 19 11, 96 19 14, 192 25 19, 256 25 20, 512 32 29
 //   5120 x 8192   32 rows 25 23, 96 37 26, 192 61 36, 256 72 39
+// silu(gate) * up of the halves, product and activation and here: 28672 x 4096 17
+//   rows 47 41, 64 57 41, 128 59 48; 14336 x 2048 32 rows 19 13, 256 32 23
+// e4m3, with the norm that adds up the parts: 4096 x 14336 16 rows 27 19, 64 31
+// 21, 128 44 28; 4096 x 4096 16 rows 15 12, 128 18 15; without: 28672 x 4096 16
+// rows 34 24, 64 30.3 29.1; 14336 x 2048 64 rows 14 11; 6144 x 4096 13.7 12.3.
+// What bounds it: w from memory (5 TB/s with 16 rows), then the bytes in flight.
 #include "tile_loop.h"
 
 namespace {
@@ -25,8 +31,10 @@ namespace {
 struct Split {
   bf16* out;
   float* part;                 // [splits, M, N] with splits > 1
-  const bf16* x;
-  const bf16* w;
+  const void* x;
+  const void* w;
+  const float* x_scale;        // FP8: of a row of x, and of a row of w
+  const float* w_scale;
   int M, N, K;
   long xs, ws;                 // row strides
   int mt, nt, splits;          // tiles of rows, of outputs, parts of K
@@ -34,10 +42,12 @@ struct Split {
 
 // BM rows of x, BN of w; WM * WN waves have BM / WM by BN / WN.  A stage has
 // KC chunks of 64 columns.
-template <int BM, int BN, int WM, int WN, int STAGES, int KC>
-__global__ __launch_bounds__(WM * WN * 64, WM * WN / 4)
+template <int BM, int BN, int WM, int WN, int STAGES, int KC, bool FP8,
+          bool GATED>
+__global__ __launch_bounds__(WM * WN * 64, WM * WN < 4 ? 1 : WM * WN / 4)
 void gemm_split_kernel(Split a) {
-  using Loop = TileLoop<BM, BN, WM, WN, STAGES, KC, false>;
+  using Loop = TileLoop<BM, BN, WM, WN, STAGES, KC, FP8>;
+  constexpr int ELEM = FP8 ? 1 : 2;
   constexpr int LX = Loop::LX, LW = Loop::LW, NI = Loop::NI, MI = Loop::MI;
   extern __shared__ __attribute__((aligned(16))) char lds[];
   // workgroups go to the 8 XCDs in turn: those of one tile of w, which differ
@@ -45,8 +55,10 @@ void gemm_split_kernel(Split a) {
   const int at = blockIdx.x >> 3;
   const int u = at / a.mt * 8 + (blockIdx.x & 7);
   if (u >= a.nt * a.splits) return;
-  const int m0 = at % a.mt * BM, n0 = u / a.splits * BN, z = u % a.splits;
-  const int all = a.K / (64 * KC);
+  constexpr int OUT = GATED ? BN / 2 : BN;                 // outputs
+  const int m0 = at % a.mt * BM, n0 = u / a.splits * OUT, z = u % a.splits;
+  const int outs = GATED ? a.N >> 1 : a.N;
+  const int all = a.K * ELEM / (128 * KC);
   const int first = (int)((long)all * z / a.splits);
   const int chunks = (int)((long)all * (z + 1) / a.splits) - first;
   const int lane = threadIdx.x & 63;
@@ -57,22 +69,34 @@ void gemm_split_kernel(Split a) {
 
   // this lane's 16 bytes of row lane / 8 of each 1-KB load; rows past the end
   // are the last one
-  const RowLoads x_rows(a.x + m0 * a.xs + first * (64 * KC));
-  const RowLoads w_rows(a.w + n0 * a.ws + first * (64 * KC));
+  const RowLoads x_rows(static_cast<const char*>(a.x) + m0 * a.xs * ELEM +
+                        first * (128 * KC));
+  const RowLoads w_rows(static_cast<const char*>(a.w) + n0 * a.ws * ELEM +
+                        first * (128 * KC));
   unsigned x_off[LX], w_off[LW];
   #pragma unroll
   for (int j = 0; j < LX; ++j) {
     const int r = (wid * LX + j) * 8 + (lane >> 3);
-    x_off[j] = (unsigned)(min(r, a.M - 1 - m0) * a.xs * 2) +
+    x_off[j] = (unsigned)(min(r, a.M - 1 - m0) * a.xs * ELEM) +
                ((lane & 7) ^ (r >> 1 & 7)) * 16;
   }
   #pragma unroll
   for (int j = 0; j < LW; ++j) {
     const int r = (wid * LW + j) * 8 + (lane >> 3);
-    w_off[j] = (unsigned)(min(r, a.N - 1 - n0) * a.ws * 2) +
-               ((lane & 7) ^ (r >> 1 & 7)) * 16;
+    // gated: 8 gate rows, then their 8 up rows
+    const int n = min(GATED ? (r >> 4) * 8 + (r & 7) : r, outs - 1 - n0) +
+                  (GATED && r & 8 ? outs : 0);
+    w_off[j] = (unsigned)(n * a.ws * ELEM) + ((lane & 7) ^ (r >> 1 & 7)) * 16;
   }
+  // workgroups with all of K begin at different columns, so that not all of
+  // them ask the same channels of memory at once: 64 rows of 28672 x 4096 46 ->
+  // 42 us.  Not those that wait for x: 256 decoded tokens, where 6144 x 4096
+  // takes this kernel, 3245 us, with it 3251
+  const int turn =
+      (FP8 || GATED || BM == 64) && a.splits == 1 ? at % chunks : 0;
   auto stage = [&](int slot, int d) {
+    d += turn;
+    if (d >= chunks) d -= chunks;
     char* base = lds + slot * Loop::STAGE;
     #pragma unroll
     for (int j = 0; j < LX; ++j)
@@ -97,23 +121,44 @@ void gemm_split_kernel(Split a) {
   for (int m = 0; m < MI; ++m) {
     const int row = m0 + (wm * MI + m) * 32 + col;
     if (row >= a.M) continue;
+    const float xs = FP8 ? a.x_scale[row] : 1.f;
     #pragma unroll
-    for (int n = 0; n < NI; ++n)
+    for (int n = 0; n < NI; ++n) {
+      if constexpr (GATED) {
+        #pragma unroll
+        for (int r = 0; r < 16; r += 8) {
+          const int c = n0 + (wn * NI + n) * 16 + r + hf * 4;
+          if (c >= outs) continue;
+          float y[4];
+          #pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const float g = acc[n][m][r + j], u = acc[n][m][r + 4 + j];
+            y[j] = g / (1.f + __expf(-g)) * u;
+          }
+          *reinterpret_cast<uint2*>(a.out + (long)row * outs + c) =
+              uint2{cvt_pk_bf16(y[0], y[1]), cvt_pk_bf16(y[2], y[3])};
+        }
+        continue;
+      }
       #pragma unroll
       for (int r = 0; r < 16; r += 4) {
         const int c = n0 + (wn * NI + n) * 32 + r * 2 + hf * 4;
         if (c >= a.N) continue;                  // N is a multiple of 4
-        if (a.splits > 1) {
-          *reinterpret_cast<f32x4_t*>(
-              a.part + ((long)z * a.M + row) * a.N + c) =
-              f32x4_t{acc[n][m][r], acc[n][m][r + 1], acc[n][m][r + 2],
-                      acc[n][m][r + 3]};
-        } else {
-          *reinterpret_cast<uint2*>(a.out + (long)row * a.N + c) =
-              uint2{cvt_pk_bf16(acc[n][m][r], acc[n][m][r + 1]),
-                    cvt_pk_bf16(acc[n][m][r + 2], acc[n][m][r + 3])};
+        f32x4_t y{acc[n][m][r], acc[n][m][r + 1], acc[n][m][r + 2],
+                  acc[n][m][r + 3]};
+        if constexpr (FP8) {
+          const f32x4_t ws = *reinterpret_cast<const f32x4_t*>(a.w_scale + c);
+          #pragma unroll
+          for (int i = 0; i < 4; ++i) y[i] = y[i] * xs * ws[i];
         }
+        if (a.splits > 1)
+          *reinterpret_cast<f32x4_t*>(
+              a.part + ((long)z * a.M + row) * a.N + c) = y;
+        else
+          *reinterpret_cast<uint2*>(a.out + (long)row * a.N + c) =
+              uint2{cvt_pk_bf16(y[0], y[1]), cvt_pk_bf16(y[2], y[3])};
       }
+    }
   }
 }
 
@@ -135,34 +180,56 @@ __global__ __launch_bounds__(256) void gemm_sum_kernel(
 
 }  // namespace
 
-// Tiles of bm rows by bn outputs: 128 x 64, 128 x 128, 256 x 128.  out
-// contiguous; K a multiple of 128, N of 4; rows of x and w 16-byte aligned;
-// splits 1 to 8, at most K / 128, part with more than one.  Without out the
-// parts are left for the norm that adds them up.
-void launch_gemm_split(bf16* out, float* part, const bf16* x, const bf16* w,
-                       int M, int N, int K, long xs, long ws, int bm,
-                       int bn, int splits, hipStream_t stream) {
-  Split a{out, part, x, w, M, N, K, xs, ws, 0, 0, splits};
-  #define RUN(BM, BN, WM, WN, STAGES, KC)                                   \
+// Tiles of bm rows of x by bn of w: 64 x 64, 64 x 128, 128 x 64, 128 x 128, 256 x
+// 128; with scales x and w are e4m3, in tiles of 64 x 32 or 64 x 64.  out
+// contiguous; rows of K of 256 bytes, N a multiple of 4; rows of x and w 16-byte
+// aligned; splits 1 to 8, at most one a 256 bytes, part with more than one.
+// Without out the parts are left for the norm that adds them up.  gated, of
+// bfloat16 without parts: out = silu(gate) * up of the halves of w, whose rows
+// are a multiple of 8, in tiles of up to 128 rows.
+void launch_gemm_split(bf16* out, float* part, const void* x, const void* w,
+                       const float* x_scale, const float* w_scale, int M,
+                       int N, int K, long xs, long ws, int bm, int bn,
+                       int splits, bool gated, hipStream_t stream) {
+  Split a{out, part, x, w, x_scale, w_scale, M, N, K, xs, ws, 0, 0, splits};
+  #define RUN(BM, BN, WM, WN, STAGES, KC, FP8, GATED)                       \
     {                                                                       \
       constexpr int BYTES = STAGES * KC * (BM + BN) * 128;                  \
       static const hipError_t set = hipFuncSetAttribute(                    \
           reinterpret_cast<const void*>(                                    \
-              &gemm_split_kernel<BM, BN, WM, WN, STAGES, KC>),              \
+              &gemm_split_kernel<BM, BN, WM, WN, STAGES, KC, FP8, GATED>),  \
           hipFuncAttributeMaxDynamicSharedMemorySize, BYTES);               \
       HIP_CHECK(set);                                                       \
       a.mt = (M + BM - 1) / BM;                                             \
       a.nt = (N + BN - 1) / BN;                                             \
       const unsigned units = (unsigned)(a.nt * splits + 7) / 8 * 8;         \
-      gemm_split_kernel<BM, BN, WM, WN, STAGES, KC>                           \
+      gemm_split_kernel<BM, BN, WM, WN, STAGES, KC, FP8, GATED>             \
           <<<units * a.mt, WM * WN * 64, BYTES, stream>>>(a);               \
     }
-  if (bm == 256)
-    RUN(256, 128, 4, 2, 3, 1)
+  #define KINDS(BM, BN, WM, WN, STAGES, KC)                                 \
+    {                                                                       \
+      if (gated) RUN(BM, BN, WM, WN, STAGES, KC, false, true)               \
+      else RUN(BM, BN, WM, WN, STAGES, KC, false, false)                    \
+    }
+  if (x_scale) {
+    // two workgroups a unit, with half the ring each, where there are as many
+    if (bn == 32)
+      RUN(64, 32, 2, 1, 3, 2, true, false)
+    else if ((long)((M + 63) / 64) * ((N + 63) / 64) * splits > 256)
+      RUN(64, 64, 2, 2, 2, 2, true, false)
+    else
+      RUN(64, 64, 2, 2, 4, 2, true, false)
+  } else if (bm == 256)
+    RUN(256, 128, 4, 2, 3, 1, false, false)
+  else if (bm == 128 && bn == 128)
+    KINDS(128, 128, 2, 4, 4, 1)
+  else if (bm == 128)
+    KINDS(128, 64, 4, 2, 3, 2)
   else if (bn == 128)
-    RUN(128, 128, 2, 4, 4, 1)
+    KINDS(64, 128, 2, 2, 3, 2)
   else
-    RUN(128, 64, 4, 2, 3, 2)
+    KINDS(64, 64, 2, 2, 4, 2)
+  #undef KINDS
   #undef RUN
   if (splits == 1 || !out) return;
   const long quads = (long)M * N / 4;

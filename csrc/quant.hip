@@ -74,12 +74,15 @@ __global__ __launch_bounds__(256) void quant_fp8_kernel(
   }
 }
 
-// residual <- residual + x (bf16, in place); out <- fp8(rmsnorm(residual)*w)
-template <int CH>
+// residual <- residual + x (bf16, in place); out <- fp8(rmsnorm(residual)*w).
+// With `parts` x is the sum of that many float products [parts, rows, hidden],
+// rounded as a product is, whose own launch and trip to memory this saves.
+template <int CH, bool PARTS>
 __global__ __launch_bounds__(256) void fused_add_rmsnorm_fp8_kernel(
     unsigned char* __restrict__ out, float* __restrict__ scales,
-    const bf16* __restrict__ x, bf16* __restrict__ residual,
-    const bf16* __restrict__ w, float eps, int hidden) {
+    const bf16* __restrict__ x, const float* __restrict__ part, int parts,
+    bf16* __restrict__ residual, const bf16* __restrict__ w, float eps,
+    int hidden) {
   __shared__ float scratch[4];
   const long row = blockIdx.x;
   const bf16* xr = x + row * (long)hidden;
@@ -90,9 +93,24 @@ __global__ __launch_bounds__(256) void fused_add_rmsnorm_fp8_kernel(
   for (int c = 0; c < CH; ++c) {
     const int base = (c * 256 + threadIdx.x) * 8;
     if (base < hidden) {
-      xv[c] = load_bf16x8(xr + base);
       rv[c] = load_bf16x8(rr + base);
       wv[c] = load_bf16x8(w + base);
+      if constexpr (PARTS) {
+        const long stride = (long)gridDim.x * hidden;     // of a part
+        const float* p = part + row * hidden + base;
+        f32x4_t y0 = *reinterpret_cast<const f32x4_t*>(p);
+        f32x4_t y1 = *reinterpret_cast<const f32x4_t*>(p + 4);
+        #pragma unroll 4
+        for (int z = 1; z < parts; ++z) {
+          y0 += *reinterpret_cast<const f32x4_t*>(p + z * stride);
+          y1 += *reinterpret_cast<const f32x4_t*>(p + z * stride + 4);
+        }
+        #pragma unroll
+        for (int i = 0; i < 8; ++i)
+          bf16x8_set(xv[c], i, i < 4 ? y0[i & 3] : y1[i & 3]);
+      } else {
+        xv[c] = load_bf16x8(xr + base);
+      }
     }
   }
   float r[CH][8];
@@ -219,11 +237,26 @@ void launch_fused_add_rmsnorm_fp8(unsigned char* out, float* scales,
                                   int hidden, hipStream_t stream) {
   if (hidden % 8 || hidden > QCHUNKS * 256 * 8)
     throw std::runtime_error("fused_add_rmsnorm_fp8: bad hidden");
-  const auto kernel = hidden <= 4096   ? fused_add_rmsnorm_fp8_kernel<2>
-                      : hidden <= 8192 ? fused_add_rmsnorm_fp8_kernel<4>
-                                       : fused_add_rmsnorm_fp8_kernel<QCHUNKS>;
-  kernel<<<dim3((unsigned)rows), 256, 0, stream>>>(out, scales, x, residual, w,
-                                                   eps, hidden);
+  const auto kernel =
+      hidden <= 4096   ? fused_add_rmsnorm_fp8_kernel<2, false>
+      : hidden <= 8192 ? fused_add_rmsnorm_fp8_kernel<4, false>
+                       : fused_add_rmsnorm_fp8_kernel<QCHUNKS, false>;
+  kernel<<<dim3((unsigned)rows), 256, 0, stream>>>(
+      out, scales, x, nullptr, 0, residual, w, eps, hidden);
+}
+
+// 2 to 8 parts, hidden a multiple of 8 up to 8192
+void launch_parts_add_rmsnorm_fp8(unsigned char* out, float* scales,
+                                  const float* part, int parts,
+                                  bf16* residual, const bf16* w, float eps,
+                                  long rows, int hidden, hipStream_t stream) {
+  const auto kernel = hidden <= 2048
+                          ? fused_add_rmsnorm_fp8_kernel<1, true>
+                      : hidden <= 4096
+                          ? fused_add_rmsnorm_fp8_kernel<2, true>
+                          : fused_add_rmsnorm_fp8_kernel<4, true>;
+  kernel<<<dim3((unsigned)rows), 256, 0, stream>>>(
+      out, scales, nullptr, part, parts, residual, w, eps, hidden);
 }
 
 void launch_silu_mul_fp8(unsigned char* out, float* scales, const bf16* x,

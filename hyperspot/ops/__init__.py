@@ -351,9 +351,14 @@ def _split_gemm(M: int, N: int, K: int):
     return 128, 128, wide
 
 
+def _near(*tensors: torch.Tensor) -> bool:
+    """Rows that 32 bits of offset reach from the first one of a tile."""
+    return all(t.stride(0) < 1 << 22 for t in tensors)
+
+
 def linear_parts(x: torch.Tensor, w: torch.Tensor):
     """x w^T for w [N, K], as Parts where it is formed in parts of K."""
-    if not _rows_gemm(x, w) and _plain_bf16(x, w):
+    if not _rows_gemm(x, w) and _plain_bf16(x, w) and _near(x, w):
         M, N = x.shape[0], w.shape[0]
         split = _split_gemm(M, N, x.shape[1])
         if split is not None and split[2] > 1 and N % 8 == 0 and N <= 8192:
@@ -371,7 +376,7 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
                           device=x.device)
         _native().gemm_rows(out, x, w)
         return out
-    if _plain_bf16(x, w):
+    if _plain_bf16(x, w) and _near(x, w):
         M, N = x.shape[0], w.shape[0]
         split = _split_gemm(M, N, x.shape[1])
         if split is not None:
@@ -394,6 +399,79 @@ class QTensor(NamedTuple):
     scale: torch.Tensor
 
 
+def _tiles_q(M: int, N: int, K: int, parts: bool):
+    """(rows, outputs of a tile, parts of K) where csrc/gemm_split.hip is
+    faster than the library for x e4m3 [M, K] and w e4m3 [N, K], else None.
+    With `parts` their sum costs little, for the norm that follows forms it.
+
+    Measured at 1 to 128 rows, N of 1024 to 40000 and K of 1024 to 14336 in 400
+    random sizes: 0.8 of the library's time on average, and more than 3 % slower
+    at 3 of 100.  Tiles of 64 x 64 that fill three quarters of the compute
+    units need no parts (64 rows of 28672 x 4096 30.3 -> 29.1 us, 16 33.8 ->
+    24.5; 14336 x 2048 14.3 -> 11.0); with K beyond 4096 the library catches up
+    from 17 rows on (25 rows of 27680 x 6144 34.7 35.8, 6 41.9 29.7), with more
+    than 32768 outputs for any (4 rows of 35424 x 6144 47 57).  Fewer tiles are
+    divided into parts of 1365 columns and more, about one workgroup a unit (64
+    rows of 4096 x 14336 with the norm 30.6 -> 21.5, of 2048 x 7168 16.3 ->
+    12.8), or made half as wide (6144 x 4096 13.7 -> 12.3, 3072 x 2048 9.1 ->
+    7.6).  Where another kernel adds up the parts they gain with 8192 columns,
+    or with few rows (1 of 3600 x 5120 14.0 -> 9.2; 21 of 6032 x 5120 11.7 13.0).
+    Beyond 64 rows half as many tiles lie beside each other: long rows only with
+    the norm (128 of 4096 x 14336 44 -> 28), 2048 x 7168 is even (14.0 13.7).
+    Beyond 128 rows there is no gain (200 of 4096 x 4096 17.1 17.2)."""
+    if not 1 <= M <= 128 or K % 256 or N % 4 or N * K < 1 << 22:
+        return None
+    tiles = -(-M // 64) * -(-N // 64)
+    few = M <= 16
+    if tiles >= 192:
+        return (64, 64, 1) if N <= (32768 if M <= 64 else 20480) and (
+            few or K <= 2048 or K <= 4096 and (M <= 64 or N <= 8192)) else None
+    split = min(8, max(2, K // 1365), 256 // tiles)
+    if M > 64 and K > 4096 and (K < 8192 or split == 1 or not parts):
+        return None
+    if parts and split > 1:
+        return 64, 64, split
+    if K > 4096:
+        return (64, 64, max(2, split)) \
+            if tiles <= 96 and (few or K >= 8192) else None
+    if K > 2048 and tiles < (64 if M <= 64 else 128):
+        return (64, 64, min(8, 256 // tiles)) if few else None
+    return (64, 32, 1) if tiles <= 128 else (64, 64, 1)
+
+
+def _tiled_q(x: "QTensor", w: torch.Tensor, scale: torch.Tensor, parts: bool):
+    """The tile of _tiles_q, or None."""
+    d, s = x
+    if not (d.is_cuda and d.dtype == w.dtype == torch.float8_e4m3fn
+            and s.dtype == scale.dtype == torch.float32
+            and unrecorded(d, w, s, scale) and _near(d, w)
+            and s.is_contiguous() and scale.is_contiguous()
+            and scale.data_ptr() % 16 == 0
+            and all(t.dim() == 2 and t.stride(1) == 1 and t.stride(0) % 16 == 0
+                    and t.data_ptr() % 16 == 0 for t in (d, w))):
+        return None
+    return _tiles_q(d.shape[0], w.shape[0], d.shape[1], parts)
+
+
+def linear_q(x: "QTensor", w: torch.Tensor, scale: torch.Tensor,
+             parts: bool = False):
+    """x w^T of e4m3 with scales of the rows, bf16; with `parts` as Parts where
+    it is formed in parts of K.  GPU."""
+    tile = _tiled_q(x, w, scale, parts)
+    if tile is None:
+        return torch._scaled_mm(x.data, w.t(), scale_a=x.scale.unsqueeze(1),
+                                scale_b=scale.unsqueeze(0),
+                                out_dtype=torch.bfloat16)
+    M, N = x.data.shape[0], w.shape[0]
+    part = torch.empty(tile[2], M, N, dtype=torch.float32,
+                       device=w.device) if tile[2] > 1 else None
+    keep = parts and part is not None and N % 8 == 0 and N <= 8192
+    out = None if keep else torch.empty(M, N, dtype=torch.bfloat16,
+                                        device=w.device)
+    _native().gemm_split(out, x.data, w, part, *tile, x.scale, scale)
+    return Parts(part) if keep else out
+
+
 def quant_fp8(x: torch.Tensor) -> QTensor:
     """[T,K] bf16 -> QTensor (GPU; row-per-workgroup amax+scale+pack)."""
     assert x.is_cuda
@@ -408,14 +486,16 @@ def fused_add_rmsnorm_q(x: torch.Tensor, residual: torch.Tensor,
                         weight: torch.Tensor, eps: float):
     """residual += x (in place); returns (QTensor of rmsnorm(residual)*w,
     residual).  GPU-only fused producer for the fp8 GEMM path."""
-    if isinstance(x, Parts):      # of a layer with 16-bit weights before it
-        x = x.data.sum(0).to(residual.dtype)
-    elif isinstance(x, Choices):
+    if isinstance(x, Choices):
         x = _moe_sum(x)
+    T, K = residual.shape
+    out = torch.empty(T, K, dtype=torch.float8_e4m3fn, device=residual.device)
+    scales = torch.empty(T, dtype=torch.float32, device=residual.device)
+    if isinstance(x, Parts):
+        _native().parts_add_rmsnorm_fp8(out, scales, x.data, residual, weight,
+                                        eps)
+        return QTensor(out, scales), residual
     assert x.is_cuda
-    T, K = x.shape
-    out = torch.empty(T, K, dtype=torch.float8_e4m3fn, device=x.device)
-    scales = torch.empty(T, dtype=torch.float32, device=x.device)
     _native().fused_add_rmsnorm_fp8(out, scales, x, residual, weight, eps)
     return QTensor(out, scales), residual
 

@@ -115,10 +115,7 @@ class _LinearCompute(nn.Module):
         from hyperspot import ops as _O   # local: avoids import cycle at init
         if isinstance(x, _O.QTensor):
             # pre-quantized by a fused producer kernel (csrc/quant.hip)
-            return torch._scaled_mm(
-                x.data, self.weight.t(), scale_a=x.scale.unsqueeze(1),
-                scale_b=self.weight_scale.unsqueeze(0),
-                out_dtype=torch.bfloat16)
+            return _O.linear_q(x, self.weight, self.weight_scale)
         if self.quant == "fp8":
             xq, xs = quant_fp8_rowwise(x)
             if x.is_cuda:
@@ -278,6 +275,9 @@ class RowParallelLinear(_LinearCompute):
         if self.quant is None and get_tp_size() == 1 \
                 and isinstance(x, torch.Tensor):
             return _O.linear_parts(x, self.weight)
+        if self.quant == "fp8" and get_tp_size() == 1 \
+                and isinstance(x, _O.QTensor):
+            return _O.linear_q(x, self.weight, self.weight_scale, True)
         return self.forward(x)
 
 
