@@ -24,7 +24,7 @@ from hyperspot import ops
 from hyperspot.engine.config import ModelSpec
 from hyperspot.ops.torch_ref import rope_cos_sin
 from hyperspot.parallel import (QKVParallelLinear, RowParallelLinear,
-                                MergedColumnParallelLinear, summands)
+                                MergedColumnParallelLinear, summands, watched)
 from hyperspot.parallel.state import get_tp_size
 
 
@@ -149,6 +149,10 @@ class LlamaMLP(nn.Module):
         return summands(self.down, self._inner(x))
 
     def _inner(self, x):
+        if type(self.gate_up) is MergedColumnParallelLinear \
+                and self.gate_up.quant is None and self.down.quant is None \
+                and not watched(self.gate_up) and x.is_cuda:
+            return ops.gated_linear(x, self.gate_up.weight)
         gu = self.gate_up(x)
         if self.down.quant == "fp8" and gu.is_cuda:
             return ops.silu_mul_q(gu)

@@ -4,4 +4,4 @@ from .state import (initialize_model_parallel, destroy_model_parallel,
                     tensor_model_parallel_all_reduce)
 from .layers import (ColumnParallelLinear, RowParallelLinear, QKVParallelLinear,
                      MergedColumnParallelLinear, MergedRowParallelLinear,
-                     summands)
+                     summands, watched)

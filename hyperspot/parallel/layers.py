@@ -65,13 +65,17 @@ def summands(module: nn.Module, *args):
     that is still in parts (ops.Parts), where the module's own class says how
     (`_summands`) and nothing else sees or replaces the call."""
     own = vars(type(module)).get("_summands")
-    if own is None or "forward" in vars(module) \
-            or module._compiled_call_impl is not None \
-            or module._forward_hooks or module._forward_pre_hooks \
-            or module._backward_hooks or module._backward_pre_hooks \
-            or _has_any_global_hook():
-        return module(*args)
-    return own(module, *args)
+    return module(*args) if own is None or watched(module) \
+        else own(module, *args)
+
+
+def watched(module: nn.Module) -> bool:
+    """Whether something else sees or replaces a call of this module."""
+    return "forward" in vars(module) \
+        or module._compiled_call_impl is not None \
+        or bool(module._forward_hooks or module._forward_pre_hooks
+                or module._backward_hooks or module._backward_pre_hooks) \
+        or _has_any_global_hook()
 
 
 class _LinearCompute(nn.Module):

@@ -39,6 +39,89 @@ def test_gemm_split(M, N, K, parts, bm, bn):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("bm,bn", [(64, 64), (64, 128)])
+@pytest.mark.parametrize("M,N,K,parts", [
+    (1, 4, 128, 1), (64, 60, 256, 2), (65, 132, 640, 4), (33, 1028, 896, 7)])
+def test_tiles_of_64_rows(M, N, K, parts, bm, bn):
+    test_gemm_split(M, N, K, parts, bm, bn)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(33, 2048, 2048), (64, 4096, 1280),
+                                   (128, 4096, 2560), (257, 3200, 8192),
+                                   (480, 4096, 4096), (400, 5120, 5120)])
+def test_parts_that_the_norm_adds_up(M, N, K):
+    g = torch.Generator().manual_seed(M)
+    x = torch.randn(M, K, generator=g).bfloat16().to(DEV)
+    w = torch.randn(N, K, generator=g).bfloat16().to(DEV)
+    bm, bn, parts = ops._summed_gemm(M, N, K)
+    assert -(-M // bm) * -(-N // bn) * parts <= 256 and 1 < parts <= 8
+    got = ops.linear_parts(x, w)
+    assert got.data.shape == (parts, M, N)
+    _check(got.data.sum(0), x, w)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bm,bn", [(64, 64), (64, 128), (128, 64), (128, 128)])
+@pytest.mark.parametrize("M,N,K", [
+    (1, 8, 128), (31, 120, 256), (64, 128, 384), (65, 264, 640), (128, 1032, 128),
+    (129, 8, 1024), (17, 4104, 512)])
+def test_gated(M, N, K, bm, bn):
+    """silu(gate) * up: an error e of the gate becomes at most 1.1 e |up|, one of
+    up |silu| e; the result is rounded to bf16 and the exponential is exact to
+    2^-20."""
+    g = torch.Generator().manual_seed(M)
+    x = torch.randn(M, K + 8, generator=g).bfloat16().to(DEV)[:, :K]
+    w = (torch.randn(N, K, generator=g) * 0.1).bfloat16().to(DEV)
+    out = torch.full((M, N // 2), float("nan"), dtype=torch.bfloat16,
+                     device=DEV)
+    ops._native().gemm_split(out, x, w, None, bm, bn, 1, gated=True)
+    x, w = x.double().cpu(), w.double().cpu()
+    gate, up = (x @ w.t()).chunk(2, -1)
+    err = K * 2.0 ** -24 * (x.abs() @ w.abs().t())
+    silu = torch.nn.functional.silu(gate)
+    ref = silu * up
+    bound = ref.abs() * 2.0 ** -8 + 1.1 * up.abs() * err[:, :N // 2] \
+        + silu.abs() * err[:, N // 2:] + 1e-30
+    assert ((out.double().cpu() - ref).abs() <= bound).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [16, 17, 64, 65, 128, 129, 256, 257])
+@pytest.mark.parametrize("N,K", [(2048, 1024), (14336, 2048), (28672, 512),
+                                 (28672, 4224), (2064, 640)])
+def test_gated_linear(M, N, K):
+    g = torch.Generator().manual_seed(M)
+    x = torch.randn(M, K, generator=g).bfloat16().to(DEV)
+    w = (torch.randn(N, K, generator=g) * K ** -0.5).bfloat16().to(DEV)
+    out = ops.gated_linear(x, w)
+    want = ops.silu_mul(x @ w.t())      # gate and up rounded to bf16
+    tile = ops._gated_tile(M, N, K)
+    assert tile is None or 16 < M <= 256
+    assert (out.float() - want.float()).norm() <= 2.0 ** -7 * want.float().norm()
+
+
+@pytest.mark.gpu
+def test_watched_products_get_their_calls():
+    """A hook on the gate and up product sees it, and may change it."""
+    from hyperspot.engine.config import ModelSpec
+    from hyperspot.models.llama import LlamaMLP
+    from hyperspot.parallel import layers
+    layers.set_init_device(DEV)
+    spec = ModelSpec("t", 256, 1, 2, 1, 128, 2048, 32)
+    mlp = LlamaMLP(spec, 0, torch.bfloat16).to(DEV)
+    layers.set_init_device("cpu")
+    x = torch.randn(32, 256, device=DEV).bfloat16()
+    fused = mlp(x)
+    seen = []
+    h = mlp.gate_up.register_forward_hook(
+        lambda m, a, y: seen.append(y.shape) or y * 0)
+    assert mlp(x).abs().max() == 0 and seen == [(32, 4096)]
+    h.remove()
+    assert torch.equal(mlp(x), fused)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("M", [17, 128, 129, 256, 257, 512])
 @pytest.mark.parametrize("N,K", [(4096, 4096), (2048, 7168), (5120, 8192)])
 def test_linear_takes_it(M, N, K):
