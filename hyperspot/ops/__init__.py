@@ -9,6 +9,7 @@ device without the extension is a hard error, never a silent eager fallback.
 
 from __future__ import annotations
 
+from functools import lru_cache
 from typing import NamedTuple
 
 import torch
@@ -270,6 +271,20 @@ def _rows_gemm(x: torch.Tensor, w: torch.Tensor) -> bool:
         and _native().gemm_rows_fits(*x.shape)
 
 
+MOST_ROWS = 512         # of a product that a kernel here takes
+
+
+@lru_cache(maxsize=1 << 14)
+def _route(M: int, N: int, K: int, parts: bool):
+    """How x w^T of these sizes is formed: "rows", (rows, outputs of a tile, parts
+    of K) or None, the library.  Kept, for the rules take as long as a launch: a
+    step of small prompts, which is not captured, waits for the host."""
+    if _rows_gemm_sizes(M, N, K) and _native().gemm_rows_fits(M, K):
+        return "rows"
+    return _less_padding(M, _split_gemm(M, N, K)) \
+        or (_summed_gemm(M, N, K) if parts else None)
+
+
 def _rows_gemm_sizes(M: int, N: int, K: int) -> bool:
     """Measured at 1 to 64 rows, K of 256 to 4096 and N of 256 to 160000, 40000
     random sizes (time of the kernel over the library's, means of a class).  Up
@@ -387,39 +402,39 @@ def _near(*tensors: torch.Tensor) -> bool:
     return all(t.stride(0) < 1 << 22 for t in tensors)
 
 
+def _product(x: torch.Tensor, w: torch.Tensor, parts: bool, plain: bool):
+    """x w^T for w [N, K]; with `parts` as Parts where it is formed so.  plain:
+    what _plain_bf16 says, which looks at the sizes of no traced tensor."""
+    route = _route(x.shape[0], *w.shape, parts) \
+        if plain and x.shape[0] <= MOST_ROWS else None
+    if route is None or route != "rows" and not _near(x, w):
+        return x @ w.t()
+    M, N = x.shape[0], w.shape[0]
+    if route == "rows":
+        out = torch.empty(M, N, dtype=x.dtype, device=x.device)
+        _native().gemm_rows(out, x, w)
+        return out
+    part = torch.empty(route[2], M, N, dtype=torch.float32,
+                       device=x.device) if route[2] > 1 else None
+    if parts and part is not None and N % 8 == 0 and N <= 8192:
+        _native().gemm_split(None, x, w, part, *route)
+        return Parts(part)
+    out = torch.empty(M, N, dtype=x.dtype, device=x.device)
+    _native().gemm_split(out, x, w, part, *route)
+    return out
+
+
 def linear_parts(x: torch.Tensor, w: torch.Tensor):
     """x w^T for w [N, K], as Parts where it is formed in parts of K."""
-    if not _rows_gemm(x, w) and _plain_bf16(x, w) and _near(x, w):
-        M, N = x.shape[0], w.shape[0]
-        split = _less_padding(M, _split_gemm(M, N, x.shape[1])) \
-            or _summed_gemm(M, N, x.shape[1])
-        if split is not None and split[2] > 1 and N % 8 == 0 and N <= 8192:
-            part = torch.empty(split[2], M, N, dtype=torch.float32,
-                               device=x.device)
-            _native().gemm_split(None, x, w, part, *split)
-            return Parts(part)
-    return linear(x, w)
+    return _product(x, w, True, _plain_bf16(x, w))
 
 
 def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """x w^T for w [N, K]."""
-    if _rows_gemm(x, w):
-        out = torch.empty(x.shape[0], w.shape[0], dtype=x.dtype,
-                          device=x.device)
-        _native().gemm_rows(out, x, w)
-        return out
-    if _plain_bf16(x, w) and _near(x, w):
-        M, N = x.shape[0], w.shape[0]
-        split = _less_padding(M, _split_gemm(M, N, x.shape[1]))
-        if split is not None:
-            out = torch.empty(M, N, dtype=x.dtype, device=x.device)
-            part = torch.empty(split[2] * M * N, dtype=torch.float32,
-                               device=x.device) if split[2] > 1 else None
-            _native().gemm_split(out, x, w, part, *split)
-            return out
-    return x @ w.t()
+    return _product(x, w, False, _plain_bf16(x, w))
 
 
+@lru_cache(maxsize=1 << 14)
 def _gated_tile(M: int, N: int, K: int):
     """(rows, rows of w of a tile) where csrc/gemm_split.hip forms silu(gate) *
     up of x w^T faster than a product and an activation, else None: the smallest
@@ -445,14 +460,15 @@ def _gated_tile(M: int, N: int, K: int):
 
 def gated_linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """silu_mul of x w^T, w the gate's rows and then the up rows."""
-    if _plain_bf16(x, w) and _near(x, w) and w.numel() < 1 << 31:
-        M, N = x.shape[0], w.shape[0]
-        tile = _gated_tile(M, N, x.shape[1])
-        if tile is not None:
-            out = torch.empty(M, N // 2, dtype=x.dtype, device=x.device)
+    plain = _plain_bf16(x, w)
+    if plain and x.shape[0] <= MOST_ROWS:
+        tile = _gated_tile(x.shape[0], *w.shape)
+        if tile is not None and _near(x, w) and w.numel() < 1 << 31:
+            out = torch.empty(x.shape[0], w.shape[0] // 2, dtype=x.dtype,
+                              device=x.device)
             _native().gemm_split(out, x, w, None, *tile, 1, gated=True)
             return out
-    return silu_mul(linear(x, w))
+    return silu_mul(_product(x, w, False, plain))
 
 
 class QTensor(NamedTuple):
@@ -466,6 +482,7 @@ class QTensor(NamedTuple):
     scale: torch.Tensor
 
 
+@lru_cache(maxsize=1 << 14)
 def _tiles_q(M: int, N: int, K: int, parts: bool):
     """(rows, outputs of a tile, parts of K) where csrc/gemm_split.hip is
     faster than the library for x e4m3 [M, K] and w e4m3 [N, K], else None.
@@ -509,15 +526,19 @@ def _tiles_q(M: int, N: int, K: int, parts: bool):
 def _tiled_q(x: "QTensor", w: torch.Tensor, scale: torch.Tensor, parts: bool):
     """The tile of _tiles_q, or None."""
     d, s = x
-    if not (d.is_cuda and d.dtype == w.dtype == torch.float8_e4m3fn
+    if not (d.is_cuda and unrecorded(d, w, s, scale)
+            and d.dim() == w.dim() == 2):
+        return None
+    tile = _tiles_q(d.shape[0], *w.shape, parts)
+    if tile is None or not (
+            d.dtype == w.dtype == torch.float8_e4m3fn and _near(d, w)
             and s.dtype == scale.dtype == torch.float32
-            and unrecorded(d, w, s, scale) and _near(d, w)
             and s.is_contiguous() and scale.is_contiguous()
             and scale.data_ptr() % 16 == 0
-            and all(t.dim() == 2 and t.stride(1) == 1 and t.stride(0) % 16 == 0
+            and all(t.stride(1) == 1 and t.stride(0) % 16 == 0
                     and t.data_ptr() % 16 == 0 for t in (d, w))):
         return None
-    return _tiles_q(d.shape[0], w.shape[0], d.shape[1], parts)
+    return tile
 
 
 def linear_q(x: "QTensor", w: torch.Tensor, scale: torch.Tensor,
