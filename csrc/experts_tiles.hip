@@ -16,8 +16,8 @@
 // is what covers most counts (256 rows of x, mostly padding, beside 128 of
 // weights are two thirds of what is loaded), then the products.  Mixtral 8x7B
 // layer (8 experts, 14336 x 4096, 2.8 GB), us with 256-row tiles, row tiles
-// and here: 16 choices an expert 821 617 532, 48 831 792 543, 128 943 869 730,
-// 500 2355 2100 1740.  32 experts of 1024 x 2048, 64 choices 277 172 119.
+// and here: 16 choices an expert 821 617 473, 48 831 792 487, 128 943 869 719,
+// 500 2355 2100 1650.  32 experts of 1024 x 2048, 62 choices 277 172 96.
 #include "tile_loop.h"
 
 namespace {
@@ -91,7 +91,17 @@ void experts_tiles_kernel(Tiles a) {
     else
       rows.to_lds(l, (unsigned)off, d * 128);
   };
+  // Where the weights are the bound workgroups begin at different columns, so
+  // that not all of them ask the same channels of memory at once; those of one
+  // expert and the same outputs at the same.  192 tokens of 2 choices, 8 experts
+  // of 14336 x 4096 355 + 188 -> 321 + 162 us; 4 of 32 of 1024 x 2048 65 + 29 ->
+  // 50 + 29; in tiles of 256, 500 choices an expert, 1011 + 639 1029 + 643.
+  const int stages = (int)(row_bytes / 128);
+  const int turn = BM == 256 ? 0
+      : (blockIdx.x % a.nx + e * a.nx) / 8 * (stages >= 64 ? 3 : 1) % stages;
   auto stage = [&](int slot, int d) {
+    d += turn;
+    if (d >= stages) d -= stages;
     char* l = lds + slot * Loop::STAGE;
     #pragma unroll
     for (int j = 0; j < LX; ++j)
@@ -101,7 +111,7 @@ void experts_tiles_kernel(Tiles a) {
       load(l + BM * 128 + (wid * LW + j) * 1024, w_rows, w0, w_off[j], d);
   };
   Loop loop;
-  loop.run(lds, wm, wn, (int)(row_bytes / 128), live, stage);
+  loop.run(lds, wm, wn, stages, live, stage);
   auto& acc = loop.acc;
 
   // acc[n][m][r]: weight row (r >> 2) * 8 + hf * 4 + (r & 3) of block n,

@@ -651,15 +651,18 @@ def moe_router(x, router: torch.Tensor, top: int):
 
 # Mean rows per expert up to which the kernels without a sort, and tiles of 64
 # and 128 rows are taken (and 256 beyond).  64 and 128 leave room for the spread
-# of the counts: a few rows more and an expert's weights are read twice.  us on
-# an MI355X without a sort, and in tiles of 64, 128, 256
-#   8 experts of 14336 x 4096   1 row 336 398, 4 rows 481 492, 5 531 508, 48 -
-#     543 589 732, 64 - 665 594 728, 96 - 798 601 762, 150 - 1118 937 729
-#   16 of 2048 x 4096           1 row 107 132, 4 rows 151 173, 6 162 174, 16 -
-#     202 207 230
-#   32 of 1024 x 2048           2 rows 68 81, 5 84 90, 8 97 92, 64 - 119 118 137
-#   64 of 1024 x 2048           3 rows 141 166, 4.5 159 169, 6 174 171
-MOE_ROWS, MOE_ROWS_64, MOE_ROWS_128 = 5, 52, 112
+# of the counts: a few rows more than a tile and an expert's weights are read
+# twice, by workgroups that share their compute units with others.  us on an
+# MI355X without a sort, and in tiles of 64, 128, 256, sort included
+#   8 experts of 14336 x 4096   1 row 357 383, 2 rows 420 435, 3 490 471, 5 526
+#     470, 48 - 487 507 626 (52, one of 66 rows, - 604 510), 100 - 783 555 698,
+#     125 - 968 782 719
+#   16 of 2048 x 4096           1 row 109 119, 3 rows 145 148, 5 155 149, 50 -
+#     158 161 206, 125 - 249 232 222
+#   32 of 1024 x 2048           1 row 53 61, 3 rows 75 78, 5 85 80, 37 - 82 90
+#     118, 62 - 107 96 120, 125 - 137 132 129
+#   64 of 1024 x 2048           1 row 101 104, 3 rows 141 142, 4.5 159 143
+MOE_ROWS, MOE_ROWS_64, MOE_ROWS_128 = 2.9, 44, 112
 
 
 def _moe_tile(T: int, K: int, E: int, least: int) -> int:

@@ -68,9 +68,10 @@ def test_experts_around_the_rule(tokens, experts, top, width, inner):
     (1, 4, 2, 128, 128), (5, 1, 1, 128, 256), (17, 4, 1, 256, 128),
     (33, 7, 1, 384, 640), (64, 64, 5, 128, 128), (65, 13, 1, 128, 384)])
 @pytest.mark.parametrize("kind", ["spread", "one", "gaps"])
-def test_few_choices(tokens, experts, top, width, inner, kind):
+def test_few_choices(tokens, experts, top, width, inner, kind, monkeypatch):
     """Choices that are named where they are, more than 16 or 64 of one expert,
     and places without a choice."""
+    monkeypatch.setattr(ops, "MOE_ROWS", 5)     # more than the rule gives it
     assert ops._moe_tile(tokens, top, experts, 16) == 16
     g = torch.Generator().manual_seed(tokens)
     rand = lambda *s: torch.randn(*s, generator=g)
