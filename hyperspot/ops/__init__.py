@@ -274,11 +274,31 @@ def _rows_gemm(x: torch.Tensor, w: torch.Tensor) -> bool:
 MOST_ROWS = 512         # of a product that a kernel here takes
 
 
+def _wave_gemm(M: int, N: int, K: int):
+    """Tiles of 64 rows where those of 64 or 128 outputs are one workgroup a
+    compute unit, or nearly: N of 11264 to 16384 and of 22528 to 32768.  Against
+    the kernel of few rows and the library, us: 32768 x 4096 1 row 47.1 45.3, 16
+    52.6 46.7, 24 66 46, 64 62 48; 32768 x 2048 1 row 25.7 25.9, 32 31 26, 64 35
+    26.5; 14272 x 3072 23 rows 19.9 19.2; 23744 x 4096 39 rows 45 36; 26112 x 3072
+    6 rows 37 31; 11264 x 512 39 rows 7.9 5.7.  Beyond 64 rows the library is as
+    fast (96 of 32768 x 4096 63 60, 128 64 65), and so it is with fewer or more
+    tiles (10 of 7808 x 4096 17 21; 2 of 39104 x 4096 59 64)."""
+    if not 1 <= M <= 64 or K % 128 or N % 4:
+        return None
+    for bn in (64, 128):
+        if 176 <= -(-N // bn) <= 256:
+            return 64, bn, 1
+    return None
+
+
 @lru_cache(maxsize=1 << 14)
 def _route(M: int, N: int, K: int, parts: bool):
     """How x w^T of these sizes is formed: "rows", (rows, outputs of a tile, parts
     of K) or None, the library.  Kept, for the rules take as long as a launch: a
     step of small prompts, which is not captured, waits for the host."""
+    wave = _wave_gemm(M, N, K)
+    if wave is not None:
+        return wave
     if _rows_gemm_sizes(M, N, K) and _native().gemm_rows_fits(M, K):
         return "rows"
     return _less_padding(M, _split_gemm(M, N, K)) \
@@ -374,7 +394,8 @@ def _less_padding(M: int, split):
 
 def _summed_gemm(M: int, N: int, K: int):
     """As _split_gemm, for more sizes, where the norm adds up the parts.  Measured
-    with the norm: 33 to 128 rows with K of 1024 to 4096 and less than 14M
+    with the norm: up to 16 rows of long K (1 row of 4096 x 14336 27.4 26.7, 8
+    28.6 27.1, 16 29.6 27.2; of 2048 x 7168 13.0 11.1, 13.1 11.6, 13.5 11.7); 33 to 128 rows with K of 1024 to 4096 and less than 14M
     weights, 0.87 of the library's time on average in 65 sizes and none slower by
     3 % (48 rows of 2048 x 2048 11.0 8.9 us, 64 of 4096 x 2560 13.4 12.5, 78 of
     3200 x 3584 23 14); 257 to 512 rows with K from 5120 on, or 4096 in tiles of
@@ -383,6 +404,9 @@ def _summed_gemm(M: int, N: int, K: int):
     are even (452 of 5504 x 8192 65 70, 379 of 7168 x 14336 119 116)."""
     if K % 128 or N % 8 or N > 8192:
         return None
+    if M <= 16 and K >= 5120 and N * K >= 14 << 20:
+        split = min(6, 256 // -(-N // 64), K // 1024)
+        return (64, 64, split) if split > 2 else None
     if 32 < M <= 128 and 1024 <= K <= 4096 and 1 << 20 <= N * K < 14 << 20:
         split = min(8, 256 // (-(-M // 64) * -(-N // 64)), K // 512)
         return (64, 64, split) if split > 1 else None
@@ -438,24 +462,26 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 def _gated_tile(M: int, N: int, K: int):
     """(rows, rows of w of a tile) where csrc/gemm_split.hip forms silu(gate) *
     up of x w^T faster than a product and an activation, else None: the smallest
-    tiles that are one workgroup a compute unit or less.  Measured at 17 to 256
+    tiles that are one workgroup a compute unit or less.  Measured at 1 to 256
     rows, N of 2048 to 57344 and K of 512 to 8192: 0.78 of both on average where
-    it is taken (us: 28672 x 4096 17 rows 47 41, 32 58 41, 64 57 41, 128 59 48;
-    14336 x 2048 32 rows 19 13, 64 20 15, 128 24 18, 192 30 21, 256 32 23).
-    More tiles take a second wave (192 rows of 28672 x 4096 67 73) but for up to
+    it is taken (us: 28672 x 4096 1 row 43.4 41.4, 8 rows 48 41, 17 47 41, 32 58
+    41, 64 57 41, 128 59 48; 14336 x 2048 1 row 15.1 13.4, 16 18 13, 32 19 13,
+    64 20 15, 128 24 18, 192 30 21, 256 32 23).
+    More tiles take a second wave (192 rows of 28672 x 4096 67 73) but for 17 to
     64 rows, where the library has no better tile (29 rows of 38400 x 6144 124
-    96).  Few tiles with long rows leave the chip idle (23 rows of 2048 x 3072
+    96; 6 of 52736 x 1536 36 38).  Few tiles with long rows leave the chip idle (23 rows of 2048 x 3072
     10 13), and more than 64 rows of more than 4096 columns gain nothing (71 of
     6144 x 5120 22.5 22.8, 119 of 5632 x 5120 25 27)."""
-    if not 16 < M <= 256 or K % 128 or N % 16 or M > 64 and K > 4096:
+    if not 1 <= M <= 256 or K % 128 or N % 16 or M > 64 and K > 4096:
         return None
     for bm, bn in ((64, 64), (64, 128)) if M <= 64 \
             else ((64, 64), (128, 64), (128, 128)):
         tiles = -(-M // bm) * -(-N // bn)
         if tiles <= 256:
-            least = 128 if K > 2048 else 64 if K > 1024 else 40
+            least = 128 if K > 2048 else 72 if M <= 16 else \
+                64 if K > 1024 else 40
             return (bm, bn) if tiles >= least else None
-    return (64, 64) if M <= 64 else None
+    return (64, 64) if 16 < M <= 64 else None
 
 
 def gated_linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
