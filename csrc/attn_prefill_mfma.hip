@@ -28,7 +28,9 @@
 //
 // Within a tile the operands of 8 products are loaded ahead of them, and the next
 // 16 tokens' weights are formed between the products of the last 16, not before
-// them.  Long prompts are bound by power: with zeros as data 8192 cached tokens
+// them.  Tiles come by buffer loads: beside loads from a global address to LDS
+// the compiler waited for all LDS reads wherever it needed the oldest (8192 rows
+// 613 -> 602 us, 7808 after 8192 cached tokens 2560 -> 2500).  Long prompts are bound by power: with zeros as data 8192 cached tokens
 // and 7808 rows take 1.94 ms, with normal values 2.57.
 //
 // 32 heads, 8 kv heads: a prompt of 8192 tokens 734 us (749 TFLOP/s) where
@@ -46,7 +48,7 @@
 // float; two were off by up to 2^-20 of what they weigh (and took 2.07 ms).
 #include <float.h>
 
-#include "common.h"
+#include "tile_loop.h"
 
 namespace {
 
@@ -77,13 +79,6 @@ struct Prefill {
 };
 
 DEV float exp2_fast(float x) { return __builtin_amdgcn_exp2f(x); }
-
-// 16 bytes a lane, to the wave's LDS address + lane * 16
-DEV void to_lds16(const void* g, void* l) {
-  __builtin_amdgcn_global_load_lds(
-      (const __attribute__((address_space(1))) unsigned*)g,
-      (__attribute__((address_space(3))) unsigned*)l, 16, 0, 0);
-}
 
 // four rows of one column: in every 16 lanes, lane i passes the address of
 // row i / 4, columns 4 (i % 4), and receives column i
@@ -184,10 +179,8 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(Prefill a) {
       ids[j] = bt[min(kv0 / PAGE + j, last_page)];
   };
   const int lr = 4 * wid + (lane >> 4);          // row within 16
-  const int kc = ((lane & 15) ^ lr) * 8;         // its column of K, and of V
-  const int vc = ((lane & 15) ^ (lane >> 4) << 2) * 8;
-  const bf16* k0 = a.k + g * HD + kc;            // ROWS
-  const bf16* v0 = a.v + g * HD + vc;
+  const int kc = ((lane & 15) ^ lr) * 16;        // its byte of K, and of V
+  const int vc = ((lane & 15) ^ (lane >> 4) << 2) * 16;
   uint4 raw[4];                                  // PAGES8: 32 bytes each
   auto fetch = [&](int kv0, int buf) {
     if constexpr (SRC == PAGES8) {
@@ -204,20 +197,24 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(Prefill a) {
         raw[2 + i] = reinterpret_cast<const uint4*>(vp)[i];
       }
     } else {
+      const RowLoads k_rows(a.k + (t0 + kv0) * a.sk + g * HD);
+      const RowLoads v_rows(a.v + (t0 + kv0) * a.sv + g * HD);
       #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const bf16 *kp, *vp;
+        char* kl = reinterpret_cast<char*>(
+            &lds[buf][0][(16 * j + 4 * wid) * HD]);
+        char* vl = reinterpret_cast<char*>(
+            &lds[buf][1][(16 * j + 4 * wid) * HD]);
         if constexpr (SRC == ROWS) {
-          const unsigned r = t0 + min(kv0 + 16 * j + lr, n - 1);
-          kp = k0 + (unsigned long)r * (unsigned)a.sk;
-          vp = v0 + (unsigned long)r * (unsigned)a.sv;
+          const unsigned r = min(16 * j + lr, n - 1 - kv0);
+          k_rows.to_lds(kl, r * (unsigned)a.sk * 2 + kc, 0);
+          v_rows.to_lds(vl, r * (unsigned)a.sv * 2 + vc, 0);
         } else {
-          const long at = (((long)ids[j] * a.G + g) * PAGE + lr) * HD;
-          kp = a.k + at + kc;
-          vp = a.v + at + vc;
+          const int id = __builtin_amdgcn_readfirstlane(ids[j]);
+          const long at = ((long)id * a.G + g) * (PAGE * HD);
+          RowLoads(a.k + at).to_lds(kl, lr * (HD * 2) + kc, 0);
+          RowLoads(a.v + at).to_lds(vl, lr * (HD * 2) + vc, 0);
         }
-        to_lds16(kp, &lds[buf][0][(16 * j + 4 * wid) * HD]);
-        to_lds16(vp, &lds[buf][1][(16 * j + 4 * wid) * HD]);
       }
     }
   };

@@ -373,10 +373,11 @@ void attn_prefill_mfma(torch::Tensor out, torch::Tensor q, torch::Tensor k,
   const int H = (int)q.size(1), D = (int)q.size(2);
   const int KV = (int)k.size(1);
   TORCH_CHECK(KV > 0 && H % KV == 0, "GQA group");
-  // keys and values are read 16 bytes at a time straight into LDS
+  // keys and values are read 16 bytes at a time straight into LDS, the rows of a
+  // tile by 32 bits of offset
   auto aligned = [](const torch::Tensor& t) {
     return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0 &&
-                   t.stride(0) % 8 == 0
+                   t.stride(0) % 8 == 0 && t.stride(0) < (1l << 25)
                ? t : t.clone(at::MemoryFormat::Contiguous);
   };
   k = aligned(k);

@@ -179,6 +179,26 @@ def test_attn_prefill_mfma_strided_views():
     assert torch.allclose(out.float().cpu(), ref, atol=2.5e-2, rtol=2.5e-2)
 
 
+@pytest.mark.gpu
+def test_attn_prefill_mfma_rows_far_apart():
+    """Rows of keys and values that 32 bits of offset do not reach."""
+    far = 1 << 25
+    qkv = torch.randn(70, 4, 128, device=DEV, dtype=torch.bfloat16)
+    wide = torch.empty(69 * far + 256, device=DEV, dtype=torch.bfloat16)
+    k, v = (wide[i * 128:].as_strided((70, 1, 128), (far, 128, 1))
+            for i in range(2))
+    k.copy_(qkv[:, :1])
+    v.copy_(qkv[:, 1:2])
+    start = torch.tensor([0, 70], dtype=torch.int32, device=DEV)
+    outs = []
+    for kv in ((k, v), (k.contiguous(), v.contiguous())):
+        out = torch.empty(70, 2, 128, device=DEV, dtype=torch.bfloat16)
+        ops._native().attn_prefill_mfma(out, qkv[:, 2:], *kv, start, 70, 0.09)
+        outs.append(out)
+    assert torch.equal(*outs)
+
+
+
 def test_silu_mul():
     x = _randn_bf16(65, 2 * 1024)
     out = ops.silu_mul(x)
