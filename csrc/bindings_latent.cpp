@@ -53,6 +53,9 @@ void launch_experts_route(float*, int*, const float*, int, int, int, bool,
                           bool, int, const float*, hipStream_t);
 void launch_experts_router(float*, int*, const void*, const float*,
                            const bf16*, long, int, int, int, hipStream_t);
+void launch_norm_router(float*, int*, bf16*, const bf16*, const float*, int,
+                        bf16*, const bf16*, float, const bf16*, long, int, int,
+                        int, hipStream_t);
 void launch_experts_tiles(bool, bf16*, const void*, const void*, const float*,
                           const float*, const int*, const int*, long, int, int,
                           int, int, int, hipStream_t);
@@ -543,6 +546,39 @@ void experts_router(Tensor weight, Tensor ids, Tensor x, Maybe x_scale,
                         (int)x.size(1), stream());
 }
 
+// out <- rmsnorm(residual + x) * norm, residual that sum, and the choices and
+// weights of out's rows; x bf16 [T, W] or float parts [parts, T, W]
+void norm_router(Tensor weight, Tensor ids, Tensor out, Tensor x,
+                 Tensor residual, Tensor norm, double eps, Tensor router,
+                 long top) {
+  const bool parts = x.dim() == 3;
+  check(x, parts ? torch::kFloat : torch::kBFloat16, "x");
+  check(out, torch::kBFloat16, "out");
+  check(residual, torch::kBFloat16, "residual");
+  check(norm, torch::kBFloat16, "norm");
+  check(router, torch::kBFloat16, "router");
+  TORCH_CHECK(residual.dim() == 2 && router.dim() == 2, "norm_router: shape");
+  const long T = residual.size(0), W = residual.size(1), E = router.size(0);
+  TORCH_CHECK(W % 8 == 0 && W >= 8 && W <= 8192 && router.size(1) == W &&
+                  norm.numel() == W && out.numel() == T * W &&
+                  (parts ? x.size(0) >= 2 && x.size(0) <= 8 &&
+                               x.size(1) == T && x.size(2) == W
+                         : x.numel() == T * W), "norm_router: shape");
+  TORCH_CHECK(E >= 1 && E <= 64 && top >= 1 && top <= E && T < (1l << 31),
+              "norm_router: experts");
+  for (const auto& t : {x, out, residual, norm, router})
+    TORCH_CHECK(reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0,
+                "norm_router: alignment");
+  check_param(weight, T * top, "weight");
+  check_ints(ids, T * top, "ids");
+  launch_norm_router(ptr<float>(weight), ids.data_ptr<int>(), ptr<bf16>(out),
+                     parts ? nullptr : ptr<bf16>(x),
+                     parts ? ptr<float>(x) : nullptr,
+                     parts ? (int)x.size(0) : 0, ptr<bf16>(residual),
+                     ptr<bf16>(norm), (float)eps, ptr<bf16>(router), T, (int)E,
+                     (int)top, (int)W, stream());
+}
+
 void check_sorted(const Tensor& order, const Tensor& expert,
                   const Tensor& place, long choices, long kinds, long bm) {
   const long tiles = expert.numel();
@@ -697,6 +733,7 @@ void register_latent(pybind11::module_& m) {
         py::arg("logits"), py::arg("E"), py::arg("top"),
         py::arg("correction") = py::none(), py::arg("identity") = 0);
   m.def("experts_router", &experts_router);
+  m.def("norm_router", &norm_router);
   m.def("experts_tiles", &experts_tiles);
   m.def("experts_sort", &experts_sort);
   m.def("experts_route_sort", &experts_route_sort);

@@ -178,12 +178,16 @@ class DecoderLayer(nn.Module):
         return self.mlp(h), residual
 
     def _summands(self, *args):
-        h, residual = self._hidden(*args)
+        h, residual = self._hidden(*args, routed=True)
         return summands(self.mlp, h), residual
 
     def _hidden(self, x, residual: Optional[torch.Tensor], meta: ForwardMeta,
-                kv_cache: torch.Tensor, cos_sin: torch.Tensor):
-        """The input of the feed-forward block, and the residual stream."""
+                kv_cache: torch.Tensor, cos_sin: torch.Tensor,
+                routed: bool = False):
+        """The input of the feed-forward block, and the residual stream.
+        routed: with the experts that its rows choose, where the block's own
+        class has a router for the norm (`_norm_router`) and nothing else sees
+        its call."""
         # fp8 GPU path: the norm kernels emit per-token-scaled fp8 directly
         # (csrc/quant.hip), so GEMM inputs never take an extra quant pass.
         fp8 = self.attn.qkv.quant == "fp8" \
@@ -202,6 +206,12 @@ class DecoderLayer(nn.Module):
             h, residual = ops.fused_add_rmsnorm(x, residual,
                                                 self.input_norm_w, self.eps)
         h = summands(self.attn, h, meta, kv_cache, cos_sin)
+        find = vars(type(self.mlp)).get("_norm_router") if routed else None
+        router = None if find is None or watched(self.mlp) \
+            else find(self.mlp, h, residual, self.post_norm_w)
+        if router is not None:
+            return ops.fused_add_rmsnorm_route(h, residual, self.post_norm_w,
+                                               self.eps, *router)
         if fp8:
             h, residual = ops.fused_add_rmsnorm_q(h, residual,
                                                   self.post_norm_w, self.eps)

@@ -21,7 +21,8 @@ from hyperspot import ops
 from hyperspot.engine.config import ModelSpec
 from hyperspot.models.llama import DecoderLayer, LlamaForCausalLM
 from hyperspot.parallel.layers import (_init_weight, _QUANT_MODE,
-                                       quantize_weight_fp8, summands)
+                                       quantize_weight_fp8, summands,
+                                       watched)
 from hyperspot.parallel.state import get_ep_group, get_ep_rank, get_ep_size
 
 
@@ -122,6 +123,8 @@ class MixtralMoE(nn.Module):
     def _summands(self, x):
         """The experts' outputs before their sum, where all of them are here in
         16 bits and the norm takes their width."""
+        if isinstance(x, ops.Routed):
+            return ops.moe_choices(x.data, self.w13, self.w2, x.weights, x.ids)
         if not isinstance(x, torch.Tensor) or not x.is_cuda \
                 or x.dtype != torch.bfloat16 or x.shape[0] == 0 \
                 or not 0 < x.shape[1] <= 8192 or self.quant is not None \
@@ -130,6 +133,23 @@ class MixtralMoE(nn.Module):
         weights, ids = self._route_gpu(x)
         return ops.moe_choices(x, self.w13, self.w2, weights,
                                ids.to(torch.int32))
+
+    def _norm_router(self, h, residual: torch.Tensor, norm: torch.Tensor):
+        """(router, choices) for the norm that forms this block's input from h,
+        a tensor or ops.Parts, where `_summands` would take it."""
+        data = h.data if isinstance(h, ops.Parts) else h
+        if self.quant is not None or get_ep_size() > 1 \
+                or not isinstance(data, torch.Tensor) \
+                or residual.dtype != torch.bfloat16 \
+                or norm.dtype != torch.bfloat16 \
+                or not 0 < residual.shape[1] <= 8192 or not len(residual) \
+                or not self._fused_router(residual) \
+                or not ops.unrecorded(data, norm) \
+                or isinstance(h, torch.Tensor) and h.dtype != torch.bfloat16 \
+                or not all(t.is_contiguous() and t.data_ptr() % 16 == 0
+                           for t in (data, residual, norm, self.router)):
+            return None
+        return self.router, self.top_k
 
     def _fused_router(self, x: torch.Tensor) -> bool:
         return x.is_cuda and ops.have_native() and x.is_contiguous() \
@@ -347,6 +367,11 @@ class _MoEAdapter(nn.Module):
 
     def _summands(self, x):
         return summands(self.moe, x)
+
+    def _norm_router(self, *args):
+        own = vars(type(self.moe)).get("_norm_router")
+        return None if own is None or watched(self.moe) \
+            else own(self.moe, *args)
 
 
 class MixtralForCausalLM(LlamaForCausalLM):

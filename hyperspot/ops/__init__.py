@@ -55,6 +55,14 @@ class Choices(NamedTuple):
     weights: torch.Tensor        # [T, K] float
 
 
+class Routed(NamedTuple):
+    """Rows with the experts that they choose."""
+
+    data: torch.Tensor           # [T, W]
+    weights: torch.Tensor        # [T, K] float
+    ids: torch.Tensor            # [T, K] int32
+
+
 def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
     if x.is_cuda:
         out = torch.empty_like(x)
@@ -83,6 +91,20 @@ def fused_add_rmsnorm(x: torch.Tensor, residual: torch.Tensor,
         return x, residual
     out, res = torch_ref.fused_add_rmsnorm(x, residual, weight, eps)
     return out, res
+
+
+def fused_add_rmsnorm_route(x, residual: torch.Tensor, weight: torch.Tensor,
+                            eps: float, router: torch.Tensor, top: int):
+    """fused_add_rmsnorm, x a tensor or Parts, and moe_router in one kernel:
+    (Routed, residual); residual is changed in place.  GPU."""
+    data = x.data if isinstance(x, Parts) else x
+    T, W = residual.shape
+    out = torch.empty_like(residual)
+    share = torch.empty(T, top, dtype=torch.float32, device=residual.device)
+    ids = torch.empty(T, top, dtype=torch.int32, device=residual.device)
+    _native().norm_router(share, ids, out, data, residual, weight, eps, router,
+                          top)
+    return Routed(out, share, ids), residual
 
 
 def rope_kv_append(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,

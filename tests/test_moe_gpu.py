@@ -185,3 +185,52 @@ def test_rows_beyond_32_bits():
     want = few.data[few.place[:, 0].long()].float()
     # both round the inner values and the results to bf16
     assert (got.float() - want).norm() <= 2.0 ** -7 * want.norm()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tokens,experts,top,width,parts", [
+    (1, 1, 1, 8, 0), (3, 16, 2, 2048, 0), (5, 17, 3, 2056, 2), (64, 33, 4, 4096, 8),
+    (17, 64, 8, 8192, 3), (200, 8, 2, 4104, 0)])
+def test_norm_and_router(tokens, experts, top, width, parts):
+    """As the norm, then the router of what it gives."""
+    g = torch.Generator().manual_seed(tokens)
+    rand = lambda *s: torch.randn(*s, generator=g).to(DEV)
+    x = ops.Parts(rand(parts, tokens, width)) if parts \
+        else rand(tokens, width).bfloat16()
+    res, norm = rand(tokens, width).bfloat16(), rand(width).bfloat16()
+    router = (rand(experts, width) * width ** -0.5).bfloat16()
+    got, got_res = ops.fused_add_rmsnorm_route(x, res.clone(), norm, 1e-5,
+                                               router, top)
+    h, want_res = ops.fused_add_rmsnorm(x if parts else x.clone(), res.clone(),
+                                        norm, 1e-5)
+    assert torch.equal(got_res, want_res)
+    # the squares are added in another order: the last bit of a row's scale
+    assert ((got.data.float() - h.float()).abs()
+            <= h.float().abs() * 2.0 ** -7).all()
+    # what the router makes of those rows is what it makes of them by itself
+    weights, ids = ops.moe_router(got.data, router, top)
+    assert torch.equal(got.ids, ids) and torch.equal(got.weights, weights)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("path", ["", "moe"])
+def test_watched_experts_get_tensors(path):
+    from hyperspot.engine.config import ModelSpec
+    from hyperspot.models.llama import DecoderLayer
+    from hyperspot.models.mixtral import _MoEAdapter
+    from hyperspot.parallel import layers
+    layers.set_init_device(DEV)
+    spec = ModelSpec("t", 256, 1, 2, 1, 128, 256, 32, num_experts=4,
+                     num_experts_per_tok=2)
+    layer = DecoderLayer(spec, 0, torch.bfloat16, _MoEAdapter).to(DEV)
+    layers.set_init_device("cpu")
+    x = torch.randn(6, 256, device=DEV).bfloat16()
+    routed = []
+    take = layer.mlp.moe._norm_router(x, x.clone(), layer.post_norm_w)
+    assert take is not None and take[1] == 2
+    layer.mlp.get_submodule(path).register_forward_hook(
+        lambda m, a, y: routed.append(type(a[0])))
+    assert layer.mlp._norm_router(x, x.clone(), layer.post_norm_w) is None \
+        if path else layers.watched(layer.mlp)
+    layer.mlp(x)
+    assert routed == [torch.Tensor]
