@@ -266,24 +266,32 @@ def unrecorded(*tensors: torch.Tensor) -> bool:
     """Whether a kernel may take the place of torch's operation on these: no
     gradient or tangent is formed, and no subclass, transform, trace or mode
     has to see the operation."""
-    return not torch.compiler.is_compiling() \
-        and all(type(t) in (torch.Tensor, torch.nn.Parameter)
-                for t in tensors) \
-        and not (torch.is_grad_enabled()
-                 and any(t.requires_grad for t in tensors)) \
-        and torch.autograd.forward_ad._current_level < 0 \
-        and torch._C._functorch.peek_interpreter_stack() is None \
-        and torch._C._len_torch_dispatch_stack() == 0 \
-        and torch._C._get_tracing_state() is None \
-        and not torch.is_autocast_enabled("cuda")
+    if torch.compiler.is_compiling() or _forward_ad._current_level >= 0 \
+            or _stack() is not None or _modes() or _tracing() is not None \
+            or torch.is_autocast_enabled("cuda"):
+        return False
+    grad = torch.is_grad_enabled()
+    for t in tensors:       # a loop: every product of a step comes here
+        if type(t) not in _PLAIN or grad and t.requires_grad:
+            return False
+    return True
+
+
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
+_forward_ad = torch.autograd.forward_ad
+_stack = torch._C._functorch.peek_interpreter_stack
+_modes = torch._C._len_torch_dispatch_stack
+_tracing = torch._C._get_tracing_state
 
 
 def _plain_bf16(x: torch.Tensor, w: torch.Tensor) -> bool:
     """Matrices whose rows the kernels can load 16 bytes at a time."""
-    return x.is_cuda and x.dtype == w.dtype == torch.bfloat16 \
-        and unrecorded(x, w) and all(
-            t.dim() == 2 and t.stride(1) == 1 and t.stride(0) % 8 == 0
-            and t.data_ptr() % 16 == 0 for t in (x, w))
+    if not (x.is_cuda and x.dtype == w.dtype == torch.bfloat16
+            and unrecorded(x, w) and x.dim() == w.dim() == 2):
+        return False
+    (a, b), (c, d) = x.stride(), w.stride()
+    return b == 1 and d == 1 and a % 8 == 0 and c % 8 == 0 \
+        and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
 
 
 def _rows_gemm(x: torch.Tensor, w: torch.Tensor) -> bool:
@@ -575,7 +583,7 @@ def _tiled_q(x: "QTensor", w: torch.Tensor, scale: torch.Tensor, parts: bool):
     """The tile of _tiles_q, or None."""
     d, s = x
     if not (d.is_cuda and unrecorded(d, w, s, scale)
-            and d.dim() == w.dim() == 2):
+            and d.dim() == w.dim() == 2) or d.shape[0] > 128:
         return None
     tile = _tiles_q(d.shape[0], *w.shape, parts)
     if tile is None or not (
