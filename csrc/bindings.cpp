@@ -512,7 +512,7 @@ void gemm_split(c10::optional<torch::Tensor> out, torch::Tensor x,
   TORCH_CHECK(N % 4 == 0 && K % chunk == 0 && K >= chunk && M < (1l << 20) &&
                   K < (1l << 24) && N < (1l << 24) && aligned(x) && aligned(w),
               "gemm_split: sizes");
-  TORCH_CHECK(fp8 ? bm == 64 && (bn == 32 || bn == 64)
+  TORCH_CHECK(fp8 ? bm == 64 && (bn == 32 || bn == 64 || bn == 128)
                   : ((bm == 64 || bm == 128) && (bn == 64 || bn == 128)) ||
                         (bm == 256 && bn == 128), "gemm_split: tile");
   if (gated)      // 32 bits of offset reach the up rows

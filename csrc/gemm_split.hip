@@ -22,7 +22,8 @@
 //   rows 47 41, 64 57 41, 128 59 48; 14336 x 2048 32 rows 19 13, 256 32 23
 // e4m3, with the norm that adds up the parts: 4096 x 14336 16 rows 27 19, 64 31
 // 21, 128 44 28; 4096 x 4096 16 rows 15 12, 128 18 15; without: 28672 x 4096 16
-// rows 34 24, 64 30.3 29.1; 14336 x 2048 64 rows 14 11; 6144 x 4096 13.7 12.3.
+// rows 34 24, 64 31 26 (29 in tiles of 64 x 64, of which 448 are not one wave);
+// 14336 x 2048 64 rows 14 11; 6144 x 4096 13.7 12.3; 3072 x 2048 9.1 6.4.
 // What bounds it: w from memory (5 TB/s with 16 rows), then the bytes in flight.
 #include "tile_loop.h"
 
@@ -181,8 +182,8 @@ __global__ __launch_bounds__(256) void gemm_sum_kernel(
 }  // namespace
 
 // Tiles of bm rows of x by bn of w: 64 x 64, 64 x 128, 128 x 64, 128 x 128, 256 x
-// 128; with scales x and w are e4m3, in tiles of 64 x 32 or 64 x 64.  out
-// contiguous; rows of K of 256 bytes, N a multiple of 4; rows of x and w 16-byte
+// 128; with scales x and w are e4m3, in tiles of 64 x 32, 64 x 64 or 64 x 128.
+// out contiguous; rows of K of 256 bytes, N a multiple of 4; rows of x and w 16-byte
 // aligned; splits 1 to 8, at most one a 256 bytes, part with more than one.
 // Without out the parts are left for the norm that adds them up.  gated, of
 // bfloat16 without parts: out = silu(gate) * up of the halves of w, whose rows
@@ -215,6 +216,8 @@ void launch_gemm_split(bf16* out, float* part, const void* x, const void* w,
     // two workgroups a unit, with half the ring each, where there are as many
     if (bn == 32)
       RUN(64, 32, 2, 1, 3, 2, true, false)
+    else if (bn == 128)
+      RUN(64, 128, 2, 2, 3, 2, true, false)
     else if ((long)((M + 63) / 64) * ((N + 63) / 64) * splits > 256)
       RUN(64, 64, 2, 2, 2, 2, true, false)
     else

@@ -547,14 +547,19 @@ def _tiles_q(M: int, N: int, K: int, parts: bool):
     Measured at 1 to 128 rows, N of 1024 to 40000 and K of 1024 to 14336 in 400
     random sizes: 0.8 of the library's time on average, and more than 3 % slower
     at 3 of 100.  Tiles of 64 x 64 that fill three quarters of the compute
-    units need no parts (64 rows of 28672 x 4096 30.3 -> 29.1 us, 16 33.8 ->
-    24.5; 14336 x 2048 14.3 -> 11.0); with K beyond 4096 the library catches up
-    from 17 rows on (25 rows of 27680 x 6144 34.7 35.8, 6 41.9 29.7), with more
-    than 32768 outputs for any (4 rows of 35424 x 6144 47 57).  Fewer tiles are
+    units need no parts (16 rows of 28672 x 4096 33.8 -> 24.5 us, 64 of 14336 x
+    2048 14.3 -> 11.0), and more than one wave of them are one wave of twice the
+    width (64 rows of 28672 x 4096 31.1 -> 25.7, 64 wide 28.8; 16 of 21184 x 4096
+    28.9 20.4 21.7), but not with a second wave that is nearly full and few rows
+    (32 of 28672 x 4096 25.8 and 25.0), or short rows (64 of 23232 x 1024 11.1
+    10.9).  With K beyond 4096 in tiles of 64, beyond 6144 in wider ones, the
+    library catches up from 17 rows on (20 rows of 12768 x 6144 18.1 18.0; 64 of
+    19936 x 6144 34.0 34.4 wide, 48 of 24336 47.7 33.3), with more than 32768
+    outputs for any (16 rows of 35312 x 6144 48 57).  Fewer tiles are
     divided into parts of 1365 columns and more, about one workgroup a unit (64
     rows of 4096 x 14336 with the norm 30.6 -> 21.5, of 2048 x 7168 16.3 ->
     12.8), or made half as wide (6144 x 4096 13.7 -> 12.3, 3072 x 2048 9.1 ->
-    7.6).  Where another kernel adds up the parts they gain with 8192 columns,
+    6.4).  Where another kernel adds up the parts they gain with 8192 columns,
     or with few rows (1 of 3600 x 5120 14.0 -> 9.2; 21 of 6032 x 5120 11.7 13.0).
     Beyond 64 rows half as many tiles lie beside each other: long rows only with
     the norm (128 of 4096 x 14336 44 -> 28), 2048 x 7168 is even (14.0 13.7).
@@ -564,8 +569,11 @@ def _tiles_q(M: int, N: int, K: int, parts: bool):
     tiles = -(-M // 64) * -(-N // 64)
     few = M <= 16
     if tiles >= 192:
-        return (64, 64, 1) if N <= (32768 if M <= 64 else 20480) and (
-            few or K <= 2048 or K <= 4096 and (M <= 64 or N <= 8192)) else None
+        wide = 256 < tiles <= 512 and K >= 2048 and (tiles <= 384 or M > 32)
+        return (64, 128 if wide else 64, 1) \
+            if N <= (32768 if M <= 64 else 20480) and (
+                few or K <= 2048 or K <= 4096 and (M <= 64 or N <= 8192)
+                or wide and M <= 64 and K <= 6144) else None
     split = min(8, max(2, K // 1365), 256 // tiles)
     if M > 64 and K > 4096 and (K < 8192 or split == 1 or not parts):
         return None

@@ -30,7 +30,7 @@ def _check(out, q, w, ws):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("bm,bn", [(64, 32), (64, 64)])
+@pytest.mark.parametrize("bm,bn", [(64, 32), (64, 64), (64, 128)])
 @pytest.mark.parametrize("M,N,K,parts", [
     (1, 4, 256, 1), (31, 60, 512, 2), (64, 64, 768, 3), (65, 132, 1280, 4),
     (128, 64, 2048, 8), (129, 260, 2304, 8), (33, 1028, 1792, 7),
@@ -52,7 +52,8 @@ def test_gemm(M, N, K, parts, bm, bn):
 @pytest.mark.gpu
 @pytest.mark.parametrize("M", [1, 16, 17, 64, 65, 128, 129])
 @pytest.mark.parametrize("N,K", [(4096, 4096), (2048, 7168), (12288, 1024),
-                                 (3600, 5120), (2048, 2048), (4096, 14336)])
+                                 (3600, 5120), (2048, 2048), (4096, 14336),
+                                 (20480, 2048)])
 @pytest.mark.parametrize("parts", [False, True])
 def test_linear_q(M, N, K, parts):
     q, w, ws = _operands(M, N, K)
@@ -99,7 +100,7 @@ def test_rule_stays_in_what_the_kernel_takes():
                         continue
                     taken += 1
                     bm, bn, z = rule
-                    assert (bm, bn) in ((64, 32), (64, 64))
+                    assert (bm, bn) in ((64, 32), (64, 64), (64, 128))
                     assert 1 <= z <= min(8, K // 256)
     assert taken > 100
     assert ops._tiles_q(64, 4096, 4096 + 128, False) is None
