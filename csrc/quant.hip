@@ -1,6 +1,6 @@
 // fp8 (OCP e4m3fn) activation-quant kernels for gfx950.
 //
-// The fp8 GEMM path (torch._scaled_mm -> hipBLASLt fp8 MFMA) needs
+// e4m3 products (csrc/gemm_split.hip for few rows, or the library's) need
 // per-token-scaled fp8 activations; doing amax+scale+cast as separate
 // torch ops costs an extra read+write of every activation and erased the
 // fp8 GEMM win (bench_kernels.py fp8: mm-only 1.7-1.8x faster than bf16,

@@ -2,7 +2,7 @@
 
 Decode steps are captured into hipGraphs per batch-size bucket (torch's CUDA
 graph API is hipGraph on ROCm).  The capture includes the whole transformer
-forward — custom CDNA4 kernels, hipBLASLt GEMMs and (at TP>1) the RCCL
+forward — custom CDNA4 kernels, library GEMMs and (at TP>1) the RCCL
 all-reduces — so steady-state decode replays with one graph launch instead
 of ~1k kernel launches (MI355X boundary cost ≈1.2-1.9 us each, see
 /opt/skills/guides/MI355X_MICROARCH.md 'boundary').

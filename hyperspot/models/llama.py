@@ -6,7 +6,8 @@ Design notes (vs a CUDA port):
   - RoPE + paged-KV append is ONE fused HIP kernel pass (hyperspot.ops)
   - rmsnorm + residual-add fused; SwiGLU fused; attention reads the paged
     cache directly (no gather/cat of past keys)
-  - GEMMs via torch.matmul -> hipBLASLt; everything else hand-written CDNA4
+  - products of many rows through hipBLASLt; those of few rows, and everything
+    else, hand-written CDNA4
 
 Model set and serving contract per the reference's spec-only llm-gateway
 (reference modules/llm-gateway/docs/DESIGN.md; SURVEY.md §2.9 kernel list).

@@ -519,7 +519,8 @@ def gated_linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     plain = _plain_bf16(x, w)
     if plain and x.shape[0] <= MOST_ROWS:
         tile = _gated_tile(x.shape[0], *w.shape)
-        if tile is not None and _near(x, w) and w.numel() < 1 << 31:
+        if tile is not None and _near(x, w) \
+                and w.stride(0) * (w.shape[0] + 256) < 1 << 32:
             out = torch.empty(x.shape[0], w.shape[0] // 2, dtype=x.dtype,
                               device=x.device)
             _native().gemm_split(out, x, w, None, *tile, 1, gated=True)
@@ -532,7 +533,7 @@ class QTensor(NamedTuple):
 
     Produced on GPU by the fused quant kernels (csrc/quant.hip) so fp8
     GEMM inputs never take an extra elementwise pass; consumed by the TP
-    linear layers via torch._scaled_mm (hipBLASLt fp8 MFMA)."""
+    linear layers via linear_q."""
 
     data: torch.Tensor
     scale: torch.Tensor

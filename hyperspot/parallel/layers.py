@@ -1,7 +1,7 @@
 """Tensor-parallel linear layers.
 
-GEMMs go through torch.matmul → hipBLASLt on ROCm (library GEMMs); the
-hand-written kernels cover the fused non-GEMM hot ops (csrc/).  Sharding:
+Products are `ops.linear` and its relatives: of few and of some hundred rows
+the kernels of csrc/, beyond that the library.  Sharding:
 
   - ColumnParallelLinear: weight [out/tp, in], output stays sharded
   - RowParallelLinear:    weight [out, in/tp], all-reduce on the output
@@ -34,10 +34,9 @@ def set_init_device(device) -> None:
 def set_quant_mode(mode) -> None:
     """Weight format for subsequently-constructed linear layers.
 
-    "fp8": per-output-channel float8_e4m3fn weights + fp32 scales; GEMMs run
-    torch._scaled_mm (hipBLASLt fp8 MFMA on gfx950) with per-token dynamic
-    activation scales.  BASELINE config 5 (fp8 checkpoints, halved weight
-    stream).  None: plain bf16.
+    "fp8": per-output-channel float8_e4m3fn weights + fp32 scales; products
+    take per-token dynamic activation scales (`ops.linear_q`).  For fp8
+    checkpoints, and half the weights to read.  None: plain bf16.
     """
     global _QUANT_MODE
     assert mode in (None, "fp8"), mode

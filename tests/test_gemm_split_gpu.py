@@ -116,6 +116,17 @@ def test_gated_linear(M, N, K):
 
 
 @pytest.mark.gpu
+def test_gated_linear_rows_far_apart():
+    """Up rows that 32 bits of offset do not reach from the gate rows."""
+    M, N, K, far = 17, 2560, 256, 1 << 21
+    assert ops._gated_tile(M, N, K) is not None
+    x = torch.randn(M, K, device=DEV).bfloat16()
+    w = torch.empty(N * far, device=DEV, dtype=torch.bfloat16).view(N, far)[:, :K]
+    w.normal_(0, K ** -0.5)
+    assert torch.equal(ops.gated_linear(x, w), ops.silu_mul(ops.linear(x, w)))
+
+
+@pytest.mark.gpu
 def test_watched_products_get_their_calls():
     """A hook on the gate and up product sees it, and may change it."""
     from hyperspot.engine.config import ModelSpec
