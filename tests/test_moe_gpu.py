@@ -234,3 +234,26 @@ def test_watched_experts_get_tensors(path):
         if path else layers.watched(layer.mlp)
     layer.mlp(x)
     assert routed == [torch.Tensor]
+
+
+@pytest.mark.parametrize("width,inner", [(4096, 1024), (1024, 4096)])
+def test_tiles_of_an_expert_together(width, inner):
+    """Experts of 0 to 34 tiles of 256, beside each other up to 32."""
+    counts = [8500, 1, 300, 0, 513, 256]
+    g = torch.Generator(device=DEV).manual_seed(width)
+    new = lambda *s: torch.randn(*s, generator=g, device=DEV).bfloat16()
+    ids = torch.repeat_interleave(torch.arange(6, dtype=torch.int32),
+                                  torch.tensor(counts))
+    ids = ids[torch.randperm(len(ids))].to(DEV)
+    x = new(len(ids), width)
+    w13 = new(6, 2 * inner, width) * width ** -0.5
+    w2 = new(6, width, inner) * inner ** -0.5
+    out = ops.moe_ffn(x, w13, w2, torch.ones(len(ids), 1, device=DEV),
+                      ids[:, None])
+    for e in range(6):
+        mine = ids == e
+        gate, up = (x[mine].float() @ w13[e].float().t()).chunk(2, 1)
+        want = (torch.nn.functional.silu(gate) * up) @ w2[e].float().t()
+        # both round the inner values and the results to bf16
+        assert (out[mine].float() - want).norm(dim=-1).le(
+            2.0 ** -7 * want.norm(dim=-1)).all()
