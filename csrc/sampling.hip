@@ -959,8 +959,8 @@ __global__ __launch_bounds__(NT) void sample_slices_kernel(
     near += __popcll(__ballot((own[q] - mx) * w.hi > -7.f));
   // steps below the largest value, down to where weights are zero
   const float zero = 43.f / w.hi;
-  const float scale = NT / fmaxf(mn >= -FLT_MAX ? fminf(mx - mn, zero) : zero,
-                                 1e-30f);
+  const float range = mn >= -FLT_MAX ? fminf(mx - mn, zero) : zero;
+  const float scale = NT / fmaxf(range, 1e-30f);
   __syncthreads();
   if (lane == 0) atomicAdd(&s.n, (unsigned)near);
   #pragma unroll
@@ -976,7 +976,7 @@ __global__ __launch_bounds__(NT) void sample_slices_kernel(
     if (lane == 63) s.wave_count[wid] = upto;
     if (tid == 0) {
       s.n = 0;
-      s.step = NT;
+      s.step = NT + 1;
     }
     __syncthreads();
     unsigned before = 0;
@@ -985,7 +985,9 @@ __global__ __launch_bounds__(NT) void sample_slices_kernel(
     if (before + upto >= want && before + upto - s.count[tid] < want)
       s.step = tid + 1;
     __syncthreads();
-    const float end = (float)s.step;
+    // NT + 1: fewer units than wanted are in the steps.  Then every value that
+    // has weight may stay, the smallest ones, which no step has, among them.
+    const float end = s.step <= NT || range >= zero ? (float)s.step : INFINITY;
     #pragma unroll
     for (int q = 0; q < UNITS; ++q)
       if ((mx - own[q]) * scale < end) {

@@ -174,6 +174,52 @@ def test_rows_in_slices(vocab, rows):
             assert out[b] == int(row.argmax())
 
 
+def _few_above(kind, vocab):
+    """Rows whose top_k-th largest value is the smallest one, or nearly."""
+    x = torch.full((vocab,), 1.0)
+    if kind == "three":                      # above all others, which are equal
+        x[[vocab // 5, vocab // 2, vocab - 1]] = 2.0
+    elif kind == "tail":                     # smaller values in the last load
+        x[vocab // 3] = 1.5
+        x[vocab - vocab % 8 - 1:] = 0.0
+    elif kind == "masked":                   # and others without weight
+        x[vocab // 4:] = float("-inf")
+        x[: min(9, vocab // 4)] = 2.0
+    elif kind == "steps":                    # more values than are listed below
+        x = (torch.arange(vocab) % 700).float() * -0.01
+    elif kind == "end":                      # one value below all others
+        x[vocab // 3] = 0.0
+    return x
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rows", [4, 1030])
+@pytest.mark.parametrize("vocab", [2, 5, 9, 40, 700, 8191, 8192, 32768, 32773])
+def test_the_smallest_values_may_stay(vocab, rows, dtype):
+    """top_k where fewer values than that are above the smallest one: in slices
+    (4 rows) and without, over uniforms that reach every part of a row."""
+    kinds = ["three", "tail", "masked", "steps", "end"]
+    options = [(1.0, 1.0, 50), (0.7, 1.0, 3), (1.0, 0.6, 50), (2.0, 1.0, 256),
+               (1.0, 1.0, 1), (0.05, 1.0, 200)]
+    x = torch.stack([_few_above(kind, vocab) for kind in kinds]).to(dtype)
+    pick = [(i, o, (n + 0.5) / 8) for i in range(len(kinds))
+            for o in range(len(options)) for n in range(8)]
+    t, p, k = (torch.tensor(c) for c in
+               zip(*(options[o] for _, o, _ in pick)))
+    which = torch.tensor([i for i, _, _ in pick])
+    u = torch.tensor([n for _, _, n in pick])
+    out = torch.cat([
+        ops.sample(*(c.to(DEV) for c in (x[which[a]], t[a], p[a], k[a].int(),
+                                         u[a])))
+        for a in torch.arange(len(pick)).repeat(
+            -(-rows // len(pick))).split(rows)])[:len(pick)].tolist()
+    for b, (i, o, n) in enumerate(pick):
+        if not torch.isfinite(x[i].float()).any():
+            continue
+        ok, _ = _allowed(x[i].float(), *options[o], float(u[b]))
+        assert ok[out[b]], (kinds[i], options[o], out[b], n)
+
+
 def test_one_option_for_all_rows():
     """Options of one element count for every row; top_k of 64 bits."""
     g = torch.Generator().manual_seed(1)
