@@ -1031,14 +1031,14 @@ __global__ __launch_bounds__(NT) void sample_slices_kernel(
   if (tid == 0) out[b] = drawn;
 }
 
-// Slices of a row, 0: none.  As many as give every compute unit a workgroup, if
+// Slices of a row, 0: none (or no rows).  As many as give every compute unit a workgroup, if
 // each has a load for every thread.  Beyond two workgroups a unit the chip is
 // full of whole rows (256 rows of 128256 52 us, in 4 slices 57; of 50257 50 and
 // in 2 slices 50; of 32000 31 and in one 28).
 int sample_slices(long rows, int vocab) {
   const int least = (vocab + HELD * NT * 8 - 1) / (HELD * NT * 8);
   const int most = min(SLICES, max(1, vocab / (NT * 8)));
-  if (least > SLICES || rows * least > 512) return 0;
+  if (rows == 0 || least > SLICES || rows * least > 512) return 0;
   return max(least, min(most, (int)(256 / rows)));
 }
 

@@ -232,6 +232,15 @@ def test_one_option_for_all_rows():
     assert torch.equal(ops.sample(x, *one, k, u), ref)
 
 
+@pytest.mark.parametrize("vocab", [1, 7, 32768, 128256])
+def test_no_rows(vocab):
+    none = torch.empty(0, device=DEV)
+    for dtype in (torch.bfloat16, torch.float32):
+        out = ops.sample(torch.empty(0, vocab, dtype=dtype, device=DEV), none,
+                         none, none.int(), none)
+        assert out.shape == (0,) and out.dtype == torch.long
+
+
 def test_a_vocabulary_beyond_the_kernel():
     v = (1 << 23) + 8
     x = torch.zeros(2, v, device=DEV, dtype=torch.bfloat16)
