@@ -42,10 +42,11 @@ struct Split {
 };
 
 // BM rows of x, BN of w; WM * WN waves have BM / WM by BN / WN.  A stage has
-// KC chunks of 64 columns.
+// KC chunks of 64 columns.  Two waves a SIMD (128 threads are less) keep the
+// sums in vector registers.
 template <int BM, int BN, int WM, int WN, int STAGES, int KC, bool FP8,
           bool GATED>
-__global__ __launch_bounds__(WM * WN * 64, WM * WN < 4 ? 1 : WM * WN / 4)
+__global__ __launch_bounds__(WM * WN * 64, 2)
 void gemm_split_kernel(Split a) {
   using Loop = TileLoop<BM, BN, WM, WN, STAGES, KC, FP8>;
   constexpr int ELEM = FP8 ? 1 : 2;

@@ -139,10 +139,21 @@ struct TileLoop {
       }
       if (live) products(f[1]);
       slot = next;
-      // The last sums are there before they are read.  The compiler's own wait
-      // was found missing on the way out of this loop, where it copies them
-      // from accumulation registers, so this one is inside.
-      if (d + 1 == stages) asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
     }
+    // The last sums are there before anything reads them.  The compiler's own
+    // wait is not there on every way out of the loop: where the first reads were
+    // copies from accumulation registers in a block of their own, the second one
+    // came 6 instructions after the products, which take 11.  As operands before
+    // and after it the sums can pass this wait in neither direction; in vector
+    // registers (two waves a SIMD or more) there are no copies.
+    in_order();
+    asm volatile("s_nop 15\n\ts_nop 7" ::: "memory");
+    in_order();
+  }
+  DEV void in_order() {
+    #pragma unroll
+    for (int n = 0; n < NI; ++n)
+      #pragma unroll
+      for (int m = 0; m < MI; ++m) asm volatile("" : "+v"(acc[n][m]));
   }
 };
