@@ -116,6 +116,31 @@ def test_gated_linear(M, N, K):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("kind,tiles", [
+    ("bf16", [(64, 64), (64, 128), (128, 64)]),
+    ("gated", [(64, 64), (64, 128), (128, 64), (128, 128)]),
+    ("e4m3", [(64, 32), (64, 64), (64, 128)])])
+def test_equal_rows_have_equal_bits(kind, tiles):
+    """In whatever tile of rows they are, whose workgroups begin at the same
+    column."""
+    M, N, K = 300, 2064, 1280
+    g = torch.Generator().manual_seed(3)
+    x = torch.randn(1, K, generator=g).bfloat16().expand(M, K).contiguous() \
+        .to(DEV)
+    w = (torch.randn(N, K, generator=g) * 0.1).bfloat16().to(DEV)
+    scales = ()
+    if kind == "e4m3":
+        x, w = x.to(torch.float8_e4m3fn), w.to(torch.float8_e4m3fn)
+        scales = (torch.ones(M, device=DEV), torch.ones(N, device=DEV))
+    for bm, bn in tiles:
+        out = torch.empty(M, N // 2 if kind == "gated" else N,
+                          dtype=torch.bfloat16, device=DEV)
+        ops._native().gemm_split(out, x, w, None, bm, bn, 1, *scales,
+                                 gated=kind == "gated")
+        assert torch.equal(out, out[:1].expand_as(out)), (bm, bn)
+
+
+@pytest.mark.gpu
 def test_gated_linear_rows_far_apart():
     """Up rows that 32 bits of offset do not reach from the gate rows."""
     M, N, K, far = 17, 2560, 256, 1 << 21
