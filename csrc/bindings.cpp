@@ -207,8 +207,8 @@ void fused_add_rmsnorm(torch::Tensor x, torch::Tensor residual,
 }
 
 // Products of P choices with their experts' weights w [E, 2N (up) or N, K]:
-// out [P, N], x [P / div, K] (up) or [P, K], ids [P] int32 from -1 (none); place
-// [P] int32 becomes p, or -1 where there is none
+// out [P, N], x [P / div, K] (up) or [P, K], ids [P] int32; place [P] int32
+// becomes p, or -1 where ids names no expert, whose row of out is left as it is
 void experts_few(bool up, torch::Tensor out,
                  c10::optional<torch::Tensor> place, torch::Tensor x,
                  torch::Tensor w, torch::Tensor ids, long div) {
@@ -222,7 +222,7 @@ void experts_few(bool up, torch::Tensor out,
   TORCH_CHECK(P >= 1 && P <= 384 && out.size(0) == P &&
                   x.size(0) * (up ? div : 1) == P && w.size(2) == K &&
                   w.size(1) == (up ? 2 * N : N) && w.size(0) >= 1 &&
-                  N % 128 == 0 && K % 128 == 0,
+                  w.size(0) <= 64 && N % 128 == 0 && K % 128 == 0,
               "experts_few: shape");
   if (place.has_value()) {
     check(*place, torch::kInt32, "place");

@@ -39,7 +39,7 @@ __global__ __launch_bounds__(WAVES * 64) void experts_few_kernel(Few a) {
   const int n0 = blockIdx.x * OUT;
   if (a.place && blockIdx.x == 0 && blockIdx.y == 0)
     for (int p = threadIdx.x; p < a.P; p += WAVES * 64)
-      a.place[p] = a.ids[p] < 0 ? -1 : p;
+      a.place[p] = (unsigned)a.ids[p] < (unsigned)a.E ? p : -1;
   // as many experts as choices at most: the choices' own, each where it is
   // named first; otherwise all of them
   int e = blockIdx.y;
@@ -103,7 +103,8 @@ __global__ __launch_bounds__(WAVES * 64) void experts_few_kernel(Few a) {
 
 }  // namespace
 
-// P choices, 1 to 384; N and K multiples of 128; everything contiguous
+// P choices, 1 to 384, of 64 experts at most; N and K multiples of 128;
+// everything contiguous
 void launch_experts_few(bool up, bf16* out, int* place, const bf16* x,
                         const bf16* w, const int* ids, int P, int E, int N,
                         int K, int div, hipStream_t stream) {

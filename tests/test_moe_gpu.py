@@ -95,6 +95,24 @@ def test_few_choices(tokens, experts, top, width, inner, kind, monkeypatch):
     assert (out - ref).abs().max() <= 2.0 ** -5 * ref.abs().max()
 
 
+def test_choices_that_name_no_expert():
+    """Without a sort: no place, and nothing of them in the sum; and no more
+    experts than a load of their numbers has."""
+    few = ops._native().experts_few
+    x = torch.randn(6, 128, device=DEV).bfloat16()
+    w = torch.randn(4, 256, 128, device=DEV).bfloat16()
+    ids = torch.tensor([1, -1, 4, 3, 1 << 30, -(1 << 31)], dtype=torch.int32,
+                       device=DEV)
+    out = torch.full((6, 128), 7.0, device=DEV).bfloat16()
+    place = torch.empty_like(ids)
+    few(True, out, place, x, w, ids, 1)
+    assert place.tolist() == [0, -1, -1, 3, -1, -1]
+    assert (out[place < 0] == 7).all() and not (out[place >= 0] == 7).all(1).any()
+    many = torch.randn(65, 256, 128, device=DEV).bfloat16()
+    with pytest.raises(RuntimeError):
+        few(True, out, place, x, many, ids, 1)
+
+
 @pytest.mark.parametrize("tokens", [1, 26, 27, 56, 57, 300])
 @pytest.mark.parametrize("experts,top,width,inner", [
     (4, 2, 256, 384), (3, 1, 1024, 256)])
