@@ -313,7 +313,7 @@ def _wave_gemm(M: int, N: int, K: int):
     6 rows 37 31; 11264 x 512 39 rows 7.9 5.7.  Beyond 64 rows the library is as
     fast (96 of 32768 x 4096 63 60, 128 64 65), and so it is with fewer or more
     tiles (10 of 7808 x 4096 17 21; 2 of 39104 x 4096 59 64)."""
-    if not 1 <= M <= 64 or K % 128 or N % 4:
+    if not 1 <= M <= 64 or K == 0 or K % 128 or N % 4:
         return None
     for bn in (64, 128):
         if 176 <= -(-N // bn) <= 256:
@@ -326,6 +326,8 @@ def _route(M: int, N: int, K: int, parts: bool):
     """How x w^T of these sizes is formed: "rows", (rows, outputs of a tile, parts
     of K) or None, the library.  Kept, for the rules take as long as a launch: a
     step of small prompts, which is not captured, waits for the host."""
+    if K >= 1 << 24:                # the kernels' chunks are counted in 32 bits
+        return None
     wave = _wave_gemm(M, N, K)
     if wave is not None:
         return wave
@@ -432,7 +434,7 @@ def _summed_gemm(M: int, N: int, K: int):
     128 rows, 0.92 in 40 (480 of 4096 x 4096 33 32, 395 of 5120 x 7168 60 51, 298
     of 3968 x 6144 40 35, 454 of 4224 x 11008 93 68).  Two parts of tall tiles
     are even (452 of 5504 x 8192 65 70, 379 of 7168 x 14336 119 116)."""
-    if K % 128 or N % 8 or N > 8192:
+    if K % 128 or N % 8 or not 0 < N <= 8192:
         return None
     if M <= 16 and K >= 5120 and N * K >= 14 << 20:
         split = min(6, 256 // -(-N // 64), K // 1024)
@@ -502,7 +504,8 @@ def _gated_tile(M: int, N: int, K: int):
     96; 6 of 52736 x 1536 36 38).  Few tiles with long rows leave the chip idle (23 rows of 2048 x 3072
     10 13), and more than 64 rows of more than 4096 columns gain nothing (71 of
     6144 x 5120 22.5 22.8, 119 of 5632 x 5120 25 27)."""
-    if not 1 <= M <= 256 or K % 128 or N % 16 or M > 64 and K > 4096:
+    if not 1 <= M <= 256 or K == 0 or K % 128 or N % 16 \
+            or M > 64 and K > 4096 or max(N, K) >= 1 << 24:
         return None
     for bm, bn in ((64, 64), (64, 128)) if M <= 64 \
             else ((64, 64), (128, 64), (128, 128)):
@@ -565,7 +568,8 @@ def _tiles_q(M: int, N: int, K: int, parts: bool):
     Beyond 64 rows half as many tiles lie beside each other: long rows only with
     the norm (128 of 4096 x 14336 44 -> 28), 2048 x 7168 is even (14.0 13.7).
     Beyond 128 rows there is no gain (200 of 4096 x 4096 17.1 17.2)."""
-    if not 1 <= M <= 128 or K % 256 or N % 4 or N * K < 1 << 22:
+    if not 1 <= M <= 128 or K % 256 or N % 4 or N * K < 1 << 22 \
+            or K >= 1 << 24:
         return None
     tiles = -(-M // 64) * -(-N // 64)
     few = M <= 16

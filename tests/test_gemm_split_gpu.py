@@ -233,3 +233,28 @@ def test_sizes_where_the_library_is_faster():
     for m, n, k in ((321, 3072, 8192), (257, 3584, 8192), (64, 4096, 16384),
                     (144, 6144, 7168), (145, 7168, 7168)):
         assert ops._split_gemm(m, n, k) is not None
+
+
+def test_rules_leave_sizes_beyond_the_kernel_to_the_library(monkeypatch):
+    """No columns, and sizes from 2^24 on."""
+    monkeypatch.setattr(ops, "_native", lambda: type("", (), {
+        "gemm_rows_fits": staticmethod(lambda M, K: True)}))
+    ops._route.cache_clear()
+    for M in (0, 1, 16, 17, 64, 65, 128, 256, 512):
+        for N, K in ((16384, 0), (28672, 0), (4096, 0), (0, 4096), (0, 0),
+                     (8, 1 << 24), (4096, 1 << 24), (1 << 24, 128)):
+            for parts in (False, True):
+                route = ops._route(M, N, K, parts)
+                assert route is None or route == "rows" and N * K, (M, N, K)
+                assert ops._tiles_q(M, N, K, parts) is None
+            assert ops._gated_tile(M, N, K) is None, (M, N, K)
+    ops._route.cache_clear()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N", [(1, 16384), (17, 28672), (64, 4096)])
+def test_products_of_no_columns(M, N):
+    x, w = (torch.empty(n, 0, dtype=torch.bfloat16, device=DEV) for n in (M, N))
+    assert torch.equal(ops.linear(x, w), x @ w.t())
+    assert torch.equal(ops.linear_parts(x, w), x @ w.t())
+    assert torch.equal(ops.gated_linear(x, w), ops.silu_mul(x @ w.t()))
