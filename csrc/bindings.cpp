@@ -505,13 +505,15 @@ void gemm_split(c10::optional<torch::Tensor> out, torch::Tensor x,
                     reinterpret_cast<uintptr_t>(out->data_ptr()) % 8 == 0,
                 "gemm_split: out");
   const long unit = fp8 ? 16 : 8, chunk = fp8 ? 256 : 128;
-  auto aligned = [&](const torch::Tensor& t) {
+  // 16 bytes at a time, the rows of a tile by 32 bits of offset
+  auto fits = [&](const torch::Tensor& t, long rows) {
+    const long reach = (std::min(t.size(0), rows) - 1) * t.stride(0) + K;
     return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0 &&
-           t.stride(0) % unit == 0 && t.stride(0) < (1l << 22);
+           t.stride(0) % unit == 0 && reach < 0xfffffff0l / (fp8 ? 1 : 2);
   };
   TORCH_CHECK(N % 4 == 0 && K % chunk == 0 && K >= chunk && M < (1l << 20) &&
-                  K < (1l << 24) && N < (1l << 24) && aligned(x) && aligned(w),
-              "gemm_split: sizes");
+                  K < (1l << 24) && N < (1l << 24) && fits(x, bm) &&
+                  fits(w, bn), "gemm_split: sizes");
   TORCH_CHECK(fp8 ? bm == 64 && (bn == 32 || bn == 64 || bn == 128)
                   : ((bm == 64 || bm == 128) && (bn == 64 || bn == 128)) ||
                         (bm == 256 && bn == 128), "gemm_split: tile");

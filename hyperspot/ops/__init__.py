@@ -453,9 +453,10 @@ def _summed_gemm(M: int, N: int, K: int):
     return None
 
 
-def _near(*tensors: torch.Tensor) -> bool:
-    """Rows that 32 bits of offset reach from the first one of a tile."""
-    return all(t.stride(0) < 1 << 22 for t in tensors)
+def _near(x: torch.Tensor, w: torch.Tensor, bm: int, bn: int) -> bool:
+    """32 bits of offset reach the rows of a tile of bm by bn from its first."""
+    return all(((min(t.shape[0], rows) - 1) * t.stride(0) + t.shape[1])
+               * t.itemsize < 0xfffffff0 for t, rows in ((x, bm), (w, bn)))
 
 
 def _product(x: torch.Tensor, w: torch.Tensor, parts: bool, plain: bool):
@@ -463,7 +464,7 @@ def _product(x: torch.Tensor, w: torch.Tensor, parts: bool, plain: bool):
     what _plain_bf16 says, which looks at the sizes of no traced tensor."""
     route = _route(x.shape[0], *w.shape, parts) \
         if plain and x.shape[0] <= MOST_ROWS else None
-    if route is None or route != "rows" and not _near(x, w):
+    if route is None or route != "rows" and not _near(x, w, *route[:2]):
         return x @ w.t()
     M, N = x.shape[0], w.shape[0]
     if route == "rows":
@@ -522,7 +523,7 @@ def gated_linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     plain = _plain_bf16(x, w)
     if plain and x.shape[0] <= MOST_ROWS:
         tile = _gated_tile(x.shape[0], *w.shape)
-        if tile is not None and _near(x, w) \
+        if tile is not None and _near(x, w, *tile) \
                 and w.stride(0) * (w.shape[0] + 256) < 1 << 32:
             out = torch.empty(x.shape[0], w.shape[0] // 2, dtype=x.dtype,
                               device=x.device)
@@ -600,7 +601,8 @@ def _tiled_q(x: "QTensor", w: torch.Tensor, scale: torch.Tensor, parts: bool):
         return None
     tile = _tiles_q(d.shape[0], *w.shape, parts)
     if tile is None or not (
-            d.dtype == w.dtype == torch.float8_e4m3fn and _near(d, w)
+            d.dtype == w.dtype == torch.float8_e4m3fn
+            and _near(d, w, *tile[:2])
             and s.dtype == scale.dtype == torch.float32
             and s.is_contiguous() and scale.is_contiguous()
             and scale.data_ptr() % 16 == 0

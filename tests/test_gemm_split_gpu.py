@@ -152,6 +152,39 @@ def test_gated_linear_rows_far_apart():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("stride", [1 << 22, (1 << 22) + 8])
+def test_rows_far_apart(stride, monkeypatch):
+    """Up to where 32 bits of offset reach the last row of a tile; one row of x,
+    whose stride means nothing."""
+    M, N, K = 17, 132, 640
+    x = torch.empty(M * stride, device=DEV, dtype=torch.bfloat16).view(
+        M, stride)[:, :K].normal_()
+    w = torch.randn(N, K, device=DEV).bfloat16()
+    monkeypatch.setattr(ops, "_route", lambda *a: (64, 64, 2))
+    seen = []
+    kernel = ops._native().gemm_split
+    monkeypatch.setattr(ops._native(), "gemm_split", lambda *a: (
+        seen.append(1), kernel(*a)))
+    _check(ops.linear(x, w), x, w)
+    one = x[:1].as_strided((1, K), (1 << 40, 1))
+    _check(ops.linear(one, w), one, w)
+    assert len(seen) == 2
+
+
+def test_reach_of_a_tile():
+    """The farthest rows that 32 bits of offset reach, and the next ones."""
+    for dtype, size in ((torch.bfloat16, 2), (torch.float8_e4m3fn, 1)):
+        near = torch.empty(8, 128, dtype=dtype, device="meta")
+        for rows in (1, 2, 64, 65, 300):
+            for stride in (1 << 22, 1 << 25, 1 << 26, 1 << 40):
+                far = torch.empty_strided((rows, 128), (stride, 1),
+                                          dtype=dtype, device="meta")
+                last = (min(rows, 64) - 1) * stride * size + 256
+                assert ops._near(far, near, 64, 128) == (last < 1 << 32)
+                assert ops._near(near, far, 128, 64) == (last < 1 << 32)
+
+
+@pytest.mark.gpu
 def test_watched_products_get_their_calls():
     """A hook on the gate and up product sees it, and may change it."""
     from hyperspot.engine.config import ModelSpec
