@@ -49,12 +49,16 @@ void experts_tiles_kernel(Tiles a) {
   const int e = a.expert[tile];
   if (e < 0) return;
   // The tiles of an expert that take the same weights go to one die together,
-  // whose L2 then has them: 4 layers of 8 experts of 14336 x 4096, 500 choices an
-  // expert 5421 -> 5278 us, 1027 8407 -> 8366.  (Full tiles of all experts first,
-  // so that the shorter ones end the launch: 6426.)  Where rows are short the
-  // search for the other tiles takes longer (300 choices an expert, 32 of 1024 x
-  // 2048, 2332 2361).  More than 32 tiles share them without it.
-  if (BM == 256 && a.K >= 4096 && a.nx % 8 == 0) {
+  // whose L2 then has them, where an expert has 128 MB of them, half of what the
+  // memory's cache holds: later tiles would find them gone.  180 random sizes (2
+  // to 16 experts, 100 to 1100 choices each, N of 2048 to 16384, K of 1024 to
+  // 15000), time over that without: 256 x 256 from 128 MB on 0.962, two of 29 more
+  // than 1.2 % slower (16 of 16384 x 5760, 1060 choices 6666 -> 6335 us, 8 of 16384
+  // x 2432, 590 841 -> 767, 8 of 8192 x 14080, 320 1.041), with 50 to 128 MB 0.997,
+  // with less 1.024; 256 x 128, which are fewer, 1.032 (2 of 10240 x 3072 77 ->
+  // 96).  More than 32 tiles share them without it.
+  if (BM == 256 && BN == 256 && a.nx % 8 == 0 &&
+      (GATED ? 2 : 1) * a.N * ((long)a.K * ELEM) >= 128l << 20) {
     const int t = threadIdx.x & 63, tiles = gridDim.x / a.nx;
     const unsigned long back =
         ~__ballot(t <= tile && a.expert[t <= tile ? tile - t : 0] == e);
