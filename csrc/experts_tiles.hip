@@ -121,9 +121,13 @@ void experts_tiles_kernel(Tiles a) {
   // expert and the same outputs at the same.  192 tokens of 2 choices, 8 experts
   // of 14336 x 4096 355 + 188 -> 321 + 162 us; 4 of 32 of 1024 x 2048 65 + 29 ->
   // 50 + 29; in tiles of 256, 500 choices an expert, 1011 + 639 1029 + 643.
+  // Three times as far apart where rows are long: 140 random sizes (4 to 64
+  // experts, K of 1024 to 14336), time over that of once as far: rows of 12 KB and
+  // more 0.984, 8 and 10 KB in tiles of 128 0.985, of 64 1.02 (16 of 4096 x 4096,
+  // 22 choices each, 99 108), shorter ones 1.01 (64 of 3072 x 2048 150 162).
   const int stages = (int)(row_bytes / 128);
-  const int turn = BM == 256 ? 0
-      : (nb + e * a.nx) / 8 * (stages >= 64 ? 3 : 1) % stages;
+  const int apart = stages >= (BM == 64 ? 96 : 64) ? 3 : 1;
+  const int turn = BM == 256 ? 0 : (nb + e * a.nx) / 8 * apart % stages;
   auto stage = [&](int slot, int d) {
     d += turn;
     if (d >= stages) d -= stages;
