@@ -426,19 +426,26 @@ def _less_padding(M: int, split):
 
 def _summed_gemm(M: int, N: int, K: int):
     """As _split_gemm, for more sizes, where the norm adds up the parts.  Measured
-    with the norm: up to 16 rows of long K (1 row of 4096 x 14336 27.4 26.7, 8
-    28.6 27.1, 16 29.6 27.2; of 2048 x 7168 13.0 11.1, 13.1 11.6, 13.5 11.7); 33 to 128 rows with K of 1024 to 4096 and less than 14M
-    weights, 0.87 of the library's time on average in 65 sizes and none slower by
-    3 % (48 rows of 2048 x 2048 11.0 8.9 us, 64 of 4096 x 2560 13.4 12.5, 78 of
-    3200 x 3584 23 14); 257 to 512 rows with K from 5120 on, or 4096 in tiles of
-    128 rows, 0.92 in 40 (480 of 4096 x 4096 33 32, 395 of 5120 x 7168 60 51, 298
-    of 3968 x 6144 40 35, 454 of 4224 x 11008 93 68).  Two parts of tall tiles
-    are even (452 of 5504 x 8192 65 70, 379 of 7168 x 14336 119 116)."""
+    with the norm.  1 to 16 rows, K of 5120 to 20000 and N of 64 to 8192 in 400
+    random sizes: with 5 parts or more (N up to 3264) 0.62 of the library's time on
+    average (9 rows of 512 x 5632 9.6 9.1, 1 of 2048 x 7168 14.3 11.8, 15 of 3072 x
+    5120 13.7 12.8; the slowest 5 of 3072 x 16384 26.6 28.1).  With 3 or 4 about even
+    up to 8192 columns (2 of 4096 x 7168 16.7 17.4, 10 of 5168 x 7168 23.2 21.4) but
+    where K is no multiple of 512 (8 of 4392 x 6784 31 19), beyond 0.8 (1 of 4096 x
+    14336 28.8 27.5, 9 of 4096 x 11264 24.1 24.2), and slower where rows lie a
+    multiple of 16 KB apart (8 of 4096 x 8192 18.7 22.9).  33 to 128 rows with K of
+    1024 to 4096 and less than 14M weights: 0.87 in 65 sizes, none slower by 3 % (48
+    rows of 2048 x 2048 11.0 8.9 us, 64 of 4096 x 2560 13.4 12.5, 78 of 3200 x 3584
+    23 14).  257 to 512 rows with K from 5120 on, or 4096 in tiles of 128 rows: 0.92
+    in 40 (480 of 4096 x 4096 33 32, 395 of 5120 x 7168 60 51, 298 of 3968 x 6144 40
+    35, 454 of 4224 x 11008 93 68).  Two parts of tall tiles are even (452 of 5504 x
+    8192 65 70, 379 of 7168 x 14336 119 116)."""
     if K % 128 or N % 8 or not 0 < N <= 8192:
         return None
-    if M <= 16 and K >= 5120 and N * K >= 14 << 20:
+    if M <= 16 and K >= 5120 and N * K >= 2 << 20:
         split = min(6, 256 // -(-N // 64), K // 1024)
-        return (64, 64, split) if split > 2 else None
+        return (64, 64, split) if split >= 5 or split >= 3 and K % 8192 and (
+            K > 8192 or K % 512) else None
     if 32 < M <= 128 and 1024 <= K <= 4096 and 1 << 20 <= N * K < 14 << 20:
         split = min(8, 256 // (-(-M // 64) * -(-N // 64)), K // 512)
         return (64, 64, split) if split > 1 else None

@@ -48,6 +48,8 @@ def test_tiles_of_64_rows(M, N, K, parts, bm, bn):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K", [(1, 2048, 7168), (16, 4096, 14336),
+                                   (1, 416, 5120), (16, 3264, 5120),
+                                   (9, 5440, 8704), (7, 3272, 6784),
                                    (33, 2048, 2048), (64, 4096, 1280),
                                    (128, 4096, 2560), (257, 3200, 8192),
                                    (480, 4096, 4096), (400, 5120, 5120)])
@@ -243,6 +245,21 @@ def test_rule_stays_in_what_the_kernel_takes():
                 assert 1 <= parts <= min(8, K // 128) and K % 128 == 0
                 assert -(-M // bm) * -(-N // bn) * parts <= 256
     assert taken
+
+
+def test_rule_of_few_rows_of_long_columns():
+    """From 5 parts on, or with 3 where the library has no better tile; as
+    many workgroups as units at most."""
+    taken = lambda N, K: ops._summed_gemm(8, N, K) is not None
+    assert taken(3264, 5120) and not taken(3272, 5120) and not taken(3264, 4992)
+    assert taken(3272, 6784) and not taken(3272, 7168) and taken(3272, 9216)
+    assert taken(2048, 16384) and not taken(4096, 16384)
+    assert not taken(5504, 9216)
+    for N in range(8, 8193, 104):
+        for K in range(5120, 20481, 128):
+            rule = ops._summed_gemm(8, N, K)
+            if rule is not None:
+                assert -(-N // 64) * rule[2] <= 256 and 3 <= rule[2] <= K // 512
 
 
 def test_rule_leaves_no_workgroup_for_a_second_wave():
