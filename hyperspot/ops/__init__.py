@@ -294,13 +294,6 @@ def _plain_bf16(x: torch.Tensor, w: torch.Tensor) -> bool:
         and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
 
 
-def _rows_gemm(x: torch.Tensor, w: torch.Tensor) -> bool:
-    """Whether csrc/gemm_rows.hip takes x w^T: few rows, and sizes at which it
-    is faster than the library on average of some hundred random ones."""
-    return _plain_bf16(x, w) and _rows_gemm_sizes(x.shape[0], *w.shape) \
-        and _native().gemm_rows_fits(*x.shape)
-
-
 MOST_ROWS = 512         # of a product that a kernel here takes
 
 
@@ -822,9 +815,9 @@ def moe_ffn_fp8(xq: "QTensor", w13q: torch.Tensor, w13s: torch.Tensor,
                 w2q: torch.Tensor, w2s: torch.Tensor,
                 weights: torch.Tensor, ids: torch.Tensor) -> torch.Tensor:
     """fp8 grouped expert FFN: e4m3fn activations (QTensor from the fused
-    norm producer) x e4m3fn expert weights through
-    v_mfma_f32_32x32x16_fp8_fp8; the silu stage re-quantizes via the fused
-    silu_mul_fp8 kernel so no extra passes appear."""
+    norm producer) x e4m3fn expert weights in tiles (csrc/experts_tiles.hip); the
+    silu stage re-quantizes via the fused silu_mul_fp8 kernel so no extra passes
+    appear."""
     n = _native()
     (T, H), K, (E, _, I) = xq.data.shape, ids.shape[1], w2q.shape
     if T == 0:
@@ -865,7 +858,8 @@ def sample(logits: torch.Tensor, temperature: torch.Tensor,
            top_p: torch.Tensor, top_k: torch.Tensor,
            uniform: torch.Tensor) -> torch.Tensor:
     """Batch sampling: temperature (0: the largest logit), top-k, top-p and an
-    inverse-CDF draw over the tokens in order of their ids, in one kernel."""
+    inverse-CDF draw over the tokens in order of their ids, in one kernel or, of
+    few rows, in two (csrc/sampling.hip)."""
     if not logits.is_cuda:
         return torch_ref.sample(logits, temperature, top_p, top_k, uniform)
     rows, vocab = logits.shape

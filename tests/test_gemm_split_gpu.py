@@ -217,9 +217,11 @@ def test_linear_takes_it(M, N, K):
     _check(out, x, w)
     route = "rows" if M == 17 and K == 4096 \
         else "library" if M > 256 and (N, K) != (2048, 7168) else "split"
-    rule = None if ops._rows_gemm(x, w) else ops._split_gemm(M, N, K)
-    assert ops._rows_gemm(x, w) == (route == "rows")
-    assert (rule is None) == (route != "split")
+    rule = ops._route(M, N, K, False)
+    assert (rule == "rows") == (route == "rows")
+    assert (rule is None) == (route == "library")
+    if (M, N, K) == (17, 2048, 7168):
+        assert rule[:2] == (64, 64)
     again = torch.empty_like(out)
     if route == "rows":
         ops._native().gemm_rows(again, x, w)
@@ -229,6 +231,18 @@ def test_linear_takes_it(M, N, K):
         part = torch.empty(rule[2] * M * N, device=DEV)
         ops._native().gemm_split(again, x, w, part, *rule)
     assert torch.equal(out, again)
+
+
+@pytest.mark.gpu
+def test_one_wave_goes_before_rows():
+    """Where both rules would take a product of few rows."""
+    M, N, K = 4, 16384, 2048
+    assert ops._rows_gemm_sizes(M, N, K) and ops._native().gemm_rows_fits(M, K)
+    assert ops._route(M, N, K, False) == ops._wave_gemm(M, N, K) == (64, 64, 1)
+    x, w = (torch.randn(n, K, device=DEV).bfloat16() for n in (M, N))
+    again = torch.empty(M, N, dtype=torch.bfloat16, device=DEV)
+    ops._native().gemm_split(again, x, w, None, 64, 64, 1)
+    assert torch.equal(ops.linear(x, w), again)
 
 
 def test_rule_stays_in_what_the_kernel_takes():

@@ -45,7 +45,7 @@ def test_what_a_kernel_may_replace():
 @pytest.mark.gpu
 def test_gradients_and_transforms_of_products():
     x, w = _operands("cuda:0")
-    assert ops._rows_gemm(x, w)
+    assert ops._plain_bf16(x, w) and ops._route(4, 2048, 1024, False) == "rows"
     ref = x.clone().requires_grad_()
     (ref @ w.t()).float().square().sum().backward()
     got = x.clone().requires_grad_()

@@ -136,6 +136,46 @@ def test_nan_is_not_drawn(vocab, dtype):
     assert not gone[:-1].gather(1, nan[:-1, None].cpu()).any()
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("vocab", [7, 1001, 8192, 50257, 128256])
+def test_rows_whole_and_in_slices(vocab, dtype):
+    """The same rows in a batch that is not divided and in one that is: both
+    against float64, NaN as -inf and infinities as the largest value."""
+    g = torch.Generator().manual_seed(vocab)
+    kinds = ["normal", "peaked", "ties", "masked", "wide"]
+    options = [(1.0, 1.0, 0), (0.7, 0.9, 0), (1.3, 0.5, 40), (0.0, 1.0, 0),
+               (1.0, 1.0, 5), (2.0, 0.95, 600)]
+    pick = [(i, o) for i in range(2 * len(kinds)) for o in range(len(options))]
+    x = torch.stack([_row(kind, vocab, g) for kind in kinds * 2])
+    x[len(kinds):].masked_fill_(torch.rand(len(kinds), vocab, generator=g) < .3,
+                                float("nan"))
+    x[2::3, vocab // 2] = float("inf")
+    x = x.to(dtype)
+    t, p, k = (torch.tensor(c) for c in zip(*(options[o] for _, o in pick)))
+    u = torch.rand(len(pick), generator=g)
+    which = torch.tensor([i for i, _ in pick])
+    least = -(-vocab // 32768)
+    all_rows = torch.arange(len(pick)).repeat(513 // (least * len(pick)) + 1)
+    assert len(all_rows) * least > 512 >= 20 * least
+    args = [a.to(DEV) for a in (x, t, p, k.int(), u, which)]
+
+    def draw(a):
+        x, t, p, k, u, which = args
+        a = a.to(DEV)
+        return ops.sample(x[which[a]], t[a], p[a], k[a], u[a])
+    whole = draw(all_rows)[:len(pick)].tolist()
+    sliced = torch.cat([draw(a) for a in all_rows[:len(pick)].split(20)]) \
+        .tolist()
+    for b, (i, o) in enumerate(pick):
+        row = x[i].float().nan_to_num(
+            float("-inf"), posinf=torch.finfo(torch.float32).max,
+            neginf=float("-inf"))
+        if not torch.isfinite(row).any():
+            continue
+        ok, _ = _allowed(row, *options[o], float(u[b]))
+        assert ok[whole[b]] and ok[sliced[b]], (i, o, whole[b], sliced[b])
+
+
 @pytest.mark.parametrize("vocab,rows", [
     (16384, 1), (32768, 100), (32776, 100), (65537, 40), (128256, 1),
     (128256, 30), (128256, 60), (128256, 129), (524288, 1), (524296, 1)])
