@@ -323,10 +323,14 @@ __global__ __launch_bounds__(256, 3) void paged_attn_mfma_kernel(Paged a) {
   __shared__ __attribute__((aligned(16))) char v_lds[4][BLOCK * HD * 2];
   __shared__ float m_lds[4][16], l_lds[4][16];
   // Without parts the heads of a row, whose pages lie beside each other, come
-  // first, which memory reads faster than rows first: us of 256 rows x 8 kv heads
-  // of 4, 1000 tokens 196 -> 189, e4m3 112 -> 105, of 64 tokens 25.5 26.0; 192 of
-  // 500 81 -> 77; 40 of 2000 81 -> 73; 64 x 4 kv heads of 1000 30.6 31.2.  With
-  // parts, rows first (8 x 8 of 8000 in 4 parts 54, the other way 55).
+  // first, which memory reads faster than rows first where contexts are ragged:
+  // us of a step of 8 layers with 8 kv heads of 4, 256 rows of about 1000 tokens
+  // 3236 -> 3102, of 64 1775 1765, 100 of 1000 1908 -> 1859; of 4 layers with e4m3
+  // pages, 256 of 1000 1120 -> 1059, of 64 741 -> 707; 8 layers with 4 kv heads 256
+  // of 1000 1577 1564; within 1 % with 64 rows.  Contexts of one length read as
+  // fast either way (the attention alone 196 194), and 64 tokens of each slower
+  // (19.6 20.3, e4m3 15.0 16.3).  With parts, rows first (8 x 8 of 8000 in 4 parts
+  // 54, the other way 55).
   const int group = a.group, split = a.split;
   const bool whole = split == 1;
   const int g = whole ? blockIdx.x : blockIdx.y;

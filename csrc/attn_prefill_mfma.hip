@@ -29,16 +29,15 @@
 // Within a tile the operands of 8 products are loaded ahead of them, and the next
 // 16 tokens' weights are formed between the products of the last 16, not before
 // them.  Tiles come by buffer loads: beside loads from a global address to LDS
-// the compiler waited for all LDS reads wherever it needed the oldest (8192 rows
-// 613 -> 602 us, 7808 after 8192 cached tokens 2560 -> 2500).  Long prompts are bound by power: with zeros as data 8192 cached tokens
-// and 7808 rows take 1.94 ms, with normal values 2.57.
+// the compiler waited for all LDS reads wherever it needed the oldest.  Long
+// prompts are bound by power: with zeros as data 7808 rows after 8192 cached
+// tokens take 1.86 ms, with normal values 2.47.
 //
-// 32 heads, 8 kv heads: a prompt of 8192 tokens 734 us (749 TFLOP/s) where
-// weights that went through LDS and tiles of 256 rows of one head took 2628
-// (209); of 512 17.9, and 18.9 with weights and products in turn; 8 prompts of
-// 1000, 133 us; 7808 tokens after 8192 cached ones 2.60 ms (2.65 in turn; e4m3
-// pages 2.69, 2.72), 500 after 500 36 us (41), where one workgroup a row took
-// 37.6 ms.
+// 32 heads, 8 kv heads, us without those two steps and now: a prompt of 8192
+// tokens 612 601 (915 TFLOP/s), of 512 18.6 17.8, 8 of 1000 124 122; 7808 tokens
+// after 8192 cached ones 2587 2487, of e4m3 2630 2592, 500 after 500 39 34.
+// Weights that went through LDS and tiles of 256 rows of one head took 3.6 times
+// as long for 8192 tokens, one workgroup a row 37.6 ms for 7808 after 8192.
 //
 // ROWS: weights are rounded to bf16, relative to the maximum after each tile of
 // 64 tokens, and summed in a fixed order.  Both are a part of the result: a

@@ -1,8 +1,9 @@
 // Sampling kernels: greedy argmax, and the whole of temperature, top-k, top-p
 // and draw.
 //
-// One workgroup per batch row over vocab-size logits (128256 for Llama-3).
-// Vectorized bf16/f32 reads; fp32 math, sums of weights in 64-bit integers.
+// A batch row of vocab-size logits (128256 for Llama-3) is one workgroup's, or
+// that of several and a second kernel where there are few rows.  Vectorized
+// bf16/f32 reads; fp32 math, sums of weights in 64-bit integers.
 #include <float.h>
 
 #include <type_traits>
@@ -70,7 +71,7 @@ __global__ __launch_bounds__(256) void greedy_sample_kernel(
 // the chains of steps that a row's workgroup takes one after the other.  So a row
 // is divided into slices where there are few rows (below): 64 rows of 128256 are
 // 256 workgroups, 7 us for the largest values, 12 with the weights, and a second
-// kernel of 3 (greedy) to 13 us (a share).  8 values are looked at together where
+// kernel of 2 (greedy) to 13 us (a share).  8 values are looked at together where
 // that decides about all of them.  Where few values stay, and next-token logits
 // have a few dozen that matter, they are listed and the rest is done on the list,
 // up to 8 threads a value.  Otherwise no sort either: one histogram of counts and
@@ -81,13 +82,16 @@ __global__ __launch_bounds__(256) void greedy_sample_kernel(
 // lanes that add to the same few counters in LDS would go one by one.
 //
 // 64 rows of 128256, 48 values far above the others, us with a workgroup a row
-// and now: temperature 41 17, top_p 0.9 42 24, top_k 50 30 17, greedy 14 10; a
-// mix 43 24.5, where the library's sorts, scans and selections took 2625.
-// Normal logits, whose share is thousands of values, 132 124.
+// and now, rows in cache (from memory 2 to 3 more): temperature 36 16, top_p 0.9
+// 43 24, top_k 50 24 15, greedy 9.4 9.0; a mix 42 24, where the library's sorts,
+// scans and selections took 2625.  Normal logits, whose share is thousands of
+// values, 137 129.  A call that is waited for and not captured 60 44.
 //
 // Weights are 2^-40 fixed point relative to the largest (of the row or of the
-// slice), so every sum is exact, does not depend on its order, and the same
-// inputs give the same token.
+// slice), so sums within a row or a slice are exact; slices are brought to the
+// row's scale by one rounded factor each and added in their order.  So the same
+// inputs give the same token; a batch of another size, which is divided
+// otherwise, may give another one where the draw falls on a boundary to 2^-40.
 namespace {
 
 typedef unsigned long long u64;
