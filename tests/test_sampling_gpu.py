@@ -233,8 +233,9 @@ def _few_above(kind, vocab):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("rows", [4, 1030])
-@pytest.mark.parametrize("vocab", [2, 5, 9, 40, 700, 8191, 8192, 32768, 32773])
+@pytest.mark.parametrize("vocab,rows", [
+    (v, r) for v in (2, 5, 9, 40, 700, 8191, 8192, 32768, 32773)
+    for r in (4, 1030)] + [(128256, 4)])
 def test_the_smallest_values_may_stay(vocab, rows, dtype):
     """top_k where fewer values than that are above the smallest one: in slices
     (4 rows) and without, over uniforms that reach every part of a row."""
