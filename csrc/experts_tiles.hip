@@ -128,16 +128,16 @@ void experts_tiles_kernel(Tiles a) {
   const int stages = (int)(row_bytes / 128);
   const int apart = stages >= (BM == 64 ? 96 : 64) ? 3 : 1;
   const int turn = BM == 256 ? 0 : (nb + e * a.nx) / 8 * apart % stages;
-  auto stage = [&](int slot, int d) {
+  // load i of a stage: first those of x, then those of w
+  auto stage = [&](int slot, int d, int i) {
     d += turn;
     if (d >= stages) d -= stages;
     char* l = lds + slot * Loop::STAGE;
-    #pragma unroll
-    for (int j = 0; j < LX; ++j)
-      load(l + (wid * LX + j) * 1024, x_rows, x0, x_off[j], d);
-    #pragma unroll
-    for (int j = 0; j < LW; ++j)
-      load(l + BM * 128 + (wid * LW + j) * 1024, w_rows, w0, w_off[j], d);
+    if (i < LX)
+      load(l + (wid * LX + i) * 1024, x_rows, x0, x_off[i], d);
+    else
+      load(l + BM * 128 + (wid * LW + i - LX) * 1024, w_rows, w0,
+           w_off[i - LX], d);
   };
   Loop loop;
   loop.run(lds, wm, wn, stages, live, stage);

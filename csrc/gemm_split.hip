@@ -99,22 +99,21 @@ void gemm_split_kernel(Split a) {
   // kernel, 3245 us, with it 3251
   const int turn =
       (FP8 || GATED || BM == 64) && a.splits == 1 ? at / a.mt * a.mt % chunks : 0;
-  auto stage = [&](int slot, int d) {
+  // load i of a stage: first those of x, then those of w
+  auto stage = [&](int slot, int d, int i) {
     d += turn;
     if (d >= chunks) d -= chunks;
-    char* base = lds + slot * Loop::STAGE;
-    #pragma unroll
-    for (int j = 0; j < LX; ++j)
-      #pragma unroll
-      for (int s = 0; s < KC; ++s)
-        x_rows.to_lds(base + s * Loop::SUB + (wid * LX + j) * 1024, x_off[j],
-                      (d * KC + s) * 128);
-    #pragma unroll
-    for (int j = 0; j < LW; ++j)
-      #pragma unroll
-      for (int s = 0; s < KC; ++s)
-        w_rows.to_lds(base + s * Loop::SUB + BM * 128 + (wid * LW + j) * 1024,
-                      w_off[j], (d * KC + s) * 128);
+    const int s = i % KC;
+    char* base = lds + slot * Loop::STAGE + s * Loop::SUB;
+    if (i < LX * KC) {
+      const int j = i / KC;
+      x_rows.to_lds(base + (wid * LX + j) * 1024, x_off[j],
+                    (d * KC + s) * 128);
+    } else {
+      const int j = i / KC - LX;
+      w_rows.to_lds(base + BM * 128 + (wid * LW + j) * 1024, w_off[j],
+                    (d * KC + s) * 128);
+    }
   };
   Loop loop;
   loop.run(lds, wm, wn, chunks, live, stage);

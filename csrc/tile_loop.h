@@ -38,6 +38,15 @@ typedef __attribute__((ext_vector_type(8))) int int32x8_t;
 
 // BM rows of x, BN of w; WM * WN waves have BM / WM by BN / WN.  A stage has KC
 // chunks: BM rows of x, then BN of w, of each.
+//
+// SPREAD: a stage's loads are issued between the products of the next one, not
+// all behind the barrier that frees its slot, where 48 KB take a compute unit's
+// memory pipe some 770 cycles and no wave that waits to issue its own gets to a
+// product.  They have one stage less to arrive in, so it takes three.  us, with
+// weights from memory: 512 rows of 4096 x 14336 in 4 parts 66 -> 62, of 6144 x
+// 4096 in 2 36.1 -> 34.0, 256 of 28672 x 4096 75 -> 70.  128 x 128 tiles, which
+// have less to issue, are even (256 rows of 4096 x 14336 45.1 45.5), smaller ones
+// slower (32 of 2048 x 7168 8.3 8.9).
 template <int BM, int BN, int WM, int WN, int STAGES, int KC, bool FP8>
 struct TileLoop {
   static constexpr int WAVES = WM * WN;
@@ -89,7 +98,9 @@ struct TileLoop {
         }
   }
 
-  // stage(slot, d) issues this wave's LOADS loads of stage d of the ring.
+  static constexpr bool SPREAD = BM == 256 && STAGES > 2;
+
+  // stage(slot, d, i) issues load i of this wave's LOADS of stage d of the ring.
   // Every wave has to call this; those that are not live only load.
   template <class Stage>
   DEV void run(char* lds, int wm, int wn, int stages, bool live,
@@ -97,13 +108,18 @@ struct TileLoop {
     const int lane = threadIdx.x & 63, col = lane & 31, hf = lane >> 5;
     const int x_at = chunk_unit(wm * MI * 32 + col, hf);
     const int w_at = BM * 128 + chunk_unit(wn * NI * 32 + col, hf);
+    auto loads = [&](int slot, int d, int from, int to) {
+      #pragma unroll
+      for (int i = 0; i < LOADS; ++i)
+        if (i >= from && i < to) stage(slot, d, i);
+    };
     #pragma unroll
     for (int n = 0; n < NI; ++n)
       #pragma unroll
       for (int m = 0; m < MI; ++m) acc[n][m] = f32x16_t(0.f);
     #pragma unroll
     for (int d = 0; d < STAGES; ++d)
-      if (d < stages) stage(d, d);
+      if (d < stages) loads(d, d, 0, LOADS);
     if (stages >= STAGES)
       asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier"
                    ::"n"((STAGES - 1) * LOADS) : "memory");
@@ -114,13 +130,21 @@ struct TileLoop {
     int slot = 0;
     for (int d = 0; d < stages; ++d) {
       const char* base = lds + slot * STAGE;
-      if (live) {
+      // SPREAD: the slot of stage d - 1
+      const int last = slot == 0 ? STAGES - 1 : slot - 1;
+      const bool more = SPREAD && d > 0 && d - 1 + STAGES < stages;
+      if (SPREAD || live) {
         #pragma unroll
         for (int k = 0; k < STEPS - 1; ++k) {
-          read(f[(k + 1) & 1], base, x_at, w_at, k + 1);
-          __builtin_amdgcn_sched_barrier(0);
-          products(f[k & 1]);
-          __builtin_amdgcn_sched_barrier(0);
+          if (live) read(f[(k + 1) & 1], base, x_at, w_at, k + 1);
+          if (more)
+            loads(last, d - 1 + STAGES, LOADS * k / (STEPS - 1),
+                  LOADS * (k + 1) / (STEPS - 1));
+          if (live) {
+            __builtin_amdgcn_sched_barrier(0);
+            products(f[k & 1]);
+            __builtin_amdgcn_sched_barrier(0);
+          }
         }
       }
       const int next = slot == STAGES - 1 ? 0 : slot + 1;
@@ -134,7 +158,7 @@ struct TileLoop {
           asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier"
                        ::: "memory");
         if (live) read(f[0], lds + next * STAGE, x_at, w_at, 0);
-        if (d + STAGES < stages) stage(slot, d + STAGES);
+        if (!SPREAD && d + STAGES < stages) loads(slot, d + STAGES, 0, LOADS);
         __builtin_amdgcn_sched_barrier(0);
       }
       if (live) products(f[1]);
