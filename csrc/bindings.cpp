@@ -518,7 +518,7 @@ void gemm_split(c10::optional<torch::Tensor> out, torch::Tensor x,
                   : ((bm == 64 || bm == 128) && (bn == 64 || bn == 128)) ||
                         (bm == 256 && bn == 128), "gemm_split: tile");
   if (gated)      // 32 bits of offset reach the up rows
-    TORCH_CHECK(!fp8 && splits == 1 && bm <= 128 && N % 8 == 0 &&
+    TORCH_CHECK(!fp8 && splits == 1 && N % 8 == 0 &&
                     (N / 2 + 128) * w.stride(0) < (1l << 31),
                 "gemm_split: gated");
   TORCH_CHECK(splits >= 1 && splits <= 8 && splits <= K / chunk,

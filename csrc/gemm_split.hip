@@ -20,7 +20,8 @@
 //   2048 x 7168   32 rows 19 11, 96 19 14, 192 25 19, 256 25 20, 512 32 29
 //   5120 x 8192   32 rows 25 23, 96 37 26, 192 61 36, 256 72 39
 // silu(gate) * up of the halves, product and activation and here: 28672 x 4096 17
-//   rows 47 41, 64 57 41, 128 59 48; 14336 x 2048 32 rows 19 13, 256 32 23
+//   rows 47 41, 64 57 41, 128 59 48; 14336 x 2048 32 rows 19 13, 256 32 23; in
+//   tiles of 256 x 128 28672 x 4096 256 rows 79 69, 14336 x 1664 512 36 27
 // e4m3, with the norm that adds up the parts: 4096 x 14336 16 rows 27 19, 64 31
 // 21, 128 44 28; 4096 x 4096 16 rows 15 12, 128 18 15; without: 28672 x 4096 16
 // rows 34 24, 64 31 26 (29 in tiles of 64 x 64, of which 448 are not one wave);
@@ -190,7 +191,7 @@ __global__ __launch_bounds__(256) void gemm_sum_kernel(
 // aligned; splits 1 to 8, at most one a 256 bytes, part with more than one.
 // Without out the parts are left for the norm that adds them up.  gated, of
 // bfloat16 without parts: out = silu(gate) * up of the halves of w, whose rows
-// are a multiple of 8, in tiles of up to 128 rows.
+// are a multiple of 8.
 void launch_gemm_split(bf16* out, float* part, const void* x, const void* w,
                        const float* x_scale, const float* w_scale, int M,
                        int N, int K, long xs, long ws, int bm, int bn,
@@ -226,7 +227,7 @@ void launch_gemm_split(bf16* out, float* part, const void* x, const void* w,
     else
       RUN(64, 64, 2, 2, 4, 2, true, false)
   } else if (bm == 256)
-    RUN(256, 128, 4, 2, 3, 1, false, false)
+    KINDS(256, 128, 4, 2, 3, 1)
   else if (bm == 128 && bn == 128)
     KINDS(128, 128, 2, 4, 4, 1)
   else if (bm == 128)

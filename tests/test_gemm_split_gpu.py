@@ -118,6 +118,29 @@ def test_gated_linear(M, N, K):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [
+    (1, 16, 128), (129, 136, 256), (256, 1040, 384), (257, 240, 512),
+    (512, 264, 640), (300, 4112, 128)])
+def test_gated_in_tiles_of_256_rows(M, N, K):
+    """One to five stages of the ring; the bound as in test_gated."""
+    test_gated(M, N, K, 256, 128)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [
+    (129, 16528, 256), (256, 32768, 640), (257, 16384, 128), (512, 6144, 1024)])
+def test_gated_wave(M, N, K):
+    assert ops._gated_tile(M, N, K) is None
+    assert ops._gated_wave(M, N, K) == (256, 128)
+    assert ops._gated_wave(M, 32768 + 16, 4608) is None
+    g = torch.Generator().manual_seed(M)
+    x = torch.randn(M, K, generator=g).bfloat16().to(DEV)
+    w = (torch.randn(N, K, generator=g) * K ** -0.5).bfloat16().to(DEV)
+    out, want = ops.gated_linear(x, w), ops.silu_mul(x @ w.t())
+    assert (out.float() - want.float()).norm() <= 2.0 ** -7 * want.float().norm()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("kind,tiles", [
     ("bf16", [(64, 64), (64, 128), (128, 64)]),
     ("gated", [(64, 64), (64, 128), (128, 64), (128, 128)]),
