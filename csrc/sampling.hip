@@ -70,22 +70,26 @@ __global__ __launch_bounds__(256) void greedy_sample_kernel(
 // What bounds it: vector instructions on every value, about 20 for a weight, and
 // the chains of steps that a row's workgroup takes one after the other.  So a row
 // is divided into slices where there are few rows (below): 64 rows of 128256 are
-// 256 workgroups, 7 us for the largest values, 12 with the weights, and a second
-// kernel of 2 (greedy) to 13 us (a share).  8 values are looked at together where
-// that decides about all of them.  Where few values stay, and next-token logits
-// have a few dozen that matter, they are listed and the rest is done on the list,
-// up to 8 threads a value.  Otherwise no sort either: one histogram of counts and
-// weights over 2048 equal steps between the largest and the smallest logit finds
-// the step where the wanted count or share is reached, and ranks the few values
-// in it exactly (or divides that step again).  Equal steps of the logit, and not
-// digits of its bit pattern, because next-token logits fill few exponents: 64
-// lanes that add to the same few counters in LDS would go one by one.
+// 256 workgroups, which have the largest values after 2.5 us and the weights after
+// 4, and 5 us later a second kernel of 1 (greedy) to 9 us (a share).  Lanes are
+// combined by DPP, and what the 16 waves found by 16 lanes: with shuffles, and with
+// every lane adding up 16 values, a mix of options took 24.3 us, so 21.9.  8 values
+// are looked at together where that decides about all of them.  Where few values
+// stay, and next-token logits have a few dozen that matter, they are listed and the
+// rest is done on the list, up to 8 threads a value; n values take n^2 steps, so a
+// share is looked for among 64 first (21.9 -> 19.7 us), then among 128.  Otherwise
+// no sort either: one histogram of counts and weights over 2048 equal steps between
+// the largest and the smallest logit finds the step where the wanted count or share
+// is reached, and ranks the few values in it exactly (or divides that step again).
+// Equal steps of the logit, and not digits of its bit pattern, because next-token
+// logits fill few exponents: 64 lanes that add to the same few counters in LDS would
+// go one by one.
 //
 // 64 rows of 128256, 48 values far above the others, us with a workgroup a row
-// and now, rows in cache (from memory 2 to 3 more): temperature 36 16, top_p 0.9
-// 43 24, top_k 50 24 15, greedy 9.4 9.0; a mix 42 24, where the library's sorts,
+// and now, rows in cache (from memory 2 to 3 more): temperature 36 14, top_p 0.9
+// 43 20, top_k 50 24 13, greedy 9.4 7.4; a mix 42 20, where the library's sorts,
 // scans and selections took 2625.  Normal logits, whose share is thousands of
-// values, 137 129.  A call that is waited for and not captured 60 44.
+// values, 137 115.  A call that is waited for and not captured 60 36.
 //
 // Weights are 2^-40 fixed point relative to the largest (of the row or of the
 // slice), so sums within a row or a slice are exact; slices are brought to the
@@ -139,15 +143,57 @@ DEV float smallest(const float* x) {
                fminf(fminf(x[4], x[5]), fminf(x[6], x[7])));
 }
 
-template <typename I> DEV I wave_scan(I x) {      // inclusive
-  const int lane = threadIdx.x & 63;
-  #pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const I v = __shfl_up(x, o);
-    if (lane >= o) x += v;
+// Combinations over lanes by DPP, which takes a few cycles a step where a shuffle
+// goes through LDS.  x of another lane, or `none` where CTRL and the rows of
+// ROWS have no such lane:
+template <int CTRL, int ROWS, typename I> DEV I from_lane(I x, I none) {
+  if constexpr (sizeof(I) == 8) {
+    const u64 a = __builtin_bit_cast(u64, x), b = __builtin_bit_cast(u64, none);
+    const u64 lo = from_lane<CTRL, ROWS>((unsigned)a, (unsigned)b);
+    const u64 hi = from_lane<CTRL, ROWS>((unsigned)(a >> 32),
+                                         (unsigned)(b >> 32));
+    return __builtin_bit_cast(I, hi << 32 | lo);
+  } else {
+    return __builtin_bit_cast(I, __builtin_amdgcn_update_dpp(
+        __builtin_bit_cast(int, none), __builtin_bit_cast(int, x), CTRL, ROWS,
+        0xf, false));
   }
-  return x;
 }
+// f over the lanes of 16 up to this one: row_shr by 1, 2, 4 and 8
+template <typename I, typename F> DEV I row_scan(I x, I none, F f) {
+  x = f(x, from_lane<0x111, 0xf>(x, none));
+  x = f(x, from_lane<0x112, 0xf>(x, none));
+  x = f(x, from_lane<0x114, 0xf>(x, none));
+  return f(x, from_lane<0x118, 0xf>(x, none));
+}
+// f over the lanes up to this one, then row_bcast of lanes 15 and 31
+template <typename I, typename F> DEV I wave_scan(I x, I none, F f) {
+  x = row_scan(x, none, f);
+  x = f(x, from_lane<0x142, 0xa>(x, none));
+  return f(x, from_lane<0x143, 0xc>(x, none));
+}
+template <typename I> DEV I wave_scan(I x) {      // inclusive sums
+  return wave_scan(x, I(0), [](I a, I b) { return a + b; });
+}
+template <typename I> DEV I lane_of(I x, int lane) {       // uniform
+  if constexpr (sizeof(I) == 8) {
+    const u64 a = __builtin_bit_cast(u64, x);
+    const u64 lo = (unsigned)__builtin_amdgcn_readlane((int)a, lane);
+    const u64 hi = (unsigned)__builtin_amdgcn_readlane((int)(a >> 32), lane);
+    return __builtin_bit_cast(I, hi << 32 | lo);
+  } else {
+    return __builtin_bit_cast(
+        I, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), lane));
+  }
+}
+// the sum of 16 values in LDS, and of those before `before` of them; all lanes
+template <typename I> DEV I sum_of_16(const I* x, int before, I* sum) {
+  const I upto = row_scan(x[threadIdx.x & 15], I(0),
+                          [](I a, I b) { return a + b; });
+  *sum = lane_of(upto, 15);
+  return before ? lane_of(upto, before - 1) : I(0);
+}
+DEV float min_of(float a, float b) { return fminf(a, b); }
 
 struct alignas(16) Entry {        // one LDS load
   u64 key, mass;
@@ -457,13 +503,10 @@ DEV void reach(Scratch& s, const R& row, const Weight& w, float lo, float hi,
 }
 
 DEV u64 sum_of_all(Scratch& s, u64 x) {
-  #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o);
-  if ((threadIdx.x & 63) == 0) s.wave_mass[threadIdx.x >> 6] = x;
+  x = wave_scan(x);
+  if ((threadIdx.x & 63) == 63) s.wave_mass[threadIdx.x >> 6] = x;
   __syncthreads();
-  x = 0;
-  #pragma unroll
-  for (int v = 0; v < 16; ++v) x += s.wave_mass[v];
+  sum_of_16(s.wave_mass, 0, &x);
   return x;
 }
 
@@ -549,7 +592,7 @@ DEV bool draw_from_list(Scratch& s, const Weight& w, int vocab, int k, float p,
 template <typename R>
 DEV bool draw_from_few(Scratch& s, const R& row, const Weight& w, float own,
                        int k, float p, float u, u64* all, int* drawn) {
-  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+  const int tid = threadIdx.x;
   const int want_n = k > 0 ? k : FEW;
   const unsigned key = ordered(own);
   unsigned prefix = 0;            // 16 bits are close enough
@@ -578,11 +621,7 @@ DEV bool draw_from_few(Scratch& s, const R& row, const Weight& w, float own,
           }
         }
   });
-  z = wave_scan(z);
-  if (lane == 63) s.wave_mass[wid] = z;
-  __syncthreads();
-  z = 0;
-  for (int v = 0; v < 16; ++v) z += s.wave_mass[v];
+  z = sum_of_all(s, z);
   *all = z;
   return draw_from_list(s, w, row.vocab, k, p, u, z, drawn);
 }
@@ -591,31 +630,18 @@ DEV bool draw_from_few(Scratch& s, const R& row, const Weight& w, float own,
 // that hold it first, and the smallest value mn.
 DEV void best_of_all(Scratch& s, float& mx, int& at, float& mn) {
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    const float x = __shfl_xor(mx, o);
-    const int i = __shfl_xor(at, o);
-    if (x > mx || (x == mx && i < at)) {
-      mx = x;
-      at = i;
-    }
-    mn = fminf(mn, __shfl_xor(mn, o));
-  }
-  if (lane == 0) {
-    s.list[wid] = mx;
-    s.list[16 + wid] = mn;
-    s.count[wid] = at;
+  const auto larger = [](u64 a, u64 b) { return a > b ? a : b; };
+  u64 key = wave_scan((u64)ordered(mx + 0.f) << 32 | (unsigned)~at, u64(0), larger);
+  mn = wave_scan(mn, INFINITY, min_of);
+  if (lane == 63) {
+    s.wave_mass[wid] = key;
+    s.list[wid] = mn;
   }
   __syncthreads();
-  for (int v = 0; v < 16; ++v) {
-    const float x = s.list[v];
-    const int i = s.count[v];
-    if (x > mx || (x == mx && i < at)) {
-      mx = x;
-      at = i;
-    }
-    mn = fminf(mn, s.list[16 + v]);
-  }
+  key = lane_of(row_scan(s.wave_mass[lane & 15], u64(0), larger), 15);
+  mn = lane_of(row_scan(s.list[lane & 15], INFINITY, min_of), 15);
+  mx = from_ordered((unsigned)(key >> 32));
+  at = (int)~(unsigned)key;
   __syncthreads();
 }
 
@@ -839,9 +865,8 @@ __global__ __launch_bounds__(NT) void sample_slice_kernel(
     if (w.any(largest(x)))
       #pragma unroll
       for (int i = 0; i < 8; ++i) z += w.always(x[i]);
-    #pragma unroll
-    for (int i = 32; i > 0; i >>= 1) z += __shfl_xor(z, i);
-    if (lane == 0) mine.mass[q * 16 + wid] = z;
+    z = wave_scan(z);
+    if (lane == 63) mine.mass[q * 16 + wid] = z;
   }
 }
 
@@ -874,17 +899,12 @@ __global__ __launch_bounds__(NT) void sample_slices_kernel(
   const Options o = options_of(b, temperature, top_p, top_k, uniform, vocab);
   if (tid == 0) s.n = 0;
   s.count[tid] = 0;
-  #pragma unroll
-  for (int x = 1; x < 16; x <<= 1) {
-    const float m = __shfl_xor(mx, x);
-    const int i = __shfl_xor(at, x);
-    if (m > mx || (m == mx && i < at)) {
-      mx = m;
-      at = i;
-    }
-    mn = fminf(mn, __shfl_xor(mn, x));
-  }
-  mn = fminf(mn, mx);
+  const u64 best = lane_of(
+      row_scan((u64)ordered(mx + 0.f) << 32 | (unsigned)~at, u64(0),
+               [](u64 a, u64 b) { return a > b ? a : b; }), 15);
+  mx = from_ordered((unsigned)(best >> 32));
+  at = (int)~(unsigned)best;
+  mn = fminf(lane_of(row_scan(mn, INFINITY, min_of), 15), mx);
   if (o.t == 0.f || !(mx >= -FLT_MAX)) {
     if (tid == 0)
       out[b] = greedy_index(row.p, mx, at, vocab, o.t == 0.f ? 0 : vocab - 1);
@@ -905,11 +925,7 @@ __global__ __launch_bounds__(NT) void sample_slices_kernel(
     const u64 upto = wave_scan(mass);
     if (lane == 63) s.wave_mass[wid] = upto;
     __syncthreads();
-    u64 before = 0;
-    for (int v = 0; v < 16; ++v) {
-      if (v == wid) before = z;
-      z += s.wave_mass[v];
-    }
+    const u64 before = sum_of_16(s.wave_mass, wid, &z);
     if (!(o.p < 1.f)) {
       // the token is in the chunk where the running sum passes the target;
       // there sums are those of the slice's own weights again
@@ -974,8 +990,9 @@ __global__ __launch_bounds__(NT) void sample_slices_kernel(
   }
   __syncthreads();
   int drawn;
-  bool done = o.k ? o.k <= LIST / 2 : s.n <= 2 * FEW;
-  if (done) {
+  bool done = false;
+  const bool few = o.k ? o.k <= LIST / 2 : s.n <= 2 * FEW;
+  for (unsigned want = o.k ? o.k : FEW / 2; few && !done; want = FEW) {
     const unsigned upto = wave_scan(s.count[tid]);
     if (lane == 63) s.wave_count[wid] = upto;
     if (tid == 0) {
@@ -983,9 +1000,8 @@ __global__ __launch_bounds__(NT) void sample_slices_kernel(
       s.step = NT + 1;
     }
     __syncthreads();
-    unsigned before = 0;
-    for (int v = 0; v < wid; ++v) before += s.wave_count[v];
-    const unsigned want = o.k ? o.k : FEW;
+    unsigned all;
+    const unsigned before = sum_of_16(s.wave_count, wid, &all);
     if (before + upto >= want && before + upto - s.count[tid] < want)
       s.step = tid + 1;
     __syncthreads();
@@ -1029,6 +1045,7 @@ __global__ __launch_bounds__(NT) void sample_slices_kernel(
       done = draw_from_list(s, w, vocab, o.k, o.p, o.uniform, z, &drawn);
     }
     __syncthreads();
+    if (o.k || want == FEW || units > LIST) break;
   }
   if (!done)
     drawn = draw_from_row(s, row, w, mn, o.hi, o.k, o.p, o.uniform, z);

@@ -214,6 +214,39 @@ def test_rows_in_slices(vocab, rows):
             assert out[b] == int(row.argmax())
 
 
+@pytest.mark.parametrize("vocab", [8192, 50257, 128256])
+def test_shares_of_more_values_than_are_listed_first(vocab):
+    """Divided rows list 64 values for a share, then 128: shares of 1 to 200 equal
+    or almost equal values, far above the others, at every part of the draw."""
+    g = torch.Generator().manual_seed(vocab)
+    counts = [1, 60, 63, 64, 65, 66, 80, 100, 127, 128, 129, 130, 200]
+    pick = [(n, same, (i + 0.5) / 7) for n in counts for same in (0, 1)
+            for i in range(7)]
+    x = torch.randn(len(pick), vocab, generator=g) - 30
+    for b, (n, same, _) in enumerate(pick):
+        at = torch.randperm(vocab, generator=g)[:n]
+        x[b, at] = 4.0 if same else 4 + torch.rand(n, generator=g)
+    x = x.bfloat16()
+    t, p = torch.ones(len(pick)), torch.full((len(pick),), 0.98)
+    u = torch.tensor([v for _, _, v in pick])
+    k = torch.zeros(len(pick), dtype=torch.int32)
+    out = ops.sample(*(a.to(DEV) for a in (x, t, p, k, u))).tolist()
+    for b, (n, same, _) in enumerate(pick):
+        ok, _ = _allowed(x[b].float(), 1.0, 0.98, 0, float(u[b]))
+        assert ok[out[b]], (n, same, float(u[b]))
+
+
+@pytest.mark.parametrize("vocab", [1000, 32768])
+def test_zeros_of_either_sign_are_equal(vocab):
+    """The first of the largest values is -0."""
+    x = torch.full((2, vocab), -1.0)
+    x[0, [vocab // 3, vocab - 1]] = torch.tensor([-0.0, 0.0])
+    x[1, [vocab // 5, vocab // 5 + 1]] = torch.tensor([-0.0, 0.0])
+    opt = torch.zeros(2, device=DEV)
+    out = ops.sample(x.bfloat16().to(DEV), opt, opt + 1, opt.int(), opt + 0.5)
+    assert out.tolist() == [vocab // 3, vocab // 5]
+
+
 def _few_above(kind, vocab):
     """Rows whose top_k-th largest value is the smallest one, or nearly."""
     x = torch.full((vocab,), 1.0)
