@@ -387,13 +387,30 @@ def _split_gemm(M: int, N: int, K: int):
     x 8192, 288 rows 34 38; 3136 x 7680, 257 rows 32 37), 129 to 144 rows of
     more than 6528 outputs (7168 x 7168 42 45; 6400 x 6400 at 0.68), and up to
     32 rows where those of w lie a multiple of 32 KB apart (4096 x 16384 31
-    42).  Narrow tiles where K is short and they fill as many units."""
+    42).  Narrow tiles where K is short and they fill as many units.
+    129 to 256 rows in one tile, which loads three quarters of what two do, where
+    that saves more than twice the parts cost: 120 sizes of K from 4608 to 20480,
+    over what was there 0.86 with 4 or 5 parts (256 of 5648 x 7552 45 37, 192 of 7152
+    x 5376 33 31), 0.92 with 6 or 7 of at least 8960 columns (189 of 4616 x 14464 52
+    48) and with 8 of 15360 and up to 4 in tiles of 128, 0.96 to 1.15 else (256 of
+    4096 x 14336 in a decode step even); with 2 or 3, against the library, 0.82 (256
+    of 10112 x 4480 51 39, of 11168 x 7424 85 67; 163 of 15136 x 6656 65 65).  All of
+    these in 50 other sizes, with x from memory, 0.83, the worst 1.03 (172 of 10576 x
+    4352)."""
     if not 16 < M <= 512 or K < (4096 if M <= 256 else 7168) or K % 128 \
             or N % 4 or N * K < 14 << 20:
         return None
     if M <= 32 and K % 16384 == 0 and N >= 3072 \
             or 128 < M <= 144 and N > 6528 and K <= 16384:
         return None
+
+    nt = -(-N // 128)
+    if 128 < M <= 256 and nt <= 128:
+        tall = min(8, 256 // nt)
+        if K >= (6784 if tall == 2 else 4096 if tall == 3 else
+                 4608 if tall <= 5 else 8960 if tall <= 7 else 15360) \
+                and 128 // nt <= 4:
+            return 256, 128, tall
 
     def parts(bm, bn):
         mt, nt = -(-M // bm), -(-N // bn)
@@ -432,7 +449,8 @@ def _summed_gemm(M: int, N: int, K: int):
     23 14).  257 to 512 rows with K from 5120 on, or 4096 in tiles of 128 rows: 0.92
     in 40 (480 of 4096 x 4096 33 32, 395 of 5120 x 7168 60 51, 298 of 3968 x 6144 40
     35, 454 of 4224 x 11008 93 68).  Two parts of tall tiles are even (452 of 5504 x
-    8192 65 70, 379 of 7168 x 14336 119 116)."""
+    8192 65 70, 379 of 7168 x 14336 119 116) but with long columns and full tiles, 0.86
+    in 8 of 8704 and more (512 of 6504 x 10496 100 84, 454 of 6336 x 8192 66 67)."""
     if K % 128 or N % 8 or not 0 < N <= 8192:
         return None
     if M <= 16 and K >= 5120 and N * K >= 2 << 20:
@@ -448,7 +466,7 @@ def _summed_gemm(M: int, N: int, K: int):
         if wide >= 2 and (M > 384 and tall < 3 or K < 5120 or
                           M <= 384 and mt * wide >= 1.6 * tall):
             return 128, 128, min(8, wide)
-        if tall >= 3 and K >= 5120:
+        if tall >= (2 if K >= 8704 else 3) and K >= 5120:
             return 256, 128, tall
     return None
 

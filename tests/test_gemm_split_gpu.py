@@ -299,6 +299,33 @@ def test_rule_of_few_rows_of_long_columns():
                 assert -(-N // 64) * rule[2] <= 256 and 3 <= rule[2] <= K // 512
 
 
+def test_rule_of_one_tile_of_rows():
+    """129 to 256 rows: one tile of 256 from as many columns on as pay for the
+    parts, which fill the units; not where narrower ones have five parts."""
+    for M, N, K, rule in [
+            (256, 4096, 14336, (128, 128, 4)), (129, 4096, 15360, (256, 128, 8)),
+            (129, 4104, 8832, (128, 128, 3)), (256, 3200, 16384, (128, 128, 5)),
+            (200, 4104, 8960, (256, 128, 7)), (200, 8192, 4608, (256, 128, 4)),
+            (200, 8192, 4480, (128, 64, 1)), (200, 10880, 4096, (256, 128, 3)),
+            (200, 10888, 6656, None), (200, 16384, 6784, (256, 128, 2)),
+            (200, 16388, 6784, None), (257, 16384, 8192, None)]:
+        assert ops._split_gemm(M, N, K) == rule, (M, N, K)
+    assert ops._summed_gemm(512, 6504, 8704) == (256, 128, 2)
+    assert ops._summed_gemm(512, 6504, 8576) is None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(129, 4096, 15360), (256, 16384, 6784),
+                                   (255, 4104, 9088), (200, 8196, 4096),
+                                   (145, 8188, 4608)])
+def test_one_tile_of_rows(M, N, K):
+    g = torch.Generator().manual_seed(M)
+    x = torch.randn(M, K, generator=g).bfloat16().to(DEV)
+    w = torch.randn(N, K, generator=g).bfloat16().to(DEV)
+    assert ops._route(M, N, K, False)[:2] == (256, 128)
+    _check(ops.linear(x, w), x, w)
+
+
 def test_rule_leaves_no_workgroup_for_a_second_wave():
     """Workgroups go to 8 dies of 32 units in turn, those of one tile of w to
     the same."""
