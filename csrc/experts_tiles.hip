@@ -18,6 +18,8 @@
 // layer (8 experts, 14336 x 4096, 2.8 GB), us with 256-row tiles, row tiles
 // and here: 16 choices an expert 821 617 473, 48 831 792 487, 128 943 869 719,
 // 500 2355 2100 1650.  32 experts of 1024 x 2048, 62 choices 277 172 96.
+#include <type_traits>
+
 #include "tile_loop.h"
 
 namespace {
@@ -106,15 +108,17 @@ void experts_tiles_kernel(Tiles a) {
     const int r = (wid * LW + j) * 8 + lr;
     w_off[j] = w_row(r) * row_bytes + column(r);
   }
-  auto load = [&](char* l, const RowLoads& rows, const char* base, long off,
-                  int d) {
+  auto load = [&](auto once, char* l, const RowLoads& rows, const char* base,
+                  long off, int d) {
+    // several tiles of 256 rows take the same weights, one after the other
+    constexpr int AUX = decltype(once)::value && BM < 256 ? ONCE : 0;
     if constexpr (FAR)
       __builtin_amdgcn_global_load_lds(
           (__attribute__((address_space(1))) const unsigned*)(base + off +
                                                               d * 128),
-          (__attribute__((address_space(3))) unsigned*)l, 16, 0, 0);
+          (__attribute__((address_space(3))) unsigned*)l, 16, 0, AUX);
     else
-      rows.to_lds(l, (unsigned)off, d * 128);
+      rows.to_lds<AUX>(l, (unsigned)off, d * 128);
   };
   // Where the weights are the bound workgroups begin at different columns, so
   // that not all of them ask the same channels of memory at once; those of one
@@ -134,10 +138,11 @@ void experts_tiles_kernel(Tiles a) {
     if (d >= stages) d -= stages;
     char* l = lds + slot * Loop::STAGE;
     if (i < LX)
-      load(l + (wid * LX + i) * 1024, x_rows, x0, x_off[i], d);
+      load(std::false_type(), l + (wid * LX + i) * 1024, x_rows, x0, x_off[i],
+           d);
     else
-      load(l + BM * 128 + (wid * LW + i - LX) * 1024, w_rows, w0,
-           w_off[i - LX], d);
+      load(std::true_type(), l + BM * 128 + (wid * LW + i - LX) * 1024, w_rows,
+           w0, w_off[i - LX], d);
   };
   Loop loop;
   loop.run(lds, wm, wn, stages, live, stage);

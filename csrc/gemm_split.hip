@@ -112,8 +112,8 @@ void gemm_split_kernel(Split a) {
                     (d * KC + s) * 128);
     } else {
       const int j = i / KC - LX;
-      w_rows.to_lds(base + BM * 128 + (wid * LW + j) * 1024, w_off[j],
-                    (d * KC + s) * 128);
+      w_rows.to_lds<ONCE>(base + BM * 128 + (wid * LW + j) * 1024, w_off[j],
+                          (d * KC + s) * 128);
     }
   };
   Loop loop;

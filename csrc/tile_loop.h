@@ -17,15 +17,27 @@
 // 4 GB) + `from`, which is uniform, to LDS address l + lane * 16.  Loads by a
 // buffer's address, for the compiler takes those by a global one for flat ones,
 // and then waits for all LDS reads where it needs the oldest.
+//
+// ONCE (non-temporal): rows that no other workgroup reads, or few at the same
+// time, as weights.  A load that waits for memory otherwise holds a line of the
+// unit's cache, of which there are 256, and answers come in order: a unit gets 47
+// GB/s from memory and with this 87, all of them 6.2 TB/s and 7.3.  What is read
+// again, as x by the tiles of all outputs, is slower with it.  us: 64 rows of 28672
+// x 4096 41.4 -> 38.4, 1 of 4096 x 14336 in 4 parts 21.8 -> 19.7, 256 of 28672 x
+// 4096 74 -> 66, 512 of 4096 x 14336 64 -> 61; weights that the memory's cache of
+// 256 MB has from the last time, which a model's layers together leave no room
+// for, 0 to 20 % slower.
+enum { ONCE = 2 };
 struct RowLoads {
   __amdgpu_buffer_rsrc_t rows;
   DEV explicit RowLoads(const void* base)
       : rows(__builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0,
                                                0xffffffff, 0x00020000)) {}
+  template <int AUX = 0>
   DEV void to_lds(char* l, unsigned at, unsigned from) const {
     __builtin_amdgcn_raw_ptr_buffer_load_lds(
         rows, (__attribute__((address_space(3))) unsigned*)l, 16, at, from, 0,
-        0);
+        AUX);
   }
 };
 
