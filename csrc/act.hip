@@ -4,8 +4,10 @@
 // the HBM stream floor at the MoE shape (172 us vs ~44 us for 352 MB).
 #include "common.h"
 
-// CLAMPED: the clamped unit instead of silu(gate) * up
-template <bool CLAMPED>
+// CLAMPED: the clamped unit instead of silu(gate) * up.  ONCE: x by non-temporal
+// loads, from 160 MB on, which the memory's cache has no room for: us 8192 rows of
+// 28672 124 -> 108, 4096 63 -> 55; 2000 27.9 29.1, 256 6.1 6.6
+template <bool CLAMPED, bool ONCE>
 __global__ __launch_bounds__(256) void silu_mul_kernel(
     bf16* __restrict__ out, const bf16* __restrict__ x, long rows,
     int inter, float limit) {
@@ -16,8 +18,9 @@ __global__ __launch_bounds__(256) void silu_mul_kernel(
   for (int v = blockIdx.x * 256 + threadIdx.x; v < nv;
        v += gridDim.x * 256) {
     const int j = v * 8;
-    bf16x8 g = load_bf16x8(row + j);
-    bf16x8 p = load_bf16x8(row + inter + j);
+    bf16x8 g = ONCE ? once_bf16x8(row + j) : load_bf16x8(row + j);
+    bf16x8 p = ONCE ? once_bf16x8(row + inter + j)
+                    : load_bf16x8(row + inter + j);
     bf16x8 o;
     #pragma unroll
     for (int i = 0; i < 8; ++i) {
@@ -42,7 +45,10 @@ static void run_silu_mul(bf16* out, const bf16* x, long rows, int inter,
   const unsigned bx = (unsigned)min((nv + 255) / 256, 32);
   for (long r0 = 0; r0 < rows; r0 += 65535) {
     const long nr = min(rows - r0, (long)65535);
-    silu_mul_kernel<CLAMPED><<<dim3(bx, (unsigned)nr), 256, 0, stream>>>(
+    const auto kernel = rows * inter >= 40l << 20
+                            ? silu_mul_kernel<CLAMPED, true>
+                            : silu_mul_kernel<CLAMPED, false>;
+    kernel<<<dim3(bx, (unsigned)nr), 256, 0, stream>>>(
         out + r0 * inter, x + r0 * 2 * (long)inter, nr, inter, limit);
   }
 }

@@ -38,6 +38,13 @@ DEV bf16x8 load_bf16x8(const bf16* p) {
   return r;
 }
 
+// the same without a place in the caches: what is not read again
+DEV bf16x8 once_bf16x8(const bf16* p) {
+  typedef __attribute__((ext_vector_type(4))) unsigned u4;
+  const u4 v = __builtin_nontemporal_load(reinterpret_cast<const u4*>(p));
+  return bf16x8{uint4{v.x, v.y, v.z, v.w}};
+}
+
 DEV void store_bf16x8(bf16* p, const bf16x8& v) {
   *reinterpret_cast<uint4*>(p) = v.raw;
 }

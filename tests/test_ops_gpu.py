@@ -206,6 +206,17 @@ def test_silu_mul():
     assert torch.allclose(out.float().cpu(), ref, atol=2e-2, rtol=2e-2)
 
 
+def test_silu_mul_of_many_rows():
+    """Beyond 40 M outputs its loads are others; a row's bits are not."""
+    rows, inter = 2999, 13992
+    g = torch.Generator(device=DEV).manual_seed(1)
+    x = torch.randn(rows, 2 * inter, generator=g, device=DEV).bfloat16()
+    assert rows * inter >= 40 << 20
+    out = ops.silu_mul(x)
+    for a in range(0, rows, 1000):
+        assert torch.equal(out[a:a + 1000], ops.silu_mul(x[a:a + 1000]))
+
+
 def test_greedy_sample():
     torch.manual_seed(0)
     logits = _randn_bf16(64, 128256)
