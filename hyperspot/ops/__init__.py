@@ -314,6 +314,42 @@ def _wave_gemm(M: int, N: int, K: int):
     return None
 
 
+def _full(tiles: int) -> float:
+    """How full the units are over all waves of these."""
+    return tiles / (-(-tiles // 256) * 256)
+
+
+def _waves_gemm(M: int, N: int, K: int):
+    """Tiles of 64 rows by 64 or 128 outputs where they are half a wave or more of
+    one workgroup a compute unit, or several waves, against the kernel of few rows
+    and the library.  130 random sizes, time over what was there: 9153 to 11264 and
+    16385 to 22528 outputs 0.85 (4 of 10628 x 3328 20 17; 16 of 10168 x 4224 34 19; 64
+    of 18736 x 896 15 11; 32 of 10008 x 5120 26 27); several waves and up to 16 rows
+    0.87, wide tiles but where narrow ones fill the units better (1 of 128256 x 4096
+    185 163, 2 of 144224 x 2304 132 113, 2 of 49448 x 3456 62 59), 17 to 32 rows 0.85
+    (128256 x 4096 201 172), 33 to 64 with up to 4096 columns 0.80 (64 of 128256 x 4096
+    215 183).  Left are 257 to 384 wide tiles, which are nearly one wave more than
+    needed, and narrow ones that fill no wave either (1.0 to 1.13); few columns for few
+    rows (1 of 100164 x 640 28 30); long ones for many rows (62 of 58064 x 7296 156
+    161)."""
+    if not 1 <= M <= 64 or not 640 <= K <= 16384 or K % 128 or N % 4:
+        return None
+    narrow, wide = -(-N // 64), -(-N // 128)
+    if 144 <= narrow < 176:
+        return 64, 64, 1
+    if 128 < wide < 176:
+        return 64, 128, 1
+    if wide > 384 and (
+            K >= 896 if M <= 16 else
+            wide > 512 or _full(wide) >= 0.78 if M <= 32 else
+            K <= 4096 and wide >= 500 and _full(wide) >= 0.75):
+        return (64, 64, 1) if M <= 16 and _full(narrow) > _full(wide) + 0.08 \
+            else (64, 128, 1)
+    if 256 < wide <= 384 and M <= 16 and K >= 1152 and _full(narrow) >= 0.78:
+        return 64, 64, 1
+    return None
+
+
 @lru_cache(maxsize=1 << 14)
 def _route(M: int, N: int, K: int, parts: bool):
     """How x w^T of these sizes is formed: "rows", (rows, outputs of a tile, parts
@@ -321,7 +357,7 @@ def _route(M: int, N: int, K: int, parts: bool):
     step of small prompts, which is not captured, waits for the host."""
     if K >= 1 << 24:                # the kernels' chunks are counted in 32 bits
         return None
-    wave = _wave_gemm(M, N, K)
+    wave = _wave_gemm(M, N, K) or _waves_gemm(M, N, K)
     if wave is not None:
         return wave
     if _rows_gemm_sizes(M, N, K) and _native().gemm_rows_fits(M, K):

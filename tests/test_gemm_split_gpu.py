@@ -299,6 +299,34 @@ def test_rule_of_few_rows_of_long_columns():
                 assert -(-N // 64) * rule[2] <= 256 and 3 <= rule[2] <= K // 512
 
 
+def test_rule_of_several_waves():
+    """Half a wave and more, and several; not nearly empty ones."""
+    for M, N, K, rule in [
+            (1, 9152, 2048, None), (1, 9153 + 3, 2048, (64, 64, 1)),
+            (64, 11264, 640, None), (64, 11200, 512, None),
+            (1, 16388, 2048, (64, 128, 1)), (64, 22400, 768, (64, 128, 1)),
+            (1, 33000, 2048, None), (1, 45000, 1024, None),
+            (1, 45000, 1152, (64, 64, 1)), (17, 45000, 1152, None),
+            (16, 49156, 896, (64, 128, 1)), (1, 49156, 768, None),
+            (32, 65700, 640, (64, 128, 1)), (1, 69632, 2048, (64, 64, 1)),
+            (32, 49156, 1024, None), (64, 128256, 4096, (64, 128, 1)),
+            (64, 128256, 4224, None), (64, 69632, 1024, None),
+            (65, 128256, 4096, None), (1, 128256, 4100, None)]:
+        assert ops._waves_gemm(M, N, K) == rule, (M, N, K)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [
+    (1, 9156, 640), (64, 11196, 896), (33, 16388, 640), (16, 22396, 768),
+    (3, 45000, 1152), (17, 65668, 640), (64, 75268, 640), (5, 69644, 896)])
+def test_several_waves(M, N, K):
+    g = torch.Generator().manual_seed(M)
+    x = torch.randn(M, K, generator=g).bfloat16().to(DEV)
+    w = torch.randn(N, K, generator=g).bfloat16().to(DEV)
+    assert ops._route(M, N, K, False) == ops._waves_gemm(M, N, K) is not None
+    _check(ops.linear(x, w), x, w)
+
+
 def test_rule_of_one_tile_of_rows():
     """129 to 256 rows: one tile of 256 from as many columns on as pay for the
     parts, which fill the units; not where narrower ones have five parts."""
