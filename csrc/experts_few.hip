@@ -7,16 +7,31 @@
 // What bounds it: the chosen experts' weights, read once.  A sort is a launch
 // that everything waits for, and of a handful of choices every workgroup finds
 // its own: it looks the expert numbers up, 64 a load, and has the choices of one
-// expert as the columns of its products, 16 at a time, however few they are.
-// Weights are the A operand of 16x16x32 products straight from memory; the waves
-// divide K.  Of 16 rows of weights 8 are a gate's and 8 its up row's, so that
-// there are twice as many workgroups as with 16 of each: those of the experts
-// that are chosen spread over the compute units more evenly.
+// expert as the columns of its products, however few they are.  A workgroup has
+// 16 rows of weights, 8 of a gate and 8 of its up row or 16 in turn, so that the
+// chosen experts spread over the compute units evenly; its waves divide K.
+//
+// Weights are the A operand of 16x16x32 products straight from memory, and a
+// load takes whole lines of them, 128 bytes of 8 rows, non-temporal: those do
+// not hold a line of the unit's cache each while they wait, but two loads of
+// half a line would read it twice.  So row i of A is the first half of a line
+// of 8 rows, row 8 + i its second half; the columns of B are the halves of the
+// lines of 8 choices likewise, and of a product the two squares count where the
+// halves are the same.  us, up and down, and with halves of 16 lines a load (not
+// non-temporal; that was slower still):
+//   32 experts of 1024 x 2048, 4 each   1 row 9.0 5.8 (10.1 7.2), 4 rows 22.7
+//     12.9 (25.5 14.4), 16 rows 44 24 (49 27)
+//   8 experts of 14336 x 4096, 2 each   1 row 78 45 (82 59), 4 rows 179 105
+//     (200 125), 10 rows 268 157 (302 177)
+#include <type_traits>
+
 #include "common.h"
 
 namespace {
 
 constexpr int MOST = 384;            // choices
+constexpr int WAVES = 4;             // divide K
+constexpr int STEP = WAVES * 64;     // columns of a step of all waves
 
 struct Few {
   bf16* out;
@@ -27,15 +42,14 @@ struct Few {
   int P, E, N, K, div;
 };
 
-// WAVES divide K
-template <int WAVES, bool UP>
+template <bool UP>
 __global__ __launch_bounds__(WAVES * 64) void experts_few_kernel(Few a) {
   constexpr int OUT = UP ? 8 : 16;
-  __shared__ __attribute__((aligned(16))) float red[WAVES * 256];
+  __shared__ f32x4_t red[WAVES][2][2][16];     // rows of 8, halves, 4 rows of 1
   __shared__ int rows[WAVES][MOST];
   const int lane = threadIdx.x & 63;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int col = lane & 15, gr = lane >> 4;
+  const int col = lane & 7, half = lane >> 3 & 1, gr = lane >> 4;
   const int n0 = blockIdx.x * OUT;
   if (a.place && blockIdx.x == 0 && blockIdx.y == 0)
     for (int p = threadIdx.x; p < a.P; p += WAVES * 64)
@@ -58,46 +72,81 @@ __global__ __launch_bounds__(WAVES * 64) void experts_few_kernel(Few a) {
   }
   if (count == 0) return;
 
-  // rows of weights: gate and up rows in turn, 8 each
-  const int n = n0 + (UP ? (col & 7) + (col & 8 ? a.N : 0) : col);
+  const int at = half * 32 + gr * 8;           // a lane's part of a line
   const bf16* wp =
-      a.w + ((long)e * (UP ? 2 * a.N : a.N) + n) * a.K + gr * 8;
+      a.w + ((long)e * (UP ? 2 * a.N : a.N) + n0 + col) * a.K + at;
+  const long next = (long)(UP ? a.N : 8) * a.K;    // up rows, or 8 rows on
   for (int r0 = 0; r0 < count; r0 += 16) {
-    const bool live = r0 + col < count;
-    const int choice = rows[wid][min(r0 + col, count - 1)];
-    const bf16* xp = a.x + (long)(UP ? choice / a.div : choice) * a.K + gr * 8;
-    f32x4_t acc = f32x4_t(0.f);
-    #pragma unroll 2
-    for (int k0 = wid * 64; k0 < a.K; k0 += WAVES * 64) {
-      short8_t wf[2], xf[2];
-      #pragma unroll
-      for (int s = 0; s < 2; ++s) {
-        wf[s] = *reinterpret_cast<const short8_t*>(wp + k0 + 32 * s);
-        xf[s] = live ? *reinterpret_cast<const short8_t*>(xp + k0 + 32 * s)
-                     : short8_t{};
-      }
-      #pragma unroll
-      for (int s = 0; s < 2; ++s) acc = mfma16(wf[s], xf[s], acc);
+    const bf16* xp[2];                         // of 8 choices and 8 more
+    bool live[2];
+    #pragma unroll
+    for (int g = 0; g < 2; ++g) {
+      const int r = r0 + g * 8 + col;
+      live[g] = r < count;
+      const int choice = rows[wid][min(r, count - 1)];
+      xp[g] = a.x + (long)(UP ? choice / a.div : choice) * a.K + at;
     }
-    if (r0) __syncthreads();
-    *reinterpret_cast<f32x4_t*>(red + (wid * 64 + lane) * 4) = acc;
-    __syncthreads();
-    if (wid || !live || (UP && lane >= 32)) continue;
-    auto total = [&](int l) {
-      f32x4_t s = f32x4_t(0.f);
+    const bool more = r0 + 8 < count;
+    f32x4_t acc[2][2];
+    #pragma unroll
+    for (int i = 0; i < 4; ++i) acc[i >> 1][i & 1] = f32x4_t(0.f);
+    auto products = [&](int k, auto steps) {
+      constexpr int S = decltype(steps)::value;
+      short8_t wf[S][2], xf[S];
+      #pragma unroll
+      for (int u = 0; u < S; ++u)
+        #pragma unroll
+        for (int s = 0; s < 2; ++s)
+          wf[u][s] = __builtin_nontemporal_load(
+              reinterpret_cast<const short8_t*>(wp + s * next + k + u * STEP));
+      auto add = [&](int g) {
+        #pragma unroll
+        for (int u = 0; u < S; ++u)
+          xf[u] = live[g] ? *reinterpret_cast<const short8_t*>(
+                                xp[g] + k + u * STEP)
+                          : short8_t{};
+        #pragma unroll
+        for (int u = 0; u < S; ++u)
+          #pragma unroll
+          for (int s = 0; s < 2; ++s)
+            acc[g][s] = mfma16(wf[u][s], xf[u], acc[g][s]);
+      };
+      add(0);
+      if (more) add(1);
+    };
+    int k = wid * 64;
+    #pragma unroll 1
+    for (; k + STEP < a.K; k += 2 * STEP)
+      products(k, std::integral_constant<int, 2>{});
+    if (k < a.K) products(k, std::integral_constant<int, 1>{});
+
+    #pragma unroll
+    for (int g = 0; g < 2; ++g) {
+      if (g && !more) break;
+      if (r0 || g) __syncthreads();
+      if (half == gr >> 1)
+        #pragma unroll
+        for (int s = 0; s < 2; ++s)
+          red[wid][s][half][(gr & 1) * 8 + col] = acc[g][s];
+      __syncthreads();
+      if (wid) continue;
+      // lane: half, 8 rows, 4 rows of them, choice
+      f32x4_t y = f32x4_t(0.f);
       #pragma unroll
       for (int v = 0; v < WAVES; ++v)
-        s += *reinterpret_cast<const f32x4_t*>(red + (v * 64 + l) * 4);
-      return s;
-    };
-    f32x4_t y = total(lane);
-    if constexpr (UP) {
-      const f32x4_t u = total(lane + 32);
+        y += red[v][lane >> 4 & 1][lane >> 5][lane & 15];
       #pragma unroll
-      for (int j = 0; j < 4; ++j) y[j] = y[j] / (1.f + __expf(-y[j])) * u[j];
+      for (int j = 0; j < 4; ++j) y[j] += __shfl_xor(y[j], 32);
+      if constexpr (UP)
+        #pragma unroll
+        for (int j = 0; j < 4; ++j)
+          y[j] = y[j] / (1.f + __expf(-y[j])) * __shfl_xor(y[j], 16);
+      if (!live[g] || lane >= (UP ? 16 : 32)) continue;
+      *reinterpret_cast<uint2*>(a.out +
+                                (long)rows[0][r0 + g * 8 + col] * a.N + n0 +
+                                (lane >> 3) * 4) =
+          uint2{cvt_pk_bf16(y[0], y[1]), cvt_pk_bf16(y[2], y[3])};
     }
-    *reinterpret_cast<uint2*>(a.out + (long)choice * a.N + n0 + gr * 4) =
-        uint2{cvt_pk_bf16(y[0], y[1]), cvt_pk_bf16(y[2], y[3])};
   }
 }
 
@@ -111,9 +160,7 @@ void launch_experts_few(bool up, bf16* out, int* place, const bf16* x,
   const Few a{out, place, x, w, ids, P, E, N, K, div};
   const int y = P < E ? P : E;
   if (up)
-    experts_few_kernel<8, true>
-        <<<dim3(N / 8, y), 512, 0, stream>>>(a);
+    experts_few_kernel<true><<<dim3(N / 8, y), WAVES * 64, 0, stream>>>(a);
   else
-    experts_few_kernel<4, false>
-        <<<dim3(N / 16, y), 256, 0, stream>>>(a);
+    experts_few_kernel<false><<<dim3(N / 16, y), WAVES * 64, 0, stream>>>(a);
 }
