@@ -17,7 +17,8 @@
 // weights are two thirds of what is loaded), then the products.  Mixtral 8x7B
 // layer (8 experts, 14336 x 4096, 2.8 GB), us with 256-row tiles, row tiles
 // and here: 16 choices an expert 821 617 473, 48 831 792 487, 128 943 869 719,
-// 500 2355 2100 1650.  32 experts of 1024 x 2048, 62 choices 277 172 96.
+// 500 2355 2100 1650.  32 experts of 1024 x 2048, 62 choices 277 172 96.  With
+// weights by non-temporal loads 443, 459, 686 and 1550; 95.
 #include <type_traits>
 
 #include "tile_loop.h"
@@ -48,8 +49,19 @@ void experts_tiles_kernel(Tiles a) {
   static_assert(!(GATED && FP8), "the activation's scale needs whole rows");
   extern __shared__ __attribute__((aligned(16))) char lds[];
   int tile = blockIdx.x / a.nx, nb = blockIdx.x % a.nx;
+  const int tiles = gridDim.x / a.nx;
   const int e = a.expert[tile];
+  const int last = a.expert[max(tile - 1, 0)];
+  const int next = a.expert[min(tile + 1, tiles - 1)];
   if (e < 0) return;
+  // Of 256 rows weights that one tile takes are read once (ONCE), those of several
+  // not; smaller tiles are taken where most experts have one.  us, up and down of 8
+  // experts of 14336 x 4096, 112 choices each 718 -> 660, 160 752 -> 722, of 16 of
+  // 2048 x 4096, 112 226 -> 214; those of several tiles by ONCE 1.1 times slower.
+  // (Tiles of 64 and 128 rows with both ways: two tiles an expert 0.9, one 1.02.)
+  const bool alone =
+      BM < 256 || (((tile == 0) | (last != e)) &
+                   ((tile + 1 == tiles) | (next != e)));
   // The tiles of an expert that take the same weights go to one die together,
   // whose L2 then has them, where an expert has 128 MB of them, half of what the
   // memory's cache holds: later tiles would find them gone.  180 random sizes (2
@@ -61,7 +73,7 @@ void experts_tiles_kernel(Tiles a) {
   // 96).  More than 32 tiles share them without it.
   if (BM == 256 && BN == 256 && a.nx % 8 == 0 &&
       (GATED ? 2 : 1) * a.N * ((long)a.K * ELEM) >= 128l << 20) {
-    const int t = threadIdx.x & 63, tiles = gridDim.x / a.nx;
+    const int t = threadIdx.x & 63;
     const unsigned long back =
         ~__ballot(t <= tile && a.expert[t <= tile ? tile - t : 0] == e);
     const unsigned long on = ~__ballot(
@@ -110,8 +122,7 @@ void experts_tiles_kernel(Tiles a) {
   }
   auto load = [&](auto once, char* l, const RowLoads& rows, const char* base,
                   long off, int d) {
-    // several tiles of 256 rows take the same weights, one after the other
-    constexpr int AUX = decltype(once)::value && BM < 256 ? ONCE : 0;
+    constexpr int AUX = decltype(once)::value ? ONCE : 0;
     if constexpr (FAR)
       __builtin_amdgcn_global_load_lds(
           (__attribute__((address_space(1))) const unsigned*)(base + off +
@@ -133,7 +144,7 @@ void experts_tiles_kernel(Tiles a) {
   const int apart = stages >= (BM == 64 ? 96 : 64) ? 3 : 1;
   const int turn = BM == 256 ? 0 : (nb + e * a.nx) / 8 * apart % stages;
   // load i of a stage: first those of x, then those of w
-  auto stage = [&](int slot, int d, int i) {
+  auto stage = [&](auto once, int slot, int d, int i) {
     d += turn;
     if (d >= stages) d -= stages;
     char* l = lds + slot * Loop::STAGE;
@@ -141,11 +152,19 @@ void experts_tiles_kernel(Tiles a) {
       load(std::false_type(), l + (wid * LX + i) * 1024, x_rows, x0, x_off[i],
            d);
     else
-      load(std::true_type(), l + BM * 128 + (wid * LW + i - LX) * 1024, w_rows,
-           w0, w_off[i - LX], d);
+      load(once, l + BM * 128 + (wid * LW + i - LX) * 1024, w_rows, w0,
+           w_off[i - LX], d);
   };
   Loop loop;
-  loop.run(lds, wm, wn, stages, live, stage);
+  auto run = [&](auto once) {
+    loop.run(lds, wm, wn, stages, live, [&](int slot, int d, int i) {
+      stage(once, slot, d, i);
+    });
+  };
+  if (alone)
+    run(std::true_type());
+  else if constexpr (BM == 256)
+    run(std::false_type());
   auto& acc = loop.acc;
 
   // acc[n][m][r]: weight row (r >> 2) * 8 + hf * 4 + (r & 3) of block n,

@@ -802,15 +802,16 @@ def moe_router(x, router: torch.Tensor, top: int):
 # of the counts: a few rows more than a tile and an expert's weights are read
 # twice, by workgroups that share their compute units with others.  us on an
 # MI355X without a sort, and in tiles of 64, 128, 256, sort included
-#   8 experts of 14336 x 4096   1 row 357 383, 2 rows 420 435, 3 490 471, 5 526
-#     470, 48 - 487 507 626 (52, one of 66 rows, - 604 510), 100 - 783 555 698,
-#     125 - 968 782 719
-#   16 of 2048 x 4096           1 row 109 119, 3 rows 145 148, 5 155 149, 50 -
-#     158 161 206, 125 - 249 232 222
-#   32 of 1024 x 2048           1 row 53 61, 3 rows 75 78, 5 85 80, 37 - 82 90
-#     118, 62 - 107 96 120, 125 - 137 132 129
-#   64 of 1024 x 2048           1 row 101 104, 3 rows 141 142, 4.5 159 143
-MOE_ROWS, MOE_ROWS_64, MOE_ROWS_128 = 2.9, 44, 112
+#   8 experts of 14336 x 4096   1 row 324 345, 2 rows 425 432, 3 423 417, 5 445
+#     430, 48 - 464 500 604 (56, one of 66 rows, - 510 510), 100 - 853 571 653,
+#     112 - 923 625 659, 125 - 1096 815 681
+#   16 of 2048 x 4096           1 row 104 115, 3 rows 137 138, 5 146 135, 48 -
+#     144 156 204, 52 - 166 156, 112 - 281 217 218, 125 - 283 231 219
+#   32 of 1024 x 2048           1 row 56 64, 3 rows 71 75, 5 78 77, 44 - 80 91
+#     119, 48 - 93 91 121, 112 - 146 129 126, 125 - 150 133 129
+#   64 of 1024 x 2048           1 row 94 101, 3 rows 131 129, 5 154 134, 48 -
+#     163 172 228, 112 - 279 222 242, 125 - 309 257 247
+MOE_ROWS, MOE_ROWS_64, MOE_ROWS_128 = 2.9, 48, 112
 
 
 def _moe_tile(T: int, K: int, E: int, least: int) -> int:

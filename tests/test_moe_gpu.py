@@ -64,6 +64,33 @@ def test_experts_around_the_rule(tokens, experts, top, width, inner):
     assert (out - ref).abs().max() <= 2.0 ** -5 * ref.abs().max()
 
 
+@pytest.mark.parametrize("counts", [(256, 257, 0, 1), (1, 512, 200, 255),
+                                    (96, 32, 64, 0), (97, 32, 64, 0)])
+@pytest.mark.parametrize("width,inner", [(256, 32768), (384, 640)])
+def test_tiles_of_one_and_of_several(counts, width, inner):
+    """Experts of one tile, of several and of none, beside each other."""
+    g = torch.Generator().manual_seed(sum(counts))
+    rand = lambda *s: torch.randn(*s, generator=g)
+    experts, tokens = len(counts), sum(counts)
+    assert ops._moe_tile(tokens, 1, experts, 16) == (
+        64 if tokens == 192 else 128 if tokens == 193 else 256)
+    x = rand(tokens, width).bfloat16().to(DEV)
+    w13 = (rand(experts, 2 * inner, width) * width ** -0.5).bfloat16().to(DEV)
+    w2 = (rand(experts, width, inner) * inner ** -0.5).bfloat16().to(DEV)
+    ids = torch.cat([torch.full((n,), e) for e, n in enumerate(counts)])
+    ids = ids[torch.randperm(tokens, generator=g)].int()[:, None].to(DEV)
+    weight = rand(tokens, 1).abs().to(DEV)
+    out = ops.moe_ffn(x, w13, w2, weight, ids).double()
+    ref = torch.zeros_like(out)
+    for e in range(experts):
+        rows = (ids[:, 0] == e).nonzero()[:, 0]
+        gate, up = (x[rows].double() @ w13[e].double().t()).chunk(2, -1)
+        y = torch.nn.functional.silu(gate) * up @ w2[e].double().t()
+        ref[rows] = y * weight[rows].double()
+    assert (out - ref).norm() <= 2.0 ** -7 * ref.norm()
+    assert (out - ref).abs().max() <= 2.0 ** -5 * ref.abs().max()
+
+
 @pytest.mark.parametrize("tokens,experts,top,width,inner", [
     (1, 4, 2, 128, 128), (5, 1, 1, 128, 256), (17, 4, 1, 256, 128),
     (33, 7, 1, 384, 640), (64, 64, 5, 128, 128), (65, 13, 1, 128, 384)])
