@@ -14,16 +14,23 @@
 // (64 rows of 3904 x 384 12.4 -> 5.2 us, of 1760 x 768 12.8 -> 6.2, where each
 // waited for the one before).
 //
-// us, library and here, weights from memory (which gives about 5 TB/s); and of
-// tiles of 16 rows where others are taken:
-//   28672 x 4096  1 row 64 46, 16 rows 66 48    4096 x 4096   1 15 10, 16 15 11
-//   32768 x 4096  1 row 64 52, 16 rows 63 55    32768 x 2048  1 35 28, 32 37 34
-//   12: 6144 x 4096  1 row 14.4 12.0 (14.5), 8 rows 14.4 13.5 (15.8)
-//       3072 x 2048  1 row 11.2  5.5  (6.0), 32 rows 11.7 7.8 (8.2)
-//       5120 x 4096  1 row 14.0 11.4 (13.7)
-//   8: 2048 x 2048   1 row  8.7  4.7  (5.3), 32 rows 8.6 7.1 (7.5)
-//      1536 x 4096   1 row 14.6  6.3  (7.9)
-//      10240 x 4096  1 row 27.1 19.4 (21.0); 14336 x 2048 16.3 13.3 (14.8)
+// A load has whole lines of w, 128 bytes of 8 rows, and is non-temporal: those do
+// not hold a line of the unit's cache each while they wait, but what is left of
+// half a line is read again.  An operand has 64 bytes of 16 rows, so two loads
+// exchange halves.  Against loads of half lines, us: 1 row of 28672 x 4096 46 ->
+// 39, of 4096 x 14336 27.5 -> 23, of 10240 x 4096 19.6 -> 16.5, of 2048 x 2048 4.5
+// -> 4.2, 16 rows of 14336 x 2048 17.1 -> 14.3, 32 of 3072 x 2048 7.5 -> 7.0.
+//
+// us, library and here, weights from memory; and of tiles of 16 rows where others
+// are taken (with loads of half lines):
+//   28672 x 4096  1 row 64 39, 16 rows 66 42    4096 x 4096   1 15  9, 16 15 11
+//   32768 x 4096  1 row 64 44, 16 rows 63 47    32768 x 2048  1 35 25, 32 37 29
+//   12: 6144 x 4096  1 row 14.4 11.4 (14.5), 8 rows 14.4 13.2 (15.8)
+//       3072 x 2048  1 row 11.2  5.0  (6.0), 32 rows 11.7 7.0 (8.2)
+//       5120 x 4096  1 row 14.0 11.0 (13.7)
+//   8: 2048 x 2048   1 row  8.7  4.2  (5.3), 32 rows 8.6 6.4 (7.5)
+//      1536 x 4096   1 row 14.6  5.8  (7.9)
+//      10240 x 4096  1 row 27.1 16.5 (21.0); 14336 x 2048 16.3 12.5 (14.8)
 #include <type_traits>
 
 #include "common.h"
@@ -50,9 +57,22 @@ DEV void to_lds16(const void* g, void* l) {
       (__attribute__((address_space(3))) unsigned*)l, 16, 0, 0);
 }
 
+// Two loads have whole lines of 8 rows each, operands half the lines of 16 rows:
+// lanes 8 to 15 of each 16 exchange theirs with lanes 0 to 7
+DEV void turn(short8_t* f, const short8_t* l) {
+  union V { short8_t s; int d[4]; } a{l[0]}, b{l[1]}, x, y;
+  #pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    x.d[j] = __builtin_amdgcn_update_dpp(a.d[j], b.d[j], 0x128, 15, 0xc, false);
+    y.d[j] = __builtin_amdgcn_update_dpp(b.d[j], a.d[j], 0x128, 15, 0x3, false);
+  }
+  f[0] = x.s;
+  f[1] = y.s;
+}
+
 // CT * 16 rows of x
 template <int CT>
-__global__ __launch_bounds__(WAVES * 64, 2)
+__global__ __launch_bounds__(WAVES * 64, 4)
 void gemm_rows_kernel(Rows a) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   float* red = reinterpret_cast<float*>(smem);
@@ -61,22 +81,26 @@ void gemm_rows_kernel(Rows a) {
   const int lane = threadIdx.x & 63;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 15, gr = lane >> 4;
+  const int at = gr * 16 + (col & 8);          // of a line's 64 columns
   const int tiles = (a.N + a.rows - 1) / a.rows;
   const int batches = (a.K + U * STEP - 1) / (U * STEP);
 
   short8_t wf[U][2], wn[U][2];
   auto fetch = [&](int tile, int batch) {
-    const int n = min(tile * a.rows + col, a.N - 1);
-    const bf16* p = a.w + (long)n * a.ws + gr * 8;
     const int k0 = batch * U * STEP + wid * 64;
+    const bf16* p[2];
+    #pragma unroll
+    for (int s = 0; s < 2; ++s)
+      p[s] = a.w +
+             (long)min(tile * a.rows + s * 8 + (col & 7), a.N - 1) * a.ws + at;
     #pragma unroll
     for (int u = 0; u < U; ++u)
       #pragma unroll
       for (int s = 0; s < 2; ++s) {
-        const int k = k0 + u * STEP + 32 * s;
-        wn[u][s] = k + gr * 8 < a.K && col < a.rows
+        const int k = k0 + u * STEP;
+        wn[u][s] = k + at < a.K && s * 8 + (col & 7) < a.rows
             ? __builtin_nontemporal_load(
-                  reinterpret_cast<const short8_t*>(p + k))
+                  reinterpret_cast<const short8_t*>(p[s] + k))
             : short8_t{};
       }
   };
@@ -110,7 +134,7 @@ void gemm_rows_kernel(Rows a) {
   const short* xr[CT];
   #pragma unroll
   for (int t = 0; t < CT; ++t)       // rows past the end: not stored
-    xr[t] = xl + min(t * 16 + col, a.M - 1) * xp + gr * 8;
+    xr[t] = xl + min(t * 16 + col, a.M - 1) * xp + gr * 16;
   f32x4_t acc[CT];
   #pragma unroll
   for (int t = 0; t < CT; ++t) acc[t] = f32x4_t(0.f);
@@ -118,9 +142,7 @@ void gemm_rows_kernel(Rows a) {
 
   while (tile < tiles) {
     #pragma unroll
-    for (int u = 0; u < U; ++u)
-      #pragma unroll
-      for (int s = 0; s < 2; ++s) wf[u][s] = wn[u][s];
+    for (int u = 0; u < U; ++u) turn(wf[u], wn[u]);
     const int k0 = batch * U * STEP + wid * 64, now = tile;
     if (++batch == batches) {
       batch = 0;
@@ -134,9 +156,9 @@ void gemm_rows_kernel(Rows a) {
         for (int s = 0; s < 2; ++s) {
           // columns past the end: x is zero as w is, for the last ones may
           // hold an infinity
-          const int k = k0 + u * STEP + 32 * s;
+          const int k = k0 + u * STEP + 8 * s;
           if (!whole && k >= a.K) continue;
-          const bool in = whole || k + gr * 8 < a.K;
+          const bool in = whole || k + gr * 16 < a.K;
           #pragma unroll
           for (int t = 0; t < CT; ++t) {
             const short8_t v = *reinterpret_cast<const short8_t*>(
