@@ -233,7 +233,11 @@ __global__ __launch_bounds__(256) void paged_attn_kernel(
 // barrier until the waves' parts are added up.  Decoded rows read their pages once,
 // by non-temporal loads, which do not wait for a place in the unit's cache: a step
 // of 8 layers of 256 rows of about 1000 tokens 3019 -> 2903 us, of 8 of 8000 1249
-// -> 1237, of 32 with 4 kv heads 548 -> 537, 1 of 1000 839 -> 833.
+// -> 1237, of 32 with 4 kv heads 548 -> 537, 1 of 1000 839 -> 833.  Such a load has
+// whole lines: of K 128 bytes of 8 rows, and two exchange halves across lanes (64 of
+// 16 rows, the operands, asked for every line twice): 32 x 4 kv heads of 1000 21.1 ->
+// 19.8 us, 256 x 8 188 -> 182, e4m3 64 x 8 32.2 -> 30.9, but 8 of 8000 in two parts
+// 50.2 50.9; the steps 2918 -> 2888, 1222 -> 1198 and 533 -> 524.
 //
 // us against dot products on the vector units, ragged contexts around the
 // mean: 256 rows x 8 kv heads of 4, 1000 tokens 239 -> 208 (5.0 TB/s), with
@@ -293,6 +297,17 @@ DEV u32x4 widen(unsigned x, unsigned y) {
 // (x, y) by an angle, rounded as in rope_kv_append
 DEV float2 turn(float x, float y, float c, float s) {
   return make_float2(fmaf(x, c, -(y * s)), fmaf(y, c, x * s));
+}
+
+// a: 64 bytes of rows 0 to 7 in lanes 0 to 7 of each 16 and 64 more in the others,
+// b: the same of rows 8 to 15; then a has the first bytes of all rows, b the others
+DEV void exchange_halves(u32x4& a, u32x4& b) {
+  #pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int x = a[j], y = b[j];
+    a[j] = __builtin_amdgcn_update_dpp(x, y, 0x128, 15, 0xc, false);
+    b[j] = __builtin_amdgcn_update_dpp(y, x, 0x128, 15, 0x3, false);
+  }
 }
 
 struct Paged {
@@ -402,7 +417,10 @@ __global__ __launch_bounds__(256, 3) void paged_attn_mfma_kernel(Paged a) {
   float m = -FLT_MAX, l = 0.f;
 
   // matrix row i of half t takes token 8 (i / 4) + 4 t + i % 4
-  const int tok0 = 8 * (col >> 2) + (col & 3);
+  // of a page: rows 0 to 7 are on the first, 8 to 15 on the second; a load has the
+  // whole lines of 8 rows, and two exchange halves
+  const int k_at = (8 * (col >> 2 & 1) + (col & 3)) * (HD * ELEM) +
+                   (col >> 3) * 64 + gr * 16;
   const int blocks = (ctx + BLOCK - 1) / BLOCK;
   const int last_page = (ctx - 1) / ATTN_BS;
   const int step = 4 * split;
@@ -422,14 +440,11 @@ __global__ __launch_bounds__(256, 3) void paged_attn_mfma_kernel(Paged a) {
     const char* kc = static_cast<const char*>(a.k_cache);
     const char* vc = static_cast<const char*>(a.v_cache);
     #pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      const int tok = tok0 + 4 * t;
-      const char* kp = kc + (tok < ATTN_BS ? p0 : p1) +
-                       (tok % ATTN_BS) * (HD * ELEM) + gr * 16;
+    for (int t = 0; t < 2; ++t)
       #pragma unroll
       for (int c = 0; c < (KV8 ? 2 : 4); ++c)
-        kr[t][c] = page(kp + c * 64);
-    }
+        kr[t][c] = page(kc + (c & 1 ? p1 : p0) + k_at + 4 * t * HD * ELEM +
+                        (c >> 1) * 128);
     #pragma unroll
     for (int i = 0; i < (KV8 ? 4 : 8); ++i)
       vr[i] = page(vc + (i < (KV8 ? 2 : 4) ? p0 : p1) +
@@ -501,6 +516,9 @@ __global__ __launch_bounds__(256, 3) void paged_attn_mfma_kernel(Paged a) {
     f32x4_t sc[2];
     #pragma unroll
     for (int t = 0; t < 2; ++t) {
+      #pragma unroll
+      for (int c = 0; c < (KV8 ? 2 : 4); c += 2)
+        exchange_halves(kr[t][c], kr[t][c + 1]);
       sc[t] = f32x4_t(0.f);
       #pragma unroll
       for (int c = 0; c < 4; ++c) {
