@@ -571,8 +571,7 @@ __global__ __launch_bounds__(256, 3) void paged_attn_mfma_kernel(Paged a) {
     }
     #pragma unroll
     for (int j = 0; j < 8; ++j) mx = fmaxf(mx, p[j]);
-    mx = fmaxf(mx, __shfl_xor(mx, 16));
-    mx = fmaxf(mx, __shfl_xor(mx, 32));
+    mx = reduce_32(reduce_16(mx, MaxOf()), MaxOf());
     if (__any(mx > m + GROW)) {
       const float top = fmaxf(m, mx);
       const float alpha = m == -FLT_MAX ? 0.f : exp2_fast(m - top);
@@ -601,8 +600,7 @@ __global__ __launch_bounds__(256, 3) void paged_attn_mfma_kernel(Paged a) {
       for (int n = 0; n < 3; ++n) acc[e] = mfma16(vf.v, part[n], acc[e]);
     }
   }
-  l += __shfl_xor(l, 16);
-  l += __shfl_xor(l, 32);
+  l = reduce_32(reduce_16(l, SumOf()), SumOf());
   __syncthreads();
   float* comb = reinterpret_cast<float*>(v_lds);     // [4][group][HD]
   if (gr == 0) {

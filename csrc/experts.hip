@@ -82,16 +82,29 @@ DEV void route_token(const Route& r, const float* z, int* id, float* weight) {
         best = v[i];
         at = lane + 64 * i;
       }
-    #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-      const float b = __shfl_xor(best, o);
-      const int a = __shfl_xor(at, o);
+    auto better = [&](unsigned v, int a) {
+      const float b = __uint_as_float(v);
       if (a != INT_MAX &&
           (at == INT_MAX || b > best || (b == best && a < at))) {
         best = b;
         at = a;
       }
-    }
+    };
+    auto swapped = [&](auto v, auto a) {       // both lanes' in both
+      best = __uint_as_float(v[0]);
+      at = a[0];
+      better(v[1], a[1]);
+    };
+    unsigned u = __float_as_uint(best);
+    swapped(__builtin_amdgcn_permlane32_swap(u, u, false, false),
+            __builtin_amdgcn_permlane32_swap(at, at, false, false));
+    u = __float_as_uint(best);
+    swapped(__builtin_amdgcn_permlane16_swap(u, u, false, false),
+            __builtin_amdgcn_permlane16_swap(at, at, false, false));
+    better(row_turned<8>(__float_as_uint(best)), row_turned<8>(at));
+    better(row_turned<4>(__float_as_uint(best)), row_turned<4>(at));
+    better(row_turned<2>(__float_as_uint(best)), row_turned<2>(at));
+    better(row_turned<1>(__float_as_uint(best)), row_turned<1>(at));
     if ((at & 63) == lane) taken |= 1u << (at >> 6);
     if (k == 0) first = best;
     float s = 0.f;
@@ -208,7 +221,10 @@ __global__ __launch_bounds__(1024) void router_kernel(
 // router.  In one kernel the router's rows are on their way while the row is
 // normed, and one launch and one trip to memory are left out: us of norm and
 // router and here, 32 x 2048, 4 tokens 8.6 7.2; 8 x 4096, 192 tokens 9.2 6.7, with
-// 3 parts 10.9 8.0, 2000 tokens 33.6 31.3; 64 x 4096, 1000 tokens 47 44.
+// 3 parts 10.9 8.0, 2000 tokens 33.6 31.3; 64 x 4096, 1000 tokens 47 44.  Lanes
+// combined in registers, not by permutes through LDS, router and weights from memory:
+// 8.0 -> 6.9, 7.6 -> 6.8, 36.5 -> 29.5 and 49 -> 44; a decode step of 4 rows and 8
+// layers 579 -> 565.
 template <int JN, bool PARTS>
 __global__ __launch_bounds__(1024) void norm_router_kernel(
     Route r, bf16* __restrict__ out, const bf16* __restrict__ x,
