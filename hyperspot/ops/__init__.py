@@ -350,6 +350,22 @@ def _waves_gemm(M: int, N: int, K: int):
     return None
 
 
+def _wave_of_rows(M: int, N: int, K: int):
+    """Tiles of 64 x 64 for 65 to 192 rows where they are 144 to 256, so that every
+    unit has at most one, on each of the 8 dies (of one tile of w all go to the same:
+    3 tiles of rows and 84 of outputs are 252, but 33 on some).  250 random sizes, time
+    over the library's: 2 tiles of rows, K of 384 to 1024 0.72, to 2304 0.9 (2 of 100
+    more than 3 % slower), beyond 1.02; 3 0.73, beyond 2304 1.06 and more for every
+    second one.  192 rows of 3072 x 2048 22 -> 12.6 us, 129 12.6 -> 11.1; decode steps
+    of 8 layers with that product, 130 rows 964 -> 869 us, 192 1037 -> 939.  More rows
+    gain in some steps and lose in others (256 1049 -> 1011, a prompt of 256 758
+    766)."""
+    if not 64 < M <= 192 or K % 128 or N % 4 or not 384 <= K <= 2304:
+        return None
+    mt, nt = -(-M // 64), -(-N // 64)
+    return (64, 64, 1) if mt * nt >= 144 and -(-nt // 8) * mt <= 32 else None
+
+
 @lru_cache(maxsize=1 << 14)
 def _route(M: int, N: int, K: int, parts: bool):
     """How x w^T of these sizes is formed: "rows", (rows, outputs of a tile, parts
@@ -363,7 +379,7 @@ def _route(M: int, N: int, K: int, parts: bool):
     if _rows_gemm_sizes(M, N, K) and _native().gemm_rows_fits(M, K):
         return "rows"
     return _less_padding(M, _split_gemm(M, N, K)) \
-        or (_summed_gemm(M, N, K) if parts else None)
+        or (_summed_gemm(M, N, K) if parts else None) or _wave_of_rows(M, N, K)
 
 
 def _rows_gemm_sizes(M: int, N: int, K: int) -> bool:

@@ -354,6 +354,30 @@ def test_one_tile_of_rows(M, N, K):
     _check(ops.linear(x, w), x, w)
 
 
+def test_rule_of_a_wave_of_rows():
+    """65 to 192 rows: 144 to 256 tiles, none for a second wave on any die."""
+    for M, N, K, rule in [
+            (65, 4608, 384, (64, 64, 1)), (65, 4544, 2048, None),
+            (128, 8192, 2304, (64, 64, 1)), (128, 8196, 2048, None),
+            (128, 8192, 2432, None), (192, 3072, 2048, (64, 64, 1)),
+            (129, 5120, 640, (64, 64, 1)), (129, 5124, 640, None),
+            (193, 3072, 2048, None), (64, 8192, 640, None),
+            (128, 8192, 256, None), (128, 8192, 700, None),
+            (128, 8190, 640, None)]:
+        assert ops._wave_of_rows(M, N, K) == rule, (M, N, K)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [
+    (65, 4612, 384), (128, 8188, 640), (129, 3204, 2304), (192, 5120, 896)])
+def test_wave_of_rows(M, N, K):
+    g = torch.Generator().manual_seed(M)
+    x = torch.randn(M, K, generator=g).bfloat16().to(DEV)
+    w = torch.randn(N, K, generator=g).bfloat16().to(DEV)
+    assert ops._route(M, N, K, False) == ops._wave_of_rows(M, N, K) is not None
+    _check(ops.linear(x, w), x, w)
+
+
 def test_rule_leaves_no_workgroup_for_a_second_wave():
     """Workgroups go to 8 dies of 32 units in turn, those of one tile of w to
     the same."""
