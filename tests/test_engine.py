@@ -251,3 +251,14 @@ def test_per_request_sampling_seed_reproducible():
     b = run(321)
     assert a1 == a2          # same request seed => identical draws
     assert a1 != b           # different seed diverges (w.h.p.)
+
+
+def test_steps_between_prefill_sizes():
+    from hyperspot.engine.model_runner import _nearest, _with_between
+    assert _with_between((128, 256, 512)) == [128, 160, 192, 256, 320, 384, 512]
+    assert _with_between((64, 192, 256)) == [64, 192, 256]
+    assert _with_between((1024,)) == [640, 768, 1024] and not _with_between(())
+    for n, size, want in ((129, 256, 160), (160, 256, 160), (161, 256, 192),
+                          (193, 256, 256), (100, 128, 128), (1, 256, 160)):
+        assert _nearest(n, size, {160, 192, 256}) == want
+        assert _nearest(n, size, {}) == size    # nothing is captured early

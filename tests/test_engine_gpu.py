@@ -155,6 +155,49 @@ def test_prefill_graph_matches_eager():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("experts", [0, 4])
+def test_prompts_of_the_steps_between(experts):
+    """Logits and pages of prompts around the steps between two sizes, against a
+    pass that is not captured, and repeated."""
+    from hyperspot.engine import (EngineConfig, LLMEngine, ModelSpec,
+                                  SamplingParams)
+    from hyperspot.engine.request import Request
+
+    class Config(EngineConfig):
+        def spec(self):
+            return ModelSpec("steps", 256, 2, 4, 2, 128, 512, 512,
+                             max_position=1024, num_experts=experts,
+                             num_experts_per_tok=min(experts, 2))
+
+    lengths = (127, 160, 161, 192, 193, 256, 130)
+    outs = []
+    for eager in (False, True):
+        eng = LLMEngine(Config(
+            model="steps", max_num_seqs=4, max_model_len=512, num_gpu_blocks=128,
+            enforce_eager=eager, graph_batch_sizes=(1,),
+            prefill_graph_sizes=(128, 256), seed=3), device="cuda:0")
+        eng.capture_graphs()
+        assert sorted(eng.runner._pgraphs) == (
+            [] if eager else [128, 160, 192, 256])
+        got = []
+        for rep in range(2):
+            for n in lengths:
+                toks = [(7 * i + n) % 251 for i in range(n + 1)]
+                req = Request(f"{rep}-{n}", toks[:n], SamplingParams())
+                for tail in (n, 1):
+                    batch = eng.scheduler.schedule_portions([(req, tail)])
+                    got.append(eng.runner.forward(batch).float().cpu())
+                    req.prompt_token_ids.append(toks[n])
+                eng.scheduler.release(req)
+        outs.append(torch.cat(got))
+        del eng
+    half = len(outs[0]) // 2
+    assert torch.equal(outs[0][:half], outs[0][half:])
+    # bf16 activations: other tiles for other numbers of rows
+    assert (outs[0] - outs[1]).norm() <= 0.02 * outs[1].norm()
+
+
+@pytest.mark.gpu
 def test_guided_json_decode_gpu():
     """Guided mask on DEVICE logits (advanced indexing + -inf fill on
     the sampler path): grammar holds on hardware exactly as on CPU."""
