@@ -44,9 +44,9 @@ struct Split {
 
 // BM rows of x, BN of w; WM * WN waves have BM / WM by BN / WN.  A stage has
 // KC chunks of 64 columns.  Two waves a SIMD (128 threads are less) keep the
-// sums in vector registers.
+// sums in vector registers.  AUX: of the loads of w.
 template <int BM, int BN, int WM, int WN, int STAGES, int KC, bool FP8,
-          bool GATED>
+          bool GATED, int AUX>
 __global__ __launch_bounds__(WM * WN * 64, 2)
 void gemm_split_kernel(Split a) {
   using Loop = TileLoop<BM, BN, WM, WN, STAGES, KC, FP8>;
@@ -112,8 +112,8 @@ void gemm_split_kernel(Split a) {
                     (d * KC + s) * 128);
     } else {
       const int j = i / KC - LX;
-      w_rows.to_lds<ONCE>(base + BM * 128 + (wid * LW + j) * 1024, w_off[j],
-                          (d * KC + s) * 128);
+      w_rows.to_lds<AUX>(base + BM * 128 + (wid * LW + j) * 1024, w_off[j],
+                         (d * KC + s) * 128);
     }
   };
   Loop loop;
@@ -196,20 +196,33 @@ void launch_gemm_split(bf16* out, float* part, const void* x, const void* w,
                        const float* x_scale, const float* w_scale, int M,
                        int N, int K, long xs, long ws, int bm, int bn,
                        int splits, bool gated, hipStream_t stream) {
+  // A tile of w that several tiles of rows share is read once where they go through
+  // it together.  One that has few rows does not keep step, for the rows past the end
+  // cost it nothing, and non-temporal loads leave the others nothing.  us, plain and
+  // so: 128 rows a tile, 129 rows of 4096 x 14336 43 49, 192 43 47, 256 46.5 45, 257
+  // 69 80, 350 74 73, 420 71 81,
+  // 480 77.5 77; 256 a tile, 320 55.6 55.8, 512 62.5 59.5.
+  const int last = (M - 1) % bm + 1;
+  const bool once = M <= bm || last * 4 >= bm * 3;
   Split a{out, part, x, w, x_scale, w_scale, M, N, K, xs, ws, 0, 0, splits};
-  #define RUN(BM, BN, WM, WN, STAGES, KC, FP8, GATED)                       \
+  #define WITH(BM, BN, WM, WN, STAGES, KC, FP8, GATED, AUX)                 \
     {                                                                       \
       constexpr int BYTES = STAGES * KC * (BM + BN) * 128;                  \
+      constexpr auto kernel =                                               \
+          &gemm_split_kernel<BM, BN, WM, WN, STAGES, KC, FP8, GATED, AUX>;  \
       static const hipError_t set = hipFuncSetAttribute(                    \
-          reinterpret_cast<const void*>(                                    \
-              &gemm_split_kernel<BM, BN, WM, WN, STAGES, KC, FP8, GATED>),  \
+          reinterpret_cast<const void*>(kernel),                            \
           hipFuncAttributeMaxDynamicSharedMemorySize, BYTES);               \
       HIP_CHECK(set);                                                       \
       a.mt = (M + BM - 1) / BM;                                             \
       a.nt = (N + BN - 1) / BN;                                             \
       const unsigned units = (unsigned)(a.nt * splits + 7) / 8 * 8;         \
-      gemm_split_kernel<BM, BN, WM, WN, STAGES, KC, FP8, GATED>             \
-          <<<units * a.mt, WM * WN * 64, BYTES, stream>>>(a);               \
+      kernel<<<units * a.mt, WM * WN * 64, BYTES, stream>>>(a);             \
+    }
+  #define RUN(BM, BN, WM, WN, STAGES, KC, FP8, GATED)                       \
+    {                                                                       \
+      if (once) WITH(BM, BN, WM, WN, STAGES, KC, FP8, GATED, ONCE)          \
+      else WITH(BM, BN, WM, WN, STAGES, KC, FP8, GATED, 0)                  \
     }
   #define KINDS(BM, BN, WM, WN, STAGES, KC)                                 \
     {                                                                       \
@@ -238,6 +251,7 @@ void launch_gemm_split(bf16* out, float* part, const void* x, const void* w,
     KINDS(64, 64, 2, 2, 4, 2)
   #undef KINDS
   #undef RUN
+  #undef WITH
   if (splits == 1 || !out) return;
   const long quads = (long)M * N / 4;
   #define SUM(S)                                                            \
