@@ -54,8 +54,8 @@ void launch_experts_route(float*, int*, const float*, int, int, int, bool,
 void launch_experts_router(float*, int*, const void*, const float*,
                            const bf16*, long, int, int, int, hipStream_t);
 void launch_norm_router(float*, int*, bf16*, const bf16*, const float*, int,
-                        bf16*, const bf16*, float, const bf16*, long, int, int,
-                        int, hipStream_t);
+                        bf16*, const bf16*, float, const bf16*, const long*,
+                        long, int, int, int, hipStream_t);
 void launch_experts_tiles(bool, bf16*, const void*, const void*, const float*,
                           const float*, const int*, const int*, long, int, int,
                           int, int, int, hipStream_t);
@@ -550,7 +550,7 @@ void experts_router(Tensor weight, Tensor ids, Tensor x, Maybe x_scale,
 // weights of out's rows; x bf16 [T, W] or float parts [parts, T, W]
 void norm_router(Tensor weight, Tensor ids, Tensor out, Tensor x,
                  Tensor residual, Tensor norm, double eps, Tensor router,
-                 long top) {
+                 long top, c10::optional<Tensor> slots) {
   const bool parts = x.dim() == 3;
   check(x, parts ? torch::kFloat : torch::kBFloat16, "x");
   check(out, torch::kBFloat16, "out");
@@ -571,12 +571,17 @@ void norm_router(Tensor weight, Tensor ids, Tensor out, Tensor x,
                 "norm_router: alignment");
   check_param(weight, T * top, "weight");
   check_ints(ids, T * top, "ids");
+  if (slots.has_value()) {
+    check(*slots, torch::kLong, "slots");
+    TORCH_CHECK(slots->numel() == T, "norm_router: slots");
+  }
   launch_norm_router(ptr<float>(weight), ids.data_ptr<int>(), ptr<bf16>(out),
                      parts ? nullptr : ptr<bf16>(x),
                      parts ? ptr<float>(x) : nullptr,
                      parts ? (int)x.size(0) : 0, ptr<bf16>(residual),
-                     ptr<bf16>(norm), (float)eps, ptr<bf16>(router), T, (int)E,
-                     (int)top, (int)W, stream());
+                     ptr<bf16>(norm), (float)eps, ptr<bf16>(router),
+                     slots.has_value() ? slots->data_ptr<long>() : nullptr, T,
+                     (int)E, (int)top, (int)W, stream());
 }
 
 void check_sorted(const Tensor& order, const Tensor& expert,

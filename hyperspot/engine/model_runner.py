@@ -431,7 +431,7 @@ class ModelRunner:
             slot_mapping=io["slot_mapping"],
             seq_start=io["seq_start"],
             max_seqlen=T, fresh_prefill=True,
-            logits_indices=io["lidx"])
+            logits_indices=io["lidx"], padded=True)
         if self.spec.is_hybrid:
             self._add_hybrid_meta(meta, [-1], [T])
             io["state_slots"] = meta.state_slots
@@ -494,7 +494,7 @@ class ModelRunner:
         meta = ForwardMeta(mode="decode", positions=io["positions"],
                            slot_mapping=io["slot_mapping"],
                            block_tables=io["block_tables"],
-                           seq_lens=io["seq_lens"])
+                           seq_lens=io["seq_lens"], padded=True)
         if self.spec.is_hybrid:
             io["state_slots"] = torch.full((bucket,), -1, dtype=torch.int32,
                                            device=d)

@@ -81,6 +81,8 @@ class ForwardMeta:
     latent: Optional[Dict[int, LatentSpan]] = None
     # debugging: a list that collects the residual stream after every layer
     residual_trail: Optional[list] = None
+    # captured: rows of a negative slot are padding
+    padded: bool = False
 
 
 TILE_TOKENS = 64
@@ -211,8 +213,9 @@ class DecoderLayer(nn.Module):
         router = None if find is None or watched(self.mlp) \
             else find(self.mlp, h, residual, self.post_norm_w)
         if router is not None:
-            return ops.fused_add_rmsnorm_route(h, residual, self.post_norm_w,
-                                               self.eps, *router)
+            return ops.fused_add_rmsnorm_route(
+                h, residual, self.post_norm_w, self.eps, *router,
+                meta.slot_mapping if meta.padded else None)
         if fp8:
             h, residual = ops.fused_add_rmsnorm_q(h, residual,
                                                   self.post_norm_w, self.eps)

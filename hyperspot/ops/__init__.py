@@ -94,16 +94,18 @@ def fused_add_rmsnorm(x: torch.Tensor, residual: torch.Tensor,
 
 
 def fused_add_rmsnorm_route(x, residual: torch.Tensor, weight: torch.Tensor,
-                            eps: float, router: torch.Tensor, top: int):
+                            eps: float, router: torch.Tensor, top: int,
+                            slots: Optional[torch.Tensor] = None):
     """fused_add_rmsnorm, x a tensor or Parts, and moe_router in one kernel:
-    (Routed, residual); residual is changed in place.  GPU."""
+    (Routed, residual); residual is changed in place.  Rows of a negative slot
+    (int64) choose no expert.  GPU."""
     data = x.data if isinstance(x, Parts) else x
     T, W = residual.shape
     out = torch.empty_like(residual)
     share = torch.empty(T, top, dtype=torch.float32, device=residual.device)
     ids = torch.empty(T, top, dtype=torch.int32, device=residual.device)
     _native().norm_router(share, ids, out, data, residual, weight, eps, router,
-                          top)
+                          top, slots)
     return Routed(out, share, ids), residual
 
 

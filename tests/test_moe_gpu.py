@@ -258,6 +258,38 @@ def test_norm_and_router(tokens, experts, top, width, parts):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("tokens,experts,top", [(4, 32, 4), (60, 4, 2), (200, 8, 2)])
+def test_padding_chooses_no_expert(tokens, experts, top):
+    """Without a sort and in tiles; the other rows are as without padding, and the
+    padding's own get nothing from the experts."""
+    g = torch.Generator().manual_seed(tokens)
+    rand = lambda *s: torch.randn(*s, generator=g).to(DEV)
+    W, I = 256, 128
+    x, res, norm = (rand(tokens, W).bfloat16(), rand(tokens, W).bfloat16(),
+                    rand(W).bfloat16())
+    router = (rand(experts, W) * W ** -0.5).bfloat16()
+    w13 = (rand(experts, 2 * I, W) * W ** -0.5).bfloat16()
+    w2 = (rand(experts, W, I) * I ** -0.5).bfloat16()
+    slots = torch.arange(tokens, device=DEV) - 1
+    slots[tokens // 2:tokens * 3 // 4] = -1
+    pad = slots < 0
+    out = []
+    for s in (None, slots):
+        h, r = ops.fused_add_rmsnorm_route(x, res.clone(), norm, 1e-5, router,
+                                           top, s)
+        c = ops.moe_choices(h.data, w13, w2, h.weights, h.ids)
+        out.append((h, *ops.fused_add_rmsnorm(c, r, norm, 1e-5), r))
+    (h0, y0, r0, _), (h1, y1, r1, _) = out
+    assert (h1.ids[pad] == -1).all() and (h1.weights[pad] == 0).all()
+    assert torch.equal(h0.ids[~pad], h1.ids[~pad])
+    assert torch.equal(h0.weights[~pad], h1.weights[~pad])
+    assert torch.equal(h0.data, h1.data)
+    assert torch.equal(y0[~pad], y1[~pad]) and torch.equal(r0[~pad], r1[~pad])
+    # the first norm's sum, and nothing added
+    assert torch.equal(r1[pad], (x.float() + res.float()).bfloat16()[pad])
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("path", ["", "moe"])
 def test_watched_experts_get_tensors(path):
     from hyperspot.engine.config import ModelSpec
