@@ -73,6 +73,48 @@ def test_rope_kv_append():
     assert (kc[untouched] == 0).all()
 
 
+@pytest.mark.parametrize("heads,kv,dim,fp8", [
+    (8, 2, 128, False), (1, 1, 128, True), (32, 8, 128, True), (28, 4, 128, False),
+    (5, 3, 64, False)])
+def test_rope_kv_append_of_any_stride(heads, kv, dim, fp8):
+    """Rows 16 bytes apart or not, the same bits; one whose slot is negative."""
+    T, BS, NB = 37, 16, 5
+    g = torch.Generator().manual_seed(heads)
+    x = torch.randn(T, heads + 2 * kv, dim, generator=g).bfloat16().to(DEV)
+    pos = torch.randint(0, 256, (T,), generator=g).to(DEV)
+    slots = (torch.randperm(NB * BS, generator=g)[:T]).to(DEV)
+    slots[5] = -1
+    cos_sin = R.rope_cos_sin(torch.arange(256), dim, 500000.0).to(DEV)
+    got = []
+    for gap in (0, 4):                      # elements between two rows of q, k
+        caches = [torch.zeros(NB, kv, BS, dim, device=DEV).to(
+            torch.float8_e4m3fn if fp8 else torch.bfloat16) for _ in "kv"]
+        parts = [torch.zeros(T, n * dim + gap, device=DEV).bfloat16()
+                 for n in (heads, kv)]
+        q, k = (p[:, :n * dim].unflatten(1, (n, dim))
+                for p, n in zip(parts, (heads, kv)))
+        q.copy_(x[:, :heads])
+        k.copy_(x[:, heads:heads + kv])
+        v = x[:, heads + kv:].contiguous()
+        ops.rope_kv_append(q, k, v, pos, cos_sin, slots, *caches)
+        assert all((p[:, -gap:] == 0).all() for p in parts if gap)
+        got.append([t.contiguous().view(torch.uint8)
+                    for t in (q, k, *caches)])
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
+    cos, sin = cos_sin[pos].double().chunk(2, -1)
+    want = R._rotate_neox(x[:, :heads].double(), cos, sin)
+    out = got[0][0].view(torch.bfloat16).view(want.shape).double()
+    # rounded once
+    assert ((out - want).abs() <= want.abs() * 2.0 ** -8 + 1e-6).all()
+    rows = caches[1].float().transpose(1, 2).reshape(NB * BS, kv, dim)
+    kept = slots >= 0
+    assert torch.equal(rows[slots[kept]],
+                       x[:, heads + kv:][kept].to(caches[1].dtype).float())
+    rows[slots[kept]] = 0
+    assert (rows == 0).all()
+
+
 @pytest.mark.parametrize("group,heads_kv", [(4, 8), (8, 1), (1, 2)])
 def test_paged_attn_decode(group, heads_kv):
     torch.manual_seed(0)
