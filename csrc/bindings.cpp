@@ -108,8 +108,9 @@ bool gemm_rows_fits(long, long);
 void launch_gemm_split(bf16*, float*, const void*, const void*, const float*,
                        const float*, int, int, int, long, long, int, int, int,
                        bool, hipStream_t);
-void launch_gemm_rows(bf16*, const bf16*, const bf16*, int, int, int, long,
-                      long, long, hipStream_t);
+void launch_gemm_rows(bf16*, const bf16*, const bf16*, const float*,
+                      const float*, int, int, int, long, long, long,
+                      hipStream_t);
 void launch_silu_mul(bf16*, const bf16*, long, int, hipStream_t);
 void launch_quant_fp8(unsigned char*, float*, const bf16*, long, int, long,
                       hipStream_t);
@@ -455,24 +456,42 @@ void decode_inputs(torch::Tensor stage, long B, long cap, long staged,
                        (int)staged, (int)tables.size(1), stream());
 }
 
-// out = x w^T
-void gemm_rows(torch::Tensor out, torch::Tensor x, torch::Tensor w) {
+// out = x w^T; with scales of the rows x and w are e4m3
+void gemm_rows(torch::Tensor out, torch::Tensor x, torch::Tensor w,
+               c10::optional<torch::Tensor> x_scale,
+               c10::optional<torch::Tensor> w_scale) {
+  const bool fp8 = x_scale.has_value();
+  const auto kind = fp8 ? torch::kFloat8_e4m3fn : torch::kBFloat16;
   for (const auto& t : {out, x, w})
-    TORCH_CHECK(t.is_cuda() && t.scalar_type() == torch::kBFloat16 &&
-                    t.dim() == 2 && t.stride(1) == 1, "gemm_rows: matrices");
-  const long M = x.size(0), K = x.size(1), N = w.size(0);
-  TORCH_CHECK(w.size(1) == K && out.size(0) == M && out.size(1) == N,
-              "gemm_rows: shape");
+    TORCH_CHECK(t.is_cuda() && t.dim() == 2 && t.stride(1) == 1,
+                "gemm_rows: matrices");
+  TORCH_CHECK(out.scalar_type() == torch::kBFloat16 &&
+                  x.scalar_type() == kind && w.scalar_type() == kind &&
+                  w_scale.has_value() == fp8, "gemm_rows: matrices");
+  const long M = x.size(0), N = w.size(0), per = fp8 ? 2 : 1;
+  const long K = x.size(1) / per;            // units of 2 bytes
+  TORCH_CHECK(w.size(1) == x.size(1) && x.size(1) % per == 0 &&
+                  out.size(0) == M && out.size(1) == N, "gemm_rows: shape");
   auto aligned = [](const torch::Tensor& t, long n) {
     return reinterpret_cast<uintptr_t>(t.data_ptr()) % (2 * n) == 0 &&
-           t.stride(0) % n == 0;
+           t.stride(0) * t.element_size() % (2 * n) == 0;
   };
+  if (fp8) {
+    check(*x_scale, torch::kFloat, "x_scale");
+    check(*w_scale, torch::kFloat, "w_scale");
+    TORCH_CHECK(x_scale->numel() == M && w_scale->numel() == N &&
+                    reinterpret_cast<uintptr_t>(w_scale->data_ptr()) % 16 == 0,
+                "gemm_rows: scales");
+  }
   TORCH_CHECK(gemm_rows_fits(M, K) && N % 4 == 0 && K % 8 == 0 &&
                   N < (1l << 31) && aligned(x, 8) && aligned(w, 8) &&
                   aligned(out, 4), "gemm_rows: sizes");
   if (N == 0) return;
-  launch_gemm_rows(bf(out), cbf(x), cbf(w), (int)M, (int)N, (int)K,
-                   x.stride(0), w.stride(0), out.stride(0), stream());
+  launch_gemm_rows(bf(out), cbf(x), cbf(w),
+                   fp8 ? x_scale->data_ptr<float>() : nullptr,
+                   fp8 ? w_scale->data_ptr<float>() : nullptr, (int)M, (int)N,
+                   (int)K, x.stride(0) / per, w.stride(0) / per, out.stride(0),
+                   stream());
 }
 
 // out = x w^T, K in `splits` parts that a second kernel adds up; without out
@@ -1264,7 +1283,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("attn_prefill_mfma", &attn_prefill_mfma);
   m.def("attn_portions", &attn_portions);
   m.def("decode_inputs", &decode_inputs);
-  m.def("gemm_rows", &gemm_rows);
+  m.def("gemm_rows", &gemm_rows, pybind11::arg("out"), pybind11::arg("x"),
+        pybind11::arg("w"), pybind11::arg("x_scale") = pybind11::none(),
+        pybind11::arg("w_scale") = pybind11::none());
   m.def("gemm_rows_fits", &gemm_rows_fits);
   m.def("gemm_split", &gemm_split, pybind11::arg("out"), pybind11::arg("x"),
         pybind11::arg("w"), pybind11::arg("part"), pybind11::arg("bm"),

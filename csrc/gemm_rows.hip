@@ -1,5 +1,5 @@
 // out[M, N] = x[M, K] w[N, K]^T for few rows (gfx950), bf16 in and out, float
-// sums.
+// sums; or e4m3 in, with scales of the rows, of which 16 bytes are two products'.
 //
 // What bounds it: reading w once.  So w is the A operand of 16x16x32 products
 // straight from memory.  The rows of x, which every tile of w needs whole, go
@@ -31,6 +31,8 @@
 //   8: 2048 x 2048   1 row  8.7  4.2  (5.3), 32 rows 8.6 6.4 (7.5)
 //      1536 x 4096   1 row 14.6  5.8  (7.9)
 //      10240 x 4096  1 row 27.1 16.5 (21.0); 14336 x 2048 16.3 12.5 (14.8)
+// e4m3, tiles of 64 x 32 and here: 6144 x 4096 1 row 9.8 6.8, 16 rows 11.1 8.9, 2048 x
+// 2048 6.0 4.0 and 6.4 4.2; a decode step of 1 row, 4 wide layers, 405 -> 397.
 #include <type_traits>
 
 #include "common.h"
@@ -48,6 +50,8 @@ struct Rows {
   int M, N, K;
   int rows;                          // of w a tile, at most 16
   long xs, ws, os;                   // row strides
+  const float* x_scale;              // FP8: of a row of x, and of a row of w
+  const float* w_scale;
 };
 
 // 16 bytes a lane, to the wave's LDS address + lane * 16
@@ -70,8 +74,17 @@ DEV void turn(short8_t* f, const short8_t* l) {
   f[1] = y.s;
 }
 
-// CT * 16 rows of x
-template <int CT>
+// 32 products of a lane's 16 bytes, or 64 of e4m3
+template <bool FP8>
+DEV f32x4_t products_of(short8_t a, short8_t b, f32x4_t c) {
+  if constexpr (!FP8) return mfma16(a, b, c);
+  union { short8_t s; long d[2]; } x{a}, y{b};
+  c = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(x.d[0], y.d[0], c, 0, 0, 0);
+  return __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(x.d[1], y.d[1], c, 0, 0, 0);
+}
+
+// CT * 16 rows of x.  FP8: a column is two of e4m3
+template <int CT, bool FP8>
 __global__ __launch_bounds__(WAVES * 64, 4)
 void gemm_rows_kernel(Rows a) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -163,7 +176,7 @@ void gemm_rows_kernel(Rows a) {
           for (int t = 0; t < CT; ++t) {
             const short8_t v = *reinterpret_cast<const short8_t*>(
                 xr[t] + (in ? k : 0));
-            acc[t] = mfma16(wf[u][s], in ? v : short8_t{}, acc[t]);
+            acc[t] = products_of<FP8>(wf[u][s], in ? v : short8_t{}, acc[t]);
           }
         }
     };
@@ -186,9 +199,16 @@ void gemm_rows_kernel(Rows a) {
         y += *reinterpret_cast<const f32x4_t*>(
             red + ((v * CT + wid) * 64 + lane) * 4);
       const int n = now * a.rows + gr * 4, m = wid * 16 + col;
-      if (m < a.M && n < a.N && gr * 4 < a.rows)     // multiples of 4
+      if (m < a.M && n < a.N && gr * 4 < a.rows) {   // multiples of 4
+        if constexpr (FP8) {
+          const float xs = a.x_scale[m];
+          const f32x4_t ws = *reinterpret_cast<const f32x4_t*>(a.w_scale + n);
+          #pragma unroll
+          for (int j = 0; j < 4; ++j) y[j] = y[j] * xs * ws[j];
+        }
         *reinterpret_cast<uint2*>(a.out + m * a.os + n) =
             uint2{cvt_pk_bf16(y[0], y[1]), cvt_pk_bf16(y[2], y[3])};
+      }
     }
     __syncthreads();
   }
@@ -225,21 +245,28 @@ bool gemm_rows_fits(long M, long K) {
          lds_bytes((int)M, (int)K) <= LDS;
 }
 
-// N a multiple of 4, K of 8; rows of x and w 16-byte, of out 8-byte aligned
-void launch_gemm_rows(bf16* out, const bf16* x, const bf16* w, int M, int N,
+// N a multiple of 4, K of 8; rows of x and w 16-byte, of out 8-byte aligned.  With
+// scales x and w are e4m3, and K and their strides half of what they are
+void launch_gemm_rows(bf16* out, const bf16* x, const bf16* w,
+                      const float* x_scale, const float* w_scale, int M, int N,
                       int K, long xs, long ws, long os, hipStream_t stream) {
   const int rows = tile_rows(N);
-  const Rows a{out, x, w, M, N, K, rows, xs, ws, os};
+  const Rows a{out, x, w, M, N, K, rows, xs, ws, os, x_scale, w_scale};
   const int lds = lds_bytes(M, K), tiles = (N + rows - 1) / rows;
   const int most = lds * 2 <= LDS ? 512 : 256;     // that a CU holds at once
   const unsigned grid = (unsigned)(tiles < most ? tiles : most);
-  #define RUN(CT)                                                           \
+  #define KIND(CT, FP8)                                                     \
     {                                                                       \
       static const hipError_t set = hipFuncSetAttribute(                    \
-          reinterpret_cast<const void*>(&gemm_rows_kernel<CT>),             \
+          reinterpret_cast<const void*>(&gemm_rows_kernel<CT, FP8>),        \
           hipFuncAttributeMaxDynamicSharedMemorySize, LDS);                 \
       HIP_CHECK(set);                                                       \
-      gemm_rows_kernel<CT><<<grid, WAVES * 64, lds, stream>>>(a);           \
+      gemm_rows_kernel<CT, FP8><<<grid, WAVES * 64, lds, stream>>>(a);      \
+    }
+  #define RUN(CT)                                                           \
+    {                                                                       \
+      if (x_scale) KIND(CT, true)                                           \
+      else KIND(CT, false)                                                  \
     }
   switch (row_tiles(M)) {
     case 1: RUN(1) break;
@@ -247,4 +274,5 @@ void launch_gemm_rows(bf16* out, const bf16* x, const bf16* w, int M, int N,
     default: RUN(4)
   }
   #undef RUN
+  #undef KIND
 }

@@ -688,29 +688,63 @@ def _tiles_q(M: int, N: int, K: int, parts: bool):
     return (64, 32, 1) if tiles <= 128 else (64, 64, 1)
 
 
+def _plain_q(x: "QTensor", w: torch.Tensor, scale: torch.Tensor) -> bool:
+    """Whether csrc/ reads these as they lie, and nothing records the call."""
+    d, s = x
+    return d.is_cuda and unrecorded(d, w, s, scale) \
+        and d.dim() == w.dim() == 2 and d.shape[0] <= 128
+
+
+def _aligned_q(x: "QTensor", w: torch.Tensor, scale: torch.Tensor) -> bool:
+    d, s = x
+    return d.dtype == w.dtype == torch.float8_e4m3fn \
+        and s.dtype == scale.dtype == torch.float32 \
+        and s.is_contiguous() and scale.is_contiguous() \
+        and scale.data_ptr() % 16 == 0 \
+        and all(t.stride(1) == 1 and t.stride(0) % 16 == 0
+                and t.data_ptr() % 16 == 0 for t in (d, w))
+
+
 def _tiled_q(x: "QTensor", w: torch.Tensor, scale: torch.Tensor, parts: bool):
     """The tile of _tiles_q, or None."""
-    d, s = x
-    if not (d.is_cuda and unrecorded(d, w, s, scale)
-            and d.dim() == w.dim() == 2) or d.shape[0] > 128:
+    if not _plain_q(x, w, scale):
         return None
-    tile = _tiles_q(d.shape[0], *w.shape, parts)
-    if tile is None or not (
-            d.dtype == w.dtype == torch.float8_e4m3fn
-            and _near(d, w, *tile[:2])
-            and s.dtype == scale.dtype == torch.float32
-            and s.is_contiguous() and scale.is_contiguous()
-            and scale.data_ptr() % 16 == 0
-            and all(t.stride(1) == 1 and t.stride(0) % 16 == 0
-                    and t.data_ptr() % 16 == 0 for t in (d, w))):
+    tile = _tiles_q(x.data.shape[0], *w.shape, parts)
+    if tile is None or not (_near(x.data, w, *tile[:2])
+                            and _aligned_q(x, w, scale)):
         return None
     return tile
+
+
+def _rows_q_sizes(M: int, N: int, K: int, parts: bool) -> bool:
+    """Where csrc/gemm_rows.hip is faster for e4m3, which reads whole lines of w
+    without a tile's padding: up to 32 rows that the library or the narrowest tiles
+    took, and up to 16 in parts of up to 8192 columns that a kernel of their own would
+    add up.  180 sizes, time over that of what was there: against the library 0.34 to
+    0.98 (8 of 8880 x 14592 79 30, 16 of 1280 x 2304 7.0 4.5), tiles of 32 outputs
+    0.64 to 0.92 (1 of 6144 x 4096 9.8 6.8, 16 11.1 8.9, 32 of 2048 x 2048 6.5 5.0; 38
+    of 6112 x 2304 7.5 9.2), parts 0.63 to 0.99 (8 of 1760 x 3072 6.6 4.3; of longer
+    ones up to 1.27).  Full waves of wider tiles are faster (16 of 14336 x 2048 8.8
+    10.9), and so are parts that the norm adds up."""
+    if not 1 <= M <= 32 or K % 16 or N % 4 or N * K < 1 << 19 or K > 1 << 17:
+        return False
+    tile = _tiles_q(M, N, K, parts)
+    return tile is None or tile[1] == 32 or (
+        tile[2] > 1 and not parts and M <= 16 and K <= 8192)
 
 
 def linear_q(x: "QTensor", w: torch.Tensor, scale: torch.Tensor,
              parts: bool = False):
     """x w^T of e4m3 with scales of the rows, bf16; with `parts` as Parts where
     it is formed in parts of K.  GPU."""
+    if x.data.dim() == w.dim() == 2 and x.data.shape[1] == w.shape[1] \
+            and _rows_q_sizes(x.data.shape[0], *w.shape, parts) \
+            and _plain_q(x, w, scale) and _aligned_q(x, w, scale) \
+            and _native().gemm_rows_fits(x.data.shape[0], w.shape[1] // 2):
+        out = torch.empty(x.data.shape[0], w.shape[0], dtype=torch.bfloat16,
+                          device=w.device)
+        _native().gemm_rows(out, x.data, w, x.scale, scale)
+        return out
     tile = _tiled_q(x, w, scale, parts)
     if tile is None:
         return torch._scaled_mm(x.data, w.t(), scale_a=x.scale.unsqueeze(1),

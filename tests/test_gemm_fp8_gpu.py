@@ -50,6 +50,32 @@ def test_gemm(M, N, K, parts, bm, bn):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [
+    (1, 4, 16), (3, 20, 528), (16, 260, 1040), (17, 2052, 2048), (32, 4100, 272),
+    (33, 516, 2064), (64, 12, 1024), (8, 6144, 4096), (1, 36, 28672)])
+def test_products_of_few_rows(M, N, K):
+    """Columns that end within a line or a load, outputs within a tile."""
+    q, w, ws = _operands(M, N, K, 16)       # rows are views into wider ones
+    out = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device=DEV)
+    ops._native().gemm_rows(out, q.data, w, q.scale, ws)
+    _check(out, q, w, ws)
+    with pytest.raises(RuntimeError):
+        ops._native().gemm_rows(out, q.data, w, q.scale)
+
+
+def test_rule_of_few_rows():
+    for M, N, K, parts, rule in [
+            (1, 6144, 4096, False, True), (32, 6144, 4096, False, True),
+            (33, 6144, 4096, False, False), (1, 4096, 4096, True, False),
+            (16, 2048, 7168, False, True), (17, 2048, 7168, False, True),
+            (16, 4096, 14336, False, False), (1, 4096, 14336, True, False),
+            (1, 28672, 4096, False, False), (8, 8880, 14592, False, True),
+            (0, 4096, 4096, False, False), (1, 4098, 4096, False, False),
+            (1, 4096, 4104, False, False), (1, 64, 1024, False, False)]:
+        assert ops._rows_q_sizes(M, N, K, parts) == rule, (M, N, K, parts)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("M", [1, 16, 17, 64, 65, 128, 129])
 @pytest.mark.parametrize("N,K", [(4096, 4096), (2048, 7168), (12288, 1024),
                                  (3600, 5120), (2048, 2048), (4096, 14336),
