@@ -52,7 +52,8 @@ void launch_latent_attn_prefill(bf16*, const bf16*, const bf16*, const bf16*,
 void launch_experts_route(float*, int*, const float*, int, int, int, bool,
                           bool, int, const float*, hipStream_t);
 void launch_experts_router(float*, int*, const void*, const float*,
-                           const bf16*, long, int, int, int, hipStream_t);
+                           const bf16*, const long*, long, int, int, int,
+                           hipStream_t);
 void launch_norm_router(float*, int*, bf16*, const bf16*, const float*, int,
                         bf16*, const bf16*, float, const bf16*, const long*,
                         long, int, int, int, hipStream_t);
@@ -527,8 +528,16 @@ void experts_tiles(Tensor out, Tensor x, Tensor w, Maybe x_scale,
 }
 
 // choices and weights of the rows of x [T, W], bf16 or e4m3 with x_scale [T]
+// slots of T rows, or null; pointer of it
+const long* slots_of(const c10::optional<Tensor>& slots, long T) {
+  if (!slots.has_value()) return nullptr;
+  check(*slots, torch::kLong, "slots");
+  TORCH_CHECK(slots->numel() == T, "slots: shape");
+  return slots->data_ptr<long>();
+}
+
 void experts_router(Tensor weight, Tensor ids, Tensor x, Maybe x_scale,
-                    Tensor router, long top) {
+                    Tensor router, long top, c10::optional<Tensor> slots) {
   check(x, x_scale.has_value() ? torch::kFloat8_e4m3fn : torch::kBFloat16,
         "x");
   check(router, torch::kBFloat16, "router");
@@ -542,8 +551,8 @@ void experts_router(Tensor weight, Tensor ids, Tensor x, Maybe x_scale,
   check_param(weight, T * top, "weight");
   check_ints(ids, T * top, "ids");
   launch_experts_router(ptr<float>(weight), ids.data_ptr<int>(), x.data_ptr(),
-                        opt(x_scale), ptr<bf16>(router), T, (int)E, (int)top,
-                        (int)x.size(1), stream());
+                        opt(x_scale), ptr<bf16>(router), slots_of(slots, T), T,
+                        (int)E, (int)top, (int)x.size(1), stream());
 }
 
 // out <- rmsnorm(residual + x) * norm, residual that sum, and the choices and
@@ -571,17 +580,12 @@ void norm_router(Tensor weight, Tensor ids, Tensor out, Tensor x,
                 "norm_router: alignment");
   check_param(weight, T * top, "weight");
   check_ints(ids, T * top, "ids");
-  if (slots.has_value()) {
-    check(*slots, torch::kLong, "slots");
-    TORCH_CHECK(slots->numel() == T, "norm_router: slots");
-  }
   launch_norm_router(ptr<float>(weight), ids.data_ptr<int>(), ptr<bf16>(out),
                      parts ? nullptr : ptr<bf16>(x),
                      parts ? ptr<float>(x) : nullptr,
                      parts ? (int)x.size(0) : 0, ptr<bf16>(residual),
                      ptr<bf16>(norm), (float)eps, ptr<bf16>(router),
-                     slots.has_value() ? slots->data_ptr<long>() : nullptr, T,
-                     (int)E, (int)top, (int)W, stream());
+                     slots_of(slots, T), T, (int)E, (int)top, (int)W, stream());
 }
 
 void check_sorted(const Tensor& order, const Tensor& expert,

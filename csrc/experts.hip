@@ -149,14 +149,15 @@ __global__ __launch_bounds__(256) void route_kernel(Route r) {
 // are too few for a tile of the matrix cores, and one launch replaces the
 // conversions, the product, the softmax, the selection and the division.
 // What bounds it is the latency of one row of the router: 16 waves have JN
-// experts each, whose loads do not wait for each other.
+// experts each, whose loads do not wait for each other.  slots: as below.
 template <bool FP8, int JN>
 __global__ __launch_bounds__(1024) void router_kernel(
     Route r, const void* __restrict__ x, const float* __restrict__ x_scale,
-    const bf16* __restrict__ router, int W) {
+    const bf16* __restrict__ router, const long* __restrict__ slots, int W) {
   constexpr int HELD = 4, COLS = HELD * 512;   // columns at a time
   __shared__ float z[64];
   const long t = blockIdx.x;
+  const bool padding = slots && slots[t] < 0;
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   float sum[JN];                     // experts wid + 16 j
   #pragma unroll
@@ -207,6 +208,10 @@ __global__ __launch_bounds__(1024) void router_kernel(
   int id;
   float w;
   route_token<1>(r, z, &id, &w);
+  if (padding) {
+    id = -1;
+    w = 0.f;
+  }
   if (lane < r.top) {
     r.weight[t * r.top + lane] = w;
     r.ids[t * r.top + lane] = id;
@@ -662,13 +667,14 @@ void launch_experts_route(float* weight, int* ids, const float* logits, int T,
 
 // E <= 64, W a multiple of 8; x bf16, or e4m3 where x_scale is given
 void launch_experts_router(float* weight, int* ids, const void* x,
-                           const float* x_scale, const bf16* router, long T,
-                           int E, int top, int W, hipStream_t stream) {
+                           const float* x_scale, const bf16* router,
+                           const long* slots, long T, int E, int top, int W,
+                           hipStream_t stream) {
   if (T == 0) return;
   const Route r{weight, ids, nullptr, (int)T, E, top, 0, 0, E, nullptr};
   #define RUN(FP8, JN)                                                      \
-    router_kernel<FP8, JN><<<(unsigned)T, 1024, 0, stream>>>(r, x, x_scale,  \
-                                                             router, W)
+    router_kernel<FP8, JN><<<(unsigned)T, 1024, 0, stream>>>(               \
+        r, x, x_scale, router, slots, W)
   #define BY_EXPERTS16(FP8)                                                 \
     if (E <= 16) RUN(FP8, 1);                                               \
     else if (E <= 32) RUN(FP8, 2);                                          \

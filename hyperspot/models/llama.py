@@ -219,6 +219,9 @@ class DecoderLayer(nn.Module):
         if fp8:
             h, residual = ops.fused_add_rmsnorm_q(h, residual,
                                                   self.post_norm_w, self.eps)
+            if find is not None and meta.padded:
+                h = ops.PaddedQ(*h)
+                h.slots = meta.slot_mapping
         else:
             h, residual = ops.fused_add_rmsnorm(h, residual, self.post_norm_w,
                                                 self.eps)

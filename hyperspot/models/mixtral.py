@@ -101,7 +101,8 @@ class MixtralMoE(nn.Module):
             # dequantize only the router's [T,E] logits input
             xq = x
             if self._fused_router(xq.data) and get_ep_size() == 1:
-                weights, ids = ops.moe_router(xq, self.router, self.top_k)
+                weights, ids = ops.moe_router(xq, self.router, self.top_k,
+                                              getattr(xq, "slots", None))
                 return ops.moe_ffn_fp8(xq, self.w13, self.w13_scale, self.w2,
                                        self.w2_scale, weights, ids)
             x = (xq.data.float() * xq.scale[:, None]).to(torch.bfloat16)

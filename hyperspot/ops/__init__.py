@@ -10,7 +10,7 @@ device without the extension is a hard error, never a silent eager fallback.
 from __future__ import annotations
 
 from functools import lru_cache
-from typing import NamedTuple
+from typing import NamedTuple, Optional
 
 import torch
 
@@ -638,6 +638,12 @@ class QTensor(NamedTuple):
     scale: torch.Tensor
 
 
+class PaddedQ(QTensor):
+    """Rows of a captured step: those of a negative slot are padding."""
+
+    slots: Optional[torch.Tensor] = None
+
+
 @lru_cache(maxsize=1 << 14)
 def _tiles_q(M: int, N: int, K: int, parts: bool):
     """(rows, outputs of a tile, parts of K) where csrc/gemm_split.hip is
@@ -838,14 +844,16 @@ def moe_router_takes(tokens: int, experts: int) -> bool:
         16384 if experts <= 16 else 6144 if experts <= 32 else 1280)
 
 
-def moe_router(x, router: torch.Tensor, top: int):
+def moe_router(x, router: torch.Tensor, top: int,
+               slots: Optional[torch.Tensor] = None):
     """(weights [T, top] float, expert ids [T, top] int32) of the rows of x, a
-    bf16 tensor or a QTensor: the softmax over the chosen.  GPU."""
+    bf16 tensor or a QTensor: the softmax over the chosen.  Rows of a negative slot
+    (int64) choose none.  GPU."""
     data, scale = x if isinstance(x, QTensor) else (x, None)
     T = data.shape[0]
     weight = torch.empty(T, top, dtype=torch.float32, device=data.device)
     ids = torch.empty(T, top, dtype=torch.int32, device=data.device)
-    _native().experts_router(weight, ids, data, scale, router, top)
+    _native().experts_router(weight, ids, data, scale, router, top, slots)
     return weight, ids
 
 

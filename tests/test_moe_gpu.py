@@ -290,6 +290,33 @@ def test_padding_chooses_no_expert(tokens, experts, top):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("tokens", [5, 130])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_padding_of_the_router(tokens, fp8):
+    """By itself, and through the experts in 8 bits."""
+    from hyperspot.parallel.layers import quantize_weight_fp8
+    g = torch.Generator().manual_seed(tokens)
+    rand = lambda *s: torch.randn(*s, generator=g).to(DEV)
+    E, W, I, top = 4, 256, 256, 2
+    x, router = rand(tokens, W).bfloat16(), rand(E, W).bfloat16()
+    xq = ops.quant_fp8(x) if fp8 else x
+    slots = torch.arange(tokens, device=DEV) % 4 - 1
+    pad = slots < 0
+    weight, ids = ops.moe_router(xq, router, top)
+    got, got_ids = ops.moe_router(xq, router, top, slots)
+    assert torch.equal(got[~pad], weight[~pad]) and (got[pad] == 0).all()
+    assert torch.equal(got_ids[~pad], ids[~pad]) and (got_ids[pad] == -1).all()
+    if not fp8:
+        return
+    w13, s13, w2, s2 = (torch.stack(t) for t in zip(*(
+        quantize_weight_fp8(rand(2 * I, W) * W ** -0.5)
+        + quantize_weight_fp8(rand(W, I) * I ** -0.5) for _ in range(E))))
+    want = ops.moe_ffn_fp8(xq, w13, s13, w2, s2, weight, ids)
+    out = ops.moe_ffn_fp8(xq, w13, s13, w2, s2, got, got_ids)
+    assert torch.equal(out[~pad], want[~pad]) and (out[pad] == 0).all()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("path", ["", "moe"])
 def test_watched_experts_get_tensors(path):
     from hyperspot.engine.config import ModelSpec
