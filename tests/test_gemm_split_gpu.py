@@ -302,13 +302,15 @@ def test_rule_of_few_rows_of_long_columns():
 def test_rule_of_several_waves():
     """Half a wave and more, and several; not nearly empty ones."""
     for M, N, K, rule in [
-            (1, 9152, 2048, None), (1, 9153 + 3, 2048, (64, 64, 1)),
+            (1, 9152, 2048, None), (1, 9153 + 3, 2048, "rows"),
+            (5, 9156, 2048, (64, 64, 1)), (1, 9156, 1024, (64, 64, 1)),
+            (4, 9156, 5120, "rows"), (4, 9156, 5248, (64, 64, 1)),
             (64, 11264, 640, None), (64, 11200, 512, None),
-            (1, 16388, 2048, (64, 128, 1)), (64, 22400, 768, (64, 128, 1)),
+            (5, 16388, 2048, (64, 128, 1)), (64, 22400, 768, (64, 128, 1)),
             (1, 33000, 2048, None), (1, 45000, 1024, None),
-            (1, 45000, 1152, (64, 64, 1)), (17, 45000, 1152, None),
+            (5, 45000, 1152, (64, 64, 1)), (17, 45000, 1152, None),
             (16, 49156, 896, (64, 128, 1)), (1, 49156, 768, None),
-            (32, 65700, 640, (64, 128, 1)), (1, 69632, 2048, (64, 64, 1)),
+            (32, 65700, 640, (64, 128, 1)), (5, 69632, 2048, (64, 64, 1)),
             (32, 49156, 1024, None), (64, 128256, 4096, (64, 128, 1)),
             (64, 128256, 4224, None), (64, 69632, 1024, None),
             (65, 128256, 4096, None), (1, 128256, 4100, None)]:
