@@ -7,25 +7,26 @@
 // or 256 bytes of a row, go from memory to LDS directly, 16 bytes a lane, into
 // a ring that fills most of LDS.
 //
-// What bounds it: w from memory up to about 100 rows (4.3 TB/s in parts, 5.3 in
-// one wave of tiles, as 28672 x 4096, and 4.4 of e4m3), then what the tiles take
+// What bounds it: w from memory up to about 100 rows (5.5 TB/s in parts, 5.9 in
+// one wave of tiles, as 28672 x 4096, and 4.8 of e4m3), then what the tiles take
 // from L2, so that 128 x 128 beat 128 x 64 where K is long, and the
 // narrow ones, with longer chunks, where it is short; then the products.  A
-// ring of 5 stages, or of chunks twice as long, takes as long.
+// ring of 5 stages, or of chunks twice as long, takes as long, and waves that divide
+// a stage's chunks up to 5 % longer.
 //
-// us, library and here:
-//   4096 x 14336  32 rows 35 27, 96 63 32, 192 102 45, 256 62 49, 512 88 76
-//   6144 x 4096   96 rows 23 19, 192 34 28, 256 40 30
-//   4096 x 4096   32 rows 13 12, 96 22 14, 192 33 22, 256 23 23
-//   2048 x 7168   32 rows 19 11, 96 19 14, 192 25 19, 256 25 20, 512 32 29
-//   5120 x 8192   32 rows 25 23, 96 37 26, 192 61 36, 256 72 39
-// silu(gate) * up of the halves, product and activation and here: 28672 x 4096 17
-//   rows 47 41, 64 57 41, 128 59 48; 14336 x 2048 32 rows 19 13, 256 32 23; in
-//   tiles of 256 x 128 28672 x 4096 256 rows 79 69, 14336 x 1664 512 36 27
+// us, library and here, x and w from memory:
+//   4096 x 14336  32 rows 33 26, 96 68 38, 192 112 46, 256 66 52, 512 98 70
+//   6144 x 4096   96 rows 24 23, 192 35 28, 256 44 29
+//   4096 x 4096   32 rows 14 11, 96 23 16, 192 34 21, 256 23 23
+//   2048 x 7168   32 rows 19 11, 96 20 15, 192 26 19, 256 26 22, 512 33 32
+//   5120 x 8192   32 rows 27 22, 96 39 28, 192 64 36, 256 79 38
+// silu(gate) * up of the halves, product and activation and here: 28672 x 4096 1 row
+//   64 41, 17 rows 52 41, 64 53 42, 128 61 53; 14336 x 2048 32 rows 18 13, 256 33 24;
+//   in tiles of 256 x 128 28672 x 4096 256 rows 80 69, 14336 x 1664 512 37 30
 // e4m3, with the norm that adds up the parts: 4096 x 14336 16 rows 27 19, 64 31
 // 21, 128 44 28; 4096 x 4096 16 rows 15 12, 128 18 15; without: 28672 x 4096 16
-// rows 34 24, 64 31 26 (29 in tiles of 64 x 64, of which 448 are not one wave);
-// 14336 x 2048 64 rows 14 11; 6144 x 4096 13.7 12.3; 3072 x 2048 9.1 6.4.
+// rows 34 23, 64 31 24 (27 in tiles of 64 x 64, of which 448 are not one wave);
+// 14336 x 2048 64 rows 14 10; 64 of 6144 x 4096 13.4 11.3, 3072 x 2048 10.7 7.2.
 #include "tile_loop.h"
 
 namespace {

@@ -302,12 +302,13 @@ MOST_ROWS = 512         # of a product that a kernel here takes
 def _wave_gemm(M: int, N: int, K: int):
     """Tiles of 64 rows where those of 64 or 128 outputs are one workgroup a
     compute unit, or nearly: N of 11264 to 16384 and of 22528 to 32768.  Against
-    the kernel of few rows and the library, us: 32768 x 4096 1 row 47.1 45.3, 16
-    52.6 46.7, 24 66 46, 64 62 48; 32768 x 2048 1 row 25.7 25.9, 32 31 26, 64 35
-    26.5; 14272 x 3072 23 rows 19.9 19.2; 23744 x 4096 39 rows 45 36; 26112 x 3072
-    6 rows 37 31; 11264 x 512 39 rows 7.9 5.7.  Beyond 64 rows the library is as
-    fast (96 of 32768 x 4096 63 60, 128 64 65), and so it is with fewer or more
-    tiles (10 of 7808 x 4096 17 21; 2 of 39104 x 4096 59 64)."""
+    the kernel of few rows or the library, us, x and w from memory: 32768 x 4096 1 row
+    44.3 45.9, 16 47.3 46.0, 24 68 45, 64 66 47; 32768 x 2048 1 row 24.6 25.5, 32 29
+    26, 64 38 26.5; 14272 x 3072 23 rows 20.5 18.2; 23744 x 4096 39 rows 47 35; 26112 x
+    3072 6 rows 45 28; 60 random sizes, over the kernel of few rows 0.98 up to 4 rows,
+    0.88 of 8 and 16.  Beyond 64 rows the library is as fast (96 of 32768 x 4096 63 60,
+    128 64 65), and so it is with fewer or more tiles (10 of 7808 x 4096 17 21; 2 of
+    39104 x 4096 59 64)."""
     if not 1 <= M <= 64 or K == 0 or K % 128 or N % 4:
         return None
     for bn in (64, 128):
@@ -577,9 +578,9 @@ def _gated_tile(M: int, N: int, K: int):
     up of x w^T faster than a product and an activation, else None: the smallest
     tiles that are one workgroup a compute unit or less.  Measured at 1 to 256
     rows, N of 2048 to 57344 and K of 512 to 8192: 0.78 of both on average where
-    it is taken (us: 28672 x 4096 1 row 43.4 41.4, 8 rows 48 41, 17 47 41, 32 58
-    41, 64 57 41, 128 59 48; 14336 x 2048 1 row 15.1 13.4, 16 18 13, 32 19 13,
-    64 20 15, 128 24 18, 192 30 21, 256 32 23).
+    it is taken (us, x and w from memory: 28672 x 4096 1 row 64 41, 8 rows 65 41, 17
+    52 41, 32 52 41, 64 53 42, 128 61 53; 14336 x 2048 1 row 19 13, 16 18 12, 32 18 13,
+    64 20 15, 128 23 19, 192 30 23, 256 33 24).
     More tiles take a second wave (192 rows of 28672 x 4096 67 73) but for 17 to
     64 rows, where the library has no better tile (29 rows of 38400 x 6144 124
     96; 6 of 52736 x 1536 36 38).  Few tiles with long rows leave the chip idle (23 rows of 2048 x 3072
