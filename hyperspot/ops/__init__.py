@@ -731,6 +731,7 @@ def _tiled_q(x: "QTensor", w: torch.Tensor, scale: torch.Tensor, parts: bool):
     return tile
 
 
+@lru_cache(maxsize=1 << 14)
 def _rows_q_sizes(M: int, N: int, K: int, parts: bool) -> bool:
     """Where csrc/gemm_rows.hip is faster for e4m3, which reads whole lines of w
     without a tile's padding: up to 32 rows that the library or the narrowest tiles
@@ -752,15 +753,17 @@ def linear_q(x: "QTensor", w: torch.Tensor, scale: torch.Tensor,
              parts: bool = False):
     """x w^T of e4m3 with scales of the rows, bf16; with `parts` as Parts where
     it is formed in parts of K.  GPU."""
-    if x.data.dim() == w.dim() == 2 and x.data.shape[1] == w.shape[1] \
-            and _rows_q_sizes(x.data.shape[0], *w.shape, parts) \
+    # the host's time is what an eager step of small prompts waits for
+    rows = len(x.data) if x.data.dim() == 2 else MOST_ROWS
+    if rows <= 32 and w.dim() == 2 and x.data.shape[1] == w.shape[1] \
+            and _rows_q_sizes(rows, *w.shape, parts) \
             and _plain_q(x, w, scale) and _aligned_q(x, w, scale) \
-            and _native().gemm_rows_fits(x.data.shape[0], w.shape[1] // 2):
-        out = torch.empty(x.data.shape[0], w.shape[0], dtype=torch.bfloat16,
+            and _native().gemm_rows_fits(rows, w.shape[1] // 2):
+        out = torch.empty(rows, w.shape[0], dtype=torch.bfloat16,
                           device=w.device)
         _native().gemm_rows(out, x.data, w, x.scale, scale)
         return out
-    tile = _tiled_q(x, w, scale, parts)
+    tile = _tiled_q(x, w, scale, parts) if rows <= 128 else None
     if tile is None:
         return torch._scaled_mm(x.data, w.t(), scale_a=x.scale.unsqueeze(1),
                                 scale_b=scale.unsqueeze(0),
