@@ -323,21 +323,22 @@ def _full(tiles: int) -> float:
 
 
 def _waves_gemm(M: int, N: int, K: int):
-    """Tiles of 64 rows by 64 or 128 outputs where they are half a wave or more of
-    one workgroup a compute unit, or several waves, against the kernel of few rows
-    and the library; or that kernel, "rows", which reads whole lines since.  130 random sizes, time over what was there: 9153 to 11264 and
-    16385 to 22528 outputs 0.85 (4 of 10628 x 3328 20 17; 16 of 10168 x 4224 34 19; 64
-    of 18736 x 896 15 11; 32 of 10008 x 5120 26 27); several waves and up to 16 rows
-    0.87, wide tiles but where narrow ones fill the units better (1 of 128256 x 4096
-    185 163, 2 of 144224 x 2304 132 113, 2 of 49448 x 3456 62 59), 17 to 32 rows 0.85
-    (128256 x 4096 201 172), 33 to 64 with up to 4096 columns 0.80 (64 of 128256 x 4096
-    215 183).  Left are 257 to 384 wide tiles, which are nearly one wave more than
-    needed, and narrow ones that fill no wave either (1.0 to 1.13); few columns for few
-    rows (1 of 100164 x 640 28 30); long ones for many rows (62 of 58064 x 7296 156
-    161).  The kernel of few rows in place of these tiles, up to 4 rows of 1152 to 5120
-    columns: 150 sizes 0.93 (1 of 9600 x 4096 19.1 16.3, of 128256 x 4096 165 159, 2 of
-    100352 x 2048 77 66; worst 4 of 256000 x 2048 162 172); 8 rows 0.89 to 1.2, longer
-    columns 0.78 to 1.14, shorter ones 0.9 to 1.3."""
+    """Tiles of 64 rows by 64 or 128 outputs where they are half a wave or more of one
+    workgroup a compute unit, or several waves, against the kernel of few rows and the
+    library; or that kernel, "rows", which reads whole lines since. 130 random sizes,
+    time over what was there: 9153 to 11264 and 16385 to 22528 outputs 0.85 (4 of
+    10628 x 3328 20 17; 16 of 10168 x 4224 34 19; 64 of 18736 x 896 15 11; 32 of 10008
+    x 5120 26 27); several waves and up to 16 rows 0.87, wide tiles but where narrow
+    ones fill the units better (1 of 128256 x 4096 185 163, 2 of 144224 x 2304 132
+    113, 2 of 49448 x 3456 62 59), 17 to 32 rows 0.85 (128256 x 4096 201 172), 33 to
+    64 with up to 4096 columns 0.80 (64 of 128256 x 4096 215 183). Left are 257 to 384
+    wide tiles, which are nearly one wave more than needed, and narrow ones that fill
+    no wave either (1.0 to 1.13); few columns for few rows (1 of 100164 x 640 28 30);
+    long ones for many rows (62 of 58064 x 7296 156 161). The kernel of few rows in
+    place of these tiles, up to 4 rows of 1152 to 5120 columns: 150 sizes 0.93 (1 of
+    9600 x 4096 19.1 16.3, of 128256 x 4096 165 159, 2 of 100352 x 2048 77 66; worst 4
+    of 256000 x 2048 162 172); 8 rows 0.89 to 1.2, longer columns 0.78 to 1.14,
+    shorter ones 0.9 to 1.3."""
     tile = _several_waves(M, N, K)
     return "rows" if tile and M <= 4 and 1152 <= K <= 5120 else tile
 
