@@ -344,7 +344,8 @@ def _waves_gemm(M: int, N: int, K: int):
 
 
 def _several_waves(M: int, N: int, K: int):
-    if not 1 <= M <= 64 or not 640 <= K <= 16384 or K % 128 or N % 4:
+    if not 1 <= M <= 64 or not 640 <= K <= 16384 or K % 128 or N % 4 \
+            or N >= 1 << 24:        # outputs that the tiles count
         return None
     narrow, wide = -(-N // 64), -(-N // 128)
     if 144 <= narrow < 176:

@@ -317,6 +317,21 @@ def test_rule_of_several_waves():
         assert ops._waves_gemm(M, N, K) == rule, (M, N, K)
 
 
+def test_rules_leave_what_no_tile_takes():
+    """Tiles count up to 2^24 outputs, the kernel of few rows up to 2^31."""
+    for M in (1, 4, 5, 8, 16, 17, 32, 33, 64, 65, 192, 256, 512):
+        for N in (1 << 24, (1 << 24) + 128, 3 << 23, 1 << 25):
+            for K in (128, 640, 1024, 1152, 2048, 4096, 5120, 16384):
+                for parts in (False, True):
+                    assert ops._route(M, N, K, parts) in (None, "rows")
+                assert ops._gated_tile(M, N, K) is None
+                assert ops._gated_wave(M, N, K) is None
+    # a product that the tiles still take, and the first that they do not
+    assert ops._route(8, (1 << 24) - 4, 1152, False) == (64, 128, 1)
+    assert ops._route(8, 1 << 24, 1152, False) == \
+        ("rows" if ops._rows_gemm_sizes(8, 1 << 24, 1152) else None)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K", [
     (1, 9156, 640), (64, 11196, 896), (33, 16388, 640), (16, 22396, 768),
