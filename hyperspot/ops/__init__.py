@@ -744,7 +744,8 @@ def _rows_q_sizes(M: int, N: int, K: int, parts: bool) -> bool:
     of 6112 x 2304 7.5 9.2), parts 0.63 to 0.99 (8 of 1760 x 3072 6.6 4.3; of longer
     ones up to 1.27).  Full waves of wider tiles are faster (16 of 14336 x 2048 8.8
     10.9), and so are parts that the norm adds up."""
-    if not 1 <= M <= 32 or K % 16 or N % 4 or N * K < 1 << 19 or K > 1 << 17:
+    if not 1 <= M <= 32 or K % 16 or N % 4 or N * K < 1 << 19 or K > 1 << 17 \
+            or N >= 1 << 24:        # not measured; the kernel counts to 2^31
         return False
     tile = _tiles_q(M, N, K, parts)
     return tile is None or tile[1] == 32 or (

@@ -71,7 +71,9 @@ def test_rule_of_few_rows():
             (16, 4096, 14336, False, False), (1, 4096, 14336, True, False),
             (1, 28672, 4096, False, False), (8, 8880, 14592, False, True),
             (0, 4096, 4096, False, False), (1, 4098, 4096, False, False),
-            (1, 4096, 4104, False, False), (1, 64, 1024, False, False)]:
+            (1, 4096, 4104, False, False), (1, 64, 1024, False, False),
+            (1, (1 << 24) - 4, 16, False, True), (1, 1 << 24, 16, False, False),
+            (32, 1 << 31, 16, False, False)]:
         assert ops._rows_q_sizes(M, N, K, parts) == rule, (M, N, K, parts)
 
 
