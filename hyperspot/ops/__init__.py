@@ -705,13 +705,6 @@ def _tiles_q(M: int, N: int, K: int, parts: bool):
     return (64, 32, 1) if tiles <= 128 else (64, 64, 1)
 
 
-def _plain_q(x: "QTensor", w: torch.Tensor, scale: torch.Tensor) -> bool:
-    """Whether csrc/ reads these as they lie, and nothing records the call."""
-    d, s = x
-    return d.is_cuda and unrecorded(d, w, s, scale) \
-        and d.dim() == w.dim() == 2 and d.shape[0] <= 128
-
-
 def _aligned_q(x: "QTensor", w: torch.Tensor, scale: torch.Tensor) -> bool:
     d, s = x
     return d.dtype == w.dtype == torch.float8_e4m3fn \
@@ -724,13 +717,9 @@ def _aligned_q(x: "QTensor", w: torch.Tensor, scale: torch.Tensor) -> bool:
 
 def _tiled_q(x: "QTensor", w: torch.Tensor, scale: torch.Tensor, parts: bool):
     """The tile of _tiles_q, or None."""
-    if not _plain_q(x, w, scale):
-        return None
     tile = _tiles_q(x.data.shape[0], *w.shape, parts)
-    if tile is None or not (_near(x.data, w, *tile[:2])
-                            and _aligned_q(x, w, scale)):
-        return None
-    return tile
+    return tile if tile is not None and _near(x.data, w, *tile[:2]) \
+        and _aligned_q(x, w, scale) else None
 
 
 @lru_cache(maxsize=1 << 14)
@@ -756,17 +745,23 @@ def linear_q(x: "QTensor", w: torch.Tensor, scale: torch.Tensor,
              parts: bool = False):
     """x w^T of e4m3 with scales of the rows, bf16; with `parts` as Parts where
     it is formed in parts of K.  GPU."""
-    # the host's time is what an eager step of small prompts waits for
-    rows = len(x.data) if x.data.dim() == 2 else MOST_ROWS
-    if rows <= 32 and w.dim() == 2 and x.data.shape[1] == w.shape[1] \
-            and _rows_q_sizes(rows, *w.shape, parts) \
-            and _plain_q(x, w, scale) and _aligned_q(x, w, scale) \
-            and _native().gemm_rows_fits(rows, w.shape[1] // 2):
-        out = torch.empty(rows, w.shape[0], dtype=torch.bfloat16,
-                          device=w.device)
-        _native().gemm_rows(out, x.data, w, x.scale, scale)
-        return out
-    tile = _tiled_q(x, w, scale, parts) if rows <= 128 else None
+    # The host's time is what an eager step of small prompts waits for, so rows are
+    # counted first.  But not those of a traced tensor, which a comparison would fix:
+    # their number is no int, or only looks like one to what compiles.
+    d, rows, tile = x.data, None, None
+    if not torch.compiler.is_compiling() and d.dim() == w.dim() == 2:
+        rows = d.shape[0]
+    if type(rows) is int and rows <= 128 and d.is_cuda \
+            and unrecorded(d, w, x.scale, scale):
+        if rows <= 32 and d.shape[1] == w.shape[1] \
+                and _rows_q_sizes(rows, *w.shape, parts) \
+                and _aligned_q(x, w, scale) \
+                and _native().gemm_rows_fits(rows, w.shape[1] // 2):
+            out = torch.empty(rows, w.shape[0], dtype=torch.bfloat16,
+                              device=w.device)
+            _native().gemm_rows(out, d, w, x.scale, scale)
+            return out
+        tile = _tiled_q(x, w, scale, parts)
     if tile is None:
         return torch._scaled_mm(x.data, w.t(), scale_a=x.scale.unsqueeze(1),
                                 scale_b=scale.unsqueeze(0),
