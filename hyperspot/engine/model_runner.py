@@ -68,14 +68,21 @@ def _load_tunableop_results() -> None:
 # 995 -> 886, 4153 -> 2534; 1500 6394 -> 5306, 2467 -> 2132, 7350 -> 5777.  Seven
 # eighths gain less, or lose (1792 rows of wide layers 6437 6774); steps of decoded
 # rows, whose sizes lie closer, stay as they are (150 rows 1764 1813, 130 869 860).
-_EIGHTHS = (5, 6)
+# Each costs a capture at startup: of Llama-3-8B 13 prompt graphs take 0.34 s where 5
+# took 0.16, and all graphs 1068 MB in place of 706.
+#
+# Steps are whole tiles of 32 rows: eighths of any size are not, and latent attention
+# takes 8 rows at a time.
+def _between(size: int) -> List[int]:
+    """The steps below a captured size, from 256 on."""
+    return [-(-size * k // 256) * 32 for k in (5, 6)] if size >= 256 else []
 
 
 def _with_between(sizes) -> List[int]:
     """The sizes, and the steps between those from 256 on."""
     out, before = [], 0
     for s in sizes:
-        out += [s * k // 8 for k in _EIGHTHS if s >= 256 and s * k // 8 > before]
+        out += [t for t in _between(s) if t > before]
         out.append(s)
         before = s
     return out
@@ -85,9 +92,9 @@ def _nearest(n: int, size: int, captured) -> int:
     """`size`, or the smallest captured step below it that holds n: without
     capture_all_graphs there is none, for a step that has to capture first takes the
     sizes themselves."""
-    for k in _EIGHTHS:
-        if n <= size * k // 8 and size * k // 8 in captured:
-            return size * k // 8
+    for t in _between(size):
+        if n <= t and t in captured:
+            return t
     return size
 
 

@@ -258,6 +258,13 @@ def test_steps_between_prefill_sizes():
     assert _with_between((128, 256, 512)) == [128, 160, 192, 256, 320, 384, 512]
     assert _with_between((64, 192, 256)) == [64, 192, 256]
     assert _with_between((1024,)) == [640, 768, 1024] and not _with_between(())
+    # whole tiles: latent attention takes no other number of rows than of 8
+    assert _with_between((264, 1000)) == [192, 224, 264, 640, 768, 1000]
+    for s in range(256, 9000):
+        a, b, c = _with_between((s,))
+        assert a % 32 == b % 32 == 0 and 5 * s <= 8 * a < 8 * b < 8 * c == 8 * s
+        for n, want in ((a, a), (a + 1, b), (b, b), (b + 1, s), (1, a)):
+            assert _nearest(n, s, {a, b, s}) == want
     for n, size, want in ((129, 256, 160), (160, 256, 160), (161, 256, 192),
                           (193, 256, 256), (100, 128, 128), (1, 256, 160)):
         assert _nearest(n, size, {160, 192, 256}) == want
