@@ -20,6 +20,8 @@
 // per head — the pool unit sized for 288 GB HBM3E).
 #include <float.h>
 
+#include <type_traits>
+
 #include "common.h"
 
 #define ATTN_BS 16   // KV page size in tokens
@@ -230,14 +232,23 @@ __global__ __launch_bounds__(256) void paged_attn_kernel(
 // operands; V is turned by an LDS tile of the wave's own and the transposing
 // LDS load, e4m3 pages are widened on the way.  A wave has 32 tokens at a time
 // and issues the next ones' loads as soon as these are in their operands; no
-// barrier until the waves' parts are added up.  Decoded rows read their pages once,
-// by non-temporal loads, which do not wait for a place in the unit's cache: a step
-// of 8 layers of 256 rows of about 1000 tokens 3019 -> 2903 us, of 8 of 8000 1249
+// barrier until the waves' parts are added up.  Decoded rows read pages of their own
+// once, by non-temporal loads, which do not wait for a place in the unit's cache: a
+// step of 8 layers of 256 rows of about 1000 tokens 3019 -> 2903 us, of 8 of 8000 1249
 // -> 1237, of 32 with 4 kv heads 548 -> 537, 1 of 1000 839 -> 833.  Such a load has
 // whole lines: of K 128 bytes of 8 rows, and two exchange halves across lanes (64 of
 // 16 rows, the operands, asked for every line twice): 32 x 4 kv heads of 1000 21.1 ->
 // 19.8 us, 256 x 8 188 -> 182, e4m3 64 x 8 32.2 -> 30.9, but 8 of 8000 in two parts
 // 50.2 50.9; the steps 2918 -> 2888, 1222 -> 1198 and 533 -> 524.
+//
+// Rows that begin with the same prompt share its pages, and pages that others read
+// too are slower so.  They are looked for where one of the next 16 rows begins with
+// the same page: its table is read along, and what both name is loaded as usual.  us
+// with all pages by non-temporal loads, none, and so, 100 tokens of each row's own: 32
+// x 4 kv heads after 1024 shared tokens 17.7 14.7 15.4, 16 x 8 after 8192 75.7 52.6
+// 54.0, 256 x 8 in 8 groups after 4096 each 475 322 320; with 1000 of their own 256 x
+// 8 after 1024 222 228 216; without shared pages 256 x 8 of 1000 170 188 168, 32 x 4
+// 17.9 19.9 18.1, 8 of 8000 47.0 53.6 47.4.
 //
 // us against dot products on the vector units, ragged contexts around the
 // mean: 256 rows x 8 kv heads of 4, 1000 tokens 239 -> 208 (5.0 TB/s), with
@@ -335,6 +346,7 @@ struct Paged {
 };
 
 constexpr unsigned GRID_Y = 65535;
+constexpr int NEAR = 16;             // rows after a row that are looked at
 
 template <bool KV8, bool ROPE>
 __global__ __launch_bounds__(256, 3) void paged_attn_mfma_kernel(Paged a) {
@@ -360,10 +372,19 @@ __global__ __launch_bounds__(256, 3) void paged_attn_mfma_kernel(Paged a) {
       a.seq_start[table + 1] - a.seq_start[table] > a.max_portion)
     return;
   const int ctx = a.ctx_lens[row];
-  // scalar loads also after the stores to the pages
-  const auto bt = (const __attribute__((address_space(4))) int*)
-      (a.block_tables + (long)table * a.max_blocks);
   const int lane = threadIdx.x & 63;
+  // ROPE: where the next rows begin, and how long they are
+  int near_page = 0, near_ctx = 0, near_row = row;
+  if constexpr (ROPE) {
+    near_row += 1 + lane % NEAR;
+    if (near_row >= a.rows) near_row -= a.rows;
+    if (near_row >= a.rows) near_row = row;
+    near_page = a.block_tables[(long)near_row * a.max_blocks];
+    near_ctx = a.ctx_lens[near_row];
+  }
+  // scalar loads also after the stores to the pages
+  typedef const __attribute__((address_space(4))) int* Ints;
+  const auto bt = (Ints)(a.block_tables + (long)table * a.max_blocks);
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 15, gr = lane >> 4;
 
@@ -425,16 +446,27 @@ __global__ __launch_bounds__(256, 3) void paged_attn_mfma_kernel(Paged a) {
   const int last_page = (ctx - 1) / ATTN_BS;
   const int step = 4 * split;
   long b0 = 0, b1 = 0;               // page ids, read one block ahead
+  auto bn = bt;                      // a row that begins as this one,
+  int n0 = 0, shared = 0;            // its page there, and its blocks
+  bool both = false;
+  if constexpr (ROPE) {              // known with the first page: the next row
+    const int next = row + 1 < a.rows ? row + 1 : 0;
+    bn = (Ints)(a.block_tables + (long)next * a.max_blocks);
+    const int of = ((Ints)a.ctx_lens)[next];
+    if (next != row && bn[0] == bt[0]) shared = of / BLOCK;
+  }
   auto pages = [&](int i) {
     b0 = bt[min(2 * i, last_page)];
     b1 = bt[min(2 * i + 1, last_page)];
+    n0 = bn[min(2 * i, last_page)];
+    both = i < shared;
   };
   u32x4 kr[2][KV8 ? 2 : 4], vr[KV8 ? 4 : 8];
-  auto page = [](const char* p) {    // rows of a portion share its pages
-    const auto at = reinterpret_cast<const u32x4*>(p);
-    return ROPE ? __builtin_nontemporal_load(at) : *at;
-  };
-  auto fetch = [&]() {
+  auto load = [&](auto once) {
+    auto page = [](const char* p) {
+      const auto at = reinterpret_cast<const u32x4*>(p);
+      return decltype(once)::value ? __builtin_nontemporal_load(at) : *at;
+    };
     const long p0 = (b0 * a.G + g) * (ATTN_BS * HD * ELEM);
     const long p1 = (b1 * a.G + g) * (ATTN_BS * HD * ELEM);
     const char* kc = static_cast<const char*>(a.k_cache);
@@ -450,6 +482,17 @@ __global__ __launch_bounds__(256, 3) void paged_attn_mfma_kernel(Paged a) {
       vr[i] = page(vc + (i < (KV8 ? 2 : 4) ? p0 : p1) +
                    (i % (KV8 ? 2 : 4)) * 1024 + lane * 16);
   };
+  // Rows of a portion share its pages.  The two ways differ by more than the hint,
+  // or the compiler makes one of them, without it.
+  auto fetch = [&]() {
+    if (!ROPE || (both && n0 == (int)b0)) {
+      load(std::false_type());
+    } else {
+      asm volatile("; read once" ::: "memory");
+      load(std::true_type());
+      asm volatile("; read once" ::: "memory");
+    }
+  };
   char* vl = v_lds[wid];
   const int vr0 = gr * 8 + (col >> 2);
   const int v_at = v_byte(vr0, (col & 3) >> 1) + (col & 1) * 8;
@@ -460,6 +503,17 @@ __global__ __launch_bounds__(256, 3) void paged_attn_mfma_kernel(Paged a) {
     pages(i);
     if (at_once) {
       fetch();
+      if (ROPE && !shared) {         // others, not waited for until here
+        const auto with = __ballot(near_page == bt[0] && near_row != row &&
+                                   near_ctx >= 2 * BLOCK);
+        if (with) {
+          const int l = __ffsll(with) - 1;
+          bn = (Ints)(a.block_tables +
+                      (long)__builtin_amdgcn_readlane(near_row, l) *
+                          a.max_blocks);
+          shared = __builtin_amdgcn_readlane(near_ctx, l) / BLOCK;
+        }
+      }
       if (i + step < blocks) pages(i + step);
     }
   }
@@ -508,7 +562,7 @@ __global__ __launch_bounds__(256, 3) void paged_attn_mfma_kernel(Paged a) {
       }
       if (!at_once && i < blocks) {
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
-        fetch();
+        load(std::true_type());
       }
     }
   }
@@ -761,6 +815,8 @@ void launch_rope_paged_attn(bf16* out, const bf16* q, const bf16* k,
                             int max_blocks, float scale, long qs, long ks,
                             long vs, float* split_ws, int split, bool kv_fp8,
                             hipStream_t stream) {
+  // every row's first page is read, also where no row has a page
+  if (max_blocks == 0) block_tables = ctx_lens;
   launch_mfma<true>({out, q, k_cache, v_cache, block_tables, ctx_lens, nullptr,
                      nullptr, 0, max_blocks, num_kv_heads, group,
                      scale * LOG2E, qs, split_ws, k, v, cos_sin, positions,

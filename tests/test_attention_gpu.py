@@ -178,6 +178,52 @@ def test_rope_in_decode_attention(lens, group, kv, fp8):
     assert (outs[0] - outs[1]).abs().max() <= 2.0 ** -8 * outs[1].abs().max()
 
 
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("rows,kv,groups,shared", [
+    (2, 1, 1, 16), (3, 2, 1, 32), (5, 2, 2, 48), (17, 1, 16, 96), (18, 1, 18, 512),
+    (33, 2, 17, 80), (40, 8, 3, 176), (8, 1, 1, 1600)])
+def test_pages_of_shared_prompts(rows, kv, groups, shared, fp8):
+    """Rows that begin with the same pages, one after the other or at a distance,
+    some as long as those, against copies of the pages for every row: same bits."""
+    g = torch.Generator().manual_seed(rows)
+    group, kind = 4, torch.float8_e4m3fn if fp8 else torch.bfloat16
+    heads, first = group * kv, shared // 16
+    lens = torch.randint(shared + 1, shared + 150, (rows,), generator=g)
+    lens[rows // 2:rows // 2 + 2] = shared + 1
+    own = -(-lens // 16) - first
+    total = groups * first + int(own.sum())
+    caches = [torch.randn(total, kv, 16, D, generator=g).to(kind)
+              for _ in range(2)]
+    order = torch.randperm(total, generator=g).int()
+    bt = torch.zeros(rows, first + int(own.max()) + 1, dtype=torch.int32)
+    at = groups * first
+    for i in range(rows):
+        bt[i, :first] = order[i % groups * first:][:first]
+        bt[i, first:first + own[i]] = order[at:at + own[i]]
+        at += int(own[i])
+    each = torch.arange(bt.numel(), dtype=torch.int32).view_as(bt)
+    cos_sin = torch.randn(2000, D, generator=g).to(DEV)
+    qkv = torch.randn(rows, heads + 2 * kv, D, generator=g).bfloat16().to(DEV)
+    outs, pages = [], []
+    for table, kept in ((bt, caches),
+                        (each, [c[bt.flatten().long()] for c in caches])):
+        last = table.gather(1, (lens - 1).div(16, rounding_mode="floor")[:, None])
+        slots = (last[:, 0].long() * 16 + (lens - 1) % 16).to(DEV)
+        meta = ForwardMeta("decode", (lens - 1).to(DEV), slots,
+                           block_tables=table.to(DEV),
+                           seq_lens=lens.int().to(DEV))
+        kc, vc = (c.clone().to(DEV) for c in kept)
+        q, k, v = qkv.clone().split([heads, kv, kv], 1)
+        assert ops._rope_in_attention(q, k, v, kc, meta)
+        outs.append(ops.rope_attention(q, k, v, meta.positions, cos_sin, slots,
+                                       kc, vc, meta, D ** -0.5))
+        pages.append([c.view(torch.uint8)[last[:, 0].long().to(DEV)]
+                      for c in (kc, vc)])
+    assert torch.isfinite(outs[0].float()).all()
+    assert torch.equal(*outs)
+    assert all(torch.equal(a, b) for a, b in zip(*pages))
+
+
 @pytest.mark.parametrize("parts", [2, 15, 16, 17, 33, 64])
 def test_parts_of_decode_attention(parts):
     """More parts than one has 32 tokens for, and than are loaded at a time."""
