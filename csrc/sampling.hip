@@ -77,13 +77,15 @@ __global__ __launch_bounds__(256) void greedy_sample_kernel(
 // are looked at together where that decides about all of them.  Where few values
 // stay, and next-token logits have a few dozen that matter, they are listed and the
 // rest is done on the list, up to 8 threads a value; n values take n^2 steps, so a
-// share is looked for among 64 first (21.9 -> 19.7 us), then among 128.  Otherwise
-// no sort either: one histogram of counts and weights over 2048 equal steps between
-// the largest and the smallest logit finds the step where the wanted count or share
-// is reached, and ranks the few values in it exactly (or divides that step again).
-// Equal steps of the logit, and not digits of its bit pattern, because next-token
-// logits fill few exponents: 64 lanes that add to the same few counters in LDS would
-// go one by one.
+// share is looked for among 64 first (21.9 -> 19.7 us), then among 128, which is
+// where a share of 65 to 128 values is found: with both lists 28 us of 64 rows of
+// 128256, with 128 at once 25, as other shares then take too in place of 22.
+// Otherwise no sort either: one histogram of counts and weights over 2048 equal steps
+// between the largest and the smallest logit finds the step where the wanted count or
+// share is reached, and ranks the few values in it exactly (or divides that step
+// again).  Equal steps of the logit, and not digits of its bit pattern, because
+// next-token logits fill few exponents: 64 lanes that add to the same few counters in
+// LDS would go one by one.
 //
 // 64 rows of 128256, 48 values far above the others, us with a workgroup a row
 // and now, rows in cache (from memory 2 to 3 more): temperature 36 14, top_p 0.9
@@ -523,11 +525,21 @@ DEV bool draw_from_list(Scratch& s, const Weight& w, int vocab, int k, float p,
   }
   // in descending order, and by index among equals, larger keys are earlier;
   // the zeros are equal
-  if (tid < n)
+  u64 mass = 0;
+  if (tid < n) {
+    mass = w(s.list[tid]);
     s.entry[tid] = {(u64)ordered(s.list[tid] + 0.f) << 32 |
                         (unsigned)~s.list_at[tid],
-                    w(s.list[tid])};
+                    mass};
+  }
   if (tid == 0) s.found = vocab - 1;
+  // a list that is too short is left before its values are ranked
+  const bool share_of_all = k == 0 && p < 1.f;
+  const u64 part_of = share_of_all ? (u64)ceil((double)p * (double)z) : 0;
+  if (share_of_all && sum_of_all(s, mass) < part_of) {
+    __syncthreads();
+    return false;
+  }
   __syncthreads();
   // `share` neighbouring threads a value, each with a part of the others
   const int share = n <= NT / 8 ? 8 : n <= NT / 4 ? 4 : 2;
@@ -552,14 +564,12 @@ DEV bool draw_from_list(Scratch& s, const Weight& w, int vocab, int k, float p,
   above = sum(above);
   greater = sum(greater);
   bool stays = one_of && (k == 0 || greater < k);
-  const u64 listed = sum_of_all(s, stays && part == 0 ? own.mass : 0);
-  if (p < 1.f) {
-    const u64 want = (u64)ceil((double)p * (double)(k ? listed : z));
-    if (listed < want) {
-      __syncthreads();
-      return false;
-    }
-    stays = stays && above < want;
+  if (p < 1.f && !share_of_all) {
+    const u64 kept = sum_of_all(s, stays && part == 0 ? own.mass : 0);
+    stays = stays && above < (u64)ceil((double)p * (double)kept);
+  } else {
+    stays = stays && (!share_of_all || above < part_of);
+    __syncthreads();
   }
   // every thread has read the entries: now by index, what does not stay as 0
   const int index = (int)~(unsigned)own.key;
@@ -622,6 +632,7 @@ DEV bool draw_from_few(Scratch& s, const R& row, const Weight& w, float own,
         }
   });
   z = sum_of_all(s, z);
+  __syncthreads();                // the list's sum goes the same way
   *all = z;
   return draw_from_list(s, w, row.vocab, k, p, u, z, drawn);
 }
