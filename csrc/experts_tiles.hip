@@ -54,14 +54,16 @@ void experts_tiles_kernel(Tiles a) {
   const int last = a.expert[max(tile - 1, 0)];
   const int next = a.expert[min(tile + 1, tiles - 1)];
   if (e < 0) return;
-  // Of 256 rows weights that one tile takes are read once (ONCE), those of several
-  // not; smaller tiles are taken where most experts have one.  us, up and down of 8
-  // experts of 14336 x 4096, 112 choices each 718 -> 660, 160 752 -> 722, of 16 of
-  // 2048 x 4096, 112 226 -> 214; those of several tiles by ONCE 1.1 times slower.
-  // (Tiles of 64 and 128 rows with both ways: two tiles an expert 0.9, one 1.02.)
-  const bool alone =
-      BM < 256 || (((tile == 0) | (last != e)) &
-                   ((tile + 1 == tiles) | (next != e)));
+  // Weights that one tile takes are read once (ONCE), those of several not: they
+  // would leave the others nothing.  us, up and down of 8 experts of 14336 x 4096,
+  // 112 choices each 718 -> 660, 160 752 -> 722, of 16 of 2048 x 4096, 112 226 ->
+  // 214; those of several tiles of 256 by ONCE 1.1 times slower.  Where tokens prefer
+  // the same experts, smaller tiles are several too, by ONCE and so: 300 choices of
+  // each of 2 experts of 16 in tiles of 64 95 -> 71, 64 experts of 1024 x 2048, up to
+  // 190 each 104 -> 92, 150 of each of 2 of 8 343 -> 305, 100 to 200 uneven tokens of
+  // 8 604 -> 577 and 606 -> 588; even ones 440 442, 138 138, 149 149.
+  const bool alone = ((tile == 0) | (last != e)) &
+                     ((tile + 1 == tiles) | (next != e));
   // The tiles of an expert that take the same weights go to one die together,
   // whose L2 then has them, where an expert has 128 MB of them, half of what the
   // memory's cache holds: later tiles would find them gone.  180 random sizes (2
@@ -163,7 +165,7 @@ void experts_tiles_kernel(Tiles a) {
   };
   if (alone)
     run(std::true_type());
-  else if constexpr (BM == 256)
+  else
     run(std::false_type());
   auto& acc = loop.acc;
 
