@@ -536,11 +536,12 @@ DEV bool draw_from_list(Scratch& s, const Weight& w, int vocab, int k, float p,
   // a list that is too short is left before its values are ranked
   const bool share_of_all = k == 0 && p < 1.f;
   const u64 part_of = share_of_all ? (u64)ceil((double)p * (double)z) : 0;
-  if (share_of_all && sum_of_all(s, mass) < part_of) {
+  if (!share_of_all) {
+    __syncthreads();
+  } else if (sum_of_all(s, mass) < part_of) {    // a barrier on the way
     __syncthreads();
     return false;
   }
-  __syncthreads();
   // `share` neighbouring threads a value, each with a part of the others
   const int share = n <= NT / 8 ? 8 : n <= NT / 4 ? 4 : 2;
   const int mine = tid / share, part = tid % share;
