@@ -310,17 +310,6 @@ DEV float2 turn(float x, float y, float c, float s) {
   return make_float2(fmaf(x, c, -(y * s)), fmaf(y, c, x * s));
 }
 
-// a: 64 bytes of rows 0 to 7 in lanes 0 to 7 of each 16 and 64 more in the others,
-// b: the same of rows 8 to 15; then a has the first bytes of all rows, b the others
-DEV void exchange_halves(u32x4& a, u32x4& b) {
-  #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int x = a[j], y = b[j];
-    a[j] = __builtin_amdgcn_update_dpp(x, y, 0x128, 15, 0xc, false);
-    b[j] = __builtin_amdgcn_update_dpp(y, x, 0x128, 15, 0x3, false);
-  }
-}
-
 struct Paged {
   bf16* out;
   const bf16* q;

@@ -527,8 +527,7 @@ void experts_tiles(Tensor out, Tensor x, Tensor w, Maybe x_scale,
                        (int)K, (int)div, (int)bm, stream());
 }
 
-// choices and weights of the rows of x [T, W], bf16 or e4m3 with x_scale [T]
-// slots of T rows, or null; pointer of it
+// slots of T rows, or null
 const long* slots_of(const c10::optional<Tensor>& slots, long T) {
   if (!slots.has_value()) return nullptr;
   check(*slots, torch::kLong, "slots");
@@ -536,6 +535,8 @@ const long* slots_of(const c10::optional<Tensor>& slots, long T) {
   return slots->data_ptr<long>();
 }
 
+// choices and weights of the rows of x [T, W], bf16 or e4m3 with x_scale [T]; a row
+// whose slot is negative is padding: numbers -1, weights 0
 void experts_router(Tensor weight, Tensor ids, Tensor x, Maybe x_scale,
                     Tensor router, long top, c10::optional<Tensor> slots) {
   check(x, x_scale.has_value() ? torch::kFloat8_e4m3fn : torch::kBFloat16,
@@ -556,7 +557,7 @@ void experts_router(Tensor weight, Tensor ids, Tensor x, Maybe x_scale,
 }
 
 // out <- rmsnorm(residual + x) * norm, residual that sum, and the choices and
-// weights of out's rows; x bf16 [T, W] or float parts [parts, T, W]
+// weights of out's rows, as above; x bf16 [T, W] or float parts [parts, T, W]
 void norm_router(Tensor weight, Tensor ids, Tensor out, Tensor x,
                  Tensor residual, Tensor norm, double eps, Tensor router,
                  long top, c10::optional<Tensor> slots) {

@@ -201,6 +201,21 @@ DEV f32x16_t mfma32(short8_t a, short8_t b, f32x16_t c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
 }
 
+// Two loads have whole lines of 8 rows each, operands half the lines of 16 rows.  a: 64
+// bytes of rows 0 to 7 in lanes 0 to 7 of each 16 and 64 more in the others, b: the same
+// of rows 8 to 15; then a has the first bytes of all rows, b the others
+template <typename V> DEV void exchange_halves(V& a, V& b) {
+  union { V v; int d[4]; } x{a}, y{b}, u, w;
+  static_assert(sizeof(V) == 16, "16 bytes a lane");
+  #pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    u.d[j] = __builtin_amdgcn_update_dpp(x.d[j], y.d[j], 0x128, 15, 0xc, false);
+    w.d[j] = __builtin_amdgcn_update_dpp(y.d[j], x.d[j], 0x128, 15, 0x3, false);
+  }
+  a = u.v;
+  b = w.v;
+}
+
 // ---- reductions ---------------------------------------------------------
 // The lanes are combined in the vector registers: a permute through LDS takes some
 // 50 ns, six of them one after the other a tenth of a row's norm (decode steps of 8

@@ -61,19 +61,6 @@ DEV void to_lds16(const void* g, void* l) {
       (__attribute__((address_space(3))) unsigned*)l, 16, 0, 0);
 }
 
-// Two loads have whole lines of 8 rows each, operands half the lines of 16 rows:
-// lanes 8 to 15 of each 16 exchange theirs with lanes 0 to 7
-DEV void turn(short8_t* f, const short8_t* l) {
-  union V { short8_t s; int d[4]; } a{l[0]}, b{l[1]}, x, y;
-  #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    x.d[j] = __builtin_amdgcn_update_dpp(a.d[j], b.d[j], 0x128, 15, 0xc, false);
-    y.d[j] = __builtin_amdgcn_update_dpp(b.d[j], a.d[j], 0x128, 15, 0x3, false);
-  }
-  f[0] = x.s;
-  f[1] = y.s;
-}
-
 // 32 products of a lane's 16 bytes, or 64 of e4m3
 template <bool FP8>
 DEV f32x4_t products_of(short8_t a, short8_t b, f32x4_t c) {
@@ -155,7 +142,11 @@ void gemm_rows_kernel(Rows a) {
 
   while (tile < tiles) {
     #pragma unroll
-    for (int u = 0; u < U; ++u) turn(wf[u], wn[u]);
+    for (int u = 0; u < U; ++u) {
+      wf[u][0] = wn[u][0];
+      wf[u][1] = wn[u][1];
+      exchange_halves(wf[u][0], wf[u][1]);
+    }
     const int k0 = batch * U * STEP + wid * 64, now = tile;
     if (++batch == batches) {
       batch = 0;
