@@ -248,7 +248,9 @@ __global__ __launch_bounds__(256) void paged_attn_kernel(
 // x 4 kv heads after 1024 shared tokens 17.7 14.7 15.4, 16 x 8 after 8192 75.7 52.6
 // 54.0, 256 x 8 in 8 groups after 4096 each 475 322 320; with 1000 of their own 256 x
 // 8 after 1024 222 228 216; without shared pages 256 x 8 of 1000 170 188 168, 32 x 4
-// 17.9 19.9 18.1, 8 of 8000 47.0 53.6 47.4.
+// 17.9 19.9 18.1, 8 of 8000 47.0 53.6 47.4.  Steps of 8 layers, all non-temporal and
+// so: 32 narrow rows after 1024 shared tokens 502 -> 481, 16 after 8192 1306 -> 1234, 64
+// after 2048 1311 -> 1293, 256 after 512 2344 -> 2331.
 //
 // us against dot products on the vector units, ragged contexts around the
 // mean: 256 rows x 8 kv heads of 4, 1000 tokens 239 -> 208 (5.0 TB/s), with
