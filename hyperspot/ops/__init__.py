@@ -881,6 +881,9 @@ def moe_router(x, router: torch.Tensor, top: int,
 #     119, 48 - 93 91 121, 112 - 146 129 126, 125 - 150 133 129
 #   64 of 1024 x 2048           1 row 94 101, 3 rows 131 129, 5 154 134, 48 -
 #     163 172 228, 112 - 279 222 242, 125 - 309 257 247
+# Choices that are uneven are better in the next larger tiles where several experts
+# have a little more than a tile: 190 tokens of 8 experts, 47.5 choices on average, up
+# to 56 458 512, up to 84 588 511, up to 127 556 514, up to 150 640 688.
 MOE_ROWS, MOE_ROWS_64, MOE_ROWS_128 = 2.9, 48, 112
 
 
