@@ -58,8 +58,8 @@ void launch_norm_router(float*, int*, bf16*, const bf16*, const float*, int,
                         bf16*, const bf16*, float, const bf16*, const long*,
                         long, int, int, int, hipStream_t);
 void launch_experts_tiles(bool, bf16*, const void*, const void*, const float*,
-                          const float*, const int*, const int*, long, int, int,
-                          int, int, int, hipStream_t);
+                          const float*, const int*, const int*, int, long, int,
+                          int, int, int, int, hipStream_t);
 void launch_experts_sort(int*, int*, int*, const int*, int, int, int, int,
                          hipStream_t);
 void launch_experts_route_sort(float*, int*, int*, int*, int*, const float*,
@@ -523,8 +523,8 @@ void experts_tiles(Tensor out, Tensor x, Tensor w, Maybe x_scale,
   }
   launch_experts_tiles(gated, ptr<bf16>(out), x.data_ptr(), w.data_ptr(),
                        opt(x_scale), opt(w_scale), order.data_ptr<int>(),
-                       expert.data_ptr<int>(), x.size(0), (int)tiles, (int)N,
-                       (int)K, (int)div, (int)bm, stream());
+                       expert.data_ptr<int>(), (int)E, x.size(0), (int)tiles,
+                       (int)N, (int)K, (int)div, (int)bm, stream());
 }
 
 // slots of T rows, or null

@@ -347,7 +347,9 @@ __global__ __launch_bounds__(1024) void norm_router_kernel(
   }
 }
 
-// One workgroup.  order[pos] = choice (-1: padding), expert[tile] (-1: none),
+// One workgroup.  Tiles of 256 are as even as blocks of 32 let them be, for a product's
+// tile costs what it holds (302 choices are 160 and 142, not 256 and 46); smaller ones
+// are full but for an expert's last.  order[pos] = choice (-1: padding), expert[tile] (-1: none),
 // place[choice] = pos (-1: an identity expert).  ROUTE: the choices are made
 // here first.
 template <int LE, bool ROUTE>
@@ -358,6 +360,8 @@ __global__ __launch_bounds__(1024) void sort_kernel(
   extern __shared__ int lds[];
   int* cnt = lds;                    // choices per expert
   int* cur = lds + kinds;            // next free position
+  int* high = lds + 2 * kinds;       // choices a tile
+  int* from = lds + 3 * kinds;       // first position
   __shared__ int wave_sum[16];
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
   for (int e = tid; e < kinds; e += 1024) cnt[e] = 0;
@@ -390,15 +394,26 @@ __global__ __launch_bounds__(1024) void sort_kernel(
     }
     const int first = before + x - n;
     if (e < kinds) {
-      cur[e] = first * bm;
+      cur[e] = 0;
+      high[e] = bm == 256 && n ? ((cnt[e] + n - 1) / n + 31) & ~31 : bm;
+      from[e] = first * bm;
       for (int t = first; t < first + n && t < tiles; ++t) expert[t] = e;
     }
     base = total;
     __syncthreads();
   }
   for (int p = tid; p < choices; p += 1024) {
-    const int pos = ids[p] < 0 ? -1 : atomicAdd(&cur[ids[p]], 1);
-    if (pos >= 0) order[pos] = p;
+    const int e = ids[p];
+    int pos = -1;
+    if (e >= 0) {
+      // tile and row by a reciprocal: divisions took 2 us for 32000 choices
+      const int at = atomicAdd(&cur[e], 1), h = high[e];
+      int t = (int)(at * __builtin_amdgcn_rcpf(h)), row = at - t * h;
+      for (; row < 0; row += h) --t;
+      for (; row >= h; row -= h) ++t;
+      pos = from[e] + t * bm + row;
+      order[pos] = p;
+    }
     place[p] = pos;
   }
 }
@@ -715,7 +730,7 @@ void launch_norm_router(float* weight, int* ids, bf16* out, const bf16* x,
 void launch_experts_sort(int* order, int* expert, int* place, const int* ids,
                          int choices, int kinds, int bm, int tiles,
                          hipStream_t stream) {
-  sort_kernel<1, false><<<1, 1024, 2 * kinds * sizeof(int), stream>>>(
+  sort_kernel<1, false><<<1, 1024, 4 * kinds * sizeof(int), stream>>>(
       Route{}, order, expert, place, ids, choices, kinds, bm, tiles);
 }
 
@@ -736,7 +751,7 @@ void launch_experts_route_sort(float* weight, int* ids, int* place,
   const Route r{weight, ids, logits, T, E, top, shared, shared, E + identity,
                 correction};
   #define RUN(LE)                                                           \
-    sort_kernel<LE, true><<<1, 1024, 2 * kinds * sizeof(int), stream>>>(    \
+    sort_kernel<LE, true><<<1, 1024, 4 * kinds * sizeof(int), stream>>>(    \
         r, order, expert, place, ids, choices, kinds, bm, tiles)
   BY_EXPERTS(RUN);
   #undef RUN

@@ -13,12 +13,10 @@
 // its own.
 //
 // What bounds it: the weights' bytes up to about 100 choices an expert, so bm
-// is what covers most counts (256 rows of x, mostly padding, beside 128 of
-// weights are two thirds of what is loaded), then the products.  Mixtral 8x7B
-// layer (8 experts, 14336 x 4096, 2.8 GB), us with 256-row tiles, row tiles
-// and here: 16 choices an expert 821 617 473, 48 831 792 487, 128 943 869 719,
-// 500 2355 2100 1650.  32 experts of 1024 x 2048, 62 choices 277 172 96.  With
-// weights by non-temporal loads 443, 459, 686 and 1550; 95.
+// is what covers most counts, then the products.  Mixtral 8x7B layer (8 experts,
+// 14336 x 4096, 2.8 GB), us: 16 choices an expert 443, 48 459, 128 650, 302 906, 500
+// 1210.  32 experts of 1024 x 2048, 62 choices 95.
+#include <algorithm>
 #include <type_traits>
 
 #include "tile_loop.h"
@@ -36,6 +34,61 @@ struct Tiles {
   int N, K, div, nx;           // N outputs a choice, nx blocks of them
 };
 
+DEV int row_of(const Tiles& a, int p) {
+  const int choice = a.order[p];
+  return a.div ? (choice >= 0 ? choice / a.div : 0) : p;
+}
+
+// The sums of a wave, of choices p0 on and outputs n0 on.  acc[n][m][r]: weight row
+// (r >> 2) * 8 + hf * 4 + (r & 3) of block n, choice col of block m.
+template <bool GATED, bool FP8, int NI, int MI>
+DEV void store_tile(const Tiles& a, const f32x16_t (&acc)[NI][MI], int e,
+                    int p0, int n0) {
+  const int lane = threadIdx.x & 63, col = lane & 31, hf = lane >> 5;
+  #pragma unroll
+  for (int m = 0; m < MI; ++m) {
+    const int p = p0 + m * 32 + col;
+    if (a.order[p] < 0) continue;
+    bf16* op = a.out + (long)p * a.N + n0 + hf * 4;
+    const float xs = FP8 ? a.x_scale[row_of(a, p)] : 1.f;
+    #pragma unroll
+    for (int n = 0; n < NI; ++n) {
+      if constexpr (GATED) {
+        #pragma unroll
+        for (int r = 0; r < 16; r += 8) {
+          float y[4];
+          #pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const float g = acc[n][m][r + j], u = acc[n][m][r + 4 + j];
+            y[j] = g / (1.f + __expf(-g)) * u;
+          }
+          *reinterpret_cast<uint2*>(op + n * 16 + r) =
+              uint2{cvt_pk_bf16(y[0], y[1]), cvt_pk_bf16(y[2], y[3])};
+        }
+      } else {
+        #pragma unroll
+        for (int r = 0; r < 16; r += 4) {
+          float y[4];
+          #pragma unroll
+          for (int j = 0; j < 4; ++j) y[j] = acc[n][m][r + j];
+          if constexpr (FP8) {
+            const float4 ws = *reinterpret_cast<const float4*>(
+                a.w_scale + (long)e * a.N + n0 + n * 32 + r * 2 + hf * 4);
+            y[0] = y[0] * xs * ws.x;
+            y[1] = y[1] * xs * ws.y;
+            y[2] = y[2] * xs * ws.z;
+            y[3] = y[3] * xs * ws.w;
+          }
+          *reinterpret_cast<uint2*>(op + n * 32 + r * 2) =
+              uint2{cvt_pk_bf16(y[0], y[1]), cvt_pk_bf16(y[2], y[3])};
+        }
+      }
+    }
+  }
+}
+
+constexpr int HIGH_BYTES = 160 << 10;      // of LDS
+
 // BM choices, BN rows of weights; WM * WN waves have BM / WM by BN / WN
 template <int BM, int BN, int WM, int WN, int STAGES, bool GATED, bool FP8,
           bool FAR>
@@ -43,12 +96,12 @@ __global__ __launch_bounds__(WM * WN * 64,
                              WM * WN == 4 ? 2 : WM * WN / 4)
 void experts_tiles_kernel(Tiles a) {
   using Loop = TileLoop<BM, BN, WM, WN, STAGES, 1, FP8>;
-  constexpr int LX = Loop::LX, LW = Loop::LW, NI = Loop::NI, MI = Loop::MI;
+  constexpr int LX = Loop::LX, LW = Loop::LW;
   constexpr int OUT = GATED ? BN / 2 : BN;                 // outputs
   constexpr int ELEM = FP8 ? 1 : 2;
   static_assert(!(GATED && FP8), "the activation's scale needs whole rows");
   extern __shared__ __attribute__((aligned(16))) char lds[];
-  int tile = blockIdx.x / a.nx, nb = blockIdx.x % a.nx;
+  const int tile = blockIdx.x / a.nx, nb = blockIdx.x % a.nx;
   const int tiles = gridDim.x / a.nx;
   const int e = a.expert[tile];
   const int last = a.expert[max(tile - 1, 0)];
@@ -64,34 +117,9 @@ void experts_tiles_kernel(Tiles a) {
   // 8 604 -> 577 and 606 -> 588; even ones 440 442, 138 138, 149 149.
   const bool alone = ((tile == 0) | (last != e)) &
                      ((tile + 1 == tiles) | (next != e));
-  // The tiles of an expert that take the same weights go to one die together,
-  // whose L2 then has them, where an expert has 128 MB of them, half of what the
-  // memory's cache holds: later tiles would find them gone.  180 random sizes (2
-  // to 16 experts, 100 to 1100 choices each, N of 2048 to 16384, K of 1024 to
-  // 15000), time over that without: 256 x 256 from 128 MB on 0.962, two of 29 more
-  // than 1.2 % slower (16 of 16384 x 5760, 1060 choices 6666 -> 6335 us, 8 of 16384
-  // x 2432, 590 841 -> 767, 8 of 8192 x 14080, 320 1.041), with 50 to 128 MB 0.997,
-  // with less 1.024; 256 x 128, which are fewer, 1.032 (2 of 10240 x 3072 77 ->
-  // 96).  More than 32 tiles share them without it.
-  if (BM == 256 && BN == 256 && a.nx % 8 == 0 &&
-      (GATED ? 2 : 1) * a.N * ((long)a.K * ELEM) >= 128l << 20) {
-    const int t = threadIdx.x & 63;
-    const unsigned long back =
-        ~__ballot(t <= tile && a.expert[t <= tile ? tile - t : 0] == e);
-    const unsigned long on = ~__ballot(
-        tile + t < tiles && a.expert[tile + t < tiles ? tile + t : 0] == e);
-    const int before = (back ? __builtin_ctzll(back) : 64) - 1;
-    const int count = before + (on ? __builtin_ctzll(on) : 64);
-    if (count <= 32) {
-      const int at = before * a.nx + nb;
-      nb = at / (8 * count) * 8 + at % 8;
-      tile += at / 8 % count - before;
-    }
-  }
   const int n0 = nb * OUT, p0 = tile * BM;
   const int lane = threadIdx.x & 63;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int col = lane & 31, hf = lane >> 5;
   // a SIMD has waves of different choices: those without any do nothing
   const int wm = wid / WN, wn = wid % WN;
   const bool live = a.order[p0 + wm * (BM / WM)] >= 0;
@@ -100,10 +128,6 @@ void experts_tiles_kernel(Tiles a) {
   const int lr = lane >> 3;
   auto column = [&](int r) { return ((lane & 7) ^ (r >> 1 & 7)) * 16; };
   const long row_bytes = (long)a.K * ELEM;
-  auto row_of = [&](int p) {
-    const int choice = a.order[p];
-    return a.div ? (choice >= 0 ? choice / a.div : 0) : p;
-  };
   auto w_row = [&](int r) {    // gated: 8 gate rows, then their 8 up rows
     return GATED ? (r >> 4) * 8 + (r & 7) + (r & 8 ? a.N : 0) : r;
   };
@@ -115,7 +139,7 @@ void experts_tiles_kernel(Tiles a) {
   #pragma unroll
   for (int j = 0; j < LX; ++j) {
     const int r = (wid * LX + j) * 8 + lr;
-    x_off[j] = (row_of(p0 + r) - (a.div ? 0 : p0)) * row_bytes + column(r);
+    x_off[j] = (row_of(a, p0 + r) - (a.div ? 0 : p0)) * row_bytes + column(r);
   }
   #pragma unroll
   for (int j = 0; j < LW; ++j) {
@@ -137,14 +161,14 @@ void experts_tiles_kernel(Tiles a) {
   // that not all of them ask the same channels of memory at once; those of one
   // expert and the same outputs at the same.  192 tokens of 2 choices, 8 experts
   // of 14336 x 4096 355 + 188 -> 321 + 162 us; 4 of 32 of 1024 x 2048 65 + 29 ->
-  // 50 + 29; in tiles of 256, 500 choices an expert, 1011 + 639 1029 + 643.
+  // 50 + 29.
   // Three times as far apart where rows are long: 140 random sizes (4 to 64
   // experts, K of 1024 to 14336), time over that of once as far: rows of 12 KB and
   // more 0.984, 8 and 10 KB in tiles of 128 0.985, of 64 1.02 (16 of 4096 x 4096,
   // 22 choices each, 99 108), shorter ones 1.01 (64 of 3072 x 2048 150 162).
   const int stages = (int)(row_bytes / 128);
   const int apart = stages >= (BM == 64 ? 96 : 64) ? 3 : 1;
-  const int turn = BM == 256 ? 0 : (nb + e * a.nx) / 8 * apart % stages;
+  const int turn = (nb + e * a.nx) / 8 * apart % stages;
   // load i of a stage: first those of x, then those of w
   auto stage = [&](auto once, int slot, int d, int i) {
     d += turn;
@@ -167,51 +191,161 @@ void experts_tiles_kernel(Tiles a) {
     run(std::true_type());
   else
     run(std::false_type());
-  auto& acc = loop.acc;
+  store_tile<GATED, FP8>(a, loop.acc, e, p0 + wm * (BM / WM),
+                         n0 + wn * (OUT / WN));
+}
 
-  // acc[n][m][r]: weight row (r >> 2) * 8 + hf * 4 + (r & 3) of block n,
-  // choice col of block m
+// A tile of up to 256 choices, as high as it has choices: H blocks of 32, and BN rows
+// of weights.  Of the 8 waves 4 have the first blocks of every kind, 4 the others, MB
+// each, and the two of a SIMD are one of both, so that all SIMDs have the same
+// products if H is odd too.  bf16: 2 of the 4 share the choices, and every second wave
+// has the same half of the weights; blocks of 16.  e4m3: each has a quarter of the
+// weights; blocks of 32.  What is not there is neither formed nor loaded.
+//
+// What bounds it: 160 x 256 what a unit loads, 52 KB a chunk at some 45 GB/s, and the
+// products (8 experts of 14336 x 4096, 302 choices each, up 500 us without products, 440
+// without loads, 613 with both), larger ones power.  us, with tiles of 256 of which the
+// last of an expert is mostly padding, two stages and 32 x 32 products, and here, up and
+// down: 302 choices 743 431 and 613 293, 512 872 473 and 817 394, 2000 3168 1593 and
+// 2912 1428, 130 454 232 and 430 211; 16 of 2048 x 4096, 300 239 132 and 170 95; 32 of
+// 1024 x 2048, 300 131 89 and 92 67, 1000 264 169 and 255 147.  e4m3: 302 404 216 and
+// 335 146, 2000 1815 943 and 1671 752.  Even: two workgroups of one expert with its
+// choices together and half of the weights each; weights begun at different columns.
+template <int H, bool LATER, int BN, bool GATED, bool FP8, bool FAR>
+DEV void high_tile_part(const Tiles& a, char* lds, int e, int p0, int nb,
+                        bool alone) {
+  constexpr int BM = H * 32, OUT = GATED ? BN / 2 : BN;
+  constexpr int MB = LATER ? H / 2 : H - H / 2, FIRST = LATER ? H - H / 2 : 0;
+  constexpr int PARTS = FP8 ? 4 : 2;           // of the weights
+  constexpr int B = FP8 ? 32 : 16, NB = BN / PARTS / B, LW = BN / 64;
+  constexpr int ROWS = MB ? MB : 1;
+  using Loop = RingLoop<BM, BN, ROWS, NB, MB, LW, FP8>;
+  const int n0 = nb * OUT;
+  const int lane = threadIdx.x & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int part = wid % PARTS;
+  const int x_row = FIRST * 32 + (wid & 3) / PARTS * (MB * B);
+  const int lr = lane >> 3;
+  auto column = [&](int r) { return ((lane & 7) ^ (r >> 1 & 7)) * 16; };
+  const long row_bytes = (long)a.K * (FP8 ? 1 : 2);
+  const char* x0 = static_cast<const char*>(a.x) + (a.div ? 0 : p0 * row_bytes);
+  const char* w0 = static_cast<const char*>(a.w) +
+                   ((long)e * (GATED ? 2 * a.N : a.N) + n0) * row_bytes;
+  const RowLoads x_rows(x0), w_rows(w0);
+  using Offset = std::conditional_t<FAR, long, unsigned>;
+  Offset x_off[ROWS], w_off[LW];
   #pragma unroll
-  for (int m = 0; m < MI; ++m) {
-    const int p = p0 + (wm * MI + m) * 32 + col;
-    if (a.order[p] < 0) continue;
-    bf16* op = a.out + (long)p * a.N + n0 + hf * 4;
-    const float xs = FP8 ? a.x_scale[row_of(p)] : 1.f;
+  for (int j = 0; j < MB; ++j) {
+    const int r = FIRST * 32 + ((wid & 3) * MB + j) * 8 + lr;
+    x_off[j] = (Offset)((row_of(a, p0 + r) - (a.div ? 0 : p0)) * row_bytes +
+                        column(r));
+  }
+  #pragma unroll
+  for (int j = 0; j < LW; ++j) {
+    const int r = (wid * LW + j) * 8 + lr;
+    const int n = FP8 ? plain_row_32(r) : GATED ? gated_row(r, a.N) : plain_row(r);
+    w_off[j] = (Offset)(n * row_bytes + column(r));
+  }
+  auto load = [&](auto once, char* l, const RowLoads& rows, const char* base,
+                  Offset off, int d) {
+    constexpr int AUX = decltype(once)::value ? ONCE : 0;
+    if constexpr (FAR)
+      __builtin_amdgcn_global_load_lds(
+          (__attribute__((address_space(1))) const unsigned*)(base + off +
+                                                              d * 128),
+          (__attribute__((address_space(3))) unsigned*)l, 16, 0, AUX);
+    else
+      rows.to_lds<AUX>(l, off, d * 128);
+  };
+  Loop loop;
+  auto run = [&](auto once) {
+    loop.run(lds, x_row, part * (BN / PARTS), (int)(row_bytes / 128), MB > 0,
+             [&](char* l, int d, int i) {
+               load(std::false_type(), l + (FIRST * 4 + (wid & 3) * MB + i) * 1024,
+                    x_rows, x0, x_off[i], d);
+             },
+             [&](char* l, int d, int i) {
+               load(once, l + (wid * LW + i) * 1024, w_rows, w0, w_off[i], d);
+             });
+  };
+  if (alone)
+    run(std::true_type());
+  else
+    run(std::false_type());
+  if constexpr (MB > 0 && FP8) {
     #pragma unroll
-    for (int n = 0; n < NI; ++n) {
-      if constexpr (GATED) {
-        #pragma unroll
-        for (int r = 0; r < 16; r += 8) {
-          float y[4];
-          #pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const float g = acc[n][m][r + j], u = acc[n][m][r + 4 + j];
-            y[j] = g / (1.f + __expf(-g)) * u;
-          }
-          *reinterpret_cast<uint2*>(op + (wn * NI + n) * 16 + r) =
-              uint2{cvt_pk_bf16(y[0], y[1]), cvt_pk_bf16(y[2], y[3])};
-        }
-      } else {
-        const int c = (wn * NI + n) * 32;
-        #pragma unroll
-        for (int r = 0; r < 16; r += 4) {
-          float y[4];
-          #pragma unroll
-          for (int j = 0; j < 4; ++j) y[j] = acc[n][m][r + j];
-          if constexpr (FP8) {
-            const float4 ws = *reinterpret_cast<const float4*>(
-                a.w_scale + (long)e * a.N + n0 + c + r * 2 + hf * 4);
-            y[0] = y[0] * xs * ws.x;
-            y[1] = y[1] * xs * ws.y;
-            y[2] = y[2] * xs * ws.z;
-            y[3] = y[3] * xs * ws.w;
-          }
-          *reinterpret_cast<uint2*>(op + c + r * 2) =
-              uint2{cvt_pk_bf16(y[0], y[1]), cvt_pk_bf16(y[2], y[3])};
-        }
-      }
+    for (int m = 0; m < MB; ++m) {
+      const int p = p0 + x_row + m * 32 + (lane & 31);
+      if (a.order[p] < 0) continue;
+      const int c = n0 + part * (OUT / PARTS);
+      store_row_32(loop.acc, m, a.out + (long)p * a.N + c,
+                   a.x_scale[row_of(a, p)], a.w_scale + (long)e * a.N + c);
+    }
+  } else if constexpr (MB > 0) {
+    #pragma unroll
+    for (int m = 0; m < MB; ++m) {
+      const int p = p0 + x_row + m * 16 + (lane & 15);
+      if (a.order[p] < 0) continue;
+      store_row<GATED>(loop.acc, m, a.out + (long)p * a.N + n0 +
+                                        part * (OUT / PARTS));
     }
   }
+}
+
+template <int BN, bool GATED, bool FP8, bool FAR>
+__global__ __launch_bounds__(512, 2) void experts_high_kernel(Tiles a) {
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  int tile = blockIdx.x / a.nx, nb = blockIdx.x % a.nx;
+  const int tiles = gridDim.x / a.nx;
+  const int e = a.expert[tile];
+  const int last = a.expert[max(tile - 1, 0)];
+  const int next = a.expert[min(tile + 1, tiles - 1)];
+  if (e < 0) return;
+  const bool alone = ((tile == 0) | (last != e)) &
+                     ((tile + 1 == tiles) | (next != e));
+  // The tiles of an expert that take the same weights go to one die together,
+  // whose L2 then has them, where an expert has 128 MB of them, half of what the
+  // memory's cache holds: later tiles would find them gone.  180 random sizes (2
+  // to 16 experts, 100 to 1100 choices each, N of 2048 to 16384, K of 1024 to
+  // 15000), time over that without: 256 x 256 from 128 MB on 0.962, two of 29 more
+  // than 1.2 % slower (16 of 16384 x 5760, 1060 choices 6666 -> 6335 us, 8 of 16384
+  // x 2432, 590 841 -> 767, 8 of 8192 x 14080, 320 1.041), with 50 to 128 MB 0.997,
+  // with less 1.024; 256 x 128, which are fewer, 1.032 (2 of 10240 x 3072 77 ->
+  // 96).  More than 32 tiles share them without it.
+  if (BN == 256 && a.nx % 8 == 0 &&
+      (GATED ? 2 : 1) * a.N * ((long)a.K * (FP8 ? 1 : 2)) >= 128l << 20) {
+    const int t = threadIdx.x & 63;
+    const unsigned long back =
+        ~__ballot(t <= tile && a.expert[t <= tile ? tile - t : 0] == e);
+    const unsigned long on = ~__ballot(
+        tile + t < tiles && a.expert[tile + t < tiles ? tile + t : 0] == e);
+    const int before = (back ? __builtin_ctzll(back) : 64) - 1;
+    const int count = before + (on ? __builtin_ctzll(on) : 64);
+    if (count <= 32) {
+      const int at = before * a.nx + nb;
+      nb = at / (8 * count) * 8 + at % 8;
+      tile += at / 8 % count - before;
+    }
+  }
+  const int p0 = tile * 256;
+  const int lane = threadIdx.x & 63;
+  // a tile's choices come first, then its padding
+  const int high = __builtin_popcountll(
+      __ballot(lane < 8 && a.order[p0 + (lane & 7) * 32] >= 0));
+  const bool first = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) < 4;
+  #define HIGH(H)                                                           \
+    case H:                                                                 \
+      if (first)                                                            \
+        high_tile_part<H, false, BN, GATED, FP8, FAR>(a, lds, e, p0, nb,    \
+                                                      alone);               \
+      else                                                                  \
+        high_tile_part<H, true, BN, GATED, FP8, FAR>(a, lds, e, p0, nb,     \
+                                                     alone);                \
+      break;
+  switch (high) {
+    HIGH(1) HIGH(2) HIGH(3) HIGH(4) HIGH(5) HIGH(6) HIGH(7) HIGH(8)
+  }
+  #undef HIGH
 }
 
 }  // namespace
@@ -221,8 +355,8 @@ void experts_tiles_kernel(Tiles a) {
 // w are e4m3.
 void launch_experts_tiles(bool gated, bf16* out, const void* x, const void* w,
                           const float* x_scale, const float* w_scale,
-                          const int* order, const int* expert, long x_rows,
-                          int tiles, int N, int K, int div, int bm,
+                          const int* order, const int* expert, int experts,
+                          long x_rows, int tiles, int N, int K, int div, int bm,
                           hipStream_t stream) {
   if (tiles == 0) return;
   Tiles a{out, x, w, x_scale, w_scale, order, expert, N, K, div, 0};
@@ -245,11 +379,33 @@ void launch_experts_tiles(bool gated, bf16* out, const void* x, const void* w,
       else if (gated) RUN(BM, BN, WM, WN, STAGES, true, false, FAR)         \
       else RUN(BM, BN, WM, WN, STAGES, false, false, FAR)                   \
     }
-  // 256 rows of weights need fewer loads of x and LDS reads, and leave units
-  // idle where they make few workgroups: Mixtral 8x7B, 500 choices an expert,
-  // up (2000 workgroups of 256) 1055 us against 1223, down (290) 753 against
-  // 682; 32 experts of 1024 x 2048, 250 choices, 120 108 and 79 67
+  #define LAUNCH(BN, GATED, FP8, FAR)                                       \
+    {                                                                       \
+      constexpr auto kernel = &experts_high_kernel<BN, GATED, FP8, FAR>;    \
+      static const hipError_t set = hipFuncSetAttribute(                    \
+          reinterpret_cast<const void*>(kernel),                            \
+          hipFuncAttributeMaxDynamicSharedMemorySize, HIGH_BYTES);          \
+      HIP_CHECK(set);                                                       \
+      a.nx = N / (GATED ? BN / 2 : BN);                                     \
+      kernel<<<(unsigned)(tiles * a.nx), 512, HIGH_BYTES, stream>>>(a);     \
+    }
+  #define HIGH(BN, FAR)                                                     \
+    {                                                                       \
+      if (x_scale) LAUNCH(BN, false, true, FAR)                             \
+      else if (gated) LAUNCH(BN, true, false, FAR)                          \
+      else LAUNCH(BN, false, false, FAR)                                    \
+    }
+  // 256 rows of weights need fewer loads of x and LDS reads, 128 make twice the
+  // workgroups, a wave of which takes three fifths of the time.  us, 128 and 256, 8
+  // experts of 14336 x 4096: down 130 choices each 211 262, 256 255 305 (of 128 tiles
+  // of 256), 302 361 293, 512 477 394; up 130 460 430, 302 784 610, 2000 3570 2910; 32
+  // of 1024 x 2048 up 300 choices 112 92, 1000 286 255, down 190 47 43, 500 97 75.
   const int wide = gated ? 128 : 256;
+  const auto waves = [](long groups) { return (groups + 255) / 256; };
+  // tiles with choices, if they are even
+  const long all = std::max(experts, 1);
+  const long mean = std::max((tiles * 256l - 255 * all) / all, 1l);
+  const long live = std::min<long>(tiles, (mean + 255) / 256 * all);
   // what 32 bits of offset do not reach
   const long row_bytes = (long)K * (x_scale ? 1 : 2);
   const bool far = (div ? x_rows : bm) * row_bytes >= 1l << 32 ||
@@ -261,12 +417,15 @@ void launch_experts_tiles(bool gated, bf16* out, const void* x, const void* w,
     if (far) KINDS(128, 128, 2, 4, 3, true)
     else KINDS(128, 128, 2, 4, 3, false)
   } else if (far) {
-    KINDS(256, 128, 4, 2, 3, true)
-  } else if (N % wide == 0 && (long)tiles * (N / wide) >= 1024) {
-    KINDS(256, 256, 4, 2, 2, false)
+    HIGH(128, true)
+  } else if (N % wide == 0 && waves(live * (N / wide)) * 5 <=
+                                  waves(live * (N / wide) * 2) * 3) {
+    HIGH(256, false)
   } else {
-    KINDS(256, 128, 4, 2, 3, false)
+    HIGH(128, false)
   }
+  #undef HIGH
+  #undef LAUNCH
   #undef KINDS
   #undef RUN
 }

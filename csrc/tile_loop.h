@@ -193,3 +193,217 @@ struct TileLoop {
       for (int m = 0; m < MI; ++m) asm volatile("" : "+v"(acc[n][m]));
   }
 };
+
+// The loop of tiles as wide as registers allow, 8 waves.  A wave has MB blocks of B
+// rows of x and NB of w, and loads LX and LW times 8 rows of a chunk.  bf16 takes 16 x
+// 16 x 32 products, e4m3 32 x 32 x 64: a chunk is two steps of 64 bytes.
+//
+// 256 x 256 tiles have room for two stages, in which a chunk has less time to arrive
+// than memory needs; so x and w have slots apart, w, which comes from farther away,
+// always three, x three (XS) where they fit.  Reads of the next step and loads are
+// issued between the rows of a step's products, and not all at once.
+//
+// What bounds it is power, and then the bytes on their way: 256 x 256 tiles of 2000
+// rows of 28672 x 4096 an expert without loads 2670 us with 32 x 32 products, 2390 with
+// 16 x 16 ones, which read and write half the sums; without products 2590 with two
+// stages, 1970 with slots apart.
+template <int BM, int BN, int MB, int NB, int LX, int LW, bool FP8>
+struct RingLoop {
+  static constexpr int XB = BM * 128, WB = BN * 128;
+  static constexpr int XS = 3 * (XB + WB) <= 160 << 10 ? 3 : 2;
+  static constexpr int W_AT = XS * XB, BYTES = W_AT + 3 * WB;
+  static constexpr int B = FP8 ? 32 : 16, UNITS = FP8 ? 2 : 1;
+  static constexpr int READS = MB + NB;
+  // loads that may be on their way while a chunk is read
+  static constexpr int AHEAD = XS == 2 ? LW : LX + LW;
+  static_assert(BYTES <= 160 << 10, "LDS");
+
+  using Acc = __attribute__((ext_vector_type(B * B / 64))) float;
+  struct Frag {
+    short8_t x[MB][UNITS], w[NB][UNITS];
+  };
+  Acc acc[NB][MB];
+  int x_at, w_at;
+
+  // read i of a step
+  DEV void read(Frag& f, const char* x, const char* w, int step, int i) {
+    #pragma unroll
+    for (int u = 0; u < UNITS; ++u) {
+      const int k = FP8 ? (step * 2 + u) << 5 : step << 6;
+      if (i < MB)
+        f.x[i][u] = *reinterpret_cast<const short8_t*>(x + (x_at ^ k) +
+                                                       i * B * 128);
+      else
+        f.w[i - MB][u] = *reinterpret_cast<const short8_t*>(
+            w + (w_at ^ k) + (i - MB) * B * 128);
+    }
+  }
+  DEV void product(const Frag& f, int n, int m) {
+    if constexpr (FP8) {
+      union { short8_t s[2]; int32x8_t v; } u{{f.w[n][0], f.w[n][1]}},
+          v{{f.x[m][0], f.x[m][1]}};
+      acc[n][m] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(
+          u.v, v.v, acc[n][m], 0, 0, 0, 0, 0, 0);    // e4m3, no scales
+    } else {
+      acc[n][m] = mfma16(f.w[n][0], f.x[m][0], acc[n][m]);
+    }
+  }
+
+  // The products of rows x_row and w_row of the tile on.  x_load(l, d, i) and
+  // w_load(l, d, i) issue load i of chunk d to the slot l.  Every wave has to call
+  // this; those that are not live only load.
+  template <class X, class W>
+  DEV void run(char* lds, int x_row, int w_row, int chunks, bool live,
+               X x_load, W w_load) {
+    const int lane = threadIdx.x & 63;
+    x_at = chunk_unit(x_row + lane % B, lane / B);
+    w_at = chunk_unit(w_row + lane % B, lane / B);
+    #pragma unroll
+    for (int n = 0; n < NB; ++n)
+      #pragma unroll
+      for (int m = 0; m < MB; ++m) acc[n][m] = Acc(0.f);
+    #pragma unroll
+    for (int i = 0; i < LX; ++i) x_load(lds, 0, i);
+    #pragma unroll
+    for (int i = 0; i < LW; ++i) w_load(lds + W_AT, 0, i);
+    if (chunks > 1) {
+      if constexpr (XS > 2)
+        #pragma unroll
+        for (int i = 0; i < LX; ++i) x_load(lds + XB, 1, i);
+      #pragma unroll
+      for (int i = 0; i < LW; ++i) w_load(lds + W_AT + WB, 1, i);
+      asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(AHEAD) : "memory");
+    } else {
+      asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+    }
+    // slots of this chunk, and of the one before, which are free
+    int xs = 0, ws = 0, x_free = XS - 1, w_free = 2;
+    // the loads that go with row r of the 2 * NB of chunk d: x, whose time is shorter,
+    // first
+    auto loads = [&](int d, int r) {
+      #pragma unroll
+      for (int i = 0; i < LX; ++i)
+        if (i * (NB / 2) / LX == r && d + XS - 1 < chunks)
+          x_load(lds + x_free * XB, d + XS - 1, i);
+      #pragma unroll
+      for (int i = 0; i < LW; ++i)
+        if (NB / 2 + i * (2 * NB - NB / 2) / LW == r && d + 2 < chunks)
+          w_load(lds + W_AT + w_free * WB, d + 2, i);
+    };
+    Frag f[2];
+    // the products of f, the reads of the step after it, g, and loads
+    auto step = [&](const Frag& f, Frag& g, const char* x, const char* w, int k,
+                    bool more, int d, int r) {
+      #pragma unroll
+      for (int n = 0; n < NB; ++n) {
+        if (live && more) {
+          #pragma unroll
+          for (int i = 0; i < READS; ++i)
+            if (i * (NB > 1 ? NB - 1 : 1) / READS == n) read(g, x, w, k, i);
+        }
+        loads(d, r + n);
+        if (live) {
+          #pragma unroll
+          for (int m = 0; m < MB; ++m) product(f, n, m);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+    };
+    if (live) {
+      #pragma unroll
+      for (int i = 0; i < READS; ++i) read(f[0], lds, lds + W_AT, 0, i);
+    }
+    #pragma unroll
+    for (int n = 0; n < NB; ++n) loads(0, n);
+    for (int d = 0; d < chunks; ++d) {
+      step(f[0], f[1], lds + xs * XB, lds + W_AT + ws * WB, 1, true, d, NB);
+      x_free = xs;
+      w_free = ws;
+      xs = xs == XS - 1 ? 0 : xs + 1;
+      ws = ws == 2 ? 0 : ws + 1;
+      // chunk d + 1 has landed and all of d has been read, by every wave: its slots
+      // are free
+      if (d + 2 < chunks)
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier"
+                     ::"n"(AHEAD) : "memory");
+      else
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier"
+                     ::: "memory");
+      step(f[1], f[0], lds + xs * XB, lds + W_AT + ws * WB, 0, d + 1 < chunks,
+           d + 1, 0);
+    }
+    // as above
+    in_order();
+    asm volatile("s_nop 15\n\ts_nop 7" ::: "memory");
+    in_order();
+  }
+  DEV void in_order() {
+    #pragma unroll
+    for (int n = 0; n < NB; ++n)
+      #pragma unroll
+      for (int m = 0; m < MB; ++m) asm volatile("" : "+v"(acc[n][m]));
+  }
+};
+
+// The sums of 16 x 16 products: a lane has 4 consecutive rows of w of every block of
+// 16, (lane >> 4) * 4 on, and row lane & 15 of x.  Rows of w lie in LDS such that those
+// of two blocks are 8 outputs beside each other, so that a store has 16 bytes a lane
+// and 64 of a row: 256 x 256 tiles of 8192 rows of 28672 x 4096 with 8 bytes a lane, 32
+// of a row, 10 us a tile for the stores alone, so 3.
+//
+// Row of w of row r in LDS: of 32 outputs, and of 32 gates and their 32 up rows, `up`
+// rows on.
+DEV int plain_row(int r) {
+  return (r & ~31) | (r >> 2 & 3) << 3 | (r >> 4 & 1) << 2 | (r & 3);
+}
+DEV int gated_row(int r, int up) {
+  return (r >> 6) * 32 + ((r >> 2 & 3) << 3 | (r >> 5 & 1) << 2 | (r & 3)) +
+         (r & 16 ? up : 0);
+}
+// this lane's outputs of its row of block m of x, whose first output is at `out`
+template <bool GATED, int NB, int MB>
+DEV void store_row(const f32x4_t (&acc)[NB][MB], int m, bf16* out) {
+  typedef __attribute__((ext_vector_type(4))) unsigned u4;
+  out += (threadIdx.x & 63) >> 4 << 3;
+  constexpr int EACH = GATED ? 2 : 1;          // blocks of 4 outputs a lane
+  #pragma unroll
+  for (int n = 0; n < NB; n += 2 * EACH) {
+    u4 v;
+    #pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      f32x4_t y = acc[n + h * EACH][m];
+      if constexpr (GATED) {
+        #pragma unroll
+        for (int j = 0; j < 4; ++j)
+          y[j] = y[j] / (1.f + __expf(-y[j])) * acc[n + 2 * h + 1][m][j];
+      }
+      v[2 * h] = cvt_pk_bf16(y[0], y[1]);
+      v[2 * h + 1] = cvt_pk_bf16(y[2], y[3]);
+    }
+    *reinterpret_cast<u4*>(out + n * (16 / EACH)) = v;
+  }
+}
+
+// The same for 32 x 32 products with scales: a lane has 4 of every 8 rows of w, and two
+// such are 8 outputs beside each other.
+DEV int plain_row_32(int r) {
+  return (r & ~15) | (r >> 2 & 1) << 3 | (r >> 3 & 1) << 2 | (r & 3);
+}
+template <int NB, int MB>
+DEV void store_row_32(const f32x16_t (&acc)[NB][MB], int m, bf16* out,
+                      float x_scale, const float* w_scale) {
+  const int at = (threadIdx.x & 63) >> 5 << 3;
+  #pragma unroll
+  for (int n = 0; n < NB; ++n)
+    #pragma unroll
+    for (int r = 0; r < 16; r += 8) {
+      const int c = n * 32 + r * 2 + at;
+      float y[8];
+      load_vec<float, 8>(w_scale + c, y);
+      #pragma unroll
+      for (int j = 0; j < 8; ++j) y[j] = acc[n][m][r + j] * x_scale * y[j];
+      *reinterpret_cast<uint4*>(out + c) =
+          uint4{cvt_pk_bf16(y[0], y[1]), cvt_pk_bf16(y[2], y[3]),
+                cvt_pk_bf16(y[4], y[5]), cvt_pk_bf16(y[6], y[7])};
+    }
+}

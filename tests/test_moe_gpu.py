@@ -361,3 +361,57 @@ def test_tiles_of_an_expert_together(width, inner):
         # both round the inner values and the results to bf16
         assert (out[mine].float() - want).norm(dim=-1).le(
             2.0 ** -7 * want.norm(dim=-1)).all()
+
+
+@pytest.mark.parametrize("kind", ["gated", "plain", "fp8"])
+@pytest.mark.parametrize("outputs", [384, 2560])    # tiles of 128 and of 256
+@pytest.mark.parametrize("chunks", [2, 3, 5])
+def test_tiles_as_high_as_their_choices(kind, outputs, chunks):
+    """Tiles of 1 to 8 blocks of 32 choices, at the edges of the blocks; experts of
+    several tiles have even ones.  A sum is rounded to bf16: half a step is at most
+    2^-8 of it."""
+    counts = [1, 32, 33, 64, 65, 96, 97, 128, 129, 160, 161, 192, 193, 224, 225,
+              256, 257, 0, 300, 513]
+    E, T, fp8 = len(counts), sum(counts), kind == "fp8"
+    K = chunks * (128 if fp8 else 64)
+    g = torch.Generator().manual_seed(chunks)
+    rand = lambda *s: torch.randn(*s, generator=g).to(DEV)
+    ids = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))
+    ids = ids[torch.randperm(T, generator=g)].int().to(DEV)
+    order, expert, place = ops._moe_sort(ids[:, None], E, 128, 128, 256)
+    live = (order.view(-1, 256) >= 0).sum(1)
+    for e, n in enumerate(counts):
+        tiles = live[expert == e]
+        assert int(tiles.sum()) == n and len(tiles) == -(-n // 256)
+        assert n == 0 or int(tiles.max() - tiles.min()) < 32 * len(tiles)
+    gated = kind == "gated"
+    x, w = rand(T, K), rand(E, outputs, K) * K ** -0.5
+    N = outputs // 2 if gated else outputs
+    out = torch.empty(len(order), N, dtype=torch.bfloat16, device=DEV)
+    sx = sw = None
+    if fp8:
+        x, w = x.to(torch.float8_e4m3fn), w.to(torch.float8_e4m3fn)
+        sx, sw = rand(T).abs(), rand(E, outputs).abs()
+    else:
+        x, w = x.bfloat16(), w.bfloat16()
+    ops._native().experts_tiles(out, x, w, sx, sw, order, expert, gated, 1, 256)
+    got = out[place[:, 0].long()].double()
+    for e in range(E):
+        mine = ids == e
+        want = x[mine].double() @ w[e].double().t()
+        # of a sum of magnitudes: float sums, and the 8-bit products of the card,
+        # which keep fewer bits of a part of K
+        slack = (x[mine].double().abs() @ w[e].double().abs().t()) \
+            * 2.0 ** (-16 if fp8 else -22)
+        if gated:
+            gate, up = want.chunk(2, -1)
+            want = torch.nn.functional.silu(gate) * up
+            # |silu'| <= 1.1, |silu(g)| <= |g|; the exponential's error is 2^-20
+            dg, du = slack.chunk(2, -1)
+            slack = 1.1 * dg * up.abs() + gate.abs() * du \
+                + 2.0 ** -20 * want.abs()
+        if fp8:
+            scale = sx[mine, None].double() * sw[e].double()
+            want, slack = want * scale, slack * scale
+        assert ((got[mine] - want).abs()
+                <= 2.0 ** -8 * want.abs() + 1.01 * slack).all()
