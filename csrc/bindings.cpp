@@ -108,6 +108,8 @@ bool gemm_rows_fits(long, long);
 void launch_gemm_split(bf16*, float*, const void*, const void*, const float*,
                        const float*, int, int, int, long, long, int, int, int,
                        bool, hipStream_t);
+void launch_gemm_wide(bf16*, float*, const bf16*, const bf16*, int, int, int,
+                      long, long, int, int, int, bool, hipStream_t);
 void launch_gemm_rows(bf16*, const bf16*, const bf16*, const float*,
                       const float*, int, int, int, long, long, long,
                       hipStream_t);
@@ -555,6 +557,50 @@ void gemm_split(c10::optional<torch::Tensor> out, torch::Tensor x,
                     fp8 ? w_scale->data_ptr<float>() : nullptr, (int)M, (int)N,
                     (int)K, x.stride(0), w.stride(0), (int)bm, (int)bn,
                     (int)splits, gated, stream());
+}
+
+// products of many rows in tiles of 32 * high by bn: out, or the parts
+void gemm_wide(c10::optional<torch::Tensor> out, torch::Tensor x,
+               torch::Tensor w, c10::optional<torch::Tensor> part, long high,
+               long bn, long splits, bool gated) {
+  for (const auto& t : {x, w})
+    TORCH_CHECK(t.is_cuda() && t.scalar_type() == torch::kBFloat16 &&
+                    t.dim() == 2 && t.stride(1) == 1, "gemm_wide: matrices");
+  const long M = x.size(0), K = x.size(1), N = w.size(0);
+  const long outs = gated ? N / 2 : N;
+  TORCH_CHECK(w.size(1) == K && out.has_value() != (splits > 1) &&
+                  !(gated && splits > 1), "gemm_wide: shape");
+  if (out.has_value())
+    TORCH_CHECK(out->is_cuda() && out->scalar_type() == torch::kBFloat16 &&
+                    out->dim() == 2 && out->size(0) == M &&
+                    out->size(1) == outs && out->is_contiguous() &&
+                    reinterpret_cast<uintptr_t>(out->data_ptr()) % 16 == 0,
+                "gemm_wide: out");
+  TORCH_CHECK(high >= 4 && high <= 8 && (bn == 128 || bn == 256) &&
+                  splits >= 1 && splits <= 8 && K >= 64 * splits &&
+                  K % 64 == 0 && N % (gated ? 16 : 8) == 0,
+              "gemm_wide: sizes");
+  // 16 bytes at a time, the rows of a tile by 32 bits of offset
+  auto fits = [&](const torch::Tensor& t, long rows) {
+    return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0 &&
+           t.stride(0) % 8 == 0 && t.stride(0) >= 0 &&
+           (rows - 1) * t.stride(0) + K < 0x7ffffff8l;
+  };
+  const long tiles = (M / (32 * high) + 1) * (outs / 64 + 1) * splits;
+  TORCH_CHECK(fits(x, std::min(M, 32 * high)) &&
+                  fits(w, gated ? std::min(N, outs + 128) : std::min(N, bn)) &&
+                  tiles < (1l << 30), "gemm_wide: offsets");
+  float* ws = nullptr;
+  if (splits > 1) {
+    TORCH_CHECK(part.has_value(), "gemm_wide: parts need a workspace");
+    check(*part, torch::kFloat, "part");
+    TORCH_CHECK(part->numel() >= splits * M * N, "gemm_wide: workspace");
+    ws = part->data_ptr<float>();
+  }
+  if (M == 0 || N == 0) return;
+  launch_gemm_wide(out.has_value() ? bf(*out) : nullptr, ws, cbf(x), cbf(w),
+                   (int)M, (int)N, (int)K, x.stride(0), w.stride(0), (int)high,
+                   (int)bn, (int)splits, gated, stream());
 }
 
 void silu_mul(torch::Tensor out, torch::Tensor x) {
@@ -1275,6 +1321,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("fused_add_rmsnorm_fp8", &fused_add_rmsnorm_fp8);
   m.def("parts_add_rmsnorm_fp8", &parts_add_rmsnorm_fp8);
   m.def("silu_mul_fp8", &silu_mul_fp8);
+  m.def("gemm_wide", &gemm_wide, py::arg("out"), py::arg("x"), py::arg("w"),
+        py::arg("part"), py::arg("high"), py::arg("bn"), py::arg("splits") = 1,
+        py::arg("gated") = false);
   m.def("moe_gemm", &moe_gemm);
   m.def("fused_add_rmsnorm", &fused_add_rmsnorm);
   m.def("rope_kv_append", &rope_kv_append);

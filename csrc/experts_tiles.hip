@@ -287,7 +287,7 @@ DEV void high_tile_part(const Tiles& a, char* lds, int e, int p0, int nb,
       const int p = p0 + x_row + m * 16 + (lane & 15);
       if (a.order[p] < 0) continue;
       store_row<GATED>(loop.acc, m, a.out + (long)p * a.N + n0 +
-                                        part * (OUT / PARTS));
+                                        part * (OUT / PARTS), OUT / PARTS);
     }
   }
 }

@@ -201,7 +201,7 @@ struct TileLoop {
 // 256 x 256 tiles have room for two stages, in which a chunk has less time to arrive
 // than memory needs; so x and w have slots apart, w, which comes from farther away,
 // always three, x three (XS) where they fit.  Reads of the next step and loads are
-// issued between the rows of a step's products, and not all at once.
+// issued one by one between a step's products, and not all at once.
 //
 // What bounds it is power, and then the bytes on their way: 256 x 256 tiles of 2000
 // rows of 28672 x 4096 an expert without loads 2670 us with 32 x 32 products, 2390 with
@@ -278,35 +278,36 @@ struct RingLoop {
     }
     // slots of this chunk, and of the one before, which are free
     int xs = 0, ws = 0, x_free = XS - 1, w_free = 2;
-    // the loads that go with row r of the 2 * NB of chunk d: x, whose time is shorter,
-    // first
-    auto loads = [&](int d, int r) {
-      #pragma unroll
-      for (int i = 0; i < LX; ++i)
-        if (i * (NB / 2) / LX == r && d + XS - 1 < chunks)
-          x_load(lds + x_free * XB, d + XS - 1, i);
-      #pragma unroll
-      for (int i = 0; i < LW; ++i)
-        if (NB / 2 + i * (2 * NB - NB / 2) / LW == r && d + 2 < chunks)
-          w_load(lds + W_AT + w_free * WB, d + 2, i);
+    // The loads of chunk d between the products of a step: those of x after the barrier
+    // that chunk d begins with, for their time is shorter, then those of w.
+    constexpr int Q = NB * MB;
+    auto loads = [&](int d, bool after, int q) {
+      if (after) {
+        #pragma unroll
+        for (int i = 0; i < LX; ++i)
+          if (i * Q / LX == q && d + XS - 1 < chunks)
+            x_load(lds + x_free * XB, d + XS - 1, i);
+      } else {
+        #pragma unroll
+        for (int i = 0; i < LW; ++i)
+          if (i * Q / LW == q && d + 2 < chunks)
+            w_load(lds + W_AT + w_free * WB, d + 2, i);
+      }
     };
     Frag f[2];
-    // the products of f, the reads of the step after it, g, and loads
+    // the products of f, and between them the reads of the step after it, g, and loads
     auto step = [&](const Frag& f, Frag& g, const char* x, const char* w, int k,
-                    bool more, int d, int r) {
+                    bool more, int d, bool after) {
       #pragma unroll
-      for (int n = 0; n < NB; ++n) {
+      for (int q = 0; q < Q; ++q) {
+        if (live) product(f, q / MB, q % MB);
         if (live && more) {
           #pragma unroll
           for (int i = 0; i < READS; ++i)
-            if (i * (NB > 1 ? NB - 1 : 1) / READS == n) read(g, x, w, k, i);
+            if (i * (Q * 3 / 4) / READS == q) read(g, x, w, k, i);
         }
-        loads(d, r + n);
-        if (live) {
-          #pragma unroll
-          for (int m = 0; m < MB; ++m) product(f, n, m);
-          __builtin_amdgcn_sched_barrier(0);
-        }
+        loads(d, after, q);
+        if (live) __builtin_amdgcn_sched_barrier(0);
       }
     };
     if (live) {
@@ -314,9 +315,10 @@ struct RingLoop {
       for (int i = 0; i < READS; ++i) read(f[0], lds, lds + W_AT, 0, i);
     }
     #pragma unroll
-    for (int n = 0; n < NB; ++n) loads(0, n);
+    for (int i = 0; i < LX; ++i)
+      if (XS - 1 < chunks) x_load(lds + x_free * XB, XS - 1, i);
     for (int d = 0; d < chunks; ++d) {
-      step(f[0], f[1], lds + xs * XB, lds + W_AT + ws * WB, 1, true, d, NB);
+      step(f[0], f[1], lds + xs * XB, lds + W_AT + ws * WB, 1, true, d, false);
       x_free = xs;
       w_free = ws;
       xs = xs == XS - 1 ? 0 : xs + 1;
@@ -330,7 +332,7 @@ struct RingLoop {
         asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier"
                      ::: "memory");
       step(f[1], f[0], lds + xs * XB, lds + W_AT + ws * WB, 0, d + 1 < chunks,
-           d + 1, 0);
+           d + 1, true);
     }
     // as above
     in_order();
@@ -360,15 +362,15 @@ DEV int gated_row(int r, int up) {
   return (r >> 6) * 32 + ((r >> 2 & 3) << 3 | (r >> 5 & 1) << 2 | (r & 3)) +
          (r & 16 ? up : 0);
 }
-// this lane's outputs of its row of block m of x, whose first output is at `out`
+// this lane's outputs of its row of block m of x, whose first output is at `out`, of
+// `left` that there are
 template <bool GATED, int NB, int MB>
-DEV void store_row(const f32x4_t (&acc)[NB][MB], int m, bf16* out) {
-  typedef __attribute__((ext_vector_type(4))) unsigned u4;
-  out += (threadIdx.x & 63) >> 4 << 3;
+DEV void store_row(const f32x4_t (&acc)[NB][MB], int m, bf16* out, int left) {
+  const int at = (threadIdx.x & 63) >> 4 << 3;
   constexpr int EACH = GATED ? 2 : 1;          // blocks of 4 outputs a lane
   #pragma unroll
   for (int n = 0; n < NB; n += 2 * EACH) {
-    u4 v;
+    unsigned v[4];
     #pragma unroll
     for (int h = 0; h < 2; ++h) {
       f32x4_t y = acc[n + h * EACH][m];
@@ -380,8 +382,21 @@ DEV void store_row(const f32x4_t (&acc)[NB][MB], int m, bf16* out) {
       v[2 * h] = cvt_pk_bf16(y[0], y[1]);
       v[2 * h + 1] = cvt_pk_bf16(y[2], y[3]);
     }
-    *reinterpret_cast<u4*>(out + n * (16 / EACH)) = v;
+    if (n * (16 / EACH) + at < left)
+      *reinterpret_cast<uint4*>(out + n * (16 / EACH) + at) =
+          uint4{v[0], v[1], v[2], v[3]};
   }
+}
+// the same of a part, floats
+template <int NB, int MB>
+DEV void store_part(const f32x4_t (&acc)[NB][MB], int m, float* out, int left) {
+  const int at = (threadIdx.x & 63) >> 4 << 3;
+  #pragma unroll
+  for (int n = 0; n < NB; n += 2)
+    if (n * 16 + at < left) {
+      *reinterpret_cast<f32x4_t*>(out + n * 16 + at) = acc[n][m];
+      *reinterpret_cast<f32x4_t*>(out + n * 16 + at + 4) = acc[n + 1][m];
+    }
 }
 
 // The same for 32 x 32 products with scales: a lane has 4 of every 8 rows of w, and two

@@ -536,6 +536,90 @@ def _summed_gemm(M: int, N: int, K: int):
     return None
 
 
+# Tiles of csrc/gemm_wide.hip, 32 * high rows by bn outputs: us of a wave of 256 and of
+# 64 columns of it, least squares over 2900 random sizes (6 % off on average).
+_WIDE_TIMES = {(4, 128): (0.0, 0.60), (5, 128): (0.5, 0.65),
+               (6, 128): (1.8, 0.68), (7, 128): (2.6, 0.75),
+               (8, 128): (3.1, 0.84), (4, 256): (3.6, 0.80),
+               (5, 256): (1.8, 0.96), (6, 256): (2.6, 1.08),
+               (7, 256): (4.5, 1.21), (8, 256): (5.3, 1.40)}
+
+
+def _wide_tile(M: int, N: int, K: int, parts=(1,)):
+    """(us, high, bn, parts of K, tiles) of the tiles that take the least time: even
+    tiles of up to 256 rows, or one more of them.  Parts are floats that the norm
+    reads."""
+    best = None
+    for mt in (-(-M // 256), -(-M // 256) + 1):
+        high = -(-M // (mt * 32))
+        for bn in (128, 256):
+            if (high, bn) not in _WIDE_TIMES:
+                continue
+            fixed, chunk = _WIDE_TIMES[high, bn]
+            for split in parts:
+                tiles = -(-M // (high * 32)) * -(-N // bn) * split
+                if split > 1 and (tiles > 256 or K < 256 * split):
+                    continue
+                us = -(-tiles // 256) * (fixed + chunk * K / 64 / split) \
+                    + M * N * (4 if split == 1 else 8 * split) / 5e6
+                if best is None or us < best[0]:
+                    best = us, high, bn, split, tiles
+    return best
+
+
+@lru_cache(maxsize=1 << 14)
+def _wide_gated(M: int, N: int, K: int):
+    """(high, bn) where csrc/gemm_wide.hip forms silu(gate) * up of more than 256
+    rows faster than what was there, mostly the library's product and a pass.  2000
+    random sizes from 257 to 8192 rows, N of 6000 to 36000 and K of 1024 to 8192, time
+    over that: up to 1200 rows at 0.7 PFLOP/s and more by the tiles' times 0.88, 2 of
+    100 more than 3 % slower (512 of 28672 x 4096 112 104 us, 880 203 176; 512 of 14336
+    x 2048 32 30); more of up to 3072 columns 0.85, 6 of 100 (2600 of 14336 x 2048 183
+    146).  More of longer columns 0.95, but every fourth slower, by up to 10 % (8192
+    of 28672 x 4096 1335 1400): those are the library's."""
+    if not 256 < M < 1 << 20 or not 1024 <= K <= 8192 or K % 64 or N % 16 \
+            or not 6000 <= N < 1 << 17 or M > 1200 and K > 3072:
+        return None
+    us, high, bn, _, _ = _wide_tile(M, N, K)
+    return (high, bn) if 2e-9 * M * N * K / us >= 0.7 else None
+
+
+@lru_cache(maxsize=1 << 14)
+def _wide_parts(M: int, N: int, K: int):
+    """(high, bn, parts) where csrc/gemm_wide.hip and the norm that adds up its parts
+    are faster than what was there and the norm.  760 random sizes from 257 to 3000
+    rows, time over that: 10240 columns and more, up to 1400 rows 0.79 (262 rows of
+    4096 x 14336 58 48 us, 600 112 76, 1000 137 110, 1268 161 132; worst 998 of 2720 x
+    16384 at 0.83, but 1.09 for tiles that fill no wave); from 4608 on 513 to 1024 rows
+    0.90 (worst 973 of 3216 x 4864 42 45); up to 2560, 513 to 1024 rows and up to 4096
+    outputs 0.87 (600 of 2048 x 2048 25 23).  Between, 0.98 to 1.07; more rows 1.0."""
+    if K % 64 or N % 8 or not 1024 <= N <= 8192 or not 1024 <= K <= 20480 \
+            or not 256 < M <= (1400 if K >= 10240 else 1024) \
+            or M <= 512 and (K < 10240 or N < 1536) \
+            or 2560 < K < 4608 or K <= 2560 and N > 4096:
+        return None
+    _, high, bn, split, tiles = _wide_tile(M, N, K, (1, 2, 3, 4, 6, 8))
+    return (high, bn, split) if 176 <= tiles <= 256 or K <= 2560 else None
+
+
+@lru_cache(maxsize=1 << 14)
+def _wide_long(M: int, N: int, K: int):
+    """(high, bn, 1) for long columns where 256 x 256 tiles are several waves of which
+    the last is neither nearly empty nor full.  The library has tiles of 0.7 to 1.0
+    PFLOP/s for half of these sizes and of 1.3 to 1.5 for the others, 1.03 on average
+    over 70 of N from 3584 to 8192 and K from 11008 to 28672; here 1.2 to 1.4 (7411
+    rows of 4096 x 14336 971 640 us, 5888 of 5120 x 13824 958 600; worst 7680 of 4096 x
+    11008 441 508).  With up to 10240 columns it has 1.3 to 1.55."""
+    if not 1024 < M < 1 << 20 or not 10240 <= K <= 1 << 15 or K % 64 or N % 8 \
+            or not 2048 <= N <= 8192:
+        return None
+    tiles = -(-M // 256) * -(-N // 256)
+    if tiles <= 256 or not 0.8 <= _full(tiles) < 0.96:
+        return None
+    _, high, bn, _, _ = _wide_tile(M, N, K)
+    return high, bn, 1
+
+
 def _near(x: torch.Tensor, w: torch.Tensor, bm: int, bn: int) -> bool:
     """32 bits of offset reach the rows of a tile of bm by bn from its first."""
     return all(((min(t.shape[0], rows) - 1) * t.stride(0) + t.shape[1])
@@ -545,11 +629,20 @@ def _near(x: torch.Tensor, w: torch.Tensor, bm: int, bn: int) -> bool:
 def _product(x: torch.Tensor, w: torch.Tensor, parts: bool, plain: bool):
     """x w^T for w [N, K]; with `parts` as Parts where it is formed so.  plain:
     what _plain_bf16 says, which looks at the sizes of no traced tensor."""
-    route = _route(x.shape[0], *w.shape, parts) \
-        if plain and x.shape[0] <= MOST_ROWS else None
+    M, N = x.shape[0], w.shape[0]
+    wide = plain and M > 256 and (parts and _wide_parts(M, *w.shape)
+                                  or _wide_long(M, *w.shape))
+    if wide and _near(x, w, wide[0] * 32, wide[1]):
+        high, bn, split = wide
+        part = torch.empty(split, M, N, dtype=torch.float32,
+                           device=x.device) if split > 1 else None
+        out = None if part is not None else \
+            torch.empty(M, N, dtype=x.dtype, device=x.device)
+        _native().gemm_wide(out, x, w, part, high, bn, split)
+        return out if part is None else Parts(part)
+    route = _route(M, *w.shape, parts) if plain and M <= MOST_ROWS else None
     if route is None or route != "rows" and not _near(x, w, *route[:2]):
         return x @ w.t()
-    M, N = x.shape[0], w.shape[0]
     if route == "rows":
         out = torch.empty(M, N, dtype=x.dtype, device=x.device)
         _native().gemm_rows(out, x, w)
@@ -626,8 +719,14 @@ def _gated_wave(M: int, N: int, K: int):
 def gated_linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """silu_mul of x w^T, w the gate's rows and then the up rows."""
     plain = _plain_bf16(x, w)
+    sizes = (x.shape[0], *w.shape) if plain else None
+    wide = plain and _wide_gated(*sizes)
+    if wide and _near(x, w, wide[0] * 32, w.shape[0] // 2 + 128):
+        out = torch.empty(x.shape[0], w.shape[0] // 2, dtype=x.dtype,
+                          device=x.device)
+        _native().gemm_wide(out, x, w, None, *wide, gated=True)
+        return out
     if plain and x.shape[0] <= MOST_ROWS:
-        sizes = (x.shape[0], *w.shape)
         tile = _gated_tile(*sizes) or _gated_wave(*sizes)
         if tile is not None and _near(x, w, *tile) \
                 and w.stride(0) * (w.shape[0] + 256) < 1 << 32:

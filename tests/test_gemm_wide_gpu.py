@@ -1,0 +1,158 @@
+"""Products of many rows in tiles of 128 to 256 rows, against float64, at the edges
+of tiles, and the rules that choose them.
+
+Bounds: products are exact in float and summed in float, 2^-22 of the sum of
+magnitudes; results are rounded to bf16, half a step is at most 2^-8 of them."""
+
+import random
+
+import pytest
+import torch
+
+import hyperspot.engine  # noqa: F401  (before the models, which it imports)
+import hyperspot.ops as ops
+
+DEV = "cuda:0"
+
+
+def _inputs(M, N, K, pad=0):
+    g = torch.Generator().manual_seed(M + N + K)
+    x = torch.randn(M, K + pad, generator=g).bfloat16().to(DEV)[:, :K]
+    w = (torch.randn(N, K + pad, generator=g) * K ** -0.5).bfloat16()
+    return x, w.to(DEV)[:, :K]
+
+
+def _bounds(x, w):
+    x, w = x.double(), w.double()
+    return x @ w.t(), x.abs() @ w.abs().t() * 2.0 ** -22
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("high", [4, 5, 6, 7, 8])
+@pytest.mark.parametrize("bn", [128, 256])
+@pytest.mark.parametrize("M,N,K,pad", [
+    (1, 8, 64, 0), (-1, 264, 128, 8), (0, 256, 192, 0), (1, 520, 320, 64),
+    (700, 1032, 448, 0)])
+def test_tiles(high, bn, M, N, K, pad):
+    """M: rows beside a whole number of tiles, or some tiles of rows and nine of
+    them, more than go together."""
+    M = 9 * 32 * high + 5 if M == 700 else 32 * high + M
+    x, w = _inputs(M, N, K, pad)
+    want, slack = _bounds(x, w)
+    out = torch.full((M, N), 7.0, dtype=torch.bfloat16, device=DEV)
+    ops._native().gemm_wide(out, x, w, None, high, bn)
+    assert ((out.double() - want).abs()
+            <= 2.0 ** -8 * want.abs() + 1.01 * slack).all()
+    for parts in {2, K // 64} - {1}:
+        if parts > K // 64 or parts > 8:
+            continue
+        part = torch.full((parts, M, N), 7.0, device=DEV)
+        ops._native().gemm_wide(None, x, w, part, high, bn, parts)
+        edge = [K // 64 * z // parts * 64 for z in range(parts + 1)]
+        for z in range(parts):
+            p, s = _bounds(x[:, edge[z]:edge[z + 1]], w[:, edge[z]:edge[z + 1]])
+            assert ((part[z].double() - p).abs() <= s).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("high", [4, 5, 8])
+@pytest.mark.parametrize("bn", [128, 256])
+@pytest.mark.parametrize("N,K", [(16, 64), (272, 128), (784, 320)])
+def test_gated_tiles(high, bn, N, K):
+    M = 32 * high * 2 - 7
+    x, w = _inputs(M, N, K)
+    out = torch.full((M, N // 2), 7.0, dtype=torch.bfloat16, device=DEV)
+    ops._native().gemm_wide(out, x, w, None, high, bn, gated=True)
+    (gate, up), (dg, du) = (t.chunk(2, -1) for t in _bounds(x, w))
+    want = torch.nn.functional.silu(gate) * up
+    # |silu'| <= 1.1, |silu(g)| <= |g|; the exponential's error is 2^-20
+    slack = 1.1 * dg * up.abs() + gate.abs() * du + 2.0 ** -20 * want.abs()
+    assert ((out.double() - want).abs()
+            <= 2.0 ** -8 * want.abs() + 1.01 * slack).all()
+
+
+@pytest.mark.gpu
+def test_numbers_that_are_not_finite():
+    """They stay in their rows, and rows past the end do not matter."""
+    x, w = _inputs(300, 264, 192)
+    x[7, 3], x[299, 191], w[5, 0] = float("nan"), float("inf"), float("inf")
+    out = torch.empty(300, 264, dtype=torch.bfloat16, device=DEV)
+    ops._native().gemm_wide(out, x, w, None, 5, 128)
+    want = x.float() @ w.float().t()
+    assert torch.equal(out.isfinite(), want.isfinite())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [
+    (257, 4096, 14336), (600, 4096, 10240), (513, 2048, 7168),
+    (1024, 2048, 2048), (1400, 4096, 10240)])
+def test_parts_and_norm(M, N, K):
+    assert ops._wide_parts(M, N, K) and not ops._wide_parts(256, N, K)
+    x, w = _inputs(M, N, K)
+    y = ops.linear_parts(x, w)
+    y = y.data.sum(0) if isinstance(y, ops.Parts) else y
+    want, slack = _bounds(x, w)
+    assert ((y.double() - want).abs()
+            <= 2.0 ** -8 * want.abs() + 2 * slack).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(700, 16384, 1024), (1201, 6016, 3072),
+                                   (1200, 14336, 3136)])
+def test_gated_linear(M, N, K, monkeypatch):
+    assert ops._wide_gated(M, N, K)
+    x, w = _inputs(M, N, K)
+    got = ops.gated_linear(x, w)
+    monkeypatch.setattr(ops, "_wide_gated", lambda *a: None)
+    want = ops.gated_linear(x, w).float()
+    # one side rounds the halves to bf16 first
+    assert (got.float() - want).norm() <= 2.0 ** -7 * want.norm()
+
+
+@pytest.mark.gpu
+def test_long_columns():
+    M, N, K = 3600, 5120, 10240              # 300 tiles are 0.59 of two waves
+    assert ops._wide_long(M, N, K) is None
+    M = 5400                                 # 440 are 0.86
+    high, bn, parts = ops._wide_long(M, N, K)
+    assert parts == 1 and (high, bn) == (8, 256)
+    x, w = _inputs(M, N, K)
+    got, want = ops.linear(x, w).float(), x.float() @ w.float().t()
+    assert (got - want).norm() <= 2.0 ** -8 * want.norm()
+
+
+@pytest.mark.gpu
+def test_refused():
+    x, w = _inputs(300, 256, 128)
+    out = torch.empty(300, 256, dtype=torch.bfloat16, device=DEV)
+    part = torch.empty(2, 300, 256, device=DEV)
+    wide = ops._native().gemm_wide
+    for args in ((out, x, w, None, 3, 128), (out, x, w, None, 8, 64),
+                 (None, x, w, None, 8, 128), (None, x, w, part, 8, 128, 3),
+                 (None, x, w, part[:1], 8, 128, 2),
+                 (out, x[:, :96], w[:, :96], None, 8, 128),
+                 (out, x, w[:250], None, 8, 128),
+                 (out[:, :128], x, w, None, 8, 128)):
+        with pytest.raises(RuntimeError):
+            wide(*args)
+
+
+def test_rules_cover_all_rows():
+    """Every size that a rule takes has tiles that the kernel has, enough of them
+    for all rows and outputs, and parts with columns."""
+    rng = random.Random(1)
+    taken = 0
+    for _ in range(20000):
+        M, N = rng.randint(1, 9000), rng.randint(1, 5000) * 8
+        K = rng.randint(1, 400) * rng.choice([32, 64])
+        for rule in (ops._wide_gated, ops._wide_parts, ops._wide_long):
+            tile = rule(M, N, K)
+            if tile is None:
+                continue
+            taken += 1
+            high, bn, parts = (*tile, 1)[:3]
+            assert M > 256 and K % 64 == 0 and N % (
+                16 if rule is ops._wide_gated else 8) == 0
+            assert 4 <= high <= 8 and bn in (128, 256)
+            assert 1 <= parts <= 8 and parts * 64 <= K
+    assert taken > 200

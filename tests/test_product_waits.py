@@ -95,3 +95,13 @@ def test_sums_of_products_are_waited_for():
         for kernel, text in zip(kernels, pool.map(asm, kernels)):
             products, early = _early(text)
             assert products and not early, (kernel, early[:3])
+
+
+@pytest.mark.skipif(not shutil.which(native.HIPCC), reason="no compiler")
+def test_sums_of_wide_tiles_are_waited_for():
+    asm = subprocess.run(
+        [native.HIPCC, "-S", "--cuda-device-only", "-o", "-",
+         str(native.CSRC / "gemm_wide.hip")] + native.COMMON + native.DEVICE,
+        capture_output=True, text=True, check=True).stdout
+    products, early = _early(asm)
+    assert products and not early, early[:3]
