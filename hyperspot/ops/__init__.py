@@ -547,10 +547,10 @@ _WIDE_TIMES = {(4, 128): (0.0, 0.60), (5, 128): (0.5, 0.65),
 
 def _wide_tile(M: int, N: int, K: int, parts=(1,)):
     """(us, high, bn, parts of K, tiles) of the tiles that take the least time: even
-    tiles of up to 256 rows, or one more of them.  Parts are floats that the norm
-    reads."""
-    best = None
-    for mt in (-(-M // 256), -(-M // 256) + 1):
+    tiles of up to 256 rows, or one more of them if they are several.  Parts are floats
+    that the norm reads."""
+    best, least = None, -(-M // 256)
+    for mt in (least, least + (least > 1)):
         high = -(-M // (mt * 32))
         for bn in (128, 256):
             if (high, bn) not in _WIDE_TIMES:
@@ -592,14 +592,22 @@ def _wide_parts(M: int, N: int, K: int):
     4096 x 14336 58 48 us, 600 112 76, 1000 137 110, 1268 161 132; worst 998 of 2720 x
     16384 at 0.83, but 1.09 for tiles that fill no wave); from 4608 on 513 to 1024 rows
     0.90 (worst 973 of 3216 x 4864 42 45); up to 2560, 513 to 1024 rows and up to 4096
-    outputs 0.87 (600 of 2048 x 2048 25 23).  Between, 0.98 to 1.07; more rows 1.0."""
+    outputs 0.87 (600 of 2048 x 2048 25 23).  Between, 0.98 to 1.07; more rows 1.0.
+    129 to 256 rows in 380 other sizes of 10240 columns and more, one tile of rows and
+    more than 192 in all, 0.89 (135 rows of 4096 x 14336 44 36 us, 248 53 45); decode
+    steps of 140, 200 and 256 rows, 8 layers, 1 % less.  Fewer rows are as fast in the
+    step (100 1730 1738), fewer tiles slower (200 of 2048 x 7168 17 21)."""
     if K % 64 or N % 8 or not 1024 <= N <= 8192 or not 1024 <= K <= 20480 \
-            or not 256 < M <= (1400 if K >= 10240 else 1024) \
-            or M <= 512 and (K < 10240 or N < 1536) \
-            or 2560 < K < 4608 or K <= 2560 and N > 4096:
+            or not 128 < M <= (1400 if K >= 10240 else 1024):
         return None
-    _, high, bn, split, tiles = _wide_tile(M, N, K, (1, 2, 3, 4, 6, 8))
-    return (high, bn, split) if 176 <= tiles <= 256 or K <= 2560 else None
+    _, high, bn, split, tiles = _wide_tile(M, N, K, (1, 2, 3, 4, 5, 6, 7, 8))
+    if M <= 256:
+        fits = tiles > 192 and K >= 10240
+    elif M <= 512:
+        fits = 176 <= tiles <= 256 and K >= 10240 and N >= 1536
+    else:
+        fits = K <= 2560 and N <= 4096 or K >= 4608 and 176 <= tiles <= 256
+    return (high, bn, split) if fits else None
 
 
 @lru_cache(maxsize=1 << 14)
@@ -630,8 +638,8 @@ def _product(x: torch.Tensor, w: torch.Tensor, parts: bool, plain: bool):
     """x w^T for w [N, K]; with `parts` as Parts where it is formed so.  plain:
     what _plain_bf16 says, which looks at the sizes of no traced tensor."""
     M, N = x.shape[0], w.shape[0]
-    wide = plain and M > 256 and (parts and _wide_parts(M, *w.shape)
-                                  or _wide_long(M, *w.shape))
+    wide = plain and M > 128 and (parts and _wide_parts(M, *w.shape)
+                                 or _wide_long(M, *w.shape))
     if wide and _near(x, w, wide[0] * 32, wide[1]):
         high, bn, split = wide
         part = torch.empty(split, M, N, dtype=torch.float32,

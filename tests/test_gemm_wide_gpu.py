@@ -85,9 +85,10 @@ def test_numbers_that_are_not_finite():
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K", [
     (257, 4096, 14336), (600, 4096, 10240), (513, 2048, 7168),
-    (1024, 2048, 2048), (1400, 4096, 10240)])
+    (1024, 2048, 2048), (1400, 4096, 10240), (129, 4096, 14336),
+    (256, 4096, 10240)])
 def test_parts_and_norm(M, N, K):
-    assert ops._wide_parts(M, N, K) and not ops._wide_parts(256, N, K)
+    assert ops._wide_parts(M, N, K) and not ops._wide_parts(128, N, K)
     x, w = _inputs(M, N, K)
     y = ops.linear_parts(x, w)
     y = y.data.sum(0) if isinstance(y, ops.Parts) else y
@@ -151,7 +152,8 @@ def test_rules_cover_all_rows():
                 continue
             taken += 1
             high, bn, parts = (*tile, 1)[:3]
-            assert M > 256 and K % 64 == 0 and N % (
+            assert M > (128 if rule is ops._wide_parts else 256)
+            assert K % 64 == 0 and N % (
                 16 if rule is ops._wide_gated else 8) == 0
             assert 4 <= high <= 8 and bn in (128, 256)
             assert 1 <= parts <= 8 and parts * 64 <= K
