@@ -258,20 +258,37 @@ DEV void high_tile_part(const Tiles& a, char* lds, int e, int p0, int nb,
       rows.to_lds<AUX>(l, off, d * 128);
   };
   Loop loop;
-  auto run = [&](auto once) {
-    loop.run(lds, x_row, part * (BN / PARTS), (int)(row_bytes / 128), MB > 0,
+  const int chunks = (int)(row_bytes / 128);
+  auto run = [&](auto once, int turn) {
+    // which is 0 at compile time where it is
+    const auto at = [&](int d) {
+      d += turn;
+      return turn && d >= chunks ? d - chunks : d;
+    };
+    loop.run(lds, x_row, part * (BN / PARTS), chunks, MB > 0,
              [&](char* l, int d, int i) {
                load(std::false_type(), l + (FIRST * 4 + (wid & 3) * MB + i) * 1024,
-                    x_rows, x0, x_off[i], d);
+                    x_rows, x0, x_off[i], at(d));
              },
              [&](char* l, int d, int i) {
-               load(once, l + (wid * LW + i) * 1024, w_rows, w0, w_off[i], d);
+               load(once, l + (wid * LW + i) * 1024, w_rows, w0, w_off[i],
+                    at(d));
              });
   };
-  if (alone)
-    run(std::true_type());
+  // Weights of one tile, in rows that lie 4 or 8 KB apart: of one column they are all a
+  // few channels'.  So each die, which has every eighth of the tiles of outputs, begins
+  // at a column of its own, and its workgroups still share x.  us, up: 8 experts of
+  // 14336 x 4096, 120 choices each 411 -> 389, 160 417 -> 381, 256 492 489; 8 of 8192 x
+  // 4096, 150 257 -> 205; 16 of 2048 x 4096, 130 134 -> 104, 250 145 -> 123; 32 of 1024 x
+  // 2048, 130 70 -> 55, 250 78 -> 68; 64, 130 138 -> 117.  Rows of 16 and 28 KB, experts of
+  // several tiles, which wait for more than weights, and few tiles of outputs (16 of 1024
+  // x 4096, 200 61 66) are 2 to 8 % slower.
+  if (!alone)
+    run(std::false_type(), 0);
+  else if ((row_bytes == 4096 || row_bytes == 8192) && a.nx >= 16)
+    run(std::true_type(), nb % 8 * chunks / 8);
   else
-    run(std::false_type());
+    run(std::true_type(), 0);
   if constexpr (MB > 0 && FP8) {
     #pragma unroll
     for (int m = 0; m < MB; ++m) {
