@@ -67,19 +67,23 @@ __global__ __launch_bounds__(256) void greedy_sample_kernel(
 // temperature 0: the largest logit, the first among equals.  A logit that is
 // NaN is not drawn.
 //
-// What bounds it: vector instructions on every value, about 20 for a weight, and
-// the chains of steps that a row's workgroup takes one after the other.  So a row
-// is divided into slices where there are few rows (below): 64 rows of 128256 are
-// 256 workgroups, which have the largest values after 2.5 us and the weights after
-// 4, and 5 us later a second kernel of 1 (greedy) to 9 us (a share).  Lanes are
-// combined by DPP, and what the 16 waves found by 16 lanes: with shuffles, and with
-// every lane adding up 16 values, a mix of options took 24.3 us, so 21.9.  8 values
-// are looked at together where that decides about all of them.  Where few values
-// stay, and next-token logits have a few dozen that matter, they are listed and the
-// rest is done on the list, up to 8 threads a value; n values take n^2 steps, so a
-// share is looked for among 64 first (21.9 -> 19.7 us), then among 128, which is
-// where a share of 65 to 128 values is found: with both lists 28 us of 64 rows of
-// 128256, with 128 at once 25, as other shares then take too in place of 22.
+// What bounds it: vector instructions on every value, 14 (the exponential as 4) for
+// a weight of less than 2^-12 of the largest and 19 for another, and the chains of
+// steps that a row's workgroup takes one after the other.  So a row is divided into
+// slices where there are few rows (below): 64 rows of 128256 are 256 workgroups,
+// which have the largest values after 2.5 us and the weights after 6; a second kernel
+// of a workgroup a row takes 2 (greedy) to 4.5 us (a share).  Lanes are combined by
+// DPP, and what the 16 waves found by 16 lanes: with shuffles, and with every lane
+// adding up 16 values, a mix of options took 24.3 us, so 21.9.  8 values are looked at
+// together where that decides about all of them.
+// Where few values stay, and next-token logits have a few dozen that matter, they
+// are listed and the rest is done on the list, up to 8 threads a value.  n values
+// take n^2 steps, so the lists are kept short.  Each slice lists its own largest, so
+// many that a share is found among the 64 largest of the row, or top_k up to 128:
+// that takes 0.8 us where weights are computed and 2 where not, and the second kernel
+// has the row's list without a pass of its own over the row, which took it 4.5 us (a
+// mix 19.0 -> 14.5 us with the sums of weights, below).  Where that list is too short,
+// the second kernel makes one of 128 (or of top_k up to 256), as before.
 // Otherwise no sort either: one histogram of counts and weights over 2048 equal steps
 // between the largest and the smallest logit finds the step where the wanted count or
 // share is reached, and ranks the few values in it exactly (or divides that step
@@ -87,11 +91,15 @@ __global__ __launch_bounds__(256) void greedy_sample_kernel(
 // next-token logits fill few exponents: 64 lanes that add to the same few counters in
 // LDS would go one by one.
 //
-// 64 rows of 128256, 48 values far above the others, us with a workgroup a row
-// and now, rows in cache (from memory 2 to 3 more): temperature 36 14, top_p 0.9
-// 43 20, top_k 50 24 13, greedy 9.4 7.4; a mix 42 20, where the library's sorts,
-// scans and selections took 2625.  Normal logits, whose share is thousands of
-// values, 137 115.  A call that is waited for and not captured 60 36.
+// 64 rows of 128256 in bfloat16, 48 values far above the others, us with a workgroup
+// a row, in slices, and with lists of the slices (rows in cache; from memory 2 to 3
+// more): temperature 36 13.2 11.7, top_p 0.9 43 18.9 14.4, top_k 50 24 12.6 11.6,
+// greedy 9.4 6.7 6.9; a mix 42 19.0 14.5, where the library's sorts, scans and
+// selections took 2625.  A mix of 1 row 15.4 -> 12.5, of 128 26.6 -> 23.8; 64 rows of
+// 32000 16.5 -> 13.2.  What the lists cost where they do not help: normal logits, whose
+// share is thousands of values, 112 -> 114; top_k 50 of 128 rows, which are two
+// workgroups a compute unit, 16.9 -> 17.4.  A call that is waited for and not captured
+// 60 36.
 //
 // Weights are 2^-40 fixed point relative to the largest (of the row or of the
 // slice), so sums within a row or a slice are exact; slices are brought to the
@@ -109,16 +117,24 @@ constexpr int FEW = 128;          // values that a share is looked for in
 
 struct Weight {
   float mx, hi, lo;               // hi + lo = log2(e) / temperature
+  // to be cut to a whole number
+  DEV float scaled(float x) const {
+    const float d = x - mx, t = d * hi;
+    const float r = fmaf(d, hi, -t) + d * lo;
+    const float e = __builtin_amdgcn_exp2f(t);
+    return fmaf(e * r, 0.69314718f, e) * 1099511627776.f + 0.5f;
+  }
   // false: weights of x and less are below half of 2^-40
   DEV bool any(float x) const { return (x - mx) * hi > -42.f; }
   DEV u64 operator()(float x) const { return any(x) ? always(x) : 0; }
+  // the same of less than 2^-8 of the largest
+  DEV unsigned small(float x) const {
+    return (unsigned)scaled(x);
+  }
   // the same without a branch: the weights that `any` rules out, an infinity's
   // and a NaN's among them, come out as zero
   DEV u64 always(float x) const {
-    const float d = x - mx, t = d * hi;
-    const float r = fmaf(d, hi, -t) + d * lo;
-    float e = __builtin_amdgcn_exp2f(t);
-    e = fmaf(e * r, 0.69314718f, e) * 1099511627776.f + 0.5f;
+    const float e = scaled(x);
     const unsigned h = (unsigned)(e * 2.3283064e-10f);
     return (u64)h << 32 | (unsigned)fmaf((float)h, -4294967296.f, e);
   }
@@ -177,6 +193,21 @@ template <typename I, typename F> DEV I wave_scan(I x, I none, F f) {
 template <typename I> DEV I wave_scan(I x) {      // inclusive sums
   return wave_scan(x, I(0), [](I a, I b) { return a + b; });
 }
+// x[i % 4] summed over the lanes, in lane i: one step divides the four among
+// two neighbours, the next among four
+DEV u64 wave_sums(const u64* x) {
+  const int lane = threadIdx.x;
+  const bool odd = lane & 1, high = lane & 2;
+  const u64 a = (odd ? x[1] : x[0]) +
+                from_lane<0xb1, 0xf>(odd ? x[0] : x[1], u64(0));
+  const u64 b = (odd ? x[3] : x[2]) +
+                from_lane<0xb1, 0xf>(odd ? x[2] : x[3], u64(0));
+  u64 c = (high ? b : a) + from_lane<0x4e, 0xf>(high ? a : b, u64(0));
+  c += from_lane<0x124, 0xf>(c, u64(0));          // row_ror by 4 and 8
+  c += from_lane<0x128, 0xf>(c, u64(0));
+  c += __shfl_xor(c, 16);
+  return c + __shfl_xor(c, 32);
+}
 template <typename I> DEV I lane_of(I x, int lane) {       // uniform
   if constexpr (sizeof(I) == 8) {
     const u64 a = __builtin_bit_cast(u64, x);
@@ -195,6 +226,14 @@ template <typename I> DEV I sum_of_16(const I* x, int before, I* sum) {
   *sum = lane_of(upto, 15);
   return before ? lane_of(upto, before - 1) : I(0);
 }
+// the sum alone: row_ror by 8, 4, 2 and 1
+DEV u64 sum_of_16(const u64* x) {
+  u64 y = x[threadIdx.x & 15];
+  y += from_lane<0x128, 0xf>(y, u64(0));
+  y += from_lane<0x124, 0xf>(y, u64(0));
+  y += from_lane<0x122, 0xf>(y, u64(0));
+  return y + from_lane<0x121, 0xf>(y, u64(0));
+}
 DEV float min_of(float a, float b) { return fminf(a, b); }
 
 struct alignas(16) Entry {        // one LDS load
@@ -209,8 +248,8 @@ struct Scratch {
   Entry entry[LIST];
   u64 wave_mass[16];
   unsigned wave_count[16];
-  u64 before_mass, kept_mass;
-  unsigned before_count, n, key_min, key_max, keep;
+  u64 before_mass, kept_mass, list_mass[16];
+  unsigned before_count, n, key_min, key_max, keep, stay;
   int step, found;
   float value;
 };
@@ -512,86 +551,122 @@ DEV u64 sum_of_all(Scratch& s, u64 x) {
   return x;
 }
 
+// the sum over `share` neighbouring lanes: quad_perm, and row_half_mirror
+template <typename I> DEV I sum_of_neighbours(I x, int share) {
+  x += from_lane<0xb1, 0xf>(x, I(0));
+  if (share > 2) x += from_lane<0x4e, 0xf>(x, I(0));
+  if (share > 4) x += from_lane<0x141, 0xf>(x, I(0));
+  return x;
+}
+
+// of the weight z; some value has it
+DEV u64 part_of(float p, u64 z) { return (u64)ceil((double)p * (double)z); }
+
+// in descending order, and by index among equals, larger keys are earlier; the
+// zeros are equal
+DEV u64 key_of(float x, int at) {
+  return (u64)ordered(x + 0.f) << 32 | (unsigned)~at;
+}
+
+// threads a value, each with a part of the others
+DEV int share_of(int n) { return n <= NT / 8 ? 8 : n <= NT / 4 ? 4 : 2; }
+
+// Draws from the n entries, among which is all that stays, and writes the token.
+// k 0: no top_k, and the first values with `part` of the weight stay.  s.stay is
+// 0.
+DEV void draw_from_entries(Scratch& s, int n, int vocab, int k, float p,
+                           float u, u64 part, long* out) {
+  const int tid = threadIdx.x;
+  Entry* const stay = reinterpret_cast<Entry*>(s.mass);
+  {
+    const int share = share_of(n), mine = tid / share, first = tid % share;
+    const bool one_of = mine < n;
+    Entry own{0, 0};
+    if (one_of) own = s.entry[mine];
+    const unsigned value = own.key >> 32;
+    int greater = 0;
+    bool stays = one_of;
+    if (p < 1.f) {
+      u64 above = 0;
+      if (one_of)
+        #pragma unroll 4
+        for (int j = first; j < n; j += share) {
+          const Entry e = s.entry[j];
+          above += e.key > own.key ? e.mass : 0;
+          greater += (unsigned)(e.key >> 32) > value;
+        }
+      above = sum_of_neighbours(above, share);
+      if (k) {
+        stays = stays && sum_of_neighbours(greater, share) < k;
+        part = part_of(p, sum_of_all(s, stays && first == 0 ? own.mass : 0));
+      }
+      stays = stays && above < part;
+    } else {
+      if (one_of)
+        #pragma unroll 4
+        for (int j = first; j < n; j += share)
+          greater += (unsigned)(s.entry[j].key >> 32) > value;
+      stays = stays && sum_of_neighbours(greater, share) < k;
+    }
+    if (stays && first == 0)
+      stay[atomicAdd(&s.stay, 1u)] = {(u64)~(unsigned)own.key, own.mass};
+    __syncthreads();
+  }
+  // in the order of indices
+  n = (int)s.stay;
+  const int share = share_of(n), mine = tid / share, first = tid % share;
+  const bool one_of = mine < n;
+  u64 all = 0, upto = 0;
+  Entry own{0, 0};
+  if (one_of) {
+    own = stay[mine];
+    #pragma unroll 4
+    for (int j = first; j < n; j += share) {
+      const Entry e = stay[j];
+      all += e.mass;
+      upto += (unsigned)e.key < (unsigned)own.key ? e.mass : 0;
+    }
+  }
+  all = sum_of_neighbours(all, share);
+  upto = sum_of_neighbours(upto, share);
+  if (one_of && first == 0) {
+    const u64 target = (u64)((double)u * (double)all);
+    if (target >= all)
+      *out = vocab - 1;
+    else if (upto <= target && upto + own.mass > target)
+      *out = (int)(unsigned)own.key;
+  }
+}
+
 // The draw from the s.n values that are listed, if all that stays is among
 // them.  k 0: no top_k, and z is the weight of all values, of which top_p is a
 // share.  False if the list is too short for the share or too long.
 DEV bool draw_from_list(Scratch& s, const Weight& w, int vocab, int k, float p,
-                        float u, u64 z, int* drawn) {
+                        float u, u64 z, long* out) {
   const int tid = threadIdx.x;
   const int n = (int)s.n;
   if (n > LIST) {
     __syncthreads();
     return false;
   }
-  // in descending order, and by index among equals, larger keys are earlier;
-  // the zeros are equal
   u64 mass = 0;
+  if (tid == 0) s.stay = 0;
   if (tid < n) {
     mass = w(s.list[tid]);
-    s.entry[tid] = {(u64)ordered(s.list[tid] + 0.f) << 32 |
-                        (unsigned)~s.list_at[tid],
-                    mass};
+    s.entry[tid] = {key_of(s.list[tid], s.list_at[tid]), mass};
   }
-  if (tid == 0) s.found = vocab - 1;
   // a list that is too short is left before its values are ranked
-  const bool share_of_all = k == 0 && p < 1.f;
-  const u64 part_of = share_of_all ? (u64)ceil((double)p * (double)z) : 0;
-  if (!share_of_all) {
-    __syncthreads();
-  } else if (sum_of_all(s, mass) < part_of) {    // a barrier on the way
-    __syncthreads();
-    return false;
-  }
-  // `share` neighbouring threads a value, each with a part of the others
-  const int share = n <= NT / 8 ? 8 : n <= NT / 4 ? 4 : 2;
-  const int mine = tid / share, part = tid % share;
-  const bool one_of = mine < n;
-  auto sum = [&](auto v) {
-    for (int o = 1; o < share; o <<= 1) v += __shfl_xor(v, o);
-    return v;
-  };
-  Entry own{0, 0};
-  u64 above = 0;
-  int greater = 0;
-  if (one_of) {
-    own = s.entry[mine];
-    #pragma unroll 4
-    for (int j = part; j < n; j += share) {
-      const Entry e = s.entry[j];
-      above += e.key > own.key ? e.mass : 0;
-      greater += (unsigned)(e.key >> 32) > (unsigned)(own.key >> 32);
+  u64 part = 0;
+  if (k == 0 && p < 1.f) {
+    part = part_of(p, z);
+    if (sum_of_all(s, mass) < part) {            // a barrier on the way
+      __syncthreads();
+      return false;
     }
-  }
-  above = sum(above);
-  greater = sum(greater);
-  bool stays = one_of && (k == 0 || greater < k);
-  if (p < 1.f && !share_of_all) {
-    const u64 kept = sum_of_all(s, stays && part == 0 ? own.mass : 0);
-    stays = stays && above < (u64)ceil((double)p * (double)kept);
   } else {
-    stays = stays && (!share_of_all || above < part_of);
     __syncthreads();
   }
-  // every thread has read the entries: now by index, what does not stay as 0
-  const int index = (int)~(unsigned)own.key;
-  if (one_of && part == 0)
-    s.entry[mine] = {(u64)(unsigned)index, stays ? own.mass : 0};
-  __syncthreads();
-  u64 all = 0, upto = 0;
-  if (stays) {
-    #pragma unroll 4
-    for (int j = part; j < n; j += share) {
-      const Entry e = s.entry[j];
-      all += e.mass;
-      upto += (int)e.key < index ? e.mass : 0;
-    }
-  }
-  all = sum(all);
-  upto = sum(upto);
-  const u64 target = (u64)((double)u * (double)all);
-  if (stays && upto <= target && upto + own.mass > target) s.found = index;
-  __syncthreads();
-  *drawn = s.found;
+  draw_from_entries(s, n, vocab, k, p, u, part, out);
   return true;
 }
 
@@ -602,7 +677,7 @@ DEV bool draw_from_list(Scratch& s, const Weight& w, int vocab, int k, float p,
 // if the list is too short for the share or too long.
 template <typename R>
 DEV bool draw_from_few(Scratch& s, const R& row, const Weight& w, float own,
-                       int k, float p, float u, u64* all, int* drawn) {
+                       int k, float p, float u, u64* all, long* out) {
   const int tid = threadIdx.x;
   const int want_n = k > 0 ? k : FEW;
   const unsigned key = ordered(own);
@@ -635,7 +710,7 @@ DEV bool draw_from_few(Scratch& s, const R& row, const Weight& w, float own,
   z = sum_of_all(s, z);
   __syncthreads();                // the list's sum goes the same way
   *all = z;
-  return draw_from_list(s, w, row.vocab, k, p, u, z, drawn);
+  return draw_from_list(s, w, row.vocab, k, p, u, z, out);
 }
 
 // Best of all threads: the largest value mx, the lowest index `at` of the 8
@@ -783,43 +858,80 @@ __global__ __launch_bounds__(NT) void sample_kernel(
     return;
   }
   u64 kept = 0;
-  int drawn;
   // a share is not looked for where many threads' largest values weigh more
   // than 2^-7 of the largest: the list would be too short
-  bool done = o.k ? o.k <= LIST / 2
-                  : o.p < 1.f && __syncthreads_count((own - mx) * w.hi > -7.f)
-                                     <= 2 * FEW;
-  if (done) {
-    done = draw_from_few(s, row, w, own, o.k, o.p, o.uniform, &kept, &drawn);
-    __syncthreads();
-  }
-  if (!done)
-    drawn = draw_from_row(s, row, w, mn, o.hi, o.k, o.p, o.uniform, kept);
+  const bool few = o.k
+      ? o.k <= LIST / 2
+      : o.p < 1.f && __syncthreads_count((own - mx) * w.hi > -7.f) <= 2 * FEW;
+  if (few && draw_from_few(s, row, w, own, o.k, o.p, o.uniform, &kept, out + b))
+    return;
+  __syncthreads();
+  const int drawn =
+      draw_from_row(s, row, w, mn, o.hi, o.k, o.p, o.uniform, kept);
   if (tid == 0) out[b] = drawn;
 }
 
 // ---- rows in slices -------------------------------------------------------
 // A row a workgroup leaves most of the chip idle.  Here a row is divided into
 // slices of a workgroup each, which read their values once; what they find out
-// meets in a second kernel, a workgroup a row.  Weights are relative to the
+// meets in a second kernel, a workgroup a row, with the largest values of each.  Weights are relative to the
 // slice's own largest value, so that no slice waits for another one; the sums of
 // 512 values are exact, and are brought to the row's largest value by one factor
 // a slice.
-constexpr int HELD = 4;           // 8 values each, that a thread has
+constexpr int HELD = 4;           // 8 values each, that a thread has (wave_sums)
 constexpr int SLICES = 16;        // of a row at most
 constexpr int UNITS = 4;          // a thread of the second kernel has at most
 constexpr int CHUNKS = HELD * 16; // 512 values of a wave each
+constexpr int NEAR = 256;         // values that are listed of a row
+constexpr int SHARE = 64;         // among so many a share is looked for first
 
 struct Slice {
   u64 mass[CHUNKS];               // weights of the chunks, where asked for
   float mx, mn;                   // largest (-inf: no value), smallest
   int at;                         // first of the 8 with the first largest
-  int pad;
+  float low;                      // values from it on are listed
+  int n;                          // as many
+  int list_at[NEAR];
+  float list[NEAR];
   float own[NT];                  // largest values of the threads, or of 2 or 4
 };
 
 // threads of a slice whose values are looked at together
 DEV int together(int slices) { return slices <= 4 ? 1 : slices <= 8 ? 2 : 4; }
+
+// whether slices list values for top_k (0: there is none)
+DEV bool listed_k(int k) { return k > 0 && k <= NEAR / 2; }
+
+constexpr int COUNTS = 256;       // steps that a slice's threads are counted in
+
+// From s.count, how many threads' largest values are in each of COUNTS steps: the
+// end of the step in which `want` of them are reached; COUNTS + 1 if there are
+// fewer.  Each wave by itself, 4 steps a lane.
+DEV int end_of(const Scratch& s, unsigned want) {
+  const int lane = threadIdx.x & 63;
+  const uint4 c = reinterpret_cast<const uint4*>(s.count)[lane];
+  const unsigned upto = wave_scan(c.x + c.y + c.z + c.w);
+  const u64 there = __ballot(upto >= want);
+  if (!there) return COUNTS + 1;
+  const int end = lane * 4 + 4 - (upto - c.w >= want) -
+                  (upto - c.w - c.z >= want) -
+                  (upto - c.w - c.z - c.y >= want);
+  return lane_of(end, __ffsll(there) - 1);
+}
+
+// Steps below the largest value, down to where weights are zero
+struct Steps {
+  float mx, zero, range, scale;
+  bool whole;                     // down to there, and not only to the smallest
+  DEV void between(float largest, float mn, float hi, int steps) {
+    mx = largest;
+    zero = 43.f / hi;
+    range = mn >= -FLT_MAX ? fminf(mx - mn, zero) : zero;
+    scale = (float)steps * __builtin_amdgcn_rcpf(fmaxf(range, 1e-30f));
+    whole = range >= zero;
+  }
+  DEV float of(float x) const { return (mx - x) * scale; }
+};
 
 template <typename T, bool VEC>
 __global__ __launch_bounds__(NT) void sample_slice_kernel(
@@ -839,20 +951,24 @@ __global__ __launch_bounds__(NT) void sample_slice_kernel(
     row.hold(first + (q * NT + tid) * 8, end, raw[q]);
   const Options o = options_of(b, temperature, top_p, top_k, temperature,
                                vocab);
+  s.count[tid] = 0;
+  if (tid == 0) s.n = 0;
   float mx = -INFINITY, mn = INFINITY;
   int at = vocab;
+  float top[HELD];                // largest of each 8
   #pragma unroll
   for (int q = 0; q < HELD; ++q) {
     const int i = first + (q * NT + tid) * 8;
     float x[8];
     row.spread(raw[q], x);
-    const float m = largest(x), n = smallest(x);
+    const float m = top[q] = largest(x), n = smallest(x);
     if (m > mx && mx < FLT_MAX) {
       mx = fminf(m, FLT_MAX);
       at = i;
     }
     if (i + 8 <= end) mn = fminf(mn, n);
   }
+  const float thread_mx = mx;
   float own = mx;
   const int group = together(slices);
   for (int i = 1; i < group; i <<= 1) own = fmaxf(own, __shfl_xor(own, i));
@@ -863,22 +979,107 @@ __global__ __launch_bounds__(NT) void sample_slice_kernel(
     mine.mn = mn;
     mine.at = at;
   }
-  if (o.t == 0.f || o.k || !(mx >= -FLT_MAX)) {
+  if (o.t == 0.f || !(mx >= -FLT_MAX)) {
     if (tid < CHUNKS) mine.mass[tid] = 0;
+    if (tid == 0) {
+      mine.low = -INFINITY;
+      mine.n = 0;
+    }
     return;
   }
-  const Weight w = o.weight(mx);
+  // What is listed: for top_k as many values as a slice has where the k largest
+  // are spread by chance, and 4 times the root of that (with 3 times a row in 16
+  // slices had less than k in them now and then: 16 rows with top_k 50 12.2 -> 13.8
+  // us), or all that have weight; for a share the same of SHARE, but none of less
+  // than 2^-16 of the largest.
+  const bool listing = o.k ? listed_k(o.k) : o.p < 1.f;
+  Steps steps;
+  float last = COUNTS;
+  if (listing) {
+    steps.between(mx, mn, o.hi, COUNTS);
+    if (!o.k) last = fminf(16.f / 43.f * steps.zero * steps.scale, COUNTS);
+    const float step = steps.of(thread_mx);
+    if (step < last) atomicAdd(&s.count[(int)step], 1u);
+  }
   row.finite = mx < FLT_MAX;
-  #pragma unroll
-  for (int q = 0; q < HELD; ++q) {
-    float x[8];
-    row.spread(raw[q], x);
-    u64 z = 0;
-    if (w.any(largest(x)))
+  if (!o.k) {
+    const Weight w = o.weight(mx);
+    u64 sum[HELD];
+    #pragma unroll
+    for (int q = 0; q < HELD; ++q) {
+      float x[8];
+      row.spread(raw[q], x);
+      u64 z = 0;
+      // 8 weights of less than 2^-12 are a sum of 32 bits
+      if (__all(!((top[q] - mx) * w.hi >= -12.f))) {
+        unsigned of8 = 0;
+        if (w.any(top[q]))
+          #pragma unroll
+          for (int i = 0; i < 8; ++i) of8 += w.small(x[i]);
+        z = of8;
+      } else if (w.any(top[q])) {
+        #pragma unroll
+        for (int i = 0; i < 8; ++i) z += w.always(x[i]);
+      }
+      sum[q] = z;
+    }
+    const u64 z = wave_sums(sum);
+    if (lane < HELD) mine.mass[lane * 16 + wid] = z;
+  }
+  const float none = from_ordered(ordered(mx) + 1);
+  if (!listing) {
+    if (tid == 0) {
+      mine.low = none;
+      mine.n = 0;
+    }
+    return;
+  }
+  __syncthreads();
+  const float part = (float)(o.k ? o.k : SHARE) *
+                     __builtin_amdgcn_rcpf((float)slices);
+  const int reached =
+      end_of(s, (unsigned)(part + 4.f * __builtin_amdgcn_sqrtf(part)) + 2);
+  const float low = reached > COUNTS && o.k && !steps.whole
+      ? none
+      : fmaxf(mx - fminf((float)reached, last) * (steps.range / COUNTS), -FLT_MAX);
+  // too many: without a look at each of them
+  const int most = NEAR / group;
+  if (__popcll(__ballot(thread_mx >= low)) > most / 4) {
+    if (lane == 0) atomicAdd(&s.n, NEAR + 1u);
+  } else {
+    // a thread has few, so each goes through its own: one of its 8 values, and
+    // one of these
+    unsigned loads = 0;
+    #pragma unroll
+    for (int q = 0; q < HELD; ++q) loads |= (top[q] >= low) << q;
+    for (; loads; loads &= loads - 1) {
+      const int q = __ffs(loads) - 1;
+      auto r = raw[0];
       #pragma unroll
-      for (int i = 0; i < 8; ++i) z += w.always(x[i]);
-    z = wave_scan(z);
-    if (lane == 63) mine.mass[q * 16 + wid] = z;
+      for (int j = 1; j < HELD; ++j)
+        if (q == j) r = raw[j];
+      float x[8];
+      row.spread(r, x);
+      unsigned hits = 0;
+      #pragma unroll
+      for (int i = 0; i < 8; ++i) hits |= (x[i] >= low) << i;
+      for (; hits; hits &= hits - 1) {
+        const int i = __ffs(hits) - 1;
+        float y = x[0];
+        #pragma unroll
+        for (int j = 1; j < 8; ++j) y = i == j ? x[j] : y;
+        const int n = (int)atomicAdd(&s.n, 1u);
+        if (n < most) {
+          mine.list[n] = y;
+          mine.list_at[n] = first + (q * NT + tid) * 8 + i;
+        }
+      }
+    }
+  }
+  __syncthreads();
+  if (tid == 0) {
+    mine.low = (int)s.n <= most ? low : none;
+    mine.n = (int)s.n <= most ? (int)s.n : 0;
   }
 }
 
@@ -894,10 +1095,17 @@ __global__ __launch_bounds__(NT) void sample_slices_kernel(
   const long b = blockIdx.x;
   slice += b * slices;
   Row<T, VEC> row{logits + b * vocab, vocab, true};
-  // All loads are issued before anything waits: chunk `tid` of the row, the
-  // largest values of UNITS units, and by lane i of 16 what slice i says.
+  // All loads are issued before anything waits: chunk `tid` of the row, a value
+  // that a slice lists, the largest values of UNITS units, and by lane i of 16 what
+  // slice i says.
   const u64 chunk = slice[min(tid / CHUNKS, slices - 1)].mass[tid % CHUNKS];
-  const int group = together(slices), each = NT / group;   // units a slice
+  const int group = together(slices), most = NEAR / group;
+  // all of a wave are in one list
+  const int from_list = __builtin_amdgcn_readfirstlane(tid / most);
+  const Slice& listing = slice[min(from_list, slices - 1)];
+  const float x = listing.list[tid % most];
+  const int x_at = listing.list_at[tid % most];
+  const int each = NT / group;  // units a slice
   float own[UNITS];
   #pragma unroll
   for (int q = 0; q < UNITS; ++q) {
@@ -906,17 +1114,15 @@ __global__ __launch_bounds__(NT) void sample_slices_kernel(
   }
   const Slice& head = slice[min(lane & 15, slices - 1)];
   const float slice_mx = head.mx;
-  float mx = slice_mx, mn = head.mn;
+  const int slice_n = head.n;
+  float mx = slice_mx, mn = head.mn, low = head.low;
   int at = head.at;
   const Options o = options_of(b, temperature, top_p, top_k, uniform, vocab);
-  if (tid == 0) s.n = 0;
-  s.count[tid] = 0;
   const u64 best = lane_of(
       row_scan((u64)ordered(mx + 0.f) << 32 | (unsigned)~at, u64(0),
                [](u64 a, u64 b) { return a > b ? a : b; }), 15);
   mx = from_ordered((unsigned)(best >> 32));
   at = (int)~(unsigned)best;
-  mn = fminf(lane_of(row_scan(mn, INFINITY, min_of), 15), mx);
   if (o.t == 0.f || !(mx >= -FLT_MAX)) {
     if (tid == 0)
       out[b] = greedy_index(row.p, mx, at, vocab, o.t == 0.f ? 0 : vocab - 1);
@@ -927,90 +1133,120 @@ __global__ __launch_bounds__(NT) void sample_slices_kernel(
     return;
   }
   const Weight w = o.weight(mx);
-  u64 z = 0;                      // weight of all
-  if (!o.k) {
-    const double factor = exp2(((double)slice_mx - (double)mx) *
+  u64 mass = 0, upto = 0;         // of the wave's chunks, which are of one slice
+  if (!o.k && wid < slices) {
+    const double factor = exp2(((double)lane_of(slice_mx, wid) - (double)mx) *
                                ((double)o.hi + (double)o.lo));
-    const double share = __shfl(factor, tid / CHUNKS & 15);
-    const u64 mass = tid < slices * CHUNKS && chunk
-        ? (u64)rint((double)chunk * share) : 0;
-    const u64 upto = wave_scan(mass);
-    if (lane == 63) s.wave_mass[wid] = upto;
+    if (chunk) mass = (u64)rint((double)chunk * factor);
+    upto = wave_scan(mass);
+  }
+  if (lane == 63) s.wave_mass[wid] = upto;
+  if (!o.k && !(o.p < 1.f)) {
     __syncthreads();
+    u64 z;
     const u64 before = sum_of_16(s.wave_mass, wid, &z);
-    if (!(o.p < 1.f)) {
-      // the token is in the chunk where the running sum passes the target;
-      // there sums are those of the slice's own weights again
-      const u64 target = (u64)((double)o.uniform * (double)z);
-      if (target >= z) {
-        if (tid == 0) out[b] = vocab - 1;
-        return;
-      }
-      // a wave has the chunks of one slice, in the order of its values
-      const u64 over = __ballot(before + upto > target);
-      if (before > target || !over) return;
-      const int i = __ffsll(over) - 1, of = wid;
-      const u64 all = __shfl(chunk, i);
-      const double part = (double)(target - before - __shfl(upto - mass, i)) /
-                          (double)__shfl(mass, i);
-      const u64 goal = min((u64)(part * (double)all), all - 1);
-      const Weight wi = o.weight(__shfl(slice_mx, of));
-      row.finite = wi.mx < FLT_MAX;
-      const int stop = min((of + 1) * span, vocab);
-      const int from = of * span + i * 512 + lane * 8;
-      typename Row<T, VEC>::Raw raw;
-      row.hold(from, stop, raw);
-      float x[8];
-      row.spread(raw, x);
-      u64 sum = 0;
-      #pragma unroll
-      for (int j = 0; j < 8; ++j) sum += wi.always(x[j]);
-      const u64 mine = wave_scan(sum);
-      const u64 here = __ballot(mine > goal);
-      if (lane == __ffsll(here) - 1) {
-        u64 c = mine - sum;
-        int found = 0;
-        #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          c += wi.always(x[j]);
-          found += c <= goal;
-        }
-        out[b] = from + found;
-      }
+    // the token is in the chunk where the running sum passes the target;
+    // there sums are those of the slice's own weights again
+    const u64 target = (u64)((double)o.uniform * (double)z);
+    if (target >= z) {
+      if (tid == 0) out[b] = vocab - 1;
       return;
     }
+    // a wave has the chunks of one slice, in the order of its values
+    const u64 over = __ballot(before + upto > target);
+    if (before > target || !over) return;
+    const int i = __ffsll(over) - 1, of = wid;
+    const u64 all = __shfl(chunk, i);
+    const double part = (double)(target - before - __shfl(upto - mass, i)) /
+                        (double)__shfl(mass, i);
+    const u64 goal = min((u64)(part * (double)all), all - 1);
+    const Weight wi = o.weight(__shfl(slice_mx, of));
+    row.finite = wi.mx < FLT_MAX;
+    const int stop = min((of + 1) * span, vocab);
+    const int from = of * span + i * 512 + lane * 8;
+    typename Row<T, VEC>::Raw raw;
+    row.hold(from, stop, raw);
+    float x[8];
+    row.spread(raw, x);
+    u64 sum = 0;
+    #pragma unroll
+    for (int j = 0; j < 8; ++j) sum += wi.always(x[j]);
+    const u64 mine = wave_scan(sum);
+    const u64 here = __ballot(mine > goal);
+    if (lane == __ffsll(here) - 1) {
+      u64 c = mine - sum;
+      int found = 0;
+      #pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        c += wi.always(x[j]);
+        found += c <= goal;
+      }
+      out[b] = from + found;
+    }
+    return;
   }
-  row.finite = mx < FLT_MAX;
+  // What the slices list of the values from the highest of their ends on is all
+  // that the row has of them.
+  low = lane_of(row_scan(low, -INFINITY, [](float a, float b) {
+    return fmaxf(a, b);
+  }), 15);
+  const bool listed = from_list < slices && x >= low &&
+                      tid % most < lane_of(slice_n, from_list & 15);
+  const u64 lanes = __ballot(listed);
+  u64 x_mass = 0, list_mass = 0;
+  if (lanes) {
+    x_mass = listed ? w(x) : 0;
+    if (!o.k) list_mass = wave_scan(x_mass);
+  }
+  if (lane == 63) {
+    s.list_mass[wid] = list_mass;
+    s.wave_count[wid] = __popcll(lanes);
+  }
+  if (tid == 0) s.n = s.keep = s.stay = 0;
+  s.count[tid] = 0;
+  __syncthreads();
+  u64 z = 0, part = 0;            // weight of all
+  unsigned n;
+  const int place = (int)sum_of_16(s.wave_count, wid, &n) +
+                    __popcll(lanes & ((u64(1) << lane) - 1));
+  bool done = n > 0 && n <= NEAR;
+  if (o.k) {
+    // or below the list there is no weight
+    done = done && ((int)n >= o.k || !w.any(low));
+  } else {
+    z = sum_of_16(s.wave_mass);
+    part = part_of(o.p, z);
+    done = done && sum_of_16(s.list_mass) >= part;
+  }
+  if (done) {
+    if (listed) s.entry[place] = {key_of(x, x_at), x_mass};
+    __syncthreads();
+    draw_from_entries(s, (int)n, vocab, o.k, o.p, o.uniform, part, out + b);
+    return;
+  }
   // The draw where all that stays is among few values: the want-th largest of
   // the units' largest values has at least that many values at or above it, and
   // hardly more.  A share is not looked for where many units' largest values
   // weigh more than 2^-7 of the largest: the list would be too short.
+  mn = fminf(lane_of(row_scan(mn, INFINITY, min_of), 15), mx);
+  row.finite = mx < FLT_MAX;
   int near = 0;
   #pragma unroll
   for (int q = 0; q < UNITS; ++q)
     near += __popcll(__ballot((own[q] - mx) * w.hi > -7.f));
-  // steps below the largest value, down to where weights are zero
-  const float zero = 43.f / w.hi;
-  const float range = mn >= -FLT_MAX ? fminf(mx - mn, zero) : zero;
-  const float scale = NT / fmaxf(range, 1e-30f);
-  __syncthreads();
+  Steps steps;
+  steps.between(mx, mn, w.hi, NT);
   if (lane == 0) atomicAdd(&s.n, (unsigned)near);
   #pragma unroll
   for (int q = 0; q < UNITS; ++q) {
-    const float step = (mx - own[q]) * scale;
+    const float step = steps.of(own[q]);
     if (step < (float)NT) atomicAdd(&s.count[(int)step], 1u);
   }
   __syncthreads();
-  int drawn;
-  bool done = false;
-  const bool few = o.k ? o.k <= LIST / 2 : s.n <= 2 * FEW;
-  for (unsigned want = o.k ? o.k : FEW / 2; few && !done; want = FEW) {
-    const unsigned upto = wave_scan(s.count[tid]);
+  if (o.k ? o.k <= LIST / 2 : s.n <= 2 * FEW) {
+    const unsigned want = o.k ? o.k : FEW, upto = wave_scan(s.count[tid]);
     if (lane == 63) s.wave_count[wid] = upto;
-    if (tid == 0) {
-      s.n = 0;
-      s.step = NT + 1;
-    }
+    if (tid == 0) s.step = NT + 1;
     __syncthreads();
     unsigned all;
     const unsigned before = sum_of_16(s.wave_count, wid, &all);
@@ -1019,20 +1255,18 @@ __global__ __launch_bounds__(NT) void sample_slices_kernel(
     __syncthreads();
     // NT + 1: fewer units than wanted are in the steps.  Then every value that
     // has weight may stay, the smallest ones, which no step has, among them.
-    const float end = s.step <= NT || range >= zero ? (float)s.step : INFINITY;
+    const float end = s.step <= NT || steps.whole ? (float)s.step : INFINITY;
     #pragma unroll
     for (int q = 0; q < UNITS; ++q)
-      if ((mx - own[q]) * scale < end) {
-        const unsigned n = atomicAdd(&s.n, 1u);
+      if (steps.of(own[q]) < end) {
+        const unsigned n = atomicAdd(&s.keep, 1u);
         if (n < LIST) unit[n] = q * NT + tid;
       }
     __syncthreads();
-    const int units = (int)s.n;
-    __syncthreads();
+    const int units = (int)s.keep;
     if (tid == 0) s.n = 0;
     __syncthreads();
-    done = units <= LIST;
-    if (done) {
+    if (units <= LIST) {
       // loads of 8 values: of `group` threads, as often as those loaded
       const int loads = group * ((span + NT * 8 - 1) / (NT * 8));
       for (int i = tid; i < units * loads; i += NT) {
@@ -1045,7 +1279,7 @@ __global__ __launch_bounds__(NT) void sample_slices_kernel(
         row.spread(raw, x);
         #pragma unroll
         for (int v = 0; v < 8; ++v)
-          if ((mx - x[v]) * scale < end) {
+          if (steps.of(x[v]) < end) {
             const unsigned n = atomicAdd(&s.n, 1u);
             if (n < LIST) {
               s.list[n] = x[v];
@@ -1054,13 +1288,12 @@ __global__ __launch_bounds__(NT) void sample_slices_kernel(
           }
       }
       __syncthreads();
-      done = draw_from_list(s, w, vocab, o.k, o.p, o.uniform, z, &drawn);
+      if (draw_from_list(s, w, vocab, o.k, o.p, o.uniform, z, out + b)) return;
     }
-    __syncthreads();
-    if (o.k || want == FEW || units > LIST) break;
   }
-  if (!done)
-    drawn = draw_from_row(s, row, w, mn, o.hi, o.k, o.p, o.uniform, z);
+  __syncthreads();
+  const int drawn =
+      draw_from_row(s, row, w, mn, o.hi, o.k, o.p, o.uniform, z);
   if (tid == 0) out[b] = drawn;
 }
 

@@ -236,6 +236,42 @@ def test_shares_of_more_values_than_are_listed_first(vocab):
         assert ok[out[b]], (n, same, float(u[b]))
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("vocab,rows", [
+    (8200, 64), (16384, 130), (50257, 40), (128256, 3), (128256, 60)])
+def test_lists_of_slices(vocab, rows, dtype):
+    """What 1 to 15 slices list of their largest values: these in one slice, in one
+    wave or in none more than elsewhere, more equal ones than a list takes, weights
+    about 2^-12 of the largest, and top_k and shares that just have a list or not."""
+    g = torch.Generator().manual_seed(vocab + rows)
+    x = torch.randn(8, vocab, generator=g)
+    anywhere = torch.randperm(vocab, generator=g)
+    x[0, 5:65] += 20                           # one wave has all
+    x[1, anywhere[:300]] = 9.0                 # equal, more than are listed
+    x[2, anywhere[:250]] = 9.0 + torch.rand(250, generator=g)
+    x[3] = -torch.log(anywhere + 1.0) * 1.2    # a power law
+    x[4] = 12 - 12 * 0.6931472 + 0.02 * x[4]   # many of 2^-12
+    x[4, anywhere[:9]] = 12.0
+    x[5, anywhere[20:]] = float("-inf")        # fewer values than top_k
+    x[6, anywhere[:40]] = 60.0                 # and others without weight
+    x[7, vocab // 2:] -= 30                    # slices far below the others
+    x = x.to(dtype)
+    options = [(1.0, 0.9, 0), (0.8, 0.999, 0), (1.0, 1.0, 0), (1.0, 1.0, 50),
+               (0.7, 0.95, 128), (1.0, 1.0, 129), (1.0, 0.3, 1)]
+    pick = [(i, o, (n + 0.5) / 5) for i in range(8)
+            for o in range(len(options)) for n in range(5)]
+    t, p, k = (torch.tensor(c) for c in zip(*(options[o] for _, o, _ in pick)))
+    which = torch.tensor([i for i, _, _ in pick])
+    u = torch.tensor([n for _, _, n in pick])
+    out = torch.cat([
+        ops.sample(*(c.to(DEV) for c in (x[which[a]], t[a], p[a], k[a].int(),
+                                         u[a])))
+        for a in torch.arange(len(pick)).split(rows)]).tolist()
+    for b, (i, o, n) in enumerate(pick):
+        ok, _ = _allowed(x[i].float(), *options[o], float(u[b]))
+        assert ok[out[b]], (i, options[o], out[b], n)
+
+
 @pytest.mark.parametrize("vocab", [1000, 32768])
 def test_zeros_of_either_sign_are_equal(vocab):
     """The first of the largest values is -0."""
