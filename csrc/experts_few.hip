@@ -21,8 +21,9 @@
 // non-temporal; that was slower still):
 //   32 experts of 1024 x 2048, 4 each   1 row 9.0 5.8 (10.1 7.2), 4 rows 22.7
 //     12.9 (25.5 14.4), 16 rows 44 24 (49 27)
-//   8 experts of 14336 x 4096, 2 each   1 row 78 45 (82 59), 4 rows 179 105
-//     (200 125), 10 rows 268 157 (302 177)
+//   8 experts of 14336 x 4096, 2 each   1 row 74 40 (82 59), 4 rows 179 105
+//     (200 125), 10 rows 268 157 (302 177); the last two before workgroups began at
+//     different columns (below), which is 2 to 9 %
 #include <type_traits>
 
 #include "common.h"
@@ -76,6 +77,16 @@ __global__ __launch_bounds__(WAVES * 64) void experts_few_kernel(Few a) {
   const bf16* wp =
       a.w + ((long)e * (UP ? 2 * a.N : a.N) + n0 + col) * a.K + at;
   const long next = (long)(UP ? a.N : 8) * a.K;    // up rows, or 8 rows on
+  // Workgroups begin at different columns where rows are multiples of 4 KB, of
+  // which one column is a few channels of memory; by their rows of weights, so
+  // that a choice's sums do not depend on the others.  us, up and down: 8 experts of
+  // 14336 x 4096, 2 choices 79.3 43.8 -> 74.4 39.9, 16 258 145 -> 247 133; 16 of 2048
+  // x 4096, 8 48.1 26.7 -> 44.4 23.3; of 3072 x 6144, 88.2 -> 86.5 (up).  Of other
+  // lengths it is 0 to 2 % slower, and even where the up product has rows of 4 KB: 32 of
+  // 1024 x 2048, 16 21.7 21.9, 64 of 1408 x 2048, 24 42.1 41.1.
+  const int batches = a.K / (2 * STEP);
+  const int begin = a.K % 2048 == 0 && a.K > (UP ? 2048 : 1024)
+      ? (int)(blockIdx.x / 8 % (unsigned)batches) : 0;
   for (int r0 = 0; r0 < count; r0 += 16) {
     const bf16* xp[2];                         // of 8 choices and 8 more
     bool live[2];
@@ -114,11 +125,14 @@ __global__ __launch_bounds__(WAVES * 64) void experts_few_kernel(Few a) {
       add(0);
       if (more) add(1);
     };
-    int k = wid * 64;
+    int turn = begin;
     #pragma unroll 1
-    for (; k + STEP < a.K; k += 2 * STEP)
-      products(k, std::integral_constant<int, 2>{});
-    if (k < a.K) products(k, std::integral_constant<int, 1>{});
+    for (int i = 0; i < batches; ++i) {
+      products(turn * 2 * STEP + wid * 64, std::integral_constant<int, 2>{});
+      if (++turn == batches) turn = 0;
+    }
+    for (int k = batches * 2 * STEP + wid * 64; k < a.K; k += STEP)
+      products(k, std::integral_constant<int, 1>{});
 
     #pragma unroll
     for (int g = 0; g < 2; ++g) {

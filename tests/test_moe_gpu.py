@@ -122,6 +122,38 @@ def test_few_choices(tokens, experts, top, width, inner, kind, monkeypatch):
     assert (out - ref).abs().max() <= 2.0 ** -5 * ref.abs().max()
 
 
+@pytest.mark.parametrize("up", [True, False])
+@pytest.mark.parametrize("columns", [128, 1024, 1152, 2048, 2176, 4096, 6144])
+def test_few_choices_and_where_their_columns_begin(up, columns):
+    """Rows of multiples of 4 KB, whose workgroups begin at columns of their own, and
+    others.  A sum is rounded to bf16, half a step being at most 2^-8 of it; a choice
+    has the same bits alone."""
+    E, N, T = 3, 256, 21
+    g = torch.Generator().manual_seed(columns)
+    rand = lambda *s: torch.randn(*s, generator=g).to(DEV)
+    x = rand(T, columns).bfloat16()
+    w = (rand(E, (2 if up else 1) * N, columns) * columns ** -0.5).bfloat16()
+    ids = (torch.arange(T) ** 2 % E).int().to(DEV)[:, None].contiguous()
+    few = ops._native().experts_few
+    out = torch.empty(T, N, dtype=torch.bfloat16, device=DEV)
+    place = torch.empty_like(ids) if up else None
+    few(up, out, place, x, w, ids, 1)
+    for t in range(T):
+        e = int(ids[t])
+        want = w[e].double() @ x[t].double()
+        slack = (w[e].double().abs() @ x[t].double().abs()) * 2.0 ** -22
+        if up:
+            # |silu'| <= 1.1, |silu(g)| <= |g|; the exponential's error is 2^-20
+            (gate, v), (dg, dv) = want.chunk(2), slack.chunk(2)
+            want = torch.nn.functional.silu(gate) * v
+            slack = 1.1 * dg * v.abs() + gate.abs() * dv + 2.0 ** -20 * want.abs()
+        assert ((out[t].double() - want).abs()
+                <= 2.0 ** -8 * want.abs() + 1.01 * slack).all()
+    one = torch.empty(1, N, dtype=torch.bfloat16, device=DEV)
+    few(up, one, place[:1].clone() if up else None, x[20:], w, ids[20:].clone(), 1)
+    assert torch.equal(one[0], out[20])
+
+
 def test_choices_that_name_no_expert():
     """Without a sort: no place, and nothing of them in the sum; and no more
     experts than a load of their numbers has."""
