@@ -379,6 +379,19 @@ def _wave_of_rows(M: int, N: int, K: int):
     return (64, 64, 1) if mt * nt >= 144 and -(-nt // 8) * mt <= 32 else None
 
 
+def _wave_of_longer_rows(M: int, N: int, K: int):
+    """The same tiles for 65 to 128 rows and longer columns where they are at least 176,
+    before parts of K that a pass adds up.  70 random sizes, time over what was there:
+    K up to 6400 0.90 (94 rows of 6144 x 4096 23.9 -> 19.6 us, 128 26.4 22.7, 65 of 7168
+    x 4096 23.8 19.9, 77 of 8064 x 5120 29.9 24.8; 6144 x 5120 0.91 to 1.04, the worst
+    128 rows 27.8 28.8), beyond 1.14; fewer tiles 1.05 to 1.2.  Where the norm adds up
+    the parts those are faster (96 rows 17.4)."""
+    if not 64 < M <= 128 or K % 128 or N % 4 or not 2304 < K <= 6400:
+        return None
+    nt = -(-N // 64)
+    return (64, 64, 1) if 88 <= nt <= 128 else None
+
+
 @lru_cache(maxsize=1 << 14)
 def _route(M: int, N: int, K: int, parts: bool):
     """How x w^T of these sizes is formed: "rows", (rows, outputs of a tile, parts
@@ -386,7 +399,8 @@ def _route(M: int, N: int, K: int, parts: bool):
     step of small prompts, which is not captured, waits for the host."""
     if K >= 1 << 24:                # the kernels' chunks are counted in 32 bits
         return None
-    wave = _wave_gemm(M, N, K) or _waves_gemm(M, N, K)
+    wave = _wave_gemm(M, N, K) or _waves_gemm(M, N, K) \
+        or (None if parts else _wave_of_longer_rows(M, N, K))
     if wave is not None:
         return wave
     if _rows_gemm_sizes(M, N, K) and _native().gemm_rows_fits(M, K):

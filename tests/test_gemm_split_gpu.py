@@ -395,6 +395,30 @@ def test_wave_of_rows(M, N, K):
     _check(ops.linear(x, w), x, w)
 
 
+def test_rule_of_a_wave_of_longer_rows():
+    """65 to 128 rows: 176 to 256 tiles, without a norm that adds up parts."""
+    for M, N, K, rule in [
+            (65, 5632, 2432, (64, 64, 1)), (65, 5568, 4096, None),
+            (128, 8192, 6400, (64, 64, 1)), (128, 8196, 4096, None),
+            (96, 6144, 6528, None), (96, 6144, 2304, None),
+            (129, 6144, 4096, None), (64, 6144, 4096, None),
+            (96, 6144, 4160, None), (96, 6142, 4096, None)]:
+        assert ops._wave_of_longer_rows(M, N, K) == rule, (M, N, K)
+    assert ops._route(96, 6144, 4096, False) == (64, 64, 1)
+    assert ops._route(96, 6144, 4096, True) == ops._split_gemm(96, 6144, 4096)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(65, 5572, 2432), (96, 6144, 4096),
+                                   (128, 8188, 6400)])
+def test_wave_of_longer_rows(M, N, K):
+    g = torch.Generator().manual_seed(M)
+    x = torch.randn(M, K, generator=g).bfloat16().to(DEV)
+    w = torch.randn(N, K, generator=g).bfloat16().to(DEV)
+    assert ops._route(M, N, K, False) == (64, 64, 1)
+    _check(ops.linear(x, w), x, w)
+
+
 def test_rule_leaves_no_workgroup_for_a_second_wave():
     """Workgroups go to 8 dies of 32 units in turn, those of one tile of w to
     the same."""
