@@ -405,8 +405,9 @@ def _route(M: int, N: int, K: int, parts: bool):
         return wave
     if _rows_gemm_sizes(M, N, K) and _native().gemm_rows_fits(M, K):
         return "rows"
-    return _less_padding(M, _split_gemm(M, N, K)) \
-        or (_summed_gemm(M, N, K) if parts else None) or _wave_of_rows(M, N, K)
+    return _less_padding(M, N, K, _split_gemm(M, N, K)) \
+        or (_summed_gemm(M, N, K) or _few_parts(M, N, K) if parts else None) \
+        or _wave_of_rows(M, N, K)
 
 
 def _rows_gemm_sizes(M: int, N: int, K: int) -> bool:
@@ -507,10 +508,37 @@ def _split_gemm(M: int, N: int, K: int):
     return 128, 128, wide
 
 
-def _less_padding(M: int, split):
+def _less_padding(M: int, N: int, K: int, split):
     """Narrow tiles of 64 rows where those are enough: 17 rows of 2048 x 7168 8.2
-    -> 8.0 us, 32 of 4096 x 4096 9.2 -> 8.7, 64 9.9 -> 9.5; the same bits."""
-    return (64, 64, split[2]) if split and M <= 64 and split[1] == 64 else split
+    -> 8.0 us, 32 of 4096 x 4096 9.2 -> 8.7, 64 9.9 -> 9.5; the same bits.  In place of
+    tiles of 128 x 128, in parts of their own: 260 random sizes, 17 to 64 rows, N of 1088
+    to 6528 and K of 4352 to 28672, with the norm: 5 parts and more 0.80 of the time (48
+    of 3072 x 8192 19.8 -> 16.6 us, 33 of 2560 x 10240 19.9 16.6, 24 of 1344 x 19456 24
+    17; none slower), 4 0.95 (32 of 4096 x 11008 25.5 22.3, the worst 1.02) but with rows
+    of 16 KB (24 of 4096 x 8192 20.8 21.6), 3 0.95 up to 12288 columns (32 of 4608 x 8192
+    24.1 21.7, the worst 1.03) and 1.03 beyond, 2 1.06."""
+    if not split or M > 64 or split[0] != 128:
+        return split
+    if split[1] == 64:
+        return 64, 64, split[2]
+    narrow = min(8, 256 // -(-N // 64))
+    return (64, 64, narrow) if narrow >= 5 or narrow == 4 and K % 8192 \
+        or narrow == 3 and K <= 12288 else split
+
+
+def _few_parts(M: int, N: int, K: int):
+    """Two or three parts of one tile of up to 64 rows, where the norm adds them up and
+    no other rule has a kernel.  330 sizes, N of 4160 to 8192 and K of 4352 to 28672, with
+    the norm, over the library's time: 0.73 on average (1 row of 8192 x 28672 94 77 us,
+    12 of 7168 x 18432 113 47, 1 of 6656 x 17920 90 44, 64 of 6592 x 4736 28.5 22.4, 4 of
+    5120 x 5120 17.2 15.9; the worst, 5120 x 8192, even), but with rows of 16 KB in two
+    parts (8 of 8192 x 8192 33 36), and with 4096 columns and fewer (16 of 8192 x 4096 20
+    22.5)."""
+    if not 1 <= M <= 64 or K % 128 or N % 8 or not 0 < N <= 8192 \
+            or not 4096 < K <= 28672:
+        return None
+    split = 256 // -(-N // 64)
+    return (64, 64, split) if split == 3 or split == 2 and K != 8192 else None
 
 
 def _summed_gemm(M: int, N: int, K: int):

@@ -299,6 +299,44 @@ def test_rule_of_few_rows_of_long_columns():
                 assert -(-N // 64) * rule[2] <= 256 and 3 <= rule[2] <= K // 512
 
 
+def test_rule_of_few_parts_of_one_tile():
+    """Up to 64 rows: at most a workgroup a unit, none where rows are 16 KB apart."""
+    for M, N, K, few, narrow in [
+            (1, 8192, 28672, (64, 64, 2), None), (64, 8192, 4224, (64, 64, 2), None),
+            (64, 8192, 4096, None, None), (1, 8192, 8192, None, None),
+            (1, 8192, 28800, None, None), (65, 8192, 28672, None, None),
+            (8, 5440, 8192, (64, 64, 3), None), (8, 5448, 9216, (64, 64, 2), None),
+            (8, 4096, 9216, None, None), (8, 8196, 9216, None, None),
+            (33, 4096, 11008, None, (64, 64, 4)), (33, 4096, 8192, None, (128, 128, 8)),
+            (17, 1088, 16384, None, (64, 64, 8)), (64, 5120, 12288, (64, 64, 3),
+                                                   (64, 64, 3)),
+            (64, 5120, 12416, (64, 64, 3), (128, 128, 6)),
+            (17, 6144, 6144, (64, 64, 2), (128, 128, 5))]:
+        assert ops._few_parts(M, N, K) == few, (M, N, K)
+        assert ops._less_padding(M, N, K, ops._split_gemm(M, N, K)) == narrow
+        route = ops._route(M, N, K, True)
+        assert route == (narrow or few or route), (M, N, K)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [
+    (1, 8192, 4224), (64, 6592, 9216), (7, 4168, 4352), (33, 4096, 11008),
+    (17, 1088, 16384), (64, 5120, 6272), (40, 3080, 8192)])
+def test_parts_of_one_tile_of_rows(M, N, K):
+    """Workgroups of a tile of w begin at a column of its own in each part."""
+    g = torch.Generator().manual_seed(M)
+    x = torch.randn(M, K, generator=g).bfloat16().to(DEV)
+    w = torch.randn(N, K, generator=g).bfloat16().to(DEV)
+    bm, bn, parts = ops._route(M, N, K, True)
+    assert bm == bn == 64 and -(-N // 64) * parts <= 256
+    got = ops.linear_parts(x, w)
+    assert got.data.shape == (parts, M, N)
+    _check(got.data.sum(0), x, w)
+    one = ops.linear_parts(x[M - 1:], w)
+    if one.__class__ is got.__class__ and one.data.shape[0] == parts:
+        assert torch.equal(one.data[:, 0], got.data[:, M - 1])
+
+
 def test_rule_of_several_waves():
     """Half a wave and more, and several; not nearly empty ones."""
     for M, N, K, rule in [
