@@ -95,15 +95,18 @@ void gemm_split_kernel(Split a) {
   // workgroups begin at different columns, so that not all of them ask the same
   // channels of memory at once: 64 rows of 28672 x 4096 46 -> 42 us; those of one part
   // of K, 1 row of 8192 x 28672 in 2 parts 91 -> 75, of 5120 x 8192 in 3 19.6 -> 18.2,
-  // 32 rows 19.6 18.2, 32 of 4096 x 11008 in 4 19.9 -> 18.5, e4m3 12.4 -> 11.7; 4096 x
-  // 14336 and 4096 x 4096 in 4 are even.  Those of one tile of w begin at the same,
-  // which costs up to 3 % in places (192 rows of 14336 x 2048 gated 23.1 -> 23.7, 96 of
-  // 28672 x 4096 49.2 49.0), so that a row's sums do not depend on its place among the
-  // rows.  Not those that wait for x: 256 decoded tokens, where 6144 x 4096 takes this
-  // kernel, 3245 us, with it 3251; 512 rows of 5120 x 8192 in 3 parts of 256 x 128 tiles
-  // 49 67
-  const int turn = BM == 64 || GATED
-      ? (a.splits == 1 ? at / a.mt * a.mt : u / a.splits) % chunks : 0;
+  // 32 rows 19.6 18.2, 32 of 4096 x 11008 in 4 19.9 -> 18.5, e4m3 12.4 -> 11.7, e4m3 1
+  // of 5120 x 12288 in 3 16.1 -> 14.3; other rows of 8192 columns and more within 2 %
+  // (4096 x 14336, 5120 x 13824, 7168 x 18432), and shorter ones too (64 rows of 2048 x
+  // 7168 in 8 9.3 9.3, 1 of 5120 x 5120 in 3 11.2 11.5), which begin together.  Those of
+  // one tile of w begin at the same, which costs up to 3 % in places (192 rows of 14336 x
+  // 2048 gated 23.1 -> 23.7, 96 of 28672 x 4096 49.2 49.0), so that a row's sums do not
+  // depend on its place among the rows.  Not those that wait for x: 256 decoded tokens,
+  // where 6144 x 4096 takes this kernel, 3245 us, with it 3251; 512 rows of 5120 x 8192 in
+  // 3 parts of 256 x 128 tiles 49 67
+  const int turn = !(BM == 64 || GATED) ? 0
+      : a.splits == 1 ? at / a.mt * a.mt % chunks
+      : a.K >= 8192 ? u / a.splits % chunks : 0;
   // load i of a stage: first those of x, then those of w
   auto stage = [&](int slot, int d, int i) {
     d += turn;

@@ -307,6 +307,8 @@ def test_rule_of_few_parts_of_one_tile():
             (1, 8192, 28800, None, None), (65, 8192, 28672, None, None),
             (8, 5440, 8192, (64, 64, 3), None), (8, 5448, 9216, (64, 64, 2), None),
             (8, 4096, 9216, None, None), (8, 8196, 9216, None, None),
+            (1, 5120, 5120, None, None), (2, 5120, 5120, (64, 64, 3), None),
+            (1, 5120, 5248, (64, 64, 3), None),
             (33, 4096, 11008, None, (64, 64, 4)), (33, 4096, 8192, None, (128, 128, 8)),
             (17, 1088, 16384, None, (64, 64, 8)), (64, 5120, 12288, (64, 64, 3),
                                                    (64, 64, 3)),
