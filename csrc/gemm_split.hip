@@ -14,7 +14,9 @@
 // ring of 5 stages, or of chunks twice as long, takes as long, and waves that divide
 // a stage's chunks up to 5 % longer.
 //
-// us, library and here, x and w from memory:
+// us, library and here, x and w from memory; more than 256 rows with an activation or
+// in parts, and from 129 on with long columns, are csrc/gemm_wide.hip's where its rules
+// take them (4096 x 14336 256 rows 45, 512 66):
 //   4096 x 14336  32 rows 33 26, 96 68 38, 192 112 46, 256 66 52, 512 98 70
 //   6144 x 4096   96 rows 24 23, 192 35 28, 256 44 29
 //   4096 x 4096   32 rows 14 11, 96 23 16, 192 34 21, 256 23 23
