@@ -1297,10 +1297,13 @@ __global__ __launch_bounds__(NT) void sample_slices_kernel(
   if (tid == 0) out[b] = drawn;
 }
 
-// Slices of a row, 0: none (or no rows).  As many as give every compute unit a workgroup, if
-// each has a load for every thread.  Beyond two workgroups a unit the chip is
-// full of whole rows (256 rows of 128256 52 us, in 4 slices 57; of 50257 50 and
-// in 2 slices 50; of 32000 31 and in one 28).
+// Slices of a row, 0: none (or no rows).  As many as give every compute unit a
+// workgroup, if each has a load for every thread.  Beyond two workgroups a unit the
+// chip is full of whole rows.  A mix of options would gain in slices there (us, 256
+// rows of 128256 43, in 4 slices 39, 384 of 50257 in 2 83 59), but rows that are all
+// greedy (13 and 20) and shares of thousands of values (132 and 147) lose, and weights
+// relative to a slice's largest value are other last bits, which decide a draw now
+// and then.
 int sample_slices(long rows, int vocab) {
   const int least = (vocab + HELD * NT * 8 - 1) / (HELD * NT * 8);
   const int most = min(SLICES, max(1, vocab / (NT * 8)));

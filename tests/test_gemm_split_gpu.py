@@ -334,6 +334,8 @@ def test_parts_of_one_tile_of_rows(M, N, K):
     got = ops.linear_parts(x, w)
     assert got.data.shape == (parts, M, N)
     _check(got.data.sum(0), x, w)
+    apart = [torch.nn.functional.pad(t, (0, 8))[:, :K] for t in (x, w)]
+    assert torch.equal(ops.linear_parts(*apart).data, got.data)
     one = ops.linear_parts(x[M - 1:], w)
     if one.__class__ is got.__class__ and one.data.shape[0] == parts:
         assert torch.equal(one.data[:, 0], got.data[:, M - 1])
@@ -457,6 +459,8 @@ def test_wave_of_longer_rows(M, N, K):
     w = torch.randn(N, K, generator=g).bfloat16().to(DEV)
     assert ops._route(M, N, K, False) == (64, 64, 1)
     _check(ops.linear(x, w), x, w)
+    apart = [torch.nn.functional.pad(t, (0, 8))[:, :K] for t in (x, w)]
+    assert torch.equal(ops.linear(*apart), ops.linear(x, w))
 
 
 def test_rule_leaves_no_workgroup_for_a_second_wave():
