@@ -43,6 +43,7 @@ struct Split {
   int M, N, K;
   long xs, ws;                 // row strides
   int mt, nt, splits;          // tiles of rows, of outputs, parts of K
+  bool apart;                  // workgroups of a part begin at columns of their own
 };
 
 // BM rows of x, BN of w; WM * WN waves have BM / WM by BN / WN.  A stage has
@@ -95,20 +96,16 @@ void gemm_split_kernel(Split a) {
     w_off[j] = (unsigned)(n * a.ws * ELEM) + ((lane & 7) ^ (r >> 1 & 7)) * 16;
   }
   // workgroups begin at different columns, so that not all of them ask the same
-  // channels of memory at once: 64 rows of 28672 x 4096 46 -> 42 us; those of one part
-  // of K, 1 row of 8192 x 28672 in 2 parts 91 -> 75, of 5120 x 8192 in 3 19.6 -> 18.2,
-  // 32 rows 19.6 18.2, 32 of 4096 x 11008 in 4 19.9 -> 18.5, e4m3 12.4 -> 11.7, e4m3 1
-  // of 5120 x 12288 in 3 16.1 -> 14.3; other rows of 8192 columns and more within 2 %
-  // (4096 x 14336, 5120 x 13824, 7168 x 18432), and shorter ones too (64 rows of 2048 x
-  // 7168 in 8 9.3 9.3, 1 of 5120 x 5120 in 3 11.2 11.5), which begin together.  Those of
-  // one tile of w begin at the same, which costs up to 3 % in places (192 rows of 14336 x
-  // 2048 gated 23.1 -> 23.7, 96 of 28672 x 4096 49.2 49.0), so that a row's sums do not
-  // depend on its place among the rows.  Not those that wait for x: 256 decoded tokens,
-  // where 6144 x 4096 takes this kernel, 3245 us, with it 3251; 512 rows of 5120 x 8192 in
-  // 3 parts of 256 x 128 tiles 49 67
+  // channels of memory at once: 64 rows of 28672 x 4096 46 -> 42 us; those of parts of
+  // K only where that matters (few_channels, below).  Those of one tile of w begin at
+  // the same, which costs up to 3 % in places (192 rows of 14336 x 2048 gated 23.1 ->
+  // 23.7, 96 of 28672 x 4096 49.2 49.0), so that a row's sums do not depend on its place
+  // among the rows.  Not those that wait for x: 256 decoded tokens, where 6144 x 4096
+  // takes this kernel, 3245 us, with it 3251; 512 rows of 5120 x 8192 in 3 parts of 256 x
+  // 128 tiles 49 67
   const int turn = !(BM == 64 || GATED) ? 0
       : a.splits == 1 ? at / a.mt * a.mt % chunks
-      : a.K >= 8192 ? u / a.splits % chunks : 0;
+      : a.apart ? u / a.splits % chunks : 0;
   // load i of a stage: first those of x, then those of w
   auto stage = [&](int slot, int d, int i) {
     d += turn;
@@ -192,6 +189,26 @@ __global__ __launch_bounds__(256) void gemm_sum_kernel(
       uint2{cvt_pk_bf16(x[0][0], x[0][1]), cvt_pk_bf16(x[0][2], x[0][3])};
 }
 
+// Whether the workgroups of a product in parts, if they begin together, ask few
+// channels of memory: 256 bytes are one channel's, and 32 KB go through all 128.  Rows a
+// multiple of 4 KB apart begin on 8 channels or fewer, and every part on others, unless
+// they begin a multiple of 4 KB apart too.  1 and 32 rows of w in tiles of 64 x 64, 500
+// sizes in 2 to 8 parts, K of 4096 to 28672, time with columns of their own over that
+// without: 2 to 4 channels 0.78 (8192 x 16384 70 -> 46 us, 4096 x 14336 in rows of 32 KB
+// 38.7 -> 21.9, 5120 x 16384 37 -> 30), 6 0.95 (5120 x 8192 18.2 16.7), 8 0.86 (8192 x
+// 28672 90 -> 70, 8192 x 12288 43 -> 34, 5120 x 6144 14.9 12.9, e4m3 5120 x 12288 16.2
+// 14.3), 12 of rows of 16 KB 0.9 (2560 x 8192), of others 1.0, 16 and more 1.0 (4096 x
+// 14336 21.3 21.7).  Where rows lie no multiple of 4 KB apart the mean of 270 is 1.0 too,
+// and single sizes are 10 % faster or slower (8192 x 22016 72 -> 66, 8192 x 16128 1.13).
+bool few_channels(long row_bytes, long stretches, int splits) {
+  const long period = row_bytes % 32768 ? row_bytes & -row_bytes : 32768;
+  if (period < 4096 || period >= 16384) return period >= 16384;
+  unsigned begins = 0;         // of the stretches of a period
+  for (long z = 0; z < splits; ++z)
+    begins |= 1u << stretches * z / splits % (period / 256);
+  return 32768 / period * __builtin_popcount(begins) <= 8;
+}
+
 }  // namespace
 
 // Tiles of bm rows of x by bn of w: 64 x 64, 64 x 128, 128 x 64, 128 x 128, 256 x
@@ -213,7 +230,9 @@ void launch_gemm_split(bf16* out, float* part, const void* x, const void* w,
   // 480 77.5 77; 256 a tile, 320 55.6 55.8, 512 62.5 59.5.
   const int last = (M - 1) % bm + 1;
   const bool once = M <= bm || last * 4 >= bm * 3;
-  Split a{out, part, x, w, x_scale, w_scale, M, N, K, xs, ws, 0, 0, splits};
+  const int size = x_scale ? 1 : 2;
+  Split a{out, part, x, w, x_scale, w_scale, M, N, K, xs, ws, 0, 0, splits,
+          few_channels(ws * size, (long)K * size / 256, splits)};
   #define WITH(BM, BN, WM, WN, STAGES, KC, FP8, GATED, AUX)                 \
     {                                                                       \
       constexpr int BYTES = STAGES * KC * (BM + BN) * 128;                  \

@@ -334,8 +334,10 @@ def test_parts_of_one_tile_of_rows(M, N, K):
     got = ops.linear_parts(x, w)
     assert got.data.shape == (parts, M, N)
     _check(got.data.sum(0), x, w)
-    apart = [torch.nn.functional.pad(t, (0, 8))[:, :K] for t in (x, w)]
-    assert torch.equal(ops.linear_parts(*apart).data, got.data)
+    # where it begins depends on how far the rows of w lie apart, but for 32 KB more
+    pad = lambda t, n: torch.nn.functional.pad(t, (0, n))[:, :K]
+    assert torch.equal(ops.linear_parts(pad(x, 8), pad(w, 16384)).data, got.data)
+    _check(ops.linear_parts(pad(x, 8), pad(w, 8)).data.sum(0), x, w)
     one = ops.linear_parts(x[M - 1:], w)
     if one.__class__ is got.__class__ and one.data.shape[0] == parts:
         assert torch.equal(one.data[:, 0], got.data[:, M - 1])
@@ -509,3 +511,42 @@ def test_products_of_no_columns(M, N):
     assert torch.equal(ops.linear(x, w), x @ w.t())
     assert torch.equal(ops.linear_parts(x, w), x @ w.t())
     assert torch.equal(ops.gated_linear(x, w), ops.silu_mul(x @ w.t()))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,K,pad,parts,fp8,apart", [
+    (4096, 14336, 0, 4, False, False), (4096, 14336, 2048, 4, False, True),
+    (4096, 14336, 0, 4, True, False), (5120, 8192, 0, 3, False, True),
+    (5120, 8192, 64, 3, False, False), (5120, 6144, 0, 3, False, True),
+    (5120, 6144, 64, 3, False, False), (5120, 12288, 0, 3, True, True),
+    (2560, 9472, 0, 6, True, False), (8192, 12288, 0, 2, False, True),
+    (8192, 14336, 0, 2, False, False), (4096, 12288, 0, 4, False, False)])
+def test_where_parts_begin(N, K, pad, parts, fp8, apart):
+    """Tiles of w begin at columns of their own where rows and parts would begin on few
+    channels of memory, by what lies between rows; elsewhere at the same, so that their
+    sums do not depend on where among the outputs they are."""
+    g = torch.Generator().manual_seed(K)
+    x = torch.randn(5, K, generator=g)
+    w = torch.randn(N, K + pad, generator=g)
+    scales = ()
+    if fp8:
+        x, w = x.to(torch.float8_e4m3fn), w.to(torch.float8_e4m3fn)
+        scales = torch.ones(5, device=DEV), torch.ones(N, device=DEV)
+    else:
+        x, w = x.bfloat16(), w.bfloat16()
+    x, w = x.to(DEV), w.to(DEV)
+
+    def product(w):
+        part = torch.full((parts, 5, N), float("nan"), device=DEV)
+        ops._native().gemm_split(None, x, w[:, :K], part, 64, 64, parts, *scales)
+        return part
+
+    got = product(w)
+    other = product(w.view(torch.uint8).roll(64, 0).view(w.dtype))
+    same = torch.equal(other.roll(-64, 2), got)
+    assert same or apart
+    if not fp8:                 # whose sums are exact here in any order
+        assert same != apart
+        _check(got.sum(0), x, w[:, :K])
+    ref = x.double() @ w[:, :K].double().t()
+    assert (got.sum(0).double() - ref).norm() <= 2.0 ** -14 * ref.norm()
