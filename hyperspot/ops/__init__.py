@@ -632,17 +632,18 @@ def _wide_gated(M: int, N: int, K: int):
 @lru_cache(maxsize=1 << 14)
 def _wide_parts(M: int, N: int, K: int):
     """(high, bn, parts) where csrc/gemm_wide.hip and the norm that adds up its parts
-    are faster than what was there and the norm.  760 random sizes from 257 to 3000
-    rows, time over that: 10240 columns and more, up to 1400 rows 0.79 (262 rows of
-    4096 x 14336 58 48 us, 600 112 76, 1000 137 110, 1268 161 132; worst 998 of 2720 x
-    16384 at 0.83, but 1.09 for tiles that fill no wave); from 4608 on 513 to 1024 rows
-    0.90 (worst 973 of 3216 x 4864 42 45); up to 2560, 513 to 1024 rows and up to 4096
-    outputs 0.87 (600 of 2048 x 2048 25 23).  Between, 0.98 to 1.07; more rows 1.0.
-    129 to 256 rows in 380 other sizes of 10240 columns and more, one tile of rows and
-    more than 192 in all, 0.89 (135 rows of 4096 x 14336 44 36 us, 248 53 45); decode
-    steps of 140, 200 and 256 rows, 8 layers, 1 % less.  Fewer rows are as fast in the
-    step (100 1730 1738), fewer tiles slower (200 of 2048 x 7168 17 21)."""
-    if K % 64 or N % 8 or not 1024 <= N <= 8192 or not 1024 <= K <= 20480 \
+    are faster than what was there and the norm.  Random sizes, x and w from memory,
+    time over that: 10240 columns and more, up to 1400 rows 0.69 in 97 (262 rows of
+    4096 x 14336 58 48 us, 600 112 76, 1000 137 110, 1268 161 132; the worst 1154 of 6336
+    x 15360 even), but 1.09 for tiles that fill no wave; from 4608 on 513 to 1024 rows
+    0.90 in 57 (the worst 989 of 8032 x 4992 89 92).  Shorter ones are slower (up to 2560
+    columns and 4096 outputs, 513 to 1024 rows, 1.14 in 93, 630 of 1768 x 2048 17.6 21.1), and
+    so are more rows (1.0).
+    129 to 256 rows of 10240 columns and more, one tile of rows and more than 192 in all,
+    0.65 (135 rows of 4096 x 14336 44 36 us, 248 53 45); decode steps of 140, 200 and 256
+    rows, 8 layers, 1 % less.  Fewer rows are as fast in the step (100 1730 1738), fewer
+    tiles slower (200 of 2048 x 7168 17 21)."""
+    if K % 64 or N % 8 or not 1024 <= N <= 8192 or not 4608 <= K <= 20480 \
             or not 128 < M <= (1400 if K >= 10240 else 1024):
         return None
     _, high, bn, split, tiles = _wide_tile(M, N, K, (1, 2, 3, 4, 5, 6, 7, 8))
@@ -651,7 +652,7 @@ def _wide_parts(M: int, N: int, K: int):
     elif M <= 512:
         fits = 176 <= tiles <= 256 and K >= 10240 and N >= 1536
     else:
-        fits = K <= 2560 and N <= 4096 or K >= 4608 and 176 <= tiles <= 256
+        fits = 176 <= tiles <= 256
     return (high, bn, split) if fits else None
 
 

@@ -85,8 +85,7 @@ def test_numbers_that_are_not_finite():
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K", [
     (257, 4096, 14336), (600, 4096, 10240), (513, 2048, 7168),
-    (1024, 2048, 2048), (1400, 4096, 10240), (129, 4096, 14336),
-    (256, 4096, 10240)])
+    (1400, 4096, 10240), (129, 4096, 14336), (256, 4096, 10240)])
 def test_parts_and_norm(M, N, K):
     assert ops._wide_parts(M, N, K) and not ops._wide_parts(128, N, K)
     x, w = _inputs(M, N, K)
@@ -136,6 +135,17 @@ def test_refused():
                  (out[:, :128], x, w, None, 8, 128)):
         with pytest.raises(RuntimeError):
             wide(*args)
+
+
+def test_rule_of_parts():
+    """From 4608 columns on, up to 512 rows from 10240 on, in a nearly full wave."""
+    for M, N, K, taken in [
+            (600, 2048, 2048, False), (1024, 4096, 2560, False), (513, 2048, 4544, False),
+            (600, 4096, 4608, True), (1025, 4096, 4608, False), (1024, 4096, 9216, True),
+            (512, 4096, 9216, False), (512, 4096, 10240, True), (1400, 4096, 10240, True),
+            (1401, 4096, 10240, False), (129, 4096, 14336, True),
+            (128, 4096, 14336, False)]:
+        assert bool(ops._wide_parts(M, N, K)) == taken, (M, N, K)
 
 
 def test_rules_cover_all_rows():
