@@ -635,7 +635,8 @@ def _wide_parts(M: int, N: int, K: int):
     are faster than what was there and the norm.  Random sizes, x and w from memory,
     time over that: 10240 columns and more, up to 1400 rows 0.69 in 97 (262 rows of
     4096 x 14336 58 48 us, 600 112 76, 1000 137 110, 1268 161 132; the worst 1154 of 6336
-    x 15360 even), but 1.09 for tiles that fill no wave; from 4608 on 513 to 1024 rows
+    x 15360 even), but 1.09 for tiles that fill no wave and 1.10 in 45 for one part of
+    tiles of 256 outputs, which are 180 to 217 (1114 of 8144 x 12928 231 252); from 4608 on 513 to 1024 rows
     0.90 in 57 (the worst 989 of 8032 x 4992 89 92).  Shorter ones are slower (up to 2560
     columns and 4096 outputs, 513 to 1024 rows, 1.14 in 93, 630 of 1768 x 2048 17.6 21.1), and
     so are more rows (1.0).
@@ -652,7 +653,7 @@ def _wide_parts(M: int, N: int, K: int):
     elif M <= 512:
         fits = 176 <= tiles <= 256 and K >= 10240 and N >= 1536
     else:
-        fits = 176 <= tiles <= 256
+        fits = 176 <= tiles <= 256 and (split > 1 or bn == 128)
     return (high, bn, split) if fits else None
 
 

@@ -138,13 +138,15 @@ def test_refused():
 
 
 def test_rule_of_parts():
-    """From 4608 columns on, up to 512 rows from 10240 on, in a nearly full wave."""
+    """From 4608 columns on, up to 512 rows from 10240 on, in a nearly full wave;
+    not in one part of tiles of 256 outputs."""
     for M, N, K, taken in [
             (600, 2048, 2048, False), (1024, 4096, 2560, False), (513, 2048, 4544, False),
             (600, 4096, 4608, True), (1025, 4096, 4608, False), (1024, 4096, 9216, True),
             (512, 4096, 9216, False), (512, 4096, 10240, True), (1400, 4096, 10240, True),
             (1401, 4096, 10240, False), (129, 4096, 14336, True),
-            (128, 4096, 14336, False)]:
+            (128, 4096, 14336, False), (1114, 8144, 12928, False),
+            (1028, 7992, 18624, False), (785, 6464, 18048, True)]:
         assert bool(ops._wide_parts(M, N, K)) == taken, (M, N, K)
 
 
