@@ -615,15 +615,17 @@ def _wide_tile(M: int, N: int, K: int, parts=(1,)):
 @lru_cache(maxsize=1 << 14)
 def _wide_gated(M: int, N: int, K: int):
     """(high, bn) where csrc/gemm_wide.hip forms silu(gate) * up of more than 256
-    rows faster than what was there, mostly the library's product and a pass.  2000
-    random sizes from 257 to 8192 rows, N of 6000 to 36000 and K of 1024 to 8192, time
-    over that: up to 1200 rows at 0.7 PFLOP/s and more by the tiles' times 0.88, 2 of
-    100 more than 3 % slower (512 of 28672 x 4096 112 104 us, 880 203 176; 512 of 14336
-    x 2048 32 30); more of up to 3072 columns 0.85, 6 of 100 (2600 of 14336 x 2048 183
-    146).  More of longer columns 0.95, but every fourth slower, by up to 10 % (8192
-    of 28672 x 4096 1335 1400): those are the library's."""
-    if not 256 < M < 1 << 20 or not 1024 <= K <= 8192 or K % 64 or N % 16 \
-            or not 6000 <= N < 1 << 17 or M > 1200 and K > 3072:
+    rows faster than what was there, mostly the library's product and a pass.  Random
+    sizes, N of 6000 to 36000, at 0.7 PFLOP/s and more by the tiles' times, time over
+    that: up to 1200 rows 0.88 in 186 (512 of 28672 x 4096 115 115 us, 880 203 176, 512
+    of 14336 x 2048 38 37), 8 of them more than 3 % slower, up to 8 %, and 769 and more
+    of them of over 5376 columns 0.93 in 74, but 19 slower, up to 14 % (1192 of 16384 x
+    5888 210 239): those are the library's.  More rows of up to 3072 columns 0.86 in 20
+    (2600 of 14336 x 2048 183 146), of longer ones 0.95, but every fourth slower, by up
+    to 10 % (8192 of 28672 x 4096 1335 1400): those are the library's too."""
+    if not 256 < M < 1 << 20 or K < 1024 or K % 64 or N % 16 \
+            or not 6000 <= N < 1 << 17 \
+            or K > (8192 if M <= 768 else 5376 if M <= 1200 else 3072):
         return None
     us, high, bn, _, _ = _wide_tile(M, N, K)
     return (high, bn) if 2e-9 * M * N * K / us >= 0.7 else None

@@ -150,6 +150,18 @@ def test_rule_of_parts():
         assert bool(ops._wide_parts(M, N, K)) == taken, (M, N, K)
 
 
+def test_rule_of_gated_tiles():
+    """The more rows, the shorter the columns."""
+    for M, N, K, taken in [
+            (257, 28672, 8192, True), (768, 28672, 8192, True),
+            (769, 28672, 5440, False), (769, 28672, 5376, True),
+            (1192, 16384, 5888, False), (901, 29712, 8064, False),
+            (1200, 28672, 5376, True), (1201, 28672, 3136, False),
+            (1201, 28672, 3072, True), (512, 28672, 4096, True),
+            (512, 28672, 8256, False)]:
+        assert bool(ops._wide_gated(M, N, K)) == taken, (M, N, K)
+
+
 def test_rules_cover_all_rows():
     """Every size that a rule takes has tiles that the kernel has, enough of them
     for all rows and outputs, and parts with columns."""
