@@ -661,17 +661,21 @@ def _wide_parts(M: int, N: int, K: int):
 
 @lru_cache(maxsize=1 << 14)
 def _wide_long(M: int, N: int, K: int):
-    """(high, bn, 1) for long columns where 256 x 256 tiles are several waves of which
-    the last is neither nearly empty nor full.  The library has tiles of 0.7 to 1.0
-    PFLOP/s for half of these sizes and of 1.3 to 1.5 for the others, 1.03 on average
-    over 70 of N from 3584 to 8192 and K from 11008 to 28672; here 1.2 to 1.4 (7411
-    rows of 4096 x 14336 971 640 us, 5888 of 5120 x 13824 958 600; worst 7680 of 4096 x
-    11008 441 508).  With up to 10240 columns it has 1.3 to 1.55."""
-    if not 1024 < M < 1 << 20 or not 10240 <= K <= 1 << 15 or K % 64 or N % 8 \
+    """(high, bn, 1) for long columns where 256 x 256 tiles are two or three waves of
+    which the last is neither nearly empty nor full.  The library has two kinds of
+    tiles, of 0.65 to 1.1 PFLOP/s and of 1.2 to 1.5; here it is 1.1 to 1.35.  N from 2048
+    to 8192, K from 10240 to 32768, time over the library's: two waves 0.73 in 85 (7411
+    rows of 4096 x 14336 971 640 us, 5888 of 5120 x 13824 958 600), four of them more
+    than 3 % slower, by up to 15 % (7425 of 4096 x 11008), three 0.87 in 81, three
+    slower, by up to 12 % (5889 of 7168 x 18432), but multiples of 64 tiles, for which
+    it mostly has the better ones, 1.04 in two waves; more waves 1.0 in 20, every second
+    one slower.  With up to 10240 columns it has 1.3 to 1.55."""
+    if not 1024 < M <= 16384 or not 10240 <= K <= 1 << 15 or K % 64 or N % 8 \
             or not 2048 <= N <= 8192:
         return None
     tiles = -(-M // 256) * -(-N // 256)
-    if tiles <= 256 or not 0.8 <= _full(tiles) < 0.96:
+    if not 256 < tiles <= 768 or tiles % 64 == 0 \
+            or not 0.8 <= _full(tiles) < 0.96:
         return None
     _, high, bn, _, _ = _wide_tile(M, N, K)
     return high, bn, 1

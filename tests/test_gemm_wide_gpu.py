@@ -162,6 +162,21 @@ def test_rule_of_gated_tiles():
         assert bool(ops._wide_gated(M, N, K)) == taken, (M, N, K)
 
 
+def test_rule_of_long_columns():
+    """Two or three waves of 256 x 256 tiles, but not multiples of 64 of them."""
+    for M, N, K, tiles, taken in [
+            (6657, 4096, 11008, 27 * 16, True), (7041, 4096, 11008, 28 * 16, False),
+            (7411, 4096, 14336, 29 * 16, True), (7680, 4096, 11008, 30 * 16, True),
+            (7681, 4096, 11008, 31 * 16, False), (4353, 4096, 11008, 18 * 16, False),
+            (6657, 6144, 16384, 27 * 24, True), (8960, 5120, 13824, 35 * 20, True),
+            (8960, 4096, 13824, 35 * 16, False), (8193, 5120, 13824, 33 * 20, True),
+            (7984, 7584, 18688, 32 * 30, False), (7489, 7256, 21120, 30 * 29, False),
+            (16384, 2816, 14336, 64 * 11, False), (16380, 2560, 14336, 64 * 10, False),
+            (16128, 2560, 14336, 63 * 10, True), (16385, 2560, 14336, 65 * 10, False)]:
+        assert -(-M // 256) * -(-N // 256) == tiles
+        assert bool(ops._wide_long(M, N, K)) == taken, (M, N, K)
+
+
 def test_rules_cover_all_rows():
     """Every size that a rule takes has tiles that the kernel has, enough of them
     for all rows and outputs, and parts with columns."""
