@@ -381,12 +381,14 @@ def _wave_of_rows(M: int, N: int, K: int):
 
 def _wave_of_longer_rows(M: int, N: int, K: int):
     """The same tiles for 65 to 128 rows and longer columns where they are at least 176,
-    before parts of K that a pass adds up.  70 random sizes, time over what was there:
-    K up to 6400 0.90 (94 rows of 6144 x 4096 23.9 -> 19.6 us, 128 26.4 22.7, 65 of 7168
-    x 4096 23.8 19.9, 77 of 8064 x 5120 29.9 24.8; 6144 x 5120 0.91 to 1.04, the worst
-    128 rows 27.8 28.8), beyond 1.14; fewer tiles 1.05 to 1.2.  Where the norm adds up
-    the parts those are faster (96 rows 17.4)."""
-    if not 64 < M <= 128 or K % 128 or N % 4 or not 2304 < K <= 6400:
+    before parts of K that a pass adds up.  Random sizes, time over what was there: K up
+    to 4608 0.92 in 158 (96 rows of 6144 x 4096 21.8 -> 20.0 us, 128 23.8 23.2, 66 of
+    7168 x 4096 24.6 20.2), one more than 3 % slower, but of 97 to 128 rows up to 3712 columns 1.03 in 62,
+    up to 1.32 (125 of 6032 x 2560 13.7 17.0); up to 5632 0.97, every seventh slower, up
+    to 1.11 (128 of 6144 x 5120 27.4 28.8), beyond 1.06; fewer tiles 1.05 to 1.2.  Where
+    the norm adds up the parts those are faster (96 rows 17.4)."""
+    if not 64 < M <= 128 or K % 128 or N % 4 \
+            or not (2304 if M <= 96 else 3712) < K <= 4608:
         return None
     nt = -(-N // 64)
     return (64, 64, 1) if 88 <= nt <= 128 else None

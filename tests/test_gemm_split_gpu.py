@@ -443,8 +443,10 @@ def test_rule_of_a_wave_of_longer_rows():
     """65 to 128 rows: 176 to 256 tiles, without a norm that adds up parts."""
     for M, N, K, rule in [
             (65, 5632, 2432, (64, 64, 1)), (65, 5568, 4096, None),
-            (128, 8192, 6400, (64, 64, 1)), (128, 8196, 4096, None),
-            (96, 6144, 6528, None), (96, 6144, 2304, None),
+            (128, 8192, 4608, (64, 64, 1)), (128, 8196, 4096, None),
+            (96, 6144, 4736, None), (96, 6144, 2304, None),
+            (97, 6144, 3712, None), (125, 6032, 2560, None),
+            (97, 6144, 3840, (64, 64, 1)), (128, 6144, 5120, None),
             (129, 6144, 4096, None), (64, 6144, 4096, None),
             (96, 6144, 4160, None), (96, 6142, 4096, None)]:
         assert ops._wave_of_longer_rows(M, N, K) == rule, (M, N, K)
@@ -454,7 +456,7 @@ def test_rule_of_a_wave_of_longer_rows():
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K", [(65, 5572, 2432), (96, 6144, 4096),
-                                   (128, 8188, 6400)])
+                                   (128, 8188, 4608)])
 def test_wave_of_longer_rows(M, N, K):
     g = torch.Generator().manual_seed(M)
     x = torch.randn(M, K, generator=g).bfloat16().to(DEV)
