@@ -513,37 +513,39 @@ def _split_gemm(M: int, N: int, K: int):
 def _less_padding(M: int, N: int, K: int, split):
     """Narrow tiles of 64 rows where those are enough: 17 rows of 2048 x 7168 8.2
     -> 8.0 us, 32 of 4096 x 4096 9.2 -> 8.7, 64 9.9 -> 9.5; the same bits.  In place of
-    tiles of 128 x 128, in parts of their own: 260 random sizes, 17 to 64 rows, N of 1088
-    to 6528 and K of 4352 to 28672, with the norm: 5 parts and more 0.80 of the time (48
-    of 3072 x 8192 19.8 -> 16.6 us, 33 of 2560 x 10240 19.9 16.6, 24 of 1344 x 19456 24
-    17; none slower), 4 0.95 (32 of 4096 x 11008 25.5 22.3, the worst 1.02) but with rows
-    of 16 KB (24 of 4096 x 8192 20.8 21.6), 3 0.95 up to 12288 columns (32 of 4608 x 8192
-    24.1 21.7, the worst 1.03) and 1.03 beyond, 2 1.06."""
+    tiles of 128 x 128, in parts of their own, N of 1088 to 5440 and K of 4352 to 28672,
+    with the norm or without: 5 parts and more 0.80 of the time (48 of 3072 x 8192 19.8
+    -> 16.6 us, 33 of 2560 x 10240 19.9 16.6, 24 of 1344 x 19456 24 17; none slower).  4
+    up to 18432 columns, or 12288 of more than 48 rows, 0.94 in 83 (40 of 4096 x 16384
+    45 30, 24 of 4096 x 8192 21.0 20.0), beyond 1.0 in 78, up to 1.24; 3 up to 12288, or
+    8192, 0.97 in 39 (32 of 4608 x 8192 24.1 21.7), beyond 1.04 in 166, up to 1.29; 2
+    1.06.  2 of the 122 that are taken are more than 3 % slower."""
     if not split or M > 64 or split[0] != 128:
         return split
     if split[1] == 64:
         return 64, 64, split[2]
     narrow = min(8, 256 // -(-N // 64))
-    return (64, 64, narrow) if narrow >= 5 or narrow == 4 and K % 8192 \
-        or narrow == 3 and K <= 12288 else split
+    most = (8192, 12288) if M > 48 else (12288, 18432)
+    return (64, 64, narrow) if narrow >= 5 \
+        or narrow >= 3 and K <= most[narrow - 3] else split
 
 
 def _few_parts(M: int, N: int, K: int):
     """Two or three parts of one tile of up to 64 rows, where the norm adds them up and
-    no other rule has a kernel.  330 sizes, N of 4160 to 8192 and K of 4352 to 28672, with
-    the norm, over the library's time: 0.73 on average (1 row of 8192 x 28672 94 77 us,
-    12 of 7168 x 18432 113 47, 1 of 6656 x 17920 90 44, 64 of 6592 x 4736 28.5 22.4, 4 of
-    5120 x 5120 17.2 15.9; the worst, 5120 x 8192, even), but with rows of 16 KB in two
-    parts (8 of 8192 x 8192 33 36), and with 4096 columns and fewer (16 of 8192 x 4096 20
-    22.5).  In a step of 6 layers 5120 x 5120 in three gains with 12 rows (823 -> 813 us)
-    and loses with 1 (783 785)."""
+    no other rule has a kernel.  N of 4160 to 8192 and K of 4224 to 28672, with the norm,
+    over the library's time: 2 parts 0.72 in 66, none above 0.96 (1 row of 8192 x 28672
+    94 77 us, 12 of 7168 x 18432 113 47, 1 of 6656 x 17920 90 44, 8 of 8192 x 8192 34.4
+    30.5), 3 0.9 (4 of 5120 x 5120 18.2 16.7, 1 17.7 16.6), but up to 5120 columns, of
+    multiples of 256, and up to 4992 outputs 1.1 and more for every second size (2 of
+    4608 x 4608 13.4 15.1, 1 of 4168 x 5120 13.3 15.6, 1 of 4864 x 5120 0.97); those are
+    the library's, and so are 4096 columns and fewer (16 of 8192 x 4096 20 22.5)."""
     if not 1 <= M <= 64 or K % 128 or N % 8 or not 0 < N <= 8192 \
             or not 4096 < K <= 28672:
         return None
     split = 256 // -(-N // 64)
-    if split == 3:
-        return (64, 64, 3) if M > 1 or K > 5120 else None
-    return (64, 64, 2) if split == 2 and K != 8192 else None
+    if split == 3 and K <= 5120 and K % 256 == 0 and N <= 4992:
+        return None
+    return (64, 64, split) if 2 <= split <= 3 else None
 
 
 def _summed_gemm(M: int, N: int, K: int):

@@ -300,20 +300,24 @@ def test_rule_of_few_rows_of_long_columns():
 
 
 def test_rule_of_few_parts_of_one_tile():
-    """Up to 64 rows: at most a workgroup a unit, none where rows are 16 KB apart."""
+    """Up to 64 rows: at most a workgroup a unit; what rows of 16 KB took is right for
+    them by now, and few parts of many columns are not narrow ones."""
+    few2, few3, four, wide = (64, 64, 2), (64, 64, 3), (64, 64, 4), (128, 128, 8)
     for M, N, K, few, narrow in [
-            (1, 8192, 28672, (64, 64, 2), None), (64, 8192, 4224, (64, 64, 2), None),
-            (64, 8192, 4096, None, None), (1, 8192, 8192, None, None),
+            (1, 8192, 28672, few2, None), (64, 8192, 4224, few2, None),
+            (64, 8192, 4096, None, None), (1, 8192, 8192, few2, None),
             (1, 8192, 28800, None, None), (65, 8192, 28672, None, None),
-            (8, 5440, 8192, (64, 64, 3), None), (8, 5448, 9216, (64, 64, 2), None),
+            (8, 5440, 8192, few3, None), (8, 5448, 9216, few2, None),
             (8, 4096, 9216, None, None), (8, 8196, 9216, None, None),
-            (1, 5120, 5120, None, None), (2, 5120, 5120, (64, 64, 3), None),
-            (1, 5120, 5248, (64, 64, 3), None),
-            (33, 4096, 11008, None, (64, 64, 4)), (33, 4096, 8192, None, (128, 128, 8)),
-            (17, 1088, 16384, None, (64, 64, 8)), (64, 5120, 12288, (64, 64, 3),
-                                                   (64, 64, 3)),
-            (64, 5120, 12416, (64, 64, 3), (128, 128, 6)),
-            (17, 6144, 6144, (64, 64, 2), (128, 128, 5))]:
+            (1, 5120, 5120, few3, None), (1, 4992, 5120, None, None),
+            (2, 4608, 4608, None, None), (2, 4608, 4736, few3, None),
+            (1, 4168, 5376, few3, None), (33, 4096, 11008, None, four),
+            (33, 4096, 8192, None, four), (48, 4096, 18432, None, four),
+            (48, 4096, 18560, None, wide), (49, 4096, 12288, None, four),
+            (49, 4096, 14336, None, wide), (17, 1088, 16384, None, (64, 64, 8)),
+            (64, 5120, 8192, few3, few3), (64, 5120, 12288, few3, (128, 128, 6)),
+            (48, 5120, 12288, few3, few3), (48, 5120, 12416, few3, (128, 128, 6)),
+            (17, 6144, 6144, few2, (128, 128, 5))]:
         assert ops._few_parts(M, N, K) == few, (M, N, K)
         assert ops._less_padding(M, N, K, ops._split_gemm(M, N, K)) == narrow
         route = ops._route(M, N, K, True)
@@ -322,7 +326,7 @@ def test_rule_of_few_parts_of_one_tile():
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K", [
-    (1, 8192, 4224), (64, 6592, 9216), (7, 4168, 4352), (33, 4096, 11008),
+    (1, 8192, 4224), (64, 6592, 9216), (7, 4168, 4480), (33, 4096, 11008),
     (17, 1088, 16384), (64, 5120, 6272), (40, 3080, 8192)])
 def test_parts_of_one_tile_of_rows(M, N, K):
     """Workgroups of a tile of w begin at a column of its own in each part."""
