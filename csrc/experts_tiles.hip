@@ -275,17 +275,21 @@ DEV void high_tile_part(const Tiles& a, char* lds, int e, int p0, int nb,
                     at(d));
              });
   };
-  // Weights of one tile, in rows that lie 4 or 8 KB apart: of one column they are all a
-  // few channels'.  So each die, which has every eighth of the tiles of outputs, begins
-  // at a column of its own, and its workgroups still share x.  us, up: 8 experts of
-  // 14336 x 4096, 120 choices each 411 -> 389, 160 417 -> 381, 256 492 489; 8 of 8192 x
-  // 4096, 150 257 -> 205; 16 of 2048 x 4096, 130 134 -> 104, 250 145 -> 123; 32 of 1024 x
-  // 2048, 130 70 -> 55, 250 78 -> 68; 64, 130 138 -> 117.  Rows of 16 and 28 KB, experts of
-  // several tiles, which wait for more than weights, and few tiles of outputs (16 of 1024
-  // x 4096, 200 61 66) are 2 to 8 % slower.
+  // Weights of one tile, in rows of 4 KB, and with gates of 8 KB: of one column they are
+  // all a few channels'.  So each die, which has every eighth of the tiles of outputs,
+  // begins at a column of its own, and its workgroups still share x.  130 to 250 choices
+  // an expert, time over that without, two of the same differing by up to 10 %: 4 KB 0.94
+  // in 42 sizes (8 experts of 14336 x 2048 up, 150 224 -> 198 us, 16 of 2048 x 2048 73 59,
+  // down 16 of 4096 x 2048 76 64, e4m3 8 of 16384 x 4096 148 127), 8 KB with gates 0.94 in
+  // 14 (8 of 8192 x 4096,
+  // 170 261 220, 8 of 14336 x 4096, 130 396 367) but with few tiles of outputs 1.0; plain
+  // ones and e4m3 of 8 KB 1.03, up to 1.2 (16 of 4096 x 4096, 150 138 145, e4m3 8 of 8192
+  // x 16384, 130 246 273).  12 KB 0.95, and with 250 choices up to 1.07; 2, 6, 10, 14, 16
+  // KB and more 1.0 to 1.15 (8 of 4096 x 14336, 250 428 454), e4m3 of 20 KB 0.99.
   if (!alone)
     run(std::false_type(), 0);
-  else if ((row_bytes == 4096 || row_bytes == 8192) && a.nx >= 16)
+  else if (row_bytes == 4096 ? a.nx >= 8
+                             : GATED && row_bytes == 8192 && a.nx >= 16)
     run(std::true_type(), nb % 8 * chunks / 8);
   else
     run(std::true_type(), 0);

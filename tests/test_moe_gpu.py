@@ -447,3 +447,54 @@ def test_tiles_as_high_as_their_choices(kind, outputs, chunks):
             want, slack = want * scale, slack * scale
         assert ((got[mine] - want).abs()
                 <= 2.0 ** -8 * want.abs() + 1.01 * slack).all()
+
+
+@pytest.mark.parametrize("kind", ["gated", "plain", "fp8"])
+@pytest.mark.parametrize("outputs", [1152, 4096])   # tiles of 128 and of 256
+@pytest.mark.parametrize("row_kb", [4, 6, 8])
+def test_where_tiles_of_one_expert_begin(kind, outputs, row_kb):
+    """Tiles of rows of 4 KB, and with gates of 8 KB, begin their weights at columns of
+    their own, but not those of an expert that has two.  Bounds as above."""
+    gated, fp8 = kind == "gated", kind == "fp8"
+    counts = [130, 200, 256, 131, 257, 140, 180, 150, 222, 160]
+    E, T = len(counts), sum(counts)
+    K = row_kb * (1024 if fp8 else 512)
+    rows = outputs * (2 if gated else 1)
+    g = torch.Generator(DEV).manual_seed(row_kb)
+    rand = lambda *s: torch.randn(*s, generator=g, device=DEV)
+    ids = torch.repeat_interleave(torch.arange(E), torch.tensor(counts)).int().to(DEV)
+    order, expert, place = ops._moe_sort(ids[:, None], E, 128, 128, 256)
+    x, w = rand(T, K).bfloat16(), (rand(E, rows, K) * K ** -0.5).bfloat16()
+    sx = sw = None
+    if fp8:
+        x, w = x.to(torch.float8_e4m3fn), (w * 64).to(torch.float8_e4m3fn)
+        sx, sw = rand(T).abs(), rand(E, rows).abs()
+
+    def product(w):
+        out = torch.empty(len(order), outputs, dtype=torch.bfloat16, device=DEV)
+        ops._native().experts_tiles(out, x, w, sx, sw, order, expert, gated, 1, 256)
+        return out[place[:, 0].long()]
+
+    got = product(w)
+    for e in range(E):
+        mine = ids == e
+        a, b = x[mine].double(), w[e].double()
+        want, slack = a @ b.t(), a.abs() @ b.abs().t() * 2.0 ** (-16 if fp8 else -22)
+        if gated:
+            (gate, up), (dg, du) = want.chunk(2, -1), slack.chunk(2, -1)
+            want = torch.nn.functional.silu(gate) * up
+            slack = 1.1 * dg * up.abs() + gate.abs() * du + 2.0 ** -20 * want.abs()
+        if fp8:
+            scale = sx[mine, None].double() * sw[e].double()
+            want, slack = want * scale, slack * scale
+        assert ((got[mine].double() - want).abs()
+                <= 2.0 ** -8 * want.abs() + 1.01 * slack).all()
+    if fp8:
+        return
+    # 256 outputs on, the same weights are another tile's; roundings hide most changes
+    turned = w.view(E, 2 if gated else 1, outputs, K).roll(256, 2).reshape(w.shape)
+    other = product(turned).roll(-256, 1)
+    apart = (other != got).any(-1)
+    alone = torch.tensor([n <= 256 for n in counts], device=DEV)[ids.long()]
+    assert not apart[~alone].any()
+    assert bool(apart[alone].any()) == (row_kb == 4 or row_kb == 8 and gated)
