@@ -93,13 +93,13 @@ __global__ __launch_bounds__(256) void greedy_sample_kernel(
 //
 // 64 rows of 128256 in bfloat16, 48 values far above the others, us with a workgroup
 // a row, in slices, and with lists of the slices (rows in cache; from memory 2 to 3
-// more): temperature 36 13.2 11.7, top_p 0.9 43 18.9 14.4, top_k 50 24 12.6 11.6,
-// greedy 9.4 6.7 6.9; a mix 42 19.0 14.5, where the library's sorts, scans and
-// selections took 2625.  A mix of 1 row 15.4 -> 12.5, of 128 26.6 -> 23.8; 64 rows of
-// 32000 16.5 -> 13.2.  What the lists cost where they do not help: normal logits, whose
-// share is thousands of values, 112 -> 114; top_k 50 of 128 rows, which are two
-// workgroups a compute unit, 16.9 -> 17.4.  A call that is waited for and not captured
-// 60 36.
+// more): temperature 36 13.2 12.5, top_p 0.9 43 20.2 15.6, top_k 50 24 13.7 12.6,
+// greedy 9.4 7.8 7.9; a mix 42 19.9 15.6, where the library's sorts, scans and
+// selections took 2625.  A mix of 1 row 16.4 -> 13.4, of 128 27.2 -> 24.0; 64 rows of
+// 32000 17.2 -> 13.9.  What the lists cost where they do not help: top_k of 65 to 128 rows
+// of 128256, which are two workgroups a compute unit, 2 to 4 % (50 of 128 17.6 -> 18.0;
+// without them a mix loses, 24.0 -> 26.5), greedy rows if they are few 0.3 (16 7.4 -> 7.8).
+// A call that is waited for and not captured 60 36.
 //
 // Weights are 2^-40 fixed point relative to the largest (of the row or of the
 // slice), so sums within a row or a slice are exact; slices are brought to the
@@ -905,18 +905,36 @@ DEV bool listed_k(int k) { return k > 0 && k <= NEAR / 2; }
 constexpr int COUNTS = 256;       // steps that a slice's threads are counted in
 
 // From s.count, how many threads' largest values are in each of COUNTS steps: the
-// end of the step in which `want` of them are reached; COUNTS + 1 if there are
-// fewer.  Each wave by itself, 4 steps a lane.
-DEV int end_of(const Scratch& s, unsigned want) {
+// end of the step in which `want` of them are reached, COUNTS + 1 if there are
+// fewer, how many are up to there, and how many up to about step `near`.  Each wave by
+// itself, 4 steps a lane.
+struct Reached {
+  int end;
+  unsigned n, near;
+};
+DEV Reached end_of(const Scratch& s, unsigned want, int near) {
   const int lane = threadIdx.x & 63;
   const uint4 c = reinterpret_cast<const uint4*>(s.count)[lane];
   const unsigned upto = wave_scan(c.x + c.y + c.z + c.w);
+  const unsigned nearer = lane_of(upto, min(near / 4, 63));
   const u64 there = __ballot(upto >= want);
-  if (!there) return COUNTS + 1;
-  const int end = lane * 4 + 4 - (upto - c.w >= want) -
-                  (upto - c.w - c.z >= want) -
-                  (upto - c.w - c.z - c.y >= want);
-  return lane_of(end, __ffsll(there) - 1);
+  if (!there) return {COUNTS + 1, lane_of(upto, 63), nearer};
+  int end = lane * 4 + 4;
+  unsigned n = upto;
+  if (n - c.w >= want) {
+    n -= c.w;
+    --end;
+    if (n - c.z >= want) {
+      n -= c.z;
+      --end;
+      if (n - c.y >= want) {
+        n -= c.y;
+        --end;
+      }
+    }
+  }
+  const int first = __ffsll(there) - 1;
+  return {lane_of(end, first), lane_of(n, first), nearer};
 }
 
 // Steps below the largest value, down to where weights are zero
@@ -1037,43 +1055,53 @@ __global__ __launch_bounds__(NT) void sample_slice_kernel(
   __syncthreads();
   const float part = (float)(o.k ? o.k : SHARE) *
                      __builtin_amdgcn_rcpf((float)slices);
-  const int reached =
-      end_of(s, (unsigned)(part + 4.f * __builtin_amdgcn_sqrtf(part)) + 2);
-  const float low = reached > COUNTS && o.k && !steps.whole
+  const Reached reached =
+      end_of(s, (unsigned)(part + 4.f * __builtin_amdgcn_sqrtf(part)) + 2,
+             (int)fminf(7.f / 43.f * steps.zero * steps.scale, COUNTS));
+  const float low = reached.end > COUNTS && o.k && !steps.whole
       ? none
-      : fmaxf(mx - fminf((float)reached, last) * (steps.range / COUNTS), -FLT_MAX);
-  // too many: without a look at each of them
+      : fmaxf(mx - fminf((float)reached.end, last) * (steps.range / COUNTS),
+              -FLT_MAX);
+  // Too many values, or a share where more threads' largest than FEW twice weigh more
+  // than 2^-7 of the slice's largest, as below: without a look at each of them.  us
+  // before lists, with lists and so: share of normal logits 64 rows of 128256 118 120 118,
+  // 240 of 32768 48.5 50.6 48.6, top_k 50 of logits of 4 values 155 161 157, 52 58 54
   const int most = NEAR / group;
-  if (__popcll(__ballot(thread_mx >= low)) > most / 4) {
-    if (lane == 0) atomicAdd(&s.n, NEAR + 1u);
-  } else {
-    // a thread has few, so each goes through its own: one of its 8 values, and
-    // one of these
-    unsigned loads = 0;
+  if ((int)reached.n > most || !o.k && reached.near > 2 * FEW) {
+    if (tid == 0) {
+      mine.low = none;
+      mine.n = 0;
+    }
+    return;
+  }
+  // a thread has few, so each goes through its own: one of its 8 values, and
+  // one of these
+  unsigned loads = 0;
+  #pragma unroll
+  for (int q = 0; q < HELD; ++q) loads |= (top[q] >= low) << q;
+  for (; loads; loads &= loads - 1) {
+    const int q = __ffs(loads) - 1;
+    auto r = raw[0];
     #pragma unroll
-    for (int q = 0; q < HELD; ++q) loads |= (top[q] >= low) << q;
-    for (; loads; loads &= loads - 1) {
-      const int q = __ffs(loads) - 1;
-      auto r = raw[0];
+    for (int j = 1; j < HELD; ++j)
+      if (q == j) r = raw[j];
+    float x[8];
+    row.spread(r, x);
+    unsigned hits = 0;
+    #pragma unroll
+    for (int i = 0; i < 8; ++i) hits |= (x[i] >= low) << i;
+    for (; hits; hits &= hits - 1) {
+      const int i = __ffs(hits) - 1;
+      float y = x[0];
       #pragma unroll
-      for (int j = 1; j < HELD; ++j)
-        if (q == j) r = raw[j];
-      float x[8];
-      row.spread(r, x);
-      unsigned hits = 0;
-      #pragma unroll
-      for (int i = 0; i < 8; ++i) hits |= (x[i] >= low) << i;
-      for (; hits; hits &= hits - 1) {
-        const int i = __ffs(hits) - 1;
-        float y = x[0];
-        #pragma unroll
-        for (int j = 1; j < 8; ++j) y = i == j ? x[j] : y;
-        const int n = (int)atomicAdd(&s.n, 1u);
-        if (n < most) {
-          mine.list[n] = y;
-          mine.list_at[n] = first + (q * NT + tid) * 8 + i;
-        }
+      for (int j = 1; j < 8; ++j) y = i == j ? x[j] : y;
+      const int n = (int)atomicAdd(&s.n, 1u);
+      if (n >= most) {
+        loads = 0;
+        break;
       }
+      mine.list[n] = y;
+      mine.list_at[n] = first + (q * NT + tid) * 8 + i;
     }
   }
   __syncthreads();

@@ -272,6 +272,40 @@ def test_lists_of_slices(vocab, rows, dtype):
         assert ok[out[b]], (i, options[o], out[b], n)
 
 
+@pytest.mark.parametrize("vocab,rows", [(8200, 64), (32768, 200), (50257, 40),
+                                        (128256, 30)])
+def test_slices_that_list_nothing(vocab, rows):
+    """Slices whose values are too many for a list, or for a share of a list, and those
+    that just have one: 230 to 300 equal ones in one wave, in one slice and all over, so
+    many within 2^-7 of a largest, and nothing but equal values."""
+    g = torch.Generator().manual_seed(vocab)
+    x = torch.randn(8, vocab, generator=g)
+    anywhere = torch.randperm(vocab, generator=g)
+    x[0] = 1.5
+    x[1] = torch.randint(0, 4, (vocab,), generator=g).float()
+    x[2, 8:248] = 9.0                          # one wave
+    x[3, :4 * 300:4] = 9.0                     # one slice
+    x[4, anywhere[:230]] = 9.0
+    for i, n in ((5, 250), (6, 270), (7, 2000)):
+        x[i, anywhere[:n]] = 12 - 4 * torch.rand(n, generator=g)
+        x[i, anywhere[0]] = 12.0
+    x = x.bfloat16()
+    options = [(1.0, 0.9, 0), (1.0, 0.2, 0), (1.0, 1.0, 50), (0.7, 0.95, 100),
+               (1.0, 1.0, 101), (1.0, 1.0, 0)]
+    pick = [(i, o, (n + 0.5) / 3) for i in range(8)
+            for o in range(len(options)) for n in range(3)]
+    t, p, k = (torch.tensor(c) for c in zip(*(options[o] for _, o, _ in pick)))
+    which = torch.tensor([i for i, _, _ in pick])
+    u = torch.tensor([n for _, _, n in pick])
+    out = torch.cat([
+        ops.sample(*(c.to(DEV) for c in (x[which[a]], t[a], p[a], k[a].int(),
+                                         u[a])))
+        for a in torch.arange(len(pick)).split(rows)]).tolist()
+    for b, (i, o, n) in enumerate(pick):
+        ok, _ = _allowed(x[i].float(), *options[o], float(u[b]))
+        assert ok[out[b]], (i, options[o], out[b], n)
+
+
 @pytest.mark.parametrize("vocab", [1000, 32768])
 def test_zeros_of_either_sign_are_equal(vocab):
     """The first of the largest values is -0."""
