@@ -79,7 +79,7 @@ __global__ __launch_bounds__(256) void greedy_sample_kernel(
 // Where few values stay, and next-token logits have a few dozen that matter, they
 // are listed and the rest is done on the list, up to 8 threads a value.  n values
 // take n^2 steps, so the lists are kept short.  Each slice lists its own largest, so
-// many that a share is found among the 64 largest of the row, or top_k up to 128:
+// many that a share is found among the 64 largest of the row, or top_k up to 100:
 // that takes 0.8 us where weights are computed and 2 where not, and the second kernel
 // has the row's list without a pass of its own over the row, which took it 4.5 us (a
 // mix 19.0 -> 14.5 us with the sums of weights, below).  Where that list is too short,
@@ -899,8 +899,10 @@ struct Slice {
 // threads of a slice whose values are looked at together
 DEV int together(int slices) { return slices <= 4 ? 1 : slices <= 8 ? 2 : 4; }
 
-// whether slices list values for top_k (0: there is none)
-DEV bool listed_k(int k) { return k > 0 && k <= NEAR / 2; }
+// Whether slices list values for top_k (0: there is none).  Up to 100: of more, the
+// row's list is too long now and then (128 of 16, 64 and 240 rows 16.6 16.7 16.3 ->
+// 17.5 17.8 17.9 us, 100 of 64 15.4 -> 14.6).
+DEV bool listed_k(int k) { return k > 0 && k <= 100; }
 
 constexpr int COUNTS = 256;       // steps that a slice's threads are counted in
 
