@@ -281,11 +281,10 @@ DEV void high_tile_part(const Tiles& a, char* lds, int e, int p0, int nb,
   // an expert, time over that without, two of the same differing by up to 10 %: 4 KB 0.94
   // in 42 sizes (8 experts of 14336 x 2048 up, 150 224 -> 198 us, 16 of 2048 x 2048 73 59,
   // down 16 of 4096 x 2048 76 64, e4m3 8 of 16384 x 4096 148 127), 8 KB with gates 0.94 in
-  // 14 (8 of 8192 x 4096,
-  // 170 261 220, 8 of 14336 x 4096, 130 396 367) but with few tiles of outputs 1.0; plain
-  // ones and e4m3 of 8 KB 1.03, up to 1.2 (16 of 4096 x 4096, 150 138 145, e4m3 8 of 8192
-  // x 16384, 130 246 273).  12 KB 0.95, and with 250 choices up to 1.07; 2, 6, 10, 14, 16
-  // KB and more 1.0 to 1.15 (8 of 4096 x 14336, 250 428 454), e4m3 of 20 KB 0.99.
+  // 14 (8 of 8192 x 4096, 170 261 220, 8 of 14336 x 4096, 130 396 367) but with few tiles
+  // of outputs 1.0; plain ones and e4m3 of 8 KB 1.03, up to 1.2 (16 of 4096 x 4096, 150
+  // 138 145, e4m3 8 of 16384 x 8192, 130 246 273).  12 KB 0.95, and with 250 choices up to
+  // 1.07; 2, 6, 10, 14, 16 KB and more 1.0 to 1.15 (8 of 4096 x 14336, 250 428 454).
   if (!alone)
     run(std::false_type(), 0);
   else if (row_bytes == 4096 ? a.nx >= 8

@@ -383,10 +383,10 @@ def _wave_of_longer_rows(M: int, N: int, K: int):
     """The same tiles for 65 to 128 rows and longer columns where they are at least 176,
     before parts of K that a pass adds up.  Random sizes, time over what was there: K up
     to 4608 0.92 in 158 (96 rows of 6144 x 4096 21.8 -> 20.0 us, 128 23.8 23.2, 66 of
-    7168 x 4096 24.6 20.2), one more than 3 % slower, but of 97 to 128 rows up to 3712 columns 1.03 in 62,
-    up to 1.32 (125 of 6032 x 2560 13.7 17.0); up to 5632 0.97, every seventh slower, up
-    to 1.11 (128 of 6144 x 5120 27.4 28.8), beyond 1.06; fewer tiles 1.05 to 1.2.  Where
-    the norm adds up the parts those are faster (96 rows 17.4)."""
+    7168 x 4096 24.6 20.2), one more than 3 % slower, but of 97 to 128 rows up to 3712
+    columns 1.03 in 62, up to 1.32 (125 of 6032 x 2560 13.7 17.0); up to 5632 0.97, every
+    seventh slower, up to 1.11 (128 of 6144 x 5120 27.4 28.8), beyond 1.06; fewer tiles
+    1.05 to 1.2.  Where the norm adds up the parts those are faster (96 rows 17.4)."""
     if not 64 < M <= 128 or K % 128 or N % 4 \
             or not (2304 if M <= 96 else 3712) < K <= 4608:
         return None
@@ -642,10 +642,10 @@ def _wide_parts(M: int, N: int, K: int):
     time over that: 10240 columns and more, up to 1400 rows 0.69 in 97 (262 rows of
     4096 x 14336 58 48 us, 600 112 76, 1000 137 110, 1268 161 132; the worst 1154 of 6336
     x 15360 even), but 1.09 for tiles that fill no wave and 1.10 in 45 for one part of
-    tiles of 256 outputs, which are 180 to 217 (1114 of 8144 x 12928 231 252); from 4608 on 513 to 1024 rows
-    0.90 in 57 (the worst 989 of 8032 x 4992 89 92).  Shorter ones are slower (up to 2560
-    columns and 4096 outputs, 513 to 1024 rows, 1.14 in 93, 630 of 1768 x 2048 17.6 21.1), and
-    so are more rows (1.0).
+    tiles of 256 outputs, which are 180 to 217 (1114 of 8144 x 12928 231 252); from 4608
+    on 513 to 1024 rows 0.90 in 57 (the worst 989 of 8032 x 4992 89 92).  Shorter ones
+    are slower (up to 2560 columns and 4096 outputs, 513 to 1024 rows, 1.14 in 93, 630 of
+    1768 x 2048 17.6 21.1), and so are more rows (1.0).
     129 to 256 rows of 10240 columns and more, one tile of rows and more than 192 in all,
     0.65 (135 rows of 4096 x 14336 44 36 us, 248 53 45); decode steps of 140, 200 and 256
     rows, 8 layers, 1 % less.  Fewer rows are as fast in the step (100 1730 1738), fewer
@@ -1032,23 +1032,30 @@ def moe_router(x, router: torch.Tensor, top: int,
 
 
 # Mean rows per expert up to which the kernels without a sort, and tiles of 64
-# and 128 rows are taken (and 256 beyond).  64 and 128 leave room for the spread
-# of the counts: a few rows more than a tile and an expert's weights are read
-# twice, by workgroups that share their compute units with others.  us on an
-# MI355X without a sort, and in tiles of 64, 128, 256, sort included
-#   8 experts of 14336 x 4096   1 row 324 345, 2 rows 425 432, 3 423 417, 5 445
-#     430, 48 - 464 500 604 (56, one of 66 rows, - 510 510), 100 - 853 571 653,
-#     112 - 923 625 659, 125 - 1096 815 681
-#   16 of 2048 x 4096           1 row 104 115, 3 rows 137 138, 5 146 135, 48 -
-#     144 156 204, 52 - 166 156, 112 - 281 217 218, 125 - 283 231 219
-#   32 of 1024 x 2048           1 row 56 64, 3 rows 71 75, 5 78 77, 44 - 80 91
-#     119, 48 - 93 91 121, 112 - 146 129 126, 125 - 150 133 129
-#   64 of 1024 x 2048           1 row 94 101, 3 rows 131 129, 5 154 134, 48 -
-#     163 172 228, 112 - 279 222 242, 125 - 309 257 247
+# and 128 rows are taken (and 256 beyond).  64 leave room for the spread of the
+# counts: a few rows more than a tile and an expert's weights are read twice, by
+# workgroups that share their compute units with others.  Tiles of 256 are as high as
+# their choices, so 128 are no faster from 80 on and 1.3 times as slow where an expert
+# has more of them.  us on an MI355X without a sort, and in tiles of 64, 128, 256, sort
+# included, and where the first experts are chosen 1.9 times as often as the last
+#   8 experts of 14336 x 4096   1 row 280 342, 2 rows 430 447, 3 438 453, 5 450
+#     449, 48 - 470 521 507, 56 - 589 526 527, 80 - 766 564 533, 100 - 804 580 575,
+#     112 - 813 589 566, uneven 80 - 746 547 536, 112 - 898 723 568
+#   16 of 2048 x 4096           1 row 86 106, 3 rows 133 141, 5 137 140, 48 -
+#     145 152 164, 56 - 163 153 162, 80 - 197 163 169, 100 - 213 172 169, 112 - 235 199
+#     176, uneven 80 - 206 165 169, 100 - 225 203 172
+#   32 of 1024 x 2048           1 row 51 60, 3 rows 71 75, 5 77 75, 48 - 81 89
+#     83, 56 - 101 91 84, 80 - 112 96 92, 100 - 114 101 93, uneven 100 - 129 121 98
+#   64 of 1024 x 2048           1 row 86 97, 3 rows 131 135, 5 153 140, 48 - 145
+#     170 161, 80 - 208 191 178, 100 - 234 202 183, uneven 100 - 253 228 183
+# 256 over 128 in seven stacks, even and uneven, and e4m3 in four: 56 0.99 0.97 1.02, 80
+# 0.97 0.97 0.99, 90 0.96 0.96 0.97, 100 0.96 0.87 0.98, 112 0.88 0.84 0.94; the worst
+# from 90 on 16 of 3072 x 6144, 366 401, up to 80 16 of 2048 x 4096.
 # Choices that are uneven are better in the next larger tiles where several experts
-# have a little more than a tile: 190 tokens of 8 experts, 47.5 choices on average, up
-# to 56 458 512, up to 84 588 511, up to 127 556 514, up to 150 640 688.
-MOE_ROWS, MOE_ROWS_64, MOE_ROWS_128 = 2.9, 48, 112
+# have a little more than a tile: 190 tokens of 8 experts, 47.5 choices on average, us
+# in tiles of 64, 128, 256, even 477 519 511, the first 1.5 times as often as the last
+# 481 515 512, 2.3 times 566 514 514.
+MOE_ROWS, MOE_ROWS_64, MOE_ROWS_128 = 2.9, 48, 80
 
 
 def _moe_tile(T: int, K: int, E: int, least: int) -> int:

@@ -39,7 +39,8 @@ def test_router(tokens, experts, top, width, fp8):
     assert (weight.double() - ref).abs().max() <= 4 * slack + 1e-6
 
 
-@pytest.mark.parametrize("tokens", [1, 2, 12, 13, 64, 104, 105, 224, 225, 416, 600])
+@pytest.mark.parametrize("tokens", [1, 2, 12, 13, 64, 104, 105, 160, 161, 224, 225, 416,
+                                    600])
 @pytest.mark.parametrize("experts,top,width,inner", [
     (4, 2, 256, 128), (8, 1, 128, 384), (2, 2, 384, 32768)])
 def test_experts_around_the_rule(tokens, experts, top, width, inner):
@@ -62,6 +63,13 @@ def test_experts_around_the_rule(tokens, experts, top, width, inner):
         ref += y * (weight * (ids == e)).sum(-1)[:, None].double()
     assert (out - ref).norm() <= 2.0 ** -7 * ref.norm()
     assert (out - ref).abs().max() <= 2.0 ** -5 * ref.abs().max()
+
+
+def test_tiles_of_the_mean_of_choices():
+    """Beyond 80 an expert, tiles of 256 rows, which are as high as their choices."""
+    assert [ops._moe_tile(t, 2, 8, 16) for t in (11, 12, 192, 193, 320, 321, 448)] \
+        == [16, 64, 64, 128, 128, 256, 256]
+    assert ops._moe_tile(11, 2, 8, 64) == 64
 
 
 @pytest.mark.parametrize("counts", [(256, 257, 0, 1), (1, 512, 200, 255),
