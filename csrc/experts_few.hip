@@ -21,9 +21,8 @@
 // non-temporal; that was slower still):
 //   32 experts of 1024 x 2048, 4 each   1 row 9.0 5.8 (10.1 7.2), 4 rows 22.7
 //     12.9 (25.5 14.4), 16 rows 44 24 (49 27)
-//   8 experts of 14336 x 4096, 2 each   1 row 74 40 (82 59), 4 rows 179 105
-//     (200 125), 10 rows 268 157 (302 177); the last two before workgroups began at
-//     different columns (below), which is 2 to 9 %
+//   8 experts of 14336 x 4096, 2 each   1 row 75 40 (82 59), 4 rows 175 92
+//     (200 125), 10 rows 242 138 (302 177)
 #include <type_traits>
 
 #include "common.h"
@@ -85,7 +84,7 @@ __global__ __launch_bounds__(WAVES * 64) void experts_few_kernel(Few a) {
   // lengths it is 0 to 2 % slower, and even where the up product has rows of 4 KB: 32 of
   // 1024 x 2048, 16 21.7 21.9, 64 of 1408 x 2048, 24 42.1 41.1.
   const int batches = a.K / (2 * STEP);
-  const int begin = a.K % 2048 == 0 && a.K > (UP ? 2048 : 1024)
+  const int begin = a.K % 2048 == 0 && a.K > (UP ? 2048 : 0)
       ? (int)(blockIdx.x / 8 % (unsigned)batches) : 0;
   for (int r0 = 0; r0 < count; r0 += 16) {
     const bf16* xp[2];                         // of 8 choices and 8 more
