@@ -6,16 +6,17 @@
 //
 // A workgroup has bm choices of one expert and BN rows of its weights, K in
 // chunks of 128 bytes.  Both go from memory to LDS directly, 16 bytes a lane
-// and whole 128-byte lines, into a ring of chunks; weights are the A operand
-// of 32x32x16 products, so that a lane's results are 4 consecutive outputs of
-// one choice, and of every 16 rows of weights 8 are a gate's and 8 its up
-// row's: both of a pair are in one lane, and the activation needs no pass of
-// its own.
+// and whole 128-byte lines, into a ring of chunks; weights are the A operand of
+// matrix products, so that a lane's results are consecutive outputs of one choice,
+// and rows of gates and their up rows alternate in LDS: both of a pair are in one
+// lane, and the activation needs no pass of its own.  Tiles of 64 and 128 choices
+// form 32 x 32 products, with 8 gates and their 8 up rows in turn; those of up to 256
+// (experts_high_kernel) 16 x 16 of bf16, with 16 and 16.
 //
 // What bounds it: the weights' bytes up to about 100 choices an expert, so bm
 // is what covers most counts, then the products.  Mixtral 8x7B layer (8 experts,
-// 14336 x 4096, 2.8 GB), us: 16 choices an expert 443, 48 459, 128 650, 302 906, 500
-// 1210.  32 experts of 1024 x 2048, 62 choices 95.
+// 14336 x 4096, 2.8 GB), us: 16 choices an expert 443, 48 470, 112 566, 140 601, 302
+// 906, 500 1210.  32 experts of 1024 x 2048, 64 choices 93.
 #include <algorithm>
 #include <type_traits>
 
@@ -108,10 +109,9 @@ void experts_tiles_kernel(Tiles a) {
   const int next = a.expert[min(tile + 1, tiles - 1)];
   if (e < 0) return;
   // Weights that one tile takes are read once (ONCE), those of several not: they
-  // would leave the others nothing.  us, up and down of 8 experts of 14336 x 4096,
-  // 112 choices each 718 -> 660, 160 752 -> 722, of 16 of 2048 x 4096, 112 226 ->
-  // 214; those of several tiles of 256 by ONCE 1.1 times slower.  Where tokens prefer
-  // the same experts, smaller tiles are several too, by ONCE and so: 300 choices of
+  // would leave the others nothing.  us, up and down, in tiles of 128, of 8 experts of
+  // 14336 x 4096, 112 choices each 718 -> 660, of 16 of 2048 x 4096 226 -> 214.  Where
+  // tokens prefer the same experts, tiles are several, by ONCE and so: 300 choices of
   // each of 2 experts of 16 in tiles of 64 95 -> 71, 64 experts of 1024 x 2048, up to
   // 190 each 104 -> 92, 150 of each of 2 of 8 343 -> 305, 100 to 200 uneven tokens of
   // 8 604 -> 577 and 606 -> 588; even ones 440 442, 138 138, 149 149.
@@ -210,7 +210,7 @@ void experts_tiles_kernel(Tiles a) {
 // 2912 1428, 130 454 232 and 430 211; 16 of 2048 x 4096, 300 239 132 and 170 95; 32 of
 // 1024 x 2048, 300 131 89 and 92 67, 1000 264 169 and 255 147.  e4m3: 302 404 216 and
 // 335 146, 2000 1815 943 and 1671 752.  Even: two workgroups of one expert with its
-// choices together and half of the weights each; weights begun at different columns.
+// choices together and half of the weights each.
 template <int H, bool LATER, int BN, bool GATED, bool FP8, bool FAR>
 DEV void high_tile_part(const Tiles& a, char* lds, int e, int p0, int nb,
                         bool alone) {
@@ -279,12 +279,13 @@ DEV void high_tile_part(const Tiles& a, char* lds, int e, int p0, int nb,
   // all a few channels'.  So each die, which has every eighth of the tiles of outputs,
   // begins at a column of its own, and its workgroups still share x.  130 to 250 choices
   // an expert, time over that without, two of the same differing by up to 10 %: 4 KB 0.94
-  // in 42 sizes (8 experts of 14336 x 2048 up, 150 224 -> 198 us, 16 of 2048 x 2048 73 59,
-  // down 16 of 4096 x 2048 76 64, e4m3 8 of 16384 x 4096 148 127), 8 KB with gates 0.94 in
-  // 14 (8 of 8192 x 4096, 170 261 220, 8 of 14336 x 4096, 130 396 367) but with few tiles
-  // of outputs 1.0; plain ones and e4m3 of 8 KB 1.03, up to 1.2 (16 of 4096 x 4096, 150
-  // 138 145, e4m3 8 of 16384 x 8192, 130 246 273).  12 KB 0.95, and with 250 choices up to
-  // 1.07; 2, 6, 10, 14, 16 KB and more 1.0 to 1.15 (8 of 4096 x 14336, 250 428 454).
+  // in 42 sizes (8 experts of 14336 x 2048 up, 150 224 -> 198 us, 16 of 2048 x 2048 73
+  // 59, down 16 of 4096 x 2048 76 64, e4m3 8 of 16384 x 4096 148 127), 8 KB with gates
+  // 0.94 in 14 (8 of 8192 x 4096, 170 261 220, 8 of 14336 x 4096, 130 396 367) but with
+  // few tiles of outputs 1.0; plain ones and e4m3 of 8 KB 1.03, up to 1.2 (16 of 4096 x
+  // 4096, 150 138 145, e4m3 8 of 16384 x 8192, 130 246 273).  12 KB 0.95, and with 250
+  // choices up to 1.07; 2, 6, 10, 14, 16 KB and more 1.0 to 1.15 (8 of 4096 x 14336, 250
+  // 428 454).
   if (!alone)
     run(std::false_type(), 0);
   else if (row_bytes == 4096 ? a.nx >= 8

@@ -10,10 +10,11 @@
 // different columns are 2 to 8 % slower; 4 waves of 128 x 128 as fast.
 //
 // us, what was there (mostly the library's product, its pass or its norm) and here:
-// silu(gate) * up 28672 x 4096 300 rows 83 76, 512 112 104, 880 203 176, 14336 x 2048
-// 600 45 36, 2600 183 146; 4096 x 14336 with the norm 262 rows 58 48, 600 112 76, 1000
-// 137 110, 7411 without 971 640; 2048 x 7168, 600 rows 37 25.  The library is faster for
-// thousands of rows of full waves (8192 of 4096 x 14336 605 690).
+// silu(gate) * up 28672 x 4096 300 rows 85 79, 512 109 109 (but 6 less in the step),
+// 880 197 187, 14336 x 2048 600 48 40, 2600 181 143; 4096 x 14336 with the norm 262 rows
+// 64 52, 600 121 80, 1000 145 114, 7411 without 1006 647; 2048 x 7168, 600 rows 38 32.
+// The library is faster for thousands of rows of full waves (8192 of 4096 x 14336 605
+// 690).
 #include <algorithm>
 
 #include "tile_loop.h"

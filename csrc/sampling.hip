@@ -93,13 +93,13 @@ __global__ __launch_bounds__(256) void greedy_sample_kernel(
 //
 // 64 rows of 128256 in bfloat16, 48 values far above the others, us with a workgroup
 // a row, in slices, and with lists of the slices (rows in cache; from memory 2 to 3
-// more): temperature 36 13.2 12.5, top_p 0.9 43 20.2 15.6, top_k 50 24 13.7 12.6,
+// more): temperature 36 14.1 12.5, top_p 0.9 43 20.2 15.6, top_k 50 24 13.7 12.6,
 // greedy 9.4 7.8 7.9; a mix 42 19.9 15.6, where the library's sorts, scans and
 // selections took 2625.  A mix of 1 row 16.4 -> 13.4, of 128 27.2 -> 24.0; 64 rows of
-// 32000 17.2 -> 13.9.  What the lists cost where they do not help: top_k of 65 to 128 rows
-// of 128256, which are two workgroups a compute unit, 2 to 4 % (50 of 128 17.6 -> 18.0;
-// without them a mix loses, 24.0 -> 26.5), greedy rows if they are few 0.3 (16 7.4 -> 7.8).
-// A call that is waited for and not captured 60 36.
+// 32000 17.2 -> 13.9.  What the lists cost where they do not help: top_k of 65 to 128
+// rows of 128256, which are two workgroups a compute unit, 2 to 4 % (50 of 128 17.6 ->
+// 18.0; without them a mix loses, 24.0 -> 26.5), greedy rows if they are few 0.3 (16 7.4
+// -> 7.8).  A call that is waited for and not captured 60 36.
 //
 // Weights are 2^-40 fixed point relative to the largest (of the row or of the
 // slice), so sums within a row or a slice are exact; slices are brought to the
@@ -127,7 +127,7 @@ struct Weight {
   // false: weights of x and less are below half of 2^-40
   DEV bool any(float x) const { return (x - mx) * hi > -42.f; }
   DEV u64 operator()(float x) const { return any(x) ? always(x) : 0; }
-  // the same of less than 2^-8 of the largest
+  // the same of less than 2^-8 of the largest; 8 of less than 2^-12 add up to 32 bits
   DEV unsigned small(float x) const {
     return (unsigned)scaled(x);
   }
@@ -874,10 +874,10 @@ __global__ __launch_bounds__(NT) void sample_kernel(
 // ---- rows in slices -------------------------------------------------------
 // A row a workgroup leaves most of the chip idle.  Here a row is divided into
 // slices of a workgroup each, which read their values once; what they find out
-// meets in a second kernel, a workgroup a row, with the largest values of each.  Weights are relative to the
-// slice's own largest value, so that no slice waits for another one; the sums of
-// 512 values are exact, and are brought to the row's largest value by one factor
-// a slice.
+// meets in a second kernel, a workgroup a row, with the largest values of each.
+// Weights are relative to the slice's own largest value, so that no slice waits for
+// another one; the sums of 512 values are exact, and are brought to the row's largest
+// value by one factor a slice.
 constexpr int HELD = 4;           // 8 values each, that a thread has (wave_sums)
 constexpr int SLICES = 16;        // of a row at most
 constexpr int UNITS = 4;          // a thread of the second kernel has at most
@@ -1064,10 +1064,10 @@ __global__ __launch_bounds__(NT) void sample_slice_kernel(
       ? none
       : fmaxf(mx - fminf((float)reached.end, last) * (steps.range / COUNTS),
               -FLT_MAX);
-  // Too many values, or a share where more threads' largest than FEW twice weigh more
-  // than 2^-7 of the slice's largest, as below: without a look at each of them.  us
-  // before lists, with lists and so: share of normal logits 64 rows of 128256 118 120 118,
-  // 240 of 32768 48.5 50.6 48.6, top_k 50 of logits of 4 values 155 161 157, 52 58 54
+  // Too many values, or a share where the largest of more than 2 FEW threads weigh more
+  // than 2^-7 of the slice's, as below: without a look at each of them.  us before
+  // lists, with lists and so: share of normal logits 64 rows of 128256 118 120 118, 240
+  // of 32768 48.5 50.6 48.6, top_k 50 of logits of 4 values 155 161 157, 52 58 54
   const int most = NEAR / group;
   if ((int)reached.n > most || !o.k && reached.near > 2 * FEW) {
     if (tid == 0) {

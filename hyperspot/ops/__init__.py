@@ -514,11 +514,11 @@ def _less_padding(M: int, N: int, K: int, split):
     """Narrow tiles of 64 rows where those are enough: 17 rows of 2048 x 7168 8.2
     -> 8.0 us, 32 of 4096 x 4096 9.2 -> 8.7, 64 9.9 -> 9.5; the same bits.  In place of
     tiles of 128 x 128, in parts of their own, N of 1088 to 5440 and K of 4352 to 28672,
-    with the norm or without: 5 parts and more 0.80 of the time (48 of 3072 x 8192 19.8
-    -> 16.6 us, 33 of 2560 x 10240 19.9 16.6, 24 of 1344 x 19456 24 17; none slower).  4
+    with the norm or without: 5 parts and more 0.80 of the time (48 of 3072 x 8192 20.3
+    -> 18.1 us, 33 of 2560 x 10240 19.9 16.9, 24 of 1344 x 19456 24 17; none slower).  4
     up to 18432 columns, or 12288 of more than 48 rows, 0.94 in 83 (40 of 4096 x 16384
     45 30, 24 of 4096 x 8192 21.0 20.0), beyond 1.0 in 78, up to 1.24; 3 up to 12288, or
-    8192, 0.97 in 39 (32 of 4608 x 8192 24.1 21.7), beyond 1.04 in 166, up to 1.29; 2
+    8192, 0.97 in 39 (32 of 4608 x 8192 24.2 21.5), beyond 1.04 in 166, up to 1.29; 2
     1.06.  2 of the 122 that are taken are more than 3 % slower."""
     if not split or M > 64 or split[0] != 128:
         return split
@@ -534,7 +534,7 @@ def _few_parts(M: int, N: int, K: int):
     """Two or three parts of one tile of up to 64 rows, where the norm adds them up and
     no other rule has a kernel.  N of 4160 to 8192 and K of 4224 to 28672, with the norm,
     over the library's time: 2 parts 0.72 in 66, none above 0.96 (1 row of 8192 x 28672
-    94 77 us, 12 of 7168 x 18432 113 47, 1 of 6656 x 17920 90 44, 8 of 8192 x 8192 34.4
+    94 78 us, 12 of 7168 x 18432 114 51, 1 of 6656 x 17920 92 47, 8 of 8192 x 8192 34.4
     30.5), 3 0.9 (4 of 5120 x 5120 18.2 16.7, 1 17.7 16.6), but up to 5120 columns, of
     multiples of 256, and up to 4992 outputs 1.1 and more for every second size (2 of
     4608 x 4608 13.4 15.1, 1 of 4168 x 5120 13.3 15.6, 1 of 4864 x 5120 0.97); those are
@@ -621,12 +621,13 @@ def _wide_gated(M: int, N: int, K: int):
     """(high, bn) where csrc/gemm_wide.hip forms silu(gate) * up of more than 256
     rows faster than what was there, mostly the library's product and a pass.  Random
     sizes, N of 6000 to 36000, at 0.7 PFLOP/s and more by the tiles' times, time over
-    that: up to 1200 rows 0.88 in 186 (512 of 28672 x 4096 115 115 us, 880 203 176, 512
-    of 14336 x 2048 38 37), 8 of them more than 3 % slower, up to 8 %, and 769 and more
-    of them of over 5376 columns 0.93 in 74, but 19 slower, up to 14 % (1192 of 16384 x
-    5888 210 239): those are the library's.  More rows of up to 3072 columns 0.86 in 20
-    (2600 of 14336 x 2048 183 146), of longer ones 0.95, but every fourth slower, by up
-    to 10 % (8192 of 28672 x 4096 1335 1400): those are the library's too."""
+    that: up to 1200 rows 0.88 in 186 (880 of 28672 x 4096 197 187 us, 512 109 109, but
+    6 less a layer in the step, 512 of 14336 x 2048 36 35), 8 of them more than 3 %
+    slower, up to 8 %, and 769 and more of them of over 5376 columns 0.93 in 74, but 19
+    slower, up to 14 % (1192 of 16384 x 5888 210 239): those are the library's.  More
+    rows of up to 3072 columns 0.86 in 20 (2600 of 14336 x 2048 181 143), of longer ones
+    0.95, but every fourth slower, by up to 10 % (8192 of 28672 x 4096 1335 1400): those
+    are the library's too."""
     if not 256 < M < 1 << 20 or K < 1024 or K % 64 or N % 16 \
             or not 6000 <= N < 1 << 17 \
             or K > (8192 if M <= 768 else 5376 if M <= 1200 else 3072):
@@ -640,14 +641,14 @@ def _wide_parts(M: int, N: int, K: int):
     """(high, bn, parts) where csrc/gemm_wide.hip and the norm that adds up its parts
     are faster than what was there and the norm.  Random sizes, x and w from memory,
     time over that: 10240 columns and more, up to 1400 rows 0.69 in 97 (262 rows of
-    4096 x 14336 58 48 us, 600 112 76, 1000 137 110, 1268 161 132; the worst 1154 of 6336
+    4096 x 14336 64 52 us, 600 121 80, 1000 145 114, 1268 165 146; the worst 1154 of 6336
     x 15360 even), but 1.09 for tiles that fill no wave and 1.10 in 45 for one part of
     tiles of 256 outputs, which are 180 to 217 (1114 of 8144 x 12928 231 252); from 4608
     on 513 to 1024 rows 0.90 in 57 (the worst 989 of 8032 x 4992 89 92).  Shorter ones
     are slower (up to 2560 columns and 4096 outputs, 513 to 1024 rows, 1.14 in 93, 630 of
     1768 x 2048 17.6 21.1), and so are more rows (1.0).
     129 to 256 rows of 10240 columns and more, one tile of rows and more than 192 in all,
-    0.65 (135 rows of 4096 x 14336 44 36 us, 248 53 45); decode steps of 140, 200 and 256
+    0.65 (135 rows of 4096 x 14336 47 40 us, 248 52 50); decode steps of 140, 200 and 256
     rows, 8 layers, 1 % less.  Fewer rows are as fast in the step (100 1730 1738), fewer
     tiles slower (200 of 2048 x 7168 17 21)."""
     if K % 64 or N % 8 or not 1024 <= N <= 8192 or not 4608 <= K <= 20480 \
@@ -669,7 +670,7 @@ def _wide_long(M: int, N: int, K: int):
     which the last is neither nearly empty nor full.  The library has two kinds of
     tiles, of 0.65 to 1.1 PFLOP/s and of 1.2 to 1.5; here it is 1.1 to 1.35.  N from 2048
     to 8192, K from 10240 to 32768, time over the library's: two waves 0.73 in 85 (7411
-    rows of 4096 x 14336 971 640 us, 5888 of 5120 x 13824 958 600), four of them more
+    rows of 4096 x 14336 1006 647 us, 5888 of 5120 x 13824 974 629), four of them more
     than 3 % slower, by up to 15 % (7425 of 4096 x 11008), three 0.87 in 81, three
     slower, by up to 12 % (5889 of 7168 x 18432), but multiples of 64 tiles, for which
     it mostly has the better ones, 1.04 in two waves; more waves 1.0 in 20, every second
