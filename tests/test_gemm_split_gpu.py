@@ -342,9 +342,15 @@ def test_parts_of_one_tile_of_rows(M, N, K):
     pad = lambda t, n: torch.nn.functional.pad(t, (0, n))[:, :K]
     assert torch.equal(ops.linear_parts(pad(x, 8), pad(w, 16384)).data, got.data)
     _check(ops.linear_parts(pad(x, 8), pad(w, 8)).data.sum(0), x, w)
+    # a row alone, where it has as many parts, has the same sums
+    alone = {1088: 6}.get(N, parts)
+    assert ops._route(1, N, K, True) == (64, 64, alone)
     one = ops.linear_parts(x[M - 1:], w)
-    if one.__class__ is got.__class__ and one.data.shape[0] == parts:
+    assert one.data.shape == (alone, 1, N)
+    if alone == parts:
         assert torch.equal(one.data[:, 0], got.data[:, M - 1])
+    else:
+        _check(one.data.sum(0), x[M - 1:], w)
 
 
 def test_rule_of_several_waves():

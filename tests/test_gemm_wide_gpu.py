@@ -89,11 +89,28 @@ def test_numbers_that_are_not_finite():
 def test_parts_and_norm(M, N, K):
     assert ops._wide_parts(M, N, K) and not ops._wide_parts(128, N, K)
     x, w = _inputs(M, N, K)
-    y = ops.linear_parts(x, w)
-    y = y.data.sum(0) if isinstance(y, ops.Parts) else y
+    got = ops.linear_parts(x, w)
+    parts = ops._wide_parts(M, N, K)[2]
+    assert isinstance(got, ops.Parts) and got.data.shape == (parts, M, N)
     want, slack = _bounds(x, w)
+    y = got.data.sum(0)
     assert ((y.double() - want).abs()
             <= 2.0 ** -8 * want.abs() + 2 * slack).all()
+    # the norms add the parts in their order and round the sum as a product is
+    g = torch.Generator().manual_seed(M)
+    rand = lambda *s: torch.randn(*s, generator=g).bfloat16().to(DEV)
+    res, norm, router = rand(M, N), rand(N), rand(8, N)
+    y = got.data[0].clone()
+    for z in range(1, parts):
+        y += got.data[z]
+    h, r = ops.fused_add_rmsnorm(y.bfloat16(), res.clone(), norm, 1e-5)
+    out, out_res = ops.fused_add_rmsnorm(got, res.clone(), norm, 1e-5)
+    routed, routed_res = ops.fused_add_rmsnorm_route(got, res.clone(), norm, 1e-5,
+                                                     router, 2)
+    assert torch.equal(out_res, r) and torch.equal(routed_res, r)
+    # the squares may be added in another order: the last bit of a row's scale
+    for n in (out, routed.data):
+        assert ((n.float() - h.float()).abs() <= h.float().abs() * 2.0 ** -7).all()
 
 
 @pytest.mark.gpu
@@ -196,4 +213,15 @@ def test_rules_cover_all_rows():
                 16 if rule is ops._wide_gated else 8) == 0
             assert 4 <= high <= 8 and bn in (128, 256)
             assert 1 <= parts <= 8 and parts * 64 <= K
+            assert parts == 1 or rule is ops._wide_parts
+            # tiles are counted as they are launched, and are no more than needed
+            every = range(1, 9) if rule is ops._wide_parts else (1,)
+            counted = ops._wide_tile(M, N, K, tuple(every))
+            assert counted[1:4] == (high, bn, parts)
+            rows = -(-M // (32 * high))
+            assert counted[4] == rows * -(-N // bn) * parts
+            assert rows * 32 * high >= M > (rows - 1) * 32 * high
+            assert rows <= -(-M // 256) + (M > 256)
+            if parts > 1:
+                assert counted[4] <= 256
     assert taken > 200
