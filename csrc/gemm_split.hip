@@ -18,7 +18,7 @@
 // in parts, and from 129 on with long columns, are csrc/gemm_wide.hip's where its rules
 // take them (4096 x 14336 256 rows 45, 512 66):
 //   4096 x 14336  32 rows 33 26, 96 68 38, 192 112 46, 256 66 52, 512 98 70
-//   6144 x 4096   96 rows 24 20, 192 35 28, 256 44 29
+//   6144 x 4096   96 rows 24 23, 192 35 28, 256 44 29
 //   4096 x 4096   32 rows 14 11, 96 23 16, 192 34 21, 256 23 23
 //   2048 x 7168   32 rows 19 11, 96 20 15, 192 26 19, 256 26 22, 512 33 32
 //   5120 x 8192   32 rows 27 22, 96 39 28, 192 64 36, 256 79 38

@@ -380,13 +380,15 @@ def _wave_of_rows(M: int, N: int, K: int):
 
 
 def _wave_of_longer_rows(M: int, N: int, K: int):
-    """The same tiles for 65 to 128 rows and longer columns where they are at least 176,
-    before parts of K that a pass adds up.  Random sizes, time over what was there: K up
-    to 4608 0.92 in 158 (96 rows of 6144 x 4096 21.8 -> 20.0 us, 128 23.8 23.2, 66 of
-    7168 x 4096 24.6 20.2), one more than 3 % slower, but of 97 to 128 rows up to 3712
-    columns 1.03 in 62, up to 1.32 (125 of 6032 x 2560 13.7 17.0); up to 5632 0.97, every
-    seventh slower, up to 1.11 (128 of 6144 x 5120 27.4 28.8), beyond 1.06; fewer tiles
-    1.05 to 1.2.  Where the norm adds up the parts those are faster (96 rows 17.4)."""
+    """The same tiles for 65 to 128 rows and longer columns where they are at least 176
+    and the product would be the library's.  Random sizes, time over that: K up to 4608
+    0.92 (66 rows of 7168 x 4096 24.6 -> 20.2 us), but of 97 to 128 rows up to 3712
+    columns 1.03 in 62, up to 1.32 (125 of 6032 x 2560 13.7 17.0); longer ones every
+    seventh slower, up to 1.11; fewer tiles 1.05 to 1.2.  In decode steps, a layer, 5632 x
+    2560 to 8192 x 4608, 66 to 128 rows 1 to 8 us less.  In place of parts of 128 x 128 and
+    the pass that adds them up, up to 6528 outputs from 4096 columns on, a product is 1 us
+    faster by itself and a layer 0 to 4 us slower (8 layers with 6144 x 4096, 66 rows 1114
+    -> 1128, 96 1143 1173, 128 1306 1330): they stay."""
     if not 64 < M <= 128 or K % 128 or N % 4 \
             or not (2304 if M <= 96 else 3712) < K <= 4608:
         return None
@@ -401,14 +403,14 @@ def _route(M: int, N: int, K: int, parts: bool):
     step of small prompts, which is not captured, waits for the host."""
     if K >= 1 << 24:                # the kernels' chunks are counted in 32 bits
         return None
-    wave = _wave_gemm(M, N, K) or _waves_gemm(M, N, K) \
-        or (None if parts else _wave_of_longer_rows(M, N, K))
+    wave = _wave_gemm(M, N, K) or _waves_gemm(M, N, K)
     if wave is not None:
         return wave
     if _rows_gemm_sizes(M, N, K) and _native().gemm_rows_fits(M, K):
         return "rows"
     return _less_padding(M, N, K, _split_gemm(M, N, K)) \
-        or (_summed_gemm(M, N, K) or _few_parts(M, N, K) if parts else None) \
+        or (_summed_gemm(M, N, K) or _few_parts(M, N, K) if parts
+            else _wave_of_longer_rows(M, N, K)) \
         or _wave_of_rows(M, N, K)
 
 
@@ -458,9 +460,9 @@ def _split_gemm(M: int, N: int, K: int):
     rows, 21 of outputs and 4 parts are 252, but 33 on some dies: 384 rows of
     2688 x 7552 took 47 us, the library 37).  Measured at 17 to 512 rows, N of
     512 to 9000 and K of 4096 to 20000: 0.67 of the library's time on average,
-    and more than 3 % slower at 1 of 100 sizes.  Few parts gain less than the library's tiles up to 128 rows and from 257 on
-    (us, library and kernel: 8192 x 8192, 4 parts, 64 rows 33 43; 5120 x 8192,
-    3 parts, 320 rows 49 54).  From 257 rows on short rows gain little or
+    and more than 3 % slower at 1 of 100 sizes.  Few parts gain less than the
+    library's tiles up to 128 rows and from 257 on (us, library and kernel: 8192 x
+    8192, 4 parts, 64 rows 33 43; 5120 x 8192, 3 parts, 320 rows 49 54).  From 257 rows on short rows gain little or
     nothing (3072 x 6144, 320 rows 28 30; 4096 x 6144 37 36, 512 rows 44 42).
     Below 14M weights it is the faster one from K of 5120 on (2048 x 6144, 64
     rows 19.5 12.3, 256 23 20) and about even with K of 4096 (2048 x 4096, 96

@@ -450,7 +450,8 @@ def test_wave_of_rows(M, N, K):
 
 
 def test_rule_of_a_wave_of_longer_rows():
-    """65 to 128 rows: 176 to 256 tiles, without a norm that adds up parts."""
+    """65 to 128 rows: 176 to 256 tiles, without a norm that adds up parts and where
+    there are none of 128 x 128 either."""
     for M, N, K, rule in [
             (65, 5632, 2432, (64, 64, 1)), (65, 5568, 4096, None),
             (128, 8192, 4608, (64, 64, 1)), (128, 8196, 4096, None),
@@ -460,12 +461,16 @@ def test_rule_of_a_wave_of_longer_rows():
             (129, 6144, 4096, None), (64, 6144, 4096, None),
             (96, 6144, 4160, None), (96, 6142, 4096, None)]:
         assert ops._wave_of_longer_rows(M, N, K) == rule, (M, N, K)
-    assert ops._route(96, 6144, 4096, False) == (64, 64, 1)
-    assert ops._route(96, 6144, 4096, True) == ops._split_gemm(96, 6144, 4096)
+    for M, N, K in [(66, 6144, 4096), (96, 6144, 4096), (128, 6528, 4608)]:
+        for parts in (True, False):
+            assert ops._route(M, N, K, parts) == ops._split_gemm(M, N, K) \
+                == (128, 128, 5)
+    for M, N, K in [(66, 6656, 4096), (128, 6144, 3968), (96, 8192, 4608)]:
+        assert ops._route(M, N, K, False) == (64, 64, 1)
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,N,K", [(65, 5572, 2432), (96, 6144, 4096),
+@pytest.mark.parametrize("M,N,K", [(65, 5572, 2432), (96, 6656, 4096),
                                    (128, 8188, 4608)])
 def test_wave_of_longer_rows(M, N, K):
     g = torch.Generator().manual_seed(M)
