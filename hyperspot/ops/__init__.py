@@ -462,16 +462,17 @@ def _split_gemm(M: int, N: int, K: int):
     512 to 9000 and K of 4096 to 20000: 0.67 of the library's time on average,
     and more than 3 % slower at 1 of 100 sizes.  Few parts gain less than the
     library's tiles up to 128 rows and from 257 on (us, library and kernel: 8192 x
-    8192, 4 parts, 64 rows 33 43; 5120 x 8192, 3 parts, 320 rows 49 54).  From 257 rows on short rows gain little or
-    nothing (3072 x 6144, 320 rows 28 30; 4096 x 6144 37 36, 512 rows 44 42).
-    Below 14M weights it is the faster one from K of 5120 on (2048 x 6144, 64
-    rows 19.5 12.3, 256 23 20) and about even with K of 4096 (2048 x 4096, 96
-    rows 12.7 12.6, 128 12.7 14.9); all these are left to the library.  So are
-    257 to 320 rows of up to 3264 outputs in tall tiles, K up to 12288 (3072
-    x 8192, 288 rows 34 38; 3136 x 7680, 257 rows 32 37), 129 to 144 rows of
-    more than 6528 outputs (7168 x 7168 42 45; 6400 x 6400 at 0.68), and up to
-    32 rows where those of w lie a multiple of 32 KB apart (4096 x 16384 31
-    42).  Narrow tiles where K is short and they fill as many units.
+    8192, 4 parts, 64 rows 33 43; 5120 x 8192, 3 parts, 320 rows 49 54).  From
+    257 rows on short rows gain little or nothing (3072 x 6144, 320 rows 28 30;
+    4096 x 6144 37 36, 512 rows 44 42).   Below 14M weights it is the faster one
+    from K of 5120 on (2048 x 6144, 64 rows 19.5 12.3, 256 23 20) and about even
+    with K of 4096 (2048 x 4096, 96 rows 12.7 12.6, 128 12.7 14.9); all these
+    are left to the library.  So are 257 to 320 rows of up to 3264 outputs in
+    tall tiles, K up to 12288 (3072 x 8192, 288 rows 34 38; 3136 x 7680, 257
+    rows 32 37), 129 to 144 rows of more than 6528 outputs (7168 x 7168 42 45;
+    6400 x 6400 at 0.68), and up to 32 rows where those of w lie a multiple of
+    32 KB apart (4096 x 16384 31 42).  Narrow tiles where K is short and they
+    fill as many units.
     129 to 256 rows in one tile, which loads three quarters of what two do, where
     that saves more than twice the parts cost: 120 sizes of K from 4608 to 20480,
     over what was there 0.86 with 4 or 5 parts (256 of 5648 x 7552 45 37, 192 of 7152
