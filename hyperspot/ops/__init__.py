@@ -464,7 +464,7 @@ def _split_gemm(M: int, N: int, K: int):
     library's tiles up to 128 rows and from 257 on (us, library and kernel: 8192 x
     8192, 4 parts, 64 rows 33 43; 5120 x 8192, 3 parts, 320 rows 49 54).  From
     257 rows on short rows gain little or nothing (3072 x 6144, 320 rows 28 30;
-    4096 x 6144 37 36, 512 rows 44 42).   Below 14M weights it is the faster one
+    4096 x 6144 37 36, 512 rows 44 42).  Below 14M weights it is the faster one
     from K of 5120 on (2048 x 6144, 64 rows 19.5 12.3, 256 23 20) and about even
     with K of 4096 (2048 x 4096, 96 rows 12.7 12.6, 128 12.7 14.9); all these
     are left to the library.  So are 257 to 320 rows of up to 3264 outputs in
